@@ -94,6 +94,40 @@ def test_gemm(a_dtype, w_dtype, o_dtype, M, N, K):
     assert rel_err(got, want) <= tol(o_dtype)
 
 
+@pytest.mark.parametrize("N,K", [(1, 1), (17, 31), (130, 260), (1000, 96), (4100, 257), (16400, 64),
+                                 (96, 3072)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_gemm_float32_does_not_depend_on_the_batch(N, K, offset):
+    """float32 operands: every kernel the number of rows leads to (edges of its tiles, K that is
+    no multiple of a step, operands 4 bytes off their alignment) is within the error bound of a
+    32-bit sum, and a row's result is the same bits in all of them."""
+    ops = _ops()
+    sizes = [1, 16, 17, 32, 33, 64, 65, 300] + ([1100] if N * K <= 300000 else [])
+    top = max(sizes)
+    a = torch.empty((top * K + offset,), device=DEV)[offset:].view(top, K)
+    w = torch.empty((N * K + offset,), device=DEV)[offset:].view(N, K)
+    a.copy_(_rand((top, K), torch.float32, 40))
+    w.copy_(_rand((N, K), torch.float32, 41, 0.05))
+    base = _rand((top, N), torch.float32, 42).to(DEV)
+    exact = a.double() @ w.double().T
+    # |error| <= n eps sum |a w| for any order of n products and sums, eps = 2^-24
+    bound = (K + 1) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T) + 1e-30
+    first = None
+    for M in sizes:
+        got = torch.full((M, N), float("nan"), device=DEV)
+        ops.gemm(a[:M], w, got)
+        assert bool(((got.double() - exact[:M]).abs() <= bound[:M]).all()), M
+        first = got if first is None else first
+        assert torch.equal(got[:len(first)], first), M
+        first = got
+        summed = base[:M].clone()
+        ops.gemm(a[:M], w, summed, accumulate=True)
+        assert torch.equal(summed, base[:M] + got), M
+        small = torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
+        ops.gemm(a[:M], w, small)
+        assert torch.equal(small, got.to(torch.bfloat16)), M
+
+
 @pytest.mark.parametrize("M", [1, 3, 8, 16, 17, 33, 64, 65, 130, 300, 517])
 @pytest.mark.parametrize("N,K", [(1000, 136), (96, 64), (777, 320), (4100, 4096), (256, 1032)])
 @pytest.mark.parametrize("o_dtype,accumulate", [(torch.bfloat16, False), (torch.float32, False),

@@ -1,9 +1,11 @@
 // Matrix products C[M,N] = A[M,K] * W[N,K]^T (the weight is [out, in], as in the reference:
 // y[r] = sum_c W[r,c] x[c], src/tensor/storage/store.zig:286-319).
 //
-//  * gemm_fma: 32-bit FMA, any storage types, any sizes.  Every output element is the sum of
-//    its products in ascending k, whatever M is and wherever the row lies in the batch, so a
-//    token's result does not depend on how the batch was cut.  This is the true 32-bit path.
+//  * gemm_f32: float32 operands, 32-bit MFMAs, any sizes: the true 32-bit path.  One order of
+//    the sum whatever M is and wherever the row lies in the batch, so a token's result does not
+//    depend on how the batch was cut.
+//  * gemm_fma: 32-bit FMA for mixed storage types, any sizes.  Every output element is the sum
+//    of its products in ascending k, whatever M is and wherever the row lies in the batch.
 #include <type_traits>
 
 #include "zf_common.h"
@@ -81,15 +83,14 @@ static void launch_fma(const void* A, const void* W, void* C, int M, int N, int 
                        (const TA*)A, (const TW*)W, (TO*)C, M, N, K);
 }
 
-// dtypes: ZF_F32 / ZF_BF16 for a, w, out.  accumulate: out += (else out =).
+// dtypes: ZF_F32 / ZF_BF16 for a, w, out, a and w not both float32 (zf_gemm_f32 takes those).
+// accumulate: out += (else out =).
 extern "C" int zf_gemm_fma(const void* A, int a_dtype, const void* W, int w_dtype, void* C,
                            int c_dtype, int M, int N, int K, int accumulate,
                            hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   const int key = a_dtype * 4 + w_dtype * 2 + c_dtype;
   switch (key) {
-    case 0: launch_fma<float, float, float>(A, W, C, M, N, K, accumulate, stream); break;
-    case 1: launch_fma<float, float, bf16_t>(A, W, C, M, N, K, accumulate, stream); break;
     case 2: launch_fma<float, bf16_t, float>(A, W, C, M, N, K, accumulate, stream); break;
     case 3: launch_fma<float, bf16_t, bf16_t>(A, W, C, M, N, K, accumulate, stream); break;
     case 4: launch_fma<bf16_t, float, float>(A, W, C, M, N, K, accumulate, stream); break;
@@ -112,6 +113,253 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
 typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2_t;
+
+// ------------------------------------------------------------------ 32-bit MFMA product
+// A, W and the sums are float32 throughout: v_mfma_f32_16x16x4_f32 multiplies and adds in full
+// 32-bit precision, at 256 flops a cycle and CU (154 TFLOP/s; a VALU loop of scalar FMAs gets
+// half of that at best and, with 4 x 4 outputs a thread, one LDS word per FMA, a tenth).
+//
+// One order of the sum for every number of rows, so that a token's result does not depend on
+// how the batch was cut: K is dealt in eight spans (F32_SPAN below, a function of K alone), each
+// summed from zero in ascending steps of 32, and the spans are added in ascending order to zero.
+// Inside a step of 32 a lane's group g = lane / 16 holds k = 8 g .. 8 g + 7, and MFMA j takes
+// element j of every group, which lets 16-byte loads of rows feed the operands as they are.
+// Two kernels follow that order:
+//   * up to 64 rows, bound by reading W (one user of the 0.6B shape's float32 weights: 1.9 GB a
+//     token): a workgroup of eight waves, one span each, takes 16 rows of W (32 with a wide
+//     output) for all tokens; a wave's loads of a step are 16 whole lines of 128 bytes, straight
+//     into the operands, four steps in flight; the eight partials meet in LDS.
+//   * above, bound by the MFMAs: tiles of 128 x 128, 64 x 64 or 32 x 32 through LDS (rows of 36
+//     words: the 16-byte operand reads of 16 rows fall into different banks), the next step's
+//     loads in flight during the products.  The largest tile that still gives 256 workgroups.
+// Measured (weights from HBM, us, against the scalar loop of 64 x 64 tiles before): 4 tokens into
+// 1024 outputs over K = 3072 290 -> 13, 6144 x 1024 107 -> 8.2, 151936 x 1024 474 -> 120 (5.2
+// TB/s), 4096 x 12288 1254 -> 64; 256 tokens into 1024 x 3072 350 -> 42, 6144 x 1024 163 -> 47;
+// 2048 tokens into 24576 x 4096 10925 -> 4071 (101 TFLOP/s; the vendor's product 154).  Up to 64
+// rows the streaming kernel wins or draws (48 tokens: 24576 x 4096 240 us, the tiles at 96: 258).
+static __host__ __device__ __forceinline__ int f32_span(int K) { return (K + 255) / 256 * 32; }
+#define F32_SPANS 8
+
+// four consecutive k of one row; what lies at or beyond k_end is 0
+template <bool VEC>
+__device__ __forceinline__ f32x4_t f32_load4(const float* __restrict__ row, int k, int k_end) {
+  if constexpr (VEC) {        // K a multiple of 4 and 16-byte aligned rows: all four or none
+    return k < k_end ? *(const f32x4_t*)(row + k) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+  } else {
+    f32x4_t v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = k + i < k_end ? row[k + i] : 0.f;
+    return v;
+  }
+}
+
+// outputs n .. n + 3 of row m (sum: their 32-bit sums); vec: 16-byte stores are aligned
+template <typename TO, bool ACC>
+__device__ __forceinline__ void f32_store4(TO* __restrict__ C, int m, int n, int N, bool vec,
+                                           f32x4_t sum) {
+  TO* c = C + (size_t)m * N + n;
+  if constexpr (std::is_same<TO, float>::value) {
+    if (vec && n + 3 < N) {
+      if constexpr (ACC) sum = *(const f32x4_t*)c + sum;
+      *(f32x4_t*)c = sum;
+      return;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (n + i < N) store_from_float<TO>(c + i, ACC ? load_as_float<TO>(c + i) + sum[i] : sum[i]);
+}
+
+template <typename TO, bool ACC, int RG, int MT, bool VEC>
+__global__ __launch_bounds__(F32_SPANS * 64) void gemm_f32_stream_kernel(
+    const float* __restrict__ A, const float* __restrict__ W, TO* __restrict__ C, int M, int N,
+    int K, int span, bool vec_out) {
+  __shared__ f32x4_t part[F32_SPANS][RG * MT][64];
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
+  const int n0 = blockIdx.x * 16 * RG, m0 = blockIdx.y * 16 * MT;
+  // rows beyond the matrices read its last row; nothing of theirs is stored
+  const float* w[RG];
+  const float* a[MT];
+#pragma unroll
+  for (int i = 0; i < RG; ++i) w[i] = W + (size_t)min(n0 + 16 * i + r, N - 1) * K;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) a[i] = A + (size_t)min(m0 + 16 * i + r, M - 1) * K;
+  f32x4_t acc[RG][MT];
+#pragma unroll
+  for (int i = 0; i < RG; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int k_end = min(K, (wave + 1) * span);
+#pragma unroll (RG * MT >= 4 ? 1 : RG * MT == 2 ? 2 : 4)
+  for (int k0 = wave * span; k0 < k_end; k0 += 32) {
+    const int k = k0 + 8 * g;
+    f32x4_t wf[RG][2], af[MT][2];
+#pragma unroll
+    for (int i = 0; i < RG; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) wf[i][h] = f32_load4<VEC>(w[i], k + 4 * h, k_end);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) af[i][h] = f32_load4<VEC>(a[i], k + 4 * h, k_end);
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+#pragma unroll
+      for (int i = 0; i < RG; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][s / 4][s % 4], af[j][s / 4][s % 4],
+                                                           acc[i][j], 0, 0, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < RG; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) part[wave][i * MT + j][lane] = acc[i][j];
+  __syncthreads();
+  if (threadIdx.x >= RG * MT * 64) return;
+  // a lane's column is a token, its four rows are outputs: tile `wave` of the RG x MT ones
+  f32x4_t sum = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < F32_SPANS; ++s) sum += part[s][wave][lane];
+  const int m = m0 + 16 * (wave % MT) + r, n = n0 + 16 * (wave / MT) + 4 * g;
+  if (m < M) f32_store4<TO, ACC>(C, m, n, N, vec_out, sum);
+}
+
+#define F32_LD 36
+// B x B outputs a workgroup of 2 x 2 waves
+template <typename TO, bool ACC, int B, bool VEC>
+__global__ __launch_bounds__(256) void gemm_f32_tile_kernel(
+    const float* __restrict__ A, const float* __restrict__ W, TO* __restrict__ C, int M, int N,
+    int K, int span, bool vec_out) {
+  constexpr int F = B / 32, L = B / 32;      // 16-wide fragments a wave and side; loads a thread
+  __shared__ float As[2][B][F32_LD];
+  __shared__ float Ws[2][B][F32_LD];
+  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64, r = lane % 16, g = lane / 16;
+  const int n0 = blockIdx.x * B, m0 = blockIdx.y * B;
+  const int wm = (wave % 2) * (B / 2), wn = (wave / 2) * (B / 2);
+  const int lr = tid / 8, lk = (tid % 8) * 4;        // staging: 32 rows x 128 bytes a pass
+  const float *ap[L], *wp[L];
+#pragma unroll
+  for (int i = 0; i < L; ++i) {
+    ap[i] = A + (size_t)min(m0 + lr + 32 * i, M - 1) * K;
+    wp[i] = W + (size_t)min(n0 + lr + 32 * i, N - 1) * K;
+  }
+  f32x4_t acc[F][F], sum[F][F], ar[L], wr[L];
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j) acc[i][j] = sum[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int steps = (K + 31) / 32, per = span / 32;
+#pragma unroll
+  for (int i = 0; i < L; ++i) {
+    ar[i] = f32_load4<VEC>(ap[i], lk, K);
+    wr[i] = f32_load4<VEC>(wp[i], lk, K);
+  }
+  int in_span = 0;
+  for (int st = 0; st < steps; ++st) {
+    const int b = st % 2;
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+      *(f32x4_t*)&As[b][lr + 32 * i][lk] = ar[i];
+      *(f32x4_t*)&Ws[b][lr + 32 * i][lk] = wr[i];
+    }
+    // one barrier a step: the buffer written next was last read before the barrier of this step
+    __syncthreads();
+    if (st + 1 < steps) {
+#pragma unroll
+      for (int i = 0; i < L; ++i) {
+        ar[i] = f32_load4<VEC>(ap[i], (st + 1) * 32 + lk, K);
+        wr[i] = f32_load4<VEC>(wp[i], (st + 1) * 32 + lk, K);
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      f32x4_t wf[F], af[F];
+#pragma unroll
+      for (int i = 0; i < F; ++i) {
+        wf[i] = *(const f32x4_t*)&Ws[b][wn + 16 * i + r][8 * g + 4 * h];
+        af[i] = *(const f32x4_t*)&As[b][wm + 16 * i + r][8 * g + 4 * h];
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < F; ++i)
+#pragma unroll
+          for (int j = 0; j < F; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][s], af[j][s], acc[i][j], 0, 0, 0);
+    }
+    if (++in_span == per || st + 1 == steps) {
+      in_span = 0;
+#pragma unroll
+      for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j) {
+          sum[i][j] += acc[i][j];
+          acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j) {
+      const int m = m0 + wm + 16 * j + r, n = n0 + wn + 16 * i + 4 * g;
+      if (m < M) f32_store4<TO, ACC>(C, m, n, N, vec_out, sum[i][j]);
+    }
+}
+
+template <typename TO, bool ACC, bool VEC>
+static void launch_f32(const float* A, const float* W, TO* C, int M, int N, int K, bool vec_out,
+                       hipStream_t stream) {
+  const int span = f32_span(K);
+#define F32_STREAM(RG, MT)                                                                       \
+  hipLaunchKernelGGL((gemm_f32_stream_kernel<TO, ACC, RG, MT, VEC>),                             \
+                     dim3((N + 16 * RG - 1) / (16 * RG), (M + 16 * MT - 1) / (16 * MT)),         \
+                     dim3(F32_SPANS * 64), 0, stream, A, W, C, M, N, K, span, vec_out)
+#define F32_TILE(B)                                                                              \
+  hipLaunchKernelGGL((gemm_f32_tile_kernel<TO, ACC, B, VEC>), dim3((N + B - 1) / B,              \
+                     (M + B - 1) / B), dim3(256), 0, stream, A, W, C, M, N, K, span, vec_out)
+  const auto tiles = [&](int b) { return (long long)((M + b - 1) / b) * ((N + b - 1) / b); };
+  if (M <= 16) {
+    if (N >= 16384) F32_STREAM(2, 1); else F32_STREAM(1, 1);
+  } else if (M <= 32) {
+    F32_STREAM(1, 2);
+  } else if (M <= 64) {
+    F32_STREAM(1, 4);
+  } else if (tiles(128) >= 256) {
+    F32_TILE(128);
+  } else if (tiles(64) >= 256) {
+    F32_TILE(64);
+  } else {
+    F32_TILE(32);
+  }
+#undef F32_STREAM
+#undef F32_TILE
+}
+
+// out = A W^T (accumulate: out += A W^T); A and W float32, out float32 or bfloat16; any sizes,
+// any alignment of the elements
+extern "C" int zf_gemm_f32(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K,
+                           int accumulate, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (K < 0 || (c_dtype != ZF_F32 && c_dtype != ZF_BF16)) return -1;
+  const bool vec = K % 4 == 0 && ((uintptr_t)A | (uintptr_t)W) % 16 == 0;
+  const bool vec_out = N % 4 == 0 && (uintptr_t)C % 16 == 0;
+  const float *a = (const float*)A, *w = (const float*)W;
+#define F32_GO(TO, ACC)                                                            \
+  do {                                                                             \
+    if (vec) launch_f32<TO, ACC, true>(a, w, (TO*)C, M, N, K, vec_out, stream);    \
+    else launch_f32<TO, ACC, false>(a, w, (TO*)C, M, N, K, vec_out, stream);       \
+  } while (0)
+  if (c_dtype == ZF_F32) {
+    if (accumulate) F32_GO(float, true); else F32_GO(float, false);
+  } else {
+    if (accumulate) return -1;
+    F32_GO(bf16_t, false);
+  }
+#undef F32_GO
+  ZF_CHECK_LAUNCH();
+}
 
 #define EPI_STORE_BF16 0
 #define EPI_STORE_F32 1

@@ -926,8 +926,9 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
 
     bfloat16 operands with K a multiple of 8 go to the MFMA kernels (weight streaming for up
     to 16 rows of ``a``, and up to 64 where the kernel for 17 to 128 rows does not cover the
-    sizes; LDS-tiled above); everything else, the whole 32-bit path included,
-    goes to the FMA kernel, whose results do not depend on how rows are batched."""
+    sizes; LDS-tiled above).  float32 operands, the whole 32-bit path, go to the kernels of
+    32-bit MFMAs, mixed ones to the FMA kernel; the results of both do not depend on how rows
+    are batched."""
     _need_gpu(a, w, out)
     M, K = a.shape
     N = w.shape[0]
@@ -990,6 +991,10 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
             _check(lib.zf_gemm_bf16_tile(_ptr(a), _ptr(w), _ptr(out), M, N, K, epi, variant,
                                          1 if w_tiled else 0, _stream()),
                    "gemm (tiled)")
+        return
+    if a.dtype == torch.float32 and w.dtype == torch.float32:
+        _check(lib.zf_gemm_f32(_ptr(a), _ptr(w), _ptr(out), _dt(out), M, N, K,
+                               1 if accumulate else 0, _stream()), "gemm (32-bit)")
         return
     _check(lib.zf_gemm_fma(_ptr(a), _dt(a), _ptr(w), _dt(w), _ptr(out), _dt(out), M, N, K,
                            1 if accumulate else 0, _stream()), "gemm")
