@@ -145,6 +145,125 @@ def test_experts(T, W, ff, E, top, dt):
     assert float(gates.max()) > limit
 
 
+@pytest.mark.parametrize("T, W, ff, E, top", [(1, 64, 64, 3, 2), (16, 128, 192, 5, 4),
+                                               (7, 320, 64, 40, 6), (16, 64, 576, 2, 16),
+                                               (9, 64, 1088, 1, 3)])
+@pytest.mark.parametrize("kind", ["gated", "plain", "shared", "shared gate"])
+def test_experts_of_a_few_tokens_against_plain(T, W, ff, E, top, kind):
+    """bfloat16, up to 16 tokens: every used expert once for all its pairs.  Ids name experts,
+    some of them twice a token (up to 3 units of 16 pairs an expert) and some none; with an expert
+    that all tokens share; a token's result is the same bits alone."""
+    dt = torch.bfloat16
+    limit, alpha, shift, sff = 0.6, 1.702, 1.0, 128
+    plain, shared = kind == "plain", kind.startswith("shared")
+    h = _rand((T, W), 14, dtype=dt)
+    gate_up = _rand((E, ff if plain else 2 * ff, W), 15, 2 / W ** 0.5, dt)
+    down = _rand((E, W, ff), 16, 2 / ff ** 0.5, dt)
+    s_gu, s_down = _rand((2 * sff, W), 17, 2 / W ** 0.5, dt), _rand((W, sff), 18, 2 / sff ** 0.5, dt)
+    g = torch.Generator().manual_seed(19)
+    ids = torch.randint(0, E + 1, (T, top), generator=g).to(torch.int32)      # E: no expert
+    share = torch.rand((T, top), generator=g)
+    factor = torch.rand((T, 2), generator=g) if kind == "shared gate" else None
+    base = _rand((T, W), 20)
+    act = "relu2" if plain else None
+    tiled = [torch.stack([ops.pretile_weight(m) for m in w.to(DEV)]) for w in (gate_up, down)]
+    assert ops.moe_few_covers(h.to(DEV), top) and ops.moe_can_pretile(*tiled)
+
+    def run(rows, add):
+        n = len(rows)
+        y = torch.full((n, top, ff), float("nan"), dtype=dt, device=DEV)
+        ys = torch.full((n, sff), float("nan"), dtype=dt, device=DEV)
+        out = base[rows].to(DEV)
+        f = None if factor is None else factor[rows].to(DEV)[:, 1]
+        more = (ops.pretile_weight(s_gu.to(DEV)), ops.pretile_weight(s_down.to(DEV)), ys, 0.7,
+                1.0, 0.0, f) if shared else None
+        ops.moe_experts(h[rows].contiguous().to(DEV), *tiled, ids[rows].contiguous().to(DEV),
+                        share[rows].contiguous().to(DEV), y, out, limit, alpha, shift, add=add,
+                        act=act, n_identity=1, w_tiled=True, shared=more)
+        return out
+
+    def unit(z, lim, a, b, ff):
+        gate, up = torch.clamp(z[:ff], max=lim), torch.clamp(z[ff:], -lim, lim)
+        return gate * torch.sigmoid(a * gate) * (up + b)
+
+    want = torch.zeros((T, W), dtype=torch.float64)
+    for t in range(T):
+        x = h[t].double()
+        for s_ in range(top):
+            e, c = int(ids[t, s_]), share[t, s_].double()
+            if e == E:
+                want[t] += c * x
+                continue
+            z = gate_up[e].double() @ x
+            z = torch.clamp(z, min=0.0) ** 2 if plain else unit(z, limit, alpha, shift, ff)
+            want[t] += c * (down[e].double() @ z.to(dt).double())
+        if shared:
+            z = unit(s_gu.double() @ x, 0.7, 1.0, 0.0, sff)
+            z = z * (1.0 if factor is None else factor[t, 1].double())
+            want[t] += s_down.double() @ z.to(dt).double()
+    everyone = list(range(T))
+    # (the activations round to bfloat16 from sums of another order: half a last place of each)
+    got = run(everyone, False)
+    assert rel_err(got, want) < 1e-2
+    assert rel_err(run(everyone, True), want + base.double()) < 1e-2
+    for t in (0, T - 1):
+        assert torch.equal(run([t], False)[0], got[t])
+    if not shared:
+        # more tokens, sorted by expert: the same bits from pre-tiled matrices as from rows
+        many = [t % T for t in range(40)]
+        outs = []
+        for w_tiled, (gu, dn) in ((True, tiled), (False, (gate_up.to(DEV), down.to(DEV)))):
+            y = torch.empty((40, top, ff), dtype=dt, device=DEV)
+            outs.append(torch.empty((40, W), device=DEV))
+            ops.moe_experts(h[many].to(DEV), gu, dn, ids[many].to(DEV), share[many].to(DEV), y,
+                            outs[-1], limit, alpha, shift, act=act, n_identity=1, w_tiled=w_tiled)
+        assert torch.equal(*outs) and rel_err(outs[0][:T], want) < 1e-2
+
+
+@pytest.mark.parametrize("E, top, extra", [(5, 5, 0), (31, 4, 2), (64, 6, 1), (128, 9, 0), (129, 9, 0)])
+@pytest.mark.parametrize("T", [1, 16, 35])
+@pytest.mark.parametrize("scoring", ["softmax", "sigmoid", "softmax_all"])
+def test_router_ties_and_what_cannot_be_chosen(E, top, extra, T, scoring):
+    """Equal logits go to the lower index, NaN and -inf are never chosen (expert 0 stands in),
+    around the number of rows where the kernel changes, at an odd width."""
+    W, extra = 33, 0 if scoring == "softmax" else extra
+    g = torch.Generator().manual_seed(3)
+    h = torch.zeros((T, W))
+    h[:, 0] = 1.0
+    router = torch.zeros((E + extra, W))
+    router[:, 0] = torch.randint(-2, 3, (E + extra,), generator=g).float()
+    router[min(3, E - 1), 0] = float("nan")
+    if scoring == "softmax":
+        router[min(4, E - 1), 0] = -float("inf")
+    ids = torch.empty((T, top), dtype=torch.int32, device=DEV)
+    wts = torch.empty((T, top), dtype=torch.float32, device=DEV)
+    more = torch.empty((T, extra), device=DEV) if extra else None
+    correction = None
+    if scoring != "softmax":
+        # (a soft-max over all with a NaN among them is NaN: bring it in behind the scores)
+        router[min(3, E - 1), 0] = 1.0
+        correction = torch.zeros(E)
+        correction[min(3, E - 1)] = float("nan")
+        correction[min(4, E - 1)] = -float("inf")
+    ops.moe_route(h.to(DEV), router.to(DEV), None, ids, wts, scoring=scoring, extra=more,
+                  correction=None if correction is None else correction.to(DEV), normalize=True)
+    z = router[:E, 0].double()
+    s = z if scoring == "softmax" else torch.sigmoid(z) if scoring == "sigmoid" else torch.softmax(z, 0)
+    choice = s if correction is None else s + correction.double()
+    order = sorted((e for e in range(E) if float(choice[e]) > -float("inf")),
+                   key=lambda e: (-float(choice[e]), e))[:top]
+    stand_in = [0] * (top - len(order))
+    assert ids.cpu().tolist() == [order + stand_in] * T
+    if scoring == "softmax":
+        w = torch.cat([torch.softmax(s[order], 0), torch.zeros(len(stand_in), dtype=torch.float64)])
+    else:
+        w = s[order + stand_in]
+        w = w / (w.sum() + 1e-20)
+    assert torch.allclose(wts.cpu().double(), w.expand(T, top), atol=1e-6)
+    if extra:
+        assert torch.allclose(more.cpu(), torch.sigmoid(router[E:, 0]).expand(T, extra), atol=1e-6)
+
+
 @pytest.mark.parametrize("T, W, ff, E, top", [(40, 64, 24, 6, 2), (300, 128, 64, 8, 3),
                                                (17, 72, 136, 1, 1), (150, 352, 104, 40, 4),
                                                (260, 64, 8, 3, 3)])

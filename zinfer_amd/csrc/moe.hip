@@ -13,10 +13,11 @@
 //
 // Expert matrices are stacked: gate_up [E, 2 * ff, W] (an expert's gate rows, then its up
 // rows) and down [E, W, ff].  Three kernels that stream the weights of the chosen experts
-// token by token; every token's result depends on that token alone and its sums run in a
+// token by token (float32, and bfloat16 sizes that the kernels for few tokens further down do
+// not take); every token's result depends on that token alone and its sums run in a
 // fixed order, so a token gives the same bits whatever else is in the batch:
 //
-//  * moe_route         a workgroup per four tokens
+//  * moe_route         a workgroup per sixteen tokens (four with more than 128 router rows)
 //  * moe_gate_up       grid (token * slot, groups of outputs): y[t, slot, :] of the expert in
 //                      that slot, the token's row staged in LDS as 32-bit numbers
 //  * moe_down          grid (token, groups of outputs): out[t, n] (=, or += into) the weighted
@@ -231,11 +232,288 @@ __global__ __launch_bounds__(MOE_ROUTE_WAVES * ZF_WAVE) void moe_route_kernel(
   }
 }
 
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float moe_f32x4_t;
+
+// Up to 128 router rows, 16 tokens a tile.  The logits are 32-bit MFMAs (16x16x4: rows of the
+// router against the tokens, h widened), K dealt into 64 spans, eight to a group: a group's spans
+// are added in order, then the groups, so a token's logits do not depend on the tokens beside it
+// nor on how many there are.  Then a wave ranks a token's logits all at once: an expert's rank is
+// the number of experts before it (larger, or equal and of a lower index), one pass over a row in
+// LDS instead of a round of twelve lane exchanges for every chosen one.
+//   * more than 64 tokens: a workgroup of 16 waves takes a tile, two groups at a time.
+//   * up to 64 (SPLIT): one compute unit draws a router of 256 KB in 8 us, so a workgroup of eight
+//     waves takes one group of K and 32 rows of the router, leaves its sums in `ws` and adds one to
+//     the tile's counter; the one that finds the count complete adds the groups and chooses.  Sums
+//     and counter go through to memory (agent scope), where every XCD sees them; the counter is
+//     back at zero when the kernel ends.
+// Measured (bfloat16 h, in a graph, us; before: four tokens a workgroup and rounds of arg-max): W =
+// 2048, 32 experts, 4 a token, 8 tokens 17.0 -> 11.9 (a single workgroup 14.1), 2048 tokens 31 ->
+// 18; W = 4096, 64 experts, 8 a token, 8 tokens 48.8 -> 16.5 (a single workgroup 41).
+#define MOE_ROUTE16_ROWS 128
+#define MOE_ROUTE16_GROUPS 8
+#define MOE_ROUTE16_SPLIT_TILES 4        // up to so many tiles of 16 tokens are split
+
+__device__ __forceinline__ void store_agent(float* p, float v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float load_agent(const float* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// eight consecutive values of a row as floats; at or beyond k_end they are 0
+template <typename T, bool VEC>
+__device__ __forceinline__ void route_load8(const T* __restrict__ row, int k, int k_end,
+                                            float (&v)[8]) {
+  if constexpr (VEC) {             // (W a multiple of 8: all eight or none)
+    if (k < k_end) {
+      if constexpr (sizeof(T) == 2) {
+        const uint4 x = *(const uint4*)(row + k);
+        const uint32_t p[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          v[2 * c] = __uint_as_float(p[c] << 16);
+          v[2 * c + 1] = __uint_as_float(p[c] & 0xffff0000u);
+        }
+      } else {
+        const float4 x = *(const float4*)(row + k), y = *(const float4*)(row + k + 4);
+        v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+        v[4] = y.x; v[5] = y.y; v[6] = y.z; v[7] = y.w;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = 0.f;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = k + i < k_end ? load_as_float<T>(row + k + i) : 0.f;
+  }
+}
+
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// how many of row[0 .. n4 * 4) come before (v, e): larger, or equal with a lower index (NaN: none)
+__device__ __forceinline__ int rank_before(const float* row, int n4, float v, int e) {
+  int rank = 0;
+  for (int j = 0; j < n4; ++j) {
+    const float4 o = *(const float4*)(row + 4 * j);
+    const float ov[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rank += ov[i] > v || (ov[i] == v && 4 * j + i < e);
+  }
+  return rank;
+}
+
+// one wave: token t's logits in `z` (LDS, -inf from E up to a multiple of 4) to its experts and
+// weights; share and chosen: room for as many numbers
+__device__ __forceinline__ void route_choose(float* z, float* share, int* chosen, int* __restrict__ ids,
+                             float* __restrict__ weights, int t, int E, int top, int scoring,
+                             const float* __restrict__ correction, int n_groups, int keep_groups,
+                             int mark_top, int normalize, float weight_scale, int lane) {
+  const int n4 = (E + 3) / 4;
+  if (scoring != 0) {
+    // scores s = sigmoid(z), or the soft-max over all of z (kept in `share`), choice scores
+    // s + correction (in `z`)
+    float zmax = 0.f, zsum = 1.f;
+    if (scoring == 2) {
+      zmax = -INFINITY;
+      for (int e = lane; e < E; e += ZF_WAVE) zmax = fmaxf(zmax, z[e]);
+      zmax = wave_max(zmax);
+      zsum = 0.f;
+      for (int e = lane; e < E; e += ZF_WAVE) zsum += expf(z[e] - zmax);
+      zsum = wave_sum(zsum);
+    }
+    for (int e = lane; e < E; e += ZF_WAVE) {
+      const float sc = scoring == 2 ? expf(z[e] - zmax) / zsum : 1.0f / (1.0f + expf(-z[e]));
+      share[e] = sc;
+      z[e] = sc + (correction != nullptr ? correction[e] : 0.f);
+    }
+    wave_lds_fence();
+    if (n_groups > 0 && keep_groups < n_groups) {
+      // a group's mark: its two largest choice scores added (its one score, if it has one)
+      float* mark = (float*)chosen;
+      const int size = E / n_groups, g4 = (n_groups + 3) / 4;
+      for (int q = lane; q < 4 * g4; q += ZF_WAVE) {
+        float a = -INFINITY, b = -INFINITY;
+        if (q < n_groups)
+          for (int e = q * size; e < (q + 1) * size; ++e) {
+            const float v = z[e];
+            if (v > a) { b = a; a = v; } else if (v > b) { b = v; }
+          }
+        // (a sum of +inf and -inf ranks last, as -inf does)
+        const float m = (size > 1 && mark_top > 1) ? a + b : a;
+        mark[q] = m == m ? m : -INFINITY;
+      }
+      wave_lds_fence();
+      // outside the kept groups nothing can be chosen
+      bool out[2] = {false, false};
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int e = lane + ZF_WAVE * i;
+        if (e < E) out[i] = rank_before(mark, g4, mark[e / size], e / size) >= keep_groups;
+      }
+      wave_lds_fence();
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        if (out[i]) z[lane + ZF_WAVE * i] = -INFINITY;
+      wave_lds_fence();
+    }
+  }
+  // the chosen in the order of their scores; where nothing but NaN or -inf is left, expert 0
+  for (int k = lane; k < top; k += ZF_WAVE) chosen[k] = -1;
+  wave_lds_fence();
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int e = lane + ZF_WAVE * i;
+    const float v = e < E ? z[e] : -INFINITY;
+    if (v > -INFINITY) {
+      const int rank = rank_before(z, n4, v, e);
+      if (rank < top) chosen[rank] = e;
+    }
+  }
+  wave_lds_fence();
+  if (scoring == 0) {
+    const float first = chosen[0] >= 0 ? z[chosen[0]] : -INFINITY;
+    for (int k = lane; k < top; k += ZF_WAVE)
+      share[k] = expf((chosen[k] >= 0 ? z[chosen[k]] : -INFINITY) - first);
+    wave_lds_fence();
+    float sum = 0.f;
+    for (int k = 0; k < top; ++k) sum += share[k];
+    for (int k = lane; k < top; k += ZF_WAVE) {
+      ids[(size_t)t * top + k] = max(chosen[k], 0);
+      weights[(size_t)t * top + k] = share[k] / sum;
+    }
+    return;
+  }
+  float sum = 0.f;
+  for (int k = 0; k < top; ++k) sum += share[max(chosen[k], 0)];
+  for (int k = lane; k < top; k += ZF_WAVE) {
+    const int e = max(chosen[k], 0);
+    ids[(size_t)t * top + k] = e;
+    weights[(size_t)t * top + k] = (normalize ? share[e] / (sum + 1e-20f) : share[e]) * weight_scale;
+  }
+}
+
+template <typename T, bool VEC, bool SPLIT>
+__global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel(
+    const T* __restrict__ h, const float* __restrict__ router, const float* __restrict__ bias,
+    int* __restrict__ ids, float* __restrict__ weights, int n_tokens, int W, int E, int top,
+    int scoring, const float* __restrict__ correction, int n_groups, int keep_groups,
+    int mark_top, int normalize, float weight_scale, int n_extra, float* __restrict__ extra,
+    float* __restrict__ ws, int* __restrict__ counters) {
+  constexpr int WAVES = SPLIT ? 8 : 16;
+  __shared__ moe_f32x4_t part[WAVES][2][ZF_WAVE];
+  __shared__ __attribute__((aligned(16))) float zs[16][MOE_ROUTE16_ROWS];
+  __shared__ __attribute__((aligned(16))) float shares[16][MOE_ROUTE16_ROWS];
+  __shared__ __attribute__((aligned(16))) int chosens[16][MOE_ROUTE16_ROWS];
+  __shared__ int arrived;
+  const int wave = threadIdx.x / ZF_WAVE, lane = threadIdx.x % ZF_WAVE;
+  const int r = lane % 16, g = lane / 16, tile = SPLIT ? blockIdx.y : blockIdx.x, t0 = tile * 16;
+  const int rows = E + n_extra, chunks = (rows + 31) / 32;        // 32 rows of the router
+  const int span = (W + 2047) / 2048 * 32;
+  const T* row = h + (size_t)min(t0 + r, n_tokens - 1) * W;
+  // column lane % 16 is a token, the four numbers are rows 4 (lane / 16) + i of the 16-row tile
+  auto take = [&](int chunk, int half, moe_f32x4_t z) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int e = chunk * 32 + 16 * half + 4 * g + i;
+      if (e < E) {
+        zs[r][e] = z[i] + (bias != nullptr ? bias[e] : 0.f);
+      } else {
+        if (e < rows && t0 + r < n_tokens)
+          extra[(size_t)(t0 + r) * n_extra + (e - E)] = 1.0f / (1.0f + expf(-z[i]));
+        if (e < MOE_ROUTE16_ROWS) zs[r][e] = -INFINITY;           // no candidates
+      }
+    }
+  };
+  const int c0 = SPLIT ? blockIdx.x / MOE_ROUTE16_GROUPS : 0, c1 = SPLIT ? c0 + 1 : chunks;
+  for (int chunk = c0; chunk < c1; ++chunk) {
+    const float *ra = router + (size_t)min(chunk * 32 + r, rows - 1) * W,
+                *rb = router + (size_t)min(chunk * 32 + 16 + r, rows - 1) * W;
+    moe_f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+    for (int grp = SPLIT ? blockIdx.x % MOE_ROUTE16_GROUPS : 0;
+         grp < (SPLIT ? (int)blockIdx.x % MOE_ROUTE16_GROUPS + 1 : MOE_ROUTE16_GROUPS);
+         grp += WAVES / 8) {
+      const int k_begin = ((grp + wave / 8) * 8 + wave % 8) * span, k_end = min(W, k_begin + span);
+      moe_f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 2
+      for (int k0 = k_begin; k0 < k_end; k0 += 32) {
+        float x[8], a[8], b[8];
+        route_load8<T, VEC>(row, k0 + 8 * g, k_end, x);
+        route_load8<float, VEC>(ra, k0 + 8 * g, k_end, a);
+        route_load8<float, VEC>(rb, k0 + 8 * g, k_end, b);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], x[i], acc[0], 0, 0, 0);
+          acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[i], x[i], acc[1], 0, 0, 0);
+        }
+      }
+      part[wave][0][lane] = acc[0];
+      part[wave][1][lane] = acc[1];
+      __syncthreads();
+      if (wave < 2) {
+#pragma unroll
+        for (int w8 = 0; w8 < WAVES / 8; ++w8) {
+          moe_f32x4_t z = part[8 * w8][wave][lane];
+#pragma unroll
+          for (int s = 1; s < 8; ++s) z += part[8 * w8 + s][wave][lane];
+          sum += z;
+        }
+      }
+      __syncthreads();
+    }
+    if constexpr (SPLIT) {
+      // [tile][chunk][half][lane][group][4]
+      if (wave < 2) {
+        float* p = ws + ((((size_t)tile * chunks + chunk) * 2 + wave) * ZF_WAVE + lane) *
+                            (MOE_ROUTE16_GROUPS * 4) + blockIdx.x % MOE_ROUTE16_GROUPS * 4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) store_agent(p + i, sum[i]);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      }
+    } else if (wave < 2) {
+      take(chunk, wave, sum);
+    }
+  }
+  __syncthreads();
+  if constexpr (SPLIT) {
+    const int all = chunks * MOE_ROUTE16_GROUPS;
+    if (threadIdx.x == 0)
+      arrived = __hip_atomic_fetch_add(counters + tile, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (arrived != all - 1) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (threadIdx.x == 0)
+      __hip_atomic_store(counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (wave < 2 * chunks) {            // (at most 128 rows: 8 halves of 16, one a wave)
+      const float* p = ws + (((size_t)tile * chunks * 2 + wave) * ZF_WAVE + lane) *
+                                (MOE_ROUTE16_GROUPS * 4);
+      float v[MOE_ROUTE16_GROUPS * 4];
+#pragma unroll
+      for (int i = 0; i < MOE_ROUTE16_GROUPS * 4; ++i) v[i] = load_agent(p + i);
+      moe_f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int grp = 0; grp < MOE_ROUTE16_GROUPS; ++grp)
+        sum += moe_f32x4_t{v[4 * grp], v[4 * grp + 1], v[4 * grp + 2], v[4 * grp + 3]};
+      take(wave / 2, wave % 2, sum);
+    }
+    __syncthreads();
+  }
+  for (int k = wave; k < 16 && t0 + k < n_tokens; k += WAVES)
+    route_choose(zs[k], shares[k], chosens[k], ids, weights, t0 + k, E, top, scoring, correction,
+                 n_groups, keep_groups, mark_top, normalize, weight_scale, lane);
+}
+
+// ws: float32 [4 tiles][(E + n_extra + 31) / 32][4096] and counters [4] at zero (both or neither;
+// the counters are at zero again when the kernel ends): what up to 64 tokens and 128 router rows
+// use to spread over workgroups.
 extern "C" int zf_moe_route(const void* h, int dtype, const float* router, const float* bias,
                             int* ids, float* weights, int T, int W, int E, int top,
                             int scoring, const float* correction, int n_groups, int keep_groups,
                             int mark_top, int normalize, float weight_scale, int n_extra,
-                            float* extra, hipStream_t stream) {
+                            float* extra, float* ws, int* counters, hipStream_t stream) {
   if (T <= 0) return 0;
   if (E <= 0 || E > MOE_MAX_EXPERTS || top <= 0 || top > E || scoring < 0 || scoring > 2 ||
       n_extra < 0 || (n_extra > 0 && extra == nullptr) || mark_top < 1 || mark_top > 2 ||
@@ -243,6 +521,30 @@ extern "C" int zf_moe_route(const void* h, int dtype, const float* router, const
                                         keep_groups > n_groups ||
                                         top > keep_groups * (E / n_groups))))
     return -2;
+  if (E + n_extra <= MOE_ROUTE16_ROWS) {
+    const bool vec = W % 8 == 0 && ((uintptr_t)h | (uintptr_t)router) % 16 == 0;
+    const bool split = T <= 16 * MOE_ROUTE16_SPLIT_TILES && ws != nullptr && counters != nullptr;
+#define MOE_ROUTE16_AS(TT, V, S, G, B)                                                           \
+  hipLaunchKernelGGL((moe_route16_kernel<TT, V, S>), G, dim3(B), 0, stream, (const TT*)h,        \
+                     router, bias, ids, weights, T, W, E, top, scoring, correction, n_groups,    \
+                     keep_groups, mark_top, normalize, weight_scale, n_extra, extra, ws, counters)
+#define MOE_ROUTE16(TT, V)                                                                       \
+  do {                                                                                           \
+    if (split)                                                                                   \
+      MOE_ROUTE16_AS(TT, V, true,                                                                \
+                     dim3((E + n_extra + 31) / 32 * MOE_ROUTE16_GROUPS, (T + 15) / 16), 512);    \
+    else                                                                                         \
+      MOE_ROUTE16_AS(TT, V, false, dim3((T + 15) / 16), 1024);                                   \
+  } while (0)
+    if (dtype == ZF_F32) {
+      if (vec) MOE_ROUTE16(float, true); else MOE_ROUTE16(float, false);
+    } else {
+      if (vec) MOE_ROUTE16(bf16_t, true); else MOE_ROUTE16(bf16_t, false);
+    }
+#undef MOE_ROUTE16_AS
+#undef MOE_ROUTE16
+    ZF_CHECK_LAUNCH();
+  }
   const dim3 grid((T + MOE_ROUTE_TOKENS - 1) / MOE_ROUTE_TOKENS), block(MOE_ROUTE_WAVES * ZF_WAVE);
   if (dtype == ZF_F32)
     hipLaunchKernelGGL(moe_route_kernel<float>, grid, block, 0, stream, (const float*)h, router,
@@ -563,6 +865,330 @@ extern "C" int zf_gated_act(const void* gu, void* out, int dtype, int T, int ff,
 }
 
 // =====================================================================================
+//  Up to 16 tokens (bfloat16, matrices pre-tiled): every used expert's matrices are read once
+//  for all tokens that chose it, 16 rows of a matrix against those tokens as columns of 16x16x32
+//  MFMAs.  Token by token, 8 tokens with 4 of 32 experts each read 32 experts' worth where about
+//  21 are used; the kernels are bound by that reading, and a CU alone draws no more than about a
+//  256th of what the chip does, so both kernels spread it over all of them.
+//    * moe_few_up    a workgroup of four waves per (unit, 16 outputs), K dealt to the waves in
+//                    blocks of 64, the partials added in wave order; the activation in the
+//                    epilogue.  A unit is an expert and up to 16 of its pairs (token, slot): the
+//                    workgroup of pair p finds with a few ballots over the ids whether p starts a
+//                    unit, else it ends.  The first workgroups take 16 outputs each of the expert
+//                    that all tokens share, if there is one.
+//    * moe_few_down  a workgroup of sixteen waves per 8 outputs, for all experts: (unit of up to 8
+//                    pairs, piece of ff) after piece by each wave.  The 16 rows and columns of an
+//                    MFMA are 8 outputs and 8 pairs at two neighbouring blocks of 64 of ff: only
+//                    the products of like halves are used, and 2048 outputs make 256 workgroups.
+//                    Partials in LDS, added per pair in order of the pieces, per token in slot
+//                    order, the shared expert last.  (Fetching the next piece's operands before a
+//                    piece's products was no faster; a workgroup per unit and 32 outputs whose last
+//                    one to arrive adds the sums took 10 % less at W = 4096, 64 experts and 8
+//                    tokens, 15 % more at 16 tokens, and more in the decode step.)
+//  The matrices lie as the matrix kernels' pre-tiled ones, [rows / 16][K / 64][2][64 lanes][8]: a
+//  wave's load is consecutive memory.  A column of an MFMA depends on its own token alone
+//  and all sums have a fixed order: a token's bits do not depend on the others.
+//  Measured (MI355X, both kernels in a graph, us, against the token-by-token kernels): W = 2048, ff
+//  = 768, 32 experts, 4 a token: 1 token 18 -> 17.6, 8 tokens 55 -> 46 (21 experts: 24.6 for the
+//  first, 5.9 TB/s, 22 for the second), 16 tokens 90 -> 71; W = 4096, ff = 1024, 64 experts, 8 a
+//  token: 1 token 50 -> 42, 8 tokens 241 -> 204 (6.1 and 5.1 TB/s), 16 tokens 448 -> 283.
+// =====================================================================================
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 moe_bf16x8_t;
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t moe_u32x4_t;
+
+#define MOE_FEW_TOKENS 16
+#define MOE_FEW_PAIRS 256
+
+// (weights are read once a step: loads that need not stay in the caches)
+__device__ __forceinline__ moe_u32x4_t few_load_w(const bf16_t* p) {
+  return __builtin_nontemporal_load((const moe_u32x4_t*)p);
+}
+
+// Whether pair p, of expert e, starts a unit: up to 16 pairs of one expert, in their order; then
+// `column` (LDS, the wave's own) holds them, -1 where there are fewer.  The same in every lane.
+// Ids from n_experts on name no expert.  (A token may name an expert twice: 17 pairs, two units.)
+__device__ __forceinline__ bool few_columns(const int* __restrict__ ids, int P, int p, int e,
+                                            int n_experts, int lane, int* column) {
+  if (e >= n_experts) return false;
+  int id[4];
+  unsigned long long uses[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int i = 64 * c + lane;
+    id[c] = i < P ? ids[i] : -1;
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) uses[c] = __ballot(id[c] == e);
+  int rank = 0;                              // pairs of this expert before p
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    if (p >= 64 * c)
+      rank += __popcll(p >= 64 * c + 64 ? uses[c] : uses[c] & ((1ull << (p - 64 * c)) - 1));
+  if (rank % 16 != 0) return false;
+  if (lane < 16) column[lane] = -1;
+  __builtin_amdgcn_wave_barrier();
+  int before = -rank;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int at = before + __popcll(uses[c] & ((1ull << lane) - 1));
+    if (id[c] == e && at >= 0 && at < 16) column[at] = 64 * c + lane;
+    before += __popcll(uses[c]);
+  }
+  wave_lds_fence();
+  return true;
+}
+
+template <bool GATED>
+__global__ __launch_bounds__(256) void moe_few_up_kernel(
+    const bf16_t* __restrict__ h, const bf16_t* __restrict__ w, const int* __restrict__ ids,
+    bf16_t* __restrict__ y, int T, int W, int ff, int top, float limit, float alpha, float shift,
+    int act, int n_experts, const bf16_t* __restrict__ shared_w, bf16_t* __restrict__ shared_y,
+    int shared_ff, float s_limit, float s_alpha, float s_shift, const float* __restrict__ factor,
+    int factor_stride) {
+  __shared__ moe_f32x4_t part[4][2][ZF_WAVE];
+  __shared__ int column[4][16];
+  const int wave = threadIdx.x / ZF_WAVE, lane = threadIdx.x % ZF_WAVE;
+  const int r = lane % 16, g = lane / 16, shared_blocks = shared_ff / 16, blocks = W / 64;
+  const bool shared = (int)blockIdx.x < shared_blocks;
+  int pair, token, j0;                         // pair: this lane's column, -1: none
+  const bf16_t *wg, *wu;
+  if (shared) {
+    j0 = blockIdx.x * 16;
+    pair = r < T ? r : -1;
+    token = r < T ? r : 0;
+    wg = shared_w + (size_t)(j0 / 16) * blocks * 1024;
+    wu = wg + (size_t)(shared_ff / 16) * blocks * 1024;
+  } else {
+    const int P = T * top, b = blockIdx.x - shared_blocks, p = b % P;
+    j0 = b / P * 16;
+    const int e = ids[p];
+    if (!few_columns(ids, P, p, e, n_experts, lane, column[wave])) return;
+    pair = column[wave][r];
+    token = (pair >= 0 ? pair : p) / top;
+    wg = w + ((size_t)e * (GATED ? 2 : 1) * ff + j0) / 16 * blocks * 1024;
+    wu = wg + (size_t)(ff / 16) * blocks * 1024;
+  }
+  wg += lane * 8;
+  wu += lane * 8;
+  const bf16_t* x = h + (size_t)token * W + 16 * g;
+  moe_f32x4_t ag = {0.f, 0.f, 0.f, 0.f}, au = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int kb = wave; kb < blocks; kb += 4) {
+    moe_u32x4_t xf[2], gf[2], uf[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      gf[i] = few_load_w(wg + (size_t)kb * 1024 + i * 512);
+      if constexpr (GATED) uf[i] = few_load_w(wu + (size_t)kb * 1024 + i * 512);
+      xf[i] = *(const moe_u32x4_t*)(x + kb * 64 + i * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      ag = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&gf[i],
+                                                   *(const moe_bf16x8_t*)&xf[i], ag, 0, 0, 0);
+      if constexpr (GATED)
+        au = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&uf[i],
+                                                     *(const moe_bf16x8_t*)&xf[i], au, 0, 0, 0);
+    }
+  }
+  part[wave][0][lane] = ag;
+  part[wave][1][lane] = au;
+  __syncthreads();
+  if (wave != 0 || pair < 0) return;
+#pragma unroll
+  for (int s = 1; s < 4; ++s) {
+    ag += part[s][0][lane];
+    au += part[s][1][lane];
+  }
+  // column r is the pair, the four numbers are outputs j0 + 4 g + i
+  const float f = shared && factor != nullptr ? factor[(size_t)pair * factor_stride] : 1.0f;
+  uint32_t v[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float o;
+    if constexpr (GATED)
+      o = shared ? gated_unit(ag[i], au[i], s_limit, s_alpha, s_shift)
+                 : gated_unit(ag[i], au[i], limit, alpha, shift);
+    else
+      o = activation_value(ag[i], act);
+    v[i] = float_to_bf16(shared ? o * f : o);
+  }
+  bf16_t* dst = (shared ? shared_y + (size_t)pair * shared_ff : y + (size_t)pair * ff) + j0 + 4 * g;
+  *(uint2*)dst = make_uint2(v[0] | v[1] << 16, v[2] | v[3] << 16);
+}
+
+__global__ __launch_bounds__(1024) void moe_few_down_kernel(
+    const bf16_t* __restrict__ y, const bf16_t* __restrict__ down, const int* __restrict__ ids,
+    const float* __restrict__ weights, float* __restrict__ out, int T, int W, int ff, int top,
+    int add, int n_experts, const bf16_t* __restrict__ h, int piece,
+    const bf16_t* __restrict__ shared_w, const bf16_t* __restrict__ shared_y, int shared_ff) {
+  __shared__ int n_units, id[MOE_FEW_PAIRS], expert[MOE_FEW_PAIRS];
+  __shared__ float share[MOE_FEW_PAIRS];
+  __shared__ short pairs[MOE_FEW_PAIRS][8];            // of a unit; -1 where it has fewer
+  extern __shared__ __attribute__((aligned(16))) float sums[];   // [pair][2 pieces][8], then shared's
+  const int wave = threadIdx.x / ZF_WAVE, lane = threadIdx.x % ZF_WAVE;
+  const int r = lane % 16, g = lane / 16, n0 = blockIdx.x * 8, P = T * top;
+  const int blocks = ff / 64, pieces = (blocks + 2 * piece - 1) / (2 * piece);
+  const int s_blocks = shared_ff / 64, s_pieces = (s_blocks + 2 * piece - 1) / (2 * piece);
+  float* s_sums = sums + (size_t)P * pieces * 16;
+  // what the sums at the end want, asked for now
+  const int t = threadIdx.x / 8, n = threadIdx.x % 8;
+  const float before = add && t < T ? out[(size_t)t * W + n0 + n] : 0.f;
+  if (wave == 1)
+    for (int i = lane; i < P; i += ZF_WAVE) share[i] = weights[i];
+  // one wave lists the units, in the order of their first pairs
+  if (wave == 0) {
+    int mine[4], rank[4] = {0, 0, 0, 0};                // this lane's pairs: experts, ranks in them
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int i = 64 * c + lane;
+      mine[c] = i < P ? ids[i] : n_experts;
+      if (i < P) id[i] = mine[c];
+      *(moe_u32x4_t*)&pairs[i][0] = moe_u32x4_t{~0u, ~0u, ~0u, ~0u};
+    }
+#pragma unroll
+    for (int cj = 0; cj < 4; ++cj)
+      for (int j = 0; j < min(64, P - 64 * cj); ++j) {
+        const int e = __builtin_amdgcn_readlane(mine[cj], j);
+#pragma unroll
+        for (int c = cj; c < 4; ++c)
+          if (64 * c < P) rank[c] += mine[c] == e && (c > cj || j < lane);
+      }
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (mine[c] >= n_experts) rank[c] = -1;
+    int units = 0;
+#pragma unroll
+    for (int cj = 0; cj < 4; ++cj)
+      for (int j = 0; j < min(64, P - 64 * cj); ++j) {
+        const int e = __builtin_amdgcn_readlane(mine[cj], j), rj = __builtin_amdgcn_readlane(rank[cj], j);
+        if (rj < 0 || rj % 8 != 0) continue;
+        if (lane == 0) expert[units] = e;
+#pragma unroll
+        for (int c = cj; c < 4; ++c)
+          if (mine[c] == e && rank[c] >= rj && rank[c] < rj + 8)
+            pairs[units][rank[c] - rj] = (short)(64 * c + lane);
+        ++units;
+      }
+    if (lane == 0) n_units = units;
+  }
+  __syncthreads();
+  const int jobs = n_units * pieces + s_pieces, half = r / 8;
+  for (int q = wave; q < jobs; q += 16) {
+    const bool shared = q < s_pieces;
+    const int unit = (q - s_pieces) / pieces, c = shared ? q : (q - s_pieces) % pieces;
+    const int nb = shared ? s_blocks : blocks;
+    int pair;
+    const bf16_t *wr, *x;
+    // rows r and columns r: output n0 + r % 8 and pair r % 8 at the blocks 2 i + r / 8
+    for (int p0 = 0; p0 < (shared ? T : 8); p0 += 8) {
+      if (shared) {
+        pair = p0 + r % 8 < T ? p0 + r % 8 : -1;
+        wr = shared_w;
+        x = shared_y + (size_t)max(pair, 0) * shared_ff;
+      } else {
+        pair = pairs[unit][r % 8];
+        wr = down + (size_t)expert[unit] * W * ff;
+        x = y + (size_t)(pair >= 0 ? pair : pairs[unit][0]) * ff;
+      }
+      wr += (size_t)(n0 / 16) * nb * 1024 + (g * 16 + n0 % 16 + r % 8) * 8;
+      x += 16 * g;
+      const int b0 = c * 2 * piece, b1 = min(nb, b0 + 2 * piece);
+      moe_f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+      for (int kb = b0; kb < b1; kb += 2) {
+        // (behind an odd last block the upper half repeats it against zeros)
+        const bool in = kb + half < b1;
+        const int k = in ? kb + half : kb;
+        moe_u32x4_t wf[2], xf[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          wf[i] = few_load_w(wr + (size_t)k * 1024 + i * 512);
+          xf[i] = *(const moe_u32x4_t*)(x + k * 64 + i * 8);
+          if (!in) wf[i] = xf[i] = moe_u32x4_t{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&wf[i],
+                                                        *(const moe_bf16x8_t*)&xf[i], acc, 0, 0, 0);
+      }
+      // rows 4 g + i of column r: like halves are g / 2 == half
+      if (pair >= 0 && g / 2 == half)
+        *(moe_f32x4_t*)((shared ? s_sums + ((size_t)pair * s_pieces + c) * 16
+                                : sums + ((size_t)pair * pieces + c) * 16) + 8 * half + 4 * (g % 2)) =
+            acc;
+    }
+  }
+  __syncthreads();
+  if (t >= T) return;
+  float total = 0.f, same = 0.f;
+  for (int s = 0; s < top; ++s) {
+    const int ts = t * top + s;
+    const float c = share[ts];
+    if (id[ts] >= n_experts) {                  // no expert: the token's own row, weighted
+      same = fmaf(c, bf16_to_float(h[(size_t)t * W + n0 + n]), same);
+      continue;
+    }
+    float dot = 0.f;
+    for (int q = 0; q < 2 * pieces; ++q) dot += sums[((size_t)ts * 2 * pieces + q) * 8 + n];
+    total = fmaf(c, dot, total);
+  }
+  total += same;
+  if (add) total += before;
+  if (s_pieces > 0) {
+    float dot = 0.f;
+    for (int q = 0; q < 2 * s_pieces; ++q) dot += s_sums[((size_t)t * 2 * s_pieces + q) * 8 + n];
+    total += dot;
+  }
+  out[(size_t)t * W + n0 + n] = total;
+}
+
+// The whole feed-forward of up to 16 tokens: y (work space, bfloat16 [T, top, ff]) and out float32
+// [T, W] (=, add: +=).  gated: gate_up [E, 2 ff, W]; else [E, ff, W] and the plain activation
+// `act`; every expert's matrices pre-tiled.  Ids from n_experts on name no expert: their term is
+// the weight times h[t].  shared_ff > 0: an expert that all tokens share is added, pre-tiled as
+// well, its activations times factor[t * factor_stride] if given, in shared_y [T, shared_ff].
+// Rows and matrices 16-byte aligned.
+extern "C" int zf_moe_few(const void* h, const void* gate_up, const void* down, const int* ids,
+                          const float* weights, void* y, float* out, int T, int W, int ff, int top,
+                          float limit, float alpha, float shift, int add, int gated, int act,
+                          int n_experts, const void* shared_gate_up, const void* shared_down,
+                          void* shared_y, int shared_ff, float s_limit, float s_alpha,
+                          float s_shift, const float* factor, int factor_stride,
+                          hipStream_t stream) {
+  if (T <= 0) return 0;
+  if (T > MOE_FEW_TOKENS || W <= 0 || ff <= 0 || top <= 0 || W % 64 != 0 || ff % 64 != 0 ||
+      T * top > MOE_FEW_PAIRS || n_experts <= 0 || act < 0 || act > 4 || shared_ff < 0 ||
+      shared_ff % 64 != 0 || (shared_ff > 0 && !gated))
+    return -2;
+  const uintptr_t all = (uintptr_t)h | (uintptr_t)gate_up | (uintptr_t)down | (uintptr_t)y |
+                        (uintptr_t)out | (uintptr_t)shared_gate_up | (uintptr_t)shared_down |
+                        (uintptr_t)shared_y;
+  if (all % 16 != 0) return -2;
+  const dim3 up_grid(shared_ff / 16 + T * top * (ff / 16));
+#define MOE_FEW_UP(G)                                                                             \
+  hipLaunchKernelGGL(moe_few_up_kernel<G>, up_grid, dim3(256), 0, stream, (const bf16_t*)h,       \
+                     (const bf16_t*)gate_up, ids, (bf16_t*)y, T, W, ff, top, limit, alpha, shift, \
+                     act, n_experts, (const bf16_t*)shared_gate_up, (bf16_t*)shared_y, shared_ff, \
+                     s_limit, s_alpha, s_shift, factor, factor_stride)
+  if (gated) MOE_FEW_UP(true); else MOE_FEW_UP(false);
+#undef MOE_FEW_UP
+  // pieces of 2 x 128 of ff, larger ones where the partials of 16 tokens would not fit 48 KB of
+  // LDS (by the layer's sizes alone: a token's sums must not depend on how many tokens there are)
+  int piece = 2;
+  const auto pieces = [](int width, int p) { return (width / 64 + 2 * p - 1) / (2 * p); };
+  const auto lds = [&](int tokens, int p) {
+    return (size_t)tokens * (top * pieces(ff, p) + pieces(shared_ff, p)) * 64;
+  };
+  while (lds(MOE_FEW_TOKENS, piece) > 48 * 1024 && piece < (ff + shared_ff) / 64) piece *= 2;
+  if (lds(T, piece) > 48 * 1024) return -2;
+  hipLaunchKernelGGL(moe_few_down_kernel, dim3(W / 8), dim3(1024), lds(T, piece), stream,
+                     (const bf16_t*)y, (const bf16_t*)down, ids, weights, out, T, W, ff, top, add,
+                     n_experts, (const bf16_t*)h, piece, (const bf16_t*)shared_down,
+                     (const bf16_t*)shared_y, shared_ff);
+  ZF_CHECK_LAUNCH();
+}
+
+// =====================================================================================
 //  Many tokens (bfloat16): the (token, slot) pairs are sorted by expert, and every expert's
 //  pairs run through MFMA tiles of 128 pairs against that expert's matrices.
 //
@@ -618,9 +1244,7 @@ extern "C" int zf_moe_sort(const int* ids, int P, int E, int* sorted, int* place
   ZF_CHECK_LAUNCH();
 }
 
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 moe_bf16x8_t;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float moe_f32x16_t;
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t moe_u32x4_t;
 
 #define MOE_BK 64
 #define MOE_LD (MOE_BK + 8)      // row stride in LDS (bfloat16): 16-byte reads of 8 lanes cover all banks
@@ -638,7 +1262,8 @@ typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t moe_u32x
 #define MOE_HALF (MOE_NB / 2)
 // MODE 0: the down pass; 1: gate and up with the gated activation; 2: up alone, w [E, N, K], with
 // the plain activation `act`.
-template <int MODE>
+// TILED: every expert's matrices pre-tiled (K a multiple of 64, their rows of 16).
+template <int MODE, bool TILED>
 __global__ __launch_bounds__(256) void moe_grouped_kernel(
     const bf16_t* __restrict__ a, long long lda, const int* __restrict__ sorted, int top,
     const bf16_t* __restrict__ w, const int* __restrict__ tile_expert,
@@ -662,6 +1287,11 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
   // what this thread stages: rows tid / 8 + 32 i of the pairs' tile (i < 4) and of the
   // weight tiles (i < 2 MOE_NB), 8 values at k0 + 8 (tid % 8)
   const int sr = tid / 8, sk = (tid % 8) * 8;
+  // of pre-tiled matrices ([rows / 16][K / 64][2][64][8]; MOE_BK = 64: a step is one block of 64)
+  // consecutive threads take consecutive memory: piece p = tid + 256 i is lane p % 64 of half
+  // (p / 64) % 2 of row group p / 128, i.e. row 16 (p / 128) + p % 16 at k 16 (p % 64 / 16) + 8
+  // half (through the row mapping above the same loads scattered 16-byte pieces: 5 to 10 % of
+  // the kernel's time)
   const bf16_t* ap[4];
   const bf16_t* bp[2 * MOE_NB];
 #pragma unroll
@@ -675,7 +1305,7 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
   }
 #pragma unroll
   for (int i = 0; i < 2 * MOE_NB; ++i) {
-    const int r = sr + 32 * i;
+    const int r = TILED ? 16 * ((tid + 256 * i) / 128) + tid % 16 : sr + 32 * i;
     const int br = r % 64, bt = r / 64;              // row br of weight tile bt
     size_t wrow;
     bool ok;
@@ -688,7 +1318,8 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
       ok = n < N;
       wrow = (size_t)e * N + n;
     }
-    bp[i] = ok ? w + wrow * K : nullptr;
+    bp[i] = !ok ? nullptr
+        : TILED ? w + wrow / 16 * (K / 64) * 1024 + tid % 128 * 8 : w + wrow * K + sk;
   }
   moe_f32x16_t acc[2][MOE_NB];
 #pragma unroll
@@ -707,7 +1338,8 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
       ra[i] = (ap[i] != nullptr && in_k) ? *(const moe_u32x4_t*)(ap[i] + k0 + sk) : zero;
 #pragma unroll
     for (int i = 0; i < 2 * MOE_NB; ++i)
-      rb[i] = (bp[i] != nullptr && in_k) ? *(const moe_u32x4_t*)(bp[i] + k0 + sk) : zero;
+      rb[i] = (bp[i] != nullptr && (TILED || in_k))
+          ? *(const moe_u32x4_t*)(bp[i] + (TILED ? (size_t)k0 * 16 : (size_t)k0)) : zero;
   };
   fetch(0);
   for (int k0 = 0; k0 < K; k0 += MOE_BK) {
@@ -715,7 +1347,10 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) *(moe_u32x4_t*)(as + (sr + 32 * i) * MOE_LD + sk) = ra[i];
 #pragma unroll
-    for (int i = 0; i < 2 * MOE_NB; ++i) *(moe_u32x4_t*)(bs + (sr + 32 * i) * MOE_LD + sk) = rb[i];
+    for (int i = 0; i < 2 * MOE_NB; ++i)
+      *(moe_u32x4_t*)(bs + (TILED ? (16 * ((tid + 256 * i) / 128) + tid % 16) * MOE_LD +
+                                        tid % 64 / 16 * 16 + tid % 128 / 64 * 8
+                                  : (sr + 32 * i) * MOE_LD + sk)) = rb[i];
     __syncthreads();
     if (k0 + MOE_BK < K) fetch(k0 + MOE_BK);         // in flight while the MFMAs run
 #pragma unroll
@@ -769,19 +1404,26 @@ extern "C" int zf_moe_grouped(const void* a, long long lda, const int* sorted, i
                               const void* w, const int* tile_expert, const int* tile_row0,
                               const int* tile_rows, const int* n_tiles, void* out, int max_tiles,
                               int N, int K, int mode, float limit, float alpha, float shift,
-                              int act, int n_experts, hipStream_t stream) {
+                              int act, int n_experts, int w_tiled, hipStream_t stream) {
   if (max_tiles <= 0) return 0;
-  if (N <= 0 || K <= 0 || K % 8 != 0 || top <= 0 || mode < 0 || mode > 2 || act < 0 || act > 4)
+  if (N <= 0 || K <= 0 || K % 8 != 0 || top <= 0 || mode < 0 || mode > 2 || act < 0 || act > 4 ||
+      (w_tiled && (K % 64 != 0 || N % 16 != 0)))
     return -2;
   max_tiles = (max_tiles + 7) / 8 * 8;
 #define MOE_GROUPED_LAUNCH(MODE, COLS)                                                           \
-  hipLaunchKernelGGL(moe_grouped_kernel<MODE>, dim3(max_tiles, (N + (COLS) - 1) / (COLS)),       \
+  if (w_tiled) MOE_GROUPED_LAUNCH_AS(MODE, true, COLS); else MOE_GROUPED_LAUNCH_AS(MODE, false, COLS)
+#define MOE_GROUPED_LAUNCH_AS(MODE, TILED, COLS)                                                 \
+  hipLaunchKernelGGL((moe_grouped_kernel<MODE, TILED>), dim3(max_tiles, (N + (COLS) - 1) / (COLS)), \
                      dim3(256), 0, stream, (const bf16_t*)a, lda, sorted, top, (const bf16_t*)w, \
                      tile_expert, tile_row0, tile_rows, n_tiles, out, N, K, limit, alpha, shift, \
                      act, n_experts)
-  if (mode == 1) MOE_GROUPED_LAUNCH(1, 64 * MOE_HALF);
-  else if (mode == 2) MOE_GROUPED_LAUNCH(2, 64 * MOE_NB);
-  else MOE_GROUPED_LAUNCH(0, 64 * MOE_NB);
+  if (mode == 1) {
+    MOE_GROUPED_LAUNCH(1, 64 * MOE_HALF);
+  } else if (mode == 2) {
+    MOE_GROUPED_LAUNCH(2, 64 * MOE_NB);
+  } else {
+    MOE_GROUPED_LAUNCH(0, 64 * MOE_NB);
+  }
   ZF_CHECK_LAUNCH();
 }
 

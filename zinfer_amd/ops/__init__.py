@@ -510,6 +510,16 @@ def _workspace(name: str, numel: int, dtype: torch.dtype, device) -> torch.Tenso
     return buf
 
 
+def _zeroed_workspace(name: str, numel: int, device) -> torch.Tensor:
+    """A persistent int32 buffer that is zero when it is made: counters that every kernel using
+    them leaves at zero again."""
+    fresh = _workspaces.get((name, str(device), torch.int32))
+    buf = _workspace(name, numel, torch.int32, device)
+    if buf is not fresh:
+        buf.zero_()
+    return buf
+
+
 # ------------------------------------------------------------------------- matrix product
 _EPI_STORE_BF16, _EPI_STORE_F32, _EPI_ACC_F32, _EPI_SWIGLU = 0, 1, 2, 3
 SKINNY_MAX_M = 64
@@ -1860,10 +1870,15 @@ def moe_route(h: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor
                                 f"{router.dtype}, ids {tuple(ids.shape)}, at most "
                                 f"{MOE_MAX_EXPERTS} experts, scoring {scoring!r}, groups {groups}")
     lib = build.load("moe")
+    ws = counters = None
+    if T <= 64 and E + n_extra <= 128:
+        ws = _workspace("moe_route", 4 * ((E + n_extra + 31) // 32) * 4096, torch.float32, h.device)
+        counters = _zeroed_workspace("moe_route_counters", 4, h.device)
     _check(lib.zf_moe_route(_ptr(h), _dt(h), _ptr(router), _ptr(bias), _ptr(ids), _ptr(weights),
                             T, W, E, top, ROUTER_SCORINGS[scoring], _ptr(correction), int(count),
                             int(keep), int(group_mark), 1 if normalize else 0,
-                            ctypes.c_float(weight_scale), n_extra, _ptr(extra), _stream()),
+                            ctypes.c_float(weight_scale), n_extra, _ptr(extra), _ptr(ws),
+                            _ptr(counters), _stream()),
            "moe_route")
 
 
@@ -1953,7 +1968,8 @@ def gated_act(gate_up: torch.Tensor, out: torch.Tensor, limit: float, alpha: flo
 
 
 MOE_TILE_ROWS = 128           # MOE_TILE_ROWS in moe.hip
-MOE_STREAM_MAX_TOKENS = 16    # up to here every (token, expert) streams its own matrices
+MOE_STREAM_MAX_TOKENS = 16    # up to here the chosen experts' matrices stream
+MOE_FEW_MAX_PAIRS = 256       # MOE_FEW_PAIRS in moe.hip
 
 
 def moe_grouped_covers(h: torch.Tensor, gate_up: torch.Tensor, act: Optional[str] = None) -> bool:
@@ -1964,10 +1980,77 @@ def moe_grouped_covers(h: torch.Tensor, gate_up: torch.Tensor, act: Optional[str
         and gate_up.shape[2] % 8 == 0 and ff % 8 == 0
 
 
+def moe_can_pretile(gate_up: torch.Tensor, down: torch.Tensor) -> bool:
+    """Whether stacked experts' matrices [E, rows, W] and [E, W, ff] can be pre-tiled, expert by
+    expert (``moe_experts(w_tiled=True)``)."""
+    return gate_up.is_cuda and can_pretile(gate_up[0]) and can_pretile(down[0]) \
+        and down.shape[2] % 64 == 0
+
+
+def moe_few_covers(h: torch.Tensor, top: int) -> bool:
+    """Whether ``moe_experts`` takes pre-tiled matrices through the kernels for few tokens: up to
+    16 of them, rows 16-byte aligned."""
+    T = h.shape[0]
+    return h.dtype == torch.bfloat16 and 0 < T <= MOE_STREAM_MAX_TOKENS \
+        and T * top <= MOE_FEW_MAX_PAIRS and h.is_contiguous() and h.data_ptr() % 16 == 0
+
+
+@_launches("products")
+def _moe_few(h, gate_up, down, ids, weights, y, out, limit, alpha, shift, add=False,
+             act: Optional[str] = None, n_identity: int = 0, shared=None) -> None:
+    """The form of ``moe_experts`` for up to 16 tokens and pre-tiled matrices (bfloat16; see there
+    and ``moe_few_covers``): every used expert's matrices are read once for all tokens that chose
+    it.  ``shared`` = (gate_up, down, y, limit, alpha, shift, factor): an expert that all tokens
+    use, its two matrices gone through ``pretile_weight`` ([2 ff, W], gate rows above up rows, and
+    [W, ff]), y [T, ff] as work space, its activations times ``factor`` (float32 [T] or a column of
+    a float32 matrix, or None); its output is added to the sum."""
+    _need_gpu(h, gate_up, down, ids, weights, y, out)
+    _i32(ids, "ids")
+    T, W = h.shape
+    E, rows, _ = gate_up.shape
+    ff = rows if act is not None else rows // 2
+    top = ids.shape[1]
+    if not moe_few_covers(h, top) or not moe_can_pretile(gate_up, down) \
+            or gate_up.shape != (E, ff if act is not None else 2 * ff, W) \
+            or down.shape != (E, W, ff) \
+            or ids.shape != (T, top) or weights.shape != (T, top) \
+            or weights.dtype != torch.float32 or y.dtype != torch.bfloat16 \
+            or y.numel() != T * top * ff or out.shape != (T, W) or out.dtype != torch.float32 \
+            or not 0 < E <= E + n_identity <= MOE_MAX_EXPERTS \
+            or (act is not None and act not in ACTIVATIONS):
+        raise KernelUnavailable(f"moe_experts: h {tuple(h.shape)} {h.dtype}, gate_up "
+                                f"{tuple(gate_up.shape)}, down {tuple(down.shape)}, ids "
+                                f"{tuple(ids.shape)}, y {tuple(y.shape)} {y.dtype}")
+    f = ctypes.c_float
+    s_gu = s_down = s_y = factor = None
+    s_ff, s_numbers, stride = 0, (0.0, 0.0, 0.0), 0
+    if shared is not None:
+        s_gu, s_down, s_y, s_limit, s_alpha, s_shift, factor = shared
+        s_numbers = (s_limit, s_alpha, s_shift)
+        _need_gpu(s_gu, s_down, s_y)
+        s_ff = s_y.shape[1]
+        if act is not None or s_y.shape != (T, s_ff) or s_y.dtype != torch.bfloat16 \
+                or s_gu.shape != (2 * s_ff, W) or s_down.shape != (W, s_ff) \
+                or not (can_pretile(s_gu) and can_pretile(s_down)) \
+                or (factor is not None and (not factor.is_cuda or factor.dtype != torch.float32
+                                            or factor.shape != (T,))):
+            raise KernelUnavailable(f"moe_experts: shared expert {tuple(s_gu.shape)}, "
+                                    f"{tuple(s_down.shape)}, y {tuple(s_y.shape)}")
+        stride = int(factor.stride(0)) if factor is not None else 0
+    lib = build.load("moe")
+    _check(lib.zf_moe_few(_ptr(h), _ptr(gate_up), _ptr(down), _ptr(ids), _ptr(weights), _ptr(y),
+                          _ptr(out), T, W, ff, top, f(limit), f(alpha), f(shift), 1 if add else 0,
+                          0 if act is not None else 1, ACTIVATIONS[act] if act is not None else 0,
+                          E, _ptr(s_gu), _ptr(s_down), _ptr(s_y), s_ff, f(s_numbers[0]),
+                          f(s_numbers[1]), f(s_numbers[2]), _ptr(factor), stride, _stream()),
+           "moe_experts (few tokens)")
+
+
 def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids: torch.Tensor,
                 weights: torch.Tensor, y: torch.Tensor, out: torch.Tensor, limit: float,
                 alpha: float, shift: float, add: bool = False,
-                act: Optional[str] = None, n_identity: int = 0) -> None:
+                act: Optional[str] = None, n_identity: int = 0, w_tiled: bool = False,
+                shared=None) -> None:
     """out[t] (=, +=) sum over s of weights[t, s] * expert ids[t, s] applied to h[t]
     (``moe_gate_up`` then ``moe_down``), with ``y`` [T, top, ff] as work space.  A few tokens
     stream each chosen expert's matrices (one workgroup row per token and slot); more tokens,
@@ -1975,11 +2058,20 @@ def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids:
     (``moe_sort``, ``moe_grouped`` twice, ``moe_combine``).  Either way a token's result
     depends on that token alone.  ``act``: experts without a gate (see ``moe_gate_up``).
     ``n_identity``: ids from E up to E + n_identity - 1 name no expert; such a term of the sum is
-    the weight times h[t] itself."""
+    the weight times h[t] itself.  ``w_tiled``: every expert's matrices went through
+    ``pretile_weight`` (``moe_can_pretile``); a few tokens then stream every used expert's
+    matrices once past all tokens that chose it.  ``shared``: an expert that all tokens use, added
+    by the same kernels (with ``w_tiled``, where ``moe_few_covers``; see ``_moe_few``)."""
     T, W = h.shape
-    if T > MOE_STREAM_MAX_TOKENS and moe_grouped_covers(h, gate_up, act):
+    if w_tiled and moe_few_covers(h, ids.shape[1]):
+        _moe_few(h, gate_up, down, ids, weights, y, out, limit, alpha, shift, add, act, n_identity,
+                 shared)
+        return
+    if shared is not None:
+        raise KernelUnavailable("moe_experts: a shared expert rides along where moe_few_covers")
+    if w_tiled or (T > MOE_STREAM_MAX_TOKENS and moe_grouped_covers(h, gate_up, act)):
         moe_grouped(h, gate_up, down, ids, weights, y, out, limit, alpha, shift, add, act,
-                    n_identity)
+                    n_identity, w_tiled)
         return
     moe_gate_up(h, gate_up, ids, y, limit, alpha, shift, act, n_identity)
     moe_down(y, down, ids, weights, out, add=add, identity=h if n_identity else None)
@@ -1987,7 +2079,7 @@ def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids:
 
 @_launches("products")
 def moe_grouped(h, gate_up, down, ids, weights, y, out, limit, alpha, shift, add=False,
-                act: Optional[str] = None, n_identity: int = 0) -> None:
+                act: Optional[str] = None, n_identity: int = 0, w_tiled: bool = False) -> None:
     """The many-token form of ``moe_experts`` (bfloat16; see there)."""
     _need_gpu(h, gate_up, down, ids, weights, y, out)
     _i32(ids, "ids")
@@ -2003,6 +2095,7 @@ def moe_grouped(h, gate_up, down, ids, weights, y, out, limit, alpha, shift, add
             or y.numel() != T * top * ff or not y.is_contiguous() \
             or out.shape != (T, W) or out.dtype != torch.float32 \
             or not 0 < E <= E + n_identity <= MOE_MAX_EXPERTS or not h.is_contiguous() \
+            or (w_tiled and not moe_can_pretile(gate_up, down)) \
             or (act is not None and act not in ACTIVATIONS):
         raise KernelUnavailable(f"moe_grouped: h {tuple(h.shape)} {h.dtype}, gate_up "
                                 f"{tuple(gate_up.shape)}, down {tuple(down.shape)}, ids "
@@ -2027,10 +2120,11 @@ def moe_grouped(h, gate_up, down, ids, weights, y, out, limit, alpha, shift, add
     _check(lib.zf_moe_grouped(_ptr(h), ctypes.c_longlong(W), _ptr(sorted_), top, _ptr(gate_up),
                               _ptr(tile_expert), _ptr(tile_row0), _ptr(tile_rows), _ptr(n_tiles),
                               _ptr(y), max_tiles, ff, W, 2 if act is not None else 1, lim, al, sh,
-                              kind, E, st), "moe_grouped (gate, up)")
+                              kind, E, 1 if w_tiled else 0, st), "moe_grouped (gate, up)")
     _check(lib.zf_moe_grouped(_ptr(y), ctypes.c_longlong(ff), _ptr(sorted_), top, _ptr(down),
                               _ptr(tile_expert), _ptr(tile_row0), _ptr(tile_rows), _ptr(n_tiles),
-                              _ptr(o), max_tiles, W, ff, 0, lim, al, sh, 0, E, st),
+                              _ptr(o), max_tiles, W, ff, 0, lim, al, sh, 0, E, 1 if w_tiled else 0,
+                              st),
            "moe_grouped (down)")
     _check(lib.zf_moe_combine(_ptr(o), _ptr(place), _ptr(weights), _ptr(out), T, W, top,
                               1 if add else 0, _ptr(ids) if n_identity else None, E,

@@ -129,6 +129,12 @@ class MoeFeedForward(FeedForward):
             if s.correction_name is not None else None
         self.gate_up, self.down = self._stack(
             tensors, [p + s.expert_prefix.format(e) for e in range(s.n_experts)])
+        # bfloat16 matrices whose sizes allow it are re-laid once into the MFMA kernels' own order
+        # (all experts' rows as one matrix: the order is by groups of 16 rows)
+        self.tiled = ops.moe_can_pretile(self.gate_up, self.down)
+        if self.tiled:
+            self.gate_up, self.down = (ops.pretile_weight(m.flatten(0, 1)).view(m.shape)
+                                       for m in (self.gate_up, self.down))
         if s.shared is not None:
             # the expert every token uses is two plain products around the activation
             gu, dn = self._stack(tensors, [p + s.shared_prefix])
@@ -154,18 +160,29 @@ class MoeFeedForward(FeedForward):
         y = step.scratch("moe_act", (T, s.top_k, ex.intermediate_size), dtype)
         if self.plain:
             ops.moe_experts(h, self.gate_up, self.down, ids, share, y, residual, 0.0, 1.0, 0.0,
-                            add=accumulate, act=ex.activation, n_identity=s.n_identity)
-        else:
-            ops.moe_experts(h, self.gate_up, self.down, ids, share, y, residual,
-                            float(ex.limit or 0.0), float(ex.alpha), float(ex.shift),
-                            add=accumulate, n_identity=s.n_identity)
+                            add=accumulate, act=ex.activation, n_identity=s.n_identity,
+                            w_tiled=self.tiled)
+            return
+        numbers = (float(ex.limit or 0.0), float(ex.alpha), float(ex.shift))
         if s.shared is not None:
             sh = s.shared
+            factor = shared_gate[:, 0] if shared_gate is not None else None
+            s_numbers = (float(sh.limit or 0.0), float(sh.alpha), float(sh.shift))
+            ys = step.scratch("moe_shared_act", (T, sh.intermediate_size), dtype)
+            if self.tiled and self.shared_gate_up.tiled and self.shared_down.tiled \
+                    and ops.moe_few_covers(h, s.top_k):
+                # a few tokens: the shared expert rides with the routed ones
+                ops.moe_experts(h, self.gate_up, self.down, ids, share, y, residual, *numbers,
+                                add=accumulate, n_identity=s.n_identity, w_tiled=True,
+                                shared=(self.shared_gate_up.weight, self.shared_down.weight, ys,
+                                        *s_numbers, factor))
+                return
+        ops.moe_experts(h, self.gate_up, self.down, ids, share, y, residual, *numbers,
+                        add=accumulate, n_identity=s.n_identity, w_tiled=self.tiled)
+        if s.shared is not None:
             gu = step.scratch("moe_shared_gate_up", (T, 2 * sh.intermediate_size), dtype)
             self.shared_gate_up.forward(h, gu)
-            ys = step.scratch("moe_shared_act", (T, sh.intermediate_size), dtype)
-            ops.gated_act(gu, ys, float(sh.limit or 0.0), float(sh.alpha), float(sh.shift),
-                          row_factor=shared_gate[:, 0] if shared_gate is not None else None)
+            ops.gated_act(gu, ys, *s_numbers, row_factor=factor)
             self.shared_down.forward(ys, residual, accumulate=True)
 
 
