@@ -641,6 +641,32 @@ def test_paged_attention_mixed_batch(dtype, nH, nKV, hd, page_size, window):
     assert rel_err(got, want) <= tol(dtype)
 
 
+@pytest.mark.parametrize("hd,page_size", [(4, 4), (60, 16), (64, 8), (128, 8), (132, 12), (260, 16),
+                                          (512, 4)])
+@pytest.mark.parametrize("window", [0, 37])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_wave_attention_vector_loads_give_the_same_bits(hd, page_size, window, dtype):
+    """The kernel's 16-byte loads against its element loads (pools one element off their
+    alignment): the same bits, whole pages, part pages and a window that begins inside a group of
+    four rows; and both against the reference."""
+    ops = _ops()
+    nH, nKV, ctx_lens, q_lens = 4, 2, [70, 3, 200, 129], [1, 3, 5, 129]
+    assert not ops.mfma_attention_covers(dtype, nH, nKV, hd, page_size)
+    s = _paged_setup(dtype, nH, nKV, hd, page_size, ctx_lens, q_lens, 3)
+    got, want = _run_attention(s, dtype, nH, nKV, hd, page_size, window, q_lens, ctx_lens)
+    assert rel_err(got, want) <= tol(dtype)
+    d = {k: v.to(DEV) for k, v in s.items() if isinstance(v, torch.Tensor)}
+    for name in ("k_pool", "v_pool"):
+        flat = torch.empty((d[name].numel() + 1,), dtype=dtype, device=DEV)
+        flat[1:] = d[name].reshape(-1)
+        d[name] = flat[1:].view(d[name].shape)
+    other = torch.full_like(got, float("nan"))
+    ops.paged_attention(d["q"], d["k_pool"], d["v_pool"], d["block_table"], d["q_start"],
+                        d["ctx_len"], d["seq_index"], other, 1.0 / math.sqrt(hd), window, nH, nKV,
+                        hd, page_size, max(q_lens), max(ctx_lens), n_single=1)
+    assert torch.equal(other, got)
+
+
 @pytest.mark.parametrize("nH,nKV,hd,page_size,window", [
     (8, 2, 32, 16, 0), (32, 8, 128, 16, 0), (6, 6, 64, 32, 0), (16, 1, 64, 16, 0),
     (9, 3, 256, 16, 0), (8, 2, 64, 16, 37), (4, 4, 128, 48, 300), (36, 4, 32, 16, 0),
