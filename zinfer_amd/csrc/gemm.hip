@@ -134,7 +134,7 @@ typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2_t;
 //     loads in flight during the products.  The largest tile that still gives 256 workgroups.
 // Measured (weights from HBM, us, against the scalar loop of 64 x 64 tiles before): 4 tokens into
 // 1024 outputs over K = 3072 290 -> 13, 6144 x 1024 107 -> 8.2, 151936 x 1024 474 -> 120 (5.2
-// TB/s), 4096 x 12288 1254 -> 64; 256 tokens into 1024 x 3072 350 -> 42, 6144 x 1024 163 -> 47;
+// TB/s), 4096 x 12288 1254 -> 64; 256 tokens into 1024 x 3072 350 -> 29, 6144 x 1024 163 -> 45;
 // 2048 tokens into 24576 x 4096 10925 -> 4071 (101 TFLOP/s; the vendor's product 154).  Up to 64
 // rows the streaming kernel wins or draws (48 tokens: 24576 x 4096 240 us, the tiles at 96: 258).
 static __host__ __device__ __forceinline__ int f32_span(int K) { return (K + 255) / 256 * 32; }
@@ -225,15 +225,19 @@ __global__ __launch_bounds__(F32_SPANS * 64) void gemm_f32_stream_kernel(
   if (m < M) f32_store4<TO, ACC>(C, m, n, N, vec_out, sum);
 }
 
-#define F32_LD 36
-// B x B outputs a workgroup of 2 x 2 waves
-template <typename TO, bool ACC, int B, bool VEC>
+// B x B outputs a workgroup of 2 x 2 waves; ST steps of 32 of K between two barriers: the small
+// tiles have little to multiply in a step, and a barrier with one step's loads in flight takes 0.45
+// us (256 tokens into 1024 outputs over K = 3072, tiles of 32: 42 us with 96 barriers, 29 with 24;
+// 4096 outputs over 1024, tiles of 64: 31.8 -> 28.9 with two steps; with more than 512 of those the
+// LDS that two steps take costs more, 24576 x 4096 at 96 tokens 258 -> 282 us).
+template <typename TO, bool ACC, int B, int ST, bool VEC>
 __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(
     const float* __restrict__ A, const float* __restrict__ W, TO* __restrict__ C, int M, int N,
     int K, int span, bool vec_out) {
   constexpr int F = B / 32, L = B / 32;      // 16-wide fragments a wave and side; loads a thread
-  __shared__ float As[2][B][F32_LD];
-  __shared__ float Ws[2][B][F32_LD];
+  constexpr int LD = 32 * ST + 4;            // (rows 4 words apart modulo the 64 banks)
+  __shared__ __attribute__((aligned(16))) float As[2][B][LD];
+  __shared__ __attribute__((aligned(16))) float Ws[2][B][LD];
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64, r = lane % 16, g = lane / 16;
   const int n0 = blockIdx.x * B, m0 = blockIdx.y * B;
   const int wm = (wave % 2) * (B / 2), wn = (wave / 2) * (B / 2);
@@ -244,59 +248,64 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(
     ap[i] = A + (size_t)min(m0 + lr + 32 * i, M - 1) * K;
     wp[i] = W + (size_t)min(n0 + lr + 32 * i, N - 1) * K;
   }
-  f32x4_t acc[F][F], sum[F][F], ar[L], wr[L];
+  f32x4_t acc[F][F], sum[F][F], ar[ST][L], wr[ST][L];
 #pragma unroll
   for (int i = 0; i < F; ++i)
 #pragma unroll
     for (int j = 0; j < F; ++j) acc[i][j] = sum[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int steps = (K + 31) / 32, per = span / 32;
+  auto fetch = [&](int st) {                         // (steps beyond the last are zeros)
 #pragma unroll
-  for (int i = 0; i < L; ++i) {
-    ar[i] = f32_load4<VEC>(ap[i], lk, K);
-    wr[i] = f32_load4<VEC>(wp[i], lk, K);
-  }
-  int in_span = 0;
-  for (int st = 0; st < steps; ++st) {
-    const int b = st % 2;
-#pragma unroll
-    for (int i = 0; i < L; ++i) {
-      *(f32x4_t*)&As[b][lr + 32 * i][lk] = ar[i];
-      *(f32x4_t*)&Ws[b][lr + 32 * i][lk] = wr[i];
-    }
-    // one barrier a step: the buffer written next was last read before the barrier of this step
-    __syncthreads();
-    if (st + 1 < steps) {
+    for (int s = 0; s < ST; ++s)
 #pragma unroll
       for (int i = 0; i < L; ++i) {
-        ar[i] = f32_load4<VEC>(ap[i], (st + 1) * 32 + lk, K);
-        wr[i] = f32_load4<VEC>(wp[i], (st + 1) * 32 + lk, K);
+        ar[s][i] = f32_load4<VEC>(ap[i], (st + s) * 32 + lk, K);
+        wr[s][i] = f32_load4<VEC>(wp[i], (st + s) * 32 + lk, K);
       }
-    }
+  };
+  fetch(0);
+  int in_span = 0;
+  for (int st = 0; st < steps; st += ST) {
+    const int b = st / ST % 2;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      f32x4_t wf[F], af[F];
+    for (int s = 0; s < ST; ++s)
 #pragma unroll
-      for (int i = 0; i < F; ++i) {
-        wf[i] = *(const f32x4_t*)&Ws[b][wn + 16 * i + r][8 * g + 4 * h];
-        af[i] = *(const f32x4_t*)&As[b][wm + 16 * i + r][8 * g + 4 * h];
+      for (int i = 0; i < L; ++i) {
+        *(f32x4_t*)&As[b][lr + 32 * i][32 * s + lk] = ar[s][i];
+        *(f32x4_t*)&Ws[b][lr + 32 * i][32 * s + lk] = wr[s][i];
       }
+    // one barrier a stage: the buffer written next was last read before the barrier of this one
+    __syncthreads();
+    if (st + ST < steps) fetch(st + ST);
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < ST; ++s) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        f32x4_t wf[F], af[F];
+#pragma unroll
+        for (int i = 0; i < F; ++i) {
+          wf[i] = *(const f32x4_t*)&Ws[b][wn + 16 * i + r][32 * s + 8 * g + 4 * h];
+          af[i] = *(const f32x4_t*)&As[b][wm + 16 * i + r][32 * s + 8 * g + 4 * h];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < F; ++i)
+#pragma unroll
+            for (int j = 0; j < F; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][e], af[j][e], acc[i][j], 0, 0, 0);
+      }
+      // a span ends behind its last step (steps beyond K add zeros to a span that is empty)
+      if (++in_span == per || st + s + 1 == steps) {
+        in_span = 0;
 #pragma unroll
         for (int i = 0; i < F; ++i)
 #pragma unroll
-          for (int j = 0; j < F; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][s], af[j][s], acc[i][j], 0, 0, 0);
-    }
-    if (++in_span == per || st + 1 == steps) {
-      in_span = 0;
-#pragma unroll
-      for (int i = 0; i < F; ++i)
-#pragma unroll
-        for (int j = 0; j < F; ++j) {
-          sum[i][j] += acc[i][j];
-          acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        }
+          for (int j = 0; j < F; ++j) {
+            sum[i][j] += acc[i][j];
+            acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          }
+      }
     }
   }
 #pragma unroll
@@ -316,8 +325,8 @@ static void launch_f32(const float* A, const float* W, TO* C, int M, int N, int 
   hipLaunchKernelGGL((gemm_f32_stream_kernel<TO, ACC, RG, MT, VEC>),                             \
                      dim3((N + 16 * RG - 1) / (16 * RG), (M + 16 * MT - 1) / (16 * MT)),         \
                      dim3(F32_SPANS * 64), 0, stream, A, W, C, M, N, K, span, vec_out)
-#define F32_TILE(B)                                                                              \
-  hipLaunchKernelGGL((gemm_f32_tile_kernel<TO, ACC, B, VEC>), dim3((N + B - 1) / B,              \
+#define F32_TILE(B, ST)                                                                          \
+  hipLaunchKernelGGL((gemm_f32_tile_kernel<TO, ACC, B, ST, VEC>), dim3((N + B - 1) / B,              \
                      (M + B - 1) / B), dim3(256), 0, stream, A, W, C, M, N, K, span, vec_out)
   const auto tiles = [&](int b) { return (long long)((M + b - 1) / b) * ((N + b - 1) / b); };
   if (M <= 16) {
@@ -327,11 +336,13 @@ static void launch_f32(const float* A, const float* W, TO* C, int M, int N, int 
   } else if (M <= 64) {
     F32_STREAM(1, 4);
   } else if (tiles(128) >= 256) {
-    F32_TILE(128);
+    F32_TILE(128, 1);
+  } else if (tiles(64) > 512) {
+    F32_TILE(64, 1);
   } else if (tiles(64) >= 256) {
-    F32_TILE(64);
+    F32_TILE(64, 2);
   } else {
-    F32_TILE(32);
+    F32_TILE(32, 4);
   }
 #undef F32_STREAM
 #undef F32_TILE
