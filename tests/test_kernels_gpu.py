@@ -1193,6 +1193,52 @@ def test_embed_multiplier_and_logit_scale_cap():
         assert rel_err(got, want) <= 1e-6
 
 
+@pytest.mark.parametrize("V", [1, 63, 1023, 1026, 5001, 40000])
+@pytest.mark.parametrize("kind", ["equal", "two levels", "signed zeros", "few", "spread"])
+def test_sample_topk_ties_and_where_the_selection_changes(V, kind):
+    """Which k are drawn from and in which order, where more than 1024 elements tie (the selection
+    over the whole row) and where they do not, at odd widths and k up to the most: larger logits
+    first, the lower id among equals, 0 and -0 equal but for who is among the k."""
+    import numpy as np
+    import zinfer_amd.ops as ops
+    rs = np.random.RandomState(V)
+    if kind == "equal":
+        row = np.full((V,), 0.25, np.float32)
+    elif kind == "two levels":
+        row = np.where(rs.rand(V) < 0.3, np.float32(1.0), np.float32(0.5))
+    elif kind == "signed zeros":
+        row = np.where(rs.rand(V) < 0.5, np.float32(0.0), np.float32(-0.0))
+        row[rs.randint(0, V, 3)] = 0.125
+    elif kind == "few":
+        row = np.full((V,), -np.inf, np.float32)
+        row[rs.randint(0, V, 5)] = rs.rand(5).astype(np.float32)
+    else:
+        row = rs.permutation(V).astype(np.float32) * np.float32(1e-5)
+    bits = row.view(np.uint32).astype(np.int64)
+    key = np.where(bits >> 31, 0xFFFFFFFF - bits, bits + 0x80000000)
+    by_key = np.lexsort((np.arange(V), -key))
+    recs, want = [], []
+    for k in (1, 2, 50, 700, 1024):
+        k = min(k, V)
+        chosen = by_key[:k]
+        chosen = chosen[np.lexsort((chosen, -row[chosen].astype(np.float64)))]
+        p = np.exp(row[chosen].astype(np.float64) - float(row[chosen[0]]))
+        for f in (0.02, 0.5, 0.97):
+            at = int(np.searchsorted(np.cumsum(p), f * p.sum()))
+            # the middle of that element's share: rounding cannot move it to a neighbour
+            u = (np.cumsum(p)[at] - 0.5 * p[at]) / p.sum()
+            recs.append((1.0, 1.0, 0.0, k, u))
+            want.append(int(chosen[at]))
+    n = len(recs)
+    rec = np.zeros((n,), dtype=ops.SAMPLE_ROW_DTYPE)
+    for i, r in enumerate(recs):
+        rec[i] = r
+    lg = torch.from_numpy(np.tile(row, (n, 1))).to(DEV)
+    out = torch.empty((n,), dtype=torch.int32, device=DEV)
+    ops.sample_topk(lg, torch.from_numpy(rec.view(np.uint8).reshape(-1).copy()).to(DEV), out)
+    assert out.cpu().tolist() == want
+
+
 def test_device_sampler_order_vectors():
     """The device's penalties and sampler on the cases in which the order of the reference's
     operations decides the token."""

@@ -50,6 +50,43 @@ struct SampleRow {
   double u;
 };
 
+// One pass of a radix select, by the first wave: the bin (from the top) in which the s_remaining-th
+// largest of the counted keys lies; the prefix takes the bin's 8 bits, s_remaining becomes the rank
+// within the bin.  A lane holds four bins; what lies above its own comes from the lanes behind it.
+__device__ __forceinline__ void narrow(const unsigned* hist, unsigned prefix, int shift,
+                                       unsigned& s_prefix, unsigned& s_remaining) {
+  if (threadIdx.x >= ZF_WAVE) return;
+  const int lane = threadIdx.x;
+  const unsigned want = s_remaining;
+  unsigned h[4], above = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) above += h[i] = hist[4 * lane + i];
+  const unsigned own = above;
+#pragma unroll
+  for (int off = 1; off < ZF_WAVE; off <<= 1) {
+    const unsigned v = __shfl_down(above, off, ZF_WAVE);
+    if (lane + off < ZF_WAVE) above += v;
+  }
+  above -= own;                              // keys in the bins of the lanes behind this one
+  // (all lanes' bins together hold at least `want` keys, so exactly one bin takes it)
+#pragma unroll
+  for (int i = 3; i >= 0; --i) {
+    if (above < want && above + h[i] >= want) {
+      s_prefix = prefix | ((unsigned)(4 * lane + i) << shift);
+      s_remaining = want - above;
+    }
+    above += h[i];
+  }
+}
+
+// A workgroup a row.  Two passes over the row do for the usual k: the first leaves every thread
+// with the largest of its 1/1024 of the row, the k-th largest of those 1024 is a bound that at least
+// k elements reach and, with k elements scattered over the row, few more, and the second collects
+// what reaches it; sorted by (value, id) the first k of these are the answer.  Only where more than
+// 1024 elements reach the bound (k in the hundreds, a row of equal logits) the k-th key is found by
+// a radix select over the whole row and gathered in id order.  What bounds it: one compute unit
+// draws a row of 152 k logits in about 8 us a pass.  Measured (V = 151936, k = 50, 4 rows): 307 us with
+// the radix select alone (six passes, a thread walking the bins), now 29.
 __global__ __launch_bounds__(SMP_THREADS) void sample_topk_kernel(
     const float* __restrict__ logits, const SampleRow* __restrict__ params,
     int* __restrict__ out, int V) {
@@ -65,10 +102,26 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_topk_kernel(
   int k = prm.top_k <= 0 || prm.top_k > V ? V : prm.top_k;
   if (k > SMP_MAX_K) k = SMP_MAX_K;     // the host refuses such rows before launching
 
-  // 1. radix select: the key of the k-th largest element, 8 bits a pass from the top
+  auto each = [&](auto&& f) {                // f(value, id) for the thread's part of the row
+    if (V % 4 == 0 && ((uintptr_t)row & 15) == 0) {
+#pragma unroll 8
+      for (int i = tid; i < V / 4; i += SMP_THREADS) {
+        const float4 v = ((const float4*)row)[i];
+        f(v.x, 4 * i);
+        f(v.y, 4 * i + 1);
+        f(v.z, 4 * i + 2);
+        f(v.w, 4 * i + 3);
+      }
+    } else {
+      for (int i = tid; i < V; i += SMP_THREADS) f(row[i], i);
+    }
+  };
+  if (tid == 0) s_count = 0;
+  uint32_t mine = 0;                         // (no float has the key 0 but a NaN, which none may reach)
+  each([&](float v, int) { mine = max(mine, float_key(v)); });
   if (tid == 0) {
     s_prefix = 0;
-    s_remaining = (unsigned)k;
+    s_remaining = (unsigned)min(k, SMP_THREADS);
   }
   for (int pass = 0; pass < 4; ++pass) {
     const int shift = 24 - 8 * pass;
@@ -76,115 +129,146 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_topk_kernel(
     __syncthreads();
     const unsigned prefix = s_prefix;
     const unsigned mask = pass == 0 ? 0u : (0xffffffffu << (shift + 8));
-    for (int i = tid; i < V; i += SMP_THREADS) {
-      const uint32_t key = float_key(row[i]);
-      if ((key & mask) == prefix) atomicAdd(&hist[(key >> shift) & 0xff], 1u);
-    }
+    if ((mine & mask) == prefix) atomicAdd(&hist[(mine >> shift) & 0xff], 1u);
     __syncthreads();
+    narrow(hist, prefix, shift, s_prefix, s_remaining);
+    __syncthreads();
+  }
+  const uint32_t bound = s_prefix;
+  each([&](float v, int i) {
+    if (float_key(v) >= bound) {
+      const unsigned at = atomicAdd(&s_count, 1u);
+      if (at < SMP_MAX_K) {
+        cval[at] = v;
+        cidx[at] = i;
+      }
+    }
+  });
+  __syncthreads();
+  int found = (int)s_count;
+  __syncthreads();
+  if (found > SMP_MAX_K) {
+    // radix select: the key of the k-th largest element, 8 bits a pass from the top
     if (tid == 0) {
-      unsigned rem = s_remaining;
-      int b = 255;
-      for (; b > 0; --b) {
-        if (hist[b] >= rem) break;
-        rem -= hist[b];
-      }
-      s_prefix = prefix | ((unsigned)b << shift);
-      s_remaining = rem;     // how many elements equal to the final key are still wanted
+      s_prefix = 0;
+      s_remaining = (unsigned)k;
     }
-    __syncthreads();
-  }
-  const uint32_t kth = s_prefix;
-  const unsigned want_equal = s_remaining;
-
-  // 2. gather: everything above the k-th key, then the lowest ids among those equal to it.
-  //    Threads own contiguous index ranges so that the block-wide scans are in id order.
-  const int per = (V + SMP_THREADS - 1) / SMP_THREADS;
-  const int lo = tid * per, hi = min(V, lo + per);
-  unsigned n_gt = 0, n_eq = 0;
-  for (int i = lo; i < hi; ++i) {
-    const uint32_t key = float_key(row[i]);
-    n_gt += key > kth;
-    n_eq += key == kth;
-  }
-  // exclusive scans of n_gt and n_eq over the threads
-  unsigned off_gt, off_eq, total_gt;
-  scan[tid] = n_gt;
-  __syncthreads();
-  for (int d = 1; d < SMP_THREADS; d <<= 1) {
-    const unsigned v = tid >= d ? scan[tid - d] : 0;
-    __syncthreads();
-    scan[tid] += v;
-    __syncthreads();
-  }
-  off_gt = scan[tid] - n_gt;
-  total_gt = scan[SMP_THREADS - 1];
-  __syncthreads();
-  scan[tid] = n_eq;
-  __syncthreads();
-  for (int d = 1; d < SMP_THREADS; d <<= 1) {
-    const unsigned v = tid >= d ? scan[tid - d] : 0;
-    __syncthreads();
-    scan[tid] += v;
-    __syncthreads();
-  }
-  off_eq = scan[tid] - n_eq;
-  __syncthreads();
-  for (int i = lo; i < hi; ++i) {
-    const float v = row[i];
-    const uint32_t key = float_key(v);
-    if (key > kth) {
-      cval[off_gt] = v;
-      cidx[off_gt] = i;
-      ++off_gt;
-    } else if (key == kth) {
-      if (off_eq < want_equal) {
-        cval[total_gt + off_eq] = v;
-        cidx[total_gt + off_eq] = i;
-      }
-      ++off_eq;
-    }
-  }
-  if (tid == 0) s_count = total_gt + want_equal;      // == k
-  __syncthreads();
-  const int n = (int)s_count;
-
-  // 3. sort descending by value, ascending id among equals (bitonic over 1024 slots)
-  for (int i = tid; i < SMP_MAX_K; i += SMP_THREADS)
-    if (i >= n) {
-      cval[i] = -INFINITY;
-      cidx[i] = 0x7fffffff;
-    }
-  __syncthreads();
-  for (int size = 2; size <= SMP_MAX_K; size <<= 1) {
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      const int i = tid;
-      const int jj = i ^ stride;
-      if (jj > i) {
-        const bool up = (i & size) == 0;      // this half ends up in "before" order
-        const float vi = cval[i], vj = cval[jj];
-        const int ii = cidx[i], ij = cidx[jj];
-        const bool i_before_j = vi > vj || (vi == vj && ii < ij);
-        if (i_before_j != up) {
-          cval[i] = vj;
-          cval[jj] = vi;
-          cidx[i] = ij;
-          cidx[jj] = ii;
-        }
+    for (int pass = 0; pass < 4; ++pass) {
+      const int shift = 24 - 8 * pass;
+      if (tid < 256) hist[tid] = 0;
+      __syncthreads();
+      const unsigned prefix = s_prefix;
+      const unsigned mask = pass == 0 ? 0u : (0xffffffffu << (shift + 8));
+      for (int i = tid; i < V; i += SMP_THREADS) {
+        const uint32_t key = float_key(row[i]);
+        if ((key & mask) == prefix) atomicAdd(&hist[(key >> shift) & 0xff], 1u);
       }
       __syncthreads();
+      narrow(hist, prefix, shift, s_prefix, s_remaining);
+      __syncthreads();
     }
-  }
+    const uint32_t kth = s_prefix;
+    const unsigned want_equal = s_remaining;
 
-  // 4. the reference's walk, by one thread: 32-bit exponentials, 64-bit sums
-  if (tid == 0) {
-    const float T = prm.temperature;
-    const float max_scaled = cval[0] / T;
-    double sum = 0.0;
-    for (int i = 0; i < n; ++i) {
-      const float p = expf(cval[i] / T - max_scaled);
-      cval[i] = p;
-      sum += (double)p;
+    // gather: everything above the k-th key, then the lowest ids among those equal to it.
+    //    Threads own contiguous index ranges so that the block-wide scans are in id order.
+    const int per = (V + SMP_THREADS - 1) / SMP_THREADS;
+    const int lo = tid * per, hi = min(V, lo + per);
+    unsigned n_gt = 0, n_eq = 0;
+    for (int i = lo; i < hi; ++i) {
+      const uint32_t key = float_key(row[i]);
+      n_gt += key > kth;
+      n_eq += key == kth;
     }
+    // exclusive scans of n_gt and n_eq over the threads
+    unsigned off_gt, off_eq, total_gt;
+    scan[tid] = n_gt;
+    __syncthreads();
+    for (int d = 1; d < SMP_THREADS; d <<= 1) {
+      const unsigned v = tid >= d ? scan[tid - d] : 0;
+      __syncthreads();
+      scan[tid] += v;
+      __syncthreads();
+    }
+    off_gt = scan[tid] - n_gt;
+    total_gt = scan[SMP_THREADS - 1];
+    __syncthreads();
+    scan[tid] = n_eq;
+    __syncthreads();
+    for (int d = 1; d < SMP_THREADS; d <<= 1) {
+      const unsigned v = tid >= d ? scan[tid - d] : 0;
+      __syncthreads();
+      scan[tid] += v;
+      __syncthreads();
+    }
+    off_eq = scan[tid] - n_eq;
+    __syncthreads();
+    for (int i = lo; i < hi; ++i) {
+      const float v = row[i];
+      const uint32_t key = float_key(v);
+      if (key > kth) {
+        cval[off_gt] = v;
+        cidx[off_gt] = i;
+        ++off_gt;
+      } else if (key == kth) {
+        if (off_eq < want_equal) {
+          cval[total_gt + off_eq] = v;
+          cidx[total_gt + off_eq] = i;
+        }
+        ++off_eq;
+      }
+    }
+    if (tid == 0) s_count = total_gt + want_equal;      // == k
+    __syncthreads();
+  }
+  const int n = min(k, (int)s_count);
+
+  // sorted: larger first, the lower id among equals (bitonic over the next power of two).  `zeros`:
+  // -0 and 0 are equal, as the reference compares; which elements are among the k goes by the
+  // keys, where -0 lies below 0.
+  auto sort = [&](int have, bool zeros) {
+    int slots = ZF_WAVE;
+    while (slots < have) slots <<= 1;
+    if (tid >= have && tid < slots) {
+      cval[tid] = __uint_as_float(0xffffffffu);         // the lowest key
+      cidx[tid] = 0x7fffffff;
+    }
+    __syncthreads();
+    auto key_of = [&](float v) { return float_key(zeros && v == 0.f ? 0.f : v); };
+    for (int size = 2; size <= slots; size <<= 1) {
+      for (int stride = size >> 1; stride > 0; stride >>= 1) {
+        const int i = tid, jj = tid ^ stride;
+        if (jj > i && i < slots) {
+          const bool up = (i & size) == 0;      // this half ends up in "before" order
+          const float vi = cval[i], vj = cval[jj];
+          const int ii = cidx[i], ij = cidx[jj];
+          const uint32_t ki = key_of(vi), kj = key_of(vj);
+          const bool i_before_j = ki > kj || (ki == kj && ii < ij);
+          if (i_before_j != up) {
+            cval[i] = vj;
+            cval[jj] = vi;
+            cidx[i] = ij;
+            cidx[jj] = ii;
+          }
+        }
+        __syncthreads();
+      }
+    }
+  };
+  static_assert(SMP_THREADS == SMP_MAX_K, "a thread an element");
+  if (found <= SMP_MAX_K) sort(found, false);           // (the gather above left exactly the k)
+  const bool low_zero = tid < n && __float_as_uint(cval[tid]) == 0x80000000u;
+  if (__syncthreads_or(low_zero) || found > SMP_MAX_K) sort(n, true);
+
+  // the reference's walk: 32-bit exponentials, then, by one thread, 64-bit sums
+  const float T = prm.temperature, max_scaled = cval[0] / T;
+  __syncthreads();
+  if (tid < n) cval[tid] = expf(cval[tid] / T - max_scaled);
+  __syncthreads();
+  if (tid == 0) {
+    double sum = 0.0;
+#pragma unroll 8
+    for (int i = 0; i < n; ++i) sum += (double)cval[i];
     int result = cidx[0];
     if (sum > 0.0) {
       int keep = n;
