@@ -1653,7 +1653,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
     int N, int K, SkinnyNorm nrm) {
   constexpr int NSS = NORM == NORM_GIVEN ? NW * 4 : NW;
   __shared__ float part[NW][RG * MT][64][4];
-  __shared__ float ssum[NSS][MT][16];
+  __shared__ float ssum[NW][MT][16];
   const float* __restrict__ gain = nrm.gain;
   const float eps = nrm.eps;
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
@@ -1703,19 +1703,80 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
       pre_g = *(const float4*)(nrm.gain_out + n);
     }
   }
-  // the producer's sums of squares per 16 columns: thread (p, j) adds groups p, p + NSS, ...
-  // of token j; the first SQ_PRE of them are asked for here, before the weights
+  // The producer's sums of squares per 16 columns, [groups][16 tokens]: thread (p, j) takes groups p,
+  // p + NSS, ... of token j.  Asked for behind the weights' first loads (in front of them the
+  // addresses of 16 loads a thread, most of them beyond the groups of a narrow row, held the
+  // weights up) and added up in norm_sums, which runs behind the last product.
   constexpr int SQ_PRE = NORM == NORM_GIVEN ? 16 : 1;
   float sqv[SQ_PRE];
-  if (NORM == NORM_GIVEN) {
-    const int j = tid % 16, p = tid / 16;
+  auto norm_ask = [&]() {
+    if constexpr (NORM == NORM_GIVEN) {
+      const int j = tid % 16, p = tid / 16;
 #pragma unroll
-    for (int i = 0; i < SQ_PRE; ++i) {
-      const int gidx = p + i * NSS;
-      sqv[i] = gidx < nrm.sq_groups ? nrm.sq_in[gidx * 16 + j] : 0.f;
+      for (int i = 0; i < SQ_PRE; ++i) {
+        sqv[i] = 0.f;
+        if (i * NSS < nrm.sq_groups)             // (uniform)
+          sqv[i] = nrm.sq_in[min(p + i * NSS, nrm.sq_groups - 1) * 16 + j];
+      }
+    }
+  };
+  auto norm_sums = [&]() {
+    if constexpr (NORM == NORM_GIVEN) {
+      const int j = tid % 16, p = tid / 16;
+      float v = 0.f;
+#pragma unroll
+      for (int i = 0; i < SQ_PRE; ++i) v += p + i * NSS < nrm.sq_groups ? sqv[i] : 0.f;
+      for (int gidx = p + SQ_PRE * NSS; gidx < nrm.sq_groups; gidx += NSS)
+        v += nrm.sq_in[gidx * 16 + j];
+      v += __shfl_xor(v, 16, 64);
+      v += __shfl_xor(v, 32, 64);
+      if (lane < 16) ssum[wave][0][lane] = v;
+    }
+  };
+  // blocks of 64 of K that are this wave's
+  const int cnt = k0 < K ? (K - 1 - k0) / kstride + 1 : 0;
+  bool asked = false;                            // (the same in every wave)
+  if constexpr (WT && NORM != NORM_FOLD && EPI_GLU(EPI) && RG * MT == 2) {
+    // a short K: both blocks of a wave at once (the loop below waits for one before it asks for the
+    // next: 6144 x 1024 with SwiGLU, one token, PAIR_TIMES)
+    if (K <= 2 * kstride) {
+      asked = true;
+      u32x4_t w0[2][RG], w1[2][RG], a0[2][MT], a1[2][MT];
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (u < cnt) {
+          const int kk = k0 + u * kstride;
+#pragma unroll
+          for (int r = 0; r < RG; ++r) {
+            const bf16_t* tile = wrow[r] + (size_t)(kk / 64) * 1024;
+            w0[u][r] = __builtin_nontemporal_load((const u32x4_t*)tile);
+            w1[u][r] = __builtin_nontemporal_load((const u32x4_t*)(tile + 512));
+          }
+#pragma unroll
+          for (int t = 0; t < MT; ++t) {
+            a0[u][t] = tok[t] ? *(const u32x4_t*)(arow[t] + kk + g * 16) : zero;
+            a1[u][t] = tok[t] ? *(const u32x4_t*)(arow[t] + kk + g * 16 + 8) : zero;
+          }
+        }
+      norm_ask();
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (u < cnt) {
+#pragma unroll
+          for (int r = 0; r < RG; ++r)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+              acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  *(bf16x8_t*)&w0[u][r], *(bf16x8_t*)&a0[u][t], acc[r][t], 0, 0, 0);
+              acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  *(bf16x8_t*)&w1[u][r], *(bf16x8_t*)&a1[u][t], acc[r][t], 0, 0, 0);
+            }
+        }
+      k0 = K;
     }
   }
-  if (WT && NORM != NORM_FOLD && (RG * MT == 1 || (RG * MT == 2 && !EPI_GLU(EPI)))) {
+  if constexpr (WT && NORM != NORM_FOLD && (RG * MT == 1 || (RG * MT == 2 && !EPI_GLU(EPI)))) {
+    asked = true;
     // Pre-tiled weights (no bounds checks; K % 64 == 0), up to two MFMA tiles per k-step:
     // batches of UNR k-steps in two register sets, the next batch asked for before the
     // MFMAs of the one that has arrived, so that a wave always has loads in flight.  The
@@ -1726,10 +1787,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
     // plain loop below.)
     constexpr int UNR = RG * MT == 1 ? 4 : 2;
     u32x4_t w0[2][UNR][RG], w1[2][UNR][RG], a0[2][UNR][MT], a1[2][UNR][MT];
-    auto load = [&](auto BUF, int kb) {
+    auto load_some = [&](auto BUF, auto COUNT, int kb) {
       constexpr int B = decltype(BUF)::value;
 #pragma unroll
-      for (int u = 0; u < UNR; ++u) {
+      for (int u = 0; u < decltype(COUNT)::value; ++u) {
         const int kk = kb + u * kstride;
 #pragma unroll
         for (int r = 0; r < RG; ++r) {
@@ -1744,10 +1805,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
         }
       }
     };
-    auto compute = [&](auto BUF) {
+    auto compute_some = [&](auto BUF, auto COUNT) {
       constexpr int B = decltype(BUF)::value;
 #pragma unroll
-      for (int u = 0; u < UNR; ++u)
+      for (int u = 0; u < decltype(COUNT)::value; ++u)
 #pragma unroll
         for (int r = 0; r < RG; ++r)
 #pragma unroll
@@ -1760,11 +1821,52 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
     };
     using B0 = std::integral_constant<int, 0>;
     using B1 = std::integral_constant<int, 1>;
-    const int bstride = UNR * kstride;
-    // whole batches of this wave: k0 + (nb * UNR - 1) * kstride < K
-    const int nb = k0 < K ? ((K - 1 - k0) / kstride + 1) / UNR : 0;
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    using All = std::integral_constant<int, UNR>;
+    auto load = [&](auto BUF, int kb) { load_some(BUF, All{}, kb); };
+    auto compute = [&](auto BUF) { compute_some(BUF, All{}); };
+    // The blocks that make no whole batch come first, in the other register set, with the first
+    // batch behind them: their loads are in flight together (one block after the other behind
+    // the batches waited for each: 1024 outputs over K = 3072 5.7 -> REM_TIMES us).
+    const int nb = cnt / UNR, rem = cnt % UNR;
+    const int bstride = UNR * kstride, k_rem = k0;
+    k0 += rem * kstride;
+    if (rem == 1) load_some(B1{}, One{}, k_rem);
+    if (UNR > 2 && rem >= 2) load_some(B1{}, Two{}, k_rem);
+    u32x4_t x0[RG], x1[RG], y0[MT], y1[MT];          // a third block
+    if (UNR > 3 && rem == 3) {
+      const int kk = k_rem + 2 * kstride;
+#pragma unroll
+      for (int r = 0; r < RG; ++r) {
+        const bf16_t* tile = wrow[r] + (size_t)(kk / 64) * 1024;
+        x0[r] = __builtin_nontemporal_load((const u32x4_t*)tile);
+        x1[r] = __builtin_nontemporal_load((const u32x4_t*)(tile + 512));
+      }
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        y0[t] = tok[t] ? *(const u32x4_t*)(arow[t] + kk + g * 16) : zero;
+        y1[t] = tok[t] ? *(const u32x4_t*)(arow[t] + kk + g * 16 + 8) : zero;
+      }
+    }
+    if (nb > 0) load(B0{}, k0);
+    norm_ask();
+    __builtin_amdgcn_sched_barrier(0);
+    if (rem == 1) compute_some(B1{}, One{});
+    if (UNR > 2 && rem >= 2) compute_some(B1{}, Two{});
+    if (UNR > 3 && rem == 3) {
+#pragma unroll
+      for (int r = 0; r < RG; ++r)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              *(bf16x8_t*)&x0[r], *(bf16x8_t*)&y0[t], acc[r][t], 0, 0, 0);
+          acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              *(bf16x8_t*)&x1[r], *(bf16x8_t*)&y1[t], acc[r][t], 0, 0, 0);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
     if (nb > 0) {
-      load(B0{}, k0);
       int b = 0;
       for (; b + 2 < nb; b += 2) {
         load(B1{}, k0 + (b + 1) * bstride);
@@ -1785,9 +1887,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
       } else {
         compute(B0{});
       }
-      k0 += nb * bstride;
     }
+    k0 = K;
   }
+  if (!asked) norm_ask();
   for (; k0 < K; k0 += kstride) {
     const int k = k0 + g * 16;
     u32x4_t w0[RG], w1[RG];
@@ -1855,24 +1958,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
       if (lane < 16) ssum[wave][t][lane] = v;
     }
   }
-  if (NORM == NORM_GIVEN) {
-    // the producer of the rows left sums of squares per 16 columns: [groups][16 tokens];
-    // thread (p, j) adds groups p, p + NSS, ... of token j, the rest follows in order of p
-    const int j = tid % 16, p = tid / 16;
-    float v = 0.f;
-#pragma unroll
-    for (int i = 0; i < SQ_PRE; ++i) v += sqv[i];
-    for (int gidx = p + SQ_PRE * NSS; gidx < nrm.sq_groups; gidx += NSS)
-      v += nrm.sq_in[gidx * 16 + j];
-    ssum[p][0][j] = v;
-  }
+  norm_sums();
   __syncthreads();
   // the token's 1 / sqrt(mean(x^2) + eps): the partial sums in a fixed order
   auto inv_rms = [&](int t, int j) {
     if (NORM == NORM_NONE) return 1.0f;
     float tot = 0.f;
 #pragma unroll
-    for (int w = 0; w < NSS; ++w) tot += ssum[w][t][j];
+    for (int w = 0; w < NW; ++w) tot += ssum[w][t][j];
     return 1.0f / sqrtf(tot / (float)K + eps);
   };
   if (EPI_GLU(EPI)) {
