@@ -77,6 +77,14 @@ def test_streams_step(dt, S, W):
         assert torch.equal(total.cpu(), x[1])
 
 
+@pytest.mark.parametrize("S,W", [(4, 4), (4, 2048), (3, 4096), (4, 4100), (5, 260), (2, 1028)])
+def test_streams_step_where_the_kernel_changes(S, W):
+    """One thread with columns, whole and ragged last waves, the widest row that one pass covers
+    and the first that it does not, one copy more than it takes."""
+    for dt in DTYPES:
+        test_streams_step(dt, S, W)
+
+
 # ------------------------------------------------------------------------------ rows of a projection
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("H,G,d,dv,rot", [(4, 2, 12, 20, 6), (3, 3, 16, 8, 16), (2, 1, 96, 160, 40),
