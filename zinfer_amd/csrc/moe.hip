@@ -248,7 +248,8 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float moe_f32x4_t;
 //     back at zero when the kernel ends.
 // Measured (bfloat16 h, in a graph, us; before: four tokens a workgroup and rounds of arg-max): W =
 // 2048, 32 experts, 4 a token, 8 tokens 17.0 -> 11.9 (a single workgroup 14.1), 2048 tokens 31 ->
-// 18; W = 4096, 64 experts, 8 a token, 8 tokens 48.8 -> 16.5 (a single workgroup 41).
+// 18; W = 4096, 64 experts, 8 a token, 8 tokens 48.8 -> 16.5 (a single workgroup 41).  In a decode
+// step, without the release fence: 32 rows 11.3 -> 9.8, 33 rows 15.2 -> 12.5.
 #define MOE_ROUTE16_ROWS 128
 #define MOE_ROUTE16_GROUPS 8
 #define MOE_ROUTE16_SPLIT_TILES 4        // up to so many tiles of 16 tokens are split
@@ -256,8 +257,12 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float moe_f32x4_t;
 __device__ __forceinline__ void store_agent(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ float load_agent(const float* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// (two floats side by side, from a multiple of 8 bytes)
+__device__ __forceinline__ void load2_agent(const float* p, float& a, float& b) {
+  const unsigned long long v = __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+  a = __uint_as_float((uint32_t)v);
+  b = __uint_as_float((uint32_t)(v >> 32));
 }
 
 // eight consecutive values of a row as floats; at or beyond k_end they are 0
@@ -471,7 +476,9 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
                             (MOE_ROUTE16_GROUPS * 4) + blockIdx.x % MOE_ROUTE16_GROUPS * 4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) store_agent(p + i, sum[i]);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        // (the stores have reached memory before the count says so; a release fence would write
+        // the whole L2 back, which is what the kernels before this one left there)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
     } else if (wave < 2) {
       take(chunk, wave, sum);
@@ -481,10 +488,9 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
   if constexpr (SPLIT) {
     const int all = chunks * MOE_ROUTE16_GROUPS;
     if (threadIdx.x == 0)
-      arrived = __hip_atomic_fetch_add(counters + tile, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+      arrived = __hip_atomic_fetch_add(counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     if (arrived != all - 1) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     if (threadIdx.x == 0)
       __hip_atomic_store(counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (wave < 2 * chunks) {            // (at most 128 rows: 8 halves of 16, one a wave)
@@ -492,7 +498,7 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
                                 (MOE_ROUTE16_GROUPS * 4);
       float v[MOE_ROUTE16_GROUPS * 4];
 #pragma unroll
-      for (int i = 0; i < MOE_ROUTE16_GROUPS * 4; ++i) v[i] = load_agent(p + i);
+      for (int i = 0; i < MOE_ROUTE16_GROUPS * 4; i += 2) load2_agent(p + i, v[i], v[i + 1]);
       moe_f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int grp = 0; grp < MOE_ROUTE16_GROUPS; ++grp)
