@@ -304,15 +304,15 @@ __device__ __forceinline__ void decode_attend(const u32x4_t (&kf)[4][HD / 32],
       sc[h * 4 + r] = v;
       m = fmaxf(m, v);
     }
-  m = fmaxf(m, __shfl_xor(m, 16, 64));
-  m = fmaxf(m, __shfl_xor(m, 32, 64));
+  m = apart_max<16>(m);
+  m = apart_max<32>(m);
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
     sc[e] = exp2_raw(sc[e] - m);
     l += sc[e];
   }
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = apart_sum<16>(l);
+  l = apart_sum<32>(l);
 #pragma unroll
   for (int hh = 0; hh < 2; ++hh) {     // two MFMAs of 32 keys: groups 2 hh and 2 hh + 1
     u32x4_t pk = u32x4_t{pack_bf16(sc[8 * hh + 0], sc[8 * hh + 1]),
@@ -966,7 +966,7 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(
           tmax = fmaxf(tmax, v);
         }
       }
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64)) * scale_log2e;
+      tmax = apart_max<32>(tmax) * scale_log2e;
       const float m_new = fmaxf(m, tmax);
       // a query whose window lies wholly beyond this tile has no key here yet
       const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
@@ -977,7 +977,7 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(
         st[r] = exp2_raw(fmaf(st[r], scale_log2e, -m_use));
         psum += st[r];
       }
-      psum += __shfl_xor(psum, 32, 64);
+      psum = apart_sum<32>(psum);
       l = l * corr + psum;
       m = m_new;
       if (__any(corr != 1.0f)) {      // after the first tiles the maxima rarely move
@@ -1342,7 +1342,7 @@ __global__ __launch_bounds__(512) void attn_prefill_shared_kernel(
           tmax = fmaxf(tmax, v);
         }
     }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64)) * scale_log2e;
+    tmax = apart_max<32>(tmax) * scale_log2e;
     const float m_new = fmaxf(m, tmax);
     // a query whose window lies wholly beyond this tile has no key here yet
     const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
@@ -1355,7 +1355,7 @@ __global__ __launch_bounds__(512) void attn_prefill_shared_kernel(
         st[h][r] = exp2_raw(fmaf(st[h][r], scale_log2e, -m_use));
         psum += st[h][r];
       }
-    psum += __shfl_xor(psum, 32, 64);
+    psum = apart_sum<32>(psum);
     l = l * corr + psum;
     m = m_new;
     if (__any(corr != 1.0f)) {      // after the first tiles the maxima rarely move

@@ -137,8 +137,8 @@ __global__ __launch_bounds__(DL_CONV_THREADS) void short_conv_kernel(
   }
   // over the lanes of a wave, then over the head's waves in their order
   ss = dl_lanes_sum<16>(ss);
-  ss += __shfl_xor(ss, 16, ZF_WAVE);
-  ss += __shfl_xor(ss, 32, ZF_WAVE);
+  ss = apart_sum<16>(ss);
+  ss = apart_sum<32>(ss);
   const int wave = threadIdx.x / ZF_WAVE, wph = tph / ZF_WAVE;
   if (threadIdx.x % ZF_WAVE == 0) sq[wave] = ss;
   __syncthreads();

@@ -1728,8 +1728,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
       for (int i = 0; i < SQ_PRE; ++i) v += p + i * NSS < nrm.sq_groups ? sqv[i] : 0.f;
       for (int gidx = p + SQ_PRE * NSS; gidx < nrm.sq_groups; gidx += NSS)
         v += nrm.sq_in[gidx * 16 + j];
-      v += __shfl_xor(v, 16, 64);
-      v += __shfl_xor(v, 32, 64);
+      v = apart_sum<16>(v);
+      v = apart_sum<32>(v);
       if (lane < 16) ssum[wave][0][lane] = v;
     }
   };
@@ -1953,8 +1953,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
       float v = ss[t];
-      v += __shfl_xor(v, 16, 64);
-      v += __shfl_xor(v, 32, 64);
+      v = apart_sum<16>(v);
+      v = apart_sum<32>(v);
       if (lane < 16) ssum[wave][t][lane] = v;
     }
   }
@@ -2045,8 +2045,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
     if (EMIT) {
       // the 16 columns of this row group: 4 per lane, lanes l, l + 16, l + 32, l + 48 of a
       // token; every item is a whole wave here (RG * MT * 64 items, NW * 64 threads)
-      sq += __shfl_xor(sq, 16, 64);
-      sq += __shfl_xor(sq, 32, 64);
+      sq = apart_sum<16>(sq);
+      sq = apart_sum<32>(sq);
       if (l < 16) nrm.sq_out[(size_t)(n0 / 16 + r) * 16 + l] = sq;
     }
   }

@@ -1043,7 +1043,7 @@ __global__ __launch_bounds__(256, 2) void masked_attention_wave_kernel(
         cmax = fmaxf(cmax, sc[r]);
       }
     }
-    cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
+    cmax = apart_max<32>(cmax);
     const float m_new = fmaxf(m, cmax);
     // nothing seen yet (and no sink): every weight below is exp(-inf) = 0
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
@@ -1054,7 +1054,7 @@ __global__ __launch_bounds__(256, 2) void masked_attention_wave_kernel(
       sc[r] = mw_exp2(sc[r] - m_use);
       psum += sc[r];
     }
-    psum += __shfl_xor(psum, 32, 64);
+    psum = apart_sum<32>(psum);
     l = l * corr + psum;
     m = m_new;
     if (__any(corr != 1.0f)) {                     // (the maximum of some row moved)

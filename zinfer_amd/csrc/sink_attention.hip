@@ -344,7 +344,7 @@ __global__ __launch_bounds__(256) void tied_attention_mfma_kernel(
         cmax = fmaxf(cmax, sc[r]);
       }
     }
-    cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
+    cmax = apart_max<32>(cmax);
     const float m_new = fmaxf(m, cmax);
     // nothing seen yet (and no silent term): every weight below is exp(-inf) = 0
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
@@ -355,7 +355,7 @@ __global__ __launch_bounds__(256) void tied_attention_mfma_kernel(
       sc[r] = ta_exp2(sc[r] - m_use);
       psum += sc[r];
     }
-    psum += __shfl_xor(psum, 32, 64);
+    psum = apart_sum<32>(psum);
     l = l * corr + psum;
     m = m_new;
     if (__any(corr != 1.0f)) {                     // (the maximum of some row moved)
@@ -585,7 +585,7 @@ __global__ __launch_bounds__(256, 2) void tied_attention_wave_kernel(
         cmax = fmaxf(cmax, sc[r]);
       }
     }
-    cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
+    cmax = apart_max<32>(cmax);
     const float m_new = fmaxf(m, cmax);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     const float corr = ta_exp2(m - m_use);
@@ -595,7 +595,7 @@ __global__ __launch_bounds__(256, 2) void tied_attention_wave_kernel(
       sc[r] = ta_exp2(sc[r] - m_use);
       psum += sc[r];
     }
-    psum += __shfl_xor(psum, 32, 64);
+    psum = apart_sum<32>(psum);
     l = l * corr + psum;
     m = m_new;
     if (__any(corr != 1.0f)) {

@@ -39,6 +39,64 @@ template <> __device__ __forceinline__ void store_from_float<bf16_t>(bf16_t* p, 
   *p = float_to_bf16(v);
 }
 
+// The value of lane (l xor OFF), for the steps of a sum or maximum over N neighbouring lanes that go
+// from OFF = N / 2 down to 1.  Register moves instead of the shuffles' way through LDS (about 60
+// cycles a step, six steps a wave).  OFF 4 takes lane (l - 4) mod 16 of the row, which is lane
+// l xor 4 or l xor 12: the same value behind a step of 8, so only where there was one.
+template <int CTRL>
+__device__ __forceinline__ float lane_move(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL,
+                                                    0xf, 0xf, true));
+}
+template <int OFF, int N>
+__device__ __forceinline__ float lane_partner(float v) {
+  static_assert(OFF == 1 || OFF == 2 || OFF == 4 || OFF == 8, "within a row of 16 lanes");
+  if constexpr (OFF == 1) return lane_move<0xB1>(v);           // quad_perm [1, 0, 3, 2]
+  else if constexpr (OFF == 2) return lane_move<0x4E>(v);      // quad_perm [2, 3, 0, 1]
+  else if constexpr (OFF == 8) return lane_move<0x128>(v);     // row_ror 8
+  else if constexpr (N > 8) return lane_move<0x124>(v);        // row_ror 4
+  else return __shfl_xor(v, 4, ZF_WAVE);
+}
+// f of the values of lanes l and l xor OFF, OFF 32 or 16: the two copies that the swap leaves hold the
+// wave's halves (the rows of 16 of each half) lane by lane
+template <int OFF, typename F>
+__device__ __forceinline__ float lanes_apart(float v, F f) {
+  static_assert(OFF == 32 || OFF == 16, "a half or a row");
+  typedef unsigned int lanes_u2 __attribute__((ext_vector_type(2)));
+  const uint32_t u = __float_as_uint(v);
+  const lanes_u2 r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false)
+                               : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return f(__uint_as_float(r.x), __uint_as_float(r.y));
+}
+template <int OFF>
+__device__ __forceinline__ float apart_sum(float v) {
+  return lanes_apart<OFF>(v, [](float a, float b) { return a + b; });
+}
+template <int OFF>
+__device__ __forceinline__ float apart_max(float v) {
+  return lanes_apart<OFF>(v, [](float a, float b) { return fmaxf(a, b); });
+}
+// all N lanes of a group (N a power of two up to 64, all of the wave's lanes active) get f over
+// the group, paired off as lane l with l xor N / 2, then N / 4, .. 1
+template <int N, typename F>
+__device__ __forceinline__ float lanes_reduce(float v, F f) {
+  if constexpr (N >= 64) v = lanes_apart<32>(v, f);
+  if constexpr (N >= 32) v = lanes_apart<16>(v, f);
+  if constexpr (N >= 16) v = f(v, lane_partner<8, N>(v));
+  if constexpr (N >= 8) v = f(v, lane_partner<4, N>(v));
+  if constexpr (N >= 4) v = f(v, lane_partner<2, N>(v));
+  if constexpr (N >= 2) v = f(v, lane_partner<1, N>(v));
+  return v;
+}
+template <int N>
+__device__ __forceinline__ float lanes_sum(float v) {
+  return lanes_reduce<N>(v, [](float a, float b) { return a + b; });
+}
+__device__ __forceinline__ float wave_sum(float v) { return lanes_sum<ZF_WAVE>(v); }
+__device__ __forceinline__ float wave_max(float v) {
+  return lanes_reduce<ZF_WAVE>(v, [](float a, float b) { return fmaxf(a, b); });
+}
+
 // RMSNorm over a head and rotation of its pairs (i, i + hd / 2) for the 8 elements a lane
 // holds: x0 = elements 4 li .. 4 li + 3 of the head, x1 = those hd / 2 further on; LPH lanes
 // side by side hold the head (src/kernel/norm/basic.zig:5-22 and src/kernel/rope/basic.zig:5-30
@@ -97,8 +155,7 @@ __device__ __forceinline__ void head_norm_rotate(float (&x0)[4], float (&x1)[4],
     float ss = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) ss += x0[e] * x0[e] + x1[e] * x1[e];
-#pragma unroll
-    for (int off = LPH / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+    ss = lanes_sum<LPH>(ss);
     const float inv = 1.0f / sqrtf(ss / (float)hd + eps);
     if (active) {
 #pragma unroll
@@ -119,17 +176,6 @@ __device__ __forceinline__ void head_norm_rotate(float (&x0)[4], float (&x1)[4],
   }
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = ZF_WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, ZF_WAVE);
-  return v;
-}
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = ZF_WAVE / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, ZF_WAVE));
-  return v;
-}
-
 // Sum over a block of up to 1024 threads; every thread gets the result.  `red` is LDS for
 // at least 16 floats.  The order of the additions depends only on the block size.
 __device__ __forceinline__ float block_sum(float v, float* red) {
@@ -139,8 +185,16 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   __syncthreads();
   if (lane == 0) red[wave] = v;
   __syncthreads();
+  // (four reads in flight at a time; a wave that is not there repeats the last one's)
   float total = 0.f;
-  for (int w = 0; w < nwaves; ++w) total += red[w];
+  for (int w0 = 0; w0 < nwaves; w0 += 4) {
+    float p[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) p[w] = red[min(w0 + w, nwaves - 1)];
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      if (w0 + w < nwaves) total += p[w];
+  }
   return total;
 }
 
