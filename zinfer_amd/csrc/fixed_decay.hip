@@ -143,11 +143,13 @@ __global__ __launch_bounds__(256) void fixed_decay_walk_kernel(
       }
       // the four columns' sums over the LPC lanes: two exchanges leave a lane with one column
       const bool odd = lane & 1, up = lane & 2;
-      const float a0 = (odd ? p[2] : p[0]) + __shfl_xor(odd ? p[0] : p[2], 1, ZF_WAVE);
-      const float a1 = (odd ? p[3] : p[1]) + __shfl_xor(odd ? p[1] : p[3], 1, ZF_WAVE);
-      float r = (up ? a1 : a0) + __shfl_xor(up ? a0 : a1, 2, ZF_WAVE);
-#pragma unroll
-      for (int m = 4; m < LPC; m <<= 1) r += __shfl_xor(r, m, ZF_WAVE);
+      const float a0 = (odd ? p[2] : p[0]) + lane_xor<1>(odd ? p[0] : p[2]);
+      const float a1 = (odd ? p[3] : p[1]) + lane_xor<1>(odd ? p[1] : p[3]);
+      float r = (up ? a1 : a0) + lane_xor<2>(up ? a0 : a1);
+      if constexpr (LPC > 4) r += lane_xor<4>(r);
+      if constexpr (LPC > 8) r += lane_xor<8>(r);
+      if constexpr (LPC > 16) r = apart_sum<16>(r);
+      if constexpr (LPC > 32) r = apart_sum<32>(r);
       const int mine = (wave * FD_NC + (odd ? 2 : 0) + (up ? 1 : 0)) * CPW + cl;
       if (cg < 4 && v0 + mine < dv)
         out[(size_t)(tc + t) * ((size_t)H * dv) + (size_t)hd * dv + v0 + mine] = r;

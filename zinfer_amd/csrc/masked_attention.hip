@@ -278,7 +278,9 @@ __global__ __launch_bounds__(256) void project_rows_vec8_kernel(
         float ss = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) ss += a[e] * a[e];
-        for (int m = 1; m < lph; m <<= 1) ss += __shfl_xor(ss, m, ZF_WAVE);
+        float sum[1] = {ss};
+        lanes_sum_up(sum, lph);
+        ss = sum[0];
         inv_i = 1.0f / sqrtf(ss / (float)g.hd + g.eps);
       } else if (g.per_head && g.gain != nullptr) {
         inv_i = inv_h[head];

@@ -187,7 +187,6 @@ extern "C" int zf_token_shift_mix(const void* h, int dtype, const float* mu, flo
 #define REC_TC 16          // tokens staged at a time (half of that for more than 128 channels)
 #define REC_MAX_THREADS 256
 #define REC_MAX_LDS 65536
-#define REC_TB 4           // tokens whose partial outputs are summed over the lanes together
 #define REC_STAGE 2        // 8-channel loads a thread has in flight when a chunk comes in
 
 __device__ __forceinline__ float decay_of(float z, int rule, float inv_tau) {
@@ -372,86 +371,66 @@ __global__ __launch_bounds__(REC_MAX_THREADS) void decay_recurrence_kernel(
         u8[0] = u0.x; u8[1] = u0.y; u8[2] = u0.z; u8[3] = u0.w;
         u8[4] = u1.x; u8[5] = u1.y; u8[6] = u1.z; u8[7] = u1.w;
       }
-      // REC_TB tokens at a time, so that their sums over the lanes are in flight together
-      for (int tb = 0; tb < n; tb += REC_TB) {
-        float acc[REC_TB][RV];
+      // A token at a time.  (Four at a time, which the sums through LDS needed to cover their way,
+      // cost the registers of a third of the waves: 16 sequences, 8 heads of 128 x 256, 2048
+      // tokens, the output spans 232 us with sums through LDS, 189 with moved registers and
+      // four tokens, 170 with one; a decode step's launch 12.8, 15.6, 12.2.)
+      for (int t = 0; t < n; ++t) {
+        float acc[RV];
+        float vv[RV];
 #pragma unroll
-        for (int tt = 0; tt < REC_TB; ++tt) {
+        for (int r = 0; r < RV; ++r) vv[r] = vs[t * VB + col + r];
+        const float4* kp = (const float4*)(ks + t * DP + cg * REC_R);
+        const float4* dp = (const float4*)(ds + t * DP + cg * REC_R);
+        const float4 k0 = kp[0], k1 = kp[1], d0 = dp[0], d1 = dp[1];
+        const float k8[REC_R] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
+        const float d8[REC_R] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w};
+        if (MODE == 1) {
 #pragma unroll
-          for (int r = 0; r < RV; ++r) acc[tt][r] = 0.f;
-          const int t = tb + tt;
-          if (t >= n) continue;
-          float vv[RV];
+          for (int r = 0; r < RV; ++r)
 #pragma unroll
-          for (int r = 0; r < RV; ++r) vv[r] = vs[t * VB + col + r];
-          const float4* kp = (const float4*)(ks + t * DP + cg * REC_R);
-          const float4* dp = (const float4*)(ds + t * DP + cg * REC_R);
-          const float4 k0 = kp[0], k1 = kp[1], d0 = dp[0], d1 = dp[1];
-          const float k8[REC_R] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
-          const float d8[REC_R] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w};
-          if (MODE == 1) {
+            for (int j = 0; j < REC_R; ++j) S[r][j] = fmaf(d8[j], S[r][j], k8[j] * vv[r]);
+          continue;
+        }
+        const float4* qp = (const float4*)(qs + t * DP + cg * REC_R);
+        const float4 q0 = qp[0], q1 = qp[1];
+        const float q8[REC_R] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
 #pragma unroll
-            for (int r = 0; r < RV; ++r)
+        for (int r = 0; r < RV; ++r) {
+          float a = 0.f;
+          if (BEFORE) {
 #pragma unroll
-              for (int j = 0; j < REC_R; ++j) S[r][j] = fmaf(d8[j], S[r][j], k8[j] * vv[r]);
-            continue;
+            for (int j = 0; j < REC_R; ++j) {
+              const float kv = k8[j] * vv[r];
+              a = fmaf(q8[j], fmaf(u8[j], kv, S[r][j]), a);
+              S[r][j] = fmaf(d8[j], S[r][j], kv);
+            }
+          } else {
+#pragma unroll
+            for (int j = 0; j < REC_R; ++j) {
+              S[r][j] = fmaf(d8[j], S[r][j], k8[j] * vv[r]);
+              a = fmaf(q8[j], S[r][j], a);
+            }
           }
-          const float4* qp = (const float4*)(qs + t * DP + cg * REC_R);
-          const float4 q0 = qp[0], q1 = qp[1];
-          const float q8[REC_R] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-#pragma unroll
-          for (int r = 0; r < RV; ++r) {
-            float a = 0.f;
-            if (BEFORE) {
-#pragma unroll
-              for (int j = 0; j < REC_R; ++j) {
-                const float kv = k8[j] * vv[r];
-                a = fmaf(q8[j], fmaf(u8[j], kv, S[r][j]), a);
-                S[r][j] = fmaf(d8[j], S[r][j], kv);
-              }
+          acc[r] = a;
+        }
+        if (shuffle) {
+          // CS is a power of two: the CS lanes of a column lie side by side in the wave, and
+          // lane 0 of them stores the sums
+          lanes_sum_up(acc, CS);
+          if (cg == 0) {
+            float* o = out + (size_t)(tc + t) * ((size_t)H * dv) + hd * dv + v0 + col;
+            if (RV == 4 && (dv & 3) == 0) {      // a thread's four columns: all within dv or none
+              if (v0 + col < dv) *(float4*)o = float4{acc[0], acc[1 % RV], acc[2 % RV], acc[3 % RV]};
             } else {
 #pragma unroll
-              for (int j = 0; j < REC_R; ++j) {
-                S[r][j] = fmaf(d8[j], S[r][j], k8[j] * vv[r]);
-                a = fmaf(q8[j], S[r][j], a);
-              }
-            }
-            acc[tt][r] = a;
-          }
-        }
-        if (MODE == 1) continue;
-        if (shuffle) {
-          // CS is a power of two: the CS lanes of a column lie side by side in the wave
-          for (int m = 1; m < CS; m <<= 1) {
-#pragma unroll
-            for (int tt = 0; tt < REC_TB; ++tt)
-#pragma unroll
-              for (int r = 0; r < RV; ++r) acc[tt][r] += __shfl_xor(acc[tt][r], m, ZF_WAVE);
-          }
-          // every lane has the sums: lane tt of a column's lanes stores token tt (lane 0 all of
-          // them where there are fewer lanes than tokens)
-#pragma unroll
-          for (int tt = 0; tt < REC_TB; ++tt) {
-            const int t = tb + tt;
-            if (t < n && cg == (CS >= REC_TB ? tt : 0)) {
-              float* o = out + (size_t)(tc + t) * ((size_t)H * dv) + hd * dv + v0 + col;
-              if (RV == 4 && (dv & 3) == 0) {    // a thread's four columns: all within dv or none
-                if (v0 + col < dv)
-                  *(float4*)o = float4{acc[tt][0], acc[tt][1], acc[tt][2], acc[tt][3]};
-              } else {
-#pragma unroll
-                for (int r = 0; r < RV; ++r)
-                  if (v0 + col + r < dv) o[r] = acc[tt][r];
-              }
+              for (int r = 0; r < RV; ++r)
+                if (v0 + col + r < dv) o[r] = acc[r];
             }
           }
         } else {
 #pragma unroll
-          for (int tt = 0; tt < REC_TB; ++tt)
-            if (tb + tt < n) {
-#pragma unroll
-              for (int r = 0; r < RV; ++r) po[((tb + tt) * VB + col + r) * CSP + cg] = acc[tt][r];
-            }
+          for (int r = 0; r < RV; ++r) po[(t * VB + col + r) * CSP + cg] = acc[r];
         }
       }
     }
@@ -633,7 +612,7 @@ __global__ __launch_bounds__(256) void head_norm_gate_kernel(
   if constexpr (WIDE) {
     ss = block_sum(ss, red);
   } else {
-    for (int m = lph / 2; m > 0; m >>= 1) ss += __shfl_xor(ss, m, ZF_WAVE);
+    ss = lanes_sum_down(ss, lph);
   }
   const float inv = 1.0f / sqrtf(ss / (float)dv + eps);
   const T* gr = g + (size_t)t * g_stride + (size_t)hd * dv;

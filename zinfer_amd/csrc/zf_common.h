@@ -39,23 +39,21 @@ template <> __device__ __forceinline__ void store_from_float<bf16_t>(bf16_t* p, 
   *p = float_to_bf16(v);
 }
 
-// The value of lane (l xor OFF), for the steps of a sum or maximum over N neighbouring lanes that go
-// from OFF = N / 2 down to 1.  Register moves instead of the shuffles' way through LDS (about 60
-// cycles a step, six steps a wave).  OFF 4 takes lane (l - 4) mod 16 of the row, which is lane
-// l xor 4 or l xor 12: the same value behind a step of 8, so only where there was one.
-template <int CTRL>
-__device__ __forceinline__ float lane_move(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL,
-                                                    0xf, 0xf, true));
+// The value of lane l xor OFF, OFF 1, 2, 4 or 8: register moves within a row of 16 lanes instead of a
+// shuffle's way through LDS (about 60 cycles a step).  OFF 4 takes the quads of four lanes with
+// an even number from the quad behind and those with an odd one from the quad before.
+template <int CTRL, int BANKS = 0xf>
+__device__ __forceinline__ float lane_move(float v, float old) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL,
+                                                    0xf, BANKS, BANKS == 0xf));
 }
-template <int OFF, int N>
-__device__ __forceinline__ float lane_partner(float v) {
+template <int OFF>
+__device__ __forceinline__ float lane_xor(float v) {
   static_assert(OFF == 1 || OFF == 2 || OFF == 4 || OFF == 8, "within a row of 16 lanes");
-  if constexpr (OFF == 1) return lane_move<0xB1>(v);           // quad_perm [1, 0, 3, 2]
-  else if constexpr (OFF == 2) return lane_move<0x4E>(v);      // quad_perm [2, 3, 0, 1]
-  else if constexpr (OFF == 8) return lane_move<0x128>(v);     // row_ror 8
-  else if constexpr (N > 8) return lane_move<0x124>(v);        // row_ror 4
-  else return __shfl_xor(v, 4, ZF_WAVE);
+  if constexpr (OFF == 1) return lane_move<0xB1>(v, v);           // quad_perm [1, 0, 3, 2]
+  else if constexpr (OFF == 2) return lane_move<0x4E>(v, v);      // quad_perm [2, 3, 0, 1]
+  else if constexpr (OFF == 8) return lane_move<0x128>(v, v);     // row_ror 8
+  else return lane_move<0x114, 0xA>(v, lane_move<0x104, 0x5>(v, v));   // row_shl 4, row_shr 4
 }
 // f of the values of lanes l and l xor OFF, OFF 32 or 16: the two copies that the swap leaves hold the
 // wave's halves (the rows of 16 of each half) lane by lane
@@ -82,15 +80,44 @@ template <int N, typename F>
 __device__ __forceinline__ float lanes_reduce(float v, F f) {
   if constexpr (N >= 64) v = lanes_apart<32>(v, f);
   if constexpr (N >= 32) v = lanes_apart<16>(v, f);
-  if constexpr (N >= 16) v = f(v, lane_partner<8, N>(v));
-  if constexpr (N >= 8) v = f(v, lane_partner<4, N>(v));
-  if constexpr (N >= 4) v = f(v, lane_partner<2, N>(v));
-  if constexpr (N >= 2) v = f(v, lane_partner<1, N>(v));
+  if constexpr (N >= 16) v = f(v, lane_xor<8>(v));
+  // (behind a step of 8 lane l xor 12 holds what lane l xor 4 does: row_ror 4 is one move)
+  if constexpr (N >= 16) v = f(v, lane_move<0x124>(v, v));
+  else if constexpr (N >= 8) v = f(v, lane_xor<4>(v));
+  if constexpr (N >= 4) v = f(v, lane_xor<2>(v));
+  if constexpr (N >= 2) v = f(v, lane_xor<1>(v));
   return v;
 }
 template <int N>
 __device__ __forceinline__ float lanes_sum(float v) {
   return lanes_reduce<N>(v, [](float a, float b) { return a + b; });
+}
+// Every number of v summed over n neighbouring lanes (a power of two up to 64, the same in the
+// whole wave), paired off the other way: lane l with l xor 1, then 2, .. n / 2.  The lanes of a
+// quad hold the same sum by the time the quads meet, so the mirrors of eight and sixteen lanes do
+// for l xor 4 and 8.
+template <int N>
+__device__ __forceinline__ void lanes_sum_up(float (&v)[N], int n) {
+  auto each = [&](auto f) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = f(v[i]);
+  };
+  if (n > 1) each([](float x) { return x + lane_xor<1>(x); });
+  if (n > 2) each([](float x) { return x + lane_xor<2>(x); });
+  if (n > 4) each([](float x) { return x + lane_move<0x141>(x, x); });      // row_half_mirror
+  if (n > 8) each([](float x) { return x + lane_move<0x140>(x, x); });      // row_mirror
+  if (n > 16) each([](float x) { return apart_sum<16>(x); });
+  if (n > 32) each([](float x) { return apart_sum<32>(x); });
+}
+// lanes_sum for a number of lanes that is known when the kernel runs
+__device__ __forceinline__ float lanes_sum_down(float v, int n) {
+  if (n > 32) v = apart_sum<32>(v);
+  if (n > 16) v = apart_sum<16>(v);
+  if (n > 8) v += lane_xor<8>(v);
+  if (n > 4) v += lane_xor<4>(v);
+  if (n > 2) v += lane_xor<2>(v);
+  if (n > 1) v += lane_xor<1>(v);
+  return v;
 }
 __device__ __forceinline__ float wave_sum(float v) { return lanes_sum<ZF_WAVE>(v); }
 __device__ __forceinline__ float wave_max(float v) {
