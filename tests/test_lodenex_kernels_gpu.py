@@ -46,6 +46,33 @@ def test_activation(dt):
     assert rel_err(want["gelu_tanh"], want["gelu"]) > 2 * tol(torch.float32)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 64, 64), (16, 64, 192), (3, 192, 320), (16, 7168, 2048),
+                                   (17, 128, 64), (4, 8192, 4096)])
+def test_activation_in_the_products_epilogue(M, N, K):
+    """The bits of the product followed by the activation, up to 16 tokens and beyond them."""
+    bf = torch.bfloat16
+    a = _rand((M, K), 3, 1.0, bf).to(DEV)
+    w = ops.pretile_weight(_rand((N, K), 4, 2 * K ** -0.5, bf).to(DEV))
+    for kind in ops.ACTIVATIONS:
+        want, got = (torch.full((M, N), float("nan"), dtype=bf, device=DEV) for _ in range(2))
+        ops.gemm(a, w, want, w_tiled=True)
+        ops.activation(want, want, kind)
+        ops.gemm_activation(a, w, got, kind, w_tiled=True)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), kind
+
+
+def test_activation_of_many_values():
+    """Eight values a thread from 2^20 values on: the bits of the same rows taken one by one."""
+    x = _rand((129, 8192), 5, 3.0, torch.bfloat16).to(DEV)
+    x[3, :4] = torch.tensor([float("inf"), float("-inf"), float("nan"), -0.0])
+    for kind in ops.ACTIVATIONS:
+        got, want = torch.empty_like(x), torch.empty_like(x)
+        ops.activation(x, got, kind)
+        for i in range(x.shape[0]):
+            ops.activation(x[i:i + 1], want[i:i + 1], kind)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), kind
+
+
 @pytest.mark.parametrize("T, W", [(1, 48), (7, 336), (3, 4096), (2, 8192)])
 @pytest.mark.parametrize("dt", DTYPES)
 def test_norm_add_store(T, W, dt):

@@ -2187,6 +2187,30 @@ def activation(x: torch.Tensor, out: torch.Tensor, kind: str) -> None:
                              ACTIVATIONS[kind], _stream()), "activation")
 
 
+def gemm_activation(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str,
+                    w_tiled: bool = False) -> None:
+    """``gemm`` and then ``activation`` over ``out`` in place, the same bits; up to 16 tokens on a
+    pre-tiled matrix in one kernel."""
+    M, K = a.shape
+    N = w.shape[0]
+    if w_tiled and 0 < M <= 16 and out.dtype == a.dtype == torch.bfloat16 and kind in ACTIVATIONS \
+            and w.shape[1] == K and out.shape == (M, N) and can_pretile(w):
+        rg, ks = _skinny_plan(M, N, K, True)
+        if ks == 1:
+            _gemm_act(a, w, out, kind, rg)
+            return
+    gemm(a, w, out, w_tiled=w_tiled)
+    activation(out, out, kind)
+
+
+@_launches("products")
+def _gemm_act(a, w, out, kind: str, rg: int) -> None:
+    _need_gpu(a, w, out)
+    M, K = a.shape
+    _check(build.load("gemm").zf_gemm_bf16_act(_ptr(a), _ptr(w), _ptr(out), M, w.shape[0], K, rg,
+                                               ACTIVATIONS[kind], _stream()), "gemm_activation")
+
+
 @_launches("norm_rope_write")
 def bias_act_rows(x: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, kind: str,
                   tail: int = 0, ones: int = 0) -> None:

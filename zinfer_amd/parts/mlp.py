@@ -112,10 +112,10 @@ class DenseMlp(FeedForward):
         if hasattr(h, "materialize"):
             h = h.materialize()
         a = step.scratch("ff_act", (h.shape[0], self.spec.intermediate_size), self.ctx.act_dtype)
-        self.up.forward(h, a)
         if self.up_bias is None:
-            ops.activation(a, a, self.spec.activation)
+            ops.gemm_activation(h, self.up.weight, a, self.spec.activation, self.up.tiled)
         else:
+            self.up.forward(h, a)
             ops.bias_act_rows(a, self.up_bias, a, self.spec.activation)
         self.down.forward(a, residual, accumulate=accumulate,
                           step=step if accumulate and self.down_bias is None else None)
