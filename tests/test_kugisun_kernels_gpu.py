@@ -207,6 +207,31 @@ def test_short_convolutions_over_two_steps(dt, taps, heads, hd, plain):
     assert torch.equal(torch.stack(got), whole.cpu())
 
 
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("taps,heads,hd,plain", [(4, 6, 8, 16), (4, 3, 64, 8), (2, 5, 128, 136),
+                                                 (8, 2, 256, 24), (4, 2, 96, 8)])
+def test_short_convolutions_of_heads_in_pieces(dt, taps, heads, hd, plain):
+    """Rows that allow 16-byte pieces: a head is a lane, a few or half a wave or all of it (96 keeps
+    the other kernel); a whole portion and token by token give the same bits."""
+    C, T = heads * hd + plain, 19
+    K, rows = _rand((C, taps), 21, 0.7).to(DEV), _rand((T, C), 30, 1.0, dt)
+    outs = []
+    for parts in ([T], [1] * T):
+        state = torch.zeros((1, (taps - 1) * C), dtype=torch.float32, device=DEV)
+        got, at = [], 0
+        for n in parts:
+            out = torch.empty((n, C), dtype=torch.float32, device=DEV)
+            ops.short_conv(rows[at:at + n].to(DEV), K, state, 0, _i32([0]), _i32([0] * n), _i32([0, n]), out,
+                           unit_heads=heads, head_dim=hd, scaled_heads=heads // 2, scale=hd ** -0.5,
+                           unit_eps=1e-6, single_tokens=n == 1)
+            got.append(out)
+            at += n
+        outs.append(torch.cat(got))
+    want = _conv_reference(rows, K.cpu(), heads, hd, heads // 2, hd ** -0.5)
+    assert rel_err(outs[0], want) < 2e-5
+    assert torch.equal(outs[0], outs[1])
+
+
 # ------------------------------------------------------------------------------ the delta rule
 def _delta_inputs(T, H, KH, d, dv, seed):
     C = 2 * KH * d + H * dv

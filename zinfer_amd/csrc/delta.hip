@@ -154,17 +154,22 @@ __global__ __launch_bounds__(DL_CONV_THREADS) void short_conv_kernel(
   }
 }
 
-// The same where no channel belongs to a head: a thread takes V neighbouring channels (16 bytes of a
-// row) of TT tokens one behind the other and keeps the rows before the token in registers, NT of
-// them with the token's own (n_taps <= NT; the rows further back meet taps of zero).  The same
-// products and sums in the same order as above.  Grid (blocks of TT tokens, blocks of channels).
+// The same in rows of pieces: a thread takes V neighbouring channels (16 bytes of a row) of TT tokens
+// one behind the other and keeps the rows before the token in registers, NT of them with the
+// token's own (n_taps <= NT; the rows further back meet taps of zero).  The same products and
+// sums in the same order as above.  A head that leaves as a unit vector is lph lanes side by side
+// (hd = lph * V, lph a power of two up to 64; a workgroup is one wave, so heads never straddle
+// one): its squares are added over a thread's channels and then over the lanes, whatever the
+// portion.  With a thread a channel that read every row once a tap, 2048 tokens of 4096 channels,
+// half of them in heads of 128, took 87 us, so 25; a decode step's eight tokens 5.3 and 4.8.
+// Grid (blocks of TT tokens, blocks of channels).
 template <typename T, typename TO, int V, int NT>
 __global__ __launch_bounds__(DL_CONV_THREADS) void short_conv_rows_kernel(
     const T* __restrict__ src, long long src_stride, const float* __restrict__ taps, int n_taps,
     const float* __restrict__ bias, float* __restrict__ state, long long state_stride,
     long long state_off, const int* __restrict__ state_slots, const int* __restrict__ seq_index,
     const int* __restrict__ q_start, TO* __restrict__ out, int n_tokens, int C, int TT,
-    int update_state) {
+    int update_state, int unit_heads, int lph, int scaled_heads, float scale, float unit_eps) {
 #pragma clang fp contract(off)
   const int c = (blockIdx.y * blockDim.x + threadIdx.x) * V;
   if (c >= C) return;
@@ -239,6 +244,16 @@ __global__ __launch_bounds__(DL_CONV_THREADS) void short_conv_rows_kernel(
 #pragma unroll
       for (int k = 0; k < NT; ++k) acc[v] = acc[v] + tp[k][v] * w[k][v];
       acc[v] = dl_silu_to<TO>(bias != nullptr ? acc[v] + b[v] : acc[v]);
+    }
+    if (c < unit_heads * lph * V) {
+      float ss = 0.f;
+#pragma unroll
+      for (int v = 0; v < V; ++v) ss += acc[v] * acc[v];
+      ss = lanes_sum_down(ss, lph);
+      float inv = 1.0f / sqrtf(ss + unit_eps);
+      if (c < scaled_heads * lph * V) inv = inv * scale;
+#pragma unroll
+      for (int v = 0; v < V; ++v) acc[v] = acc[v] * inv;
     }
     TO* o = out + (size_t)t * C + c;
     if constexpr (sizeof(TO) == 2) {
@@ -337,7 +352,10 @@ extern "C" int zf_short_conv(const void* src, int dtype, long long src_stride, c
   const dim3 grid(T, head_blocks + (plain + DL_CONV_THREADS - 1) / DL_CONV_THREADS);
   const dim3 sgrid(n_seqs, (C + DL_CONV_THREADS - 1) / DL_CONV_THREADS);
   const int V = dtype == ZF_F32 ? 4 : 8;
-  const bool rows = unit_heads == 0 && C % V == 0 && src_stride % V == 0 && state_stride % 4 == 0 &&
+  // heads of V, 2 V, .. 64 V channels: whole lanes of a wave
+  const int lph = unit_heads > 0 && hd % V == 0 ? hd / V : 0;
+  const bool rows = (unit_heads == 0 || (lph > 0 && lph <= ZF_WAVE && (lph & (lph - 1)) == 0)) &&
+                    C % V == 0 && src_stride % V == 0 && state_stride % 4 == 0 &&
                     state_off % 4 == 0 && (uintptr_t)src % 16 == 0 && (uintptr_t)out % 16 == 0 &&
                     (uintptr_t)taps % 16 == 0 && (uintptr_t)bias % 16 == 0 &&
                     (uintptr_t)state % 16 == 0;
@@ -347,7 +365,8 @@ extern "C" int zf_short_conv(const void* src, int dtype, long long src_stride, c
 #define DL_CONV_ROWS(TT_, TO_, V_, N_)                                                            \
   hipLaunchKernelGGL((short_conv_rows_kernel<TT_, TO_, V_, N_>), rgrid, dim3(threads), 0, stream,\
                      (const TT_*)src, src_stride, taps, n_taps, bias, state, state_stride,       \
-                     state_off, state_slots, seq_index, q_start, (TO_*)out, T, C, TT, single_tokens)
+                     state_off, state_slots, seq_index, q_start, (TO_*)out, T, C, TT, single_tokens, \
+                     unit_heads, lph, scaled_heads, scale, unit_eps)
 #define DL_CONV_LAUNCH(TT_, TO_, V_)                                                              \
   if (rows) {                                                                                    \
     if (n_taps <= 4) DL_CONV_ROWS(TT_, TO_, V_, 4);                                              \
