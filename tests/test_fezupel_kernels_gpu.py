@@ -264,6 +264,25 @@ def test_router_ties_and_what_cannot_be_chosen(E, top, extra, T, scoring):
         assert torch.allclose(more.cpu(), torch.sigmoid(router[E:, 0]).expand(T, extra), atol=1e-6)
 
 
+@pytest.mark.parametrize("T, W, E, extra", [(1, 2048, 32, 0), (16, 2048, 32, 1), (17, 100, 128, 0),
+                                            (64, 4104, 96, 3), (65, 64, 5, 0)])
+def test_router_over_workgroups_gives_the_same_bits(T, W, E, extra):
+    """With work space of its own a router of up to 64 tokens is spread over workgroups; used again
+    and again the space serves other sizes too."""
+    work, got = ops.moe_route_work(DEV), []
+    h, router = _rand((T, W), 1).to(DEV), _rand((E + extra, W), 2, W ** -0.5).to(DEV)
+    for w in (None, work, work):
+        ids = torch.empty((T, 4), dtype=torch.int32, device=DEV)
+        wts = torch.empty((T, 4), dtype=torch.float32, device=DEV)
+        more = torch.empty((T, extra), device=DEV) if extra else None
+        ops.moe_route(h, router, None, ids, wts, scoring="sigmoid", extra=more, work=w)
+        got.append((ids, wts.view(torch.int32), more if extra else ids))
+    assert all(torch.equal(x, y) for other in got[1:] for x, y in zip(got[0], other))
+    assert not work[-4:].any()
+    with pytest.raises(ops.KernelUnavailable):
+        ops.moe_route(h, router, None, ids, wts, scoring="sigmoid", extra=more, work=work[:-4])
+
+
 @pytest.mark.parametrize("T, W, ff, E, top", [(40, 64, 24, 6, 2), (300, 128, 64, 8, 3),
                                                (17, 72, 136, 1, 1), (150, 352, 104, 40, 4),
                                                (260, 64, 8, 3, 3)])

@@ -510,16 +510,6 @@ def _workspace(name: str, numel: int, dtype: torch.dtype, device) -> torch.Tenso
     return buf
 
 
-def _zeroed_workspace(name: str, numel: int, device) -> torch.Tensor:
-    """A persistent int32 buffer that is zero when it is made: counters that every kernel using
-    them leaves at zero again."""
-    fresh = _workspaces.get((name, str(device), torch.int32))
-    buf = _workspace(name, numel, torch.int32, device)
-    if buf is not fresh:
-        buf.zero_()
-    return buf
-
-
 # ------------------------------------------------------------------------- matrix product
 _EPI_STORE_BF16, _EPI_STORE_F32, _EPI_ACC_F32, _EPI_SWIGLU = 0, 1, 2, 3
 SKINNY_MAX_M = 64
@@ -1822,13 +1812,22 @@ MOE_MAX_EXPERTS = 1024
 ROUTER_SCORINGS = {"softmax": 0, "sigmoid": 1, "softmax_all": 2}
 
 
+_MOE_ROUTE_SUMS = 4 * 4 * 4096         # 4 tiles of tokens, 4 chunks of router rows
+
+
+def moe_route_work(device) -> torch.Tensor:
+    """Sums and (at zero) counters for ``moe_route``'s ``work``.  Two calls that overlap must not
+    share one: whoever holds a router holds its own."""
+    return torch.zeros((_MOE_ROUTE_SUMS + 4,), dtype=torch.float32, device=device)
+
+
 @_launches("other")
 def moe_route(h: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor],
               ids: torch.Tensor, weights: torch.Tensor, scoring: str = "softmax",
               correction: Optional[torch.Tensor] = None,
               groups: Optional[Tuple[int, int]] = None, group_mark: int = 2,
               normalize: bool = True, weight_scale: float = 1.0,
-              extra: Optional[torch.Tensor] = None) -> None:
+              extra: Optional[torch.Tensor] = None, work: Optional[torch.Tensor] = None) -> None:
     """Per row of ``h`` [T, W]: z = router h + bias in 32-bit (router float32 [E, W]); ``ids``
     [T, top] int32 receives the ``top`` chosen experts (the lower index wins a tie).
     ``scoring`` "softmax": the largest z are chosen and ``weights`` [T, top] float32 is the
@@ -1840,8 +1839,10 @@ def moe_route(h: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor
     ``group_mark`` 1: a group is marked by its largest choice score alone.  ``normalize`` False:
     the weights are the chosen s themselves; either way times ``weight_scale``.  ``extra``
     float32 [T, n]: the router has n more rows behind its E outputs, which are no experts; the
-    sigmoids of their products with h go there (a gate a token that rides with the router)."""
-    _need_gpu(h, router, bias, ids, weights, correction, extra)
+    sigmoids of their products with h go there (a gate a token that rides with the router).
+    ``work`` (``moe_route_work``, the caller's own, for one call at a time): up to 64 tokens then
+    spread over workgroups, the same numbers."""
+    _need_gpu(h, router, bias, ids, weights, correction, extra, work)
     _i32(ids, "ids")
     T, W = h.shape
     n_extra = 0
@@ -1871,9 +1872,10 @@ def moe_route(h: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor
                                 f"{MOE_MAX_EXPERTS} experts, scoring {scoring!r}, groups {groups}")
     lib = build.load("moe")
     ws = counters = None
-    if T <= 64 and E + n_extra <= 128:
-        ws = _workspace("moe_route", 4 * ((E + n_extra + 31) // 32) * 4096, torch.float32, h.device)
-        counters = _zeroed_workspace("moe_route_counters", 4, h.device)
+    if work is not None:
+        if work.dtype != torch.float32 or work.numel() != _MOE_ROUTE_SUMS + 4:
+            raise KernelUnavailable("moe_route: work is what moe_route_work made")
+        ws, counters = work, work[_MOE_ROUTE_SUMS:]
     _check(lib.zf_moe_route(_ptr(h), _dt(h), _ptr(router), _ptr(bias), _ptr(ids), _ptr(weights),
                             T, W, E, top, ROUTER_SCORINGS[scoring], _ptr(correction), int(count),
                             int(keep), int(group_mark), 1 if normalize else 0,
