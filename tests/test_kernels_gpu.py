@@ -520,6 +520,30 @@ def test_gemm_emit_then_given(M, H, K1, N2, kind):
     assert rel_err(got, want) <= 2.0 ** -7
 
 
+@pytest.mark.parametrize("K", [64, 1088, 4096, 9216])
+def test_the_order_of_a_given_products_norm_sums(K):
+    """The sums of squares a producer left are added in one order, bit for bit: 32 sums a token,
+    the p-th over the groups p, p + 32, ..., then these in order of p."""
+    import numpy as np
+    ops = _ops()
+    M, N, eps = 16, 64, 1e-6
+    rs = np.random.RandomState(K)
+    sq = (rs.rand(K // 16, 16) * np.exp(3 * rs.randn(K // 16, 16))).astype(np.float32)
+    parts = np.zeros((32, 16), np.float32)
+    for g in range(K // 16):
+        parts[g % 32] += sq[g]
+    total = np.zeros((16,), np.float32)
+    for p in range(32):
+        total += parts[p]
+    inv = np.float32(1) / np.sqrt(total / np.float32(K) + np.float32(eps))
+    # one product of 1 a sum: the outputs are the factors themselves
+    xg, w = torch.zeros((M, K), dtype=torch.bfloat16), torch.zeros((N, K), dtype=torch.bfloat16)
+    xg[:, 0] = w[:, 0] = 1.0
+    got = torch.empty((M, N), dtype=torch.float32, device=DEV)
+    ops.gemm_given(xg.to(DEV), torch.from_numpy(sq).to(DEV), eps, ops.pretile_weight(w.to(DEV)), got)
+    assert torch.equal(got.cpu(), torch.from_numpy(inv)[:, None].expand(M, N))
+
+
 @pytest.mark.parametrize("a_dtype", DTYPES)
 def test_gemm_accumulate_and_one_hot(a_dtype):
     """out += a w^T in 32-bit; a one-hot row picks a column of W (the reference's
