@@ -283,6 +283,31 @@ def test_router_over_workgroups_gives_the_same_bits(T, W, E, extra):
         ops.moe_route(h, router, None, ids, wts, scoring="sigmoid", extra=more, work=work[:-4])
 
 
+@pytest.mark.parametrize("W, T, dt", [(512, 1040, torch.bfloat16), (1024, 64, torch.float32),
+                                      (1100, 64, torch.float32), (2048, 64, torch.float32),
+                                      (2048, 16, torch.bfloat16), (4096, 64, torch.float32)])
+def test_router_logits_are_as_close_as_those_of_more_rows(W, T, dt):
+    """The sums of up to 128 router rows against the kernel that takes more of them (a wave a row, a
+    tree over its lanes), on rows whose exact logits are 0: no further off in the mean."""
+    E = 60
+    g = torch.Generator().manual_seed(W)
+    mix = torch.randperm(W, generator=g)
+    x, r = 64 * torch.randn((T, W // 2), generator=g), 64 * torch.randn((E + 69, W // 2), generator=g)
+    h = torch.cat([x, x], 1)[:, mix].to(dt).to(DEV)
+    router = torch.cat([r, -r], 1)[:, mix].contiguous().to(DEV)
+    off = []
+    for extra in (0, 69):                  # (69 more rows: 129, the other kernel)
+        ids = torch.empty((T, E), dtype=torch.int32, device=DEV)
+        wts = torch.empty((T, E), dtype=torch.float32, device=DEV)
+        more = torch.empty((T, extra), device=DEV) if extra else None
+        ops.moe_route(h, router[:E + extra].contiguous(), None, ids, wts, scoring="sigmoid",
+                      normalize=False, extra=more, work=ops.moe_route_work(DEV))
+        z = torch.logit(wts.cpu().double())
+        off.append(float((z ** 2).mean().sqrt()))
+    # (960 sums and more: their root mean square is known to about 2 %)
+    assert off[0] <= 1.04 * off[1], f"root mean square off: {off[0]:.3e}, {off[1]:.3e}"
+
+
 @pytest.mark.parametrize("T, W, ff, E, top", [(40, 64, 24, 6, 2), (300, 128, 64, 8, 3),
                                                (17, 72, 136, 1, 1), (150, 352, 104, 40, 4),
                                                (260, 64, 8, 3, 3)])

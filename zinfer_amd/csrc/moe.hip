@@ -236,7 +236,7 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float moe_f32x4_t;
 
 // Up to 128 router rows, 16 tokens a tile.  The logits are 32-bit MFMAs (16x16x4: rows of the
 // router against the tokens, h widened), K dealt into 64 spans, eight to a group: a group's spans
-// are added in order, then the groups, so a token's logits do not depend on the tokens beside it
+// are added in pairs, then the groups, so a token's logits do not depend on the tokens beside it
 // nor on how many there are.  Then a wave ranks a token's logits all at once: an expert's rank is
 // the number of experts before it (larger, or equal and of a lower index), one pass over a row in
 // LDS instead of a round of twelve lane exchanges for every chosen one.
@@ -292,6 +292,12 @@ __device__ __forceinline__ void route_load8(const T* __restrict__ row, int k, in
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = k + i < k_end ? load_as_float<T>(row + k + i) : 0.f;
   }
+}
+
+// f(0) + .. + f(7), added in pairs
+template <typename F>
+__device__ __forceinline__ moe_f32x4_t sum8(F f) {
+  return ((f(0) + f(1)) + (f(2) + f(3))) + ((f(4) + f(5)) + (f(6) + f(7)));
 }
 
 __device__ __forceinline__ void wave_lds_fence() {
@@ -437,13 +443,18 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
   for (int chunk = c0; chunk < c1; ++chunk) {
     const float *ra = router + (size_t)min(chunk * 32 + r, rows - 1) * W,
                 *rb = router + (size_t)min(chunk * 32 + 16 + r, rows - 1) * W;
-    moe_f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+    moe_f32x4_t lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;                  // of the groups' halves
     for (int grp = SPLIT ? blockIdx.x % MOE_ROUTE16_GROUPS : 0;
          grp < (SPLIT ? (int)blockIdx.x % MOE_ROUTE16_GROUPS + 1 : MOE_ROUTE16_GROUPS);
          grp += WAVES / 8) {
       const int k_begin = ((grp + wave / 8) * 8 + wave % 8) * span, k_end = min(W, k_begin + span);
-      moe_f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll 2
+      // (eight sums side by side, one an element of a lane's eight: sums of few terms, added in
+      // pairs)
+      moe_f32x4_t acc[8][2];
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        acc[i][0] = acc[i][1] = moe_f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll (SPLIT ? 2 : 1)                // (sixteen waves have 128 registers each)
       for (int k0 = k_begin; k0 < k_end; k0 += 32) {
         float x[8], a[8], b[8];
         route_load8<T, VEC>(row, k0 + 8 * g, k_end, x);
@@ -451,21 +462,18 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
         route_load8<float, VEC>(rb, k0 + 8 * g, k_end, b);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], x[i], acc[0], 0, 0, 0);
-          acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[i], x[i], acc[1], 0, 0, 0);
+          acc[i][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], x[i], acc[i][0], 0, 0, 0);
+          acc[i][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[i], x[i], acc[i][1], 0, 0, 0);
         }
       }
-      part[wave][0][lane] = acc[0];
-      part[wave][1][lane] = acc[1];
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+        part[wave][half][lane] = sum8([&](int i) { return acc[i][half]; });
       __syncthreads();
       if (wave < 2) {
-#pragma unroll
-        for (int w8 = 0; w8 < WAVES / 8; ++w8) {
-          moe_f32x4_t z = part[8 * w8][wave][lane];
-#pragma unroll
-          for (int s = 1; s < 8; ++s) z += part[8 * w8 + s][wave][lane];
-          sum += z;
-        }
+        moe_f32x4_t z = sum8([&](int s) { return part[s][wave][lane]; });
+        if constexpr (WAVES > 8) z += sum8([&](int s) { return part[8 + s][wave][lane]; });
+        if (grp < MOE_ROUTE16_GROUPS / 2) lo += z; else hi += z;
       }
       __syncthreads();
     }
@@ -475,13 +483,13 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
         float* p = ws + ((((size_t)tile * chunks + chunk) * 2 + wave) * ZF_WAVE + lane) *
                             (MOE_ROUTE16_GROUPS * 4) + blockIdx.x % MOE_ROUTE16_GROUPS * 4;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) store_agent(p + i, sum[i]);
+        for (int i = 0; i < 4; ++i) store_agent(p + i, lo[i] + hi[i]);
         // (the stores have reached memory before the count says so; a release fence would write
         // the whole L2 back, which is what the kernels before this one left there)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
     } else if (wave < 2) {
-      take(chunk, wave, sum);
+      take(chunk, wave, lo + hi);
     }
   }
   __syncthreads();
@@ -499,11 +507,9 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
       float v[MOE_ROUTE16_GROUPS * 4];
 #pragma unroll
       for (int i = 0; i < MOE_ROUTE16_GROUPS * 4; i += 2) load2_agent(p + i, v[i], v[i + 1]);
-      moe_f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int grp = 0; grp < MOE_ROUTE16_GROUPS; ++grp)
-        sum += moe_f32x4_t{v[4 * grp], v[4 * grp + 1], v[4 * grp + 2], v[4 * grp + 3]};
-      take(wave / 2, wave % 2, sum);
+      take(wave / 2, wave % 2, sum8([&](int grp) {
+        return moe_f32x4_t{v[4 * grp], v[4 * grp + 1], v[4 * grp + 2], v[4 * grp + 3]};
+      }));
     }
     __syncthreads();
   }
