@@ -32,6 +32,7 @@ class Scratch:
         self.device = device
         self._bufs: Dict[str, torch.Tensor] = {}
         self._views: Dict[str, Dict[tuple, torch.Tensor]] = {}   # per buffer: (shape, dtype) -> view
+        self._made: Dict[str, torch.Tensor] = {}
         self.generation = 0            # goes up whenever a buffer moves (captured graphs die)
 
     def get(self, name: str, shape, dtype: torch.dtype) -> torch.Tensor:
@@ -55,6 +56,15 @@ class Scratch:
         view = buf[:n * size].view(dtype).view(*shape)
         self._views[name][key] = view
         return view
+
+    def made(self, name: str, make) -> torch.Tensor:
+        """The buffer that ``make(device)`` gave the first time: for what a kernel finds as the
+        step before left it (counters at zero), which two engines must not share even where
+        they share a model."""
+        buf = self._made.get(name)
+        if buf is None:
+            buf = self._made[name] = make(self.device)
+        return buf
 
 
 _ELEMENT_SIZE = {torch.float32: 4, torch.bfloat16: 2, torch.int32: 4, torch.int64: 8,
@@ -98,6 +108,9 @@ class StepContext:
 
     def scratch(self, name: str, shape, dtype) -> torch.Tensor:
         return self._scratch.get(name, shape, dtype)
+
+    def made(self, name: str, make) -> torch.Tensor:
+        return self._scratch.made(name, make)
 
     def kv_tables(self, group: int) -> KVStepTables:
         return self.kv[group]

@@ -1816,8 +1816,9 @@ _MOE_ROUTE_SUMS = 4 * 4 * 4096         # 4 tiles of tokens, 4 chunks of router r
 
 
 def moe_route_work(device) -> torch.Tensor:
-    """Sums and (at zero) counters for ``moe_route``'s ``work``.  Two calls that overlap must not
-    share one: whoever holds a router holds its own."""
+    """Sums and (at zero) counters for ``moe_route``'s ``work``.  Two calls that may overlap must
+    not share one (a counter would stay off zero for good): an engine, whose launches follow each
+    other, holds its own."""
     return torch.zeros((_MOE_ROUTE_SUMS + 4,), dtype=torch.float32, device=device)
 
 

@@ -123,7 +123,6 @@ class MoeFeedForward(FeedForward):
             router = torch.cat([router, tensors[p + s.shared_prefix + s.shared_gate_name]
                                 .to(torch.float32).reshape(1, -1)], dim=0)
         self.router = place_gain(router, self.ctx)
-        self.route_work = ops.moe_route_work(self.router.device)
         self.router_bias = place_gain(tensors[p + s.router_bias_name], self.ctx) \
             if s.router_bias else None
         self.correction = place_gain(tensors[p + s.correction_name], self.ctx) \
@@ -156,7 +155,7 @@ class MoeFeedForward(FeedForward):
         ops.moe_route(h, self.router, self.router_bias, ids, share, scoring=s.scoring,
                       correction=self.correction, groups=s.groups, group_mark=s.group_mark,
                       normalize=s.normalize, weight_scale=float(s.weight_scale),
-                      extra=shared_gate, work=self.route_work)
+                      extra=shared_gate, work=step.made("moe_route_work", ops.moe_route_work))
         ex = s.expert
         y = step.scratch("moe_act", (T, s.top_k, ex.intermediate_size), dtype)
         if self.plain:
