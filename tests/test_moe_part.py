@@ -1,4 +1,9 @@
 """The mixture's part on the CPU: what it hands to the kernels."""
+import os
+import re
+import subprocess
+
+import pytest
 import torch
 
 from zinfer_amd.config.specs import GatedExpertSpec, MoeSpec
@@ -40,3 +45,39 @@ def test_engines_on_one_model_do_not_share_the_routers_counters(monkeypatch):
     assert first[0] is first[1] and second[0] is second[1]      # (its launches follow each other)
     assert first[0].data_ptr() != second[0].data_ptr()
     assert seen[4] is first[0] and seen[6] is second[0]
+
+
+def _compile_moe(arch, out):
+    from zinfer_amd.ops import build
+    if not os.path.exists("/opt/rocm/bin/hipcc"):
+        pytest.skip("no compiler")
+    flags = [f for f in build.FLAGS if f not in ("-shared", "-fPIC") and "offload-arch" not in f]
+    return subprocess.run(["/opt/rocm/bin/hipcc", f"--offload-arch={arch}", *flags,
+                           "--offload-device-only", "-S", "-I", build.CSRC,
+                           os.path.join(build.CSRC, "moe.hip"), "-o", str(out)],
+                          capture_output=True, text=True)
+
+
+def test_the_routers_hand_over_between_workgroups(tmp_path):
+    """In the code made for gfx950 the workgroups' sums leave past the caches before the count goes
+    up (a wait for the stores), and the one that counts last reads them past the caches, behind
+    the count's return.  For another target the file is refused: there the same source need not
+    come out so."""
+    out = tmp_path / "moe.s"
+    assert _compile_moe("gfx950", out).returncode == 0
+    bodies = re.findall(r"^(_Z18moe_route16_kernelI\wLb[01]ELb1EE\w+):[^\n]*\n(.*?)s_endpgm",
+                        out.read_text(), re.S | re.M)
+    assert len(bodies) == 4
+    for name, body in bodies:
+        code = [line.split(";")[0].strip() for line in body.splitlines()]
+
+        def places(word, *more):
+            return [i for i, c in enumerate(code) if c.startswith(word) and all(m in c for m in more)]
+        count, = places("global_atomic_add")
+        waits = places("s_waitcnt", "vmcnt(0)")
+        stored = [i for i in places("global_store_dword", "sc1") if i < count]
+        read = places("global_load_dwordx2", "sc1")
+        assert len(stored) >= 4 and any(stored[-1] < i < count for i in waits), name
+        assert read and all(any(count < i < r for i in waits) for r in read), name
+    other = _compile_moe("gfx942", out)
+    assert other.returncode != 0 and "written for gfx950's memory" in other.stderr

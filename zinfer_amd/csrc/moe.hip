@@ -250,6 +250,9 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float moe_f32x4_t;
 // 2048, 32 experts, 4 a token, 8 tokens 17.0 -> 11.9 (a single workgroup 14.1), 2048 tokens 31 ->
 // 18; W = 4096, 64 experts, 8 a token, 8 tokens 48.8 -> 16.5 (a single workgroup 41).  In a decode
 // step, without the release fence: 32 rows 11.3 -> 9.8, 33 rows 15.2 -> 12.5.
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "moe_route16_kernel's hand-over between workgroups is written for gfx950's memory"
+#endif
 #define MOE_ROUTE16_ROWS 128
 #define MOE_ROUTE16_GROUPS 8
 #define MOE_ROUTE16_SPLIT_TILES 4        // up to so many tiles of 16 tokens are split
@@ -484,8 +487,10 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
                             (MOE_ROUTE16_GROUPS * 4) + blockIdx.x % MOE_ROUTE16_GROUPS * 4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) store_agent(p + i, lo[i] + hi[i]);
-        // (the stores have reached memory before the count says so; a release fence would write
-        // the whole L2 back, which is what the kernels before this one left there)
+        // The stores have reached memory before the count says so: on gfx950 agent-scope stores go
+        // through the L2 and count down vmcnt once they are there.  (A release fence says the same
+        // in the language's terms, but writes the whole L2 back, which is what the kernels before
+        // this one left there.)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
     } else if (wave < 2) {
@@ -499,6 +504,10 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
       arrived = __hip_atomic_fetch_add(counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     if (arrived != all - 1) return;
+    // The others' sums are read behind the count: agent-scope loads pass the caches here, and none of
+    // them is issued before the count has come back.  (An acquire fence would drop what the caches
+    // hold for it: a decode step's router 10.3 -> 11.1 us.)
+    __atomic_signal_fence(__ATOMIC_ACQUIRE);
     if (threadIdx.x == 0)
       __hip_atomic_store(counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (wave < 2 * chunks) {            // (at most 128 rows: 8 halves of 16, one a wave)
