@@ -308,6 +308,72 @@ def test_router_logits_are_as_close_as_those_of_more_rows(W, T, dt):
     assert off[0] <= 1.04 * off[1], f"root mean square off: {off[0]:.3e}, {off[1]:.3e}"
 
 
+@pytest.mark.parametrize("T, W, E", [(64, 2048, 8), (65, 2048, 8), (256, 1024, 32), (257, 1024, 32),
+                                     (16, 1023, 40), (512, 3072, 20), (513, 3072, 20),
+                                     (1024, 2048, 128), (1025, 520, 128), (1030, 504, 65)])
+@pytest.mark.parametrize("dt", DTYPES)
+def test_router_where_the_kernel_changes(T, W, E, dt):
+    """On both sides of every line at which the router's kernel changes, against 64-bit: the chosen
+    and their weights, twice on the same work space."""
+    h, router = _rand((T, W), 5, dtype=dt), _rand((E, W), 6, W ** -0.5)
+    z = h.double() @ router.double().T
+    work = ops.moe_route_work(DEV)
+    for _ in range(2):
+        ids = torch.empty((T, E), dtype=torch.int32, device=DEV)
+        wts = torch.empty((T, E), dtype=torch.float32, device=DEV)
+        ops.moe_route(h.to(DEV), router.to(DEV), None, ids, wts, work=work)
+        at = ids.cpu().long()
+        assert torch.equal(at.sort(1).values, torch.arange(E).expand(T, E))
+        # logits of about 1 formed from W terms in 32-bit: off by a few 2^-24 of their scale
+        ordered = z.gather(1, at)
+        assert bool((ordered[:, 1:] <= ordered[:, :-1] + 4e-6).all())
+        assert torch.allclose(wts.cpu().double(), torch.softmax(ordered, 1), rtol=8e-6, atol=0)
+        assert not work[-64:].any()
+
+
+def test_router_in_float32_does_not_depend_on_the_number_of_tokens():
+    """A token's bits with 1, 300 and 1100 tokens beside it, in one workgroup and over several."""
+    W, E = 2048, 40
+    h, router = _rand((1100, W), 7).to(DEV), _rand((E, W), 8, W ** -0.5).to(DEV)
+    got = []
+    for T, work in ((1100, None), (1100, ops.moe_route_work(DEV)), (300, ops.moe_route_work(DEV)),
+                    (1, ops.moe_route_work(DEV))):
+        ids = torch.empty((T, 6), dtype=torch.int32, device=DEV)
+        wts = torch.empty((T, 6), dtype=torch.float32, device=DEV)
+        ops.moe_route(h[:T], router, None, ids, wts, work=work)
+        got.append((T, ids, wts))
+    for T, ids, wts in got[1:]:
+        assert torch.equal(ids, got[0][1][:T]) and torch.equal(wts, got[0][2][:T])
+
+
+@pytest.mark.parametrize("T, W", [(16, 64), (256, 256), (1024, 2048)])
+def test_router_of_128_rows_takes_no_longer_than_one_of_129(T, W):
+    """Where the kernel for sixteen tokens a workgroup is the slower one (narrow rows, some hundred
+    tokens; by a third to twice the time) it is not taken."""
+    h, router = _rand((T, W), 9, dtype=torch.bfloat16).to(DEV), _rand((129, W), 10, W ** -0.5).to(DEV)
+    ids = torch.empty((T, 4), dtype=torch.int32, device=DEV)
+    wts = torch.empty((T, 4), dtype=torch.float32, device=DEV)
+    work, best = ops.moe_route_work(DEV), []
+    for rows in (128, 129):
+        r = router[:rows].contiguous()
+        ops.moe_route(h, r, None, ids, wts, work=work)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                ops.moe_route(h, r, None, ids, wts, work=work)
+        times = []
+        for _ in range(12):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            graph.replay()
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        best.append(min(times))
+    assert best[0] <= 1.2 * best[1], f"{best[0] * 50:.1f} us, {best[1] * 50:.1f} us"
+
+
 @pytest.mark.parametrize("T, W, ff, E, top", [(40, 64, 24, 6, 2), (300, 128, 64, 8, 3),
                                                (17, 72, 136, 1, 1), (150, 352, 104, 40, 4),
                                                (260, 64, 8, 3, 3)])

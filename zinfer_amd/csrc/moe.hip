@@ -17,13 +17,15 @@
 // not take); every token's result depends on that token alone and its sums run in a
 // fixed order, so a token gives the same bits whatever else is in the batch:
 //
-//  * moe_route         a workgroup per sixteen tokens (four with more than 128 router rows)
+//  * moe_route         a workgroup per four tokens, or sixteen (route16_takes)
 //  * moe_gate_up       grid (token * slot, groups of outputs): y[t, slot, :] of the expert in
 //                      that slot, the token's row staged in LDS as 32-bit numbers
 //  * moe_down          grid (token, groups of outputs): out[t, n] (=, or += into) the weighted
 //                      sum over the slots in slot order, 32-bit
 //
 // With `ids` null every token uses expert 0 with weight 1 (an expert that all tokens share).
+#include <type_traits>
+
 #include "zf_common.h"
 
 #define MOE_MAX_EXPERTS 1024
@@ -240,22 +242,27 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float moe_f32x4_t;
 // nor on how many there are.  Then a wave ranks a token's logits all at once: an expert's rank is
 // the number of experts before it (larger, or equal and of a lower index), one pass over a row in
 // LDS instead of a round of twelve lane exchanges for every chosen one.
-//   * more than 64 tokens: a workgroup of 16 waves takes a tile, two groups at a time.
-//   * up to 64 (SPLIT): one compute unit draws a router of 256 KB in 8 us, so a workgroup of eight
+//   * many tokens: a workgroup of 16 waves takes a tile, two groups at a time.
+//   * else (SPLIT): one compute unit draws a router of 256 KB in 8 us, so a workgroup of eight
 //     waves takes one group of K and 32 rows of the router, leaves its sums in `ws` and adds one to
 //     the tile's counter; the one that finds the count complete adds the groups and chooses.  Sums
 //     and counter go through to memory (agent scope), where every XCD sees them; the counter is
-//     back at zero when the kernel ends.
-// Measured (bfloat16 h, in a graph, us; before: four tokens a workgroup and rounds of arg-max): W =
-// 2048, 32 experts, 4 a token, 8 tokens 17.0 -> 11.9 (a single workgroup 14.1), 2048 tokens 31 ->
-// 18; W = 4096, 64 experts, 8 a token, 8 tokens 48.8 -> 16.5 (a single workgroup 41).  In a decode
-// step, without the release fence: 32 rows 11.3 -> 9.8, 33 rows 15.2 -> 12.5.
+//     back at zero when the kernel ends.  (Up to 1024 workgroups: with 2048 of them 1024 tokens of
+//     W = 2048 and 128 rows took 86 us, without the split 60.)
+// What it takes is said at route16_takes.  Without a release fence a decode step's 32 rows take 9.8
+// us where they took 11.3, 33 rows 12.5 and 15.2.
 #if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
 #error "moe_route16_kernel's hand-over between workgroups is written for gfx950's memory"
 #endif
 #define MOE_ROUTE16_ROWS 128
 #define MOE_ROUTE16_GROUPS 8
-#define MOE_ROUTE16_SPLIT_TILES 4        // up to so many tiles of 16 tokens are split
+#define MOE_ROUTE16_SPLIT_TILES 64       // up to so many tiles of 16 tokens are split
+
+// numbers of K in a span, and groups that hold any
+static __host__ __device__ __forceinline__ int route16_span(int W) { return (W + 2047) / 2048 * 32; }
+static __host__ __device__ __forceinline__ int route16_groups(int W) {
+  return (W + 8 * route16_span(W) - 1) / (8 * route16_span(W));
+}
 
 __device__ __forceinline__ void store_agent(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -308,15 +315,28 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// how many of row[0 .. n4 * 4) come before (v, e): larger, or equal with a lower index (NaN: none)
+// how many of row[0 .. n4 * 4) come before (v, e): larger, or equal with a lower index (NaN: none).
+// No branches: the lanes of a wave part at every comparison.  BLOCK: e lies in the BLOCK-th 64 for
+// the whole wave (-1: anywhere), so that only numbers of that 64 need their index compared.
+// (Where 16 waves choose among 128, the comparisons are what the kernel spends its time on: 16
+// tokens, W = 64 in 24 us with branches, 20 without, 13 by blocks.)
+template <int BLOCK>
 __device__ __forceinline__ int rank_before(const float* row, int n4, float v, int e) {
   int rank = 0;
-  for (int j = 0; j < n4; ++j) {
-    const float4 o = *(const float4*)(row + 4 * j);
-    const float ov[4] = {o.x, o.y, o.z, o.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) rank += ov[i] > v || (ov[i] == v && 4 * j + i < e);
-  }
+  const int lo = BLOCK < 0 ? 0 : min(n4, 16 * BLOCK), hi = BLOCK < 0 ? n4 : min(n4, 16 * BLOCK + 16);
+  auto each = [&](int from, int to, auto before) {
+#pragma unroll 4
+    for (int j = from; j < to; ++j) {
+      const float4 o = *(const float4*)(row + 4 * j);
+      rank += before(o.x, 4 * j);
+      rank += before(o.y, 4 * j + 1);
+      rank += before(o.z, 4 * j + 2);
+      rank += before(o.w, 4 * j + 3);
+    }
+  };
+  if constexpr (BLOCK > 0) each(0, lo, [&](float o, int) { return (int)(o >= v); });
+  each(lo, hi, [&](float o, int i) { return (int)(o > v) + ((int)(o == v) & (int)(i < e)); });
+  if constexpr (BLOCK >= 0) each(hi, n4, [&](float o, int) { return (int)(o > v); });
   return rank;
 }
 
@@ -366,7 +386,7 @@ __device__ __forceinline__ void route_choose(float* z, float* share, int* chosen
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const int e = lane + ZF_WAVE * i;
-        if (e < E) out[i] = rank_before(mark, g4, mark[e / size], e / size) >= keep_groups;
+        if (e < E) out[i] = rank_before<-1>(mark, g4, mark[e / size], e / size) >= keep_groups;
       }
       wave_lds_fence();
 #pragma unroll
@@ -378,15 +398,14 @@ __device__ __forceinline__ void route_choose(float* z, float* share, int* chosen
   // the chosen in the order of their scores; where nothing but NaN or -inf is left, expert 0
   for (int k = lane; k < top; k += ZF_WAVE) chosen[k] = -1;
   wave_lds_fence();
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int e = lane + ZF_WAVE * i;
+  auto place = [&](auto BLOCK) {
+    const int e = lane + ZF_WAVE * decltype(BLOCK)::value;
     const float v = e < E ? z[e] : -INFINITY;
-    if (v > -INFINITY) {
-      const int rank = rank_before(z, n4, v, e);
-      if (rank < top) chosen[rank] = e;
-    }
-  }
+    const int rank = rank_before<decltype(BLOCK)::value>(z, n4, v, e);
+    if (v > -INFINITY && rank < top) chosen[rank] = e;
+  };
+  place(std::integral_constant<int, 0>{});
+  if (E > ZF_WAVE) place(std::integral_constant<int, 1>{});
   wave_lds_fence();
   if (scoring == 0) {
     const float first = chosen[0] >= 0 ? z[chosen[0]] : -INFINITY;
@@ -426,7 +445,7 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
   const int wave = threadIdx.x / ZF_WAVE, lane = threadIdx.x % ZF_WAVE;
   const int r = lane % 16, g = lane / 16, tile = SPLIT ? blockIdx.y : blockIdx.x, t0 = tile * 16;
   const int rows = E + n_extra, chunks = (rows + 31) / 32;        // 32 rows of the router
-  const int span = (W + 2047) / 2048 * 32;
+  const int span = route16_span(W), groups = route16_groups(W);
   const T* row = h + (size_t)min(t0 + r, n_tokens - 1) * W;
   // column lane % 16 is a token, the four numbers are rows 4 (lane / 16) + i of the 16-row tile
   auto take = [&](int chunk, int half, moe_f32x4_t z) {
@@ -442,14 +461,13 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
       }
     }
   };
-  const int c0 = SPLIT ? blockIdx.x / MOE_ROUTE16_GROUPS : 0, c1 = SPLIT ? c0 + 1 : chunks;
+  const int c0 = SPLIT ? blockIdx.x / groups : 0, c1 = SPLIT ? c0 + 1 : chunks;
+  const int grp0 = SPLIT ? blockIdx.x % groups : 0, grp1 = SPLIT ? grp0 + 1 : groups;
   for (int chunk = c0; chunk < c1; ++chunk) {
     const float *ra = router + (size_t)min(chunk * 32 + r, rows - 1) * W,
                 *rb = router + (size_t)min(chunk * 32 + 16 + r, rows - 1) * W;
     moe_f32x4_t lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;                  // of the groups' halves
-    for (int grp = SPLIT ? blockIdx.x % MOE_ROUTE16_GROUPS : 0;
-         grp < (SPLIT ? (int)blockIdx.x % MOE_ROUTE16_GROUPS + 1 : MOE_ROUTE16_GROUPS);
-         grp += WAVES / 8) {
+    for (int grp = grp0; grp < grp1; grp += WAVES / 8) {
       const int k_begin = ((grp + wave / 8) * 8 + wave % 8) * span, k_end = min(W, k_begin + span);
       // (eight sums side by side, one an element of a lane's eight: sums of few terms, added in
       // pairs)
@@ -484,7 +502,7 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
       // [tile][chunk][half][lane][group][4]
       if (wave < 2) {
         float* p = ws + ((((size_t)tile * chunks + chunk) * 2 + wave) * ZF_WAVE + lane) *
-                            (MOE_ROUTE16_GROUPS * 4) + blockIdx.x % MOE_ROUTE16_GROUPS * 4;
+                            (MOE_ROUTE16_GROUPS * 4) + grp0 * 4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) store_agent(p + i, lo[i] + hi[i]);
         // The stores have reached memory before the count says so: on gfx950 agent-scope stores go
@@ -499,7 +517,7 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
   }
   __syncthreads();
   if constexpr (SPLIT) {
-    const int all = chunks * MOE_ROUTE16_GROUPS;
+    const int all = chunks * groups;
     if (threadIdx.x == 0)
       arrived = __hip_atomic_fetch_add(counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
@@ -515,7 +533,10 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
                                 (MOE_ROUTE16_GROUPS * 4);
       float v[MOE_ROUTE16_GROUPS * 4];
 #pragma unroll
-      for (int i = 0; i < MOE_ROUTE16_GROUPS * 4; i += 2) load2_agent(p + i, v[i], v[i + 1]);
+      for (int i = 0; i < MOE_ROUTE16_GROUPS * 4; i += 2) {
+        v[i] = v[i + 1] = 0.f;
+        if (i < 4 * groups) load2_agent(p + i, v[i], v[i + 1]);
+      }
       take(wave / 2, wave % 2, sum8([&](int grp) {
         return moe_f32x4_t{v[4 * grp], v[4 * grp + 1], v[4 * grp + 2], v[4 * grp + 3]};
       }));
@@ -527,8 +548,26 @@ __global__ __launch_bounds__((SPLIT ? 8 : 16) * ZF_WAVE) void moe_route16_kernel
                  n_groups, keep_groups, mark_top, normalize, weight_scale, lane);
 }
 
-// ws: float32 [4 tiles][(E + n_extra + 31) / 32][4096] and counters [4] at zero (both or neither;
-// the counters are at zero again when the kernel ends): what up to 64 tokens and 128 router rows
+// Which calls the kernel for 16 tokens a tile takes.  By the router's sizes: W from 2048 on, or from
+// 1024 on and 32 rows or more.  (Narrower ones are at the cost of a launch either way, or spend
+// their time on the choice, which only as many waves as tokens work at: 4 rows of 768 7.4 us,
+// four tokens a workgroup 6.6; 128 rows of 256 19.7, 16.3.)  In bfloat16 also by the tokens: up to
+// `few` through the sums in `ws`; and above 1024, where four tokens a workgroup fill the chip more
+// than once, from W = 512 on and any number of rows.  Measured, us, this and that: W = 2048, 32
+// rows: 8 tokens 9.1 and 16.5, 256 12.5 and 16.7, 1024 17.1 and 17.3, 2048 17.1 and 29.0; 128 rows:
+// 16.5 and 49.7, 37.9 and 50.4, 60.0 and 51.1, 60.3 and 96.8; 8 rows: 8 tokens 8.1 and 9.5, 256
+// 11.0 and 9.7; W = 4096, 64 rows: 12.1 and 45.4, 18.7 and 46.0, 36.2 and 46.5, 49.9 and 87.9.  In
+// float32 the same kernel for any number of tokens, so that a token's logits do not depend on it.
+static bool route16_takes(int T, int W, int rows, bool f32, bool sums) {
+  if (rows > MOE_ROUTE16_ROWS) return false;
+  if (!f32 && T > 1024) return W >= 512;
+  if (W < 1024 || (W < 2048 && rows < 32)) return false;
+  const int few = W >= 3072 ? 512 : rows < 32 ? 64 : 256;
+  return f32 || (sums && T <= few);
+}
+
+// ws: float32 [64 tiles][(E + n_extra + 31) / 32][4096] and counters [64] at zero (both or neither;
+// the counters are at zero again when the kernel ends): what up to 1024 tokens and 128 router rows
 // use to spread over workgroups.
 extern "C" int zf_moe_route(const void* h, int dtype, const float* router, const float* bias,
                             int* ids, float* weights, int T, int W, int E, int top,
@@ -542,20 +581,20 @@ extern "C" int zf_moe_route(const void* h, int dtype, const float* router, const
                                         keep_groups > n_groups ||
                                         top > keep_groups * (E / n_groups))))
     return -2;
-  if (E + n_extra <= MOE_ROUTE16_ROWS) {
+  const int rows = E + n_extra;
+  const bool sums = ws != nullptr && counters != nullptr;
+  if (route16_takes(T, W, rows, dtype == ZF_F32, sums)) {
     const bool vec = W % 8 == 0 && ((uintptr_t)h | (uintptr_t)router) % 16 == 0;
-    const bool split = T <= 16 * MOE_ROUTE16_SPLIT_TILES && ws != nullptr && counters != nullptr;
+    const int tiles = (T + 15) / 16, parts = (rows + 31) / 32 * route16_groups(W);
+    const bool split = sums && tiles <= MOE_ROUTE16_SPLIT_TILES && tiles * parts <= 1024;
 #define MOE_ROUTE16_AS(TT, V, S, G, B)                                                           \
   hipLaunchKernelGGL((moe_route16_kernel<TT, V, S>), G, dim3(B), 0, stream, (const TT*)h,        \
                      router, bias, ids, weights, T, W, E, top, scoring, correction, n_groups,    \
                      keep_groups, mark_top, normalize, weight_scale, n_extra, extra, ws, counters)
 #define MOE_ROUTE16(TT, V)                                                                       \
   do {                                                                                           \
-    if (split)                                                                                   \
-      MOE_ROUTE16_AS(TT, V, true,                                                                \
-                     dim3((E + n_extra + 31) / 32 * MOE_ROUTE16_GROUPS, (T + 15) / 16), 512);    \
-    else                                                                                         \
-      MOE_ROUTE16_AS(TT, V, false, dim3((T + 15) / 16), 1024);                                   \
+    if (split) MOE_ROUTE16_AS(TT, V, true, dim3(parts, tiles), 512);                             \
+    else MOE_ROUTE16_AS(TT, V, false, dim3(tiles), 1024);                                        \
   } while (0)
     if (dtype == ZF_F32) {
       if (vec) MOE_ROUTE16(float, true); else MOE_ROUTE16(float, false);

@@ -1812,14 +1812,15 @@ MOE_MAX_EXPERTS = 1024
 ROUTER_SCORINGS = {"softmax": 0, "sigmoid": 1, "softmax_all": 2}
 
 
-_MOE_ROUTE_SUMS = 4 * 4 * 4096         # 4 tiles of tokens, 4 chunks of router rows
+_MOE_ROUTE_TILES = 64                   # MOE_ROUTE16_SPLIT_TILES in moe.hip
+_MOE_ROUTE_SUMS = _MOE_ROUTE_TILES * 4 * 4096          # for each 4 chunks of router rows
 
 
 def moe_route_work(device) -> torch.Tensor:
     """Sums and (at zero) counters for ``moe_route``'s ``work``.  Two calls that may overlap must
     not share one (a counter would stay off zero for good): an engine, whose launches follow each
     other, holds its own."""
-    return torch.zeros((_MOE_ROUTE_SUMS + 4,), dtype=torch.float32, device=device)
+    return torch.zeros((_MOE_ROUTE_SUMS + _MOE_ROUTE_TILES,), dtype=torch.float32, device=device)
 
 
 @_launches("other")
@@ -1841,8 +1842,8 @@ def moe_route(h: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor
     the weights are the chosen s themselves; either way times ``weight_scale``.  ``extra``
     float32 [T, n]: the router has n more rows behind its E outputs, which are no experts; the
     sigmoids of their products with h go there (a gate a token that rides with the router).
-    ``work`` (``moe_route_work``, the caller's own, for one call at a time): up to 64 tokens then
-    spread over workgroups, the same numbers."""
+    ``work`` (``moe_route_work``, the caller's own, for one call at a time): up to 1024 tokens may
+    then spread over workgroups; the same numbers, in bfloat16 up to the rounding of 32-bit sums."""
     _need_gpu(h, router, bias, ids, weights, correction, extra, work)
     _i32(ids, "ids")
     T, W = h.shape
@@ -1874,7 +1875,7 @@ def moe_route(h: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor
     lib = build.load("moe")
     ws = counters = None
     if work is not None:
-        if work.dtype != torch.float32 or work.numel() != _MOE_ROUTE_SUMS + 4:
+        if work.dtype != torch.float32 or work.numel() != _MOE_ROUTE_SUMS + _MOE_ROUTE_TILES:
             raise KernelUnavailable("moe_route: work is what moe_route_work made")
         ws, counters = work, work[_MOE_ROUTE_SUMS:]
     _check(lib.zf_moe_route(_ptr(h), _dt(h), _ptr(router), _ptr(bias), _ptr(ids), _ptr(weights),
