@@ -330,3 +330,26 @@ def test_residual_sums_of_several_hundred_tokens_over_a_long_k_take_wide_tiles_s
     for M, N, K in ((512, 5120, 17408), (640, 4096, 12288), (1281, 4096, 12288), (2048, 4096, 12288),
                     (1024, 4096, 4096), (1024, 5120, 5120)):
         assert ops._wide_ksplit(M, N, K) is None, (M, N, K)
+
+
+def test_shared_arrays_accessed_in_16_byte_pieces_say_that_they_are_aligned():
+    """A kernel's LDS arrays of smaller elements that it reads or writes as vectors carry the
+    alignment: their type alone promises two or four bytes."""
+    import glob
+    import os
+    import re
+    from zinfer_amd.ops import build
+    wide = r"(?:float4|uint4|int4|(?:moe_)?u32x4_t|(?:moe_)?f32x4_t|(?:moe_)?bf16x8_t)"
+    found = []
+    for path in sorted(glob.glob(os.path.join(build.CSRC, "*.hip"))):
+        with open(path) as f:
+            kernels = re.split(r"\b__global__\b", f.read())[1:]
+        for text in kernels:
+            name = re.search(r"void\s+(\w+)", text).group(1)
+            plain = set()
+            for kind, rest in re.findall(r"__shared__\s+((?:float|int|short|bf16_t|unsigned|uint32_t))"
+                                         r"\s+([^;]+);", text):
+                plain |= set(re.findall(r"(?:^|,)\s*(\w+)\s*\[", rest))
+            used = set(re.findall(r"\*\(\s*(?:const\s+)?" + wide + r"\s*\*\)\s*&?\s*\(?\s*(\w+)", text))
+            found += [f"{os.path.basename(path)}: {name}: {array}" for array in sorted(plain & used)]
+    assert not found

@@ -686,7 +686,7 @@ __global__ __launch_bounds__(MOE_WAVES * ZF_WAVE) void moe_gate_up_kernel(
     const T* __restrict__ h, const T* __restrict__ gate_up, const int* __restrict__ ids,
     T* __restrict__ y, int W, int ff, int slots, float limit, float alpha, float shift, int act,
     int n_experts) {
-  extern __shared__ float xs[];                    // the token's row, [W]
+  extern __shared__ __attribute__((aligned(16))) float xs[];       // the token's row, [W]
   const int ts = blockIdx.x, t = ts / slots;
   const int e = ids != nullptr ? ids[ts] : 0;
   if (e >= n_experts) return;                      // an output of the router without an expert
@@ -1083,7 +1083,7 @@ __global__ __launch_bounds__(1024) void moe_few_down_kernel(
     const bf16_t* __restrict__ shared_w, const bf16_t* __restrict__ shared_y, int shared_ff) {
   __shared__ int n_units, id[MOE_FEW_PAIRS], expert[MOE_FEW_PAIRS];
   __shared__ float share[MOE_FEW_PAIRS];
-  __shared__ short pairs[MOE_FEW_PAIRS][8];            // of a unit; -1 where it has fewer
+  __shared__ __attribute__((aligned(16))) short pairs[MOE_FEW_PAIRS][8];   // of a unit; -1: it has fewer
   extern __shared__ __attribute__((aligned(16))) float sums[];   // [pair][2 pieces][8], then shared's
   const int wave = threadIdx.x / ZF_WAVE, lane = threadIdx.x % ZF_WAVE;
   const int r = lane % 16, g = lane / 16, n0 = blockIdx.x * 8, P = T * top;
