@@ -102,12 +102,20 @@ __device__ __forceinline__ void lanes_sum_up(float (&v)[N], int n) {
 #pragma unroll
     for (int i = 0; i < N; ++i) v[i] = f(v[i]);
   };
-  if (n > 1) each([](float x) { return x + lane_xor<1>(x); });
-  if (n > 2) each([](float x) { return x + lane_xor<2>(x); });
-  if (n > 4) each([](float x) { return x + lane_move<0x141>(x, x); });      // row_half_mirror
-  if (n > 8) each([](float x) { return x + lane_move<0x140>(x, x); });      // row_mirror
-  if (n > 16) each([](float x) { return apart_sum<16>(x); });
-  if (n > 32) each([](float x) { return apart_sum<32>(x); });
+  // (Left as early as a group is done: with a branch for every step that is not taken, walks over
+  // tokens that add up few lanes took longer: 32 heads of 16 x 64, 64 tokens 49.6 us for 43.8.)
+  if (n <= 1) return;
+  each([](float x) { return x + lane_xor<1>(x); });
+  if (n <= 2) return;
+  each([](float x) { return x + lane_xor<2>(x); });
+  if (n <= 4) return;
+  each([](float x) { return x + lane_move<0x141>(x, x); });      // row_half_mirror
+  if (n <= 8) return;
+  each([](float x) { return x + lane_move<0x140>(x, x); });      // row_mirror
+  if (n <= 16) return;
+  each([](float x) { return apart_sum<16>(x); });
+  if (n <= 32) return;
+  each([](float x) { return apart_sum<32>(x); });
 }
 // lanes_sum for a number of lanes that is known when the kernel runs
 __device__ __forceinline__ float lanes_sum_down(float v, int n) {
