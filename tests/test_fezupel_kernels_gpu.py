@@ -374,6 +374,31 @@ def test_router_of_128_rows_takes_no_longer_than_one_of_129(T, W):
     assert best[0] <= 1.2 * best[1], f"{best[0] * 50:.1f} us, {best[1] * 50:.1f} us"
 
 
+@pytest.mark.parametrize("T, W, ff, E, top", [(16, 64, 64, 20, 16), (16, 128, 64, 20, 17),
+                                               (9, 64, 128, 64, 32), (1, 64, 64, 300, 257)])
+@pytest.mark.parametrize("act", [None, "relu2"])
+def test_pre_tiled_experts_of_a_few_tokens_with_many_pairs(T, W, ff, E, top, act):
+    """Up to 16 tokens whose pairs are 256 or more: beyond 256 pre-tiled matrices go through the tiles
+    sorted by expert.  Against the same matrices row by row."""
+    dt = torch.bfloat16
+    h = _rand((T, W), 24, dtype=dt).to(DEV)
+    gate_up = _rand((E, ff if act else 2 * ff, W), 25, 2 / W ** 0.5, dt).to(DEV)
+    down = _rand((E, W, ff), 26, 2 / ff ** 0.5, dt).to(DEV)
+    g = torch.Generator().manual_seed(27)
+    ids = torch.stack([torch.randperm(E + 1, generator=g)[:top] for _ in range(T)]).to(torch.int32).to(DEV)
+    share = (torch.rand((T, top), generator=g) / top).to(DEV)
+    tiled = [torch.stack([ops.pretile_weight(m) for m in w]) for w in (gate_up, down)]
+    assert (T * top > 256) == (not ops.moe_few_covers(h, top))
+    base, outs = _rand((T, W), 28).to(DEV), []
+    for w_tiled, (gu, dn) in ((False, (gate_up, down)), (True, tiled)):
+        y = torch.empty((T, top, ff), dtype=dt, device=DEV)
+        outs.append(base.clone())
+        ops.moe_experts(h, gu, dn, ids, share, y, outs[-1], 0.6, 1.702, 1.0, add=True, act=act,
+                        n_identity=1, w_tiled=w_tiled)
+    # (activations rounded to bfloat16 from sums of another order)
+    assert rel_err(outs[1], outs[0]) < 1e-2
+
+
 @pytest.mark.parametrize("T, W, ff, E, top", [(40, 64, 24, 6, 2), (300, 128, 64, 8, 3),
                                                (17, 72, 136, 1, 1), (150, 352, 104, 40, 4),
                                                (260, 64, 8, 3, 3)])
