@@ -2,6 +2,7 @@
 import os
 import re
 import subprocess
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -26,6 +27,27 @@ def _step(scratch):
                           "state_slots", "want_rows"))
     return StepContext(n_tokens=3, n_seqs=3, n_want=3, kv=[], max_q_len=1, max_ctx_len=1,
                        q_lens=[1] * 3, ctx_lens=[1] * 3, slots=[0] * 3, _scratch=scratch, **none)
+
+
+@pytest.mark.parametrize("W, ff, top, shared, tiled", [
+    (256, 128, 8, False, False), (256, 128, 8, True, False), (1024, 512, 8, False, False),
+    (1024, 1024, 4, True, False), (2048, 448, 4, True, False), (2048, 512, 2, True, True),
+    (2048, 768, 4, False, False), (2048, 768, 4, True, True), (2048, 2048, 4, False, True),
+    (2048, 2048, 2, False, False), (3072, 2048, 4, False, False), (3072, 2048, 2, True, True),
+    (4096, 1024, 4, False, True)])
+def test_experts_are_laid_out_anew_where_that_pays(monkeypatch, W, ff, top, shared, tiled):
+    """Row by row where that is the faster form for a few tokens: narrow layers, few experts a token
+    without a shared one."""
+    asked, E = [], max(top, 2)
+    monkeypatch.setattr(moe.ops, "moe_can_pretile", lambda gate_up, down: True)
+    monkeypatch.setattr(moe.ops, "pretile_weight", lambda w: asked.append(w.shape) or w)
+    monkeypatch.setattr(moe, "Linear", lambda w: SimpleNamespace(tiled=True, weight=w))
+    spec = MoeSpec(hidden_size=W, n_experts=E, top_k=top, expert=GatedExpertSpec(ff),
+                   shared=GatedExpertSpec(ff) if shared else None)
+    part = moe.MoeFeedForward(spec, BuildContext(torch.bfloat16, torch.device("cpu")), "")
+    part.bind({n: torch.zeros((1, 1), dtype=torch.bfloat16).expand(d.shape)
+               for n, d in part.declare().items()})
+    assert asked == ([(E * 2 * ff, W), (E * W, ff)] if tiled else [])
 
 
 def test_engines_on_one_model_do_not_share_the_routers_counters(monkeypatch):

@@ -1991,6 +1991,24 @@ def moe_can_pretile(gate_up: torch.Tensor, down: torch.Tensor) -> bool:
         and down.shape[2] % 64 == 0
 
 
+def moe_pretile_pays(width: int, ff: int, top: int, shared: bool) -> bool:
+    """Whether a layer's experts are pre-tiled: a few tokens then read every used expert once, in two
+    kernels, instead of streaming the chosen experts' rows token by token.  With an expert that
+    all tokens share (``shared``: its matrices pre-tiled too, so that it rides along, three
+    launches less) from W = 2048 and ff = 512 on; without one from four experts a token on where a
+    matrix is large: W * ff of 4 << 20, 8 << 20 where the down kernel's W / 8 workgroups end in a
+    part of a round.  Below, the lists of pairs and the few workgroups of the down kernel cost
+    more than the reading saves.  Measured over 2 to 8 of 8 to 128 experts and 1 to 16 tokens, time
+    pre-tiled over time row by row, (least, most): with a shared expert W = 1024 (0.63, 1.27), 1536
+    (0.61, 1.14), 2048 (0.56, 0.97 from ff = 512 on; ff = 256 1.08), 3072 (0.59, 1.02), 4096 (0.54,
+    0.97); without W = 256, ff = 128 (0.85, 2.70), 1024 x 512 (1.00, 1.46), 2048 x 768 (0.71, 1.24),
+    and from four a token on 2048 x 2048 (0.60, 0.98), 4096 x 1024 (0.54, 1.02), 3072 x 2048 (0.62,
+    1.04); 16 and 32 a token 0.25 to 0.97."""
+    if shared:
+        return width >= 2048 and ff >= 512
+    return top >= 4 and width * ff >= (4 << 20 if width % 2048 == 0 else 8 << 20)
+
+
 def moe_few_covers(h: torch.Tensor, top: int) -> bool:
     """Whether ``moe_experts`` takes pre-tiled matrices through the kernels for few tokens: up to
     16 of them, rows 16-byte aligned."""
@@ -2063,8 +2081,8 @@ def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ids:
     depends on that token alone.  ``act``: experts without a gate (see ``moe_gate_up``).
     ``n_identity``: ids from E up to E + n_identity - 1 name no expert; such a term of the sum is
     the weight times h[t] itself.  ``w_tiled``: every expert's matrices went through
-    ``pretile_weight`` (``moe_can_pretile``); a few tokens then stream every used expert's
-    matrices once past all tokens that chose it.  ``shared``: an expert that all tokens use, added
+    ``pretile_weight`` (``moe_can_pretile``; worth it where ``moe_pretile_pays``); a few tokens then
+    stream every used expert's matrices once past all tokens that chose it.  ``shared``: an expert that all tokens use, added
     by the same kernels (with ``w_tiled``, where ``moe_few_covers``; see ``_moe_few``)."""
     T, W = h.shape
     if w_tiled and moe_few_covers(h, ids.shape[1]):

@@ -129,16 +129,22 @@ class MoeFeedForward(FeedForward):
             if s.correction_name is not None else None
         self.gate_up, self.down = self._stack(
             tensors, [p + s.expert_prefix.format(e) for e in range(s.n_experts)])
-        # bfloat16 matrices whose sizes allow it are re-laid once into the MFMA kernels' own order
-        # (all experts' rows as one matrix: the order is by groups of 16 rows)
-        self.tiled = ops.moe_can_pretile(self.gate_up, self.down)
-        if self.tiled:
-            self.gate_up, self.down = (ops.pretile_weight(m.flatten(0, 1)).view(m.shape)
-                                       for m in (self.gate_up, self.down))
+        rides = False
         if s.shared is not None:
             # the expert every token uses is two plain products around the activation
             gu, dn = self._stack(tensors, [p + s.shared_prefix])
             self.shared_gate_up, self.shared_down = Linear(gu[0]), Linear(dn[0])
+            rides = self.shared_gate_up.tiled and self.shared_down.tiled
+        # bfloat16 matrices whose sizes allow it and make it worth while are re-laid once into the
+        # MFMA kernels' own order (all experts' rows as one matrix: the order is by groups of 16
+        # rows)
+        self.tiled = ops.moe_can_pretile(self.gate_up, self.down) \
+            and ops.moe_pretile_pays(s.hidden_size, s.expert.intermediate_size, s.top_k, rides)
+        if self.tiled:
+            self.gate_up, self.down = (ops.pretile_weight(m.flatten(0, 1)).view(m.shape)
+                                       for m in (self.gate_up, self.down))
+        # a few tokens: the shared expert rides with the routed ones
+        self.rides = rides and self.tiled
 
     def forward(self, h, residual, step, accumulate: bool = True) -> None:
         s = self.spec
@@ -169,9 +175,7 @@ class MoeFeedForward(FeedForward):
             factor = shared_gate[:, 0] if shared_gate is not None else None
             s_numbers = (float(sh.limit or 0.0), float(sh.alpha), float(sh.shift))
             ys = step.scratch("moe_shared_act", (T, sh.intermediate_size), dtype)
-            if self.tiled and self.shared_gate_up.tiled and self.shared_down.tiled \
-                    and ops.moe_few_covers(h, s.top_k):
-                # a few tokens: the shared expert rides with the routed ones
+            if self.rides and ops.moe_few_covers(h, s.top_k):
                 ops.moe_experts(h, self.gate_up, self.down, ids, share, y, residual, *numbers,
                                 add=accumulate, n_identity=s.n_identity, w_tiled=True,
                                 shared=(self.shared_gate_up.weight, self.shared_down.weight, ys,
