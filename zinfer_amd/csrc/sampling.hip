@@ -102,15 +102,24 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_topk_kernel(
   int k = prm.top_k <= 0 || prm.top_k > V ? V : prm.top_k;
   if (k > SMP_MAX_K) k = SMP_MAX_K;     // the host refuses such rows before launching
 
-  auto each = [&](auto&& f) {                // f(value, id) for the thread's part of the row
+  // f(value, id) for the thread's part of the row, until enough(), which is asked every eight loads
+  auto each = [&](auto&& f, auto&& enough) {
     if (V % 4 == 0 && ((uintptr_t)row & 15) == 0) {
-#pragma unroll 8
-      for (int i = tid; i < V / 4; i += SMP_THREADS) {
-        const float4 v = ((const float4*)row)[i];
-        f(v.x, 4 * i);
-        f(v.y, 4 * i + 1);
-        f(v.z, 4 * i + 2);
-        f(v.w, 4 * i + 3);
+      for (int i0 = tid; i0 < V / 4; i0 += 8 * SMP_THREADS) {
+        float4 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (i0 + u * SMP_THREADS < V / 4) v[u] = ((const float4*)row)[i0 + u * SMP_THREADS];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int i = i0 + u * SMP_THREADS;
+          if (i >= V / 4) break;
+          f(v[u].x, 4 * i);
+          f(v[u].y, 4 * i + 1);
+          f(v[u].z, 4 * i + 2);
+          f(v[u].w, 4 * i + 3);
+        }
+        if (enough()) break;
       }
     } else {
       for (int i = tid; i < V; i += SMP_THREADS) f(row[i], i);
@@ -118,7 +127,7 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_topk_kernel(
   };
   if (tid == 0) s_count = 0;
   uint32_t mine = 0;                         // (no float has the key 0 but a NaN, which none may reach)
-  each([&](float v, int) { mine = max(mine, float_key(v)); });
+  each([&](float v, int) { mine = max(mine, float_key(v)); }, [] { return false; });
   if (tid == 0) {
     s_prefix = 0;
     s_remaining = (unsigned)min(k, SMP_THREADS);
@@ -143,7 +152,7 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_topk_kernel(
         cidx[at] = i;
       }
     }
-  });
+  }, [&] { return *(volatile unsigned*)&s_count > SMP_MAX_K; });      // (they go to the radix select)
   __syncthreads();
   int found = (int)s_count;
   __syncthreads();
