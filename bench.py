@@ -656,7 +656,8 @@ def fezupel_kernels(sh: dict, T: int, ctx: int, mfma_rate: float, read_bw: float
     gate_up = rnd(E, 2 * ff, W)
     down = rnd(E, W, ff)
     res = torch.zeros((rows, W), dtype=torch.float32, device=dev)
-    moe = _moe_launcher(ops, h, router, ids, share, gate_up, down, res, top, ff)
+    moe = _mixture_launcher(ops, h, router, ids, share, gate_up, down, res, (7.0, 1.702, 1.0),
+                            rides=True)
     t_moe = _timed(moe)
     inter = top * ff
     wgu = ops.pretile_weight(ops.interleave_gate_up(rnd(inter, W), rnd(inter, W)))
@@ -689,14 +690,33 @@ def fezupel_kernels(sh: dict, T: int, ctx: int, mfma_rate: float, read_bw: float
     return out
 
 
-def _moe_launcher(ops, h, router, ids, share, gate_up, down, res, top, ff):
+def _mixture_launcher(ops, h, router, ids, share, gate_up, down, out, numbers=(0.0, 1.0, 0.0),
+                      rides=False, shared=None, n_identity=0, act=None, add=False, **route):
+    """Router and experts as the engine's mixture launches them: with work space for the router, the
+    experts' matrices as it holds them (``rides``: beside an expert that all tokens share), and for
+    a few tokens the shared expert (gate_up and down pre-tiled, its column of gates) in the same
+    kernels, else in products of its own."""
     import torch
-    rows = h.shape[0]
-    y = torch.empty((rows, top, ff), dtype=h.dtype, device=h.device)
+    rows, top = ids.shape
+    gate_up, down, tiled = ops.moe_lay_out(gate_up, down, top, rides or shared is not None)
+    y = torch.empty((rows, top, down.shape[2]), dtype=h.dtype, device=h.device)
+    work = ops.moe_route_work(h.device)
+    fused = None
+    if shared is not None:
+        s_gate_up, s_down, gate = shared
+        ys = torch.empty((rows, s_down.shape[1]), dtype=h.dtype, device=h.device)
+        s_rows = torch.empty((rows, s_gate_up.shape[0]), dtype=h.dtype, device=h.device)
+        if tiled and ops.moe_few_covers(h, top):
+            fused = (s_gate_up, s_down, ys, 0.0, 1.0, 0.0, gate)
 
     def run():
-        ops.moe_route(h, router, None, ids, share)
-        ops.moe_experts(h, gate_up, down, ids, share, y, res, 7.0, 1.702, 1.0, add=False)
+        ops.moe_route(h, router, None, ids, share, work=work, **route)
+        ops.moe_experts(h, gate_up, down, ids, share, y, out, *numbers, add=add, act=act,
+                        n_identity=n_identity, w_tiled=tiled, shared=fused)
+        if shared is not None and fused is None:
+            ops.gemm(h, s_gate_up, s_rows, w_tiled=True)
+            ops.gated_act(s_rows, ys, 0.0, 1.0, 0.0, row_factor=gate)
+            ops.gemm(ys, s_down, out, accumulate=True, w_tiled=True)
     return run
 
 
@@ -1215,13 +1235,8 @@ def nupovik_kernels(sh: dict, T: int, ctx: int, mfma_rate: float, read_bw: float
         ids = torch.empty((rows, top), dtype=torch.int32, device=dev)
         share = torch.empty((rows, top), dtype=torch.float32, device=dev)
         up, down = rnd(E, ff, W), rnd(E, W, ff)
-        y = torch.empty((rows, top, ff), dtype=bf, device=dev)
-
-        def mixture():
-            ops.moe_route(h, router, None, ids, share, scoring="sigmoid", correction=correction,
-                          groups=groups)
-            ops.moe_experts(h, up, down, ids, share, y, branch, 0.0, 1.0, 0.0, add=True,
-                            act="relu2")
+        mixture = _mixture_launcher(ops, h, router, ids, share, up, down, branch, act="relu2", add=True,
+                                    scoring="sigmoid", correction=correction, groups=groups)
         t_new = _timed_graph(mixture)
         inter = top * ff * 2 // 3 // 64 * 64
         t_old = gated_twin(inter)
@@ -1518,19 +1533,12 @@ def kugisun_kernels(sh: dict, T: int, ctx: int, mfma_rate: float, read_bw: float
     share = torch.empty((rows, top), dtype=torch.float32, device=dev)
     sgate = torch.empty((rows, 1), dtype=torch.float32, device=dev)
     gu, down = rnd(E, 2 * ff, W), rnd(E, W, ff)
-    y = torch.empty((rows, top, ff), dtype=bf, device=dev)
     wsgu = ops.pretile_weight(rnd(2 * shared, W))
     wsd = ops.pretile_weight(rnd(W, shared))
-    sgu = torch.empty((rows, 2 * shared), dtype=bf, device=dev)
-    sy = torch.empty((rows, shared), dtype=bf, device=dev)
-
-    def mixture():
-        ops.moe_route(h, router, None, ids, share, scoring="softmax_all", correction=correction,
-                      groups=groups, group_mark=1, normalize=False, weight_scale=2.5, extra=sgate)
-        ops.moe_experts(h, gu, down, ids, share, y, branch, 0.0, 1.0, 0.0, add=False, n_identity=I)
-        ops.gemm(h, wsgu, sgu, w_tiled=True)
-        ops.gated_act(sgu, sy, 0.0, 1.0, 0.0, row_factor=sgate[:, 0])
-        ops.gemm(sy, wsd, branch, accumulate=True, w_tiled=True)
+    mixture = _mixture_launcher(ops, h, router, ids, share, gu, down, branch, n_identity=I,
+                                shared=(wsgu, wsd, sgate[:, 0]), scoring="softmax_all",
+                                correction=correction, groups=groups, group_mark=1,
+                                normalize=False, weight_scale=2.5, extra=sgate)
     t_new = _timed_graph(mixture)
     inter = (top * ff + shared) // 64 * 64
     t_old = gated(inter)

@@ -69,6 +69,30 @@ def test_engines_on_one_model_do_not_share_the_routers_counters(monkeypatch):
     assert seen[4] is first[0] and seen[6] is second[0]
 
 
+@pytest.mark.parametrize("W, ff, tiled", [(64, 64, False), (2048, 512, True)])
+def test_bench_launches_a_mixture_as_the_engine_does(monkeypatch, W, ff, tiled):
+    """Experts laid out by the same rule, work space for the router, the shared expert in the
+    experts' kernels where it rides along there."""
+    import bench
+    T, E, top, calls = 4, 4, 2, []
+    ops = moe.ops
+    monkeypatch.setattr(ops, "moe_can_pretile", lambda gate_up, down: True)
+    monkeypatch.setattr(ops, "moe_few_covers", lambda h, top: True)
+    for name in ("moe_route", "moe_experts", "gemm", "gated_act"):
+        monkeypatch.setattr(ops, name, lambda *a, name=name, **kw: calls.append((name, kw)))
+    z = lambda *s, dt=torch.bfloat16: torch.zeros(s, dtype=dt)
+    gate = z(T, 1, dt=torch.float32)
+    run = bench._mixture_launcher(ops, z(T, W), z(E, W, dt=torch.float32),
+                                  z(T, top, dt=torch.int32), z(T, top, dt=torch.float32),
+                                  z(E, 2 * ff, W), z(E, W, ff), z(T, W, dt=torch.float32),
+                                  shared=(z(128, W), z(W, 64), gate[:, 0]), scoring="sigmoid")
+    run()
+    (_, route), (_, experts) = calls[:2]
+    assert route["work"] is not None and route["scoring"] == "sigmoid"
+    assert experts["w_tiled"] == tiled and (experts["shared"] is not None) == tiled
+    assert [name for name, _ in calls[2:]] == ([] if tiled else ["gemm", "gated_act", "gemm"])
+
+
 def _compile_moe(arch, out):
     from zinfer_amd.ops import build
     if not os.path.exists("/opt/rocm/bin/hipcc"):

@@ -2009,6 +2009,17 @@ def moe_pretile_pays(width: int, ff: int, top: int, shared: bool) -> bool:
     return top >= 4 and width * ff >= (4 << 20 if width % 2048 == 0 else 8 << 20)
 
 
+def moe_lay_out(gate_up: torch.Tensor, down: torch.Tensor, top: int, shared: bool):
+    """(gate_up, down, whether they are pre-tiled) of a layer's stacked experts as they are held:
+    bfloat16 matrices whose sizes allow it and make it worth while are re-laid once into the MFMA
+    kernels' own order (all experts' rows as one matrix: the order is by groups of 16 rows)."""
+    if not (moe_can_pretile(gate_up, down)
+            and moe_pretile_pays(gate_up.shape[2], down.shape[2], top, shared)):
+        return gate_up, down, False
+    gate_up, down = (pretile_weight(m.flatten(0, 1)).view(m.shape) for m in (gate_up, down))
+    return gate_up, down, True
+
+
 def moe_few_covers(h: torch.Tensor, top: int) -> bool:
     """Whether ``moe_experts`` takes pre-tiled matrices through the kernels for few tokens: up to
     16 of them, rows 16-byte aligned."""

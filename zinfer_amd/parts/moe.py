@@ -135,14 +135,8 @@ class MoeFeedForward(FeedForward):
             gu, dn = self._stack(tensors, [p + s.shared_prefix])
             self.shared_gate_up, self.shared_down = Linear(gu[0]), Linear(dn[0])
             rides = self.shared_gate_up.tiled and self.shared_down.tiled
-        # bfloat16 matrices whose sizes allow it and make it worth while are re-laid once into the
-        # MFMA kernels' own order (all experts' rows as one matrix: the order is by groups of 16
-        # rows)
-        self.tiled = ops.moe_can_pretile(self.gate_up, self.down) \
-            and ops.moe_pretile_pays(s.hidden_size, s.expert.intermediate_size, s.top_k, rides)
-        if self.tiled:
-            self.gate_up, self.down = (ops.pretile_weight(m.flatten(0, 1)).view(m.shape)
-                                       for m in (self.gate_up, self.down))
+        self.gate_up, self.down, self.tiled = ops.moe_lay_out(self.gate_up, self.down, s.top_k,
+                                                              rides)
         # a few tokens: the shared expert rides with the routed ones
         self.rides = rides and self.tiled
 
