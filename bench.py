@@ -670,7 +670,7 @@ def fezupel_kernels(sh: dict, T: int, ctx: int, mfma_rate: float, read_bw: float
     t_dense = _timed(dense)
     ff_flops = 2.0 * rows * 3 * inter * W
     if decode:
-        used = min(E, rows * top)        # at most this many experts' matrices are read
+        used = int(ids[ids < E].unique().numel())      # experts whose matrices are read
         mb, db = used * 3 * ff * W * 2, 3 * inter * W * 2
         out["feed_forward"] = {"fezupel_us": round(t_moe * 1e6, 1), "qwen3_us": round(t_dense * 1e6, 1),
                                "fezupel_frac_of_read": round(mb / t_moe / read_bw, 4),
@@ -1241,7 +1241,7 @@ def nupovik_kernels(sh: dict, T: int, ctx: int, mfma_rate: float, read_bw: float
         inter = top * ff * 2 // 3 // 64 * 64
         t_old = gated_twin(inter)
         if decode:
-            used = min(E, rows * top)        # at most this many experts' matrices are read
+            used = int(ids[ids < E].unique().numel())      # experts whose matrices are read
             row("mixture", t_new, used * 2 * ff * W * 2, read_bw, "read", t_old,
                 3 * inter * W * 2, read_bw, "read")
         else:
@@ -1543,7 +1543,7 @@ def kugisun_kernels(sh: dict, T: int, ctx: int, mfma_rate: float, read_bw: float
     inter = (top * ff + shared) // 64 * 64
     t_old = gated(inter)
     if decode:
-        used = min(E, rows * top)
+        used = int(ids[ids < E].unique().numel())
         row("mixture", t_new, (used * ff + shared) * 3 * W * 2, read_bw, "read",
             "qwen3 feed-forward of the width a token uses", t_old, 3 * inter * W * 2, read_bw,
             "read")
