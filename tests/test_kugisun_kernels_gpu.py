@@ -15,6 +15,7 @@ import torch
 
 import plain_kugisun as P
 from gpu_util import DEV, rel_err, tol
+from timing import graph_us
 from zinfer_amd import ops
 
 pytestmark = pytest.mark.gpu
@@ -83,6 +84,60 @@ def test_streams_step_where_the_kernel_changes(S, W):
     and the first that it does not, one copy more than it takes."""
     for dt in DTYPES:
         test_streams_step(dt, S, W)
+
+
+def _sum_of_256(squares):
+    """The 32-bit sum of a row's squares in the order in which 256 threads of four columns add them: a
+    thread's columns in turn, then pairs of lanes 32, 16, .. 1 apart, then the four waves."""
+    import numpy as np
+    n = len(squares)
+    part = np.zeros(256, np.float32)
+    for at in range(0, n, 1024):
+        for e in range(4):
+            c = at + 4 * np.arange(256) + e
+            part = part + np.where(c < n, squares[np.minimum(c, n - 1)], np.float32(0))
+    part = part.reshape(4, 64)
+    for off in (32, 16, 8, 4, 2, 1):
+        part = part + part[:, np.arange(64) ^ off]
+    total = np.float32(0)
+    for w in range(4):
+        total = np.float32(total + part[w, 0])
+    return total
+
+
+@pytest.mark.parametrize("W", [64, 1020, 1024, 1028, 2048, 3076, 4096, 4100])
+@pytest.mark.parametrize("T", [2, 300])
+def test_streams_step_adds_a_row_in_one_order(W, T):
+    """The norm's sum of squares, bit for bit: one order whichever kernel takes the call, and so
+    whatever the number of rows; written and read, and only read."""
+    import numpy as np
+    eps = 1e-5
+    x = _rand((1, T, W), 61)
+    one, none = torch.ones((1, 1), device=DEV), torch.zeros((1,), device=DEV)
+    gain, y = torch.ones((W,), device=DEV), torch.zeros((T, W), device=DEV)
+    rows = x[0].numpy()
+    inv = np.array([np.float32(1) / np.sqrt(_sum_of_256(r * r) / np.float32(W) + np.float32(eps))
+                    for r in rows[:20]], np.float32)
+    want = torch.from_numpy(rows[:20] * inv[:, None])
+    for branches in ((), [(y, 1.0)]):
+        out = torch.empty((T, W), device=DEV)
+        ops.streams_step(x.to(DEV), branches, one if branches else None, none if branches else None,
+                         read=True, gain=gain, eps=eps, out=out)
+        assert torch.equal(out.cpu()[:20], want)
+
+
+@pytest.mark.parametrize("S,W", [(1, 4096), (1, 2048)])
+def test_streams_that_are_only_read_take_no_longer_in_wide_workgroups(S, W):
+    """Many rows that are only read: about as long a column as those of a row that is too wide for a
+    workgroup (they took up to 1.5 times as long)."""
+    T, times = 2048, []
+    for width in (W, 4100):
+        x, gain = _rand((S, T, width), 62).to(DEV), torch.ones((width,), device=DEV)
+        out = torch.empty((T, width), dtype=torch.bfloat16, device=DEV)
+        times.append(graph_us(lambda: ops.streams_step(x, read=True, gain=gain, eps=1e-5, out=out)))
+    # (of 4100 columns a kernel of 256 threads takes 14.7 us for one copy; narrower rows have some
+    # 3 us of launch and sum that do not shrink with them)
+    assert times[0] <= 1.1 * (3 + (times[1] - 3) * W / 4100), times
 
 
 # ------------------------------------------------------------------------------ rows of a projection

@@ -473,7 +473,8 @@ __global__ __launch_bounds__(1024) void streams_row_kernel(
     const float* __restrict__ b, const float* __restrict__ a, const float* __restrict__ gain,
     float eps, TO* __restrict__ out, int W, int do_read) {
 #pragma clang fp contract(off)
-  __shared__ float red[16];
+  extern __shared__ __attribute__((aligned(16))) float4 rest[];      // u of the threads from 256 on
+  __shared__ float red[4];
   const size_t row = (size_t)blockIdx.x * W;
   const int i = threadIdx.x * 4;
   const bool mine = i < W;
@@ -520,15 +521,31 @@ __global__ __launch_bounds__(1024) void streams_row_kernel(
     u = make_float4(u.x + as * v[s].x, u.y + as * v[s].y, u.z + as * v[s].z, u.w + as * v[s].w);
   }
   if (gain != nullptr) {
+    // the squares in the order in which a workgroup of 256 adds them: thread i those of the columns
+    // 4 i, 4 (i + 256), .., then the four waves
+    if (threadIdx.x >= 256) rest[threadIdx.x - 256] = u;
+    if (W > 1024) __syncthreads();                 // (uniform)
     float ss = 0.f;
-    if (mine) {
-      ss += u.x * u.x;
-      ss += u.y * u.y;
-      ss += u.z * u.z;
-      ss += u.w * u.w;
+    auto add = [&](float4 q) {
+      ss += q.x * q.x;
+      ss += q.y * q.y;
+      ss += q.z * q.z;
+      ss += q.w * q.w;
+    };
+    if (threadIdx.x < 256) {
+      if (mine) add(u);
+#pragma unroll
+      for (int k = 1; k < 4; ++k)
+        if (i + 1024 * k < W) add(rest[threadIdx.x + 256 * (k - 1)]);
+      ss = wave_sum(ss);
+      if (threadIdx.x % ZF_WAVE == 0) red[threadIdx.x / ZF_WAVE] = ss;
     }
-    ss = block_sum(ss, red);
-    const float inv = 1.0f / sqrtf(ss / (float)W + eps);
+    __syncthreads();
+    const int last = (int)min(blockDim.x, 256u) / ZF_WAVE - 1;
+    float total = red[0];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) total += w <= last ? red[min(w, last)] : 0.f;
+    const float inv = 1.0f / sqrtf(total / (float)W + eps);
     u = make_float4(u.x * inv * g.x, u.y * inv * g.y, u.z * inv * g.z, u.w * inv * g.w);
   }
   if (!mine) return;
@@ -554,16 +571,27 @@ extern "C" int zf_streams_step(float* x, long long copy_stride, int S, const flo
   const size_t smem = (size_t)W * sizeof(float);
   const bool vec = W % 4 == 0 && copy_stride % 4 == 0 && ((uintptr_t)x % 16) == 0 &&
                    (y0 == nullptr || (uintptr_t)y0 % 16 == 0);
-  // up to four copies of rows of up to 4096 columns: a workgroup as wide as the row
-  const bool one_pass = vec && S <= 4 && W <= 4096 && (uintptr_t)y1 % 16 == 0 &&
+  // Up to four copies of rows of up to 4096 columns: a workgroup as wide as the row, the same bits,
+  // where the rows are written and read, or several copies written: at any number of rows the
+  // faster one (time with 256 threads over time so, 8 to 2048 rows of 512 to 4096 columns: both 0.98
+  // to 2.72, two copies written 0.94 to 1.87, four 1.14 to 2.82).  What only reads, or writes one
+  // copy, has little to ask for at once, and with more workgroups than compute units the wide ones
+  // wait for each other (one copy written, up to 256 rows 1.03 to 1.45, 1000 rows 0.80 to 1.01; read
+  // through the norm 1.05 to 1.24, 0.69 to 1.00, of up to 512 columns 0.98 to 1.22; read as a sum
+  // 1.03 to 1.27, 0.79 to 0.98, of up to 1024 columns 0.89 to 0.96 at any number).
+  const bool wide_pays = y0 != nullptr ? do_read || S > 1 || T <= 256
+                         : gain != nullptr ? T <= 256 || W <= 512
+                                           : T <= 256 && W > 1024;
+  const bool one_pass = vec && wide_pays && S <= 4 && W <= 4096 && (uintptr_t)y1 % 16 == 0 &&
                         (uintptr_t)gain % 16 == 0 && (uintptr_t)out % 16 == 0;
   if (one_pass) {
     const dim3 block((W / 4 + ZF_WAVE - 1) / ZF_WAVE * ZF_WAVE);
+    const size_t rest = gain != nullptr && block.x > 256 ? (block.x - 256) * sizeof(float4) : 0;
     if (out_dtype == ZF_F32)
-      hipLaunchKernelGGL((streams_row_kernel<float, 4>), dim3(T), block, 0, stream, x, copy_stride,
+      hipLaunchKernelGGL((streams_row_kernel<float, 4>), dim3(T), block, rest, stream, x, copy_stride,
                          S, y0, y1, c0, c1, M, b, a, gain, eps, (float*)out, W, do_read);
     else
-      hipLaunchKernelGGL((streams_row_kernel<bf16_t, 4>), dim3(T), block, 0, stream, x, copy_stride,
+      hipLaunchKernelGGL((streams_row_kernel<bf16_t, 4>), dim3(T), block, rest, stream, x, copy_stride,
                          S, y0, y1, c0, c1, M, b, a, gain, eps, (bf16_t*)out, W, do_read);
     ZF_CHECK_LAUNCH();
   }
