@@ -287,6 +287,23 @@ def test_short_convolutions_of_heads_in_pieces(dt, taps, heads, hd, plain):
     assert torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("T", [512, 1024])
+@pytest.mark.parametrize("dt", DTYPES)
+def test_narrow_short_convolutions_take_no_longer_in_pieces(T, dt):
+    """64 channels in heads that a thread's pieces make up, against as many in a head of 48, which keeps
+    the kernel of a thread a channel (in pieces they took up to 1.2 times as long)."""
+    C, times = 64, []
+    K, rows = _rand((C, 4), 21, 0.7).to(DEV), _rand((T, C), 30, 1.0, dt).to(DEV)
+    state = torch.zeros((1, 3 * C), dtype=torch.float32, device=DEV)
+    out = torch.empty((T, C), dtype=dt, device=DEV)
+    slots, index, starts = _i32([0]), _i32([0] * T), _i32([0, T])
+    for heads, hd in ((4, 16), (1, 48)):
+        times.append(graph_us(lambda: ops.short_conv(
+            rows, K, state, 0, slots, index, starts, out, unit_heads=heads, head_dim=hd,
+            scaled_heads=heads // 2, scale=hd ** -0.5, unit_eps=1e-6)))
+    assert times[0] <= 1.06 * times[1], times
+
+
 # ------------------------------------------------------------------------------ the delta rule
 def _delta_inputs(T, H, KH, d, dv, seed):
     C = 2 * KH * d + H * dv

@@ -163,7 +163,7 @@ __global__ __launch_bounds__(DL_CONV_THREADS) void short_conv_kernel(
 // portion.  With a thread a channel that read every row once a tap, 2048 tokens of 4096 channels,
 // half of them in heads of 128, took 87 us, so 25; a decode step's eight tokens 5.3 and 4.8.
 // Grid (blocks of TT tokens, blocks of channels).
-template <typename T, typename TO, int V, int NT>
+template <typename T, typename TO, int V, int NT, bool UNIT>
 __global__ __launch_bounds__(DL_CONV_THREADS) void short_conv_rows_kernel(
     const T* __restrict__ src, long long src_stride, const float* __restrict__ taps, int n_taps,
     const float* __restrict__ bias, float* __restrict__ state, long long state_stride,
@@ -245,7 +245,7 @@ __global__ __launch_bounds__(DL_CONV_THREADS) void short_conv_rows_kernel(
       for (int k = 0; k < NT; ++k) acc[v] = acc[v] + tp[k][v] * w[k][v];
       acc[v] = dl_silu_to<TO>(bias != nullptr ? acc[v] + b[v] : acc[v]);
     }
-    if (c < unit_heads * lph * V) {
+    if (UNIT && c < unit_heads * lph * V) {
       float ss = 0.f;
 #pragma unroll
       for (int v = 0; v < V; ++v) ss += acc[v] * acc[v];
@@ -360,17 +360,25 @@ extern "C" int zf_short_conv(const void* src, int dtype, long long src_stride, c
                     (uintptr_t)taps % 16 == 0 && (uintptr_t)bias % 16 == 0 &&
                     (uintptr_t)state % 16 == 0;
   const int threads = 64;
-  const int TT = single_tokens ? 1 : (T >= 1024 ? 8 : (T >= 256 ? 4 : 2));
+  // (a wave across all channels leaves most of the chip idle, and a head's sum over its lanes is one
+  // more chain a token: 512 tokens of 64 channels four a workgroup 6.9 us, two 5.6, through the other
+  // kernel 6.1; 1024 tokens eight a workgroup 8.7 us, through the other kernel 7.3)
+  const int TT = single_tokens ? 1
+                 : unit_heads > 0 && C <= 64 * V && T < 2048 ? 2
+                 : T >= 1024 ? 8 : T >= 256 ? 4 : 2;
   const dim3 rgrid((T + TT - 1) / TT, (C / V + threads - 1) / threads);
 #define DL_CONV_ROWS(TT_, TO_, V_, N_)                                                            \
-  hipLaunchKernelGGL((short_conv_rows_kernel<TT_, TO_, V_, N_>), rgrid, dim3(threads), 0, stream,\
+  if (unit_heads > 0) DL_CONV_ROWS_OF(TT_, TO_, V_, N_, true);                                   \
+  else DL_CONV_ROWS_OF(TT_, TO_, V_, N_, false)
+#define DL_CONV_ROWS_OF(TT_, TO_, V_, N_, U_)                                                     \
+  hipLaunchKernelGGL((short_conv_rows_kernel<TT_, TO_, V_, N_, U_>), rgrid, dim3(threads), 0, stream,\
                      (const TT_*)src, src_stride, taps, n_taps, bias, state, state_stride,       \
                      state_off, state_slots, seq_index, q_start, (TO_*)out, T, C, TT, single_tokens, \
                      unit_heads, lph, scaled_heads, scale, unit_eps)
 #define DL_CONV_LAUNCH(TT_, TO_, V_)                                                              \
   if (rows) {                                                                                    \
-    if (n_taps <= 4) DL_CONV_ROWS(TT_, TO_, V_, 4);                                              \
-    else DL_CONV_ROWS(TT_, TO_, V_, 8);                                                          \
+    if (n_taps <= 4) { DL_CONV_ROWS(TT_, TO_, V_, 4); }                                          \
+    else { DL_CONV_ROWS(TT_, TO_, V_, 8); }                                                      \
   } else {                                                                                       \
     hipLaunchKernelGGL((short_conv_kernel<TT_, TO_>), grid, dim3(DL_CONV_THREADS), 0, stream,    \
                        (const TT_*)src, src_stride, taps, n_taps, bias, state, state_stride,     \
