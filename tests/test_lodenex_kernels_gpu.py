@@ -12,6 +12,7 @@ import torch
 
 import plain_lodenex as P
 from gpu_util import DEV, rel_err, tol
+from timing import graph_us
 from zinfer_amd import ops
 
 pytestmark = pytest.mark.gpu
@@ -62,8 +63,8 @@ def test_activation_in_the_products_epilogue(M, N, K):
 
 
 def test_activation_of_many_values():
-    """Eight values a thread from 2^20 values on: the bits of the same rows taken one by one."""
-    x = _rand((129, 8192), 5, 3.0, torch.bfloat16).to(DEV)
+    """Eight values a thread from 2^21 values on: the bits of the same rows taken one by one."""
+    x = _rand((257, 8192), 5, 3.0, torch.bfloat16).to(DEV)
     x[3, :4] = torch.tensor([float("inf"), float("-inf"), float("nan"), -0.0])
     for kind in ops.ACTIVATIONS:
         got, want = torch.empty_like(x), torch.empty_like(x)
@@ -71,6 +72,17 @@ def test_activation_of_many_values():
         for i in range(x.shape[0]):
             ops.activation(x[i:i + 1], want[i:i + 1], kind)
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), kind
+
+
+def test_activation_of_a_million_values_takes_no_longer_in_pieces():
+    """2^20 values against eight fewer, which go a value a thread (in pieces they took 1.12 times as
+    long)."""
+    times = []
+    for n in (1 << 20, (1 << 20) - 8):
+        x = _rand((n,), 6, 1.0, torch.bfloat16).to(DEV)
+        out = torch.empty_like(x)
+        times.append(graph_us(lambda: ops.activation(x, out, "gelu_tanh")))
+    assert times[0] <= 1.06 * times[1], times
 
 
 @pytest.mark.parametrize("T, W", [(1, 48), (7, 336), (3, 4096), (2, 8192)])
