@@ -520,6 +520,32 @@ def test_gemm_emit_then_given(M, H, K1, N2, kind):
     assert rel_err(got, want) <= 2.0 ** -7
 
 
+@pytest.mark.parametrize("N", [64, 8192])
+@pytest.mark.parametrize("M", [1, 16])
+def test_weight_streaming_at_every_number_of_blocks(M, N):
+    """None to eight batches of a wave's blocks of 64 of K and every remainder, in some waves and in
+    others: whole numbers, so every sum is exact; stored, added, and behind a norm whose factor is 1."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(M + N)
+    for blocks in (1, 3, 8, 11, 16, 19, 24, 27, 32, 35, 40, 43, 48, 51, 56, 59, 64, 67, 72, 128, 133):
+        K = 64 * blocks
+        a = torch.randint(-3, 4, (M, K), generator=g).float()
+        w = torch.randint(-3, 4, (N, K), generator=g).float()
+        want = a.to(DEV) @ w.to(DEV).T
+        ad, wd = a.bfloat16().to(DEV), w.bfloat16().to(DEV)
+        wt = ops.pretile_weight(wd)
+        out = torch.ones((M, N), device=DEV)
+        ops.gemm(ad, wt, out, accumulate=True, w_tiled=True)
+        assert torch.equal(out, want + 1), K
+        ops.gemm(ad, wt, out, w_tiled=True)
+        assert torch.equal(out, want), K
+        if ops.norm_gemm_plan(M, N, K, wt, True) is not None:
+            sq = torch.full((K // 16, 16), 16.0, device=DEV)
+            out.zero_()
+            ops.gemm_given(ad, sq, 0.0, wt, out)
+            assert torch.equal(out, want), K
+
+
 @pytest.mark.parametrize("K", [64, 1088, 4096, 9216])
 def test_the_order_of_a_given_products_norm_sums(K):
     """The sums of squares a producer left are added in one order, bit for bit: 32 sums a token,

@@ -1737,8 +1737,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
       ssum[0][j][p] = v;
     }
   };
-  // blocks of 64 of K that are this wave's
-  const int cnt = k0 < K ? (K - 1 - k0) / kstride + 1 : 0;
+  // blocks of 64 of K that are this wave's (the same in its lanes: branches on it are scalar)
+  const int cnt = __builtin_amdgcn_readfirstlane(k0 < K ? (K - 1 - k0) / kstride + 1 : 0);
   bool asked = false;                            // (the same in every wave)
   if constexpr (WT && NORM != NORM_FOLD && EPI_GLU(EPI) && RG * MT == 2) {
     // a short K: both blocks of a wave at once (the loop below waits for one before it asks for the
@@ -1825,52 +1825,33 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
     };
     using B0 = std::integral_constant<int, 0>;
     using B1 = std::integral_constant<int, 1>;
-    using One = std::integral_constant<int, 1>;
-    using Two = std::integral_constant<int, 2>;
     using All = std::integral_constant<int, UNR>;
     auto load = [&](auto BUF, int kb) { load_some(BUF, All{}, kb); };
     auto compute = [&](auto BUF) { compute_some(BUF, All{}); };
     // The blocks that make no whole batch come first, in the other register set, with the first
     // batch behind them: their loads are in flight together (one block after the other behind
-    // the batches waited for each: 1024 outputs over K = 3072 5.7 -> 5.2 us).
+    // the batches waited for each: 1024 outputs over K = 3072 5.7 -> 5.2 us).  A path of its own
+    // for every number of them: where paths with and without such blocks meet again the compiler
+    // waits for every load before the second batch is asked for (4096 x 4096, eight tokens 9.1 us
+    // where they did, 8.8 here).
     const int nb = cnt / UNR, rem = cnt % UNR;
-    const int bstride = UNR * kstride, k_rem = k0;
-    k0 += rem * kstride;
-    if (rem == 1) load_some(B1{}, One{}, k_rem);
-    if (UNR > 2 && rem >= 2) load_some(B1{}, Two{}, k_rem);
-    u32x4_t x0[RG], x1[RG], y0[MT], y1[MT];          // a third block
-    if (UNR > 3 && rem == 3) {
-      const int kk = k_rem + 2 * kstride;
-#pragma unroll
-      for (int r = 0; r < RG; ++r) {
-        const bf16_t* tile = wrow[r] + (size_t)(kk / 64) * 1024;
-        x0[r] = __builtin_nontemporal_load((const u32x4_t*)tile);
-        x1[r] = __builtin_nontemporal_load((const u32x4_t*)(tile + 512));
+    const int bstride = UNR * kstride;
+    auto go = [&](auto REM) {
+      constexpr int R = decltype(REM)::value;
+      if constexpr (R > 0) load_some(B1{}, REM, k0);
+      k0 += R * kstride;
+      if (nb == 0) {
+        norm_ask();
+        if constexpr (R > 0) compute_some(B1{}, REM);
+        return;
       }
-#pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        y0[t] = tok[t] ? *(const u32x4_t*)(arow[t] + kk + g * 16) : zero;
-        y1[t] = tok[t] ? *(const u32x4_t*)(arow[t] + kk + g * 16 + 8) : zero;
+      load(B0{}, k0);
+      norm_ask();
+      if constexpr (R > 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        compute_some(B1{}, REM);
+        __builtin_amdgcn_sched_barrier(0);
       }
-    }
-    if (nb > 0) load(B0{}, k0);
-    norm_ask();
-    __builtin_amdgcn_sched_barrier(0);
-    if (rem == 1) compute_some(B1{}, One{});
-    if (UNR > 2 && rem >= 2) compute_some(B1{}, Two{});
-    if (UNR > 3 && rem == 3) {
-#pragma unroll
-      for (int r = 0; r < RG; ++r)
-#pragma unroll
-        for (int t = 0; t < MT; ++t) {
-          acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              *(bf16x8_t*)&x0[r], *(bf16x8_t*)&y0[t], acc[r][t], 0, 0, 0);
-          acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              *(bf16x8_t*)&x1[r], *(bf16x8_t*)&y1[t], acc[r][t], 0, 0, 0);
-        }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    if (nb > 0) {
       int b = 0;
       for (; b + 2 < nb; b += 2) {
         load(B1{}, k0 + (b + 1) * bstride);
@@ -1891,6 +1872,12 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
       } else {
         compute(B0{});
       }
+    };
+    if (rem == 0) go(std::integral_constant<int, 0>{});
+    else if (rem == 1) go(std::integral_constant<int, 1>{});
+    else if constexpr (UNR > 2) {
+      if (rem == 2) go(std::integral_constant<int, 2>{});
+      else go(std::integral_constant<int, 3>{});
     }
     k0 = K;
   }
