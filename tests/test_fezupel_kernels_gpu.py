@@ -399,6 +399,30 @@ def test_pre_tiled_experts_of_a_few_tokens_with_many_pairs(T, W, ff, E, top, act
     assert rel_err(outs[1], outs[0]) < 1e-2
 
 
+@pytest.mark.parametrize("rows", [17, 96, 97, 200])
+@pytest.mark.parametrize("act", [None, "relu2"])
+def test_pre_tiled_experts_of_some_rows_each(rows, act):
+    """Experts with up to 96 rows in the mean take their matrices past the caches, the others not: the
+    same bits as from matrices in rows, spread over the experts and all on one."""
+    W, ff, E, top, dt = 128, 192, 6, 2, torch.bfloat16
+    T = rows * E // top
+    h = _rand((T, W), 34, dtype=dt).to(DEV)
+    gate_up = _rand((E, ff if act else 2 * ff, W), 35, 2 / W ** 0.5, dt).to(DEV)
+    down = _rand((E, W, ff), 36, 2 / ff ** 0.5, dt).to(DEV)
+    tiled = [torch.stack([ops.pretile_weight(m) for m in w]) for w in (gate_up, down)]
+    g = torch.Generator().manual_seed(37)
+    spread = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).to(torch.int32)
+    share = torch.rand((T, top), generator=g).to(DEV)
+    for ids in (spread.to(DEV), torch.full((T, top), 3, dtype=torch.int32, device=DEV)):
+        outs = []
+        for w_tiled, (gu, dn) in ((False, (gate_up, down)), (True, tiled)):
+            y = torch.empty((T, top, ff), dtype=dt, device=DEV)
+            outs.append(torch.empty((T, W), device=DEV))
+            ops.moe_experts(h, gu, dn, ids, share, y, outs[-1], 0.6, 1.702, 1.0, act=act,
+                            w_tiled=w_tiled)
+        assert torch.equal(*outs)
+
+
 @pytest.mark.parametrize("T, W, ff, E, top", [(40, 64, 24, 6, 2), (300, 128, 64, 8, 3),
                                                (17, 72, 136, 1, 1), (150, 352, 104, 40, 4),
                                                (260, 64, 8, 3, 3)])

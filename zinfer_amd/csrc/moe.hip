@@ -1322,8 +1322,10 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float moe_f32x16_t;
 #define MOE_HALF (MOE_NB / 2)
 // MODE 0: the down pass; 1: gate and up with the gated activation; 2: up alone, w [E, N, K], with
 // the plain activation `act`.
-// TILED: every expert's matrices pre-tiled (K a multiple of 64, their rows of 16).
-template <int MODE, bool TILED>
+// TILED: every expert's matrices pre-tiled (K a multiple of 64, their rows of 16).  ONCE: mostly one
+// tile of rows an expert, so that nobody reads the matrices again and their loads need not stay in
+// the caches.
+template <int MODE, bool TILED, bool ONCE>
 __global__ __launch_bounds__(256) void moe_grouped_kernel(
     const bf16_t* __restrict__ a, long long lda, const int* __restrict__ sorted, int top,
     const bf16_t* __restrict__ w, const int* __restrict__ tile_expert,
@@ -1398,8 +1400,12 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
       ra[i] = (ap[i] != nullptr && in_k) ? *(const moe_u32x4_t*)(ap[i] + k0 + sk) : zero;
 #pragma unroll
     for (int i = 0; i < 2 * MOE_NB; ++i)
-      rb[i] = (bp[i] != nullptr && (TILED || in_k))
-          ? *(const moe_u32x4_t*)(bp[i] + (TILED ? (size_t)k0 * 16 : (size_t)k0)) : zero;
+      if (bp[i] == nullptr || !(TILED || in_k))
+        rb[i] = zero;
+      else if constexpr (ONCE)
+        rb[i] = few_load_w(bp[i] + (size_t)k0 * 16);
+      else
+        rb[i] = *(const moe_u32x4_t*)(bp[i] + (TILED ? (size_t)k0 * 16 : (size_t)k0));
   };
   fetch(0);
   for (int k0 = 0; k0 < K; k0 += MOE_BK) {
@@ -1460,6 +1466,7 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
 // mode 1: a = h [T, K] (rows gathered), w = gate_up [E, 2 N, K], out = y bfloat16 [P, N];
 // mode 2: the same with w = up [E, N, K] and the plain activation `act`;
 // mode 0: a = y [P, K], w = down [E, N, K], out = o float32 [P, N].  K a multiple of 8.
+// w_tiled 1: matrices pre-tiled; 2: and mostly read once (ONCE above).
 extern "C" int zf_moe_grouped(const void* a, long long lda, const int* sorted, int top,
                               const void* w, const int* tile_expert, const int* tile_row0,
                               const int* tile_rows, const int* n_tiles, void* out, int max_tiles,
@@ -1471,9 +1478,11 @@ extern "C" int zf_moe_grouped(const void* a, long long lda, const int* sorted, i
     return -2;
   max_tiles = (max_tiles + 7) / 8 * 8;
 #define MOE_GROUPED_LAUNCH(MODE, COLS)                                                           \
-  if (w_tiled) MOE_GROUPED_LAUNCH_AS(MODE, true, COLS); else MOE_GROUPED_LAUNCH_AS(MODE, false, COLS)
-#define MOE_GROUPED_LAUNCH_AS(MODE, TILED, COLS)                                                 \
-  hipLaunchKernelGGL((moe_grouped_kernel<MODE, TILED>), dim3(max_tiles, (N + (COLS) - 1) / (COLS)), \
+  if (w_tiled == 2) MOE_GROUPED_LAUNCH_AS(MODE, true, true, COLS);                               \
+  else if (w_tiled) MOE_GROUPED_LAUNCH_AS(MODE, true, false, COLS);                              \
+  else MOE_GROUPED_LAUNCH_AS(MODE, false, false, COLS)
+#define MOE_GROUPED_LAUNCH_AS(MODE, TILED, ONCE, COLS)                                           \
+  hipLaunchKernelGGL((moe_grouped_kernel<MODE, TILED, ONCE>), dim3(max_tiles, (N + (COLS) - 1) / (COLS)), \
                      dim3(256), 0, stream, (const bf16_t*)a, lda, sorted, top, (const bf16_t*)w, \
                      tile_expert, tile_row0, tile_rows, n_tiles, out, N, K, limit, alpha, shift, \
                      act, n_experts)

@@ -2150,14 +2150,19 @@ def moe_grouped(h, gate_up, down, ids, weights, y, out, limit, alpha, shift, add
                            _ptr(tile_row0), _ptr(tile_rows), _ptr(n_tiles), st), "moe_sort")
     lim, al, sh = ctypes.c_float(limit), ctypes.c_float(alpha), ctypes.c_float(shift)
     kind = ACTIVATIONS[act] if act is not None else 0
+    # Pre-tiled matrices of experts with up to 96 rows in the mean, one tile of rows as a rule, come by
+    # loads that pass the caches (us, with them and without: 64 experts of 4096 x 1024, 8 a token,
+    # 128 tokens 347 and 370, 300 tokens 387 and 408, row by row 360 and 376; 8 of 4096 x 2048, 4 a
+    # token, 128 tokens 137 and 145); more rows share what the caches hold (2048 tokens 1080 and
+    # 1020; 16 of 2048 x 2048, 175 rows each, 209 and 189).
+    layout = 0 if not w_tiled else 2 if P <= 96 * E else 1
     _check(lib.zf_moe_grouped(_ptr(h), ctypes.c_longlong(W), _ptr(sorted_), top, _ptr(gate_up),
                               _ptr(tile_expert), _ptr(tile_row0), _ptr(tile_rows), _ptr(n_tiles),
                               _ptr(y), max_tiles, ff, W, 2 if act is not None else 1, lim, al, sh,
-                              kind, E, 1 if w_tiled else 0, st), "moe_grouped (gate, up)")
+                              kind, E, layout, st), "moe_grouped (gate, up)")
     _check(lib.zf_moe_grouped(_ptr(y), ctypes.c_longlong(ff), _ptr(sorted_), top, _ptr(down),
                               _ptr(tile_expert), _ptr(tile_row0), _ptr(tile_rows), _ptr(n_tiles),
-                              _ptr(o), max_tiles, W, ff, 0, lim, al, sh, 0, E, 1 if w_tiled else 0,
-                              st),
+                              _ptr(o), max_tiles, W, ff, 0, lim, al, sh, 0, E, layout, st),
            "moe_grouped (down)")
     _check(lib.zf_moe_combine(_ptr(o), _ptr(place), _ptr(weights), _ptr(out), T, W, top,
                               1 if add else 0, _ptr(ids) if n_identity else None, E,
