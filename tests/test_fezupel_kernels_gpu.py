@@ -399,6 +399,38 @@ def test_pre_tiled_experts_of_a_few_tokens_with_many_pairs(T, W, ff, E, top, act
     assert rel_err(outs[1], outs[0]) < 1e-2
 
 
+@pytest.mark.parametrize("W, ff, top", [(4096, 1024, 8), (1024, 4096, 4)])
+def test_experts_of_a_few_tokens_are_as_close_pre_tiled(W, ff, top):
+    """Pre-tiled against row by row, both against 64 bits: the outputs from the activations that either
+    left, and how many of the activations are not the rounding of the 64-bit ones."""
+    E, T, dt = 8, 16, torch.bfloat16
+    h = _rand((T, W), 41, dtype=dt).to(DEV)
+    gate_up = _rand((E, 2 * ff, W), 42, W ** -0.5, dt).to(DEV)
+    down = _rand((E, W, ff), 43, ff ** -0.5, dt).to(DEV)
+    g = torch.Generator().manual_seed(44)
+    ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).to(torch.int32).to(DEV)
+    share = torch.rand((T, top), generator=g).to(DEV)
+    tiled = [torch.stack([ops.pretile_weight(m) for m in w]) for w in (gate_up, down)]
+    off, other = [], []
+    for w_tiled, (gu, dn) in ((False, (gate_up, down)), (True, tiled)):
+        y = torch.empty((T, top, ff), dtype=dt, device=DEV)
+        out = torch.empty((T, W), device=DEV)
+        ops.moe_experts(h, gu, dn, ids, share, y, out, 0.0, 1.0, 0.0, w_tiled=w_tiled)
+        want, wrong = torch.zeros((T, W), dtype=torch.float64, device=DEV), 0
+        for t in range(T):
+            for s_ in range(top):
+                e = int(ids[t, s_])
+                z = gate_up[e].double() @ h[t].double()
+                z = z[:ff] * torch.sigmoid(z[:ff]) * z[ff:]
+                wrong += int((z.to(dt) != y[t, s_]).sum())
+                want[t] += share[t, s_].double() * (down[e].double() @ y[t, s_].double())
+        off.append(float((out.double() - want).norm() / want.norm()))
+        other.append(wrong)
+    # (16384 outputs and more; some 20 of 131072 activations lie that close to a tie)
+    assert off[1] <= 1.04 * off[0], off
+    assert other[1] <= 1.5 * other[0] + 8, other
+
+
 @pytest.mark.parametrize("rows", [17, 96, 97, 200])
 @pytest.mark.parametrize("act", [None, "relu2"])
 def test_pre_tiled_experts_of_some_rows_each(rows, act):

@@ -940,8 +940,8 @@ extern "C" int zf_gated_act(const void* gu, void* out, int dtype, int T, int ff,
 //                    pairs, piece of ff) after piece by each wave.  The 16 rows and columns of an
 //                    MFMA are 8 outputs and 8 pairs at two neighbouring blocks of 64 of ff: only
 //                    the products of like halves are used, and 2048 outputs make 256 workgroups.
-//                    Partials in LDS, added per pair in order of the pieces, per token in slot
-//                    order, the shared expert last.  (Fetching the next piece's operands before a
+//                    Partials in LDS, added per pair every fourth piece side by side, per token
+//                    in slot order, the shared expert last.  (Fetching the next piece's operands before a
 //                    piece's products was no faster; a workgroup per unit and 32 outputs whose last
 //                    one to arrive adds the sums took 10 % less at W = 4096, 64 experts and 8
 //                    tokens, 15 % more at 16 tokens, and more in the decode step.)
@@ -998,6 +998,21 @@ __device__ __forceinline__ bool few_columns(const int* __restrict__ ids, int P, 
   return true;
 }
 
+// n (even) numbers, eight apart: four sums side by side, added in pairs
+__device__ __forceinline__ float few_sum(const float* p, int n) {
+  float a[4] = {0.f, 0.f, 0.f, 0.f};
+  int q = 0;
+#pragma unroll 4
+  for (; q + 4 <= n; q += 4)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] += p[8 * (q + i)];
+  if (q < n) {
+    a[0] += p[8 * q];
+    a[1] += p[8 * q + 8];
+  }
+  return (a[0] + a[1]) + (a[2] + a[3]);
+}
+
 template <bool GATED>
 __global__ __launch_bounds__(256) void moe_few_up_kernel(
     const bf16_t* __restrict__ h, const bf16_t* __restrict__ w, const int* __restrict__ ids,
@@ -1031,9 +1046,17 @@ __global__ __launch_bounds__(256) void moe_few_up_kernel(
   wg += lane * 8;
   wu += lane * 8;
   const bf16_t* x = h + (size_t)token * W + 16 * g;
-  moe_f32x4_t ag = {0.f, 0.f, 0.f, 0.f}, au = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int kb = wave; kb < blocks; kb += 4) {
+  // Four sums side by side, of either half of even and odd blocks, closed every four blocks: one sum
+  // over a wave's whole share of K is further off than the lane sums of the row-by-row kernel
+  // (4096 columns, of the activations 0.043 % rounded the other way than the 64-bit ones, so 0.016
+  // %, row by row 0.017 %).
+  moe_f32x4_t sg[2][2], su[2][2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) sg[j][i] = su[j][i] = moe_f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto take = [&](auto J, int kb) {
+    constexpr int j = decltype(J)::value;
     moe_u32x4_t xf[2], gf[2], uf[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -1043,22 +1066,37 @@ __global__ __launch_bounds__(256) void moe_few_up_kernel(
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      ag = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&gf[i],
-                                                   *(const moe_bf16x8_t*)&xf[i], ag, 0, 0, 0);
+      sg[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&gf[i],
+                                                         *(const moe_bf16x8_t*)&xf[i], sg[j][i], 0, 0, 0);
       if constexpr (GATED)
-        au = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&uf[i],
-                                                     *(const moe_bf16x8_t*)&xf[i], au, 0, 0, 0);
+        su[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&uf[i],
+                                                           *(const moe_bf16x8_t*)&xf[i], su[j][i], 0, 0, 0);
     }
+  };
+  int kb = wave;
+  moe_f32x4_t ag = {0.f, 0.f, 0.f, 0.f}, au = ag;
+  auto close = [&]() {
+    ag += (sg[0][0] + sg[0][1]) + (sg[1][0] + sg[1][1]);
+    if constexpr (GATED) au += (su[0][0] + su[0][1]) + (su[1][0] + su[1][1]);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) sg[j][i] = su[j][i] = moe_f32x4_t{0.f, 0.f, 0.f, 0.f};
+  };
+#pragma unroll 1
+  for (; kb + 4 < blocks; kb += 8) {
+    take(std::integral_constant<int, 0>{}, kb);
+    take(std::integral_constant<int, 1>{}, kb + 4);
+    if (kb & 8) close();
   }
+  if (kb < blocks) take(std::integral_constant<int, 0>{}, kb);
+  close();
   part[wave][0][lane] = ag;
   part[wave][1][lane] = au;
   __syncthreads();
   if (wave != 0 || pair < 0) return;
-#pragma unroll
-  for (int s = 1; s < 4; ++s) {
-    ag += part[s][0][lane];
-    au += part[s][1][lane];
-  }
+  ag = (ag + part[1][0][lane]) + (part[2][0][lane] + part[3][0][lane]);
+  au = (au + part[1][1][lane]) + (part[2][1][lane] + part[3][1][lane]);
   // column r is the pair, the four numbers are outputs j0 + 4 g + i
   const float f = shared && factor != nullptr ? factor[(size_t)pair * factor_stride] : 1.0f;
   uint32_t v[4];
@@ -1139,6 +1177,8 @@ __global__ __launch_bounds__(1024) void moe_few_down_kernel(
     const int nb = shared ? s_blocks : blocks;
     int pair;
     const bf16_t *wr, *x;
+    // (the two halves of the blocks in a sum each, the pieces' sums four side by side: the outputs of ff
+    // = 4096 from given activations 1.34e-7 off with one sum, 1.04e-7 so, 1.05e-7 row by row)
     // rows r and columns r: output n0 + r % 8 and pair r % 8 at the blocks 2 i + r / 8
     for (int p0 = 0; p0 < (shared ? T : 8); p0 += 8) {
       if (shared) {
@@ -1153,7 +1193,7 @@ __global__ __launch_bounds__(1024) void moe_few_down_kernel(
       wr += (size_t)(n0 / 16) * nb * 1024 + (g * 16 + n0 % 16 + r % 8) * 8;
       x += 16 * g;
       const int b0 = c * 2 * piece, b1 = min(nb, b0 + 2 * piece);
-      moe_f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+      moe_f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll 4
       for (int kb = b0; kb < b1; kb += 2) {
         // (behind an odd last block the upper half repeats it against zeros)
@@ -1168,14 +1208,14 @@ __global__ __launch_bounds__(1024) void moe_few_down_kernel(
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&wf[i],
-                                                        *(const moe_bf16x8_t*)&xf[i], acc, 0, 0, 0);
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&wf[i],
+                                                           *(const moe_bf16x8_t*)&xf[i], acc[i], 0, 0, 0);
       }
       // rows 4 g + i of column r: like halves are g / 2 == half
       if (pair >= 0 && g / 2 == half)
         *(moe_f32x4_t*)((shared ? s_sums + ((size_t)pair * s_pieces + c) * 16
                                 : sums + ((size_t)pair * pieces + c) * 16) + 8 * half + 4 * (g % 2)) =
-            acc;
+            acc[0] + acc[1];
     }
   }
   __syncthreads();
@@ -1188,17 +1228,11 @@ __global__ __launch_bounds__(1024) void moe_few_down_kernel(
       same = fmaf(c, bf16_to_float(h[(size_t)t * W + n0 + n]), same);
       continue;
     }
-    float dot = 0.f;
-    for (int q = 0; q < 2 * pieces; ++q) dot += sums[((size_t)ts * 2 * pieces + q) * 8 + n];
-    total = fmaf(c, dot, total);
+    total = fmaf(c, few_sum(sums + (size_t)ts * pieces * 16 + n, 2 * pieces), total);
   }
   total += same;
   if (add) total += before;
-  if (s_pieces > 0) {
-    float dot = 0.f;
-    for (int q = 0; q < 2 * s_pieces; ++q) dot += s_sums[((size_t)t * 2 * s_pieces + q) * 8 + n];
-    total += dot;
-  }
+  if (s_pieces > 0) total += few_sum(s_sums + (size_t)t * s_pieces * 16 + n, 2 * s_pieces);
   out[(size_t)t * W + n0 + n] = total;
 }
 
