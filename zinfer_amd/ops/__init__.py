@@ -2002,8 +2002,9 @@ def moe_pretile_pays(width: int, ff: int, top: int, shared: bool) -> bool:
     pre-tiled over time row by row, (least, most): with a shared expert W = 1024 (0.63, 1.27), 1536
     (0.61, 1.14), 2048 (0.56, 0.97 from ff = 512 on; ff = 256 1.08), 3072 (0.59, 1.02), 4096 (0.54,
     0.97); without W = 256, ff = 128 (0.85, 2.70), 1024 x 512 (1.00, 1.46), 2048 x 768 (0.71, 1.24),
-    and from four a token on 2048 x 2048 (0.60, 0.98), 4096 x 1024 (0.54, 1.02), 3072 x 2048 (0.62,
-    1.04); 16 and 32 a token 0.25 to 0.97."""
+    and from four a token on 2048 x 2048 (0.50, 0.94), 4096 x 1024 (0.48, 1.02), 3072 x 2048 (0.62,
+    1.04), but for two tokens of 32 experts and more (1.09 to 1.14, against 0.66 to 0.77 for
+    sixteen); 16 and 32 a token 0.25 to 0.97."""
     if shared:
         return width >= 2048 and ff >= 512
     return top >= 4 and width * ff >= (4 << 20 if width % 2048 == 0 else 8 << 20)
