@@ -1113,6 +1113,39 @@ def test_gather_rows_and_argmax():
     assert got[0].item() == 17
 
 
+@pytest.mark.parametrize("T,H", [(1, 64), (16, 1024), (3, 1088), (5, 2064), (16, 5120)])
+@pytest.mark.parametrize("source", ["embed", "embed32", "gather"])
+def test_picked_rows_leave_the_norm_s_inputs(T, H, source):
+    """The rows are what they are without the norm's inputs, bit for bit; xg is their product with
+    the gain, rounded once; a sum of 16 squares differs by the rounding of 31 operations."""
+    table = _rand((40, H), torch.float32 if source != "embed" else torch.bfloat16, 3)
+    gain = _rand((H,), torch.float32, 4) + 1.0
+    ids = torch.randint(0, 40, (T,), generator=torch.Generator().manual_seed(5)).int()
+    rows, plain = torch.empty((T, H), device=DEV), torch.empty((T, H), device=DEV)
+    xg = torch.empty((T, H), dtype=torch.bfloat16, device=DEV)
+    sq = torch.full((H // 16, 16), float("nan"), device=DEV)
+    args = (gain.to(DEV), xg, sq)
+    if source == "gather":
+        want = table[ids.long()]
+        _ops().gather_rows(table.to(DEV), ids.to(DEV), rows, given=args)
+        _ops().gather_rows(table.to(DEV), ids.to(DEV), plain)
+    else:
+        want = table[ids.long()].float() * 0.75
+        _ops().embed(table.to(DEV), ids.to(DEV), rows, 0.75, given=args)
+        _ops().embed(table.to(DEV), ids.to(DEV), plain, 0.75)
+    assert torch.equal(rows.cpu(), want) and torch.equal(plain, rows)
+    assert torch.equal(xg.cpu(), (want * gain).to(torch.bfloat16))
+    sums = want.double().view(T, H // 16, 16).square().sum(-1).T
+    assert torch.allclose(sq.cpu()[:, :T].double(), sums, rtol=31 * 2.0 ** -24, atol=0.0)
+
+
+def test_embed_of_a_width_without_whole_pieces():
+    table, ids = _rand((9, 130), torch.bfloat16, 6), torch.tensor([8, 0, 3], dtype=torch.int32)
+    out = torch.empty((3, 130), device=DEV)
+    _ops().embed(table.to(DEV), ids.to(DEV), out, 2.0)
+    assert torch.equal(out.cpu(), table[ids.long()].float() * 2.0)
+
+
 def test_cpu_tensor_is_refused():
     """There is no CPU path: a tensor that is not on the GPU is an error, not a fallback."""
     from zinfer_amd.errors import KernelUnavailable

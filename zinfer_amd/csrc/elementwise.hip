@@ -17,10 +17,76 @@ __global__ void embed_kernel(const TW* __restrict__ table, const int* __restrict
   for (int i = threadIdx.x; i < H; i += blockDim.x) o[i] = load_as_float<TW>(row + i) * scale;
 }
 
+// four values of a row that begins on a 4-value boundary
+template <typename TW> __device__ __forceinline__ float4 load_four(const TW* p);
+template <> __device__ __forceinline__ float4 load_four<float>(const float* p) {
+  return *(const float4*)p;
+}
+template <> __device__ __forceinline__ float4 load_four<bf16_t>(const bf16_t* p) {
+  const uint2 u = *(const uint2*)p;
+  return float4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u),
+                __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xffff0000u)};
+}
+
+// Rows picked from a table, out[t] = table[ids[t]] * scale in 32-bit, four columns a thread
+// (H a multiple of 4, 16-byte aligned rows).  GIVEN: and what the weight-streaming product
+// that norms these rows takes, as gemm_emit leaves it: xg = bfloat16(out * gain) and the sums of
+// squares of 16 columns, sq [H / 16][16 tokens] (H a multiple of 16, up to 16 tokens).
+// Without it that product folds the norm in, and every workgroup reads the 32-bit rows and the
+// gains again: 5120 wide into 151936 outputs, 16 tokens 329 us for 229, into 7168 17.1 for 14.0.
+// The kernel itself is bound by latency at a few rows and by memory from some hundred on (8191
+// rows of 5120: 82 us with a value a thread, 250 MB).
+template <typename TW, bool GIVEN>
+__global__ __launch_bounds__(256) void pick_rows_kernel(
+    const TW* __restrict__ table, const int* __restrict__ ids, float* __restrict__ out, int H,
+    float scale, const float* __restrict__ gain, bf16_t* __restrict__ xg, float* __restrict__ sq) {
+  const int t = blockIdx.x, i = 4 * (blockIdx.y * 256 + threadIdx.x);
+  if (i >= H) return;
+  float4 g = float4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (GIVEN) g = *(const float4*)(gain + i);
+  float4 v = load_four<TW>(table + (size_t)ids[t] * H + i);
+  v.x *= scale; v.y *= scale; v.z *= scale; v.w *= scale;
+  const size_t off = (size_t)t * H + i;
+  *(float4*)(out + off) = v;
+  if constexpr (GIVEN) {
+    *(uint2*)(xg + off) = uint2{pack_bf16x2(v.x * g.x, v.y * g.y), pack_bf16x2(v.z * g.z, v.w * g.w)};
+    // (whole groups of four lanes are here: H is a multiple of 16)
+    const float s = lanes_sum<4>(v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w);
+    if (threadIdx.x % 4 == 0) sq[(size_t)(i / 16) * 16 + t] = s;
+  }
+}
+
+// gain null: rows alone
+template <typename TW>
+static void launch_pick_rows(const TW* table, const int* ids, float* out, int T, int H, float scale,
+                             const float* gain, bf16_t* xg, float* sq, hipStream_t stream) {
+  const dim3 grid(T, (H + 1023) / 1024);
+  if (gain != nullptr)
+    hipLaunchKernelGGL((pick_rows_kernel<TW, true>), grid, dim3(256), 0, stream, table, ids, out, H,
+                       scale, gain, xg, sq);
+  else
+    hipLaunchKernelGGL((pick_rows_kernel<TW, false>), grid, dim3(256), 0, stream, table, ids, out, H,
+                       scale, nullptr, nullptr, nullptr);
+}
+
+// what every row and every vector of a given norm needs to be read in pieces of four values
+static bool picks_in_fours(const void* table, const void* out, const void* gain, const void* xg,
+                           int H) {
+  return H % 4 == 0 && ((uintptr_t)table | (uintptr_t)out | (uintptr_t)gain | (uintptr_t)xg) % 16 == 0;
+}
+
+// gain, xg and sq null: the rows alone; else up to 16 rows of a multiple of 16
 extern "C" int zf_embed(const void* table, int table_dtype, const int* ids, float* out, int T,
-                        int H, float scale, hipStream_t stream) {
+                        int H, float scale, const float* gain, void* xg, float* sq,
+                        hipStream_t stream) {
   if (T <= 0) return 0;
-  if (table_dtype == ZF_F32)
+  const bool fours = picks_in_fours(table, out, gain, xg, H);
+  if (gain != nullptr && !(fours && H % 16 == 0 && T <= 16)) return -1;
+  if (fours && table_dtype == ZF_F32)
+    launch_pick_rows((const float*)table, ids, out, T, H, scale, gain, (bf16_t*)xg, sq, stream);
+  else if (fours)
+    launch_pick_rows((const bf16_t*)table, ids, out, T, H, scale, gain, (bf16_t*)xg, sq, stream);
+  else if (table_dtype == ZF_F32)
     hipLaunchKernelGGL(embed_kernel<float>, dim3(T), dim3(256), 0, stream, (const float*)table,
                        ids, out, H, scale);
   else
@@ -797,10 +863,16 @@ __global__ void gather_rows_kernel(const float* __restrict__ x, const int* __res
   for (int i = threadIdx.x; i < H; i += blockDim.x) o[i] = row[i];
 }
 
+// gain, xg and sq as zf_embed's
 extern "C" int zf_gather_rows(const float* x, const int* idx, float* out, int n, int H,
-                              hipStream_t stream) {
+                              const float* gain, void* xg, float* sq, hipStream_t stream) {
   if (n <= 0) return 0;
-  hipLaunchKernelGGL(gather_rows_kernel, dim3(n), dim3(256), 0, stream, x, idx, out, H);
+  const bool fours = picks_in_fours(x, out, gain, xg, H);
+  if (gain != nullptr && !(fours && H % 16 == 0 && n <= 16)) return -1;
+  if (gain != nullptr)
+    launch_pick_rows(x, idx, out, n, H, 1.0f, gain, (bf16_t*)xg, sq, stream);
+  else
+    hipLaunchKernelGGL(gather_rows_kernel, dim3(n), dim3(256), 0, stream, x, idx, out, H);
   ZF_CHECK_LAUNCH();
 }
 

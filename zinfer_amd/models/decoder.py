@@ -12,6 +12,7 @@ from .. import ops
 from ..config.specs import ModelSpec
 from ..errors import ConfigError
 from ..parts import BuildContext, TensorDecl, build_part
+from ..parts.base import Norm
 from ..parts.block import NormedRows
 from ..parts.linear import Linear, place_matrix
 
@@ -144,6 +145,14 @@ class DecoderModel:
         ops.streams_step(copies, read=True, out=total)
         return total
 
+    @staticmethod
+    def _pick(norm, rows: torch.Tensor, step, pick):
+        """Runs ``pick``, which picks ``rows`` from a table, and has it leave what ``norm``, which
+        reads them next, can use; returns that, or None."""
+        left = norm.picked(rows, step) if isinstance(norm, Norm) else None
+        pick(**({} if left is None else {"given": left.buffers}))
+        return left
+
     # ---------------------------------------------------------------- forward
     def forward(self, step, caches) -> torch.Tensor:
         """Runs the tokens of ``step`` and returns float32 logits [len(step.want_rows), V].
@@ -175,7 +184,12 @@ class DecoderModel:
             ops.embed_sinusoid(self.embedding, step.token_ids, step.positions,
                                self.position_freq, x, float(s.embedding_multiplier))
         else:
-            ops.embed(self.embedding, step.token_ids, x, float(s.embedding_multiplier))
+            # and what the first block's norm needs of few rows, in the same kernel
+            first = None if self.reentry is not None or copies is not None else \
+                getattr(self.blocks[s.schedule[0].layer], "entry_norm", None)
+            step.norm_ready = self._pick(
+                first, x, step, lambda **given: ops.embed(
+                    self.embedding, step.token_ids, x, float(s.embedding_multiplier), **given))
         x0 = None
         if self.reentry is not None:
             # the stream as the embedding left it, for the runs that re-enter it
@@ -214,9 +228,9 @@ class DecoderModel:
         if step.wants_all_rows:
             rows = x
         else:
-            left = None
             rows = step.scratch("want_rows", (n_rows, s.hidden_size), torch.float32)
-            ops.gather_rows(x, step.want_rows, rows)
+            left = self._pick(self.final_norm, rows, step,
+                              lambda **given: ops.gather_rows(x, step.want_rows, rows, **given))
         make = lambda: step.scratch("final_normed", (n_rows, s.hidden_size), self.ctx.act_dtype)
         with ops.kernel_class("head_sampling"):      # what a per-class measurement counts these as
             if isinstance(left, NormedRows) and left.fits(self.final_norm, rows):

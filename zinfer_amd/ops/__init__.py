@@ -130,18 +130,36 @@ def _launches(cls: str):
 
 
 # ------------------------------------------------------------------------- elementwise
+def _check_given(given, rows: torch.Tensor) -> None:
+    """``given`` = (gain, xg, sq) of the float32 ``rows``, or None."""
+    if given is None:
+        return
+    T, H = rows.shape
+    gain, xg, sq = given
+    if not (T <= NORM_FOLD_MAX_M and H % 16 == 0 and gain.dtype == torch.float32 and gain.shape == (H,)
+            and xg.dtype == torch.bfloat16 and xg.shape == (T, H) and sq.dtype == torch.float32
+            and sq.shape == (H // 16, 16)
+            and all(t.is_contiguous() for t in (rows, gain, xg, sq))):
+        raise KernelUnavailable(f"a norm's inputs beside the rows: gain {tuple(gain.shape)}, "
+                                f"xg {tuple(xg.shape)}, sq {tuple(sq.shape)} for {tuple(rows.shape)}")
+
+
 @_launches("other")
-def embed(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, scale: float = 1.0) -> None:
-    """out[t, :] = table[ids[t], :] widened to float32, times ``scale``."""
-    _need_gpu(table, ids, out)
+def embed(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, scale: float = 1.0,
+          given: Optional[Tuple[torch.Tensor, torch.Tensor, torch.Tensor]] = None) -> None:
+    """out[t, :] = table[ids[t], :] widened to float32, times ``scale``.  ``given`` (gain, xg, sq):
+    also what ``gemm_given`` takes of these rows, as ``gemm_emit`` leaves it (up to 16 rows)."""
+    _need_gpu(table, ids, out, *(given or ()))
     _i32(ids, "ids")
     T, H = out.shape
+    _check_given(given, out)
     if table.shape[1] != H or ids.shape[0] != T or out.dtype != torch.float32:
         raise KernelUnavailable(f"embed: table {tuple(table.shape)}, ids {tuple(ids.shape)}, "
                                 f"out {tuple(out.shape)} {out.dtype}")
     lib = build.load("elementwise")
     _check(lib.zf_embed(_ptr(table), _dt(table), _ptr(ids), _ptr(out), T, H,
-                        ctypes.c_float(scale), _stream()), "embed")
+                        ctypes.c_float(scale), *(_ptr(t) for t in given or (None,) * 3),
+                        _stream()), "embed")
 
 
 @_launches("other")
@@ -300,14 +318,18 @@ def poison_pages(pool: torch.Tensor, pages: torch.Tensor) -> None:
 
 
 @_launches("head_sampling")
-def gather_rows(x: torch.Tensor, idx: torch.Tensor, out: torch.Tensor) -> None:
-    _need_gpu(x, idx, out)
+def gather_rows(x: torch.Tensor, idx: torch.Tensor, out: torch.Tensor,
+                given: Optional[Tuple[torch.Tensor, torch.Tensor, torch.Tensor]] = None) -> None:
+    """out[i, :] = x[idx[i], :]; ``given`` as ``embed``'s."""
+    _need_gpu(x, idx, out, *(given or ()))
     _i32(idx, "idx")
     n, H = out.shape
+    _check_given(given, out)
     if x.shape[1] != H or idx.shape[0] != n or x.dtype != torch.float32 or out.dtype != x.dtype:
         raise KernelUnavailable("gather_rows: float32 [T, H] -> [n, H]")
     lib = build.load("elementwise")
-    _check(lib.zf_gather_rows(_ptr(x), _ptr(idx), _ptr(out), n, H, _stream()), "gather_rows")
+    _check(lib.zf_gather_rows(_ptr(x), _ptr(idx), _ptr(out), n, H,
+                              *(_ptr(t) for t in given or (None,) * 3), _stream()), "gather_rows")
 
 
 @_launches("head_sampling")

@@ -176,13 +176,16 @@ class Part:
 
 class Norm(Part):
     """A norm may let the products next to it do part of its work.  Both ways are optional and
-    safe to leave out; the generic block and decoder only ever call these three methods.
+    safe to leave out; the generic block and decoder only ever call these four methods.
 
     * ``deferred(x, make_out, left)``: a stand-in for the norm's output on the rows ``x`` for a
       consumer that says ``accepts_lazy_norm``: an object with ``shape``, ``materialize()``
       (runs the norm once, returns the activations) and ``fold_into(linear, out, **kw)`` (the
       product of the normed rows with ``linear``'s weight in one kernel, or False).  None:
       the norm simply runs.  ``left``: what ``residual_sum`` left for this norm, or None.
+    * ``picked(x, step)``: for rows ``x`` about to be picked from a table (an embedding, the rows
+      whose logits are wanted): an object whose ``buffers`` the kernel that picks them also
+      writes, and which then is what ``residual_sum`` leaves.  None: nothing beside the rows.
     * ``residual_sum(linear, a, out, step)``: out += a W^T in a kernel that also leaves
       something for this norm, which reads ``out`` next; puts it in ``step.norm_ready`` and
       returns True, or returns False and does nothing."""
@@ -195,6 +198,9 @@ class Norm(Part):
         raise NotImplementedError
 
     def deferred(self, x: torch.Tensor, make_out, left=None):
+        return None
+
+    def picked(self, x: torch.Tensor, step):
         return None
 
     def residual_sum(self, linear, a: torch.Tensor, out: torch.Tensor, step) -> bool:

@@ -39,13 +39,22 @@ class RmsNorm(Norm):
         given = left if left is not None and left.fits(self, x) else None
         return LazyRmsNorm(self, x, make_out, given)
 
+    def picked(self, x: torch.Tensor, step):
+        if not (x.is_cuda and self.ctx.compute_dtype == torch.bfloat16
+                and x.shape[0] <= ops.NORM_FOLD_MAX_M and x.shape[1] % 64 == 0):
+            return None
+        return GivenRmsNorm(self, x, *self._given_buffers(x, step))
+
+    def _given_buffers(self, out: torch.Tensor, step):
+        return (step.scratch("normed_by_gain", out.shape, torch.bfloat16),
+                step.scratch("normed_squares", (out.shape[1] // 16, 16), torch.float32))
+
     def residual_sum(self, linear, a: torch.Tensor, out: torch.Tensor, step) -> bool:
         if a.dtype != torch.bfloat16:
             return False
         M, N, K = a.shape[0], linear.out_features, linear.in_features
         if ops.norm_emit_plan(M, N, K, linear.weight, linear.tiled) is not None:
-            xg = step.scratch("normed_by_gain", out.shape, torch.bfloat16)
-            sq = step.scratch("normed_squares", (N // 16, 16), torch.float32)
+            xg, sq = self._given_buffers(out, step)
             ops.gemm_emit(a, linear.weight, out, self.gain, xg, sq)
             step.norm_ready = GivenRmsNorm(self, out, xg, sq)
             return True
@@ -58,12 +67,17 @@ class RmsNorm(Norm):
 
 
 class GivenRmsNorm:
-    """What the kernel that last added into the residual rows ``x`` left for ``norm``:
-    xg = bfloat16(x * gain) and sq [width / 16, 16], the sums of x^2 over each 16 columns per
-    token (``ops.gemm_emit``)."""
+    """What the kernel that last added into the residual rows ``x``, or picked them from a table,
+    left for ``norm``: xg = bfloat16(x * gain) and sq [width / 16, 16], the sums of x^2 over each
+    16 columns per token (``ops.gemm_emit``)."""
 
     def __init__(self, norm: "RmsNorm", x: torch.Tensor, xg: torch.Tensor, sq: torch.Tensor):
         self.norm, self.x, self.xg, self.sq = norm, x, xg, sq
+
+    @property
+    def buffers(self):
+        """What the kernels that leave it write it with: ``given`` of ``ops.embed``."""
+        return self.norm.gain, self.xg, self.sq
 
     def fits(self, norm, x: torch.Tensor) -> bool:
         return self.norm is norm and self.x.data_ptr() == x.data_ptr() and self.x.shape == x.shape
