@@ -717,6 +717,30 @@ def test_wave_attention_vector_loads_give_the_same_bits(hd, page_size, window, d
     assert torch.equal(other, got)
 
 
+@pytest.mark.parametrize("nH,nKV,hd,page_size", [(4, 2, 64, 16), (16, 8, 128, 16), (6, 2, 128, 48),
+                                                 (8, 1, 64, 32)])
+@pytest.mark.parametrize("window", [0, 1, 37, 64, 300])
+def test_split_wave_attention_does_not_depend_on_the_batch(nH, nKV, hd, page_size, window):
+    """float32 chunks over the waves of a workgroup: contexts at the edges of a sixteen, of a chunk
+    and of the waves' turns, prompts in one step against single tokens, bit for bit, and against
+    the reference."""
+    ops = _ops()
+    ctx_lens, q_lens = [1, 16, 17, 64, 65, 256, 257, 530], [1, 2, 17, 64, 65, 3, 2, 200]
+    s = _paged_setup(torch.float32, nH, nKV, hd, page_size, ctx_lens, q_lens, 9)
+    got, want = _run_attention(s, torch.float32, nH, nKV, hd, page_size, window, q_lens, ctx_lens)
+    assert not torch.isnan(got).any() and rel_err(got, want) <= tol(torch.float32)
+    starts = [0] + list(torch.tensor(q_lens).cumsum(0))
+    for back in (0, 1):         # the sequences' last tokens, and the ones before them
+        at = [int(b) - 1 - back if n > back else int(b) - 1 for b, n in zip(starts[1:], q_lens)]
+        ctx = [c - back if n > back else c for c, n in zip(ctx_lens, q_lens)]
+        one = dict(s, q=s["q"][at], q_start=torch.arange(len(at) + 1, dtype=torch.int32),
+                   ctx_len=torch.tensor(ctx, dtype=torch.int32),
+                   seq_index=torch.arange(len(at), dtype=torch.int32))
+        alone, _ = _run_attention(one, torch.float32, nH, nKV, hd, page_size, window, [1] * len(at),
+                                  ctx)
+        assert torch.equal(alone, got[at])
+
+
 @pytest.mark.parametrize("nH,nKV,hd,page_size,window", [
     (8, 2, 32, 16, 0), (32, 8, 128, 16, 0), (6, 6, 64, 32, 0), (16, 1, 64, 16, 0),
     (9, 3, 256, 16, 0), (8, 2, 64, 16, 37), (4, 4, 128, 48, 300), (36, 4, 32, 16, 0),

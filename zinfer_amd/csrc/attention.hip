@@ -137,6 +137,161 @@ __global__ __launch_bounds__(ZF_WAVE) void paged_attention_wave_kernel(
   }
 }
 
+// The same for float32, heads of 64 or 128 and pages of whole sixteens of rows: a workgroup a token and
+// head; chunks of 64 keys, at multiples of 64, go to its SPLIT_WAVES waves in turn, and their
+// running soft-maxes meet in LDS in wave order.  Four lanes share a key (a load of the wave takes 64
+// bytes of 16 rows), their parts of the dot product are added as ((0 + 1) + (2 + 3)), and four
+// lanes share an element of the output, four rows of a sixteen each (a load takes 1 KB of consecutive
+// memory), added up the same way once at the end.  Everything else is the order of the keys, and
+// nothing depends on the batch.
+// What bounds the kernel above: a key a lane touches 64 lines with every load, which the one address
+// path of a CU takes a cycle each for, and the chunks of a token wait for one another.  Measured
+// against it (16 heads of 128 over 8, pages of 16, us): 4 single tokens behind 70 to 150 keys
+// 13.3 -> 5.9, behind 1000 76.8 -> 20.7, one behind 3000 223 -> 49; prompts of 256 tokens
+// together 52 -> 34, 512 tokens behind 1536 1295 -> 467.  Two heads of a kv head in a workgroup,
+// which reads keys and values once for both, were slower up to 256 tokens (41 us for 34) and no
+// faster at 512 behind 1536.
+#define SPLIT_WAVES 4
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
+
+template <int NV>
+__global__ __launch_bounds__(SPLIT_WAVES * ZF_WAVE) void paged_attention_split_kernel(
+    const float* __restrict__ q, const float* __restrict__ k_pool, const float* __restrict__ v_pool,
+    const int* __restrict__ block_table, const int* __restrict__ q_start,
+    const int* __restrict__ ctx_len, const int* __restrict__ seq_index, float* __restrict__ out,
+    float scale, int window, int nH, int nKV, int page_size, int max_pages) {
+  constexpr int HD = 16 * NV;
+  __shared__ __attribute__((aligned(16))) float qs[HD];
+  __shared__ __attribute__((aligned(16))) float ps[SPLIT_WAVES][ZF_WAVE];
+  __shared__ float ml[SPLIT_WAVES][2], parts[SPLIT_WAVES][HD];
+  const int t = blockIdx.x, h = blockIdx.y;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / ZF_WAVE), lane = threadIdx.x % ZF_WAVE;
+  const int kq = lane / 4, g = lane % 4;
+  const int s = seq_index[t];
+  const int q_len = q_start[s + 1] - q_start[s];
+  const int pos = ctx_len[s] - q_len + (t - q_start[s]);
+  const int lo = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
+  const int kvh = h / (nH / nKV);
+  const int* table = block_table + (size_t)s * max_pages;
+
+  if (threadIdx.x < HD) qs[threadIdx.x] = q[((size_t)t * nH + h) * HD + threadIdx.x];
+  __syncthreads();
+
+  float acc[NV];                                         // element 16 i + kq, this lane's rows
+#pragma unroll
+  for (int i = 0; i < NV; ++i) acc[i] = 0.f;
+  float m = -INFINITY, l = 0.f;
+  for (int base = lo / ZF_WAVE * ZF_WAVE + wave * ZF_WAVE; base <= pos; base += SPLIT_WAVES * ZF_WAVE) {
+    const float* kp[4];
+    const float* vp[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      // (a sixteen without a key of this token reads one that has: its own pages may be gone)
+      const int first = max(min(base + 16 * c, pos), lo) & ~15;
+      const size_t block = (size_t)table[first / page_size] * nKV + kvh;
+      const int row = first % page_size;
+      kp[c] = k_pool + (block * page_size + row + kq) * HD + 4 * g;
+      vp[c] = v_pool + block * page_size * HD + row + (size_t)kq * page_size + 4 * g;
+    }
+    f32x4_t kv[4][NV], vv[4][NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) kv[c][i] = *(const f32x4_t*)(kp[c] + 16 * i);
+    auto load_values = [&](int c) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        vv[c][i] = *(const f32x4_t*)(vp[c] + (size_t)16 * i * page_size);
+    };
+    // (half of the values with the keys, the rest into the keys' registers)
+    load_values(0);
+    load_values(1);
+    __builtin_amdgcn_sched_barrier(0);
+    float sc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const f32x4_t qv = *(const f32x4_t*)&qs[16 * i + 4 * g];
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sc[c] = fmaf(qv[e], kv[c][i][e], sc[c]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    load_values(2);
+    load_values(3);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      sc[c] += lane_xor<1>(sc[c]);
+      sc[c] += lane_xor<2>(sc[c]);
+    }
+    const int key = base + 16 * g + kq;                  // the lane's own, of the four it has a part of
+    const bool seen = key >= lo && key <= pos;
+    const float own = g == 0 ? sc[0] : g == 1 ? sc[1] : g == 2 ? sc[2] : sc[3];
+    const float score = seen ? own * scale : -INFINITY;
+    const float m_new = fmaxf(m, wave_max(score));
+    const float corr = expf(m - m_new);                  // exp(-inf) = 0 on the first chunk
+    const float w = seen ? expf(score - m_new) : 0.f;
+    l = l * corr + wave_sum(w);
+    m = m_new;
+    ps[wave][16 * g + kq] = w;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) acc[i] *= corr;
+    // (a wave's own LDS accesses run in order; this keeps the compiler from moving them)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (base < lo || base + ZF_WAVE - 1 > pos) {          // rows that are no key may hold anything
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int k = base + 16 * c + 4 * g + e;
+          if (k < lo || k > pos) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) vv[c][i][e] = 0.f;
+          }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const f32x4_t wv = *(const f32x4_t*)&ps[wave][16 * c + 4 * g];
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i] = fmaf(wv[e], vv[c][i][e], acc[i]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  if (lane == 0) {
+    ml[wave][0] = m;
+    ml[wave][1] = l;
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    float v = acc[i];
+    v += lane_xor<1>(v);
+    v += lane_xor<2>(v);
+    if (g == i % 4) parts[wave][16 * i + kq] = v;
+  }
+  __syncthreads();
+  // (the first chunk has a key of the token; a wave without keys adds zeros)
+  if (threadIdx.x < HD) {
+    float top = ml[0][0], total = 0.f, v = 0.f;
+#pragma unroll
+    for (int w = 1; w < SPLIT_WAVES; ++w) top = fmaxf(top, ml[w][0]);
+#pragma unroll
+    for (int w = 0; w < SPLIT_WAVES; ++w) {
+      const float f = expf(ml[w][0] - top);
+      total = fmaf(ml[w][1], f, total);
+      v = fmaf(parts[w][threadIdx.x], f, v);
+    }
+    out[((size_t)t * nH + h) * HD + threadIdx.x] = v * (1.0f / total);
+  }
+}
+
 extern "C" int zf_paged_attention_wave(const void* q, const void* k_pool, const void* v_pool,
                                        int dtype, const int* block_table, const int* q_start,
                                        const int* ctx_len, const int* seq_index, void* out,
@@ -147,6 +302,17 @@ extern "C" int zf_paged_attention_wave(const void* q, const void* k_pool, const 
   dim3 grid(T, nH);
   const size_t smem = (size_t)((hd + 3) / 4 * 4 + 2 * ZF_WAVE) * sizeof(float);
   const bool vec = hd % 4 == 0 && page_size % 4 == 0 && ((uintptr_t)k_pool | (uintptr_t)v_pool) % 16 == 0;
+  // (bfloat16 pools of such sizes are the MFMA kernels')
+  if (dtype == ZF_F32 && (hd == 64 || hd == 128) && page_size % 16 == 0 && vec) {
+#define SPLIT_ATTENTION(NV)                                                                         \
+  hipLaunchKernelGGL((paged_attention_split_kernel<NV>), grid, dim3(SPLIT_WAVES * ZF_WAVE), 0, stream, \
+                     (const float*)q, (const float*)k_pool, (const float*)v_pool, block_table,      \
+                     q_start, ctx_len, seq_index, (float*)out, scale, window, nH, nKV, page_size,   \
+                     max_pages)
+    if (hd == 64) SPLIT_ATTENTION(4); else SPLIT_ATTENTION(8);
+#undef SPLIT_ATTENTION
+    ZF_CHECK_LAUNCH();
+  }
 #define WAVE_ATTENTION(TT, NI, V)                                                                \
   hipLaunchKernelGGL((paged_attention_wave_kernel<TT, NI, V>), grid, dim3(ZF_WAVE), smem, stream, \
                      (const TT*)q, (const TT*)k_pool, (const TT*)v_pool, block_table, q_start,   \
@@ -184,7 +350,6 @@ extern "C" int zf_paged_attention_wave(const void* q, const void* k_pool, const 
 // =====================================================================================
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
 typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2_t;
 
