@@ -128,6 +128,49 @@ def test_gemm_float32_does_not_depend_on_the_batch(N, K, offset):
         assert torch.equal(small, got.to(torch.bfloat16)), M
 
 
+@pytest.mark.parametrize("N,K", [(4, 1024), (20, 1028), (100, 1100), (1024, 1540), (1024, 4608),
+                                 (2048, 4100)])
+def test_gemm_float32_spans_in_workgroups_of_their_own(N, K):
+    """Narrow outputs: every span's last step and batch (K up to the next multiple of 256 and
+    beyond), the tokens' groups of 16, and the norm behind the residual sum: the bits of the tiles
+    that take more rows and of the norm's own kernel."""
+    ops = _ops()
+    a, w = _rand((65, K), torch.float32, 43).to(DEV), _rand((N, K), torch.float32, 44, 0.05).to(DEV)
+    base, gain = _rand((65, N), torch.float32, 45).to(DEV), _rand((N,), torch.float32, 46).to(DEV)
+    tiles = torch.empty((65, N), device=DEV)
+    ops.gemm(a, w, tiles)
+    bound = (K + 1) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T) + 1e-30
+    assert bool(((tiles.double() - a.double() @ w.double().T).abs() <= bound).all())
+    for M in (1, 16, 17, 32, 33, 64):
+        got = torch.full((M, N), float("nan"), device=DEV)
+        assert ops._f32_spans_cover(a[:M], w, got)
+        ops.gemm(a[:M], w, got)
+        assert torch.equal(got, tiles[:M]), M
+        residual, normed = base[:M].clone(), torch.full((M, N), float("nan"), device=DEV)
+        ops.gemm_sum_norm(a[:M], w, residual, gain, 1e-6, normed)
+        assert torch.equal(residual, base[:M] + got), M
+        want = torch.empty((M, N), device=DEV)
+        ops.rmsnorm(residual, gain, 1e-6, want)
+        assert torch.equal(normed, want), M
+
+
+@pytest.mark.parametrize("I,K", [(1, 1), (17, 31), (130, 260), (3072, 1024)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_gemm_swiglu_float32_is_the_product_and_the_activation(I, K, offset):
+    ops = _ops()
+    for M in (1, 15, 16):
+        a = torch.empty((M * K + offset,), device=DEV)[offset:].view(M, K)
+        w = torch.empty((2 * I * K + offset,), device=DEV)[offset:].view(2 * I, K)
+        a.copy_(_rand((M, K), torch.float32, 47))
+        w.copy_(_rand((2 * I, K), torch.float32, 48, 0.2))
+        both, want = torch.empty((M, 2 * I), device=DEV), torch.empty((M, I), device=DEV)
+        ops.gemm(a, w, both)
+        ops.swiglu(both, want)
+        got = torch.full((M, I), float("nan"), device=DEV)
+        ops.gemm_swiglu(a, w, got)
+        assert torch.equal(got, want), M
+
+
 @pytest.mark.parametrize("M", [1, 3, 8, 16, 17, 33, 64, 65, 130, 300, 517])
 @pytest.mark.parametrize("N,K", [(1000, 136), (96, 64), (777, 320), (4100, 4096), (256, 1032)])
 @pytest.mark.parametrize("o_dtype,accumulate", [(torch.bfloat16, False), (torch.float32, False),

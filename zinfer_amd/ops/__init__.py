@@ -1015,11 +1015,46 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
                    "gemm (tiled)")
         return
     if a.dtype == torch.float32 and w.dtype == torch.float32:
+        if _f32_spans_cover(a, w, out):
+            ws = _workspace("gemm_splitk", F32_SPANS * M * N, torch.float32, a.device)
+            _check(lib.zf_gemm_f32_spans(_ptr(a), _ptr(w), _ptr(out), _ptr(ws), M, N, K,
+                                         1 if accumulate else 0, _ptr(None), ctypes.c_float(0.0),
+                                         _ptr(None), _stream()), "gemm (32-bit, spans of K)")
+            return
         _check(lib.zf_gemm_f32(_ptr(a), _ptr(w), _ptr(out), _dt(out), M, N, K,
                                1 if accumulate else 0, _stream()), "gemm (32-bit)")
         return
     _check(lib.zf_gemm_fma(_ptr(a), _dt(a), _ptr(w), _dt(w), _ptr(out), _dt(out), M, N, K,
                            1 if accumulate else 0, _stream()), "gemm")
+
+
+F32_SWIGLU_MAX_M = 16   # rows for which the 32-bit gate/up product applies the activation itself
+
+
+def f32_swiglu_covers(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``gemm_swiglu`` takes a gate's and an up projection's rows one below the other."""
+    return a.is_cuda and a.dtype == w.dtype == torch.float32 and 0 < a.shape[0] <= F32_SWIGLU_MAX_M
+
+
+F32_SPANS = 8           # spans of K whose sums a 32-bit product adds in order
+
+
+def _f32_spans_cover(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
+    """A 32-bit product of up to 64 rows whose output is too narrow for its row groups of 16 to fill
+    half of the chip: every span of K goes to a workgroup of its own and a second kernel adds
+    them, the same bits.  Measured on MI355X (4 tokens, us, both kernels): 1024 outputs over K = 2048
+    12.2 -> 8.4, over 3072 17.0 -> 9.9, 2048 over 7168 37.7 -> 20.8; 2048 over 2048 12.5 -> 10.3,
+    but of 16 tokens 11.5 -> 12.0, so a shorter K needs a narrower output."""
+    (M, K), N = a.shape, w.shape[0]
+    return 0 < M <= SKINNY_MAX_M and N % 4 == 0 and K % 4 == 0 \
+        and (K >= 1024 and N <= 1024 or K >= 4096 and N <= 2048) \
+        and out.dtype == torch.float32 and all(t.data_ptr() % 16 == 0 for t in (a, w, out))
+
+
+def f32_sum_norm_covers(a: torch.Tensor, w: torch.Tensor, residual: torch.Tensor) -> bool:
+    """Whether ``gemm_sum_norm`` takes a 32-bit residual sum."""
+    return a.is_cuda and all(t.dtype == torch.float32 for t in (a, w, residual)) \
+        and _f32_spans_cover(a, w, residual)
 
 
 def gemm_partials_plan(M: int, N: int, K: int, w: torch.Tensor, w_tiled: bool):
@@ -1133,10 +1168,24 @@ def _wide_ksplit(M: int, N: int, K: int):
 def gemm_sum_norm(a: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, gain: torch.Tensor,
                   eps: float, normed: torch.Tensor) -> None:
     """residual += a w^T in 32-bit (``w`` pre-tiled) and normed = bfloat16(rmsnorm(residual,
-    gain, eps)), the norm from the kernel that adds the product's partials."""
+    gain, eps)), the norm from the kernel that adds the product's partials.  float32 operands
+    (``f32_sum_norm_covers``): ``w`` in rows, ``normed`` float32."""
     _need_gpu(a, w, residual, gain, normed)
     M, K = a.shape
     N = w.shape[0]
+    if a.dtype == torch.float32:
+        if not f32_sum_norm_covers(a, w, residual) or w.shape[1] != K or residual.shape != (M, N) \
+                or gain.shape != (N,) or normed.shape != (M, N) \
+                or not all(t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
+                           for t in (a, w, residual, gain, normed)):
+            raise KernelUnavailable(f"gemm_sum_norm (32-bit): a {tuple(a.shape)}, w "
+                                    f"{tuple(w.shape)} {w.dtype}, residual {tuple(residual.shape)}")
+        ws = _workspace("gemm_splitk", F32_SPANS * M * N, torch.float32, a.device)
+        lib = build.load("gemm")
+        _check(lib.zf_gemm_f32_spans(_ptr(a), _ptr(w), _ptr(residual), _ptr(ws), M, N, K, 1,
+                                     _ptr(gain), ctypes.c_float(eps), _ptr(normed), _stream()),
+               "gemm_sum_norm (32-bit)")
+        return
     plan = sum_norm_plan(M, N, K, w, True)
     if plan is None or a.dtype != torch.bfloat16 or w.shape[1] != K or not can_pretile(w) \
             or residual.shape != (M, N) or residual.dtype != torch.float32 \
@@ -1245,10 +1294,19 @@ def gemm_swiglu(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled: bo
                 tile_tail: Optional[Tuple[int, int]] = None) -> None:
     """out[M, I] = silu(a Wg^T) * (a Wu^T) as bfloat16, with ``w`` [2 I, K] from
     ``interleave_gate_up`` (then possibly ``pretile_weight``): the activation is applied to
-    the 32-bit sums in the product's epilogue, nothing of width 2 I is written."""
+    the 32-bit sums in the product's epilogue, nothing of width 2 I is written.  float32
+    operands (up to ``F32_SWIGLU_MAX_M`` rows): ``w`` holds the gate's rows, then the up projection's."""
     _need_gpu(a, w, out)
     M, K = a.shape
     N = w.shape[0]
+    if all(t.dtype == torch.float32 for t in (a, w, out)):
+        if w.shape[1] != K or N % 2 != 0 or out.shape != (M, N // 2) or M > F32_SWIGLU_MAX_M:
+            raise KernelUnavailable(f"gemm_swiglu (32-bit): a {tuple(a.shape)}, w {tuple(w.shape)}, "
+                                    f"out {tuple(out.shape)}")
+        lib = build.load("gemm")
+        _check(lib.zf_gemm_f32_swiglu(_ptr(a), _ptr(w), _ptr(out), M, N // 2, K, _stream()),
+               "gemm_swiglu (32-bit)")
+        return
     if w.shape[1] != K or out.shape != (M, N // 2) or out.dtype != torch.bfloat16 \
             or a.dtype != torch.bfloat16 or not can_fuse_swiglu(w):
         raise KernelUnavailable(f"gemm_swiglu: a {tuple(a.shape)} {a.dtype}, w {tuple(w.shape)} "

@@ -55,6 +55,8 @@ class SwiGluMlp(FeedForward):
             h = h.materialize()
         if self.fused and h.dtype == torch.bfloat16:
             ops.gemm_swiglu(h, self.gate_up.weight, a, w_tiled=self.gate_up.tiled)
+        elif ops.f32_swiglu_covers(h, self.gate_up.weight):
+            ops.gemm_swiglu(h, self.gate_up.weight, a)
         else:
             gu = step.scratch("gate_up", (T, 2 * I), act)
             self.gate_up.forward(h, gu)

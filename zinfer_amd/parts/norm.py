@@ -17,7 +17,7 @@ class RmsNorm(Norm):
     Under bfloat16 on the GPU the norm can be taken apart by the products around it: the
     weight-streaming product folds it in (``LazyRmsNorm.fold_into``), and the product that
     last adds into the residual can leave the norm's inputs or its whole result
-    (``residual_sum``)."""
+    (``residual_sum``; in 32-bit its result)."""
     graph_safe = True
     defers = True
     kernel_modules = ("elementwise",)
@@ -34,9 +34,9 @@ class RmsNorm(Norm):
         return out
 
     def deferred(self, x: torch.Tensor, make_out, left=None):
-        if not (x.is_cuda and self.ctx.compute_dtype == torch.bfloat16):
-            return None
         given = left if left is not None and left.fits(self, x) else None
+        if not x.is_cuda or (self.ctx.compute_dtype != torch.bfloat16 and given is None):
+            return None
         return LazyRmsNorm(self, x, make_out, given)
 
     def picked(self, x: torch.Tensor, step):
@@ -50,8 +50,13 @@ class RmsNorm(Norm):
                 step.scratch("normed_squares", (out.shape[1] // 16, 16), torch.float32))
 
     def residual_sum(self, linear, a: torch.Tensor, out: torch.Tensor, step) -> bool:
-        if a.dtype != torch.bfloat16:
-            return False
+        if a.dtype == torch.float32:
+            if not ops.f32_sum_norm_covers(a, linear.weight, out):
+                return False
+            normed = step.scratch("normed_by_sum", out.shape, torch.float32)
+            ops.gemm_sum_norm(a, linear.weight, out, self.gain, float(self.spec.eps), normed)
+            step.norm_ready = DoneRmsNorm(self, out, normed)
+            return True
         M, N, K = a.shape[0], linear.out_features, linear.in_features
         if ops.norm_emit_plan(M, N, K, linear.weight, linear.tiled) is not None:
             xg, sq = self._given_buffers(out, step)
