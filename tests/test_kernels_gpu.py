@@ -1645,6 +1645,24 @@ def test_prefill_attention_splits_keys_over_workgroups(nH, nKV, hd, window, vari
             assert rel_err(got, want) <= 2 * tol(dtype)
 
 
+@pytest.mark.parametrize("nH,nKV,hd,page_size", [(4, 2, 128, 16), (16, 4, 64, 48), (10, 2, 128, 16),
+                                                 (12, 2, 64, 16), (14, 2, 128, 48), (8, 1, 128, 32)])
+@pytest.mark.parametrize("window", [0, 100])
+def test_prefill_attention_of_few_workgroups_behind_contexts(nH, nKV, hd, page_size, window):
+    """Portions behind their contexts on a grid that leaves the chip idle: two groups of waves on the
+    even and the odd key tiles (one of them without a tile, at a tile's edge, mid-page), five to
+    eight heads in two workgroups; against the reference and the kernel without either."""
+    ctx_lens, q_lens = [64, 65, 128, 700, 33, 900], [1, 65, 64, 70, 33, 2]
+    s = _paged_setup(torch.bfloat16, nH, nKV, hd, page_size, ctx_lens, q_lens, seed=33)
+    got, want = _run_attention(s, torch.bfloat16, nH, nKV, hd, page_size, window, q_lens, ctx_lens,
+                               tiles_hint=True)
+    assert not torch.isnan(got.float()).any(), "a slot outside the context was read"
+    assert rel_err(got, want) <= 2 * tol(torch.bfloat16)
+    plain, _ = _run_attention(s, torch.bfloat16, nH, nKV, hd, page_size, window, q_lens, ctx_lens,
+                              tiles_hint=True, variant=3)
+    assert rel_err(got, plain) <= 2 * tol(torch.bfloat16)
+
+
 # ---------------------------------------------------------------- the served decode regime
 # Contexts of thousands of keys at the served head shapes: more than 8 splits of 256 keys (where
 # a lane of the merge kernel takes a second, third, ... load) and more than 64 (where it goes

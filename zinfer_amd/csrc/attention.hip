@@ -1737,14 +1737,22 @@ extern "C" int zf_attn_prefill_bf16(const void* q, const void* k_pool, const voi
   const bool shared_ok = (hd == 64 || hd == 128) && split_keys % 64 == 0;
   if ((variant == 2 || variant == 3) && !shared_ok) return -2;
   if (variant == 2 || variant == 3 || (variant == 0 && shared_ok && G >= 2)) {
-    const int heads = G < 8 ? G : 8, head_blocks = (G + heads - 1) / heads;
-    dim3 sgrid(entries * head_blocks * nKV, split_keys > 0 ? max_splits : 1);
     // two groups of waves on the even and the odd key tiles where the heads leave room for
     // them and the longest chain of tiles sets the time: short contexts before the portions
-    // (allow_split) and a grid that fills the chip at most twice.  (8 K keys before a
-    // 2048-token portion: 14 % slower with them; a whole 2048-token prompt: 73 -> 63 us with 4
-    // heads per kv head, 66 -> 45 us with 2.)
-    const int ks = (variant != 3 && heads <= 4 && split_keys == 0 && allow_split && sgrid.x <= 1024) ? 2 : 1;
+    // (allow_split) on a grid that fills the chip at most twice (8 K keys before a 2048-token
+    // portion: 14 % slower with them; a whole 2048-token prompt: 73 -> 63 us with 4 heads per kv
+    // head, 66 -> 45 us with 2), or whatever the contexts on one of up to 400 workgroups, where the CUs wait
+    // for that chain (497 tokens behind 500 keys, 16 / 32 heads on 8: 32.1 -> 20.8, 30.3 -> 25.8 us;
+    // five portions of 300, up to 1500 keys, 400 workgroups: 45.9 -> 29.8, 44.2 -> 36.0).  Five to eight
+    // heads go to two workgroups then, up to 256 of them before: 497 tokens behind 0 / 500 / 1400 keys,
+    // 40 heads on 8, 23.2 -> 16.9, 38.9 -> 26.0, 64.9 -> 40.5 us, 1024 tokens 38.9 -> 34.0; of 312 and
+    // more the halves no longer run side by side (three prompts of 400 23.0 -> 32.1).
+    const unsigned blocks = entries * nKV;
+    const bool groups = variant != 3 && split_keys == 0 && (allow_split || blocks <= 400);
+    const bool halves = groups && G > 4 && G <= 8 && blocks <= 256;
+    const int heads = halves ? (G + 1) / 2 : G < 8 ? G : 8, head_blocks = (G + heads - 1) / heads;
+    dim3 sgrid(entries * head_blocks * nKV, split_keys > 0 ? max_splits : 1);
+    const int ks = groups && heads <= 4 && sgrid.x <= 1024 ? 2 : 1;
     const dim3 sblock(64 * heads * ks);
 #define ZF_PRE_S(HD, POW2, KS)                                                                  \
   hipLaunchKernelGGL((attn_prefill_shared_kernel<HD, POW2, KS>), sgrid, sblock, 0, stream,      \
