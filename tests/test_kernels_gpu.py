@@ -1645,6 +1645,32 @@ def test_prefill_attention_splits_keys_over_workgroups(nH, nKV, hd, window, vari
             assert rel_err(got, want) <= 2 * tol(dtype)
 
 
+@pytest.mark.parametrize("M,N,K,parts", [(257, 5120, 9728, 6), (512, 5120 - 192, 9600, 6),
+                                         (641, 4096, 8192, 5), (1025, 2560, 8192, 5),
+                                         (897, 5120, 4864, 3)])
+def test_residual_sum_through_256_token_tiles_split_along_k(M, N, K, parts):
+    """Rows and columns that end inside a tile, parts of unequal length; the sum, and the sum with the
+    norm behind it, which gives the same sum."""
+    ops = _ops()
+    a = _rand((M, K), torch.bfloat16, 34).to(DEV)
+    w = _rand((N, K), torch.bfloat16, 35, 0.05).to(DEV)
+    base, gain = _rand((M, N), torch.float32, 36).to(DEV), _rand((N,), torch.float32, 37).to(DEV)
+    wt = ops.pretile_weight(w)
+    assert ops._tile256_ksplit(M, N, K) == parts
+    want = base.double() + a.double() @ w.double().T
+    got = base.clone()
+    ops.gemm(a, wt, got, accumulate=True, w_tiled=True)
+    # a sum of K exact products in 32-bit, whatever its order
+    bound = (K + 1) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + base.double().abs())
+    assert bool(((got.double() - want).abs() <= bound).all())
+    residual, normed = base.clone(), torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
+    ops.gemm_sum_norm(a, wt, residual, gain, 1e-6, normed)
+    assert torch.equal(residual, got)
+    rows = torch.empty((M, N), dtype=torch.bfloat16)
+    ref.rmsnorm(got.cpu(), gain.cpu(), 1e-6, rows)
+    assert rel_err(normed, rows) <= tol(torch.bfloat16)
+
+
 @pytest.mark.parametrize("nH,nKV,hd,page_size", [(4, 2, 128, 16), (16, 4, 64, 48), (10, 2, 128, 16),
                                                  (12, 2, 64, 16), (14, 2, 128, 48), (8, 1, 128, 32)])
 @pytest.mark.parametrize("window", [0, 100])

@@ -1250,7 +1250,7 @@ constexpr int reads_before(int m, int nm, int cnt, int nr) {
   return done < nr ? done : nr;
 }
 
-template <int BN, int EPI>
+template <int BN, int EPI, bool SPLIT = false>
 __global__ __launch_bounds__(256) void gemm_bf16_tile256_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ Cv, int M,
     int N, int K, int tiles_m, int tiles_n, const float* __restrict__ glu_bias) {
@@ -1298,7 +1298,11 @@ __global__ __launch_bounds__(256) void gemm_bf16_tile256_kernel(
   // the pre-tiled matrix a group's 64 k lie as [h][4 k-steps][16 outputs] pieces of 8.
   // W into registers: the operand of column block j, k-step ks: column n = n0 + wn WN + 32 j
   // + lane % 32, half lane / 32.  Groups beyond N are clamped (never stored).
-  const char* a_tile = (const char*)(A + (size_t)m0 * K);
+  // SPLIT: K in gridDim.y parts of whole 128, as even as they come; a part's sums go to
+  // Cv + part * M * N
+  const int unit0 = SPLIT ? (int)((long long)blockIdx.y * (K / 128) / gridDim.y) : 0;
+  const int units = SPLIT ? (int)((blockIdx.y + 1ll) * (K / 128) / gridDim.y) - unit0 : K / 128;
+  const char* a_tile = (const char*)(A + (size_t)m0 * K + (size_t)unit0 * 128);
   uint32_t asrc[A_CHUNKS];
 #pragma unroll
   for (int c = 0; c < A_CHUNKS; ++c) {
@@ -1307,7 +1311,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_tile256_kernel(
   }
   const int kt64 = K / 64;
   const int grp0 = min(n0 / 16, N / 16 - 1);
-  const char* w_tile = (const char*)(W + (size_t)grp0 * kt64 * 1024);
+  const char* w_tile = (const char*)(W + ((size_t)grp0 * kt64 + 2 * unit0) * 1024);
   uint32_t wsrc[W_CHUNKS];
 #pragma unroll
   for (int c = 0; c < W_CHUNKS; ++c) {
@@ -1318,7 +1322,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_tile256_kernel(
   // Where k-tile t (of 32) starts in the tokens' rows and in a group's pre-tiled 64 k, as
   // offsets all lanes share; tiles behind the last one are the last one again.  (t is a
   // multiple of 4 plus a constant, so which half of the 64 k it is is known when compiling.)
-  const int ktiles = K / 32, klast = ktiles - 1;
+  const int ktiles = 4 * units, klast = ktiles - 1;
   const uint32_t last_a = (uint32_t)klast * 64, last_w = (uint32_t)(klast / 2) * 2048 + 512;
   struct TileSrc { uint32_t a; uint32_t w; };
   auto tile_src = [&](int base4, auto OFF) __attribute__((always_inline)) -> TileSrc {
@@ -1471,6 +1475,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_tile256_kernel(
   float* slab = (float*)(wave == 0 ? stage0 : wave == 1 ? stage1 : wave == 2 ? stage2 : stage3);
   static_assert(32 * (WN + 4) * sizeof(float) <= (A_PLACES + W_PLACES) * 16 || FN == 3, "slab");
   const int mw = m0 + wm * WM, nw = n0 + wn * WN;
+  if constexpr (SPLIT) Cv = (float*)Cv + (size_t)blockIdx.y * M * N;
   if constexpr (FN == 3) {
     store_through_slab<FM, 2, 64, EPI, 0, FN>(acc, slab, mw, nw, M, N, Cv, lane, glu_bias);
     store_through_slab<FM, 1, 32, EPI, 2, FN>(acc, slab, mw, nw + 64, M, N, Cv, lane, glu_bias);
@@ -2369,6 +2374,26 @@ extern "C" int zf_gemm_bf16_wide_splitk_sum_norm(const void* A, const void* W, v
   const int threads = N / 4 >= 1024 ? 1024 : (N / 4 > 256 ? 512 : 256);
   hipLaunchKernelGGL(reduce_sum_norm_kernel<bf16_t>, dim3(M), dim3(threads), 0, stream, (const float*)ws,
                      (float*)C, gain, (bf16_t*)normed, M, N, ksplit, eps);
+  return (int)hipGetLastError();
+}
+
+// C += A W^T in 32-bit through 256 x 256 tiles split along K: ws float32 [ksplit, M, N], K of at
+// least ksplit times 128.  With a gain normed = bfloat16 RMSNorm of the rows (N <= 8192), from the
+// kernel that adds the partials.
+extern "C" int zf_gemm_bf16_tile256_splitk(const void* A, const void* W, void* C, void* ws, int M,
+                                           int N, int K, int ksplit, const float* gain, float eps,
+                                           void* normed, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (N % 16 != 0 || K % 128 != 0 || ksplit < 2 || ksplit > K / 128 || ws == nullptr) return -3;
+  if (gain != nullptr && N > 8192) return -3;
+  const int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
+  hipLaunchKernelGGL((gemm_bf16_tile256_kernel<256, EPI_STORE_F32, true>),
+                     dim3(tiles_m * tiles_n, ksplit), dim3(256), 0, stream, (const bf16_t*)A,
+                     (const bf16_t*)W, ws, M, N, K, tiles_m, tiles_n, nullptr);
+  if (gain == nullptr) return launch_reduce(ws, C, M, N, ksplit, EPI_ACC_F32, stream);
+  const int threads = N / 4 >= 1024 ? 1024 : (N / 4 > 256 ? 512 : 256);
+  hipLaunchKernelGGL(reduce_sum_norm_kernel<bf16_t>, dim3(M), dim3(threads), 0, stream,
+                     (const float*)ws, (float*)C, gain, (bf16_t*)normed, M, N, ksplit, eps);
   return (int)hipGetLastError();
 }
 

@@ -986,6 +986,14 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
             _check(lib.zf_gemm_bf16_mid(_ptr(a), _ptr(w), _ptr(out), _ptr(None), M, N, K, epi, 1,
                                         _stream()), "gemm (64-token tiles)")
         else:
+            parts = _tile256_ksplit(M, N, K) if w_tiled and accumulate else None
+            if parts is not None:       # as gemm_sum_norm runs it: the same bits
+                ws = _workspace("gemm_splitk", parts * M * N, torch.float32, a.device)
+                _check(lib.zf_gemm_bf16_tile256_splitk(_ptr(a), _ptr(w), _ptr(out), _ptr(ws), M, N, K,
+                                                       parts, _ptr(None), ctypes.c_float(0.0),
+                                                       _ptr(None), _stream()),
+                       "gemm (256-token tiles, split along K)")
+                return
             wide = _wide_ksplit(M, N, K) if w_tiled and accumulate else None
             if wide is not None:        # as gemm_sum_norm runs it: the same bits
                 ws = _workspace("gemm_splitk", wide * M * N, torch.float32, a.device)
@@ -1131,8 +1139,8 @@ def norm_gemm(x: torch.Tensor, gain: torch.Tensor, eps: float, w: torch.Tensor,
 def sum_norm_plan(M: int, N: int, K: int, w: torch.Tensor, w_tiled: bool):
     """The plan if ``gemm_sum_norm`` covers residual += a w^T: a product that is split along K
     anyway (by measurement at 1 to 64 tokens, by rule at 17 to 128, or a few hundred tokens on
-    a narrow output), whose partials one kernel can add, sum into the residual and norm; else
-    None.  ('mid' | 'tile' | 'wide' | 'skinny', [row groups per workgroup,] workgroups along K)."""
+    a narrow output, or up to 2048 on a long K), whose partials one kernel can add, sum into the
+    residual and norm; else None.  ('mid' | 'tile' | 'wide' | 'tile256' | 'skinny', [row groups per workgroup,] workgroups along K)."""
     if not (w_tiled and w.dtype == torch.bfloat16 and w.is_cuda and N % 16 == 0 and N <= 8192):
         return None
     if M <= NORM_FOLD_MAX_M:
@@ -1140,11 +1148,32 @@ def sum_norm_plan(M: int, N: int, K: int, w: torch.Tensor, w_tiled: bool):
     if M <= MID_MAX_M:
         plan = _small_plan(M, N, K, True)
         return plan if plan is not None and plan[-1] >= 2 else None
+    ks = _tile256_ksplit(M, N, K)
+    if ks is not None:
+        return ("tile256", ks)
     wide = _wide_ksplit(M, N, K)
     if wide is not None:
         return ("wide", wide)
     ks = _tile_ksplit(M, N, K)
     return ("tile", ks) if ks >= 2 else None
+
+
+def _tile256_ksplit(M: int, N: int, K: int):
+    """Parts of K if a residual sum should run through the 256 x 256 tiles split along K, one workgroup
+    to a CU: where the parts fill seven eighths of the chip and are long enough for their partials.
+    These tiles run at 5.2 TFLOP/s a CU where 128 x 128 ones reach 3.8 two to a CU.  Measured on
+    MI355X, us, the norm's kernel included, against what ran before: 512 tokens over K = 17408
+    into 5120 114 -> 105, 25600 162 -> 145; 640 tokens 150 -> 131; 1024 212 -> 172; over 5120
+    into 5120 88 -> 76; 12288 into 4096 at 768 / 1100 tokens 107 -> 94, 152 -> 128.  Of parts under
+    1600 the partials cost what the tiles gain (512 tokens over 8192 into 5120, six parts: 66 -> 66,
+    768 over 5120, four: 60 -> 65).  Not in two parts: unsplit tiles fill most of the chip there as
+    well (2048 tokens into 4096 over 12288 192 -> 186, over 4096 80 -> 89, and nothing of the former
+    is left in a whole prompt's step, which the chip's power limits)."""
+    if M <= 256 or K % 128 != 0 or N % 16 != 0 or N > 8192:
+        return None
+    tiles = ((M + 255) // 256) * ((N + 255) // 256)
+    ks = 256 // tiles
+    return ks if 3 <= ks <= 6 and tiles * ks >= 224 and K >= 1600 * ks else None
 
 
 def _wide_ksplit(M: int, N: int, K: int):
@@ -1198,7 +1227,11 @@ def gemm_sum_norm(a: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, gain
     ks = plan[-1]
     ws = _workspace("gemm_splitk", ks * M * N, torch.float32, a.device)
     lib = build.load("gemm")
-    if plan[0] == "wide":
+    if plan[0] == "tile256":
+        _check(lib.zf_gemm_bf16_tile256_splitk(_ptr(a), _ptr(w), _ptr(residual), _ptr(ws), M, N, K, ks,
+                                               _ptr(gain), ctypes.c_float(eps), _ptr(normed),
+                                               _stream()), "gemm_sum_norm (256-token tiles)")
+    elif plan[0] == "wide":
         _check(lib.zf_gemm_bf16_wide_splitk_sum_norm(_ptr(a), _ptr(w), _ptr(residual), _ptr(ws),
                                                      _ptr(gain), ctypes.c_float(eps), _ptr(normed),
                                                      M, N, K, ks, _stream()),
