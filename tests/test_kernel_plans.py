@@ -134,7 +134,7 @@ TESTED_AGAINST = {
     "advance_decode": "test_engine_gpu.py:test_decode_steps_in_a_row_equal_single_steps",
     "cast": "test_kernels_gpu.py:test_cast_and_poison_pages",
     "poison_pages": "test_kernels_gpu.py:test_cast_and_poison_pages",
-    "gemm": "kernel_refs.py:gemm", "gemm_partials": "kernel_refs.py:gemm",
+    "gemm": "kernel_refs.py:gemm", "gemm_many": "kernel_refs.py:gemm", "gemm_partials": "kernel_refs.py:gemm",
     "gemm_swiglu": "kernel_refs.py:gemm_swiglu", "norm_gemm": "kernel_refs.py:rmsnorm",
     "gemm_emit": "kernel_refs.py:gemm", "gemm_given": "kernel_refs.py:rmsnorm",
     "gemm_sum_norm": "kernel_refs.py:rmsnorm", "paged_attention": "kernel_refs.py:paged_attention",

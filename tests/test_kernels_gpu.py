@@ -1213,6 +1213,33 @@ def test_embed_of_a_width_without_whole_pieces():
     assert torch.equal(out.cpu(), table[ids.long()].float() * 2.0)
 
 
+@pytest.mark.parametrize("M", [1, 7, 16])
+@pytest.mark.parametrize("K,widths", [(64, [(64, True, "bf16")] * 6), (1024, [(2048, True, "bf16"), (16, False, "tanh")]),
+                                      (2048 + 192, [(17, False, "f32"), (128, True, "f32"), (64, True, "silu")]),
+                                      (40, [(1, False, "bf16"), (33, False, "gelu")])])
+def test_gemm_many_gives_the_products_own_bits(M, K, widths):
+    """Products with their ends inside and at a row group, pre-tiled or not, every kind of result."""
+    ops = _ops()
+    items, wants = [], []
+    for i, (N, tiled, kind) in enumerate(widths):
+        a = _rand((M, K), torch.bfloat16, 90 + i).to(DEV)
+        w = _rand((N, K), torch.bfloat16, 110 + i, 0.1).to(DEV)
+        w = ops.pretile_weight(w) if tiled else w
+        act = kind if kind in ops.ACTIVATIONS else None
+        out = torch.full((M, N), float("nan"), device=DEV,
+                         dtype=torch.float32 if kind == "f32" else torch.bfloat16)
+        want = torch.empty_like(out)
+        ops.gemm(a, w, want, w_tiled=tiled)
+        if act:
+            ops.activation(want, want, act)
+        items.append((a, w, tiled, out, act))
+        wants.append(want)
+    assert ops.gemm_many_covers(items)
+    ops.gemm_many(items)
+    for (_, _, _, out, _), want in zip(items, wants):
+        assert torch.equal(out, want)
+
+
 def test_cpu_tensor_is_refused():
     """There is no CPU path: a tensor that is not on the GPU is an error, not a fallback."""
     from zinfer_amd.errors import KernelUnavailable

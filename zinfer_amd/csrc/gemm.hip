@@ -506,6 +506,10 @@ extern "C" int zf_gemm_f32_swiglu(const float* A, const float* W, float* C, int 
 #define EPI_GEGLU 4
 // an activation on the bfloat16 that EPI_STORE_BF16 would store, stored as bfloat16 (up to 16 tokens)
 #define EPI_ACT 5
+// bfloat16, float32 or an activation on the bfloat16, as SkinnyNorm::act says
+#define EPI_MANY 6
+#define MANY_BF16 -1
+#define MANY_F32 -2
 #define EPI_GLU(E) ((E) == EPI_SWIGLU || (E) == EPI_GEGLU)
 
 __device__ __forceinline__ float swiglu_f(float g, float u) { return g / (1.0f + expf(-g)) * u; }
@@ -1776,10 +1780,12 @@ extern "C" int zf_gemm_bf16_tile_splitk(const void* A, const void* W, void* C, v
 // when there is no split over workgroups), and the epilogue scales each token's sums by
 // inv = 1 / sqrt(mean(x^2) + eps), all in 32-bit  (n = x w / sqrt(mean(x^2) + eps),
 // src/kernel/core/cpu.zig:38-48 of the reference).
-template <int MT, int RG, int EPI, bool WT, int NORM, int NW = 8, bool EMIT = false>
-__global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
+// `block` of the workgroups along the outputs, `part` of `parts` along K.
+// DEEP: two register sets of loads, for a workgroup that has a CU to itself.
+template <int MT, int RG, int EPI, bool WT, int NORM, int NW, bool EMIT, bool DEEP = true>
+__device__ __forceinline__ void skinny_product(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ Cv, int M,
-    int N, int K, SkinnyNorm nrm) {
+    int N, int K, const SkinnyNorm& nrm, int block, int part_k, int parts) {
   constexpr int NSS = NORM == NORM_GIVEN ? NW * 4 : NW;
   __shared__ float part[NW][RG * MT][64][4];
   // a token's sums side by side: inv_rms reads four at a time, and the tokens' rows of NSS + 4
@@ -1788,7 +1794,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
   const float* __restrict__ gain = nrm.gain;
   const float eps = nrm.eps;
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const int n0 = blockIdx.x * (16 * RG);
+  const int n0 = block * (16 * RG);
   const int g = lane / 16;
   // plain layout: row pointer, k added later; pre-tiled: the lane's 16 bytes of chunk 0 of
   // the row group's first tile, tiles of 64 k are 1024 elements apart, chunk 1 is 512 on
@@ -1820,14 +1826,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
     for (int t = 0; t < MT; ++t) acc[r][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   const u32x4_t zero = u32x4_t{0, 0, 0, 0};
-  const int kstride = NW * 64 * gridDim.y;
-  int k0 = (blockIdx.y * NW + wave) * 64;
+  const int kstride = NW * 64 * parts;
+  int k0 = (part_k * NW + wave) * 64;
   // What the epilogue reads from memory is asked for now, so that it has arrived when the
   // last weights have: the residual and the next norm's gains (wave 0 writes the outputs of
   // one row group and up to 16 tokens), and the producer's sums of squares.
   constexpr bool PRE_EPI = EMIT && RG * MT == 1;
   float4 pre_c = float4{0.f, 0.f, 0.f, 0.f}, pre_g = float4{0.f, 0.f, 0.f, 0.f};
-  if (PRE_EPI && wave == 0 && gridDim.y == 1) {
+  if (PRE_EPI && wave == 0 && parts == 1) {
     const int token = lane % 16, n = n0 + 4 * (lane / 16);
     if (token < M && n + 3 < N) {
       pre_c = *(const float4*)((const float*)Cv + (size_t)token * N + n);
@@ -1905,7 +1911,30 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
       k0 = K;
     }
   }
-  if constexpr (WT && NORM != NORM_FOLD && (RG * MT == 1 || (RG * MT == 2 && !EPI_GLU(EPI)))) {
+  if constexpr (WT && !DEEP && RG * MT == 1) {
+    // four blocks in flight in one register set (other workgroups of the CU load meanwhile)
+    static_assert(NORM == NORM_NONE, "plain products");
+    for (; k0 + 3 * kstride < K; k0 += 4 * kstride) {
+      u32x4_t w0[4], w1[4], a0[4], a1[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int kk = k0 + u * kstride;
+        const bf16_t* tile = wrow[0] + (size_t)(kk / 64) * 1024;
+        w0[u] = __builtin_nontemporal_load((const u32x4_t*)tile);
+        w1[u] = __builtin_nontemporal_load((const u32x4_t*)(tile + 512));
+        a0[u] = tok[0] ? *(const u32x4_t*)(arow[0] + kk + g * 16) : zero;
+        a1[u] = tok[0] ? *(const u32x4_t*)(arow[0] + kk + g * 16 + 8) : zero;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(bf16x8_t*)&w0[u], *(bf16x8_t*)&a0[u],
+                                                            acc[0][0], 0, 0, 0);
+        acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(bf16x8_t*)&w1[u], *(bf16x8_t*)&a1[u],
+                                                            acc[0][0], 0, 0, 0);
+      }
+    }
+  }
+  if constexpr (WT && DEEP && NORM != NORM_FOLD && (RG * MT == 1 || (RG * MT == 2 && !EPI_GLU(EPI)))) {
     asked = true;
     // Pre-tiled weights (no bounds checks; K % 64 == 0), up to two MFMA tiles per k-step:
     // batches of UNR k-steps in two register sets, the next batch asked for before the
@@ -2144,8 +2173,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
       for (int e = 0; e < 4; ++e) {
         const int n = n0 + r * 16 + 4 * (l / 16) + e;
         if (n < N) {
-          if (gridDim.y > 1) {
-            ((float*)Cv)[((size_t)blockIdx.y * M + token) * N + n] = s[e];   // workspace
+          if (parts > 1) {
+            ((float*)Cv)[((size_t)part_k * M + token) * N + n] = s[e];   // workspace
           } else {
             const size_t off = (size_t)token * N + n;
             if (EPI == EPI_STORE_BF16) {
@@ -2153,8 +2182,12 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
             } else if (EPI == EPI_ACT) {
               ((bf16_t*)Cv)[off] =
                   float_to_bf16(activation_value(bf16_to_float(float_to_bf16(s[e])), nrm.act));
-            } else if (EPI == EPI_STORE_F32) {
+            } else if (EPI == EPI_STORE_F32 || (EPI == EPI_MANY && nrm.act == MANY_F32)) {
               ((float*)Cv)[off] = s[e];
+            } else if (EPI == EPI_MANY) {
+              const bf16_t v = float_to_bf16(s[e]);
+              ((bf16_t*)Cv)[off] = nrm.act == MANY_BF16
+                  ? v : float_to_bf16(activation_value(bf16_to_float(v), nrm.act));
             } else {
               const float old = PRE_EPI ? ((const float*)&pre_c)[e] : ((float*)Cv)[off];
               const float v = old + s[e];
@@ -2177,6 +2210,63 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
       if (l < 16) nrm.sq_out[(size_t)(n0 / 16 + r) * 16 + l] = sq;
     }
   }
+}
+
+template <int MT, int RG, int EPI, bool WT, int NORM, int NW = 8, bool EMIT = false>
+__global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ Cv, int M,
+    int N, int K, SkinnyNorm nrm) {
+  skinny_product<MT, RG, EPI, WT, NORM, NW, EMIT>(A, W, Cv, M, N, K, nrm, blockIdx.x, blockIdx.y,
+                                                  gridDim.y);
+}
+
+// Several products of up to 16 tokens over the same K in one launch, a row group of 16 a
+// workgroup: products that read the same rows or lie ready together, each too narrow for the chip
+// and as long as a launch.  In traces, 16 tokens: four of 2048 x 2048 and one of 16 x 2048 with a tanh
+// 4 x 5.6 + 6.3 + 3.7 -> 10.5 us, 6144 and 16 x 2048 7.6 + 6.3 -> 9.6; 8 tokens: 3072, 6144 and 32 x
+// 2048 5.3 + 7.1 + 5.9 -> 10.2, twice 2048 x 2048 10.2 -> 5.8.  Two workgroups and more a CU in one
+// register set: with the streaming kernel's two sets, one a CU, the first took 16.2 us.
+// Every product's bits are those of a launch of its own.
+#define ZF_MANY_PRODUCTS 6
+struct ManyProducts {
+  const bf16_t* a[ZF_MANY_PRODUCTS];
+  const bf16_t* w[ZF_MANY_PRODUCTS];
+  void* c[ZF_MANY_PRODUCTS];
+  int n[ZF_MANY_PRODUCTS];
+  int tiled[ZF_MANY_PRODUCTS];
+  int act[ZF_MANY_PRODUCTS];       // an activation's number, MANY_BF16 or MANY_F32
+  int end[ZF_MANY_PRODUCTS];       // workgroups of this product and the ones before
+  int count;
+};
+__global__ __launch_bounds__(512, 4) void gemm_bf16_many_kernel(ManyProducts p, int M, int K) {
+  int i = 0, first = 0;
+  while (i + 1 < p.count && (int)blockIdx.x >= p.end[i]) first = p.end[i++];
+  SkinnyNorm nrm{};
+  nrm.act = p.act[i];
+  if (p.tiled[i])
+    skinny_product<1, 1, EPI_MANY, true, NORM_NONE, 8, false, false>(p.a[i], p.w[i], p.c[i], M, p.n[i], K, nrm,
+                                                              blockIdx.x - first, 0, 1);
+  else
+    skinny_product<1, 1, EPI_MANY, false, NORM_NONE, 8, false, false>(p.a[i], p.w[i], p.c[i], M, p.n[i], K,
+                                                               nrm, blockIdx.x - first, 0, 1);
+}
+
+// `products`: count, n, tiled and act as above, end filled here; every operand bfloat16 with K
+// contiguous, K % 8 == 0 (pre-tiled: K % 64 == 0, n % 16 == 0) and 16-byte aligned.
+extern "C" int zf_gemm_bf16_many(ManyProducts* products, int M, int K, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (M > 16 || K <= 0 || K % 8 != 0 || products->count < 1 || products->count > ZF_MANY_PRODUCTS)
+    return -3;
+  int end = 0;
+  for (int i = 0; i < products->count; ++i) {
+    if (products->n[i] <= 0 || products->act[i] > 4 ||
+        (products->tiled[i] && (K % 64 != 0 || products->n[i] % 16 != 0)) ||
+        (((uintptr_t)products->a[i] | (uintptr_t)products->w[i]) % 16) != 0)
+      return -3;
+    products->end[i] = end += (products->n[i] + 15) / 16;
+  }
+  hipLaunchKernelGGL(gemm_bf16_many_kernel, dim3(end), dim3(512), 0, stream, *products, M, K);
+  return (int)hipGetLastError();
 }
 
 // VEC: four outputs a thread with 16-byte loads (M * N a multiple of 4, so that every

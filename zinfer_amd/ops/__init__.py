@@ -1286,6 +1286,53 @@ def gemm_emit(a: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, gain: to
                                         _ptr(sq), M, N, K, rg, _stream()), "gemm_emit")
 
 
+class _ManyProducts(ctypes.Structure):
+    """``ManyProducts`` of csrc/gemm.hip."""
+    MAX = 6
+    _fields_ = [("a", ctypes.c_void_p * 6), ("w", ctypes.c_void_p * 6), ("c", ctypes.c_void_p * 6),
+                ("n", ctypes.c_int * 6), ("tiled", ctypes.c_int * 6), ("act", ctypes.c_int * 6),
+                ("end", ctypes.c_int * 6), ("count", ctypes.c_int)]
+
+
+def gemm_many_covers(items) -> bool:
+    """Whether ``gemm_many`` takes the products ``items``: up to six of the same up to 16 rows and K,
+    of bfloat16 operands, each one that would run unsplit by itself."""
+    if not 2 <= len(items) <= _ManyProducts.MAX:
+        return False
+    M, K = items[0][0].shape
+    if not 0 < M <= NORM_FOLD_MAX_M or K % 8 != 0:
+        return False
+    for a, w, tiled, out, act in items:
+        N = w.shape[0]
+        if not (a.is_cuda and a.dtype == w.dtype == torch.bfloat16 and a.shape == (M, K)
+                and w.shape[1] == K and out.shape == (M, N)
+                and out.dtype in ((torch.bfloat16,) if act else (torch.bfloat16, torch.float32))
+                and all(t.is_contiguous() for t in (a, w, out))
+                and all(t.data_ptr() % 16 == 0 for t in (a, w))
+                and _skinny_plan(M, N, K, tiled)[1] == 1):
+            return False
+    return True
+
+
+@_launches("products")
+def gemm_many(items) -> None:
+    """Several products in one launch, each (a, w, w_tiled, out, activation or None): ``gemm``'s
+    out = a w^T, or ``gemm_activation``'s, the same bits (``gemm_many_covers``)."""
+    if not gemm_many_covers(items):
+        raise KernelUnavailable("gemm_many: 2 to 6 bfloat16 products of the same up to 16 rows and K, "
+                                f"got {[(tuple(a.shape), tuple(w.shape)) for a, w, *_ in items]}")
+    M, K = items[0][0].shape
+    p = _ManyProducts()
+    p.count = len(items)
+    # (rows as they lie come first: such a product's few workgroups take the longest)
+    for i, (a, w, tiled, out, act) in enumerate(sorted(items, key=lambda x: bool(x[2]))):
+        p.a[i], p.w[i], p.c[i] = a.data_ptr(), w.data_ptr(), out.data_ptr()
+        p.n[i], p.tiled[i] = w.shape[0], 1 if tiled else 0
+        p.act[i] = ACTIVATIONS[act] if act else -1 if out.dtype == torch.bfloat16 else -2
+    lib = build.load("gemm")
+    _check(lib.zf_gemm_bf16_many(ctypes.byref(p), M, K, _stream()), "gemm_many")
+
+
 @_launches("products")
 def gemm_given(xg: torch.Tensor, sq: torch.Tensor, eps: float, w: torch.Tensor,
                out: torch.Tensor, swiglu: bool = False) -> None:

@@ -14,6 +14,7 @@ from . import delta_recurrence, short_conv, streams_step
 from . import add_row, bias_act_rows, fixed_decay, rotation_table
 from . import embed_norm, gate_norm, gated_rows, gemm_geglu, state_space
 from . import (concat_rows, decay_recurrence, embed_sinusoid, head_norm_gate, token_shift_mix)
+from . import gemm_many
 from . import (activation, head_products, masked_attention, masked_attention_mfma,
                norm_add_store, project_rows)
 from . import (embed_position, kv_rows_write, moe_down, moe_gate_up, moe_route, norm_rows,
@@ -55,6 +56,7 @@ KERNELS: Dict[str, KernelEntry] = {
     "cast": KernelEntry(cast, "elementwise", "src/tensor/formats/bfloat16.zig:3-13"),
     "poison_pages": KernelEntry(poison_pages, "elementwise", "own: NaN into pages given back"),
     "gemm": KernelEntry(gemm, "gemm", _LINEAR),
+    "gemm_many": KernelEntry(gemm_many, "gemm", _LINEAR),
     "gemm_partials": KernelEntry(gemm_partials, "gemm", _LINEAR),
     "gemm_swiglu": KernelEntry(gemm_swiglu, "gemm", _LINEAR + "; src/kernel/core/cpu.zig:130-147"),
     "gemm_geglu": KernelEntry(gemm_geglu, "gemm", "own: a gate's and an up projection's product with "

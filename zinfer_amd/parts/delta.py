@@ -8,7 +8,7 @@ from .. import ops
 from ..config.specs import GatedDeltaRuleSpec, ParallelMixerSpec
 from ..errors import ConfigError
 from .base import KVNeed, Mixer, StateNeed, TensorDecl, build_part, register_part
-from .linear import Linear, place_gain, place_matrix
+from .linear import Linear, place_gain, place_matrix, products
 
 
 class GatedDeltaRule(Mixer):
@@ -92,17 +92,19 @@ class GatedDeltaRule(Mixer):
     def cache_need(self):
         return StateNeed((self.state_size,), torch.float32)
 
-    def forward(self, h, residual, step, cache, accumulate: bool = True) -> None:
-        s = self.spec
-        T = h.shape[0]
-        act = self.ctx.act_dtype
-        if hasattr(h, "materialize"):
-            h = h.materialize()
-        QK, V = self.qk_width, self.v_width
-        proj = step.scratch("delta_proj", (T, self.proj.out_features), act)
-        self.proj.forward(h, proj)
+    def into(self, h, step):
+        """The products that read the mixer's input, as ``products`` takes them."""
+        s, T = self.spec, h.shape[0]
+        proj = step.scratch("delta_proj", (T, self.proj.out_features), self.ctx.act_dtype)
         ab = step.scratch("delta_decay_beta", (T, 2 * s.n_heads), torch.float32)
-        self.decay_beta.forward(h, ab)
+        return [(h, self.proj, proj, None), (h, self.decay_beta, ab, None)]
+
+    def between(self, rows, step, cache):
+        """From what the products of ``into`` left (``rows``) to what the output product reads."""
+        s = self.spec
+        proj, ab = rows
+        T = proj.shape[0]
+        QK, V = self.qk_width, self.v_width
         qkv = step.scratch("delta_qkv", (T, self.conv_width), torch.float32)
         ops.short_conv(proj, self.taps, cache.state, self.matrix_size, step.state_slots,
                        step.seq_index, step.q_start, qkv, unit_heads=2 * s.n_kv_heads,
@@ -112,9 +114,17 @@ class GatedDeltaRule(Mixer):
         ops.delta_recurrence(qkv, 0, QK, 2 * QK, ab, self.decay_log, self.decay_bias, cache.state,
                              step.state_slots, step.q_start, o, s.n_heads, s.n_kv_heads,
                              s.head_dim, s.value_dim)
-        mixed = step.scratch("delta_mixed", (T, V), act)
+        mixed = step.scratch("delta_mixed", (T, V), self.ctx.act_dtype)
         ops.head_norm_gate(o, self.gain, proj[:, 2 * QK + V:], mixed, s.n_heads,
                            float(s.norm_eps))
+        return mixed
+
+    def forward(self, h, residual, step, cache, accumulate: bool = True) -> None:
+        if hasattr(h, "materialize"):
+            h = h.materialize()
+        into = self.into(h, step)
+        products(into)
+        mixed = self.between([out for _, _, out, _ in into], step, cache)
         self.o.forward(mixed, residual, accumulate=accumulate, step=step if accumulate else None)
 
 
@@ -181,13 +191,21 @@ class ParallelMixer(Mixer):
             self.left.forward(h, y, step, cache, accumulate=False)
             self.right.forward(h, y, step, cache, accumulate=True)
             return [(y, 1.0)]
-        out = []
-        for name, part, factor in (("branch", self.left, self.factors[0]),
-                                   ("branch_right", self.right, self.factors[1])):
-            y = step.scratch(name, (h.shape[0], self.spec.left.hidden_size), torch.float32)
-            part.forward(h, y, step, cache, accumulate=False)
-            out.append((y, factor))
-        return out
+        out = [step.scratch(name, (h.shape[0], self.spec.left.hidden_size), torch.float32)
+               for name in ("branch", "branch_right")]
+        if all(hasattr(part, "between") and getattr(part, "o_bias", None) is None
+               for part in self.parts):
+            # both mixers' input products in one launch where a kernel takes them, their output
+            # products in another
+            into = [part.into(h, step) for part in self.parts]
+            products(into[0] + into[1])
+            rows = [part.between([y for _, _, y, _ in i], step, cache)
+                    for part, i in zip(self.parts, into)]
+            products([(r, part.o, y, None) for r, part, y in zip(rows, self.parts, out)])
+        else:
+            for part, y in zip(self.parts, out):
+                part.forward(h, y, step, cache, accumulate=False)
+        return list(zip(out, self.factors))
 
     def forward(self, h, residual, step, cache, accumulate: bool = True) -> None:
         if self.factors != [1.0, 1.0]:

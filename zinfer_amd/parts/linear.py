@@ -49,6 +49,20 @@ class Linear:
         return ops.gemm_partials(x, self.weight, ks)
 
 
+def products(items) -> None:
+    """``items``: (x, linear, out, activation or None) each, out = activation(x W^T), in one launch
+    where a kernel takes them together, the same bits (``ops.gemm_many``)."""
+    many = [(x, linear.weight, linear.tiled, out, act) for x, linear, out, act in items]
+    if ops.gemm_many_covers(many):
+        ops.gemm_many(many)
+        return
+    for x, linear, out, act in items:
+        if act is None:
+            linear.forward(x, out)
+        else:
+            ops.gemm_activation(x, linear.weight, out, act, linear.tiled)
+
+
 def place_matrix(t: torch.Tensor, ctx) -> torch.Tensor:
     """A matrix on the device: bfloat16 stays bfloat16 under a bfloat16 build, a tensor
     stored in 32-bit stays so; a float32 build widens everything (float16 exactly).  A

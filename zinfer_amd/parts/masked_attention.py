@@ -9,7 +9,7 @@ from ..config.distance import bucket_of_distances
 from ..config.specs import LatentAttentionSpec, MaskedGqaAttentionSpec
 from ..errors import ConfigError, StepError
 from .base import KVNeed, Mixer, TensorDecl, register_part
-from .linear import Linear, place_gain, place_matrix
+from .linear import Linear, place_gain, place_matrix, products
 
 
 def _frequencies(rotary, ctx):
@@ -159,16 +159,25 @@ class MaskedGqaAttention(Mixer):
                                   f"a cache of {pool.dtype} needs a model built with that dtype")
 
     def forward(self, h, residual, step, cache, accumulate: bool = True) -> None:
-        s = self.spec
-        T = h.shape[0]
-        act = self.ctx.act_dtype
         if hasattr(h, "materialize"):
             h = h.materialize()
-        proj = step.scratch("qkvg", (T, self.proj.out_features), act)
-        self.proj.forward(h, proj)
-        attn = step.scratch("attn", (T, s.n_heads * s.value_dim), act)
-        self.inner(proj, attn, step, cache)
+        into = self.into(h, step)
+        products(into)
+        attn = self.between([out for _, _, out, _ in into], step, cache)
         finish(self.o, self.o_bias, attn, residual, accumulate, step)
+
+    def into(self, h, step):
+        """The products that read the mixer's input, as ``products`` takes them."""
+        return [(h, self.proj, step.scratch("qkvg", (h.shape[0], self.proj.out_features),
+                                            self.ctx.act_dtype), None)]
+
+    def between(self, rows, step, cache):
+        """From what the products of ``into`` left (``rows``) to what the output product reads."""
+        s = self.spec
+        proj, = rows
+        attn = step.scratch("attn", (proj.shape[0], s.n_heads * s.value_dim), self.ctx.act_dtype)
+        self.inner(proj, attn, step, cache)
+        return attn
 
     def inner(self, proj, attn, step, cache) -> None:
         """From the rows [q | k | v | head gates] of the input product to the heads' outputs."""

@@ -8,7 +8,7 @@ from .. import ops
 from ..config.specs import GatedLinearAttentionSpec, TokenShiftRecurrenceSpec
 from ..errors import ConfigError
 from .base import Mixer, StateNeed, TensorDecl, register_part
-from .linear import Linear, place_gain, place_matrix
+from .linear import Linear, place_gain, place_matrix, products
 
 
 def _check_heads(n_heads: int, head_dim: int, value_dim: int) -> None:
@@ -86,9 +86,8 @@ class GatedLinearAttention(Mixer):
             h = h.materialize()
         QK, V = self.qk_width, self.v_width
         proj = step.scratch("rec_proj", (T, self.proj.out_features), act)
-        self.proj.forward(h, proj)
         low = step.scratch("rec_decay_low", (T, self.rank), act)
-        self.decay_down.forward(h, low)
+        products([(h, self.proj, proj, None), (h, self.decay_down, low, None)])
         z = step.scratch("rec_decay_z", (T, QK), torch.float32)
         self.decay_up.forward(low, z)
         o = step.scratch("rec_out", (T, V), torch.float32)
@@ -162,11 +161,9 @@ class TokenShiftRecurrence(Mixer):
         ops.token_shift_mix(h, self.mu, cache.state, self.matrix_size, step.state_slots,
                             step.seq_index, step.q_start, mixes)
         rkvg = step.scratch("shift_rkvg", (4, T, self.width), act)
-        for i, product in enumerate(self.products):
-            product.forward(mixes[i], rkvg[i])
         low = step.scratch("rec_decay_low", (T, self.rank), act)
-        self.decay_down.forward(mixes[4], low)
-        ops.activation(low, low, "tanh")
+        products([(mixes[i], product, rkvg[i], None) for i, product in enumerate(self.products)]
+                 + [(mixes[4], self.decay_down, low, "tanh")])
         z = step.scratch("rec_decay_z", (T, self.width), torch.float32)
         self.decay_up.forward(low, z)
         o = step.scratch("rec_out", (T, self.width), torch.float32)
