@@ -378,6 +378,43 @@ def test_delta_rule_in_one_step_and_in_portions(H, KH, d, dv):
     assert torch.equal(torch.stack(rows), whole[at[0]:at[1]])
 
 
+@pytest.mark.parametrize("H,KH,d,dv", [(4, 2, 64, 64), (2, 1, 128, 32), (3, 3, 128, 16)])
+@pytest.mark.parametrize("decay", ["usual", "none", "all"])
+def test_delta_rule_of_long_portions_in_chunks(H, KH, d, dv, decay):
+    """Portions beyond the walk's longest (whole and part chunks) beside shorter ones, onto states
+    that earlier portions left: as close to the 64-bit rule as the walk, in other slots' company;
+    with decays of 1 and with some that leave nothing."""
+    lens = [129, 1, 128, 271, 400]
+    size = (ops.delta_state_size(H, d, dv) + 3) // 4 * 4 + 8
+    data = [_delta_inputs(n, H, KH, d, dv, 90 + 3 * i) for i, n in enumerate(lens)]
+    a_log, dt_bias = data[0][2], data[0][3]
+    for _, ab, _, _ in data:
+        if decay == "none":
+            ab[:, :H] = -40.0
+        elif decay == "all":
+            ab[::5, :H] = 1e4
+    slots, n_all = [6, 1, 2, 0, 4], sum(lens)
+    qkv, ab = (torch.cat([x[i] for x in data]).to(DEV) for i in (0, 1))
+    start = torch.randn((7, size), generator=torch.Generator().manual_seed(3)) * 0.3
+    matrices = ops.delta_state_matrix(start, H, d, dv).clone()
+    results = []
+    for q_lens in (lens, None):
+        state, out = start.to(DEV), torch.full((n_all, H * dv), float("nan"), device=DEV)
+        ops.delta_recurrence(qkv, 0, KH * d, 2 * KH * d, ab, a_log.to(DEV), dt_bias.to(DEV), state,
+                             _i32(slots), _i32(_starts(lens)), out, H, KH, d, dv, q_lens=q_lens)
+        assert torch.equal(state.cpu()[[3, 5]], start[[3, 5]])
+        results.append((out.cpu(), ops.delta_state_matrix(state, H, d, dv).cpu()))
+    at = _starts(lens)
+    for i, (q, z, _, _) in enumerate(data):
+        want, S = _delta_reference(q, z, a_log, dt_bias, H, KH, d, dv, matrices[slots[i]].double())
+        rows = slice(at[i], at[i + 1])
+        errors = [(rel_err(out[rows], want), rel_err(mats[slots[i]], S)) for out, mats in results]
+        if lens[i] <= ops.DELTA_WALK_MAX:
+            assert torch.equal(results[0][0][rows], results[1][0][rows])
+        for chunked, walked in zip(*errors):
+            assert chunked < max(1.5 * walked, 1e-6), (lens[i], errors)
+
+
 def test_a_token_far_back_is_kept_without_decay_and_lost_with_it():
     """Two heads, 600 tokens.  Token 3 alone writes the key e_0 with a value that stands out;
     the last token asks for e_0.  The head whose decay is 1 to rounding (a rate of exp(-30))

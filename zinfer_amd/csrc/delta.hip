@@ -12,6 +12,7 @@
 //                      from the request's state.
 //  * short_conv_state  the state takes the step's last taps - 1 rows.
 //  * delta_recurrence  the recurrence over the rows of a step, sequence by sequence.
+//  * delta_chunk_*     the same for long portions, sixteen tokens at a time as 32-bit matrix products.
 //
 // With r = S^T k and p = S^T q of the matrix *before* the token (both formed in one pass over
 // it), w = beta (v - g r), o = g p + (q . k) w and S <- g S + k w^T: the same numbers as the
@@ -414,9 +415,9 @@ __global__ __launch_bounds__(256) void delta_recurrence_kernel(
     const float* __restrict__ ab, const float* __restrict__ a_log,
     const float* __restrict__ dt_bias, float* __restrict__ state, long long state_stride,
     const int* __restrict__ state_slots, const int* __restrict__ q_start, float* __restrict__ out,
-    int H, int KH, int d, int dv, int cols) {
-  // (fused multiply-adds as the compiler forms them: this one kernel walks every portion, whole
-  // prompt or single token, so every cut of a sequence gets the same instructions)
+    int H, int KH, int d, int dv, int cols, int longest) {
+  // (fused multiply-adds as the compiler forms them: this one kernel walks every portion up to
+  // `longest` tokens, so every cut of a sequence into such gets the same instructions)
   extern __shared__ float lds[];
   const int P = CG * R;
   float* qs = lds;                          // [DL_STAGE][P]
@@ -429,7 +430,7 @@ __global__ __launch_bounds__(256) void delta_recurrence_kernel(
   const int h = blockIdx.y, seq = blockIdx.z;
   const int kh = h / (H / KH);
   const int first = q_start[seq], len = q_start[seq + 1] - first;
-  if (len <= 0) return;
+  if (len <= 0 || len > longest) return;
   const int tid = threadIdx.x, nthreads = blockDim.x;
   const int cg = tid % CG, col_l = tid / CG;
   const int col = blockIdx.x * cols + col_l;
@@ -603,12 +604,13 @@ __global__ __launch_bounds__(256) void delta_recurrence_kernel(
 }
 
 // R * CG >= d is the padded key size P the state is laid out with; cols * CG threads a workgroup
-// (a multiple of 64, at most 256).
+// (a multiple of 64, at most 256).  Sequences that bring more than `longest` tokens are left out.
 extern "C" int zf_delta_recurrence(const float* qkv, int C, int q_off, int k_off, int v_off,
                                    const float* ab, const float* a_log, const float* dt_bias,
                                    float* state, long long state_stride, const int* state_slots,
                                    const int* q_start, float* out, int n_seqs, int H, int KH,
-                                   int d, int dv, int R, int CG, int cols, hipStream_t stream) {
+                                   int d, int dv, int R, int CG, int cols, int longest,
+                                   hipStream_t stream) {
   if (n_seqs <= 0) return 0;
   const int threads = cols * CG;
   if (H < 1 || KH < 1 || H % KH != 0 || d < 1 || dv < 1 || CG < 1 || CG > DL_MAX_LANES ||
@@ -627,11 +629,11 @@ extern "C" int zf_delta_recurrence(const float* qkv, int C, int q_off, int k_off
     if (vec)                                                                                     \
       hipLaunchKernelGGL((delta_recurrence_kernel<RR, GG, true>), grid, block, smem, stream,     \
                          qkv, C, q_off, k_off, v_off, ab, a_log, dt_bias, state, state_stride,   \
-                         state_slots, q_start, out, H, KH, d, dv, cols);                         \
+                         state_slots, q_start, out, H, KH, d, dv, cols, longest);                         \
     else                                                                                         \
       hipLaunchKernelGGL((delta_recurrence_kernel<RR, GG, false>), grid, block, smem, stream,    \
                          qkv, C, q_off, k_off, v_off, ab, a_log, dt_bias, state, state_stride,   \
-                         state_slots, q_start, out, H, KH, d, dv, cols);                         \
+                         state_slots, q_start, out, H, KH, d, dv, cols, longest);                         \
     launched = true;                                                                             \
   }
   bool launched = false;
@@ -640,5 +642,253 @@ extern "C" int zf_delta_recurrence(const float* qkv, int C, int q_off, int k_off
   DL_REC_LAUNCH(8, 4) DL_REC_LAUNCH(12, 4) DL_REC_LAUNCH(8, 8) DL_REC_LAUNCH(12, 8)
   DL_REC_LAUNCH(8, 16) DL_REC_LAUNCH(12, 16) DL_REC_LAUNCH(16, 16)
   if (!launched) return -2;
+  ZF_CHECK_LAUNCH();
+}
+
+// ------------------------------------------------------------------ long portions in chunks
+// Sixteen tokens at a time as products.  With G_t the sum of the chunk's log decays up to token t, the
+// matrix S0 ahead of the chunk and w_t = beta_t (v_t - exp(G_t) S0^T k_t - sum over i < t of
+// exp(G_t - G_i) (k_t . k_i) w_i),
+//   W = Tb (V - exp(G) (K S0)),   Tb = (I + L)^-1 diag(beta),  L_ti = beta_t exp(G_t - G_i) k_t . k_i, i < t
+//   O = exp(G) (Q S0) + M W,      M_ti = exp(G_t - G_i) q_t . k_i, i <= t
+//   S = exp(G_15) S0 + K^T (exp(G_15 - G) W)
+// (the delta rule's chunked form by its triangular system, as published for linear attention).
+// Everything is 32-bit: v_mfma_f32_16x16x4_f32, expf, fused multiply-adds; no ratio of decays exceeds 1.
+// (A token that is not finite makes the whole chunk so.)
+//   * delta_chunk_prepare  a wave a (chunk, head): Tb, M and the decays, all chunks side by side.
+//   * delta_chunk_walk     a workgroup of four waves a (16 value columns, head, sequence) walks the
+//                          chunks with S in the accumulators of the waves, d / 64 blocks of 16 key
+//                          channels each.
+// The walk token by token is bound by the vector units' issue: some 100 instructions a token and
+// wave, 2.5 waves to a SIMD; here a chunk costs a wave 24 MFMAs of 32 cycles (d = 128).
+// Measured (16 heads of 128 x 128, a step of 2048 tokens of five prompts, the longest 680, us): 290
+// walked, 87 + 15 in chunks; on inputs of such sizes 2.3 to 3.3e-7 off the 64-bit rule behind 200 to 2000
+// tokens, the walk 2.9e-7 to 1.1e-6.
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float dl_f32x4_t;
+#define DL_CHUNK 16
+#define DL_CHUNK_FLOATS (2 * DL_CHUNK * DL_CHUNK + 2 * DL_CHUNK)   // Tb, M, exp(G), exp(G_15 - G)
+
+// where chunk c of a sequence keeps its numbers: below (all tokens) / 16 + sequences + 1, no two alike
+__device__ __forceinline__ size_t dl_chunk_at(int first, int seq, int c, int H, int h) {
+  return ((size_t)(first / DL_CHUNK + seq + c) * H + h) * DL_CHUNK_FLOATS;
+}
+
+template <int ND>
+__global__ __launch_bounds__(64) void delta_chunk_prepare_kernel(
+    const float* __restrict__ qkv, int C, int q_off, int k_off, const float* __restrict__ ab,
+    const float* __restrict__ a_log, const float* __restrict__ dt_bias,
+    const int* __restrict__ q_start, float* __restrict__ ws, int H, int KH, int longest) {
+  __shared__ float L[DL_CHUNK][DL_CHUNK + 1], log_g[DL_CHUNK], beta[DL_CHUNK];
+  const int h = blockIdx.y, seq = blockIdx.z, lane = threadIdx.x, m = lane % 16, g = lane / 16;
+  const int first = q_start[seq], len = q_start[seq + 1] - first;
+  const int t0 = blockIdx.x * DL_CHUNK;
+  if (len <= longest || t0 >= len) return;
+  const int n = min(DL_CHUNK, len - t0), kh = h / (H / KH);
+  constexpr int d = 16 * ND;
+  const dl_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  const float* row = qkv + (size_t)(first + t0 + min(m, n - 1)) * C + kh * d + 4 * g;
+  dl_f32x4_t kk = zero, qk = zero, kf[ND], qf[ND];
+#pragma unroll
+  for (int b = 0; b < ND; ++b) {
+    kf[b] = *(const dl_f32x4_t*)(row + k_off + 16 * b);
+    qf[b] = *(const dl_f32x4_t*)(row + q_off + 16 * b);
+  }
+  if (lane < 16) {
+    const float* z = ab + (size_t)(first + t0 + min(lane, n - 1)) * 2 * H;
+    const float za = z[h], zb = z[H + h];
+    // a token that is not there decays nothing and corrects nothing; exp(-110) is 0 as a float, and
+    // sums of such stay finite
+    const float v = -(expf(a_log[h]) * dl_softplus(za + dt_bias[h]));
+    log_g[lane] = lane >= n ? 0.f : v < -110.f ? -110.f : v;
+    beta[lane] = lane < n ? 1.0f / (1.0f + expf(-zb)) : 0.f;
+  }
+  // (rows of a token that is not there repeat the last one's; their columns are masked below)
+#pragma unroll
+  for (int b = 0; b < ND; ++b)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      kk = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[b][i], kf[b][i], kk, 0, 0, 0);
+      qk = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[b][i], kf[b][i], qk, 0, 0, 0);
+    }
+  __syncthreads();
+  // Column m is token i = m, the four rows are tokens t = 4 g + r.  The decays between two tokens
+  // are added up from the earlier one on: the difference of two sums from the chunk's start would lose
+  // the digits that a token which forgets everything has taken.
+  float* dst = ws + dl_chunk_at(first, seq, blockIdx.x, H, h);
+  float since = 0.f, start = 0.f, whole = 0.f, ratio[4];
+#pragma unroll
+  for (int t = 0; t < DL_CHUNK; ++t) {
+    const float v = log_g[t];
+    whole += v;
+    since = t > m ? since + v : 0.f;
+    if (t == m) start = whole;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (t == 4 * g + r) ratio[r] = t >= m ? expf(since) : 0.f;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int t = 4 * g + r;
+    L[t][m] = t > m && m < n ? beta[t] * ratio[r] * kk[r] : 0.f;
+    dst[DL_CHUNK * DL_CHUNK + t * DL_CHUNK + m] = m < n ? ratio[r] * qk[r] : 0.f;
+  }
+  if (lane < 16) {
+    dst[2 * DL_CHUNK * DL_CHUNK + lane] = expf(start);
+    dst[2 * DL_CHUNK * DL_CHUNK + DL_CHUNK + lane] = expf(since);
+  }
+  __syncthreads();
+  // (I + L)^-1, a column a lane, row after row
+  if (lane < 16) {
+    float x[DL_CHUNK];
+#pragma unroll
+    for (int t = 0; t < DL_CHUNK; ++t) {
+      float v = t == lane ? 1.f : 0.f;
+#pragma unroll
+      for (int i = 0; i < t; ++i) v = fmaf(-L[t][i], x[i], v);
+      x[t] = v;
+    }
+    const float b = beta[lane];
+#pragma unroll
+    for (int t = 0; t < DL_CHUNK; ++t) dst[t * DL_CHUNK + lane] = x[t] * b;
+  }
+}
+
+template <int ND>
+__global__ __launch_bounds__(256) void delta_chunk_walk_kernel(
+    const float* __restrict__ qkv, int C, int q_off, int k_off, int v_off, float* __restrict__ state,
+    long long state_stride, const int* __restrict__ state_slots, const int* __restrict__ q_start,
+    const float* __restrict__ ws, float* __restrict__ out, int H, int KH, int dv, int longest) {
+  constexpr int d = 16 * ND, B = ND / 4, LD = d + 4, LM = DL_CHUNK + 4;
+  constexpr int PIECES = DL_CHUNK * d / 4 / 256;          // 16-byte pieces of K (and of Q) a thread
+  static_assert(ND % 4 == 0 && PIECES >= 1, "blocks of channels for four waves");
+  __shared__ __attribute__((aligned(16))) float ks[DL_CHUNK][LD], qs[DL_CHUNK][LD];
+  __shared__ __attribute__((aligned(16))) float mats[2][DL_CHUNK][LM];   // Tb, M
+  __shared__ float vs[DL_CHUNK][DL_CHUNK + 1], decays[2][DL_CHUNK];
+  __shared__ dl_f32x4_t red[4][2][64];
+  const int h = blockIdx.y, seq = blockIdx.z, kh = h / (H / KH);
+  const int first = q_start[seq], len = q_start[seq + 1] - first;
+  if (len <= longest) return;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
+  const int m = lane % 16, g = lane / 16, col0 = blockIdx.x * 16;
+  // S: row 4 g + r of block wave * B + b is key channel 16 (wave B + b) + 4 g + r, column m
+  float* S_mem = state + (size_t)state_slots[seq] * state_stride + ((size_t)h * dv + col0 + m) * d
+                 + 16 * wave * B + 4 * g;
+  dl_f32x4_t S[B];
+#pragma unroll
+  for (int b = 0; b < B; ++b) S[b] = *(const dl_f32x4_t*)(S_mem + 16 * b);
+  dl_f32x4_t fk[PIECES], fq[PIECES];
+  float fv, fm[2], fd;
+  auto fetch = [&](int t0) {
+    const int n = min(DL_CHUNK, len - t0);
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+      const int i = tid + 256 * j, tok = i / (d / 4), c = i % (d / 4) * 4;
+      const float* row = qkv + (size_t)(first + t0 + min(tok, n - 1)) * C + kh * d + c;
+      fk[j] = *(const dl_f32x4_t*)(row + k_off);
+      fq[j] = *(const dl_f32x4_t*)(row + q_off);
+    }
+    const int tok = tid / 16;
+    fv = qkv[(size_t)(first + t0 + min(tok, n - 1)) * C + v_off + h * dv + col0 + tid % 16];
+    const float* src = ws + dl_chunk_at(first, seq, t0 / DL_CHUNK, H, h);
+    fm[0] = src[tid];
+    fm[1] = src[256 + tid];
+    fd = src[512 + tid % 32];
+  };
+  fetch(0);
+  for (int t0 = 0; t0 < len; t0 += DL_CHUNK) {
+    const int n = min(DL_CHUNK, len - t0);
+    __syncthreads();                        // the chunk before is done with
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+      const int i = tid + 256 * j, tok = i / (d / 4), c = i % (d / 4) * 4;
+      *(dl_f32x4_t*)&ks[tok][c] = fk[j];
+      *(dl_f32x4_t*)&qs[tok][c] = fq[j];
+    }
+    vs[tid / 16][tid % 16] = fv;
+    mats[0][tid / 16][tid % 16] = fm[0];
+    mats[1][tid / 16][tid % 16] = fm[1];
+    if (tid < 32) decays[tid / 16][tid % 16] = fd;
+    __syncthreads();
+    if (t0 + DL_CHUNK < len) fetch(t0 + DL_CHUNK);
+    // this wave's channels' share of K S0 and Q S0 (element i of a lane's four channels in MFMA i,
+    // where S has the same ones as element i of its rows)
+    dl_f32x4_t pk = {0.f, 0.f, 0.f, 0.f}, pq = pk;
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const dl_f32x4_t kv = *(const dl_f32x4_t*)&ks[m][16 * (wave * B + b) + 4 * g];
+      const dl_f32x4_t qv = *(const dl_f32x4_t*)&qs[m][16 * (wave * B + b) + 4 * g];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        pk = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i], S[b][i], pk, 0, 0, 0);
+        pq = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[i], S[b][i], pq, 0, 0, 0);
+      }
+    }
+    red[wave][0][lane] = pk;
+    red[wave][1][lane] = pq;
+    __syncthreads();
+    // rows 4 g + r are tokens, column m a value column; every wave forms W for its own channels
+    const dl_f32x4_t sk = (red[0][0][lane] + red[1][0][lane]) + (red[2][0][lane] + red[3][0][lane]);
+    const dl_f32x4_t tb = *(const dl_f32x4_t*)&mats[0][m][4 * g];
+    dl_f32x4_t x, W = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[r] = fmaf(-decays[0][4 * g + r], sk[r], vs[4 * g + r][m]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) W = __builtin_amdgcn_mfma_f32_16x16x4f32(tb[i], x[i], W, 0, 0, 0);
+    const float whole = decays[0][DL_CHUNK - 1];
+    float cw[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cw[i] = decays[1][4 * g + i] * W[i];
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      float kt[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) kt[i] = ks[4 * g + i][16 * (wave * B + b) + m];
+      S[b] = S[b] * whole;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[i], cw[i], S[b], 0, 0, 0);
+    }
+    if (wave == t0 / DL_CHUNK % 4) {        // the outputs, the waves in turn
+      const dl_f32x4_t sq = (red[0][1][lane] + red[1][1][lane]) + (red[2][1][lane] + red[3][1][lane]);
+      const dl_f32x4_t mv = *(const dl_f32x4_t*)&mats[1][m][4 * g];
+      dl_f32x4_t o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = decays[0][4 * g + r] * sq[r];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o = __builtin_amdgcn_mfma_f32_16x16x4f32(mv[i], W[i], o, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * g + r < n)
+          out[(size_t)(first + t0 + 4 * g + r) * H * dv + (size_t)h * dv + col0 + m] = o[r];
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < B; ++b) *(dl_f32x4_t*)(S_mem + 16 * b) = S[b];
+}
+
+// The sequences that bring more than `longest` tokens (max_len: what the longest one brings), in chunks;
+// d 64 or 128 (the padded key size too), dv a multiple of 16, 16-byte aligned rows; ws: (T / 16 +
+// n_seqs + 1) * H * DL_CHUNK_FLOATS floats.
+extern "C" int zf_delta_chunks(const float* qkv, int C, int q_off, int k_off, int v_off,
+                               const float* ab, const float* a_log, const float* dt_bias,
+                               float* state, long long state_stride, const int* state_slots,
+                               const int* q_start, float* out, float* ws, int n_seqs, int max_len,
+                               int H, int KH, int d, int dv, int longest, hipStream_t stream) {
+  if (n_seqs <= 0 || max_len <= longest) return 0;
+  if (H < 1 || KH < 1 || H % KH != 0 || (d != 64 && d != 128) || dv < 16 || dv % 16 != 0 ||
+      (C | q_off | k_off) % 4 != 0 || state_stride % 4 != 0 ||
+      (((uintptr_t)qkv | (uintptr_t)state) % 16) != 0 || ws == nullptr || longest < 0)
+    return -2;
+  const dim3 pgrid((max_len + DL_CHUNK - 1) / DL_CHUNK, H, n_seqs), wgrid(dv / 16, H, n_seqs);
+#define DL_CHUNKS(ND)                                                                            \
+  do {                                                                                           \
+    hipLaunchKernelGGL((delta_chunk_prepare_kernel<ND>), pgrid, dim3(64), 0, stream, qkv, C, q_off, \
+                       k_off, ab, a_log, dt_bias, q_start, ws, H, KH, longest);                  \
+    hipLaunchKernelGGL((delta_chunk_walk_kernel<ND>), wgrid, dim3(256), 0, stream, qkv, C, q_off, \
+                       k_off, v_off, state, state_stride, state_slots, q_start, ws, out, H, KH, dv, \
+                       longest);                                                                 \
+  } while (0)
+  if (d == 64) DL_CHUNKS(4); else DL_CHUNKS(8);
+#undef DL_CHUNKS
   ZF_CHECK_LAUNCH();
 }

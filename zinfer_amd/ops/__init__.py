@@ -7,7 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
-from typing import Optional, Tuple
+from typing import Optional, Sequence, Tuple
 
 import torch
 
@@ -3371,11 +3371,22 @@ def short_conv(src: torch.Tensor, taps: torch.Tensor, state: torch.Tensor, state
            "short_conv")
 
 
+DELTA_WALK_MAX = 128      # a portion of more tokens may run in chunks (``delta_recurrence``)
+DELTA_CHUNK, DELTA_CHUNK_FLOATS = 16, 2 * 16 * 16 + 2 * 16      # DL_CHUNK, DL_CHUNK_FLOATS
+
+
+def delta_chunks_cover(C: int, q_off: int, k_off: int, d: int, dv: int) -> bool:
+    """Whether long portions of the delta rule run in chunks: key sizes that are padded by nothing
+    and give four waves whole blocks of 16 channels."""
+    return d in (64, 128) and dv % 16 == 0 and C % 4 == 0 and q_off % 4 == 0 and k_off % 4 == 0
+
+
 @_launches("attention")
 def delta_recurrence(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, ab: torch.Tensor,
                      decay_log: torch.Tensor, decay_bias: torch.Tensor, state: torch.Tensor,
                      state_slots: torch.Tensor, q_start: torch.Tensor, out: torch.Tensor,
-                     n_heads: int, n_kv_heads: int, key_dim: int, value_dim: int) -> None:
+                     n_heads: int, n_kv_heads: int, key_dim: int, value_dim: int,
+                     q_lens: Optional[Sequence[int]] = None) -> None:
     """The gated delta rule a head, token by token in 32-bit, over the rows of a step:
     S <- g S; w = beta (v - S^T k); S <- S + k w^T; o = S^T q.  ``qkv`` float32 [T, C] holds
     ``n_kv_heads`` q heads of ``key_dim`` from column q_off, as many k heads from k_off and
@@ -3385,7 +3396,10 @@ def delta_recurrence(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, ab: 
     (``decay_log``, ``decay_bias`` float32 [H]).  ``out`` float32 [T, H * dv].  Sequence s owns
     the rows q_start[s] .. q_start[s + 1] - 1; its matrices (the leading ``delta_state_size``
     floats of row state_slots[s] of ``state``) are read before its first row and written behind
-    its last.  A row's result depends on the state and the rows of its own sequence alone."""
+    its last.  A row's result depends on the state and the rows of its own sequence alone; with
+    ``q_lens`` (the sequences' rows, on the host) a sequence that brings more than
+    ``DELTA_WALK_MAX`` runs in chunks of products where the sizes allow (``delta_chunks_cover``),
+    in 32-bit too, and its results then agree with the walk's up to rounding."""
     _need_gpu(qkv, ab, decay_log, decay_bias, state, state_slots, q_start, out)
     _i32(state_slots, "state_slots")
     _i32(q_start, "q_start")
@@ -3413,11 +3427,24 @@ def delta_recurrence(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, ab: 
     # a workgroup: whole waves, at most 256 threads, no more columns than the head has
     cols = min(256, (dv * lanes + 63) // 64 * 64) // lanes
     lib = build.load("delta")
+    longest = (1 << 31) - 1
+    if q_lens is not None and max(q_lens) > DELTA_WALK_MAX and len(q_lens) == n_seqs \
+            and delta_chunks_cover(C, q_off, k_off, d, dv) and qkv.data_ptr() % 16 == 0:
+        longest = DELTA_WALK_MAX
+        ws = _workspace("delta_chunks", (T // DELTA_CHUNK + n_seqs + 1) * H * DELTA_CHUNK_FLOATS,
+                        torch.float32, qkv.device)
+        _check(lib.zf_delta_chunks(_ptr(qkv), C, int(q_off), int(k_off), int(v_off), _ptr(ab),
+                                   _ptr(decay_log), _ptr(decay_bias), _ptr(state),
+                                   ctypes.c_longlong(state.stride(0)), _ptr(state_slots),
+                                   _ptr(q_start), _ptr(out), _ptr(ws), n_seqs, int(max(q_lens)), H, KH,
+                                   d, dv, longest, _stream()), "delta_recurrence (chunks)")
+        if min(q_lens) > longest:
+            return
     _check(lib.zf_delta_recurrence(_ptr(qkv), C, int(q_off), int(k_off), int(v_off), _ptr(ab),
                                    _ptr(decay_log), _ptr(decay_bias), _ptr(state),
                                    ctypes.c_longlong(state.stride(0)), _ptr(state_slots),
                                    _ptr(q_start), _ptr(out), n_seqs, H, KH, d, dv, r, lanes, cols,
-                                   _stream()), "delta_recurrence")
+                                   longest, _stream()), "delta_recurrence")
 
 
 # ------------------------------------------------------------------------- a state space with one decay a head and token

@@ -113,7 +113,9 @@ class GatedDeltaRule(Mixer):
         o = step.scratch("delta_out", (T, V), torch.float32)
         ops.delta_recurrence(qkv, 0, QK, 2 * QK, ab, self.decay_log, self.decay_bias, cache.state,
                              step.state_slots, step.q_start, o, s.n_heads, s.n_kv_heads,
-                             s.head_dim, s.value_dim)
+                             s.head_dim, s.value_dim,
+                             # (a 32-bit prompt's bits do not depend on where it is cut)
+                             q_lens=None if self.ctx.act_dtype == torch.float32 else step.q_lens)
         mixed = step.scratch("delta_mixed", (T, V), self.ctx.act_dtype)
         ops.head_norm_gate(o, self.gain, proj[:, 2 * QK + V:], mixed, s.n_heads,
                            float(s.norm_eps))
