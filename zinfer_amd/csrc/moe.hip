@@ -1135,7 +1135,9 @@ __global__ __launch_bounds__(1024) void moe_few_down_kernel(
     for (int i = lane; i < P; i += ZF_WAVE) share[i] = weights[i];
   // one wave lists the units, in the order of their first pairs
   if (wave == 0) {
-    int mine[4], rank[4] = {0, 0, 0, 0};                // this lane's pairs: experts, ranks in them
+    // This lane's pairs: experts, ranks among their expert's pairs, and the pair that starts their unit.
+    // Pair j's own rank is there when its turn comes.
+    int mine[4], rank[4] = {0, 0, 0, 0}, lead[4] = {0, 0, 0, 0};
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const int i = 64 * c + lane;
@@ -1147,25 +1149,32 @@ __global__ __launch_bounds__(1024) void moe_few_down_kernel(
     for (int cj = 0; cj < 4; ++cj)
       for (int j = 0; j < min(64, P - 64 * cj); ++j) {
         const int e = __builtin_amdgcn_readlane(mine[cj], j);
+        const bool starts = __builtin_amdgcn_readlane(rank[cj], j) % 8 == 0;
 #pragma unroll
         for (int c = cj; c < 4; ++c)
-          if (64 * c < P) rank[c] += mine[c] == e && (c > cj || j < lane);
+          if (64 * c < P) {
+            const bool same = mine[c] == e && (c > cj || j <= lane);
+            if (same && starts) lead[c] = 64 * cj + j;
+            rank[c] += same && (c > cj || j < lane);
+          }
       }
+    unsigned long long first[4];
+    int units = 0, before[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      first[c] = __ballot(mine[c] < n_experts && rank[c] % 8 == 0);
+      before[c] = units;
+      units += __popcll(first[c]);
+    }
 #pragma unroll
     for (int c = 0; c < 4; ++c)
-      if (mine[c] >= n_experts) rank[c] = -1;
-    int units = 0;
-#pragma unroll
-    for (int cj = 0; cj < 4; ++cj)
-      for (int j = 0; j < min(64, P - 64 * cj); ++j) {
-        const int e = __builtin_amdgcn_readlane(mine[cj], j), rj = __builtin_amdgcn_readlane(rank[cj], j);
-        if (rj < 0 || rj % 8 != 0) continue;
-        if (lane == 0) expert[units] = e;
-#pragma unroll
-        for (int c = cj; c < 4; ++c)
-          if (mine[c] == e && rank[c] >= rj && rank[c] < rj + 8)
-            pairs[units][rank[c] - rj] = (short)(64 * c + lane);
-        ++units;
+      if (mine[c] < n_experts) {
+        const int cl = lead[c] / 64, l = lead[c] % 64;
+        const unsigned long long f = cl == 0 ? first[0] : cl == 1 ? first[1] : cl == 2 ? first[2] : first[3];
+        const int unit = (cl == 0 ? before[0] : cl == 1 ? before[1] : cl == 2 ? before[2] : before[3]) +
+                         __popcll(f & ((1ull << l) - 1));
+        pairs[unit][rank[c] % 8] = (short)(64 * c + lane);
+        if (rank[c] % 8 == 0) expert[unit] = mine[c];
       }
     if (lane == 0) n_units = units;
   }
@@ -1177,8 +1186,8 @@ __global__ __launch_bounds__(1024) void moe_few_down_kernel(
     const int nb = shared ? s_blocks : blocks;
     int pair;
     const bf16_t *wr, *x;
-    // (the two halves of the blocks in a sum each, the pieces' sums four side by side: the outputs of ff
-    // = 4096 from given activations 1.34e-7 off with one sum, 1.04e-7 so, 1.05e-7 row by row)
+    // (the two halves of even and odd steps in a sum each, the pieces' sums four side by side: the
+    // outputs of ff = 4096 from given activations 1.34e-7 off with one sum, 1.04e-7 so, 1.05e-7 row by row)
     // rows r and columns r: output n0 + r % 8 and pair r % 8 at the blocks 2 i + r / 8
     for (int p0 = 0; p0 < (shared ? T : 8); p0 += 8) {
       if (shared) {
@@ -1193,9 +1202,12 @@ __global__ __launch_bounds__(1024) void moe_few_down_kernel(
       wr += (size_t)(n0 / 16) * nb * 1024 + (g * 16 + n0 % 16 + r % 8) * 8;
       x += 16 * g;
       const int b0 = c * 2 * piece, b1 = min(nb, b0 + 2 * piece);
-      moe_f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll 4
-      for (int kb = b0; kb < b1; kb += 2) {
+      moe_f32x4_t acc[2][2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[j][i] = moe_f32x4_t{0.f, 0.f, 0.f, 0.f};
+      auto take = [&](int kb, moe_f32x4_t (&sum)[2]) {
         // (behind an odd last block the upper half repeats it against zeros)
         const bool in = kb + half < b1;
         const int k = in ? kb + half : kb;
@@ -1208,14 +1220,19 @@ __global__ __launch_bounds__(1024) void moe_few_down_kernel(
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&wf[i],
-                                                           *(const moe_bf16x8_t*)&xf[i], acc[i], 0, 0, 0);
+          sum[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&wf[i],
+                                                           *(const moe_bf16x8_t*)&xf[i], sum[i], 0, 0, 0);
+      };
+#pragma unroll 2
+      for (int kb = b0; kb < b1; kb += 4) {
+        take(kb, acc[0]);
+        if (kb + 2 < b1) take(kb + 2, acc[1]);
       }
       // rows 4 g + i of column r: like halves are g / 2 == half
       if (pair >= 0 && g / 2 == half)
         *(moe_f32x4_t*)((shared ? s_sums + ((size_t)pair * s_pieces + c) * 16
                                 : sums + ((size_t)pair * pieces + c) * 16) + 8 * half + 4 * (g % 2)) =
-            acc[0] + acc[1];
+            (acc[0][0] + acc[0][1]) + (acc[1][0] + acc[1][1]);
     }
   }
   __syncthreads();
@@ -1266,9 +1283,11 @@ extern "C" int zf_moe_few(const void* h, const void* gate_up, const void* down, 
                      s_limit, s_alpha, s_shift, factor, factor_stride)
   if (gated) MOE_FEW_UP(true); else MOE_FEW_UP(false);
 #undef MOE_FEW_UP
-  // pieces of 2 x 128 of ff, larger ones where the partials of 16 tokens would not fit 48 KB of
-  // LDS (by the layer's sizes alone: a token's sums must not depend on how many tokens there are)
-  int piece = 2;
+  // pieces of up to 8 blocks of ff, as even as they come, larger ones where the partials of 16 tokens
+  // would not fit 48 KB of LDS (by the layer's sizes alone: a token's sums must not depend on how
+  // many tokens there are)
+  const int parts = (ff / 64 + 7) / 8;
+  int piece = (ff / 64 + 2 * parts - 1) / (2 * parts);
   const auto pieces = [](int width, int p) { return (width / 64 + 2 * p - 1) / (2 * p); };
   const auto lds = [&](int tokens, int p) {
     return (size_t)tokens * (top * pieces(ff, p) + pieces(shared_ff, p)) * 64;
