@@ -1240,6 +1240,24 @@ def test_gemm_many_gives_the_products_own_bits(M, K, widths):
         assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(64, 4096), (2048, 4160), (1984, 7168)])
+@pytest.mark.parametrize("kind", ["sum", "f32", "bf16"])
+def test_narrow_products_over_a_long_k_in_parts(M, N, K, kind):
+    ops = _ops()
+    a = _rand((M, K), torch.bfloat16, 38).to(DEV)
+    w = _rand((N, K), torch.bfloat16, 39, 0.05).to(DEV)
+    assert ops._narrow_split(M, N, K) is not None and ops._narrow_split(M, N, 4032) is None
+    out = _rand((M, N), torch.float32, 40).to(DEV)
+    want = a.double() @ w.double().T + (out.double() if kind == "sum" else 0.0)
+    bound = (K + 1) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + out.double().abs())
+    if kind == "bf16":
+        out = torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
+        bound = bound + want.abs() * 2.0 ** -8
+    ops.gemm(a, ops.pretile_weight(w), out, accumulate=kind == "sum", w_tiled=True)
+    assert bool(((out.double() - want).abs() <= bound).all())
+
+
 def test_cpu_tensor_is_refused():
     """There is no CPU path: a tensor that is not on the GPU is an error, not a fallback."""
     from zinfer_amd.errors import KernelUnavailable

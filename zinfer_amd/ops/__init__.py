@@ -578,6 +578,18 @@ def _skinny_plan(M: int, N: int, K: int, tiled: bool):
     return rg, ks
 
 
+def _narrow_split(M: int, N: int, K: int):
+    """Row groups per workgroup and workgroups along K for a product of up to 16 tokens whose output
+    has too few row groups for half of the chip, over a long K, that has no epilogue to lose by the split:
+    a second kernel adds the parts.  Measured on MI355X, us with that kernel: 2048 outputs over K =
+    4096 / 7168, 1 token 7.1 -> 7.0, 10.1 -> 9.1, 8 tokens 8.3 -> 7.7, 12.6 -> 9.6 (two parts); 16
+    tokens, which a workgroup of one row group reads as often as W, 9.0 -> 8.0, 13.7 -> 10.8 (two row
+    groups, four parts).  Over 2048 or 3072 the second kernel costs what the split gains."""
+    if not (0 < M <= 16 and N <= 2048 and N % 32 == 0 and K >= 4096 and K % 64 == 0):
+        return None
+    return (1, 2) if M <= 8 else (2, 4)
+
+
 MID_MAX_M = 128
 
 
@@ -977,7 +989,8 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
             _check(lib.zf_gemm_bf16_mid(_ptr(a), _ptr(w), _ptr(out), _ptr(ws), M, N, K, epi, mid,
                                         _stream()), "gemm (17 to 128 tokens)")
         elif M <= SKINNY_MAX_M:
-            rg, ks = plan[1:] if plan is not None else _skinny_plan(M, N, K, w_tiled)
+            rg, ks = plan[1:] if plan is not None else \
+                (w_tiled and _narrow_split(M, N, K)) or _skinny_plan(M, N, K, w_tiled)
             ws = _workspace("gemm_splitk", ks * M * N, torch.float32, a.device) if ks > 1 else None
             _check(lib.zf_gemm_bf16_skinny(_ptr(a), _ptr(w), _ptr(out), _ptr(ws), M, N, K, epi,
                                            rg, ks, 1 if w_tiled else 0, _stream()),
