@@ -552,6 +552,43 @@ def _attend(q, gate, pool, table, n_ctx, n_q, nH, nKV, hd, page_size, scale, win
     return out
 
 
+@pytest.mark.parametrize("nH, nKV, hd, page", [(4, 2, 32, 16), (9, 3, 96, 8), (16, 4, 128, 16)])
+@pytest.mark.parametrize("window", [0, 1, 33, 100])
+def test_decode_attention_stores_the_tokens_own_rows(nH, nKV, hd, page, window):
+    """Single tokens whose rows are not in the pool yet, at the edges of a page, a chunk and a wave's
+    keys: the output and the pool of the two kernels, bit for bit."""
+    ctx = [1, 2, 16, 17, 32, 33, 64, 65, 129, 300]
+    n, most = len(ctx), (max(ctx) + page - 1) // page
+    perm = torch.randperm(n * most, generator=torch.Generator().manual_seed(5)).to(torch.int32)
+    table = perm.view(n, most)
+    slots = torch.tensor([int(table[i, (c - 1) // page]) * page + (c - 1) % page
+                          for i, c in enumerate(ctx)], dtype=torch.int32, device=DEV)
+    pool = _rand((n * most, nKV * page * hd), 150, dtype=torch.bfloat16).to(DEV)
+    wide = _rand((n, (2 * nH + nKV) * hd), 151, dtype=torch.bfloat16).to(DEV)
+    q, k, gate = wide[:, :nH * hd], wide[:, nH * hd:(nH + nKV) * hd], wide[:, (nH + nKV) * hd:]
+    dev = lambda a: torch.tensor(a, dtype=torch.int32, device=DEV)
+    args = (table.to(DEV), dev(list(range(n + 1))), dev(ctx), dev(list(range(n))))
+    tail = (0.7 / hd ** 0.5, window, True, nH, nKV, hd, page, 1, max(ctx))
+    pools, outs = [pool.clone(), pool.clone()], [torch.empty((n, nH * hd), dtype=torch.bfloat16,
+                                                             device=DEV) for _ in range(2)]
+    ops.kv_rows_write(k, slots, pools[0], nKV, hd, page)
+    ops.tied_attention(q, gate, pools[0], *args, outs[0], *tail)
+    at = ops.launch_count()
+    ops.tied_attention(q, gate, pools[1], *args, outs[1], *tail, new=(k, slots))
+    assert ops.launch_count() == at + 1
+    assert torch.equal(pools[1], pools[0]) and torch.equal(outs[1], outs[0])
+    # what the decode kernel does not take is stored by the kernel for it
+    big = _rand((n, nH * 192), 152, dtype=torch.bfloat16).to(DEV)
+    rows = _rand((n, nKV * 192), 153, dtype=torch.bfloat16).to(DEV)
+    pools = [torch.zeros((n * most, nKV * page * 192), dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    outs = [torch.empty_like(big) for _ in range(2)]
+    tail = (0.05, window, True, nH, nKV, 192, page, 1, max(ctx))
+    ops.kv_rows_write(rows, slots, pools[0], nKV, 192, page)
+    ops.tied_attention(big, None, pools[0], *args, outs[0], *tail)
+    ops.tied_attention(big, None, pools[1], *args, outs[1], *tail, new=(rows, slots))
+    assert torch.equal(pools[1], pools[0]) and torch.equal(outs[1], outs[0])
+
+
 @pytest.mark.parametrize("nH, nKV, hd, page", [(4, 2, 32, 16), (9, 3, 96, 16), (5, 1, 64, 8),
                                                (2, 2, 128, 16), (3, 1, 192, 4), (2, 1, 256, 16),
                                                (40, 2, 32, 16)])

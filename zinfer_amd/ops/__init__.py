@@ -1863,23 +1863,40 @@ def tied_attention_mfma_covers(dtype, n_heads: int, n_kv_heads: int, head_dim: i
 
 
 def tied_attention(q, gate, k_pool, block_table, q_start, ctx_len, seq_index, out, scale, window,
-                   sink, n_heads, n_kv_heads, head_dim, page_size, max_q_len, max_ctx_len) -> None:
+                   sink, n_heads, n_kv_heads, head_dim, page_size, max_q_len, max_ctx_len,
+                   new=None) -> None:
     """``shared_kv_attention`` through the fastest kernel that takes the shape: in bfloat16,
     for the head sizes of ``TIED_MFMA_HEAD_DIMS``, MFMA tiles of 128 (position, head) pairs
     (``tied_attention_mfma``); else the 32-bit kernel.  Same arguments, same result up to
-    rounding."""
-    if tied_attention_mfma_covers(q.dtype, n_heads, n_kv_heads, head_dim):
+    rounding.  ``new`` (rows, slot_mapping): the step's own rows, which ``kv_rows_write`` has not
+    stored yet; the decode kernel stores them itself, else that kernel runs first."""
+    covered = tied_attention_mfma_covers(q.dtype, n_heads, n_kv_heads, head_dim)
+    if new is not None and not (covered and _tied_decodes(q, ctx_len, n_heads, n_kv_heads, head_dim,
+                                                          max_q_len)
+                                and new[0].dtype == q.dtype and new[0].stride(0) % 8 == 0
+                                and new[0].data_ptr() % 16 == 0):
+        kv_rows_write(*new, k_pool, n_kv_heads, head_dim, page_size)
+        new = None
+    if covered:
         tied_attention_mfma(q, gate, k_pool, block_table, q_start, ctx_len, out, scale, window,
-                            sink, n_heads, n_kv_heads, head_dim, page_size, max_q_len, max_ctx_len)
+                            sink, n_heads, n_kv_heads, head_dim, page_size, max_q_len, max_ctx_len,
+                            new=new)
     else:
         shared_kv_attention(q, gate, k_pool, block_table, q_start, ctx_len, seq_index, out, scale,
                             window, sink, n_heads, n_kv_heads, head_dim, page_size, max_ctx_len)
 
 
+def _tied_decodes(q, ctx_len, n_heads: int, n_kv_heads: int, head_dim: int, max_q_len: int) -> bool:
+    """Whether ``tied_attention_mfma`` runs the step through its decode kernel."""
+    return max_q_len == 1 and q.shape[0] == ctx_len.shape[0] and head_dim <= 128 \
+        and n_heads // n_kv_heads <= 32
+
+
 @_launches("attention")
 def tied_attention_mfma(q, gate, k_pool, block_table, q_start, ctx_len, out, scale, window, sink,
                         n_heads, n_kv_heads, head_dim, page_size, max_q_len, max_ctx_len,
-                        n_splits: Optional[int] = None, shared_tiles: Optional[bool] = None) -> None:
+                        n_splits: Optional[int] = None, shared_tiles: Optional[bool] = None,
+                        new=None) -> None:
     """The bfloat16 MFMA form of ``shared_kv_attention`` (see there for the arguments).  Scores
     and the soft-max are 32-bit; a weight enters the second product as the sum of two bfloat16
     numbers.  A step in which every sequence brings one token runs the decode kernel (head
@@ -1888,7 +1905,9 @@ def tied_attention_mfma(q, gate, k_pool, block_table, q_start, ctx_len, out, sca
     the window, never by the contexts themselves, so that a captured step replays for other
     contexts), and the partial results are merged.  Prompt portions of those shapes run the
     same waves-on-their-own scheme, a wave per 32 (position, head) rows; ``shared_tiles`` True
-    (and every other shape) runs the kernel whose workgroup stages the keys once for 128 rows."""
+    (and every other shape) runs the kernel whose workgroup stages the keys once for 128 rows.
+    ``new`` (rows [T, nKV * hd], slot_mapping; the decode kernel only): the tokens' own rows, not
+    yet in the pool, which the kernel stores."""
     for t in (q, gate, k_pool, block_table, q_start, ctx_len, out):
         if t is not None and not t.is_cuda:
             raise KernelUnavailable("the HIP kernels run on GPU tensors only")
@@ -1917,7 +1936,17 @@ def tied_attention_mfma(q, gate, k_pool, block_table, q_start, ctx_len, out, sca
     G = n_heads // n_kv_heads
     lib = build.load("sink_attention")
     keys = max_pages * page_size if window <= 0 else min(max_pages * page_size, window)
-    if max_q_len == 1 and T == n_seqs and head_dim <= 128 and G <= 32 and not shared_tiles:
+    decodes = _tied_decodes(q, ctx_len, n_heads, n_kv_heads, head_dim, max_q_len) and not shared_tiles
+    k_new = slots = None
+    if new is not None:
+        k_new, slots = new
+        _columns(k_new, "tied_attention_mfma: new rows")
+        _i32(slots, "slot_mapping")
+        if not decodes or not k_new.is_cuda or not slots.is_cuda or slots.shape != (T,) \
+                or k_new.shape != (T, n_kv_heads * head_dim) or k_new.dtype != q.dtype:
+            raise KernelUnavailable("tied_attention_mfma: new rows [T, nKV * hd] of the pool's dtype "
+                                    "and a slot each, in a decode step")
+    if decodes:
         # a decode step: every wave of a workgroup is a split of its own
         # (``tied_attention_decode_kernel``); about 1024 workgroups, at least 64 keys a wave
         span = keys + 31                      # the first chunk starts at a multiple of 32
@@ -1933,7 +1962,8 @@ def tied_attention_mfma(q, gate, k_pool, block_table, q_start, ctx_len, out, sca
             _ptr(q), ctypes.c_longlong(qs), _ptr(gate), ctypes.c_longlong(gs), _ptr(k_pool),
             _ptr(block_table), _ptr(ctx_len), _ptr(out), _ptr(ws_o), _ptr(ws_ml),
             ctypes.c_float(scale), int(window), 1 if sink else 0, n_seqs, n_heads, n_kv_heads,
-            head_dim, page_size, max_pages, blocks, wave_keys, _stream()),
+            head_dim, page_size, max_pages, blocks, wave_keys, _ptr(k_new),
+            ctypes.c_longlong(0 if k_new is None else k_new.stride(0)), _ptr(slots), _stream()),
             "tied_attention_mfma (decode)")
         return
     QT = max(1, TIED_MFMA_ROWS // G)

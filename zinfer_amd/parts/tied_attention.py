@@ -83,15 +83,13 @@ class TiedKeyValueAttention(Mixer):
         q = qkg[:, :self.q_width]
         k = qkg[:, self.q_width:self.q_width + self.kv_width]
         gate = qkg[:, self.q_width + self.kv_width:] if s.output_gate else None
-        if cache.writes:
-            ops.kv_rows_write(k, kv.slot_mapping, cache.k_pool, s.n_kv_heads, s.head_dim,
-                              cache.page_size)
         attn = step.scratch("attn", (T, self.q_width), act)
         ops.tied_attention(q, gate, cache.k_pool, kv.block_table, step.q_start, step.ctx_len,
                            step.seq_index, attn, float(self.scale),
                            0 if s.window is None else int(s.window), bool(s.sink),
                            s.n_heads, s.n_kv_heads, s.head_dim, cache.page_size,
-                           step.max_q_len, step.max_ctx_len)
+                           step.max_q_len, step.max_ctx_len,
+                           new=(k, kv.slot_mapping) if cache.writes else None)
         self.o.forward(attn, residual, accumulate=accumulate, step=step if accumulate else None)
 
 
