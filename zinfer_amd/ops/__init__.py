@@ -1171,6 +1171,7 @@ def sum_norm_plan(M: int, N: int, K: int, w: torch.Tensor, w_tiled: bool):
     return ("tile", ks) if ks >= 2 else None
 
 
+@functools.lru_cache(maxsize=None)
 def _tile256_ksplit(M: int, N: int, K: int):
     """Parts of K if a residual sum should run through the 256 x 256 tiles split along K, one workgroup
     to a CU: where the parts fill seven eighths of the chip and are long enough for their partials.
