@@ -124,11 +124,12 @@ typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2_t;
 // summed from zero in ascending steps of 32, and the spans are added in ascending order to zero.
 // Inside a step of 32 a lane's group g = lane / 16 holds k = 8 g .. 8 g + 7, and MFMA j takes
 // element j of every group, which lets 16-byte loads of rows feed the operands as they are.
-// Two kernels follow that order:
+// Three kernels follow that order:
 //   * up to 64 rows, bound by reading W (one user of the 0.6B shape's float32 weights: 1.9 GB a
 //     token): a workgroup of eight waves, one span each, takes 16 rows of W (32 with a wide
 //     output) for all tokens; a wave's loads of a step are 16 whole lines of 128 bytes, straight
-//     into the operands, four steps in flight; the eight partials meet in LDS.
+//     into the operands, four steps in flight; the eight partials meet in LDS.  For narrow outputs
+//     every span is a workgroup, and a second kernel adds the spans (gemm_f32_spans_kernel).
 //   * above, bound by the MFMAs: tiles of 128 x 128, 64 x 64 or 32 x 32 through LDS (rows of 36
 //     words: the 16-byte operand reads of 16 rows fall into different banks), the next step's
 //     loads in flight during the products.  The largest tile that still gives 256 workgroups.
@@ -173,7 +174,7 @@ __device__ __forceinline__ void f32_store4(TO* __restrict__ C, int m, int n, int
 // GLU (RG 2, one group of tokens): W is a gate's N rows and then an up projection's N rows; the two
 // row groups are the same rows of both, and silu(gate) * up of the 32-bit sums is stored: the bits of
 // the product and zf_swiglu behind it, without the launch and the way through memory (4 tokens,
-// 3072 x 1024: 8.2 + 4.6 us of the trace).
+// 6144 rows of 1024: 8.1 + 4.7 -> 9.1 us in the trace).
 template <typename TO, bool ACC, int RG, int MT, bool VEC, bool GLU = false>
 __global__ __launch_bounds__(F32_SPANS * 64) void gemm_f32_stream_kernel(
     const float* __restrict__ A, const float* __restrict__ W, TO* __restrict__ C, int M, int N,
@@ -249,6 +250,9 @@ __global__ __launch_bounds__(F32_SPANS * 64) void gemm_f32_stream_kernel(
 // what comes behind (the residual, the norm).  For outputs whose row groups leave most of the
 // chip idle: a group's eight waves together on one CU wait for its matrix core (32 cycles an MFMA,
 // whatever the number of tokens) and for one another's loads.  DEPTH batches of BATCH steps in flight.
+// In the trace, 4 tokens into 1024 outputs over K = 2048 and 3072, the mean of both: 14.2 -> 5.3 us, the
+// kernel that adds them in the place of the norm's (4.6 -> 4.5); deeper batches in the eight waves' own
+// kernel alone had reached 8.6 and 13.6 us in a chain (12.2 and 17.0 before, 8.4 and 9.9 so).
 template <int MT>
 __global__ __launch_bounds__(64) void gemm_f32_spans_kernel(const float* __restrict__ A,
                                                             const float* __restrict__ W,
