@@ -1240,6 +1240,38 @@ def test_gemm_many_gives_the_products_own_bits(M, K, widths):
         assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("M", [1, 9, 16])
+@pytest.mark.parametrize("K,widths", [(1024, [(6144, "bf16"), (12288, "f32"), (64, "silu")]),
+                                      (4096, [(64, "f32"), (2112, "bf16")]),
+                                      (8192, [(64, "f32"), (2048, "silu"), (2112, "gelu")])])
+def test_products_together_have_the_bits_of_the_products(M, K, widths):
+    """Widths whose own launch takes two row groups a workgroup, and products that ``gemm`` splits
+    along K, which are not joined; with an activation ``gemm_activation``'s kernel or the two."""
+    from zinfer_amd.parts.linear import Linear, products
+    ops = _ops()
+    a = _rand((M, K), torch.bfloat16, 98).to(DEV)
+    items, wants = [], []
+    for i, (N, kind) in enumerate(widths):
+        linear = Linear(_rand((N, K), torch.bfloat16, 99 + i, 0.1).to(DEV))
+        act = kind if kind in ops.ACTIVATIONS else None
+        out = torch.full((M, N), float("nan"), device=DEV,
+                         dtype=torch.float32 if kind == "f32" else torch.bfloat16)
+        want = torch.empty_like(out)
+        ops.gemm(a, linear.weight, want, w_tiled=True)
+        if act:
+            ops.activation(want, want, act)
+            alone = torch.empty_like(out)
+            ops.gemm_activation(a, linear.weight, alone, act, w_tiled=True)
+            assert torch.equal(alone, want), N
+        items.append((a, linear, out, act))
+        wants.append(want)
+    if K == 8192:
+        assert not ops.gemm_many_covers([(x, l.weight, l.tiled, o, f) for x, l, o, f in items])
+    products(items)
+    for (_, _, out, _), want in zip(items, wants):
+        assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("M", [1, 8, 9, 16])
 @pytest.mark.parametrize("N,K", [(64, 4096), (2048, 4160), (1984, 7168)])
 @pytest.mark.parametrize("kind", ["sum", "f32", "bf16"])

@@ -590,6 +590,12 @@ def _narrow_split(M: int, N: int, K: int):
     return (1, 2) if M <= 8 else (2, 4)
 
 
+def _stream_plan(M: int, N: int, K: int, tiled: bool):
+    """Row groups per workgroup and workgroups along K with which ``gemm`` streams a weight where no
+    plan by measurement serves; whoever promises the bits of ``gemm`` asks here."""
+    return (tiled and _narrow_split(M, N, K)) or _skinny_plan(M, N, K, tiled)
+
+
 MID_MAX_M = 128
 
 
@@ -989,8 +995,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
             _check(lib.zf_gemm_bf16_mid(_ptr(a), _ptr(w), _ptr(out), _ptr(ws), M, N, K, epi, mid,
                                         _stream()), "gemm (17 to 128 tokens)")
         elif M <= SKINNY_MAX_M:
-            rg, ks = plan[1:] if plan is not None else \
-                (w_tiled and _narrow_split(M, N, K)) or _skinny_plan(M, N, K, w_tiled)
+            rg, ks = plan[1:] if plan is not None else _stream_plan(M, N, K, w_tiled)
             ws = _workspace("gemm_splitk", ks * M * N, torch.float32, a.device) if ks > 1 else None
             _check(lib.zf_gemm_bf16_skinny(_ptr(a), _ptr(w), _ptr(out), _ptr(ws), M, N, K, epi,
                                            rg, ks, 1 if w_tiled else 0, _stream()),
@@ -1323,7 +1328,7 @@ def gemm_many_covers(items) -> bool:
                 and out.dtype in ((torch.bfloat16,) if act else (torch.bfloat16, torch.float32))
                 and all(t.is_contiguous() for t in (a, w, out))
                 and all(t.data_ptr() % 16 == 0 for t in (a, w))
-                and _skinny_plan(M, N, K, tiled)[1] == 1):
+                and _stream_plan(M, N, K, tiled)[1] == 1):
             return False
     return True
 
@@ -2438,12 +2443,12 @@ def activation(x: torch.Tensor, out: torch.Tensor, kind: str) -> None:
 def gemm_activation(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str,
                     w_tiled: bool = False) -> None:
     """``gemm`` and then ``activation`` over ``out`` in place, the same bits; up to 16 tokens on a
-    pre-tiled matrix in one kernel."""
+    pre-tiled matrix in one kernel, where ``gemm`` does not split K."""
     M, K = a.shape
     N = w.shape[0]
     if w_tiled and 0 < M <= 16 and out.dtype == a.dtype == torch.bfloat16 and kind in ACTIVATIONS \
             and w.shape[1] == K and out.shape == (M, N) and can_pretile(w):
-        rg, ks = _skinny_plan(M, N, K, True)
+        rg, ks = _stream_plan(M, N, K, True)
         if ks == 1:
             _gemm_act(a, w, out, kind, rg)
             return
