@@ -415,6 +415,41 @@ def test_delta_rule_of_long_portions_in_chunks(H, KH, d, dv, decay):
             assert chunked < max(1.5 * walked, 1e-6), (lens[i], errors)
 
 
+@pytest.mark.parametrize("token", [0, 3, 16, 47, 131, 144])
+@pytest.mark.parametrize("what", ["q", "k", "v", "decay", "step"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_delta_rule_in_chunks_keeps_what_is_not_finite_from_the_tokens_before(what, token, value):
+    """A portion of 145 tokens (chunks of sixteen, the last of one) with one number that is not finite,
+    at the first and the last token of the portion and of a chunk and inside: rows and columns
+    that the walk leaves finite have the bits of the portion without it, and the rest is as in the
+    walk, also in the state left behind."""
+    H, KH, d, dv, n = 2, 1, 64, 32, 145
+    qkv, ab, a_log, dt_bias = _delta_inputs(n, H, KH, d, dv, 77)
+    bad_qkv, bad_ab = qkv.clone(), ab.clone()
+    if what in ("q", "k"):
+        bad_qkv[token, 5 + (d if what == "k" else 0)] = value
+    elif what == "v":
+        bad_qkv[token, 2 * KH * d + dv + 3] = value       # a column of the second head
+    else:
+        bad_ab[token, 1 + (H if what == "step" else 0)] = value
+    size = (ops.delta_state_size(H, d, dv) + 3) // 4 * 4
+    start = torch.randn((1, size), generator=torch.Generator().manual_seed(8)) * 0.3
+
+    def run(x, z, q_lens):
+        state, out = start.to(DEV), torch.zeros((n, H * dv), device=DEV)
+        ops.delta_recurrence(x.to(DEV), 0, KH * d, 2 * KH * d, z.to(DEV), a_log.to(DEV),
+                             dt_bias.to(DEV), state, _i32([0]), _i32([0, n]), out, H, KH, d, dv,
+                             q_lens=q_lens)
+        return out.cpu(), ops.delta_state_matrix(state, H, d, dv).cpu()
+
+    clean, walked, got = run(qkv, ab, [n]), run(bad_qkv, bad_ab, None), run(bad_qkv, bad_ab, [n])
+    for mine, theirs in zip(got, walked):
+        assert torch.equal(torch.isfinite(mine), torch.isfinite(theirs))
+    before = torch.isfinite(walked[0])
+    before[token:] &= what in ("q", "v")          # (a step or decay of 1 or 0 changes what follows)
+    assert torch.equal(got[0][before], clean[0][before]) and before[:token].all()
+
+
 def test_a_token_far_back_is_kept_without_decay_and_lost_with_it():
     """Two heads, 600 tokens.  Token 3 alone writes the key e_0 with a value that stands out;
     the last token asks for e_0.  The head whose decay is 1 to rounding (a rate of exp(-30))

@@ -654,7 +654,9 @@ extern "C" int zf_delta_recurrence(const float* qkv, int C, int q_off, int k_off
 //   S = exp(G_15) S0 + K^T (exp(G_15 - G) W)
 // (the delta rule's chunked form by its triangular system, as published for linear attention).
 // Everything is 32-bit: v_mfma_f32_16x16x4_f32, expf, fused multiply-adds; no ratio of decays exceeds 1.
-// (A token that is not finite makes the whole chunk so.)
+// A token that is not finite reaches itself and the tokens behind it, as in the walk: the triangular
+// matrices hold zeros above their diagonals, and what such zeros would meet in a product is taken
+// out of the other operand first (dl_finite_rows).
 //   * delta_chunk_prepare  a wave a (chunk, head): Tb, M and the decays, all chunks side by side.
 //   * delta_chunk_walk     a workgroup of four waves a (16 value columns, head, sequence) walks the
 //                          chunks with S in the accumulators of the waves, d / 64 blocks of 16 key
@@ -730,7 +732,7 @@ __global__ __launch_bounds__(64) void delta_chunk_prepare_kernel(
   for (int r = 0; r < 4; ++r) {
     const int t = 4 * g + r;
     L[t][m] = t > m && m < n ? beta[t] * ratio[r] * kk[r] : 0.f;
-    dst[DL_CHUNK * DL_CHUNK + t * DL_CHUNK + m] = m < n ? ratio[r] * qk[r] : 0.f;
+    dst[DL_CHUNK * DL_CHUNK + t * DL_CHUNK + m] = t >= m && m < n ? ratio[r] * qk[r] : 0.f;
   }
   if (lane < 16) {
     dst[2 * DL_CHUNK * DL_CHUNK + lane] = expf(start);
@@ -749,8 +751,37 @@ __global__ __launch_bounds__(64) void delta_chunk_prepare_kernel(
     }
     const float b = beta[lane];
 #pragma unroll
-    for (int t = 0; t < DL_CHUNK; ++t) dst[t * DL_CHUNK + lane] = x[t] * b;
+    for (int t = 0; t < DL_CHUNK; ++t) dst[t * DL_CHUNK + lane] = t >= lane ? x[t] * b : 0.f;
   }
+}
+
+// Of a column's tokens (rows 4 g + r, the lanes of the column 16 apart): those that are not finite
+// become 0, the first of them is returned (DL_CHUNK: none).
+__device__ __forceinline__ int dl_finite_rows(dl_f32x4_t& x, int g) {
+  int bad = DL_CHUNK;
+#pragma unroll
+  for (int r = 3; r >= 0; --r)
+    if (!(fabsf(x[r]) < INFINITY)) {
+      bad = 4 * g + r;
+      x[r] = 0.f;
+    }
+  bad = min(bad, __shfl_xor(bad, 16));
+  return min(bad, __shfl_xor(bad, 32));
+}
+
+// acc += the 16 x 16 lower triangular matrix whose row m holds `tri` at columns 4 g + i, times x; the
+// rows from a column's first number on that is not finite are not finite.
+__device__ __forceinline__ dl_f32x4_t dl_triangle(const dl_f32x4_t& tri, dl_f32x4_t x,
+                                                  dl_f32x4_t acc, int g) {
+  int bad = DL_CHUNK;
+  // (a sum that overflows only costs the look at each number)
+  if (__any(!(fabsf((x[0] + x[1]) + (x[2] + x[3])) < INFINITY))) bad = dl_finite_rows(x, g);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(tri[i], x[i], acc, 0, 0, 0);
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (4 * g + r >= bad) acc[r] = NAN;
+  return acc;
 }
 
 template <int ND>
@@ -829,11 +860,10 @@ __global__ __launch_bounds__(256) void delta_chunk_walk_kernel(
     // rows 4 g + r are tokens, column m a value column; every wave forms W for its own channels
     const dl_f32x4_t sk = (red[0][0][lane] + red[1][0][lane]) + (red[2][0][lane] + red[3][0][lane]);
     const dl_f32x4_t tb = *(const dl_f32x4_t*)&mats[0][m][4 * g];
-    dl_f32x4_t x, W = {0.f, 0.f, 0.f, 0.f};
+    dl_f32x4_t x;
 #pragma unroll
     for (int r = 0; r < 4; ++r) x[r] = fmaf(-decays[0][4 * g + r], sk[r], vs[4 * g + r][m]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) W = __builtin_amdgcn_mfma_f32_16x16x4f32(tb[i], x[i], W, 0, 0, 0);
+    const dl_f32x4_t W = dl_triangle(tb, x, dl_f32x4_t{0.f, 0.f, 0.f, 0.f}, g);
     const float whole = decays[0][DL_CHUNK - 1];
     float cw[4];
 #pragma unroll
@@ -854,8 +884,7 @@ __global__ __launch_bounds__(256) void delta_chunk_walk_kernel(
       dl_f32x4_t o;
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = decays[0][4 * g + r] * sq[r];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o = __builtin_amdgcn_mfma_f32_16x16x4f32(mv[i], W[i], o, 0, 0, 0);
+      o = dl_triangle(mv, W, o, g);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         if (4 * g + r < n)

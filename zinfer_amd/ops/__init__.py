@@ -3448,7 +3448,8 @@ def delta_recurrence(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, ab: 
     its last.  A row's result depends on the state and the rows of its own sequence alone; with
     ``q_lens`` (the sequences' rows, on the host) a sequence that brings more than
     ``DELTA_WALK_MAX`` runs in chunks of products where the sizes allow (``delta_chunks_cover``),
-    in 32-bit too, and its results then agree with the walk's up to rounding."""
+    in 32-bit too, and its results then agree with the walk's up to rounding.  Either way a number
+    that is not finite reaches its own row and the ones behind it, none before."""
     _need_gpu(qkv, ab, decay_log, decay_bias, state, state_slots, q_start, out)
     _i32(state_slots, "state_slots")
     _i32(q_start, "q_start")
