@@ -784,6 +784,22 @@ def test_split_wave_attention_does_not_depend_on_the_batch(nH, nKV, hd, page_siz
         assert torch.equal(alone, got[at])
 
 
+@pytest.mark.parametrize("hd,page_size", [(64, 16), (128, 48)])
+@pytest.mark.parametrize("low,high", [(0, 64), (64, 128), (70, 290), (128, 512)])
+def test_split_wave_attention_of_scores_that_are_minus_infinity(hd, page_size, low, high):
+    """Whole chunks, and whole turns of a wave, whose keys weigh nothing, at the front, inside and at
+    the end of the keys."""
+    ctx_lens, q_lens = [512, 300], [1, 3]
+    s = _paged_setup(torch.float32, 4, 2, hd, page_size, ctx_lens, q_lens, 12)
+    s["q"].view(-1, 4, hd)[:, :, 0] = 1.0
+    K = s["k_pool"].view(-1, 2, page_size, hd)
+    for i, n in enumerate(ctx_lens):
+        for key in range(low, min(high, n)):
+            K[int(s["block_table"][i, key // page_size]), :, key % page_size, 0] = float("-inf")
+    got, want = _run_attention(s, torch.float32, 4, 2, hd, page_size, 0, q_lens, ctx_lens)
+    assert torch.isfinite(want).all() and rel_err(got, want) <= tol(torch.float32)
+
+
 @pytest.mark.parametrize("nH,nKV,hd,page_size,window", [
     (8, 2, 32, 16, 0), (32, 8, 128, 16, 0), (6, 6, 64, 32, 0), (16, 1, 64, 16, 0),
     (9, 3, 256, 16, 0), (8, 2, 64, 16, 37), (4, 4, 128, 48, 300), (36, 4, 32, 16, 0),

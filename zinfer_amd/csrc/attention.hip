@@ -230,8 +230,10 @@ __global__ __launch_bounds__(SPLIT_WAVES * ZF_WAVE) void paged_attention_split_k
     const float own = g == 0 ? sc[0] : g == 1 ? sc[1] : g == 2 ? sc[2] : sc[3];
     const float score = seen ? own * scale : -INFINITY;
     const float m_new = fmaxf(m, wave_max(score));
-    const float corr = expf(m - m_new);                  // exp(-inf) = 0 on the first chunk
-    const float w = seen ? expf(score - m_new) : 0.f;
+    // (scores of -inf alone, so far: they weigh nothing beside another wave's)
+    const float ref = m_new == -INFINITY ? 0.f : m_new;
+    const float corr = expf(m - ref);                    // exp(-inf) = 0 on the first chunk
+    const float w = seen ? expf(score - ref) : 0.f;
     l = l * corr + wave_sum(w);
     m = m_new;
     ps[wave][16 * g + kq] = w;
