@@ -105,6 +105,38 @@ MODES = {"whole": traces.whole, "prefill_then_32": traces.prefill_then_single,
          "token_by_token": traces.token_by_token}
 
 
+@pytest.mark.parametrize("what", ["embedding", "entry gain", "final gain", "all"])
+def test_tensors_at_odd_addresses_are_read_as_they_lie(what, tmp_path_factory):
+    """An embedding and gains that are views into a flat buffer, off any 16-byte boundary: steps of
+    few tokens give the logits of aligned ones (up to the rounding that sums of squares in
+    another order bring: 2^-8 of a bfloat16 activation)."""
+    from zinfer_amd.engine import StepEntry
+    from zinfer_amd.engine.replay import make_engine
+    path = tiny.model_dir_of("E", str(tmp_path_factory.getbasetemp()), torch.bfloat16)
+    tokens = tiny.random_tokens(7, tiny.CONFIGS["E"]["vocab_size"], 5)
+
+    def odd(t):
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+        flat[1:] = t.reshape(-1)
+        return flat[1:].view(t.shape)
+
+    def run(names):
+        eng = make_engine(path, "bfloat16", 256, DEV, page_size=16)
+        model = eng.model
+        if "embedding" in names:
+            model.embedding = odd(model.embedding)
+        if "entry gain" in names:
+            norm = model.blocks[0].entry_norm
+            norm.gain = odd(norm.gain)
+        if "final gain" in names:
+            model.final_norm.gain = odd(model.final_norm.gain)
+        return eng.step([StepEntry("a", tokens, [2, 6])]).cpu()
+
+    want = run(())
+    got = run((what,) if what != "all" else ("embedding", "entry gain", "final gain"))
+    assert torch.isfinite(got).all() and rel_err(got, want) <= LOGITS_TOL_BF16
+
+
 @pytest.mark.parametrize("mode", list(MODES))
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", ["A", "B", "C", "D", "E"])

@@ -146,10 +146,10 @@ class DecoderModel:
         return total
 
     @staticmethod
-    def _pick(norm, rows: torch.Tensor, step, pick):
-        """Runs ``pick``, which picks ``rows`` from a table, and has it leave what ``norm``, which
+    def _pick(norm, table: torch.Tensor, rows: torch.Tensor, step, pick):
+        """Runs ``pick``, which picks ``rows`` from ``table``, and has it leave what ``norm``, which
         reads them next, can use; returns that, or None."""
-        left = norm.picked(rows, step) if isinstance(norm, Norm) else None
+        left = norm.picked(table, rows, step) if isinstance(norm, Norm) else None
         pick(**({} if left is None else {"given": left.buffers}))
         return left
 
@@ -188,7 +188,7 @@ class DecoderModel:
             first = None if self.reentry is not None or copies is not None else \
                 getattr(self.blocks[s.schedule[0].layer], "entry_norm", None)
             step.norm_ready = self._pick(
-                first, x, step, lambda **given: ops.embed(
+                first, self.embedding, x, step, lambda **given: ops.embed(
                     self.embedding, step.token_ids, x, float(s.embedding_multiplier), **given))
         x0 = None
         if self.reentry is not None:
@@ -229,7 +229,7 @@ class DecoderModel:
             rows = x
         else:
             rows = step.scratch("want_rows", (n_rows, s.hidden_size), torch.float32)
-            left = self._pick(self.final_norm, rows, step,
+            left = self._pick(self.final_norm, x, rows, step,
                               lambda **given: ops.gather_rows(x, step.want_rows, rows, **given))
         make = lambda: step.scratch("final_normed", (n_rows, s.hidden_size), self.ctx.act_dtype)
         with ops.kernel_class("head_sampling"):      # what a per-class measurement counts these as

@@ -130,14 +130,21 @@ def _launches(cls: str):
 
 
 # ------------------------------------------------------------------------- elementwise
-def _check_given(given, rows: torch.Tensor) -> None:
-    """``given`` = (gain, xg, sq) of the float32 ``rows``, or None."""
+def rows_leave_norm(table: torch.Tensor, gain: torch.Tensor, rows: torch.Tensor) -> bool:
+    """Whether ``embed`` and ``gather_rows`` take ``given`` for these ``rows`` of ``table``: up to 16 of
+    them, read and written in pieces of four values, whose sums of squares go by 16 columns."""
+    return rows.shape[0] <= NORM_FOLD_MAX_M and rows.shape[1] % 16 == 0 \
+        and all(t.data_ptr() % 16 == 0 for t in (table, gain, rows))
+
+
+def _check_given(given, table: torch.Tensor, rows: torch.Tensor) -> None:
+    """``given`` = (gain, xg, sq) of the float32 ``rows`` picked from ``table``, or None."""
     if given is None:
         return
     T, H = rows.shape
     gain, xg, sq = given
-    if not (T <= NORM_FOLD_MAX_M and H % 16 == 0 and gain.dtype == torch.float32 and gain.shape == (H,)
-            and xg.dtype == torch.bfloat16 and xg.shape == (T, H) and sq.dtype == torch.float32
+    if not (rows_leave_norm(table, gain, rows) and xg.data_ptr() % 16 == 0
+            and gain.dtype == torch.float32 and gain.shape == (H,) and xg.dtype == torch.bfloat16 and xg.shape == (T, H) and sq.dtype == torch.float32
             and sq.shape == (H // 16, 16)
             and all(t.is_contiguous() for t in (rows, gain, xg, sq))):
         raise KernelUnavailable(f"a norm's inputs beside the rows: gain {tuple(gain.shape)}, "
@@ -152,7 +159,7 @@ def embed(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, scale: floa
     _need_gpu(table, ids, out, *(given or ()))
     _i32(ids, "ids")
     T, H = out.shape
-    _check_given(given, out)
+    _check_given(given, table, out)
     if table.shape[1] != H or ids.shape[0] != T or out.dtype != torch.float32:
         raise KernelUnavailable(f"embed: table {tuple(table.shape)}, ids {tuple(ids.shape)}, "
                                 f"out {tuple(out.shape)} {out.dtype}")
@@ -324,7 +331,7 @@ def gather_rows(x: torch.Tensor, idx: torch.Tensor, out: torch.Tensor,
     _need_gpu(x, idx, out, *(given or ()))
     _i32(idx, "idx")
     n, H = out.shape
-    _check_given(given, out)
+    _check_given(given, x, out)
     if x.shape[1] != H or idx.shape[0] != n or x.dtype != torch.float32 or out.dtype != x.dtype:
         raise KernelUnavailable("gather_rows: float32 [T, H] -> [n, H]")
     lib = build.load("elementwise")

@@ -183,9 +183,9 @@ class Norm(Part):
       (runs the norm once, returns the activations) and ``fold_into(linear, out, **kw)`` (the
       product of the normed rows with ``linear``'s weight in one kernel, or False).  None:
       the norm simply runs.  ``left``: what ``residual_sum`` left for this norm, or None.
-    * ``picked(x, step)``: for rows ``x`` about to be picked from a table (an embedding, the rows
-      whose logits are wanted): an object whose ``buffers`` the kernel that picks them also
-      writes, and which then is what ``residual_sum`` leaves.  None: nothing beside the rows.
+    * ``picked(table, x, step)``: for rows ``x`` about to be picked from ``table`` (an embedding,
+      the rows whose logits are wanted): an object whose ``buffers`` the kernel that picks them
+      also writes, and which then is what ``residual_sum`` leaves.  None: nothing beside the rows.
     * ``residual_sum(linear, a, out, step)``: out += a W^T in a kernel that also leaves
       something for this norm, which reads ``out`` next; puts it in ``step.norm_ready`` and
       returns True, or returns False and does nothing."""
@@ -200,7 +200,7 @@ class Norm(Part):
     def deferred(self, x: torch.Tensor, make_out, left=None):
         return None
 
-    def picked(self, x: torch.Tensor, step):
+    def picked(self, table: torch.Tensor, x: torch.Tensor, step):
         return None
 
     def residual_sum(self, linear, a: torch.Tensor, out: torch.Tensor, step) -> bool:

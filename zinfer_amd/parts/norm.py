@@ -39,9 +39,9 @@ class RmsNorm(Norm):
             return None
         return LazyRmsNorm(self, x, make_out, given)
 
-    def picked(self, x: torch.Tensor, step):
+    def picked(self, table: torch.Tensor, x: torch.Tensor, step):
         if not (x.is_cuda and self.ctx.compute_dtype == torch.bfloat16
-                and x.shape[0] <= ops.NORM_FOLD_MAX_M and x.shape[1] % 64 == 0):
+                and x.shape[1] % 64 == 0 and ops.rows_leave_norm(table, self.gain, x)):
             return None
         return GivenRmsNorm(self, x, *self._given_buffers(x, step))
 
