@@ -105,6 +105,13 @@ MODES = {"whole": traces.whole, "prefill_then_32": traces.prefill_then_single,
          "token_by_token": traces.token_by_token}
 
 
+def _off_boundary(t):
+    """The tensor as a view into a flat buffer, one element behind a 16-byte boundary."""
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    flat[1:] = t.reshape(-1)
+    return flat[1:].view(t.shape)
+
+
 @pytest.mark.parametrize("what", ["embedding", "entry gain", "final gain", "all"])
 def test_tensors_at_odd_addresses_are_read_as_they_lie(what, tmp_path_factory):
     """An embedding and gains that are views into a flat buffer, off any 16-byte boundary: steps of
@@ -115,26 +122,40 @@ def test_tensors_at_odd_addresses_are_read_as_they_lie(what, tmp_path_factory):
     path = tiny.model_dir_of("E", str(tmp_path_factory.getbasetemp()), torch.bfloat16)
     tokens = tiny.random_tokens(7, tiny.CONFIGS["E"]["vocab_size"], 5)
 
-    def odd(t):
-        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
-        flat[1:] = t.reshape(-1)
-        return flat[1:].view(t.shape)
-
     def run(names):
         eng = make_engine(path, "bfloat16", 256, DEV, page_size=16)
         model = eng.model
         if "embedding" in names:
-            model.embedding = odd(model.embedding)
+            model.embedding = _off_boundary(model.embedding)
         if "entry gain" in names:
             norm = model.blocks[0].entry_norm
-            norm.gain = odd(norm.gain)
+            norm.gain = _off_boundary(norm.gain)
         if "final gain" in names:
-            model.final_norm.gain = odd(model.final_norm.gain)
+            model.final_norm.gain = _off_boundary(model.final_norm.gain)
         return eng.step([StepEntry("a", tokens, [2, 6])]).cpu()
 
     want = run(())
     got = run((what,) if what != "all" else ("embedding", "entry gain", "final gain"))
     assert torch.isfinite(got).all() and rel_err(got, want) <= LOGITS_TOL_BF16
+
+
+def test_gains_at_odd_addresses_in_32_bit(tmp_path_factory):
+    """Norms behind residual sums over a long K, whose gains are off any 16-byte boundary: the same
+    bits as aligned ones."""
+    from zinfer_amd.engine import StepEntry
+    from zinfer_amd.engine.replay import make_engine
+    path = tiny.model_dir_of("E", str(tmp_path_factory.getbasetemp()), torch.float32)
+    tokens = tiny.random_tokens(7, tiny.CONFIGS["E"]["vocab_size"], 5)
+    results = []
+    for off in (False, True):
+        eng = make_engine(path, "float32", 256, DEV, page_size=16)
+        norms = [n for b in eng.model.blocks for n in (b.mixer_norm, b.ff_norm)]
+        for norm in norms + [eng.model.final_norm] if off else ():
+            norm.gain = _off_boundary(norm.gain)
+        results.append([eng.step([StepEntry("a", tokens, list(range(7)))]).cpu(),
+                        eng.step([StepEntry("a", [3], [0])]).cpu()])
+    for want, got in zip(*results):
+        assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("mode", list(MODES))

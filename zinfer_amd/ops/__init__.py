@@ -144,8 +144,8 @@ def _check_given(given, table: torch.Tensor, rows: torch.Tensor) -> None:
     T, H = rows.shape
     gain, xg, sq = given
     if not (rows_leave_norm(table, gain, rows) and xg.data_ptr() % 16 == 0
-            and gain.dtype == torch.float32 and gain.shape == (H,) and xg.dtype == torch.bfloat16 and xg.shape == (T, H) and sq.dtype == torch.float32
-            and sq.shape == (H // 16, 16)
+            and gain.dtype == torch.float32 and gain.shape == (H,) and xg.dtype == torch.bfloat16
+            and xg.shape == (T, H) and sq.dtype == torch.float32 and sq.shape == (H // 16, 16)
             and all(t.is_contiguous() for t in (rows, gain, xg, sq))):
         raise KernelUnavailable(f"a norm's inputs beside the rows: gain {tuple(gain.shape)}, "
                                 f"xg {tuple(xg.shape)}, sq {tuple(sq.shape)} for {tuple(rows.shape)}")
@@ -1084,10 +1084,11 @@ def _f32_spans_cover(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> boo
         and out.dtype == torch.float32 and all(t.data_ptr() % 16 == 0 for t in (a, w, out))
 
 
-def f32_sum_norm_covers(a: torch.Tensor, w: torch.Tensor, residual: torch.Tensor) -> bool:
-    """Whether ``gemm_sum_norm`` takes a 32-bit residual sum."""
-    return a.is_cuda and all(t.dtype == torch.float32 for t in (a, w, residual)) \
-        and _f32_spans_cover(a, w, residual)
+def f32_sum_norm_covers(a: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
+                        gain: torch.Tensor) -> bool:
+    """Whether ``gemm_sum_norm`` takes a 32-bit residual sum and the norm of that ``gain``."""
+    return a.is_cuda and all(t.dtype == torch.float32 for t in (a, w, residual, gain)) \
+        and gain.data_ptr() % 16 == 0 and _f32_spans_cover(a, w, residual)
 
 
 def gemm_partials_plan(M: int, N: int, K: int, w: torch.Tensor, w_tiled: bool):
@@ -1234,7 +1235,7 @@ def gemm_sum_norm(a: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, gain
     M, K = a.shape
     N = w.shape[0]
     if a.dtype == torch.float32:
-        if not f32_sum_norm_covers(a, w, residual) or w.shape[1] != K or residual.shape != (M, N) \
+        if not f32_sum_norm_covers(a, w, residual, gain) or w.shape[1] != K or residual.shape != (M, N) \
                 or gain.shape != (N,) or normed.shape != (M, N) \
                 or not all(t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
                            for t in (a, w, residual, gain, normed)):

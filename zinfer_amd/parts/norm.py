@@ -51,7 +51,7 @@ class RmsNorm(Norm):
 
     def residual_sum(self, linear, a: torch.Tensor, out: torch.Tensor, step) -> bool:
         if a.dtype == torch.float32:
-            if not ops.f32_sum_norm_covers(a, linear.weight, out):
+            if not ops.f32_sum_norm_covers(a, linear.weight, out, self.gain):
                 return False
             normed = step.scratch("normed_by_sum", out.shape, torch.float32)
             ops.gemm_sum_norm(a, linear.weight, out, self.gain, float(self.spec.eps), normed)
