@@ -90,6 +90,32 @@ def test_rms_norm_part(dtype):
     assert rel_err(out, want) <= (2e-5 if dtype == torch.float32 else 2 ** -8)
 
 
+def test_rms_norm_behind_a_32_bit_sum_in_a_bfloat16_build():
+    """A part whose rows and output matrix are 32-bit beside bfloat16 activations: the sum leaves
+    the norm nothing, whose consumer reads bfloat16 rows."""
+    from zinfer_amd.config.specs import RmsNormSpec
+    from zinfer_amd.parts import BuildContext, build_part
+    from zinfer_amd.parts.linear import Linear
+    part = build_part("norm", RmsNormSpec(256, 1e-6), BuildContext(torch.bfloat16, torch.device(DEV)),
+                      "n.")
+    part.bind({"n.weight": torch.ones(256)})
+    linear = Linear(_rand((256, 2048), 1).to(DEV))
+    x, out = _rand((3, 2048), 2).to(DEV), torch.zeros((3, 256), device=DEV)
+
+    class Step:
+        norm_after, norm_ready = part, None
+
+        def scratch(self, name, shape, dtype):
+            return torch.empty(shape, dtype=dtype, device=DEV)
+
+    step = Step()
+    linear.forward(x, out, accumulate=True, step=step)
+    assert rel_err(out, x.double() @ linear.weight.double().T) <= 2e-5
+    lazy = part.deferred(out, lambda: torch.empty((3, 256), dtype=torch.bfloat16, device=DEV),
+                         step.norm_ready)
+    assert lazy.materialize().dtype == torch.bfloat16
+
+
 def test_rotary_tables_follow_the_plain_angles():
     from zinfer_amd.parts.position import rotary_tables
     for hd, theta in ((16, 1e4), (128, 1e6), (48, 5e4)):

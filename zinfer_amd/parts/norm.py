@@ -50,6 +50,8 @@ class RmsNorm(Norm):
                 step.scratch("normed_squares", (out.shape[1] // 16, 16), torch.float32))
 
     def residual_sum(self, linear, a: torch.Tensor, out: torch.Tensor, step) -> bool:
+        if a.dtype != self.ctx.act_dtype:
+            return False            # (the norm's rows are of the activations' type)
         if a.dtype == torch.float32:
             if not ops.f32_sum_norm_covers(a, linear.weight, out, self.gain):
                 return False
