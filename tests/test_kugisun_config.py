@@ -261,3 +261,38 @@ def test_the_plain_pieces_by_hand():
     X = P.stream_step([torch.tensor([[1.0]], dtype=P.F64), torch.tensor([[10.0]], dtype=P.F64)],
                       w, 1, lambda u: 100 * u)
     assert [x.item() for x in X] == [110.0, -99.0]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("lens", [[1, 1], [1, 128], [1, 129]])
+def test_the_delta_rule_of_a_captured_step_does_not_read_the_host_s_list(dtype, lens, monkeypatch):
+    """A decode step may be captured, so its launches follow device tensors and sizes alone; steps
+    whose portions are long enough for chunks, in bfloat16, are cut by the list."""
+    from zinfer_amd import ops
+    from zinfer_amd.parts import BuildContext, build_part
+    mixer = build_part("mixer", GatedDeltaRuleSpec(64, 2, 1, 64, 16, 4, 1e-6),
+                       BuildContext(dtype, torch.device("cpu")), "m.")
+    mixer.taps = mixer.decay_log = mixer.decay_bias = mixer.gain = None
+    told = []
+    for name in ("short_conv", "head_norm_gate"):
+        monkeypatch.setattr(ops, name, lambda *args, **kw: None)
+    monkeypatch.setattr(ops, "delta_recurrence", lambda *args, **kw: told.append(kw["q_lens"]))
+
+    class Step:
+        state_slots = seq_index = q_start = None
+        max_q_len = max(lens)
+
+        @property
+        def q_lens(self):
+            assert self.max_q_len > 1, "a captured step's list was read"
+            return lens
+
+        def scratch(self, name, shape, dtype):
+            return torch.empty(shape, dtype=dtype)
+
+    class Cache:
+        state = None
+
+    rows = [torch.empty((sum(lens), 2 * 64 + 2 * 32), dtype=dtype), torch.empty((sum(lens), 4))]
+    mixer.between(rows, Step(), Cache())
+    assert told == [lens if dtype == torch.bfloat16 and max(lens) > 128 else None]

@@ -130,7 +130,8 @@ class BuildContext:
 class Part:
     """``graph_safe`` says that ``forward`` only launches work on the current stream whose
     arguments depend on the step's device tensors and sizes, never on its host-side lists
-    (``q_lens``, ``slots``, ...): only then may a decode step be captured once and replayed."""
+    (``q_lens``, ``slots``, ...), in a step where every sequence brings one token (``max_q_len``
+    1): only then may a decode step be captured once and replayed."""
     role = ""
     graph_safe = False
     kernel_modules = ()        # names of the HIP kernel libraries the part launches

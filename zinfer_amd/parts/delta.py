@@ -114,12 +114,19 @@ class GatedDeltaRule(Mixer):
         ops.delta_recurrence(qkv, 0, QK, 2 * QK, ab, self.decay_log, self.decay_bias, cache.state,
                              step.state_slots, step.q_start, o, s.n_heads, s.n_kv_heads,
                              s.head_dim, s.value_dim,
-                             # (a 32-bit prompt's bits do not depend on where it is cut)
-                             q_lens=None if self.ctx.act_dtype == torch.float32 else step.q_lens)
+                             q_lens=self._portions(step))
         mixed = step.scratch("delta_mixed", (T, V), self.ctx.act_dtype)
         ops.head_norm_gate(o, self.gain, proj[:, 2 * QK + V:], mixed, s.n_heads,
                            float(s.norm_eps))
         return mixed
+
+    def _portions(self, step):
+        """The sequences' tokens where some bring enough of them for the recurrence's chunks; None
+        for the walk.  (A step that is captured brings a token a sequence and does not read the
+        host's list; a 32-bit prompt's bits do not depend on where it is cut.)"""
+        if self.ctx.act_dtype == torch.float32 or step.max_q_len <= ops.DELTA_WALK_MAX:
+            return None
+        return step.q_lens
 
     def forward(self, h, residual, step, cache, accumulate: bool = True) -> None:
         if hasattr(h, "materialize"):
