@@ -784,6 +784,20 @@ def test_split_wave_attention_does_not_depend_on_the_batch(nH, nKV, hd, page_siz
         assert torch.equal(alone, got[at])
 
 
+@pytest.mark.parametrize("hd,page_size", [(64, 16), (128, 16), (128, 64), (64, 48)])
+@pytest.mark.parametrize("ctx_lens,q_lens", [([1, 15, 16], [1, 15, 1]), ([17, 31, 32, 5], [17, 1, 3, 1]),
+                                             ([33, 63, 64], [1, 63, 64]), ([65, 127, 128, 20], [1, 127, 2, 20])])
+def test_split_wave_attention_in_fewer_waves(hd, page_size, ctx_lens, q_lens):
+    """Tables of so few pages that no token has keys for four waves: the bits of the same tokens
+    behind a wide table."""
+    s = _paged_setup(torch.float32, 6, 2, hd, page_size, ctx_lens, q_lens, 14)
+    got, want = _run_attention(s, torch.float32, 6, 2, hd, page_size, 0, q_lens, ctx_lens)
+    assert rel_err(got, want) <= tol(torch.float32)
+    wide = dict(s, block_table=torch.nn.functional.pad(s["block_table"], (0, 20), value=-1))
+    other, _ = _run_attention(wide, torch.float32, 6, 2, hd, page_size, 0, q_lens, ctx_lens)
+    assert torch.equal(got, other)
+
+
 @pytest.mark.parametrize("hd,page_size", [(64, 16), (128, 48)])
 @pytest.mark.parametrize("low,high", [(0, 64), (64, 128), (70, 290), (128, 512)])
 def test_split_wave_attention_of_scores_that_are_minus_infinity(hd, page_size, low, high):

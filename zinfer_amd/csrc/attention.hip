@@ -138,12 +138,13 @@ __global__ __launch_bounds__(ZF_WAVE) void paged_attention_wave_kernel(
 }
 
 // The same for float32, heads of 64 or 128 and pages of whole sixteens of rows: a workgroup a token and
-// head; chunks of 64 keys, at multiples of 64, go to its SPLIT_WAVES waves in turn, and their
+// head; chunks of 64 keys, at multiples of 64, go to its NW waves in turn, and their
 // running soft-maxes meet in LDS in wave order.  Four lanes share a key (a load of the wave takes 64
 // bytes of 16 rows), their parts of the dot product are added as ((0 + 1) + (2 + 3)), and four
 // lanes share an element of the output, four rows of a sixteen each (a load takes 1 KB of consecutive
 // memory), added up the same way once at the end.  Everything else is the order of the keys, and
-// nothing depends on the batch.
+// nothing depends on the batch: NW is 4, or fewer where no token of the launch can have so many chunks,
+// and a wave without one adds zeros.
 // What bounds the kernel above: a key a lane touches 64 lines with every load, which the one address
 // path of a CU takes a cycle each for, and the chunks of a token wait for one another.  Measured
 // against it (16 heads of 128 over 8, pages of 16, us): 4 single tokens behind 70 to 150 keys
@@ -154,16 +155,23 @@ __global__ __launch_bounds__(ZF_WAVE) void paged_attention_wave_kernel(
 #define SPLIT_WAVES 4
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 
-template <int NV>
-__global__ __launch_bounds__(SPLIT_WAVES * ZF_WAVE) void paged_attention_split_kernel(
+// a wave's own LDS accesses run in order; this keeps the compiler from moving them
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int NV, int NW>
+__global__ __launch_bounds__(NW * ZF_WAVE) void paged_attention_split_kernel(
     const float* __restrict__ q, const float* __restrict__ k_pool, const float* __restrict__ v_pool,
     const int* __restrict__ block_table, const int* __restrict__ q_start,
     const int* __restrict__ ctx_len, const int* __restrict__ seq_index, float* __restrict__ out,
     float scale, int window, int nH, int nKV, int page_size, int max_pages) {
   constexpr int HD = 16 * NV;
   __shared__ __attribute__((aligned(16))) float qs[HD];
-  __shared__ __attribute__((aligned(16))) float ps[SPLIT_WAVES][ZF_WAVE];
-  __shared__ float ml[SPLIT_WAVES][2], parts[SPLIT_WAVES][HD];
+  __shared__ __attribute__((aligned(16))) float ps[NW][ZF_WAVE];
+  __shared__ float ml[NW][2], parts[NW][HD];
   const int t = blockIdx.x, h = blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / ZF_WAVE), lane = threadIdx.x % ZF_WAVE;
   const int kq = lane / 4, g = lane % 4;
@@ -173,19 +181,22 @@ __global__ __launch_bounds__(SPLIT_WAVES * ZF_WAVE) void paged_attention_split_k
   const int lo = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
   const int kvh = h / (nH / nKV);
   const int* table = block_table + (size_t)s * max_pages;
+  const size_t row_at = ((size_t)t * nH + h) * HD;
 
-  if (threadIdx.x < HD) qs[threadIdx.x] = q[((size_t)t * nH + h) * HD + threadIdx.x];
+  for (int e = threadIdx.x; e < HD; e += NW * ZF_WAVE) qs[e] = q[row_at + e];
   __syncthreads();
 
   float acc[NV];                                         // element 16 i + kq, this lane's rows
 #pragma unroll
   for (int i = 0; i < NV; ++i) acc[i] = 0.f;
   float m = -INFINITY, l = 0.f;
-  for (int base = lo / ZF_WAVE * ZF_WAVE + wave * ZF_WAVE; base <= pos; base += SPLIT_WAVES * ZF_WAVE) {
-    const float* kp[4];
-    const float* vp[4];
+  // the chunk's first NC sixteens (the others hold no key of the token)
+  auto chunk = [&](int base, auto NC_) __attribute__((always_inline)) {
+    constexpr int NC = decltype(NC_)::value, EARLY = NC < 2 ? NC : 2;
+    const float* kp[NC];
+    const float* vp[NC];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < NC; ++c) {
       // (a sixteen without a key of this token reads one that has: its own pages may be gone)
       const int first = max(min(base + 16 * c, pos), lo) & ~15;
       const size_t block = (size_t)table[first / page_size] * nKV + kvh;
@@ -193,35 +204,35 @@ __global__ __launch_bounds__(SPLIT_WAVES * ZF_WAVE) void paged_attention_split_k
       kp[c] = k_pool + (block * page_size + row + kq) * HD + 4 * g;
       vp[c] = v_pool + block * page_size * HD + row + (size_t)kq * page_size + 4 * g;
     }
-    f32x4_t kv[4][NV], vv[4][NV];
+    f32x4_t kv[NC][NV], vv[NC][NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) kv[c][i] = *(const f32x4_t*)(kp[c] + 16 * i);
+      for (int c = 0; c < NC; ++c) kv[c][i] = *(const f32x4_t*)(kp[c] + 16 * i);
     auto load_values = [&](int c) {
 #pragma unroll
       for (int i = 0; i < NV; ++i)
         vv[c][i] = *(const f32x4_t*)(vp[c] + (size_t)16 * i * page_size);
     };
     // (half of the values with the keys, the rest into the keys' registers)
-    load_values(0);
-    load_values(1);
+#pragma unroll
+    for (int c = 0; c < EARLY; ++c) load_values(c);
     __builtin_amdgcn_sched_barrier(0);
     float sc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const f32x4_t qv = *(const f32x4_t*)&qs[16 * i + 4 * g];
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int e = 0; e < 4; ++e) sc[c] = fmaf(qv[e], kv[c][i][e], sc[c]);
     }
     __builtin_amdgcn_sched_barrier(0);
-    load_values(2);
-    load_values(3);
+#pragma unroll
+    for (int c = EARLY; c < NC; ++c) load_values(c);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < NC; ++c) {
       sc[c] += lane_xor<1>(sc[c]);
       sc[c] += lane_xor<2>(sc[c]);
     }
@@ -239,13 +250,10 @@ __global__ __launch_bounds__(SPLIT_WAVES * ZF_WAVE) void paged_attention_split_k
     ps[wave][16 * g + kq] = w;
 #pragma unroll
     for (int i = 0; i < NV; ++i) acc[i] *= corr;
-    // (a wave's own LDS accesses run in order; this keeps the compiler from moving them)
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (base < lo || base + ZF_WAVE - 1 > pos) {          // rows that are no key may hold anything
+    wave_fence();
+    if (base < lo || base + 16 * NC - 1 > pos) {          // rows that are no key may hold anything
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int k = base + 16 * c + 4 * g + e;
@@ -256,18 +264,26 @@ __global__ __launch_bounds__(SPLIT_WAVES * ZF_WAVE) void paged_attention_split_k
         }
     }
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < NC; ++c) {
       const f32x4_t wv = *(const f32x4_t*)&ps[wave][16 * c + 4 * g];
 #pragma unroll
       for (int i = 0; i < NV; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[i] = fmaf(wv[e], vv[c][i][e], acc[i]);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_fence();
+  };
+  if constexpr (NW == 1) {
+    // one chunk at most: of few keys its first sixteens alone
+    const int base = lo / ZF_WAVE * ZF_WAVE;
+    if (pos - base < 16) chunk(base, std::integral_constant<int, 1>{});
+    else if (pos - base < 32) chunk(base, std::integral_constant<int, 2>{});
+    else chunk(base, std::integral_constant<int, 4>{});
+  } else {
+    for (int base = lo / ZF_WAVE * ZF_WAVE + wave * ZF_WAVE; base <= pos; base += NW * ZF_WAVE)
+      chunk(base, std::integral_constant<int, 4>{});
   }
-  if (lane == 0) {
+  if (NW > 1 && lane == 0) {
     ml[wave][0] = m;
     ml[wave][1] = l;
   }
@@ -276,21 +292,27 @@ __global__ __launch_bounds__(SPLIT_WAVES * ZF_WAVE) void paged_attention_split_k
     float v = acc[i];
     v += lane_xor<1>(v);
     v += lane_xor<2>(v);
-    if (g == i % 4) parts[wave][16 * i + kq] = v;
+    if (g == i % 4) {
+      if constexpr (NW == 1)
+        out[row_at + 16 * i + kq] = v * (1.0f / l);
+      else
+        parts[wave][16 * i + kq] = v;
+    }
   }
+  if constexpr (NW == 1) return;
   __syncthreads();
   // (the first chunk has a key of the token; a wave without keys adds zeros)
   if (threadIdx.x < HD) {
     float top = ml[0][0], total = 0.f, v = 0.f;
 #pragma unroll
-    for (int w = 1; w < SPLIT_WAVES; ++w) top = fmaxf(top, ml[w][0]);
+    for (int w = 1; w < NW; ++w) top = fmaxf(top, ml[w][0]);
 #pragma unroll
-    for (int w = 0; w < SPLIT_WAVES; ++w) {
+    for (int w = 0; w < NW; ++w) {
       const float f = expf(ml[w][0] - top);
       total = fmaf(ml[w][1], f, total);
       v = fmaf(parts[w][threadIdx.x], f, v);
     }
-    out[((size_t)t * nH + h) * HD + threadIdx.x] = v * (1.0f / total);
+    out[row_at + threadIdx.x] = v * (1.0f / total);
   }
 }
 
@@ -304,14 +326,29 @@ extern "C" int zf_paged_attention_wave(const void* q, const void* k_pool, const 
   dim3 grid(T, nH);
   const size_t smem = (size_t)((hd + 3) / 4 * 4 + 2 * ZF_WAVE) * sizeof(float);
   const bool vec = hd % 4 == 0 && page_size % 4 == 0 && ((uintptr_t)k_pool | (uintptr_t)v_pool) % 16 == 0;
-  // (bfloat16 pools of such sizes are the MFMA kernels')
-  if (dtype == ZF_F32 && (hd == 64 || hd == 128) && page_size % 16 == 0 && vec) {
-#define SPLIT_ATTENTION(NV)                                                                         \
-  hipLaunchKernelGGL((paged_attention_split_kernel<NV>), grid, dim3(SPLIT_WAVES * ZF_WAVE), 0, stream, \
+  // (bfloat16 pools of such sizes are the MFMA kernels'; a window of up to 64 keys is one chunk of the
+  // kernel above wherever it begins, and up to two of the other: 16 single tokens behind windows of 16 / 64
+  // 5.2 and 6.3 us against 5.6 and 6.1, prompts of 512 tokens 30 and 57 against 67 and 70)
+  if (dtype == ZF_F32 && (hd == 64 || hd == 128) && page_size % 16 == 0 && vec &&
+      (window <= 0 || window > ZF_WAVE)) {
+    // Chunks that a token's keys can touch, by the width of the table.  Fewer waves where that is
+    // few: waves without a chunk would hold a CU's registers (16 heads of 128 over 8, us, four waves / so
+    // / the kernel above: four prompts of 64 tokens 32.3 / 14.9 / 27.1, of 100 51.7 / 32.9 / 43.8, 64 single
+    // tokens behind 32 keys 9.9 / 6.4 / 7.3).
+    const int chunks = ((long long)max_pages * page_size + ZF_WAVE - 1) / ZF_WAVE;
+#define SPLIT_ATTENTION(NV, NW)                                                                     \
+  hipLaunchKernelGGL((paged_attention_split_kernel<NV, NW>), grid, dim3(NW * ZF_WAVE), 0, stream,   \
                      (const float*)q, (const float*)k_pool, (const float*)v_pool, block_table,      \
                      q_start, ctx_len, seq_index, (float*)out, scale, window, nH, nKV, page_size,   \
                      max_pages)
-    if (hd == 64) SPLIT_ATTENTION(4); else SPLIT_ATTENTION(8);
+#define SPLIT_ATTENTION_OF(NV)                     \
+  do {                                             \
+    if (chunks <= 1) SPLIT_ATTENTION(NV, 1);       \
+    else if (chunks == 2) SPLIT_ATTENTION(NV, 2);  \
+    else SPLIT_ATTENTION(NV, SPLIT_WAVES);         \
+  } while (0)
+    if (hd == 64) SPLIT_ATTENTION_OF(4); else SPLIT_ATTENTION_OF(8);
+#undef SPLIT_ATTENTION_OF
 #undef SPLIT_ATTENTION
     ZF_CHECK_LAUNCH();
   }

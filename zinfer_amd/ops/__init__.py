@@ -1506,6 +1506,7 @@ def gemm_geglu(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
 # ------------------------------------------------------------------------- attention
 MAX_HEAD_DIM = 512          # the wave kernel keeps a head in registers: 8 values a lane
 DECODE_SPLIT_KEYS = 256     # keys per split of the decode kernel (DEC_SPLIT in attention.hip)
+ATTENTION_CHUNK_KEYS = 64   # keys a wave of the 32-bit kernels takes at a time
 PREFILL_QUERY_TILE = 32     # queries per tile of the kernels for prompt portions
 
 
