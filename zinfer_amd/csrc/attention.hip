@@ -1776,19 +1776,24 @@ extern "C" int zf_attn_prefill_bf16(const void* q, const void* k_pool, const voi
   const bool shared_ok = (hd == 64 || hd == 128) && split_keys % 64 == 0;
   if ((variant == 2 || variant == 3) && !shared_ok) return -2;
   if (variant == 2 || variant == 3 || (variant == 0 && shared_ok && G >= 2)) {
-    // two groups of waves on the even and the odd key tiles where the heads leave room for
+    // Two groups of waves on the even and the odd key tiles where the heads leave room for
     // them and the longest chain of tiles sets the time: short contexts before the portions
     // (allow_split) on a grid that fills the chip at most twice (8 K keys before a 2048-token
     // portion: 14 % slower with them; a whole 2048-token prompt: 73 -> 63 us with 4 heads per kv
-    // head, 66 -> 45 us with 2), or whatever the contexts on one of up to 400 workgroups, where the CUs wait
-    // for that chain (497 tokens behind 500 keys, 16 / 32 heads on 8: 32.1 -> 20.8, 30.3 -> 25.8 us;
-    // five portions of 300, up to 1500 keys, 400 workgroups: 45.9 -> 29.8, 44.2 -> 36.0).  Five to eight
-    // heads go to two workgroups then, up to 256 of them before: 497 tokens behind 0 / 500 / 1400 keys,
-    // 40 heads on 8, 23.2 -> 16.9, 38.9 -> 26.0, 64.9 -> 40.5 us, 1024 tokens 38.9 -> 34.0; of 312 and
-    // more the halves no longer run side by side (three prompts of 400 23.0 -> 32.1).
+    // head, 66 -> 45 us with 2), or whatever the contexts where every workgroup has a CU, where the CUs
+    // wait for that chain: 256 workgroups, or 512 of up to two heads of 64, which share a CU (497 tokens
+    // behind 500 keys, 16 / 32 heads on 8: 32.1 -> 20.8, 30.3 -> 25.8 us; 256 workgroups, 512 tokens
+    // behind 900, 44.1 -> 37.6; 264, five portions of 200 behind 900, 36.5 -> 47.6; two heads of 64,
+    // 512 workgroups, 33.8 -> 23.1, 600 28.3 -> 28.6).  Five to eight heads go to two workgroups then, up
+    // to 128 of them before (497 tokens behind 0 / 500 / 1400 keys, 40 heads on 8, 23.2 -> 16.9, 38.9 -> 26.0,
+    // 64.9 -> 40.5 us; eight portions of 20 to 64 behind none 10.9 -> 10.5): of more the halves share
+    // CUs (208, four prompts of 200 15.6 -> 20.8; 160, three portions of 200 behind 300 25.3 -> 28.0), which
+    // pays only where portions of 768 tokens and more are unequal enough (64 heads on 8: 256, 1024 tokens
+    // behind 900, 74.4 -> 71.0; 192, 768 behind 300, 45.3 -> 40.5; 208, 400 tokens 23.5 -> 25.5).
     const unsigned blocks = entries * nKV;
-    const bool groups = variant != 3 && split_keys == 0 && (allow_split || blocks <= 400);
-    const bool halves = groups && G > 4 && G <= 8 && blocks <= 256;
+    const bool groups = variant != 3 && split_keys == 0 &&
+                        (allow_split || blocks <= (hd == 64 && G <= 2 ? 512u : 256u));
+    const bool halves = groups && G > 4 && G <= 8 && blocks <= (max_q_len >= 768 ? 256u : 128u);
     const int heads = halves ? (G + 1) / 2 : G < 8 ? G : 8, head_blocks = (G + heads - 1) / heads;
     dim3 sgrid(entries * head_blocks * nKV, split_keys > 0 ? max_splits : 1);
     const int ks = groups && heads <= 4 && sgrid.x <= 1024 ? 2 : 1;
