@@ -655,8 +655,10 @@ extern "C" int zf_delta_recurrence(const float* qkv, int C, int q_off, int k_off
 // (the delta rule's chunked form by its triangular system, as published for linear attention).
 // Everything is 32-bit: v_mfma_f32_16x16x4_f32, expf, fused multiply-adds; no ratio of decays exceeds 1.
 // A token that is not finite reaches itself and the tokens behind it, as in the walk: the triangular
-// matrices hold zeros above their diagonals, and what such zeros would meet in a product is taken
-// out of the other operand first (dl_finite_rows).
+// matrices hold zeros above their diagonals, whatever the token brings, but such zeros against its
+// numbers in a product would reach every row.  What it brings stays in S, so a sequence that leaves an
+// S that is not finite is walked once more, with its numbers taken out of those products first (a look
+// at every chunk cost all sequences 4 to 8 %, the one at the end 0.5 us).
 //   * delta_chunk_prepare  a wave a (chunk, head): Tb, M and the decays, all chunks side by side.
 //   * delta_chunk_walk     a workgroup of four waves a (16 value columns, head, sequence) walks the
 //                          chunks with S in the accumulators of the waves, d / 64 blocks of 16 key
@@ -755,37 +757,37 @@ __global__ __launch_bounds__(64) void delta_chunk_prepare_kernel(
   }
 }
 
-// Of a column's tokens (rows 4 g + r, the lanes of the column 16 apart): those that are not finite
-// become 0, the first of them is returned (DL_CHUNK: none).
-__device__ __forceinline__ int dl_finite_rows(dl_f32x4_t& x, int g) {
-  int bad = DL_CHUNK;
-#pragma unroll
-  for (int r = 3; r >= 0; --r)
-    if (!(fabsf(x[r]) < INFINITY)) {
-      bad = 4 * g + r;
-      x[r] = 0.f;
-    }
-  bad = min(bad, __shfl_xor(bad, 16));
-  return min(bad, __shfl_xor(bad, 32));
-}
-
-// acc += the 16 x 16 lower triangular matrix whose row m holds `tri` at columns 4 g + i, times x; the
-// rows from a column's first number on that is not finite are not finite.
+// acc += the 16 x 16 lower triangular matrix whose row m holds `tri` at columns 4 g + i, times x.
+// CAREFUL: of a column's rows (4 g + r, the column's lanes 16 apart) those from its first number on that
+// is not finite are not finite, and the ones before have not met it.
+template <bool CAREFUL>
 __device__ __forceinline__ dl_f32x4_t dl_triangle(const dl_f32x4_t& tri, dl_f32x4_t x,
                                                   dl_f32x4_t acc, int g) {
   int bad = DL_CHUNK;
-  // (a sum that overflows only costs the look at each number)
-  if (__any(!(fabsf((x[0] + x[1]) + (x[2] + x[3])) < INFINITY))) bad = dl_finite_rows(x, g);
+  if constexpr (CAREFUL) {
+#pragma unroll
+    for (int r = 3; r >= 0; --r)
+      if (!(fabsf(x[r]) < INFINITY)) {
+        bad = 4 * g + r;
+        x[r] = 0.f;
+      }
+    bad = min(bad, __shfl_xor(bad, 16));
+    bad = min(bad, __shfl_xor(bad, 32));
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(tri[i], x[i], acc, 0, 0, 0);
+  if constexpr (CAREFUL) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-    if (4 * g + r >= bad) acc[r] = NAN;
+    for (int r = 0; r < 4; ++r)
+      if (4 * g + r >= bad) acc[r] = NAN;
+  }
   return acc;
 }
 
+// (as many registers as leave a CU the workgroups that one walk alone would: with three of four, four
+// portions of 1024 tokens of 32 heads took 250 us for 215)
 template <int ND>
-__global__ __launch_bounds__(256) void delta_chunk_walk_kernel(
+__global__ __launch_bounds__(256, ND == 8 ? 4 : 5) void delta_chunk_walk_kernel(
     const float* __restrict__ qkv, int C, int q_off, int k_off, int v_off, float* __restrict__ state,
     long long state_stride, const int* __restrict__ state_slots, const int* __restrict__ q_start,
     const float* __restrict__ ws, float* __restrict__ out, int H, int KH, int dv, int longest) {
@@ -805,8 +807,6 @@ __global__ __launch_bounds__(256) void delta_chunk_walk_kernel(
   float* S_mem = state + (size_t)state_slots[seq] * state_stride + ((size_t)h * dv + col0 + m) * d
                  + 16 * wave * B + 4 * g;
   dl_f32x4_t S[B];
-#pragma unroll
-  for (int b = 0; b < B; ++b) S[b] = *(const dl_f32x4_t*)(S_mem + 16 * b);
   dl_f32x4_t fk[PIECES], fq[PIECES];
   float fv, fm[2], fd;
   auto fetch = [&](int t0) {
@@ -825,72 +825,84 @@ __global__ __launch_bounds__(256) void delta_chunk_walk_kernel(
     fm[1] = src[256 + tid];
     fd = src[512 + tid % 32];
   };
-  fetch(0);
-  for (int t0 = 0; t0 < len; t0 += DL_CHUNK) {
-    const int n = min(DL_CHUNK, len - t0);
-    __syncthreads();                        // the chunk before is done with
+  auto walk = [&](auto CAREFUL_) __attribute__((always_inline)) {
+    constexpr bool CAREFUL = decltype(CAREFUL_)::value;
 #pragma unroll
-    for (int j = 0; j < PIECES; ++j) {
-      const int i = tid + 256 * j, tok = i / (d / 4), c = i % (d / 4) * 4;
-      *(dl_f32x4_t*)&ks[tok][c] = fk[j];
-      *(dl_f32x4_t*)&qs[tok][c] = fq[j];
-    }
-    vs[tid / 16][tid % 16] = fv;
-    mats[0][tid / 16][tid % 16] = fm[0];
-    mats[1][tid / 16][tid % 16] = fm[1];
-    if (tid < 32) decays[tid / 16][tid % 16] = fd;
-    __syncthreads();
-    if (t0 + DL_CHUNK < len) fetch(t0 + DL_CHUNK);
-    // this wave's channels' share of K S0 and Q S0 (element i of a lane's four channels in MFMA i,
-    // where S has the same ones as element i of its rows)
-    dl_f32x4_t pk = {0.f, 0.f, 0.f, 0.f}, pq = pk;
+    for (int b = 0; b < B; ++b) S[b] = *(const dl_f32x4_t*)(S_mem + 16 * b);
+    fetch(0);
+    for (int t0 = 0; t0 < len; t0 += DL_CHUNK) {
+      const int n = min(DL_CHUNK, len - t0);
+      __syncthreads();                        // the chunk before is done with
 #pragma unroll
-    for (int b = 0; b < B; ++b) {
-      const dl_f32x4_t kv = *(const dl_f32x4_t*)&ks[m][16 * (wave * B + b) + 4 * g];
-      const dl_f32x4_t qv = *(const dl_f32x4_t*)&qs[m][16 * (wave * B + b) + 4 * g];
+      for (int j = 0; j < PIECES; ++j) {
+        const int i = tid + 256 * j, tok = i / (d / 4), c = i % (d / 4) * 4;
+        *(dl_f32x4_t*)&ks[tok][c] = fk[j];
+        *(dl_f32x4_t*)&qs[tok][c] = fq[j];
+      }
+      vs[tid / 16][tid % 16] = fv;
+      mats[0][tid / 16][tid % 16] = fm[0];
+      mats[1][tid / 16][tid % 16] = fm[1];
+      if (tid < 32) decays[tid / 16][tid % 16] = fd;
+      __syncthreads();
+      if (t0 + DL_CHUNK < len) fetch(t0 + DL_CHUNK);
+      // this wave's channels' share of K S0 and Q S0 (element i of a lane's four channels in MFMA i,
+      // where S has the same ones as element i of its rows)
+      dl_f32x4_t pk = {0.f, 0.f, 0.f, 0.f}, pq = pk;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        pk = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i], S[b][i], pk, 0, 0, 0);
-        pq = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[i], S[b][i], pq, 0, 0, 0);
+      for (int b = 0; b < B; ++b) {
+        const dl_f32x4_t kv = *(const dl_f32x4_t*)&ks[m][16 * (wave * B + b) + 4 * g];
+        const dl_f32x4_t qv = *(const dl_f32x4_t*)&qs[m][16 * (wave * B + b) + 4 * g];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          pk = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i], S[b][i], pk, 0, 0, 0);
+          pq = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[i], S[b][i], pq, 0, 0, 0);
+        }
+      }
+      red[wave][0][lane] = pk;
+      red[wave][1][lane] = pq;
+      __syncthreads();
+      // rows 4 g + r are tokens, column m a value column; every wave forms W for its own channels
+      const dl_f32x4_t sk = (red[0][0][lane] + red[1][0][lane]) + (red[2][0][lane] + red[3][0][lane]);
+      const dl_f32x4_t tb = *(const dl_f32x4_t*)&mats[0][m][4 * g];
+      dl_f32x4_t x;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[r] = fmaf(-decays[0][4 * g + r], sk[r], vs[4 * g + r][m]);
+      const dl_f32x4_t W = dl_triangle<CAREFUL>(tb, x, dl_f32x4_t{0.f, 0.f, 0.f, 0.f}, g);
+      const float whole = decays[0][DL_CHUNK - 1];
+      float cw[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) cw[i] = decays[1][4 * g + i] * W[i];
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        float kt[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) kt[i] = ks[4 * g + i][16 * (wave * B + b) + m];
+        S[b] = S[b] * whole;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[i], cw[i], S[b], 0, 0, 0);
+      }
+      if (wave == t0 / DL_CHUNK % 4) {        // the outputs, the waves in turn
+        const dl_f32x4_t sq = (red[0][1][lane] + red[1][1][lane]) + (red[2][1][lane] + red[3][1][lane]);
+        const dl_f32x4_t mv = *(const dl_f32x4_t*)&mats[1][m][4 * g];
+        dl_f32x4_t o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = decays[0][4 * g + r] * sq[r];
+        o = dl_triangle<CAREFUL>(mv, W, o, g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (4 * g + r < n)
+            out[(size_t)(first + t0 + 4 * g + r) * H * dv + (size_t)h * dv + col0 + m] = o[r];
       }
     }
-    red[wave][0][lane] = pk;
-    red[wave][1][lane] = pq;
-    __syncthreads();
-    // rows 4 g + r are tokens, column m a value column; every wave forms W for its own channels
-    const dl_f32x4_t sk = (red[0][0][lane] + red[1][0][lane]) + (red[2][0][lane] + red[3][0][lane]);
-    const dl_f32x4_t tb = *(const dl_f32x4_t*)&mats[0][m][4 * g];
-    dl_f32x4_t x;
+  };
+  walk(std::false_type{});
+  bool finite = true;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) x[r] = fmaf(-decays[0][4 * g + r], sk[r], vs[4 * g + r][m]);
-    const dl_f32x4_t W = dl_triangle(tb, x, dl_f32x4_t{0.f, 0.f, 0.f, 0.f}, g);
-    const float whole = decays[0][DL_CHUNK - 1];
-    float cw[4];
+  for (int b = 0; b < B; ++b)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) cw[i] = decays[1][4 * g + i] * W[i];
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-      float kt[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) kt[i] = ks[4 * g + i][16 * (wave * B + b) + m];
-      S[b] = S[b] * whole;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[i], cw[i], S[b], 0, 0, 0);
-    }
-    if (wave == t0 / DL_CHUNK % 4) {        // the outputs, the waves in turn
-      const dl_f32x4_t sq = (red[0][1][lane] + red[1][1][lane]) + (red[2][1][lane] + red[3][1][lane]);
-      const dl_f32x4_t mv = *(const dl_f32x4_t*)&mats[1][m][4 * g];
-      dl_f32x4_t o;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = decays[0][4 * g + r] * sq[r];
-      o = dl_triangle(mv, W, o, g);
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (4 * g + r < n)
-          out[(size_t)(first + t0 + 4 * g + r) * H * dv + (size_t)h * dv + col0 + m] = o[r];
-    }
-  }
+    for (int i = 0; i < 4; ++i) finite = finite && fabsf(S[b][i]) < INFINITY;
+  if (__syncthreads_or(!finite)) walk(std::true_type{});
 #pragma unroll
   for (int b = 0; b < B; ++b) *(dl_f32x4_t*)(S_mem + 16 * b) = S[b];
 }
