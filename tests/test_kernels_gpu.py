@@ -1303,13 +1303,13 @@ def test_products_together_have_the_bits_of_the_products(M, K, widths):
 
 
 @pytest.mark.parametrize("M", [1, 8, 9, 16])
-@pytest.mark.parametrize("N,K", [(64, 4096), (2048, 4160), (1984, 7168)])
+@pytest.mark.parametrize("N,K", [(64, 7168), (2048, 7232), (1984, 8192)])
 @pytest.mark.parametrize("kind", ["sum", "f32", "bf16"])
 def test_narrow_products_over_a_long_k_in_parts(M, N, K, kind):
     ops = _ops()
     a = _rand((M, K), torch.bfloat16, 38).to(DEV)
     w = _rand((N, K), torch.bfloat16, 39, 0.05).to(DEV)
-    assert ops._narrow_split(M, N, K) is not None and ops._narrow_split(M, N, 4032) is None
+    assert ops._narrow_split(M, N, K) is not None and ops._narrow_split(M, N, 5056) is None
     out = _rand((M, N), torch.float32, 40).to(DEV)
     want = a.double() @ w.double().T + (out.double() if kind == "sum" else 0.0)
     bound = (K + 1) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + out.double().abs())

@@ -588,11 +588,16 @@ def _skinny_plan(M: int, N: int, K: int, tiled: bool):
 def _narrow_split(M: int, N: int, K: int):
     """Row groups per workgroup and workgroups along K for a product of up to 16 tokens whose output
     has too few row groups for half of the chip, over a long K, that has no epilogue to lose by the split:
-    a second kernel adds the parts.  Measured on MI355X, us with that kernel: 2048 outputs over K =
-    4096 / 7168, 1 token 7.1 -> 7.0, 10.1 -> 9.1, 8 tokens 8.3 -> 7.7, 12.6 -> 9.6 (two parts); 16
-    tokens, which a workgroup of one row group reads as often as W, 9.0 -> 8.0, 13.7 -> 10.8 (two row
-    groups, four parts).  Over 2048 or 3072 the second kernel costs what the split gains."""
-    if not (0 < M <= 16 and N <= 2048 and N % 32 == 0 and K >= 4096 and K % 64 == 0):
+    a second kernel adds the parts.  Two parts for up to 8 tokens from K = 7168 on, two row groups in
+    four parts for more, which a workgroup of one row group reads as often as W, from 6144 on, from
+    13 tokens from 5120 on.  Measured on MI355X in chains, us, both kernels, stored sums: 64 / 512 / 1024 /
+    2048 outputs over 7168, 8 tokens 8.5 -> 6.9, 8.9 -> 7.7, 9.2 -> 8.2, 11.7 -> 9.8; 1 token 6.8 -> 6.0,
+    7.1 -> 6.5, 7.7 -> 7.4, 9.6 -> 9.2; 16 tokens 10.9 -> 8.0, 11.4 -> 8.9, 11.7 -> 9.2, 12.9 -> 10.9, 1024 over
+    5120 9.4 -> 8.4.  Of a shorter K the second kernel costs what the split gains: 2 and 4 tokens over
+    6144 into 1536 and 2048 3 to 5 % slower, over 5120 up to 8 %, over 4096 1024 outputs 5.2 -> 5.9, 5.6 ->
+    6.2, of 9 tokens 6.3 -> 6.7, over 5120 7.6 -> 8.0, of 13 over 4096 into 2048 5 %."""
+    if not (0 < M <= 16 and N <= 2048 and N % 32 == 0 and K % 64 == 0
+            and K >= (7168 if M <= 8 else 6144 if M <= 12 else 5120)):
         return None
     return (1, 2) if M <= 8 else (2, 4)
 
