@@ -1053,7 +1053,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
                    "gemm (tiled)")
         return
     if a.dtype == torch.float32 and w.dtype == torch.float32:
-        if _f32_spans_cover(a, w, out):
+        if _f32_spans_cover(a, w, out) and _f32_spans_pay(M, N, K):
             ws = _workspace("gemm_splitk", F32_SPANS * M * N, torch.float32, a.device)
             _check(lib.zf_gemm_f32_spans(_ptr(a), _ptr(w), _ptr(out), _ptr(ws), M, N, K,
                                          1 if accumulate else 0, _ptr(None), ctypes.c_float(0.0),
@@ -1080,13 +1080,21 @@ F32_SPANS = 8           # spans of K whose sums a 32-bit product adds in order
 def _f32_spans_cover(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
     """A 32-bit product of up to 64 rows whose output is too narrow for its row groups of 16 to fill
     half of the chip: every span of K goes to a workgroup of its own and a second kernel adds
-    them, the same bits.  Measured on MI355X (4 tokens, us, both kernels): 1024 outputs over K = 2048
-    12.2 -> 8.4, over 3072 17.0 -> 9.9, 2048 over 7168 37.7 -> 20.8; 2048 over 2048 12.5 -> 10.3,
-    but of 16 tokens 11.5 -> 12.0, so a shorter K needs a narrower output."""
+    them (and runs the norm behind a residual sum), the same bits.  Measured on MI355X (4 tokens,
+    us, both kernels): 1024 outputs over K = 2048 12.2 -> 8.4, over 3072 17.0 -> 9.9, 2048 over 7168
+    37.7 -> 20.8; 2048 over 2048 12.5 -> 10.3, but of 16 tokens 11.5 -> 12.0, so a shorter K needs a
+    narrower output."""
     (M, K), N = a.shape, w.shape[0]
     return 0 < M <= SKINNY_MAX_M and N % 4 == 0 and K % 4 == 0 \
         and (K >= 1024 and N <= 1024 or K >= 4096 and N <= 2048) \
         and out.dtype == torch.float32 and all(t.data_ptr() % 16 == 0 for t in (a, w, out))
+
+
+def _f32_spans_pay(M: int, N: int, K: int) -> bool:
+    """Whether the kernel that adds the spans is worth its launch with no norm to run as well.  Into 1024
+    outputs, us: 16 rows over K = 1024 6.5 -> 7.5, 1792 6 % slower, 2048 10.5 -> 8.9; 32 rows over 1024 8.3
+    -> 8.7, 1280 4 % faster (512 outputs over 1024 8.2 -> 7.9); 64 rows over 1024 12.7 -> 11.3."""
+    return K >= (2048 if M <= 16 else 1280 if M <= 32 and N > 512 else 1024)
 
 
 def f32_sum_norm_covers(a: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
