@@ -1070,8 +1070,15 @@ F32_SWIGLU_MAX_M = 16   # rows for which the 32-bit gate/up product applies the 
 
 
 def f32_swiglu_covers(a: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether ``gemm_swiglu`` takes a gate's and an up projection's rows one below the other."""
-    return a.is_cuda and a.dtype == w.dtype == torch.float32 and 0 < a.shape[0] <= F32_SWIGLU_MAX_M
+    """Whether a gate's and an up projection's rows one below the other are ``gemm_swiglu``'s: a
+    workgroup takes 16 rows of both, of which 257 to 384 pairs fill the chip one and a half times where the
+    product alone runs in twice as many workgroups.  There, over more than 1024, the two kernels are the
+    faster: 4 rows, us, 6144 pairs of rows over 2048 / 4096 29.0 and 47.8 against 29.6 and 52.6, 5120 over
+    1536 21.7 and 22.7; over 1024 16.1 against 15.9; 4096 over 2048 20.1 against 18.5, 6160 over 4096 3 % more."""
+    M, K = a.shape
+    groups = (w.shape[0] // 2 + 15) // 16
+    return a.is_cuda and a.dtype == w.dtype == torch.float32 and 0 < M <= F32_SWIGLU_MAX_M \
+        and not (256 < groups <= 384 and K > 1024)
 
 
 F32_SPANS = 8           # spans of K whose sums a 32-bit product adds in order
