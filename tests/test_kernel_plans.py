@@ -353,3 +353,13 @@ def test_shared_arrays_accessed_in_16_byte_pieces_say_that_they_are_aligned():
             used = set(re.findall(r"\*\(\s*(?:const\s+)?" + wide + r"\s*\*\)\s*&?\s*\(?\s*(\w+)", text))
             found += [f"{os.path.basename(path)}: {name}: {array}" for array in sorted(plain & used)]
     assert not found
+
+
+@pytest.mark.parametrize("rows,width,outputs,pays", [
+    (1, 1024, 151936, False), (10, 1024, 16448, False), (16, 512, 32768, False), (8, 1280, 65536, False),
+    (11, 1024, 151936, True), (1, 1024, 16384, True), (1, 1536, 151936, True), (16, 768, 32768, True),
+    (1, 64, 0, True)])
+def test_norm_inputs_beside_picked_rows_where_they_pay(rows, width, outputs, pays):
+    """Few narrow rows ahead of a wide output (and of one that is not known) on both sides of the rule."""
+    import zinfer_amd.ops as ops
+    assert ops.picked_norm_pays(rows, width, outputs) == pays

@@ -146,10 +146,10 @@ class DecoderModel:
         return total
 
     @staticmethod
-    def _pick(norm, table: torch.Tensor, rows: torch.Tensor, step, pick):
+    def _pick(norm, table: torch.Tensor, rows: torch.Tensor, step, pick, outputs: int = 0):
         """Runs ``pick``, which picks ``rows`` from ``table``, and has it leave what ``norm``, which
-        reads them next, can use; returns that, or None."""
-        left = norm.picked(table, rows, step) if isinstance(norm, Norm) else None
+        reads them next, can use; returns that, or None.  ``outputs``: as ``Norm.picked``'s."""
+        left = norm.picked(table, rows, step, outputs) if isinstance(norm, Norm) else None
         pick(**({} if left is None else {"given": left.buffers}))
         return left
 
@@ -230,7 +230,8 @@ class DecoderModel:
         else:
             rows = step.scratch("want_rows", (n_rows, s.hidden_size), torch.float32)
             left = self._pick(self.final_norm, x, rows, step,
-                              lambda **given: ops.gather_rows(x, step.want_rows, rows, **given))
+                              lambda **given: ops.gather_rows(x, step.want_rows, rows, **given),
+                              self.head.out_features)
         make = lambda: step.scratch("final_normed", (n_rows, s.hidden_size), self.ctx.act_dtype)
         with ops.kernel_class("head_sampling"):      # what a per-class measurement counts these as
             if isinstance(left, NormedRows) and left.fits(self.final_norm, rows):

@@ -137,6 +137,17 @@ def rows_leave_norm(table: torch.Tensor, gain: torch.Tensor, rows: torch.Tensor)
         and all(t.data_ptr() % 16 == 0 for t in (table, gain, rows))
 
 
+def picked_norm_pays(rows: int, width: int, outputs: int) -> bool:
+    """Whether the product of ``outputs`` columns behind picked rows is the faster for the norm's
+    inputs beside them.  A wave of it has few steps of a narrow K, which its two sets of registers do
+    nothing for: they leave a SIMD three waves, the kernel that folds the norm in seven, and where
+    workgroups run in many rounds that outweighs what folding reads for a few rows.  Gathering kernel
+    and product, us, folded / from given inputs: 1024 wide into 151936, 1 / 8 / 16 rows 54 / 61, 61 / 66,
+    84 / 75, into 16384 2 to 10 % faster from given ones; 768 wide into 65536, 8 rows 12 % slower; 1536
+    wide into 151936 level at one row, 26 % faster at 16."""
+    return not (outputs > 16384 and width <= 1280 and rows * width <= 10 * 1024)
+
+
 def _check_given(given, table: torch.Tensor, rows: torch.Tensor) -> None:
     """``given`` = (gain, xg, sq) of the float32 ``rows`` picked from ``table``, or None."""
     if given is None:

@@ -184,9 +184,10 @@ class Norm(Part):
       (runs the norm once, returns the activations) and ``fold_into(linear, out, **kw)`` (the
       product of the normed rows with ``linear``'s weight in one kernel, or False).  None:
       the norm simply runs.  ``left``: what ``residual_sum`` left for this norm, or None.
-    * ``picked(table, x, step)``: for rows ``x`` about to be picked from ``table`` (an embedding,
-      the rows whose logits are wanted): an object whose ``buffers`` the kernel that picks them
-      also writes, and which then is what ``residual_sum`` leaves.  None: nothing beside the rows.
+    * ``picked(table, x, step, outputs)``: for rows ``x`` about to be picked from ``table`` (an
+      embedding, the rows whose logits are wanted): an object whose ``buffers`` the kernel that picks
+      them also writes, and which then is what ``residual_sum`` leaves.  None: nothing beside the
+      rows.  ``outputs``: of the product that reads the normed rows, where the caller knows it.
     * ``residual_sum(linear, a, out, step)``: out += a W^T in a kernel that also leaves
       something for this norm, which reads ``out`` next; puts it in ``step.norm_ready`` and
       returns True, or returns False and does nothing."""
@@ -201,7 +202,7 @@ class Norm(Part):
     def deferred(self, x: torch.Tensor, make_out, left=None):
         return None
 
-    def picked(self, table: torch.Tensor, x: torch.Tensor, step):
+    def picked(self, table: torch.Tensor, x: torch.Tensor, step, outputs: int = 0):
         return None
 
     def residual_sum(self, linear, a: torch.Tensor, out: torch.Tensor, step) -> bool:

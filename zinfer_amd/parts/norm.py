@@ -39,9 +39,10 @@ class RmsNorm(Norm):
             return None
         return LazyRmsNorm(self, x, make_out, given)
 
-    def picked(self, table: torch.Tensor, x: torch.Tensor, step):
+    def picked(self, table: torch.Tensor, x: torch.Tensor, step, outputs: int = 0):
         if not (x.is_cuda and self.ctx.compute_dtype == torch.bfloat16
-                and x.shape[1] % 64 == 0 and ops.rows_leave_norm(table, self.gain, x)):
+                and x.shape[1] % 64 == 0 and ops.rows_leave_norm(table, self.gain, x)
+                and ops.picked_norm_pays(*x.shape, outputs)):
             return None
         return GivenRmsNorm(self, x, *self._given_buffers(x, step))
 
