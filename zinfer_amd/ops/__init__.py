@@ -1224,9 +1224,13 @@ def _tile256_ksplit(M: int, N: int, K: int):
     into 5120 114 -> 105, 25600 162 -> 145; 640 tokens 150 -> 131; 1024 212 -> 172; over 5120
     into 5120 88 -> 76; 12288 into 4096 at 768 / 1100 tokens 107 -> 94, 152 -> 128.  Of parts under
     1600 the partials cost what the tiles gain (512 tokens over 8192 into 5120, six parts: 66 -> 66,
-    768 over 5120, four: 60 -> 65), and where the 128 x 128 tiles fill the chip once they lose up to
-    K = 8192 and win from 12288 on (2048 tokens into 2048: 7168 70 -> 78, 8192 81 -> 86, 12288 115
-    -> 110, all without a norm; 1536 tokens 65 -> 70, 73 -> 72, 104 -> 97).  Not in two parts: unsplit tiles fill most of the chip there as
+    768 over 5120, four: 60 -> 65).  Where the 128 x 128 tiles fill the chip once, with 180 to 256 of them, the
+    line is 10240 (over 8192 256 tiles are level, 2048 tokens into 2048 87 -> 88, into 8192 512 tokens
+    93 -> 85, and up to 224 6 to 25 % would be gained; over 10240 4 to 20 %).  257 to 384 tokens leave a
+    quarter of these tiles empty, and of 128 x 128 ones little: only in up to five parts of 1900 and
+    more that fill fifteen sixteenths of the chip (384 tokens over 9728 into 6144 80 -> 72, 8192 98 -> 87; into
+    5120, six parts, 60 -> 65, into 7168, 224 parts, 3 % slower over any K, over 8192 into 6400 2 %).  Not in
+    two parts: unsplit tiles fill most of the chip there as
     well (2048 tokens into 4096 over 12288 192 -> 186, over 4096 80 -> 89, and nothing of the former
     is left in a whole prompt's step, which the chip's power limits)."""
     if M <= 256 or K % 128 != 0 or N % 16 != 0 or N > 8192:
@@ -1235,6 +1239,8 @@ def _tile256_ksplit(M: int, N: int, K: int):
     ks = 256 // tiles
     one_round = 180 <= ((M + 127) // 128) * ((N + 127) // 128) <= 256
     if not 3 <= ks <= 6 or tiles * ks < 224 or K < max(1600 * ks, 10240 if one_round else 0):
+        return None
+    if M <= 384 and (ks > 5 or tiles * ks < 240 or K < 1900 * ks):
         return None
     return ks
 
