@@ -1186,8 +1186,8 @@ __global__ __launch_bounds__(1024) void moe_few_down_kernel(
     const int nb = shared ? s_blocks : blocks;
     int pair;
     const bf16_t *wr, *x;
-    // (the two halves of even and odd steps in a sum each, the pieces' sums four side by side: the
-    // outputs of ff = 4096 from given activations 1.34e-7 off with one sum, 1.04e-7 so, 1.05e-7 row by row)
+    // (the two halves of the blocks in a sum each, the pieces' sums four side by side: the outputs of ff
+    // = 4096 from given activations 1.34e-7 off with one sum, 1.04e-7 so, 1.05e-7 row by row)
     // rows r and columns r: output n0 + r % 8 and pair r % 8 at the blocks 2 i + r / 8
     for (int p0 = 0; p0 < (shared ? T : 8); p0 += 8) {
       if (shared) {
@@ -1202,12 +1202,9 @@ __global__ __launch_bounds__(1024) void moe_few_down_kernel(
       wr += (size_t)(n0 / 16) * nb * 1024 + (g * 16 + n0 % 16 + r % 8) * 8;
       x += 16 * g;
       const int b0 = c * 2 * piece, b1 = min(nb, b0 + 2 * piece);
-      moe_f32x4_t acc[2][2];
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) acc[j][i] = moe_f32x4_t{0.f, 0.f, 0.f, 0.f};
-      auto take = [&](int kb, moe_f32x4_t (&sum)[2]) {
+      moe_f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 4
+      for (int kb = b0; kb < b1; kb += 2) {
         // (behind an odd last block the upper half repeats it against zeros)
         const bool in = kb + half < b1;
         const int k = in ? kb + half : kb;
@@ -1220,19 +1217,14 @@ __global__ __launch_bounds__(1024) void moe_few_down_kernel(
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-          sum[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&wf[i],
-                                                           *(const moe_bf16x8_t*)&xf[i], sum[i], 0, 0, 0);
-      };
-#pragma unroll 2
-      for (int kb = b0; kb < b1; kb += 4) {
-        take(kb, acc[0]);
-        if (kb + 2 < b1) take(kb + 2, acc[1]);
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&wf[i],
+                                                           *(const moe_bf16x8_t*)&xf[i], acc[i], 0, 0, 0);
       }
       // rows 4 g + i of column r: like halves are g / 2 == half
       if (pair >= 0 && g / 2 == half)
         *(moe_f32x4_t*)((shared ? s_sums + ((size_t)pair * s_pieces + c) * 16
                                 : sums + ((size_t)pair * pieces + c) * 16) + 8 * half + 4 * (g % 2)) =
-            (acc[0][0] + acc[0][1]) + (acc[1][0] + acc[1][1]);
+            acc[0] + acc[1];
     }
   }
   __syncthreads();
@@ -1283,11 +1275,11 @@ extern "C" int zf_moe_few(const void* h, const void* gate_up, const void* down, 
                      s_limit, s_alpha, s_shift, factor, factor_stride)
   if (gated) MOE_FEW_UP(true); else MOE_FEW_UP(false);
 #undef MOE_FEW_UP
-  // pieces of up to 8 blocks of ff, as even as they come, larger ones where the partials of 16 tokens
-  // would not fit 48 KB of LDS (by the layer's sizes alone: a token's sums must not depend on how
-  // many tokens there are)
-  const int parts = (ff / 64 + 7) / 8;
-  int piece = (ff / 64 + 2 * parts - 1) / (2 * parts);
+  // pieces of 2 x 128 of ff, larger ones where the partials of 16 tokens would not fit 48 KB of
+  // LDS (by the layer's sizes alone: a token's sums must not depend on how many tokens there are).
+  // Pieces of up to 8 blocks, their sums in four accumulators, were 4 to 8 % slower for one or two tokens of
+  // top 1 and 2 (W = 2048, ff = 512, us 12.3 for 13.1) and 2 to 4 % faster only for some of eight and more.
+  int piece = 2;
   const auto pieces = [](int width, int p) { return (width / 64 + 2 * p - 1) / (2 * p); };
   const auto lds = [&](int tokens, int p) {
     return (size_t)tokens * (top * pieces(ff, p) + pieces(shared_ff, p)) * 64;
