@@ -1785,15 +1785,18 @@ extern "C" int zf_attn_prefill_bf16(const void* q, const void* k_pool, const voi
     // behind 500 keys, 16 / 32 heads on 8: 32.1 -> 20.8, 30.3 -> 25.8 us; 256 workgroups, 512 tokens
     // behind 900, 44.1 -> 37.6; 264, five portions of 200 behind 900, 36.5 -> 47.6; two heads of 64,
     // 512 workgroups, 33.8 -> 23.1, 600 28.3 -> 28.6).  Five to eight heads go to two workgroups then, up
-    // to 128 of them before (497 tokens behind 0 / 500 / 1400 keys, 40 heads on 8, 23.2 -> 16.9, 38.9 -> 26.0,
+    // to 144 of them before (497 tokens behind 0 / 500 / 1400 keys, 40 heads on 8, 23.2 -> 16.9, 38.9 -> 26.0,
     // 64.9 -> 40.5 us; eight portions of 20 to 64 behind none 10.9 -> 10.5): of more the halves share
-    // CUs (208, four prompts of 200 15.6 -> 20.8; 160, three portions of 200 behind 300 25.3 -> 28.0), which
-    // pays only where portions of 768 tokens and more are unequal enough (64 heads on 8: 256, 1024 tokens
-    // behind 900, 74.4 -> 71.0; 192, 768 behind 300, 45.3 -> 40.5; 208, 400 tokens 23.5 -> 25.5).
+    // CUs, which up to 144 portions of unequal length leave room for (cuts of 490 to 540 tokens behind
+    // up to 1300 keys, 136 and 144 workgroups, 40, 48 and 64 heads on 8, 126 mixes, 0.86 to 1.54 times as
+    // fast, 1.18 in the mean; 152 to 176, 161 mixes, 1.10, without much before them 1.03; of equal
+    // ones 208, four prompts of 200, 15.6 -> 20.8), and beyond portions of 768 tokens and more alone (64 heads
+    // on 8: 256, 1024 tokens behind 900, 74.4 -> 71.0; 192, 768 behind 300, 45.3 -> 40.5; 208, 400 tokens
+    // 23.5 -> 25.5).
     const unsigned blocks = entries * nKV;
     const bool groups = variant != 3 && split_keys == 0 &&
                         (allow_split || blocks <= (hd == 64 && G <= 2 ? 512u : 256u));
-    const bool halves = groups && G > 4 && G <= 8 && blocks <= (max_q_len >= 768 ? 256u : 128u);
+    const bool halves = groups && G > 4 && G <= 8 && blocks <= (max_q_len >= 768 ? 256u : 144u);
     const int heads = halves ? (G + 1) / 2 : G < 8 ? G : 8, head_blocks = (G + heads - 1) / heads;
     dim3 sgrid(entries * head_blocks * nKV, split_keys > 0 ? max_splits : 1);
     const int ks = groups && heads <= 4 && sgrid.x <= 1024 ? 2 : 1;
