@@ -652,7 +652,9 @@ extern "C" int zf_delta_recurrence(const float* qkv, int C, int q_off, int k_off
 //   W = Tb (V - exp(G) (K S0)),   Tb = (I + L)^-1 diag(beta),  L_ti = beta_t exp(G_t - G_i) k_t . k_i, i < t
 //   O = exp(G) (Q S0) + M W,      M_ti = exp(G_t - G_i) q_t . k_i, i <= t
 //   S = exp(G_15) S0 + K^T (exp(G_15 - G) W)
-// (the delta rule's chunked form by its triangular system, as published for linear attention).
+// (the chunked form by its triangular system: Yang, Wang, Zhang, Shen and Kim, "Parallelizing Linear
+// Transformers with the Delta Rule over Sequence Length", 2024; with decays Yang, Kautz and Hatamizadeh,
+// "Gated Delta Networks", 2024).
 // Everything is 32-bit: v_mfma_f32_16x16x4_f32, expf, fused multiply-adds; no ratio of decays exceeds 1.
 // A token that is not finite reaches itself and the tokens behind it, as in the walk: the triangular
 // matrices hold zeros above their diagonals, whatever the token brings, but such zeros against its
@@ -664,7 +666,8 @@ extern "C" int zf_delta_recurrence(const float* qkv, int C, int q_off, int k_off
 //                          chunks with S in the accumulators of the waves, d / 64 blocks of 16 key
 //                          channels each.
 // The walk token by token is bound by the vector units' issue: some 100 instructions a token and
-// wave, 2.5 waves to a SIMD; here a chunk costs a wave 24 MFMAs of 32 cycles (d = 128).
+// wave, 2.5 waves to a SIMD; here a chunk costs a wave 28 MFMAs of 32 cycles (d = 128), 32 the one that
+// forms its outputs.
 // Measured (16 heads of 128 x 128, a step of 2048 tokens of five prompts, the longest 680, us): 290
 // walked, 87 + 15 in chunks; on inputs of such sizes 2.3 to 3.3e-7 off the 64-bit rule behind 200 to 2000
 // tokens, the walk 2.9e-7 to 1.1e-6.
