@@ -1,5 +1,6 @@
 """Which kernel serves which size: the pure decisions of `zinfer_amd.ops`, without a GPU."""
 import pytest
+import torch
 
 from zinfer_amd import ops
 
@@ -361,5 +362,20 @@ def test_shared_arrays_accessed_in_16_byte_pieces_say_that_they_are_aligned():
     (1, 64, 0, True)])
 def test_norm_inputs_beside_picked_rows_where_they_pay(rows, width, outputs, pays):
     """Few narrow rows ahead of a wide output (and of one that is not known) on both sides of the rule."""
-    import zinfer_amd.ops as ops
     assert ops.picked_norm_pays(rows, width, outputs) == pays
+
+
+@pytest.mark.parametrize("dtype,head_dim,page_size,pages,width", [
+    (torch.float32, 128, 16, 1, 4), (torch.float32, 64, 16, 4, 4), (torch.float32, 128, 16, 5, 16),
+    (torch.float32, 128, 48, 1, 1), (torch.float32, 128, 128, 1, 2), (torch.float32, 96, 16, 1, 16),
+    (torch.float32, 128, 8, 1, 32), (torch.bfloat16, 128, 16, 1, 16), (torch.float32, 128, 16, 17, None)])
+def test_table_widths_of_captured_decode_steps(dtype, head_dim, page_size, pages, width):
+    """A table of one chunk of keys where the 32-bit kernel for few waves runs, of one split of the
+    decode kernel else, and the engine's own bucket beyond."""
+    from zinfer_amd.parts.attention import GqaAttention
+
+    class Part:
+        spec = type("", (), {"head_dim": head_dim})
+        ctx = type("", (), {"act_dtype": dtype})
+
+    assert GqaAttention.graph_table_pages(Part, pages, page_size) == width

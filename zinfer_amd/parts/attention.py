@@ -106,9 +106,10 @@ class GqaAttention(Mixer):
         # contexts within one split of the decode attention get a table width of their own:
         # that kernel then writes the output itself and no merge kernel runs
         short = max(1, ops.DECODE_SPLIT_KEYS // page_size)
-        # (in 32-bit within one chunk of keys too, which one wave a head takes)
+        # (in 32-bit within one chunk of keys too, which one wave a head of 64 or 128 takes)
         chunk = ops.ATTENTION_CHUNK_KEYS // page_size
-        if self.ctx.act_dtype == torch.float32 and pages <= chunk:
+        if self.ctx.act_dtype == torch.float32 and self.spec.head_dim in (64, 128) \
+                and page_size % 16 == 0 and pages <= chunk:
             return chunk
         return short if pages <= short else None
 
