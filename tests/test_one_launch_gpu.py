@@ -1,0 +1,176 @@
+"""A decode step's layers in one launch: which sizes it takes (CPU), and on the GPU its logits against
+the plain implementation and against a launch a product, where its work is dealt unevenly."""
+import ctypes
+import gc
+import threading
+import weakref
+
+import numpy as np
+import pytest
+import torch
+
+import plain
+import tiny
+from gpu_util import DEV
+from test_engine_gpu import LOGITS_TOL_BF16
+from zinfer_amd.config import Qwen3Config
+from zinfer_amd.models import one_launch
+from zinfer_amd.models.build import declare_tensors
+from zinfer_amd.ops import build
+from zinfer_amd.ops import decode_layers as kernel
+from zinfer_amd.weights import draw_tensors
+
+
+def test_the_sizes_python_accepts_are_accepted_by_the_entry():
+    """No device here: the entry refuses sizes (-3) before it asks for one."""
+    lib = build.load("decode_layers")
+    accepted = 0
+    for wgs in (32, 256, 304):
+        for hidden in (448, 512, 576, 1000, 5120, 8192, 32768):
+            for ff in (256, 512, 1088, 12288, 25600, 32768, 53248):
+                for heads, kv in ((2, 1), (4, 4), (16, 1), (15, 1), (32, 8), (40, 8), (96, 96), (12, 5)):
+                    for page in (8, 16, 48):
+                        p = kernel._Layers()
+                        p.tokens, p.n_layers, p.hidden, p.ff = 1, 1, hidden, ff
+                        p.n_heads, p.n_kv_heads, p.page_size = heads, kv, page
+                        p.max_splits = kernel.MAX_SPLITS
+                        if kernel.sizes_covered(1, hidden, ff, heads, kv, 128, page, wgs):
+                            accepted += 1
+                            if not torch.cuda.is_available():      # (nothing is launched without one)
+                                assert lib.zf_decode_layers(ctypes.byref(p), wgs, None) != -3, \
+                                    (wgs, hidden, ff, heads, kv, page)
+    assert accepted > 100
+
+
+def _qwen3(hidden, heads, kv, ff, layers=2, vocab=1030):
+    return dict(architectures=["Qwen3ForCausalLM"], model_type="qwen3", num_hidden_layers=layers,
+                hidden_size=hidden, num_attention_heads=heads, num_key_value_heads=kv, head_dim=128,
+                intermediate_size=ff, vocab_size=vocab, rope_theta=1000000.0, rms_norm_eps=1e-6,
+                tie_word_embeddings=False, max_position_embeddings=4096, torch_dtype="bfloat16")
+
+
+def _engine(cfg, weights, page=16, tokens=4096, graphs=True):
+    from zinfer_amd.engine import Engine
+    from zinfer_amd.models.build import build_model
+    model = build_model(Qwen3Config.from_dict(cfg).model_spec(), weights, "bfloat16", DEV)
+    return Engine(model, page_size=page, num_pages=(tokens + page - 1) // page + 2, max_requests=4,
+                  use_graphs=graphs)
+
+
+def _weights(cfg, seed):
+    spec = Qwen3Config.from_dict(cfg).model_spec()
+    drawn = draw_tensors(declare_tensors(spec), seed, torch.bfloat16, tied=False, device=DEV)
+    return {k: t.cpu() for k, t in drawn.items()}
+
+
+def _answer(eng, toks, singles):
+    """The prompt's last row and every single token's, on the host."""
+    from zinfer_amd.engine import StepEntry
+    n = len(toks) - singles
+    rows = [eng.step([StepEntry("r", toks[:n], [n - 1])]).float().cpu().numpy().copy()]
+    for t in toks[n:]:
+        rows.append(eng.step([StepEntry("r", [t], [0])]).float().cpu().numpy().copy())
+    eng.release("r")
+    return np.concatenate(rows)
+
+
+# (width, heads, kv heads, feed-forward, page, tokens, of these alone): the narrowest; one head group of
+# fifteen; a kv head a head; widths that leave waves without a tile and workgroups without a row group;
+# pages of three times sixteen; contexts that begin and pass a wave's 32 keys and a split's 128; the
+# served sizes with two to nine splits
+SHAPES = [(512, 4, 2, 512, 16, 40, 36), (576, 15, 1, 1088, 48, 140, 16), (832, 4, 4, 832, 16, 262, 10),
+          (1024, 16, 8, 3072, 16, 133, 8), (2560, 32, 8, 9728, 32, 70, 8), (4096, 32, 8, 12288, 16, 1030, 12)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_single_tokens_against_the_plain_implementation(shape, monkeypatch):
+    """Logits of every single token; a launch a product stays within the same bound of them.  Workgroups
+    that come and go (more than the CUs hold, fewer than there are) leave the bits as they are, and so does a
+    graph."""
+    hidden, heads, kv, ff, page, n, singles = shape
+    cfg = _qwen3(hidden, heads, kv, ff)
+    w = _weights(cfg, hidden + heads)
+    toks = tiny.random_tokens(n, cfg["vocab_size"], n)
+    ref = plain.model_forward_batched(cfg, w, toks).numpy()[-singles - 1:]
+    monkeypatch.setattr(one_launch.OneLaunchLayers, "forward", _counted(calls := []))
+    eng = _engine(cfg, w, page)
+    assert eng.model.one_launch is not None
+    got = _answer(eng, toks, singles)
+    assert len(calls) >= 2, "the layers did not run in one launch"
+    assert eng.graph_replays > 0
+    scale = np.abs(ref).max()
+    assert np.abs(got - ref).max() <= LOGITS_TOL_BF16 * scale
+    assert np.array_equal(_answer(eng, toks, singles), got)
+    assert np.array_equal(_answer(_engine(cfg, w, page, graphs=False), toks, singles), got)
+    monkeypatch.setattr(kernel, "workgroups", lambda index: 2 * eng.model.one_launch.wgs)
+    assert np.array_equal(_answer(_engine(cfg, w, page), toks, singles), got)
+    fewer = 2 * max(ff // 256, hidden // 256, (heads + 2 * kv) // 2, kv * 8) + 3
+    monkeypatch.setattr(kernel, "workgroups", lambda index: fewer)
+    assert np.array_equal(_answer(_engine(cfg, w, page), toks, singles), got)
+    apart = _engine(cfg, w, page)
+    apart.model.one_launch = None
+    assert np.abs(_answer(apart, toks, singles) - got).max() <= LOGITS_TOL_BF16 * scale
+
+
+def _counted(calls):
+    forward = one_launch.OneLaunchLayers.forward
+
+    def counted(self, *args):
+        calls.append(1)
+        return forward(self, *args)
+    return counted
+
+
+@pytest.mark.gpu
+def test_two_engines_on_two_streams_at_once():
+    """Launches that meet deal their work among the workgroups each has: the same bits as alone."""
+    cfg = _qwen3(1024, 16, 8, 3072, layers=6)
+    w = _weights(cfg, 5)
+    toks = tiny.random_tokens(60, cfg["vocab_size"], 6)
+    engines = [_engine(cfg, w, tokens=128) for _ in range(2)]
+    alone = [_answer(e, toks, 40) for e in engines]
+    assert np.array_equal(*alone)
+    got = [[], []]
+
+    def go(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(4):
+                got[i].append(_answer(engines[i], toks, 40))
+    threads = [threading.Thread(target=go, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for rows in got:
+        assert len(rows) == 4 and all(np.array_equal(r, alone[0]) for r in rows)
+
+
+@pytest.mark.gpu
+def test_a_model_goes_with_its_last_reference():
+    cfg = _qwen3(512, 4, 2, 512)
+    eng = _engine(cfg, _weights(cfg, 7), tokens=128)
+    assert eng.model.one_launch is not None
+    model = weakref.ref(eng.model)
+    gc.disable()
+    try:
+        del eng
+        assert model() is None
+    finally:
+        gc.enable()
+
+
+@pytest.mark.gpu
+def test_a_failed_wait_is_an_error_of_the_next_step():
+    """(the flag set by the host, as the kernel sets it when a wait comes to its end)"""
+    from zinfer_amd.engine import StepEntry
+    from zinfer_amd.errors import StepError
+    cfg = _qwen3(512, 4, 2, 512)
+    eng = _engine(cfg, _weights(cfg, 7), tokens=128)
+    eng.step([StepEntry("r", [1, 2, 3], [2])])
+    eng.step([StepEntry("r", [4], [0])])
+    torch.cuda.synchronize()
+    eng._scratch.kept(one_launch.STATUS)[0] = 1
+    with pytest.raises(StepError, match="hear"):
+        eng.step([StepEntry("r", [5], [0])])
+    assert eng.length("r") == 4

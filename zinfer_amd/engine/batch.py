@@ -66,6 +66,10 @@ class Scratch:
             buf = self._made[name] = make(self.device)
         return buf
 
+    def kept(self, name: str):
+        """What ``made`` gave under this name, or None."""
+        return self._made.get(name)
+
 
 _ELEMENT_SIZE = {torch.float32: 4, torch.bfloat16: 2, torch.int32: 4, torch.int64: 8,
                  torch.float16: 2, torch.uint8: 1, torch.float64: 8}

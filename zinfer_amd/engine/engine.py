@@ -16,6 +16,7 @@ import torch
 from ..cache import CacheManager
 from ..errors import (CacheFull, ConfigError, PositionOutOfBounds, StepError,
                       TokenIdOutOfBounds)
+from ..models import one_launch
 from ..models.decoder import DecoderModel
 from ..parts.base import StepHints, StepShape
 from .batch import KVStepTables, Scratch, StepContext, StepEntry
@@ -96,6 +97,7 @@ class Engine:
         Requests in ``end`` give back what they hold after the step.  On an error the cache
         is as before: what can be refused is refused before anything runs, and a failure
         inside the run gives back what the step had reserved."""
+        self._check_waits()
         seen, wanted_len = self._check_entries(entries)
         for rid in end:
             if rid not in seen and not self.cache.has_request(rid):
@@ -272,6 +274,7 @@ class Engine:
             raise StepError("decode_steps: every entry brings one token and wants its logits")
         if records is not None and records.shape != (n_steps, n):
             raise StepError(f"decode_steps: records must be [{n_steps}, {n}]")
+        self._check_waits()
         extra = n_steps - 1
         _, wanted_len = self._check_entries(entries, extra)
         if not self.cache.can_reserve(wanted_len):
@@ -422,6 +425,12 @@ class Engine:
     def _restore_states(self, slots, saved) -> None:
         for pool, index, rows in saved:
             pool.index_copy_(0, index, rows)
+
+    def _check_waits(self) -> None:
+        """Raises once a kernel whose workgroups wait for each other has given up (its rows are NaN)."""
+        status = self._scratch.kept(one_launch.STATUS)
+        if status is not None and int(status[0]) != 0:
+            raise StepError("the workgroups of an earlier decode step did not hear from each other")
 
     def _generations(self) -> tuple:
         from .. import ops

@@ -15,6 +15,7 @@ from ..parts import BuildContext, TensorDecl, build_part
 from ..parts.base import Norm
 from ..parts.block import NormedRows
 from ..parts.linear import Linear, place_matrix
+from .one_launch import OneLaunchLayers
 
 
 class DecoderModel:
@@ -41,6 +42,7 @@ class DecoderModel:
         self.graph_safe = self.final_norm.graph_safe and all(b.graph_safe for b in self.blocks)
         # (inspection) called with (schedule position, the stream) behind every run of a block
         self.layer_probe = None
+        self.one_launch = None          # a decode step's layers in one launch, where the model allows
         # embedding, row gather and head are the model's own launches
         self.kernel_modules = tuple(sorted(
             {"elementwise", "gemm"}
@@ -118,6 +120,9 @@ class DecoderModel:
             # head's product reads a second copy in the kernels' own order (the embedding
             # itself stays in rows for the gather); elsewhere both are one tensor.
             self.head = Linear(self.embedding)
+        self.one_launch = OneLaunchLayers.of(self)
+        if self.one_launch is not None:
+            self.kernel_modules = tuple(sorted(set(self.kernel_modules) | {"decode_layers"}))
 
     def hint_providers(self):
         """One part per ``hint_key`` among all the blocks' parts: the engine asks each once a
@@ -199,7 +204,10 @@ class DecoderModel:
             for c in range(1, s.streams):
                 copies[c].copy_(x)
             x = copies
-        for pos, e in enumerate(s.schedule):
+        in_one = self.one_launch is not None and self.one_launch.takes(self, step, caches, step.norm_ready)
+        if in_one:
+            step.norm_ready = self.one_launch.forward(self, step, caches, x, step.norm_ready)
+        for pos, e in enumerate(() if in_one else s.schedule):
             if e.reentry:
                 # x = W [x ; x0]: both streams side by side in the products' type, one product
                 both = step.scratch("reentry_rows", (T, 2 * s.hidden_size), self.ctx.act_dtype)

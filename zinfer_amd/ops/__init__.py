@@ -109,6 +109,11 @@ class kernel_class:
         _class_override = self._before
 
 
+def measures_classes() -> bool:
+    """Whether a per-class measurement is running (``only_classes``)."""
+    return _class_filter is not None
+
+
 def _left_out(cls: str) -> bool:
     return _class_filter is not None and (_class_override or cls) not in _class_filter
 
