@@ -1113,6 +1113,41 @@ def test_decode_attention_one_split_writes_what_the_merge_would(nH, nKV, hd, pag
     assert rel_err(outs[0], want) <= 2 * tol(dtype)
 
 
+WHOLE_CONTEXTS = [1, 17, 63, 64, 65, 255, 256, 257, 300, 448, 511, 512, 513, 575, 576, 577, 640, 767, 768,
+                  769, 1000, 1008, 1023, 1024, 2, 100]
+
+
+@pytest.mark.parametrize("nH,nKV,page_size,window,longest", [
+    (32, 8, 16, 0, 1024), (40, 8, 16, 300, 1024), (128, 8, 32, 600, 768), (64, 16, 48, 0, 512), (90, 6, 16, 0, 1024),
+    (96, 12, 16, 40, 1024)])
+def test_decode_attention_of_whole_contexts(nH, nKV, page_size, window, longest):
+    """Two to four splits of many sequences by one workgroup each, against the same batch under a table of five
+    splits, which runs a workgroup a split and the merge kernel: the same bits.  And the form that norms,
+    rotates and stores itself against the two kernels."""
+    dtype, ops, hd = torch.bfloat16, _ops(), 128
+    ctx_lens = [c for c in WHOLE_CONTEXTS if c <= longest]
+    ctx_lens += ctx_lens[:max(0, 192 // nKV - len(ctx_lens))]
+    while len(ctx_lens) * nKV < 192:
+        ctx_lens.append(longest)
+    n = len(ctx_lens)
+    s = _paged_setup(dtype, nH, nKV, hd, page_size, ctx_lens, [1] * n, seed=33)
+    d = {k: v.to(DEV) for k, v in s.items() if isinstance(v, torch.Tensor)}
+    d["k_pool"] = ref.tile_k_pool(d["k_pool"], nKV, page_size, hd)
+    d["v_pool"] = ref.tile_v_pool(d["v_pool"], nKV, page_size, hd)
+    outs = []
+    for bound in (longest, 1280):
+        table = torch.full((n, -(-bound // page_size)), -1, dtype=torch.int32, device=DEV)
+        table[:, :d["block_table"].shape[1]] = d["block_table"]
+        out = torch.full((n, nH * hd), float("nan"), dtype=dtype, device=DEV)
+        ops.paged_attention(d["q"], d["k_pool"], d["v_pool"], table, d["q_start"], d["ctx_len"],
+                            d["seq_index"], out, 1.0 / math.sqrt(hd), window, nH, nKV, hd,
+                            page_size, 1, bound, n_single=n)
+        outs.append(out)
+    assert not torch.isnan(outs[0].float()).any()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    _fused_against_two_kernels(ops, nH, nKV, hd, page_size, window, True, True, ctx_lens)
+
+
 def _fused_against_two_kernels(ops, nH, nKV, hd, page_size, window, use_norm, use_rope, ctx_lens):
     from zinfer_amd.parts.position import rotary_tables
     dtype = torch.bfloat16

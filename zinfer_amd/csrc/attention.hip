@@ -465,36 +465,131 @@ __device__ __forceinline__ void decode_write_partial(float (&s_o)[4][16][HD], fl
   }
 }
 
+// Contexts of two to four splits by one workgroup of eight waves (WHOLE kernels): wave w takes the
+// keys [64 w, 64 w + 64) and those 512 behind them, and the partials of all meet in LDS.  The
+// merge kernel (4.6 us) and the workgroups of splits that a context does not reach are gone; a CU
+// loads 64 KB a us, though, so that this pays where sequences and kv heads alone fill the chip
+// (decode_takes_whole).  Splits are combined as decode_write_partial and the merge kernel do it, in
+// their order: the same bits.
+#define WHOLE_WAVES 8
+#define WHOLE_KEYS (WHOLE_WAVES * DEC_WAVE_KEYS)        // of one round
+#define WHOLE_SPLITS 4
+
+// floats of LDS behind one another: outputs [partial][G][HD], maxima and sums [partial][16]
 template <int HD>
-__global__ __launch_bounds__(256) void attn_decode_kernel(
+__host__ __device__ constexpr int whole_floats(int G, int rounds) {
+  return rounds * WHOLE_WAVES * (G * HD + 2 * 16);
+}
+
+// a wave's partial for query column j: rows d = 16 dt + 4 qd + r
+template <int HD>
+__device__ __forceinline__ void whole_put(float* part, int G, int rounds, int at, int j, int qd, float m, float l,
+                                          const f32x4_t (&o)[HD / 16]) {
+  if (j < G) {
+#pragma unroll
+    for (int dt = 0; dt < HD / 16; ++dt) *(f32x4_t*)(part + (at * G + j) * HD + dt * 16 + 4 * qd) = o[dt];
+  }
+  float* ml = part + rounds * WHOLE_WAVES * G * HD;
+  if (qd == 0) {
+    ml[at * 16 + j] = m;
+    ml[(rounds * WHOLE_WAVES + at) * 16 + j] = l;
+  }
+}
+
+template <int HD>
+__device__ __forceinline__ void whole_combine(const float* part, int G, int rounds, int lo, int ctx,
+                                              bf16_t* __restrict__ out_row) {
+  const float* s_m = part + rounds * WHOLE_WAVES * G * HD;
+  const float* s_l = s_m + rounds * WHOLE_WAVES * 16;
+  const int first = lo / DEC_SPLIT, last = (ctx - 1) / DEC_SPLIT;
+  for (int idx = threadIdx.x; idx < G * HD; idx += WHOLE_WAVES * 64) {
+    const int col = idx / HD;
+    float sm[WHOLE_SPLITS], so[WHOLE_SPLITS], sl[WHOLE_SPLITS], top = -INFINITY;
+#pragma unroll
+    for (int sp = 0; sp < WHOLE_SPLITS; ++sp) {
+      sm[sp] = -INFINITY;
+      so[sp] = sl[sp] = 0.f;
+      if (sp < first || sp > last) continue;
+      float mx = -INFINITY;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) mx = fmaxf(mx, s_m[(sp * 4 + w) * 16 + col]);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float f = exp2f(s_m[(sp * 4 + w) * 16 + col] - mx);     // a wave without keys: weight 0
+        so[sp] += f * part[(sp * 4 + w) * G * HD + idx];
+        sl[sp] += f * s_l[(sp * 4 + w) * 16 + col];
+      }
+      sm[sp] = mx;
+      top = fmaxf(top, mx);
+    }
+    float acc = 0.f, den = 0.f;
+#pragma unroll
+    for (int sp = 0; sp < WHOLE_SPLITS; ++sp) {
+      if (sp < first || sp > last) continue;
+      const float f = exp2f(sm[sp] - top);
+      float a = f * so[sp], b = f * sl[sp];
+      asm volatile("" : "+v"(a), "+v"(b));        // (rounded before they are added)
+      acc += a;
+      den += b;
+    }
+    out_row[idx] = float_to_bf16(acc / den);
+  }
+}
+
+// The rounds of a wave, the first one's keys and values asked for; the next one's are asked for as
+// soon as the registers are free.  `own`: the position whose key and value are k_new and v_new (-1: none).
+template <int HD, bool PATCH, typename Keys, typename Values>
+__device__ __forceinline__ void whole_rounds(u32x4_t (&kf)[4][HD / 32], u32x2_t (&vf)[4][HD / 16],
+                                             const bf16x8_t (&qf)[HD / 32], int wave, int lo, int ctx,
+                                             int rounds, int j, int qd, int G, float scale_log2e, float* part,
+                                             Keys ask_keys, Values ask_values, int own, const bf16_t* k_new,
+                                             const bf16_t* v_new) {
+  for (int r = 0; r < rounds; ++r) {
+    const int kb = r * WHOLE_KEYS + wave * DEC_WAVE_KEYS, kn = kb + WHOLE_KEYS;
+    const int k_begin = max(lo, kb), k_end = min(ctx, kb + DEC_WAVE_KEYS);
+    const int n_begin = max(lo, kn), n_end = min(ctx, kn + DEC_WAVE_KEYS);
+    const bool here = k_begin < k_end, next = r + 1 < rounds && n_begin < n_end;
+    const int pn = own >= kb && own < kb + DEC_WAVE_KEYS ? own - kb : -1;
+    float m = -INFINITY, l = 0.f, sc[16];
+    f32x4_t o[HD / 16];
+#pragma unroll
+    for (int dt = 0; dt < HD / 16; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (here) decode_scores<HD, PATCH, 4>(kf, qf, kb, k_begin, k_end, qd, scale_log2e, m, l, sc, pn, k_new);
+    __builtin_amdgcn_sched_barrier(0);
+    if (next) ask_keys(kn, n_begin, n_end);
+    __builtin_amdgcn_sched_barrier(0);
+    if (here) decode_values<HD, PATCH, 4>(vf, sc, kb, k_begin, k_end, qd, o, pn, v_new);
+    __builtin_amdgcn_sched_barrier(0);
+    if (next) ask_values();
+    whole_put<HD>(part, G, rounds, r * WHOLE_WAVES + wave, j, qd, m, l, o);
+  }
+}
+
+template <int HD, bool WHOLE>
+__global__ __launch_bounds__(WHOLE ? 64 * WHOLE_WAVES : 256) void attn_decode_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pool,
     const bf16_t* __restrict__ v_pool, const int* __restrict__ block_table,
     const int* __restrict__ q_start, const int* __restrict__ ctx_len, float* __restrict__ ws_o,
     float* __restrict__ ws_ml, bf16_t* __restrict__ out, float scale_log2e, int window, int nH,
     int nKV, int ps, int max_pages, int max_splits) {
-  __shared__ __attribute__((aligned(16))) float s_o[4][16][HD];
-  __shared__ float s_m[4][16], s_l[4][16];
-  const int kvh = blockIdx.x, sp = blockIdx.y, s = blockIdx.z;
+  extern __shared__ __attribute__((aligned(16))) float whole[];
+  const int kvh = blockIdx.x, sp = WHOLE ? 0 : blockIdx.y, s = blockIdx.z;
   if (q_start[s + 1] - q_start[s] != 1) return;
   const int ctx = ctx_len[s], pos = ctx - 1;
   const int lo = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
-  if (max(lo, sp * DEC_SPLIT) >= min(ctx, (sp + 1) * DEC_SPLIT)) return;   // whole workgroup
+  if (!WHOLE && max(lo, sp * DEC_SPLIT) >= min(ctx, (sp + 1) * DEC_SPLIT)) return;   // whole workgroup
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, qd = lane / 16;
-  const int kb = sp * DEC_SPLIT + wave * DEC_WAVE_KEYS;
-  const int k_begin = max(lo, kb), k_end = min(ctx, kb + DEC_WAVE_KEYS);
   const int G = nH / nKV;
   const int t = q_start[s];
   const int* table = block_table + (size_t)s * max_pages;
-  float m = -INFINITY, l = 0.f;
-  f32x4_t o[HD / 16];
-#pragma unroll
-  for (int dt = 0; dt < HD / 16; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  if (k_begin < k_end) {
+  bf16x8_t qf[HD / 32];
+  u32x4_t kf[4][HD / 32];
+  u32x2_t vf[4][HD / 16];
+  const bf16_t* vg[4];
+  auto ask_keys = [&](int kb, int k_begin, int k_end) __attribute__((always_inline)) {
     // the four 16-key groups of this wave; a group outside [k_begin, k_end) may have no page
     // at all: it reads the group of a key that certainly exists and is masked
     const bf16_t* kg[4];
-    const bf16_t* vg[4];
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
       const int base = kb + 16 * h;
@@ -504,34 +599,58 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
       kg[h] = k_pool + blk + lane * 8;
       vg[h] = v_pool + blk + lane * 4;
     }
-    u32x4_t kf[4][HD / 32];
 #pragma unroll
     for (int h = 0; h < 4; ++h)
 #pragma unroll
       for (int stp = 0; stp < HD / 32; ++stp)
         kf[h][stp] = __builtin_nontemporal_load((const u32x4_t*)(kg[h] + stp * 512));
-    bf16x8_t qf[HD / 32];
-    {
-      const bf16_t* qrow = q + ((size_t)t * nH + kvh * G + min(j, G - 1)) * HD + 8 * qd;
+  };
+  auto ask_query = [&]() __attribute__((always_inline)) {
+    const bf16_t* qrow = q + ((size_t)t * nH + kvh * G + min(j, G - 1)) * HD + 8 * qd;
 #pragma unroll
-      for (int st = 0; st < HD / 32; ++st) {
-        u32x4_t v = *(const u32x4_t*)(qrow + st * 32);
-        if (j >= G) v = u32x4_t{0, 0, 0, 0};
-        qf[st] = *(bf16x8_t*)&v;
-      }
+    for (int st = 0; st < HD / 32; ++st) {
+      u32x4_t v = *(const u32x4_t*)(qrow + st * 32);
+      if (j >= G) v = u32x4_t{0, 0, 0, 0};
+      qf[st] = *(bf16x8_t*)&v;
     }
-    // values: lane (d % 16 = j, keys 4 qd .. 4 qd + 3) of head-element tile dt
-    u32x2_t vf[4][HD / 16];
+  };
+  // values: lane (d % 16 = j, keys 4 qd .. 4 qd + 3) of head-element tile dt
+  auto ask_values = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int h = 0; h < 4; ++h)
 #pragma unroll
       for (int dt = 0; dt < HD / 16; ++dt)
         vf[h][dt] = __builtin_nontemporal_load((const u32x2_t*)(vg[h] + dt * 256));
-    decode_attend<HD>(kf, vf, qf, kb, k_begin, k_end, qd, scale_log2e, m, l, o);
+  };
+  bf16_t* out_row = out + ((size_t)t * nH + kvh * G) * HD;
+  if constexpr (!WHOLE) {
+    __shared__ __attribute__((aligned(16))) float s_o[4][16][HD];
+    __shared__ float s_m[4][16], s_l[4][16];
+    const int kb = sp * DEC_SPLIT + wave * DEC_WAVE_KEYS;
+    const int k_begin = max(lo, kb), k_end = min(ctx, kb + DEC_WAVE_KEYS);
+    float m = -INFINITY, l = 0.f;
+    f32x4_t o[HD / 16];
+#pragma unroll
+    for (int dt = 0; dt < HD / 16; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (k_begin < k_end) {
+      ask_keys(kb, k_begin, k_end);
+      ask_query();
+      ask_values();
+      decode_attend<HD>(kf, vf, qf, kb, k_begin, k_end, qd, scale_log2e, m, l, o);
+    }
+    decode_write_partial<HD>(s_o, s_m, s_l, wave, j, qd, m, l, o, G,
+                             ((size_t)s * nH + kvh * G) * max_splits + sp, max_splits, ws_o, ws_ml, out_row);
+  } else {
+    const int rounds = (max_splits + 1) / 2;
+    const bool keys_0 = max(lo, wave * DEC_WAVE_KEYS) < min(ctx, wave * DEC_WAVE_KEYS + DEC_WAVE_KEYS);
+    if (keys_0) ask_keys(wave * DEC_WAVE_KEYS, max(lo, wave * DEC_WAVE_KEYS), min(ctx, wave * DEC_WAVE_KEYS + DEC_WAVE_KEYS));
+    ask_query();
+    if (keys_0) ask_values();
+    whole_rounds<HD, false>(kf, vf, qf, wave, lo, ctx, rounds, j, qd, G, scale_log2e, whole, ask_keys, ask_values,
+                            -1, nullptr, nullptr);
+    __syncthreads();
+    whole_combine<HD>(whole, G, rounds, lo, ctx, out_row);
   }
-  decode_write_partial<HD>(s_o, s_m, s_l, wave, j, qd, m, l, o, G,
-                           ((size_t)s * nH + kvh * G) * max_splits + sp, max_splits, ws_o, ws_ml,
-                           out + ((size_t)t * nH + kvh * G) * HD);
 }
 
 // What the fused decode kernel needs to do the work of the kernel before it as well (the
@@ -567,24 +686,23 @@ struct DecodeFused {
 // The page of a 16-key group is the same for a whole wave, so the look-ups and the blocks'
 // addresses are scalar and a load's address is one of them plus a lane's offset: the loads
 // hold no address registers, which leaves room for what the norm holds meanwhile.
-template <int HD>
-__global__ __launch_bounds__(256, HD <= 128 ? 3 : 1) void attn_decode_fused_kernel(
+template <int HD, bool WHOLE>
+__global__ __launch_bounds__(WHOLE ? 64 * WHOLE_WAVES : 256, WHOLE ? 2 : HD <= 128 ? 3 : 1) void attn_decode_fused_kernel(
     const bf16_t* __restrict__ qkv, bf16_t* __restrict__ k_pool, bf16_t* __restrict__ v_pool,
     const int* __restrict__ block_table, const int* __restrict__ ctx_len,
     float* __restrict__ ws_o, float* __restrict__ ws_ml, bf16_t* __restrict__ out,
     float scale_log2e, int window, int nH, int nKV, int ps, int max_pages, int max_splits,
     DecodeFused fu) {
-  __shared__ __attribute__((aligned(16))) float s_o[4][16][HD];
-  __shared__ float s_m[4][16], s_l[4][16];
+  extern __shared__ __attribute__((aligned(16))) float whole[];
   // rows 0 .. G - 1: the query heads; row 16: the new key; row 17: the new value
   __shared__ __attribute__((aligned(16))) bf16_t s_q[18][HD + 8];
-  const int kvh = blockIdx.x, sp = blockIdx.y, s = blockIdx.z;
+  const int kvh = blockIdx.x, sp = WHOLE ? 0 : blockIdx.y, s = blockIdx.z;
   const int ctx = ctx_len[s], pos = ctx - 1;
   const int slot = fu.slot_mapping[s];
   // (a position beyond the tables reads their last row: wrong, but no access out of bounds)
   const int rope_pos = fu.cos_t ? min(max(fu.positions[s], 0), fu.table_rows - 1) : 0;
   const int lo = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
-  if (max(lo, sp * DEC_SPLIT) >= min(ctx, (sp + 1) * DEC_SPLIT)) return;   // whole workgroup
+  if (!WHOLE && max(lo, sp * DEC_SPLIT) >= min(ctx, (sp + 1) * DEC_SPLIT)) return;   // whole workgroup
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int lane = threadIdx.x % 64, j = lane % 16, qd = lane / 16;
   const int kb = sp * DEC_SPLIT + wave * DEC_WAVE_KEYS;
@@ -596,10 +714,10 @@ __global__ __launch_bounds__(256, HD <= 128 ? 3 : 1) void attn_decode_fused_kern
   // LPH lanes to a head, 8 elements each; the workgroup takes HEADS heads at a time.  Item
   // i < G is query head kvh * G + i, item G the new key (where the split holds the token's
   // own position).
-  constexpr int LPH = HD / 8, HEADS = 256 / LPH;
-  constexpr int V_EARLY = HD == 128 ? 2 : 4;      // groups whose values are asked for with the keys
+  constexpr int LPH = HD / 8, HEADS = (WHOLE ? 64 * WHOLE_WAVES : 256) / LPH;
+  constexpr int V_EARLY = HD == 128 && !WHOLE ? 2 : 4;      // groups whose values are asked for with the keys
   const int li = threadIdx.x % LPH;
-  const bool own = pos / DEC_SPLIT == sp;
+  const bool own = WHOLE || pos / DEC_SPLIT == sp;
   const int items = own ? G + 1 : G;
   const int row_width = (nH + 2 * nKV) * HD;
   const bf16_t* row = qkv + (size_t)s * row_width;
@@ -626,7 +744,7 @@ __global__ __launch_bounds__(256, HD <= 128 ? 3 : 1) void attn_decode_fused_kern
   u32x4_t kf[4][HD / 32];
   u32x2_t vf[4][HD / 16];
   size_t blk[4] = {0, 0, 0, 0};
-  if (has_keys) {
+  auto ask_keys = [&](int kb, int k_begin, int k_end) __attribute__((always_inline)) {
     // the four 16-key groups of this wave; a group outside [k_begin, k_end) may have no page
     // at all: it reads the group of a key that certainly exists and is masked
     // (the four look-ups are scalar loads: asked for together, waited for once)
@@ -648,12 +766,18 @@ __global__ __launch_bounds__(256, HD <= 128 ? 3 : 1) void attn_decode_fused_kern
       for (int stp = 0; stp < HD / 32; ++stp)
         kf[h][stp] = __builtin_nontemporal_load(
             (const u32x4_t*)(k_pool + blk[h] + stp * 512) + lane);
+  };
+  auto ask_values = [&](int from, int to) __attribute__((always_inline)) {
 #pragma unroll
-    for (int h = 0; h < V_EARLY; ++h)
+    for (int h = from; h < to; ++h)
 #pragma unroll
       for (int dt = 0; dt < HD / 16; ++dt)
         vf[h][dt] = __builtin_nontemporal_load(
             (const u32x2_t*)(v_pool + blk[h] + dt * 256) + lane);
+  };
+  if (has_keys) {
+    ask_keys(kb, k_begin, k_end);
+    ask_values(0, V_EARLY);
   }
   // (nothing below may move above the loads, and none of them below it)
   __builtin_amdgcn_sched_barrier(0);
@@ -701,36 +825,43 @@ __global__ __launch_bounds__(256, HD <= 128 ? 3 : 1) void attn_decode_fused_kern
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  if (has_keys) {
-#pragma unroll
-    for (int h = V_EARLY; h < 4; ++h)
-#pragma unroll
-      for (int dt = 0; dt < HD / 16; ++dt)
-        vf[h][dt] = __builtin_nontemporal_load(
-            (const u32x2_t*)(v_pool + blk[h] + dt * 256) + lane);
-  }
+  if (has_keys) ask_values(V_EARLY, 4);
   __builtin_amdgcn_sched_barrier(0);
   __syncthreads();
 
-  float m = -INFINITY, l = 0.f;
-  f32x4_t o[HD / 16];
-#pragma unroll
-  for (int dt = 0; dt < HD / 16; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  if (has_keys) {
-    bf16x8_t qf[HD / 32];
+  bf16x8_t qf[HD / 32];
+  auto read_query = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int st = 0; st < HD / 32; ++st) {
       u32x4_t v = *(const u32x4_t*)(s_q[min(j, G - 1)] + st * 32 + 8 * qd);
       if (j >= G) v = u32x4_t{0, 0, 0, 0};
       qf[st] = *(bf16x8_t*)&v;
     }
-    const int pn = (pos >= kb && pos < kb + DEC_WAVE_KEYS) ? pos - kb : -1;
-    decode_attend<HD, true>(kf, vf, qf, kb, k_begin, k_end, qd, scale_log2e, m, l, o, pn,
-                            s_q[16], s_q[17]);
+  };
+  bf16_t* out_row = out + ((size_t)s * nH + kvh * G) * HD;
+  if constexpr (!WHOLE) {
+    __shared__ __attribute__((aligned(16))) float s_o[4][16][HD];
+    __shared__ float s_m[4][16], s_l[4][16];
+    float m = -INFINITY, l = 0.f;
+    f32x4_t o[HD / 16];
+#pragma unroll
+    for (int dt = 0; dt < HD / 16; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (has_keys) {
+      read_query();
+      const int pn = (pos >= kb && pos < kb + DEC_WAVE_KEYS) ? pos - kb : -1;
+      decode_attend<HD, true>(kf, vf, qf, kb, k_begin, k_end, qd, scale_log2e, m, l, o, pn,
+                              s_q[16], s_q[17]);
+    }
+    decode_write_partial<HD>(s_o, s_m, s_l, wave, j, qd, m, l, o, G,
+                             ((size_t)s * nH + kvh * G) * max_splits + sp, max_splits, ws_o, ws_ml, out_row);
+  } else {
+    const int rounds = (max_splits + 1) / 2;
+    read_query();
+    whole_rounds<HD, true>(kf, vf, qf, wave, lo, ctx, rounds, j, qd, G, scale_log2e, whole, ask_keys,
+                           [&]() __attribute__((always_inline)) { ask_values(0, 4); }, pos, s_q[16], s_q[17]);
+    __syncthreads();
+    whole_combine<HD>(whole, G, rounds, lo, ctx, out_row);
   }
-  decode_write_partial<HD>(s_o, s_m, s_l, wave, j, qd, m, l, o, G,
-                           ((size_t)s * nH + kvh * G) * max_splits + sp, max_splits, ws_o, ws_ml,
-                           out + ((size_t)s * nH + kvh * G) * HD);
 }
 
 // Combines the splits of one (sequence, head) and writes bfloat16.  One workgroup of 4 waves.
@@ -826,6 +957,25 @@ static int launch_decode_merge(const float* ws_o, const float* ws_ml, const int*
   ZF_CHECK_LAUNCH();
 }
 
+// Tables of 257 to 1024 keys, head size 128: one workgroup a sequence and kv head.  Measured over 32 heads
+// on 8, both kernels before, us: 24 sequences with tables of 1024 keys and contexts of 150 to 296, 343 to
+// 640, 525 to 976 16.4 -> 10.2, 18.8 -> 15.1, 20.1 -> 19.9; 64 32.9 -> 18.7, 38.6 -> 29.7, 43.5 -> 42.6; 128
+// 58.4 -> 34.7, 70.2 -> 52.3, 82.3 -> 80.0; 40 and 64 heads alike.  With 128 workgroups the longest
+// contexts lose (16 sequences 17.2 -> 19.0, 8 12.6 -> 18.7), and with two heads a kv head, whose partials are
+// little work to merge (64 sequences of 16 heads 40.6 -> 42.2).
+#define ZF_SET_LDS(KERNEL, BYTES)                                                               \
+  do {                                                                                          \
+    if ((BYTES) > 48 * 1024) {                                                                  \
+      const hipError_t e_ = hipFuncSetAttribute(                                                \
+          (const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(BYTES));       \
+      if (e_ != hipSuccess) return (int)e_;                                                     \
+    }                                                                                           \
+  } while (0)
+static bool decode_takes_whole(int n_seqs, int nH, int nKV, int hd, int max_splits) {
+  return hd == 128 && max_splits > 1 && max_splits <= WHOLE_SPLITS && (long long)n_seqs * nKV >= 192 &&
+         nH / nKV >= 4;
+}
+
 extern "C" int zf_attn_decode_bf16(const void* q, const void* k_pool, const void* v_pool,
                                    const int* block_table, const int* q_start,
                                    const int* ctx_len, void* out, float* ws_o, float* ws_ml,
@@ -835,18 +985,25 @@ extern "C" int zf_attn_decode_bf16(const void* q, const void* k_pool, const void
   if (n_seqs <= 0) return 0;
   if (page_size % 16 != 0 || nKV <= 0 || nH % nKV != 0 || nH / nKV > 16) return -2;
   const float scale_log2e = scale * 1.4426950408889634f;
-  dim3 grid(nKV, max_splits, n_seqs);
-#define ZF_DEC(HD)                                                                              \
-  hipLaunchKernelGGL(attn_decode_kernel<HD>, grid, dim3(256), 0, stream, (const bf16_t*)q,      \
-                     (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_table, q_start,        \
-                     ctx_len, ws_o, ws_ml, (bf16_t*)out, scale_log2e, window, nH, nKV,          \
-                     page_size, max_pages, max_splits)
+#define ZF_DEC_AS(HD, WHOLE, GRID, THREADS, LDS)                                                \
+  hipLaunchKernelGGL((attn_decode_kernel<HD, WHOLE>), GRID, dim3(THREADS), LDS, stream,         \
+                     (const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)v_pool,            \
+                     block_table, q_start, ctx_len, ws_o, ws_ml, (bf16_t*)out, scale_log2e,     \
+                     window, nH, nKV, page_size, max_pages, max_splits)
+#define ZF_DEC(HD) ZF_DEC_AS(HD, false, dim3(nKV, max_splits, n_seqs), 256, 0)
+  if (decode_takes_whole(n_seqs, nH, nKV, hd, max_splits)) {
+    const size_t lds = whole_floats<128>(nH / nKV, (max_splits + 1) / 2) * 4;
+    ZF_SET_LDS((attn_decode_kernel<128, true>), lds);
+    ZF_DEC_AS(128, true, dim3(nKV, 1, n_seqs), 64 * WHOLE_WAVES, lds);
+    ZF_CHECK_LAUNCH();
+  }
   if (hd == 32) ZF_DEC(32);
   else if (hd == 64) ZF_DEC(64);
   else if (hd == 128) ZF_DEC(128);
   else if (hd == 256) ZF_DEC(256);
   else return -2;
 #undef ZF_DEC
+#undef ZF_DEC_AS
   return launch_decode_merge(ws_o, ws_ml, q_start, ctx_len, out, window, n_seqs, nH, hd,
                              max_splits, stream);
 }
@@ -875,18 +1032,25 @@ extern "C" int zf_attn_decode_fused_bf16(const void* qkv, const float* q_gain,
     return -2;
   const DecodeFused fu{q_gain, k_gain, eps, cos_t, sin_t, positions, slot_mapping, table_rows};
   const float scale_log2e = scale * 1.4426950408889634f;
-  dim3 grid(nKV, max_splits, n_seqs);
-#define ZF_DEC(HD)                                                                              \
-  hipLaunchKernelGGL(attn_decode_fused_kernel<HD>, grid, dim3(256), 0, stream,                  \
+#define ZF_DEC_AS(HD, WHOLE, GRID, THREADS, LDS)                                                \
+  hipLaunchKernelGGL((attn_decode_fused_kernel<HD, WHOLE>), GRID, dim3(THREADS), LDS, stream,   \
                      (const bf16_t*)qkv, (bf16_t*)k_pool, (bf16_t*)v_pool, block_table,         \
                      ctx_len, ws_o, ws_ml, (bf16_t*)out, scale_log2e, window, nH, nKV,          \
                      page_size, max_pages, max_splits, fu)
+#define ZF_DEC(HD) ZF_DEC_AS(HD, false, dim3(nKV, max_splits, n_seqs), 256, 0)
+  if (decode_takes_whole(n_seqs, nH, nKV, hd, max_splits)) {
+    const size_t lds = whole_floats<128>(nH / nKV, (max_splits + 1) / 2) * 4;
+    ZF_SET_LDS((attn_decode_fused_kernel<128, true>), lds);
+    ZF_DEC_AS(128, true, dim3(nKV, 1, n_seqs), 64 * WHOLE_WAVES, lds);
+    ZF_CHECK_LAUNCH();
+  }
   if (hd == 32) ZF_DEC(32);
   else if (hd == 64) ZF_DEC(64);
   else if (hd == 128) ZF_DEC(128);
   else if (hd == 256) ZF_DEC(256);
   else return -2;
 #undef ZF_DEC
+#undef ZF_DEC_AS
   return launch_decode_merge(ws_o, ws_ml, q_start, ctx_len, out, window, n_seqs, nH, hd,
                              max_splits, stream);
 }
