@@ -37,6 +37,36 @@ def _starts(lens):
     return out
 
 
+# ------------------------------------------------------------------------------ norms of the same rows
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("T,W,K", [(1, 4, 64), (3, 1020, 0), (16, 2048, 7168), (16, 2048, 0), (2, 2052, 0),
+                                   (5, 4096, 0), (2, 8192, 0), (9, 512, 6144), (1, 1024, 7168)])
+def test_norms_of_rows_are_the_sum_and_the_norms_one_after_the_other(T, W, K, dt):
+    """The bits of ``gemm`` added into the stream and of ``norm_rows``, where a product runs split along K
+    (K > 64) and without one; one norm and two, with biases and without, centred or not."""
+    x = _rand((T, W), 1).to(DEV)
+    gains = [_rand((W,), 2 + i, 0.2).to(DEV) + 1.0 for i in range(2)]
+    biases = [_rand((W,), 4, 0.1).to(DEV), None]
+    product = None
+    if K > 64:
+        a = _rand((T, K), 5, 1.0, torch.bfloat16).to(DEV)
+        product = (a, ops.pretile_weight(_rand((W, K), 6, 0.02, torch.bfloat16).to(DEV)))
+        assert ops.stream_parts_plan(T, W, K, product[1], True) is not None
+    for centred in (False, True):
+        for n in (1, 2):
+            norms = [(gains[i], biases[i], 1e-6 * (1 + 9 * i)) for i in range(n)]
+            want_x, got_x = x.clone(), x.clone()
+            if product:
+                ops.gemm(*product, want_x, accumulate=True, w_tiled=True)
+            want = [torch.empty((T, W), dtype=dt, device=DEV) for _ in range(n)]
+            got = [torch.empty_like(w) for w in want]
+            for (g, b, eps), w in zip(norms, want):
+                ops.norm_rows(want_x, g, b, eps, w, centred)
+            ops.norms_of_rows(got_x, norms, got, centred, ops.stream_parts(*product) if product else None)
+            assert torch.equal(got_x, want_x)
+            assert all(torch.equal(g, w) for g, w in zip(got, want))
+
+
 # ------------------------------------------------------------------------------ embedding
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("W", [6, 50, 51, 320])

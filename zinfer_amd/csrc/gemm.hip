@@ -2563,18 +2563,20 @@ extern "C" int zf_gemm_bf16_skinny_sum_norm(const void* A, const void* W, void* 
 
 // rg: row groups of 16 per workgroup (1, 2 or 4); ksplit: workgroups along K (1..16), which
 // needs a float32 workspace of ksplit * M * N elements when > 1; w_tiled: W is pre-tiled
-// (N % 16 == 0, K % 64 == 0, N a multiple of 16 * rg).
+// (N % 16 == 0, K % 64 == 0, N a multiple of 16 * rg).  keep_parts: ws keeps the parts
+// [ksplit, M, N] for a kernel of the caller's that adds them.
 extern "C" int zf_gemm_bf16_skinny(const void* A, const void* W, void* C, void* ws, int M, int N,
                                    int K, int epi, int rg, int ksplit, int w_tiled,
-                                   hipStream_t stream) {
+                                   int keep_parts, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K % 8 != 0 || M > 64 || ksplit < 1 || ksplit > 16 || (ksplit > 1 && ws == nullptr))
     return -3;
+  if (keep_parts && (ksplit < 2 || epi != EPI_STORE_F32)) return -3;
   const int mt = (M + 15) / 16;
   if (w_tiled && (N % (16 * rg) != 0 || K % 64 != 0)) return -3;
 #define ZF_SK(MT, RG)                                                                         \
-  return w_tiled ? launch_skinny<MT, RG, true>(A, W, C, ws, M, N, K, epi, ksplit, stream)     \
-                 : launch_skinny<MT, RG, false>(A, W, C, ws, M, N, K, epi, ksplit, stream)
+  return w_tiled ? launch_skinny<MT, RG, true>(A, W, C, ws, M, N, K, epi, ksplit, stream, SkinnyNorm{}, !keep_parts) \
+                 : launch_skinny<MT, RG, false>(A, W, C, ws, M, N, K, epi, ksplit, stream, SkinnyNorm{}, !keep_parts)
   if (rg == 1) { if (mt == 1) ZF_SK(1, 1); if (mt == 2) ZF_SK(2, 1); if (mt == 3) ZF_SK(3, 1); ZF_SK(4, 1); }
   if (rg == 2) { if (mt == 1) ZF_SK(1, 2); if (mt == 2) ZF_SK(2, 2); if (mt == 3) ZF_SK(3, 2); ZF_SK(4, 2); }
   if (rg == 4) { if (mt == 1) ZF_SK(1, 4); if (mt == 2) ZF_SK(2, 4); if (mt == 3) ZF_SK(3, 4); ZF_SK(4, 4); }

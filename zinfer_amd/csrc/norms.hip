@@ -143,6 +143,101 @@ extern "C" int zf_norm_rows(const float* x, const float* x_bias, const float* ga
   ZF_CHECK_LAUNCH();
 }
 
+// ---------------------------------------------------------------- norms that read the same rows
+// out_a = norm_a(x) and out_b = norm_b(x) (out_b null: the first alone), each as norm_rows gives it, the
+// row and its sums read and formed once; with parts [ksplit, T, W] of a product that ends in the
+// stream x += their sum first, added in their order.  A decode step's rows are few and its launches
+// bound it: a block of 2048 columns whose two sublayers read the same 16 rows ran a kernel that adds
+// the parts and a kernel a norm (4.2 + 3.3 + 3.5 us), 4.7 here.  NV groups of four
+// columns a thread (256 NV * 4 >= W).
+template <typename TO, int NV>
+__global__ __launch_bounds__(256) void sum_norms_kernel(
+    float* __restrict__ x, const float* __restrict__ parts, int ksplit, const float* __restrict__ gain_a,
+    const float* __restrict__ bias_a, float eps_a, TO* __restrict__ out_a, const float* __restrict__ gain_b,
+    const float* __restrict__ bias_b, float eps_b, TO* __restrict__ out_b, int W, int centred) {
+  __shared__ float red[16];
+  const size_t at = (size_t)blockIdx.x * W, stride = (size_t)gridDim.x * W;
+  const int n4 = W / 4;
+  float4* row = (float4*)(x + at);
+  float4 v[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = threadIdx.x + i * 256;
+    v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (c < n4) {
+      const float4 old = row[c];
+      if (ksplit > 0) {
+        float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+        for (int k = 0; k < ksplit; ++k) {
+          const float4 p = ((const float4*)(parts + k * stride + at))[c];
+          s.x += p.x; s.y += p.y; s.z += p.z; s.w += p.w;
+        }
+        v[i] = make_float4(old.x + s.x, old.y + s.y, old.z + s.z, old.w + s.w);
+        row[c] = v[i];
+      } else {
+        v[i] = old;
+      }
+    }
+  }
+  float mean = 0.f;
+  if (centred) {
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+    mean = block_sum(s, red) / (float)W;
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = threadIdx.x + i * 256;
+    if (c < n4) {
+      v[i].x -= mean; v[i].y -= mean; v[i].z -= mean; v[i].w -= mean;
+      ss += v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w;
+    }
+  }
+  ss = block_sum(ss, red);
+  auto store = [&](const float* gain, const float* bias, float eps, TO* out) {
+    const float inv = 1.0f / sqrtf(ss / (float)W + eps);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = threadIdx.x + i * 256;
+      if (c < n4) {
+        const float4 g = ((const float4*)gain)[c];
+        float4 b = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (bias != nullptr) b = ((const float4*)bias)[c];
+        norm_store4<TO>(out + at + 4 * c, make_float4(v[i].x * inv * g.x + b.x, v[i].y * inv * g.y + b.y,
+                                                      v[i].z * inv * g.z + b.z, v[i].w * inv * g.w + b.w));
+      }
+    }
+  };
+  store(gain_a, bias_a, eps_a, out_a);
+  if (out_b != nullptr) store(gain_b, bias_b, eps_b, out_b);
+}
+
+// ksplit 0: no parts.  W a multiple of 4 up to 8192; parts, rows, gains and biases 16-byte aligned.
+extern "C" int zf_sum_norms(float* x, const float* parts, int ksplit, const float* gain_a,
+                            const float* bias_a, float eps_a, void* out_a, const float* gain_b,
+                            const float* bias_b, float eps_b, void* out_b, int out_dtype, int T, int W,
+                            int centred, hipStream_t stream) {
+  if (T <= 0) return 0;
+  if (W <= 0 || W % 4 != 0 || W > 8192 || ksplit < 0 || (ksplit > 0 && parts == nullptr)) return -2;
+#define ZF_SUM_NORMS(TO, NV)                                                                              \
+  hipLaunchKernelGGL((sum_norms_kernel<TO, NV>), dim3(T), dim3(256), 0, stream, x, parts, ksplit, gain_a, \
+                     bias_a, eps_a, (TO*)out_a, gain_b, bias_b, eps_b, (TO*)out_b, W, centred)
+  if (out_dtype == ZF_F32) {
+    if (W <= 2048) ZF_SUM_NORMS(float, 2);
+    else if (W <= 4096) ZF_SUM_NORMS(float, 4);
+    else ZF_SUM_NORMS(float, 8);
+  } else {
+    if (W <= 2048) ZF_SUM_NORMS(bf16_t, 2);
+    else if (W <= 4096) ZF_SUM_NORMS(bf16_t, 4);
+    else ZF_SUM_NORMS(bf16_t, 8);
+  }
+#undef ZF_SUM_NORMS
+  ZF_CHECK_LAUNCH();
+}
+
 // ---------------------------------------------------------------- a norm behind a sublayer and the one before the next
 // x += norm_a(y + y_bias); out = norm_b(x): the norm that closes a sublayer adds its result into the
 // residual stream, and the norm that opens the next sublayer reads the sum while the row is

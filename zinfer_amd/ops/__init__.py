@@ -1026,7 +1026,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
             rg, ks = plan[1:] if plan is not None else _stream_plan(M, N, K, w_tiled)
             ws = _workspace("gemm_splitk", ks * M * N, torch.float32, a.device) if ks > 1 else None
             _check(lib.zf_gemm_bf16_skinny(_ptr(a), _ptr(w), _ptr(out), _ptr(ws), M, N, K, epi,
-                                           rg, ks, 1 if w_tiled else 0, _stream()),
+                                           rg, ks, 1 if w_tiled else 0, 0, _stream()),
                    "gemm (weight streaming)")
         elif w_tiled and _tile64_covers(M, N, K, accumulate):
             _check(lib.zf_gemm_bf16_mid(_ptr(a), _ptr(w), _ptr(out), _ptr(None), M, N, K, epi, 1,
@@ -1159,6 +1159,37 @@ def gemm_partials(a: torch.Tensor, w: torch.Tensor, ksplit: int) -> torch.Tensor
 
 
 gemm_partials.kernel_class = "products"     # (it hands its work buffer on even when left out)
+
+
+def stream_parts_plan(M: int, N: int, K: int, w: torch.Tensor, w_tiled: bool):
+    """(row groups, workgroups along K) if ``gemm`` would run a w^T of up to 16 rows as a weight-streaming
+    product split along K, whose parts a kernel of the caller's can add instead (``stream_parts``)."""
+    if not (w_tiled and w.dtype == torch.bfloat16 and w.is_cuda and 0 < M <= 16):
+        return None
+    rg, ks = _stream_plan(M, N, K, True)
+    return (rg, ks) if ks > 1 else None
+
+
+@_launches("products")
+def _run_stream_parts(a, w, ws, M, N, K, rg, ks) -> None:
+    lib = build.load("gemm")
+    _check(lib.zf_gemm_bf16_skinny(_ptr(a), _ptr(w), _ptr(ws), _ptr(ws), M, N, K, _EPI_STORE_F32, rg, ks,
+                                   1, 1, _stream()), "stream_parts")
+
+
+def stream_parts(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """The float32 parts [k, M, N] of a w^T in a work buffer that the next split product overwrites;
+    added in their order they are what ``gemm`` adds."""
+    _need_gpu(a, w)
+    M, K = a.shape
+    N = w.shape[0]
+    plan = stream_parts_plan(M, N, K, w, True)
+    if plan is None or a.dtype != torch.bfloat16 or w.shape[1] != K or not can_pretile(w) \
+            or not a.is_contiguous():
+        raise KernelUnavailable(f"stream_parts: a {tuple(a.shape)} {a.dtype}, w {tuple(w.shape)}")
+    ws = _workspace("gemm_splitk", plan[1] * M * N, torch.float32, a.device)
+    _run_stream_parts(a, w, ws, M, N, K, *plan)
+    return ws[:plan[1] * M * N].view(plan[1], M, N)
 
 
 def norm_gemm_plan(M: int, N: int, K: int, w: torch.Tensor, w_tiled: bool):
@@ -1481,7 +1512,7 @@ def gemm_swiglu(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled: bo
     elif M <= SKINNY_MAX_M:
         rg = plan[1] if plan is not None else 2
         _check(lib.zf_gemm_bf16_skinny(_ptr(a), _ptr(w), _ptr(out), _ptr(None), M, N, K,
-                                       _EPI_SWIGLU, rg, 1, 1 if w_tiled else 0, _stream()),
+                                       _EPI_SWIGLU, rg, 1, 1 if w_tiled else 0, 0, _stream()),
                "gemm_swiglu (weight streaming)")
     else:
         big = _tile256_variant(M, N, K) if w_tiled else None
@@ -1751,6 +1782,31 @@ def norm_rows(x: torch.Tensor, gain: torch.Tensor, bias: Optional[torch.Tensor],
     _check(lib.zf_norm_rows(_ptr(x), _ptr(x_bias), _ptr(gain), _ptr(bias), _ptr(out), _dt(out), T,
                             W, ctypes.c_float(eps), 1 if centred else 0, 1 if add else 0,
                             _stream()), "norm_rows")
+
+
+@_launches("norm_rope_write")
+def norms_of_rows(x: torch.Tensor, norms, outs, centred: bool, parts: Optional[torch.Tensor] = None) -> None:
+    """outs[i] = norm i of the rows of float32 ``x`` [T, W] for one or two ``norms`` (gain, bias or None,
+    eps), all in one kernel, each the bits of ``norm_rows``; with ``parts`` float32 [k, T, W] x += their
+    sum first.  Widths of ``norm_add_norm_covers``."""
+    T, W = x.shape
+    _need_gpu(x, parts, *outs, *(t for n in norms for t in n[:2]))
+    if not 1 <= len(norms) == len(outs) <= 2 or not norm_add_norm_covers(W) or x.dtype != torch.float32 \
+            or any(g.dtype != torch.float32 or g.shape != (W,)
+                   or (b is not None and (b.dtype != torch.float32 or b.shape != (W,)))
+                   for g, b, _ in norms) \
+            or any(o.shape != x.shape or o.dtype != outs[0].dtype or not o.is_contiguous() for o in outs) \
+            or not x.is_contiguous() \
+            or (parts is not None and (parts.dtype != torch.float32 or parts.shape[1:] != x.shape
+                                       or not parts.is_contiguous())):
+        raise KernelUnavailable(f"norms_of_rows: x {tuple(x.shape)} {x.dtype}, outputs "
+                                f"{[(tuple(o.shape), o.dtype) for o in outs]}")
+    (ga, ba, ea), (gb, bb, eb) = norms[0], norms[1] if len(norms) > 1 else (None, None, 0.0)
+    lib = build.load("norms")
+    _check(lib.zf_sum_norms(_ptr(x), _ptr(parts), 0 if parts is None else parts.shape[0], _ptr(ga),
+                            _ptr(ba), ctypes.c_float(ea), _ptr(outs[0]), _ptr(gb), _ptr(bb),
+                            ctypes.c_float(eb), _ptr(outs[1]) if len(outs) > 1 else None, _dt(outs[0]),
+                            T, W, 1 if centred else 0, _stream()), "norms_of_rows")
 
 
 NORM_ADD_NORM_MAX_WIDTH = 8192

@@ -17,7 +17,7 @@ from . import (concat_rows, decay_recurrence, embed_sinusoid, head_norm_gate, to
 from . import gemm_many
 from . import (activation, head_products, masked_attention, masked_attention_mfma,
                norm_add_store, project_rows)
-from . import (embed_position, kv_rows_write, moe_down, moe_gate_up, moe_route, norm_rows,
+from . import (embed_position, kv_rows_write, moe_down, moe_gate_up, moe_route, norm_rows, norms_of_rows,
                shared_kv_attention)
 from . import (advance_decode, apply_penalties, argmax, argmax_no_alloc, cast, check_tables,
                decode_attention_fused, embed, gather_rows, gemm, gemm_emit, gemm_given,
@@ -78,6 +78,8 @@ KERNELS: Dict[str, KernelEntry] = {
                                "own: the read stream bandwidths are measured against"),
     "norm_rows": KernelEntry(norm_rows, "norms", "own: layer norm / RMS norm with a bias, stored "
                              "or added to the stream"),
+    "norms_of_rows": KernelEntry(norms_of_rows, "norms", "own: two norms of the same rows, behind the "
+                                 "sum of a split product's parts"),
     "norm_add_norm": KernelEntry(norm_add_norm, "norms", "own: the norm behind a sublayer, the "
                                  "residual sum and the norm before the next sublayer"),
     "embed_position": KernelEntry(embed_position, "norms", "own: embedding plus a learned "

@@ -9,6 +9,7 @@ from ..config.specs import (ParallelBlockSpec, PostNormBlockSpec, PreNormBlockSp
 from ..errors import ConfigError
 from .base import Block, TensorDecl, build_part, register_part
 from .linear import Linear, place_gain, place_matrix
+from .norm import LayerNorm, NormedRows, RowNorms
 
 
 class PreNormBlock(Block):
@@ -169,17 +170,6 @@ class SandwichNormBlock(Block):
         step.norm_ready = NormedRows(after_block, x, h) if h is not None else None
 
 
-class NormedRows:
-    """The rows ``normed`` = ``norm(x)`` that a block's last kernel already made for the norm
-    that reads the stream next."""
-
-    def __init__(self, norm, x: torch.Tensor, normed: torch.Tensor):
-        self.norm, self.x, self.normed = norm, x, normed
-
-    def fits(self, norm, x: torch.Tensor) -> bool:
-        return self.norm is norm and self.x.data_ptr() == x.data_ptr() and self.x.shape == x.shape
-
-
 class StreamRows:
     """The residual rows ``x`` in the activations' type, left by the kernel that last added
     into them for a sublayer that reads the stream as it is."""
@@ -307,6 +297,7 @@ class ParallelBlock(Block):
         self.joinable = self.feed_forward is not None and self.ff_norm is None \
             and self.mixer.joins and self.feed_forward.joins
         self.joined = None
+        self.row_norms = None           # both sublayers' norms in one kernel, where they allow it
         # the norm that reads the stream first, if what a sum leaves for it is of use
         self.entry_norm = self.mixer_norm if self.joinable and self.mixer_norm.defers else None
         self.graph_safe = all(p.graph_safe for p in self.parts)
@@ -328,7 +319,9 @@ class ParallelBlock(Block):
             else:
                 part.bind(tensors)
         if not joined:
-            self.entry_norm = None
+            self.row_norms = RowNorms.of(*(n for n in (self.mixer_norm, self.ff_norm) if n is not None)) \
+                if torch.device(self.ctx.device).type == "cuda" else None
+            self.entry_norm = self.row_norms
 
     def cache_need(self):
         return self.mixer.cache_need()
@@ -361,16 +354,31 @@ class ParallelBlock(Block):
         if self.joined is not None:
             self._forward_joined(x, step, cache)
             return
+        left, after = step.norm_ready, step.norm_after_block
         step.norm_ready = step.norm_after = None
-        h1 = self.mixer_norm.forward(x, step.scratch("normed", x.shape, self.ctx.act_dtype))
-        h2 = h1
-        if self.ff_norm is not None:
-            # (before the mixer adds into the stream: both sublayers read the same rows)
-            h2 = self.ff_norm.forward(x, step.scratch("normed_ff", x.shape, self.ctx.act_dtype))
+        if self.row_norms is not None:
+            hs = left.normed if isinstance(left, NormedRows) and left.fits(self.row_norms.norms, x) \
+                else self.row_norms.forward(x, step)
+            h1, h2 = hs[0], hs[-1]
+        else:
+            h1 = self.mixer_norm.forward(x, step.scratch("normed", x.shape, self.ctx.act_dtype))
+            h2 = h1
+            if self.ff_norm is not None:
+                # (before the mixer adds into the stream: both sublayers read the same rows)
+                h2 = self.ff_norm.forward(x, step.scratch("normed_ff", x.shape, self.ctx.act_dtype))
+        closing = None
+        if isinstance(after, LayerNorm):        # (the final norm, of rows that all go to the head)
+            closing = after
+            after = RowNorms.of(after)
+        after = after if isinstance(after, RowNorms) else None
         self.mixer.forward(h1, x, step, cache)
         if self.feed_forward is not None:
+            step.norm_after = after
             self.feed_forward.forward(h2, x, step)
-        step.norm_ready = step.norm_after = None
+        step.norm_after = None
+        left = step.norm_ready
+        if closing is not None and isinstance(left, NormedRows):
+            step.norm_ready = NormedRows(closing, left.x, left.normed[0])
 
 
 class JoinedProducts:

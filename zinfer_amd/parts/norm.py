@@ -221,6 +221,59 @@ class LayerNorm(Norm):
                           bool(then.spec.centred), out, y_bias=x_bias)
         return True
 
+    @property
+    def params(self):
+        return self.gain, self.bias, float(self.spec.eps)
+
+
+class RowNorms:
+    """One or two layer norms that read the same rows of the residual stream: run in one kernel, which
+    can also add the parts of the product that ends in those rows (``residual_sum``, as a norm has it;
+    the rows normed so come as ``NormedRows``)."""
+
+    def __init__(self, norms):
+        self.norms = tuple(norms)
+
+    @staticmethod
+    def of(*norms):
+        """For ``norms`` that one kernel can run, else None."""
+        if any(type(n) is not LayerNorm for n in norms) \
+                or len({bool(n.spec.centred) for n in norms}) > 1 \
+                or not all(ops.norm_add_norm_covers(n.spec.width) for n in norms):
+            return None
+        return RowNorms(norms)
+
+    def _outs(self, x: torch.Tensor, step):
+        act = self.norms[0].ctx.act_dtype
+        return [step.scratch(name, x.shape, act) for name in ("normed", "normed_ff")[:len(self.norms)]]
+
+    def forward(self, x: torch.Tensor, step, parts=None):
+        outs = self._outs(x, step)
+        ops.norms_of_rows(x, [n.params for n in self.norms], outs,
+                          bool(self.norms[0].spec.centred), parts)
+        return outs
+
+    def residual_sum(self, linear, a: torch.Tensor, out: torch.Tensor, step) -> bool:
+        if a.dtype != torch.bfloat16 or self.norms[0].ctx.act_dtype != a.dtype or not out.is_contiguous() \
+                or not a.is_contiguous() or linear.out_features != self.norms[0].spec.width \
+                or ops.stream_parts_plan(a.shape[0], linear.out_features, linear.in_features,
+                                         linear.weight, linear.tiled) is None:
+            return False
+        parts = ops.stream_parts(a, linear.weight)
+        step.norm_ready = NormedRows(self.norms, out, self.forward(out, step, parts))
+        return True
+
+
+class NormedRows:
+    """The rows ``normed`` = ``norm(x)`` that a block's last kernel already made for the norm that
+    reads the stream next (for several norms that read it: one each)."""
+
+    def __init__(self, norm, x: torch.Tensor, normed):
+        self.norm, self.x, self.normed = norm, x, normed
+
+    def fits(self, norm, x: torch.Tensor) -> bool:
+        return self.norm == norm and self.x.data_ptr() == x.data_ptr() and self.x.shape == x.shape
+
 
 register_part("norm", RmsNormSpec, RmsNorm)
 register_part("norm", LayerNormSpec, LayerNorm)
