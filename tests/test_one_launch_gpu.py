@@ -29,17 +29,17 @@ def test_the_sizes_python_accepts_are_accepted_by_the_entry():
         for hidden in (448, 512, 576, 1000, 5120, 8192, 32768):
             for ff in (256, 512, 1088, 12288, 25600, 32768, 53248):
                 for heads, kv in ((2, 1), (4, 4), (16, 1), (15, 1), (32, 8), (40, 8), (96, 96), (12, 5)):
-                    for page in (8, 16, 48):
+                    for page, tokens in ((8, 1), (16, 1), (48, 2), (16, 3), (32, 4), (16, 5)):
                         p = kernel._Layers()
-                        p.tokens, p.n_layers, p.hidden, p.ff = 1, 1, hidden, ff
+                        p.tokens, p.n_layers, p.hidden, p.ff = tokens, 1, hidden, ff
                         p.n_heads, p.n_kv_heads, p.page_size = heads, kv, page
                         p.max_splits = kernel.MAX_SPLITS
-                        if kernel.sizes_covered(1, hidden, ff, heads, kv, 128, page, wgs):
+                        if kernel.sizes_covered(tokens, hidden, ff, heads, kv, 128, page, wgs):
                             accepted += 1
                             if not torch.cuda.is_available():      # (nothing is launched without one)
                                 assert lib.zf_decode_layers(ctypes.byref(p), wgs, None) != -3, \
-                                    (wgs, hidden, ff, heads, kv, page)
-    assert accepted > 100
+                                    (wgs, hidden, ff, heads, kv, page, tokens)
+    assert accepted > 200
 
 
 def _qwen3(hidden, heads, kv, ff, layers=2, vocab=1030):
@@ -111,6 +111,45 @@ def test_single_tokens_against_the_plain_implementation(shape, monkeypatch):
     apart = _engine(cfg, w, page)
     apart.model.one_launch = None
     assert np.abs(_answer(apart, toks, singles) - got).max() <= LOGITS_TOL_BF16 * scale
+
+
+def _together(eng, requests, singles):
+    """Prompts one after the other, then a token of every request a step: the rows of each."""
+    from zinfer_amd.engine import StepEntry
+    rows = {r: [] for r in requests}
+    for r, t in requests.items():
+        eng.step([StepEntry(r, t[:-singles], [])])
+    for k in range(singles, 0, -1):
+        logits = eng.step([StepEntry(r, [t[-k]], [0]) for r, t in requests.items()])
+        for i, r in enumerate(requests):
+            rows[r].append(logits[i].float().cpu().numpy().copy())
+    for r in requests:
+        eng.release(r)
+    return {r: np.stack(v) for r, v in rows.items()}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,lengths", [
+    ((512, 4, 2, 512, 16), (9, 130)), ((576, 15, 1, 1088, 48), (140, 33, 12)), ((832, 4, 4, 832, 16), (8, 262, 40, 128)),
+    ((1024, 16, 8, 3072, 16), (133, 10, 300, 31)), ((2560, 32, 8, 9728, 32), (70, 900)), ((4096, 32, 8, 12288, 16), (1030, 40, 129))],
+    ids=str)
+def test_several_requests_against_the_plain_implementation_and_alone(shape, lengths, monkeypatch):
+    """Two to four tokens a step, with a graph and without: within the bound of the plain implementation, and of a
+    request the bits it has alone."""
+    hidden, heads, kv, ff, page = shape
+    cfg = _qwen3(hidden, heads, kv, ff)
+    w = _weights(cfg, hidden + heads)
+    requests = {f"r{i}": tiny.random_tokens(n, cfg["vocab_size"], n) for i, n in enumerate(lengths)}
+    monkeypatch.setattr(one_launch.OneLaunchLayers, "forward", _counted(calls := []))
+    eng = _engine(cfg, w, page)
+    got = _together(eng, requests, 6)
+    assert len(calls) >= 2 and eng.graph_replays > 0
+    plainly = _together(_engine(cfg, w, page, graphs=False), requests, 6)
+    for r, toks in requests.items():
+        ref = plain.model_forward_batched(cfg, w, toks).numpy()[-6:]
+        assert np.abs(got[r] - ref).max() <= LOGITS_TOL_BF16 * np.abs(ref).max()
+        assert np.array_equal(got[r], plainly[r])
+        assert np.array_equal(got[r], _together(eng, {r: toks}, 6)[r])
 
 
 def _counted(calls):

@@ -6,7 +6,9 @@
 // takes 14 us and 75: the weights, and where these are few the five times that rows travel between all
 // workgroups (2.4 us each).  Decode steps of one token of Qwen3 shapes behind 120 tokens, four layers and
 // the head, before and after: 0.6B 197 -> 164 us, 1.7B 285 -> 244, 4B 372 -> 350, 8B 560 -> 527; from
-// 14B on the launches' ends are small beside the weights (800 -> 795).
+// 14B on the launches' ends are small beside the weights (800 -> 795).  Two tokens 0.6B 196 -> 168, 8B 542 ->
+// 521; three 200 -> 179, 547 -> 535; four tokens of the 0.6B and 1.7B shapes 202 -> 187 and 291 -> 273: what the
+// workgroups hand each other grows with the tokens.
 //
 // One workgroup a CU stays for the whole step.  Its first DL_CW waves stream weights and multiply:
 // each holds the next RING tiles (16 rows x 64 of K, 2 KB) of its own in registers and asks for one
@@ -47,9 +49,11 @@
 #define DL_MEET_MOST 1000000000  // and until a step that too few came to fails
 #define DL_CLOSED (1u << 31)
 #define DL_UNITS 16              // most units of 16 outputs a workgroup has in a phase, times tokens
-#define DL_RUNS (5 * DL_UNITS)   // (a unit at gate/up is two row groups)
-#define DL_ATT 4                 // most splits of contexts a workgroup has
+#define DL_FF_UNITS 32           // and at gate/up, where a unit is two row groups
+#define DL_RUNS (3 * DL_UNITS + 2 * DL_FF_UNITS)
+#define DL_ATT 8                 // most splits of contexts a workgroup has
 #define DL_COPIES 4
+#define DL_TOKENS 4              // most of a step
 // a run: the first tile of a row group, whether a phase begins and ends with it, which product's
 #define DL_RUN_TILE 0x0fffffffu
 #define DL_RUN_FIRST (1u << 28)
@@ -153,12 +157,13 @@ struct alignas(16) DecodeShared {
   float o[4][16][DL_HD];
   float m[4][16], l[4][16];
   bf16_t q[18][DL_HD + 8];       // query heads; row 16: the new key; row 17: the new value
-  float part[DL_UNITS * 2][DL_CW][16];         // (unit, token) by wave; at gate/up two for each
+  float part[DL_FF_UNITS * 2][DL_CW][16];         // (unit, token) by wave; at gate/up two for each
   float turn[M][2][DL_HD / 2];   // cosines and sines of the tokens' positions
   size_t blk[DL_ATT][4][2];      // where the 16-key groups of the workgroup's splits lie in the pools
   size_t put[DL_ATT];            // and the 16-row group of the token's own key and value
   int item[DL_ATT];              // kv head, split << 8, token << 16 and whether it holds the token's own
   uint32_t runs[DL_RUNS];        // the row groups of a layer's products that are this workgroup's
+  float res[M > 1 ? 256 : 1];    // the stream's elements of this workgroup (one token: in registers)
   int n_runs, late, n_att;
   int dead;
   int wg, wgs;                   // this workgroup's number among those that do the step; none: it leaves
@@ -499,12 +504,12 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
   const int cwave = wave - DL_CW;
   // What is formed from a thread's number or the arguments is formed where it is used: hoisted out of
   // the layers' loop it takes the registers that the attention's keys and values need.
-  auto thread = [&]() {
+  auto thread = [&]() __attribute__((always_inline)) {
     uint32_t t = tid - DL_CW * 64;
     asm volatile("" : "+v"(t));
     return t;
   };
-  auto args = [&]() {
+  auto args = [&]() __attribute__((always_inline)) {
     DecodeArgs a = (DecodeArgs)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(a));
     return a;
@@ -517,14 +522,14 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
   const __amdgpu_buffer_rsrc_t words =
       __builtin_amdgcn_make_buffer_rsrc(p.words, 0, (int)(2 * 16 * at.all), 0x00020000);
   constexpr int SC1 = 16;
-  auto load2 = [&](uint32_t lane_bytes, uint32_t from) {
+  auto load2 = [&](uint32_t lane_bytes, uint32_t from) __attribute__((always_inline)) {
     return __builtin_amdgcn_raw_buffer_load_b128(words, lane_bytes, from, SC1);
   };
-  auto store2 = [&](uint32_t lane_bytes, uint32_t to, uint32_t d0, uint32_t d1, unsigned epoch) {
+  auto store2 = [&](uint32_t lane_bytes, uint32_t to, uint32_t d0, uint32_t d1, unsigned epoch) __attribute__((always_inline)) {
     __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{d0, epoch, d1, epoch}, words, lane_bytes, to, SC1);
   };
   // look() loads and says (a lane) whether words are missing; until none of the wave's are
-  auto wait_for = [&](auto look) {
+  auto wait_for = [&](auto look) __attribute__((always_inline)) {
     for (int spin = 0;; ++spin) {
       asm volatile("" ::: "memory");
       const bool missing = look();
@@ -534,10 +539,10 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
     }
   };
   // `n` pairs of words behind one another from pair `from`, a pair a thread, N at a time; to(number, data)
-  auto gather_some = [&](auto N, uint32_t from, uint32_t n, unsigned epoch, auto to) {
+  auto gather_some = [&](auto N, uint32_t from, uint32_t n, unsigned epoch, auto to) __attribute__((always_inline)) {
     const uint32_t t = thread();
     u32x4_t v[decltype(N)::value];
-    wait_for([&]() {
+    wait_for([&]() __attribute__((always_inline)) {
       uint32_t bad = 0;
 #pragma unroll
       for (int i = 0; i < decltype(N)::value; ++i) v[i] = load2(t * 16, (from + i * 256) * 16);
@@ -550,10 +555,10 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
     for (int i = 0; i < decltype(N)::value; ++i)
       if (t + i * 256 < n) to(t + i * 256, u32x2_t{v[i][0], v[i][2]});
   };
-  auto gather = [&](uint32_t from, uint32_t n, unsigned epoch, auto to) {
+  auto gather = [&](uint32_t from, uint32_t n, unsigned epoch, auto to) __attribute__((always_inline)) {
     uint32_t i = 0;
-    auto some = [&](auto N) {
-      gather_some(N, from + i, n - i, epoch, [&](uint32_t w, u32x2_t d) { to(i + w, d); });
+    auto some = [&](auto N) __attribute__((always_inline)) {
+      gather_some(N, from + i, n - i, epoch, [&](uint32_t w, u32x2_t d) __attribute__((always_inline)) { to(i + w, d); });
       i += decltype(N)::value * 256;
     };
     while (i + 1024 < n) some(std::integral_constant<int, 8>{});
@@ -562,17 +567,17 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
     else if (i < n) some(std::integral_constant<int, 1>{});
   };
   // rows of n numbers a token
-  auto gather_rows = [&](uint32_t from, int n, unsigned epoch) {
+  auto gather_rows = [&](uint32_t from, int n, unsigned epoch) __attribute__((always_inline)) {
 #pragma unroll
     for (int tok = 0; tok < M; ++tok)
       gather(from + tok * (n / 4), n / 4, epoch,
-             [&](uint32_t w, u32x2_t d) { *(u32x2_t*)(s_rows + (size_t)tok * row_bytes + w * 8) = d; });
+             [&](uint32_t w, u32x2_t d) __attribute__((always_inline)) { *(u32x2_t*)(s_rows + (size_t)tok * row_bytes + w * 8) = d; });
   };
   // rows that a norm reads next: the sums of squares of each 16 columns as well
-  auto gather_normed = [&](uint32_t from, uint32_t from_sq, unsigned epoch) {
+  auto gather_normed = [&](uint32_t from, uint32_t from_sq, unsigned epoch) __attribute__((always_inline)) {
     gather_rows(from + copy * (M * p.hidden / 4), p.hidden, epoch);
     gather(from_sq + copy * (M * groups / 2), M * groups / 2, epoch,
-           [&](uint32_t w, u32x2_t d) { *(u32x2_t*)(s_sq + 2 * w) = d; });
+           [&](uint32_t w, u32x2_t d) __attribute__((always_inline)) { *(u32x2_t*)(s_sq + 2 * w) = d; });
   };
   // 1 / sqrt(mean(x^2) + eps) of every token, the same in every lane
   auto inv_rms = [&](float eps, float (&inv)[M]) {
@@ -586,7 +591,7 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
     }
   };
   // Epilogues: sixteen threads a (unit, token), one a row of the unit.  The sum over the waves:
-  auto sum_waves = [&](uint32_t pair, uint32_t r) {
+  auto sum_waves = [&](uint32_t pair, uint32_t r) __attribute__((always_inline)) {
     float v[DL_CW];
 #pragma unroll
     for (int w = 0; w < DL_CW; ++w) v[w] = sh.part[pair][w][r];
@@ -596,7 +601,7 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
     return s;
   };
   // four lanes' values as two words each of the four holds
-  auto quad_words = [&](float v, uint32_t r, uint32_t& d0, uint32_t& d1) {
+  auto quad_words = [&](float v, uint32_t r, uint32_t& d0, uint32_t& d1) __attribute__((always_inline)) {
     const float o = lane_xor<1>(v);
     const uint32_t mine = r % 2 ? pack_bf16x2(o, v) : pack_bf16x2(v, o);
     const uint32_t other = __float_as_uint(lane_xor<2>(__uint_as_float(mine)));
@@ -619,17 +624,21 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
   if (keeps) {
     const Place e = place();
     res = p.x[(size_t)e.tok * p.hidden + column(e)];
+    if constexpr (M > 1) sh.res[thread()] = res;
   }
   // The sum joins the stream's element, and what the next norm needs of the result goes to the words
   // at `to` and `to_sq`, or (last) back to memory.
-  auto residual = [&](float gain, uint32_t to, uint32_t to_sq, unsigned epoch, bool last) {
+  auto residual = [&](float gain, uint32_t to, uint32_t to_sq, unsigned epoch, bool last) __attribute__((always_inline)) {
     if (!keeps) return;
     const Place e = place();
     const uint32_t e_r = e.r, e_tok = e.tok, keeps_at = column(e);
-    res += sum_waves(e.pair, e_r);
-    const float sq = lanes_sum<16>(res * res);
+    float now = M > 1 ? sh.res[thread()] : res;
+    now += sum_waves(e.pair, e_r);
+    if constexpr (M > 1) sh.res[thread()] = now;
+    else res = now;
+    const float sq = lanes_sum<16>(now * now);
     uint32_t d0, d1;
-    quad_words(res * gain, e_r, d0, d1);
+    quad_words(now * gain, e_r, d0, d1);
     const uint32_t c = e_r % DL_COPIES;
     const uint32_t row = (c * M + e_tok) * p.hidden + (keeps_at & ~3u);       // numbers, 4 a pair of words
     if (!last) {
@@ -641,7 +650,7 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
     }
     const DecodeArgs pp = args();
     const size_t n = (size_t)e_tok * p.hidden + keeps_at;
-    pp->x[n] = res;
+    pp->x[n] = now;
     if (c == 0) *(u32x2_t*)(pp->xg + n) = u32x2_t{d0, d1};
     if (e_r == 0) pp->sq[(size_t)(keeps_at / 16) * 16 + e_tok] = sq;
   };
@@ -741,7 +750,7 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
       const uint32_t row = (set + at.qkv + s * (qkv_units * 4)) * 16;
       const uint32_t head_at = (hi < G ? kvh * G + hi : nH + kvh) * (DL_HD / 4 * 16) + l16 * 16;
       u32x4_t r0, r1, v0, v1;
-      wait_for([&]() {
+      wait_for([&]() __attribute__((always_inline)) {
         r0 = load2(head_at, row);
         r1 = load2(head_at, row + DL_HD / 8 * 16);
         const uint32_t bad = (r0[1] ^ epoch) | (r0[3] ^ epoch) | (r1[1] ^ epoch) | (r1[3] ^ epoch);
@@ -749,7 +758,7 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
       });
       if (own && cwave == 0) {
         const uint32_t value_at = row + (nH + p.nKV + kvh) * (DL_HD / 4 * 16);
-        wait_for([&]() {
+        wait_for([&]() __attribute__((always_inline)) {
           v0 = load2(l16 * 32, value_at);
           v1 = load2(l16 * 32, value_at + 16);
           return ((v0[1] ^ epoch) | (v0[3] ^ epoch) | (v1[1] ^ epoch) | (v1[3] ^ epoch)) != 0;
@@ -817,7 +826,7 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
         // (lane j: element 16 dt + j of keys 4 qd .. + 3)
         if (pos >= kb && pos < kb + DL_WAVE_KEYS) {
           const int jn = (pos - kb) % 16;
-          auto patch = [&](u32x4_t (&k)[DL_HD / 32], u32x2_t (&v)[DL_HD / 16]) {
+          auto patch = [&](u32x4_t (&k)[DL_HD / 32], u32x2_t (&v)[DL_HD / 16]) __attribute__((always_inline)) {
 #pragma unroll
             for (int stp = 0; stp < DL_HD / 32; ++stp) {
               const u32x4_t kx = *(const u32x4_t*)(sh.q[16] + stp * 32 + 8 * qd);
@@ -897,7 +906,7 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
           const uint32_t mine = min(sp0 + slot, last) * (DL_PART * 8);
           u32x4_t ml;
           u32x2_t v;
-          wait_for([&]() {
+          wait_for([&]() __attribute__((always_inline)) {
             v = __builtin_amdgcn_raw_buffer_load_b64(words, mine + (piece * 8 + d8) * 8, from, SC1);
             ml = load2(mine + DL_HD * 8, from);
             return ((v[1] ^ epoch) | (ml[1] ^ epoch) | (ml[3] ^ epoch)) != 0;
@@ -1008,23 +1017,26 @@ extern "C" long long zf_decode_layers_words(int M, int hidden, int ff, int nH, i
 extern "C" int zf_decode_layers(const DecodeLayers* args, int workgroups, hipStream_t stream) {
   DecodeLayers p = *args;
   const int M = p.tokens;
-  if (M < 1 || M > 1 || p.n_layers < 1 || workgroups < 1) return -3;
+  if (M < 1 || M > DL_TOKENS || p.n_layers < 1 || workgroups < 1) return -3;
   if (p.hidden % 64 != 0 || p.ff % 64 != 0 || p.hidden < 512 || p.ff < 512 || p.nKV < 1 || p.nKV > 255 ||
       p.nH % p.nKV != 0 || p.nH / p.nKV > 15 || p.nH * DL_HD < 512 || p.page_size % 16 != 0 ||
       p.max_splits < 1 || p.max_splits > 255)
     return -3;
   int units = (p.nH + 2 * p.nKV) * (DL_HD / 16);
   if (p.hidden / 16 > units) units = p.hidden / 16;
-  if (p.ff / 16 > units) units = p.ff / 16;
-  const int per = DL_UNITS / M, splits = M * p.nKV * p.max_splits;
+  const int per = DL_UNITS / M, ff_per = DL_FF_UNITS / M, splits = M * p.nKV * p.max_splits;
   p.need = (units + per - 1) / per;
+  if ((p.ff / 16 + ff_per - 1) / ff_per > p.need) p.need = (p.ff / 16 + ff_per - 1) / ff_per;
   if ((splits + DL_ATT - 1) / DL_ATT > p.need) p.need = (splits + DL_ATT - 1) / DL_ATT;
   if (2 * p.need > workgroups) return -3;        // (of two launches that meet at once one goes on)
   if ((p.cos_t == nullptr) != (p.sin_t == nullptr) || (p.cos_t != nullptr && p.table_rows < 1)) return -3;
-  const size_t lds = dl_lds<1>(p);
+  const size_t lds = M == 1 ? dl_lds<1>(p) : M == 2 ? dl_lds<2>(p) : M == 3 ? dl_lds<3>(p) : dl_lds<4>(p);
   if (lds > 160 * 1024) return -3;
   void* params[] = {&p};
-  const void* kernel = (const void*)decode_layers_kernel<1, 3>;
+  const void* kernel = M == 1   ? (const void*)decode_layers_kernel<1, 3>
+                       : M == 2 ? (const void*)decode_layers_kernel<2, 3>
+                       : M == 3 ? (const void*)decode_layers_kernel<3, 3>
+                                : (const void*)decode_layers_kernel<4, 3>;
   hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return (int)e;
   return (int)hipLaunchKernel(kernel, dim3(workgroups), dim3(DL_THREADS), params, lds, stream);

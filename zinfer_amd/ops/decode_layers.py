@@ -15,8 +15,9 @@ SPLIT_KEYS = 128             # DL_SPLIT
 MAX_SPLITS = 32              # of a context
 MAX_CONTEXT = MAX_SPLITS * SPLIT_KEYS
 MAX_UNITS = 16               # DL_UNITS
-MAX_ATTENTION = 4            # DL_ATT
-MAX_TOKENS = 1
+MAX_FF_UNITS = 32            # DL_FF_UNITS
+MAX_ATTENTION = 8            # DL_ATT
+MAX_TOKENS = 4               # DL_TOKENS
 MEETING = 512                # bytes of DecodeMeet
 
 _vp, _i, _f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
@@ -53,11 +54,12 @@ def sizes_covered(tokens: int, hidden: int, ff: int, n_heads: int, n_kv_heads: i
             and hidden % 64 == 0 and ff % 64 == 0
             and min(hidden, ff, n_heads * head_dim) >= 512):
         return False
-    units = (hidden // 16, ff // 16, (n_heads + 2 * n_kv_heads) * head_dim // 16)
+    units = (hidden // 16, (n_heads + 2 * n_kv_heads) * head_dim // 16)
     row = 2 * max(hidden, ff, n_heads * head_dim) + 16
-    return 2 * max(units) <= MAX_UNITS // tokens * wgs \
-        and 2 * tokens * n_kv_heads * MAX_SPLITS <= MAX_ATTENTION * wgs \
-        and 64 * 1024 + tokens * (row + hidden // 4 + 512) <= 160 * 1024
+    most = wgs // 2                # (decode_layers.hip: of two launches that meet one goes on)
+    return max(units) <= MAX_UNITS // tokens * most and ff // 16 <= MAX_FF_UNITS // tokens * most \
+        and tokens * n_kv_heads * MAX_SPLITS <= MAX_ATTENTION * most \
+        and 80 * 1024 + tokens * (row + hidden // 4 + 512) <= 160 * 1024
 
 
 def words(tokens: int, hidden: int, ff: int, n_heads: int, n_kv_heads: int, device) -> torch.Tensor:
