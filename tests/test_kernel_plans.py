@@ -164,6 +164,7 @@ TESTED_AGAINST = {
     "concat_rows": "test_nupovik_kernels_gpu.py:test_concat_rows",
     "token_shift_mix": "plain_nupovik.py:token_shift",
     "decay_recurrence": "plain_nupovik.py:decayed_outer_recurrence",
+    "decay_step": "plain_nupovik.py:decayed_outer_recurrence",
     "head_norm_gate": "test_nupovik_kernels_gpu.py:test_head_norm_gate",
     "streams_step": "plain_kugisun.py:stream_step",
     "short_conv": "plain_kugisun.py:short_convolution",

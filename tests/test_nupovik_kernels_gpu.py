@@ -37,6 +37,51 @@ def _starts(lens):
     return out
 
 
+# ------------------------------------------------------------------------------ a decode step in one kernel
+@pytest.mark.parametrize("n,H,d,dv,rank,rule,gate_kind,gain", [
+    (1, 1, 8, 1, 8, "sigmoid_root", "silu", "head"), (16, 8, 128, 256, 16, "sigmoid_root", "silu", "head"),
+    (16, 32, 64, 64, 16, "double_exp", "silu", "row"), (5, 3, 16, 50, 64, "double_exp", "sigmoid", None),
+    (3, 2, 256, 128, 512, "sigmoid_root", "silu", "row"), (2, 2, 32, 1000, 128, "double_exp", "silu", "head"),
+    (7, 4, 64, 33, 32, "sigmoid_root", "sigmoid", "row")])
+def test_a_decode_steps_recurrence_in_one_kernel(n, H, d, dv, rank, rule, gate_kind, gain):
+    """Against the product, the recurrence and the norm one after the other: the middle's sums of ``rank`` bfloat16
+    products differ in their order (1e-6), the rest does not, then the rounding to bfloat16; the slots' columns beyond
+    the matrices stay."""
+    dt = torch.bfloat16
+    assert ops.decay_step_sizes(d, dv, rank)
+    proj = _rand((n, 2 * H * d + 2 * H * dv), 1, 1.0, dt).to(DEV)
+    q, k = proj[:, :H * d], proj[:, H * d:2 * H * d]
+    v, gate = proj[:, 2 * H * d:2 * H * d + H * dv], proj[:, 2 * H * d + H * dv:]
+    low = _rand((n, rank), 2, 1.0, dt).to(DEV)
+    up = _rand((H * d, rank), 3, rank ** -0.5, dt).to(DEV)
+    z_bias = (_rand((H * d,), 4) - 1.0).to(DEV)
+    bonus = _rand((H * d,), 5, 0.5).to(DEV) if rule == "double_exp" else None
+    gains = {"head": _rand((dv,), 6, 0.1) + 1.0, "row": _rand((H * dv,), 6, 0.1) + 1.0, None: None}[gain]
+    gains = None if gains is None else gains.to(DEV)
+    need = ops.recurrence_state_size(H, d, dv)
+    state = _rand((n + 2, need + 8), 7).to(DEV)
+    slots = _i32([(3 * i + 1) % (n + 2) for i in range(n)] if (n + 2) % 3 else list(range(1, n + 1)))
+    want_state, got_state = state.clone(), state.clone()
+    z = torch.empty((n, H * d), device=DEV)
+    ops.gemm(low, up, z)
+    o = torch.empty((n, H * dv), device=DEV)
+    want, got = (torch.full((n, H * dv), float("nan"), dtype=dt, device=DEV) for _ in range(2))
+    ops.decay_recurrence(q, k, v, z, z_bias, bonus, want_state, slots, _i32(list(range(n + 1))), o, H, d, dv,
+                         rule, tau=16.0, q_scale=0.25, max_q_len=1)
+    ops.head_norm_gate(o, gains, gate, want, H, 1e-6, gate_kind)
+    ops.decay_step(q, k, v, low, up, z_bias, bonus, got_state, slots, gains, gate, got, H, d, dv, rule, 16.0,
+                   0.25, 1e-6, gate_kind)
+    assert rel_err(got_state, want_state) <= 1e-5
+    assert torch.equal(got_state[:, need:], state[:, need:])
+    assert rel_err(got, want) <= tol(dt)
+    assert float((got != want).float().mean()) <= 0.01
+
+
+def test_decay_step_refuses_what_it_does_not_take():
+    for d, dv, rank in ((24, 64, 16), (512, 64, 16), (64, 64, 12), (64, 64, 24), (256, 256, 16), (12, 8, 8)):
+        assert not ops.decay_step_sizes(d, dv, rank)
+
+
 # ------------------------------------------------------------------------------ norms of the same rows
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("T,W,K", [(1, 4, 64), (3, 1020, 0), (16, 2048, 7168), (16, 2048, 0), (2, 2052, 0),

@@ -671,6 +671,160 @@ extern "C" int zf_head_norm_gate(const float* o, const float* gain, int gain_per
   ZF_CHECK_LAUNCH();
 }
 
+// ---------------------------------------------------------------- a decode step's recurrence, whole
+// One token a sequence (bfloat16): a workgroup a (sequence, head) forms the head's decays from the narrow
+// middle (z = up low, 32-bit sums), walks the token as decay_recurrence_kernel does (the same sums over
+// the same lanes), norms the head's output and applies gain and gate as head_norm_gate does.  Of 58 us a
+// layer of 16 tokens the three kernels took 18 and 22 (32 heads of 64 x 64, 8 of 128 x 256): each waits for its first
+// loads and a launch, while
+// the state, the bulk of the bytes, is asked for here ahead of all else: 9 and 12.
+// From 1 to 64 sequences a pass of four layers is 5 to 12 % shorter.
+// Thread (vl, cg) = (tid / CS, tid % CS) holds S[8 cg .. + 8, RV vl .. + RV].  CS = d / 8 lanes share a
+// column, `parts` lanes (8 numbers of the middle each) a channel's decay: powers of two.
+struct DecayStep {
+  const bf16_t *q, *k, *v, *low, *up, *gate;
+  long long q_stride, k_stride, v_stride, low_stride, gate_stride, out_stride, slot_stride;
+  const float *z_bias, *bonus, *gain;
+  float* state;
+  const int* state_slots;
+  bf16_t* out;
+  int H, d, dv, CS, parts, rule, gain_per_head, gate_kind;
+  float inv_tau, q_scale, eps;
+};
+template <bool BEFORE, int RV>
+__global__ __launch_bounds__(1024) void decay_step_kernel(DecayStep p) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  __shared__ float red[16];
+  const int d = p.d, dv = p.dv, CS = p.CS;
+  float* qs = lds;                        // [d]
+  float* ks = qs + d;
+  float* ds = ks + d;
+  float* us = ds + d;
+  float* vs = us + d;                     // [dv up to a multiple of 4]
+  float* os = vs + (dv + 3) / 4 * 4;      // [dv]
+  const int s = blockIdx.x, hd = blockIdx.y, tid = threadIdx.x, nt = blockDim.x;
+  const int vl = tid / CS, cg = tid % CS, col = vl * RV;
+  float* st = p.state + (size_t)p.state_slots[s] * p.slot_stride + ((size_t)hd * dv + col) * d + cg * REC_R;
+  float S[RV][REC_R];
+#pragma unroll
+  for (int r = 0; r < RV; ++r) {
+    float4 a = float4{0.f, 0.f, 0.f, 0.f}, b = a;
+    if (col + r < dv) {
+      a = *(const float4*)(st + (size_t)r * d);
+      b = *(const float4*)(st + (size_t)r * d + 4);
+    }
+    S[r][0] = a.x; S[r][1] = a.y; S[r][2] = a.z; S[r][3] = a.w;
+    S[r][4] = b.x; S[r][5] = b.y; S[r][6] = b.z; S[r][7] = b.w;
+  }
+  // (every lane of a channel's group is in the same round)
+  for (int task = tid; task < d * p.parts; task += nt) {
+    const int c = task / p.parts, part = task % p.parts;
+    float a[8], b[8], z[1] = {0.f};
+    load8<bf16_t>(p.up + ((size_t)(hd * d + c) * p.parts + part) * 8, a);
+    load8<bf16_t>(p.low + (size_t)s * p.low_stride + part * 8, b);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) z[0] = fmaf(a[j], b[j], z[0]);
+    lanes_sum_up(z, p.parts);
+    if (part == 0) {
+      ds[c] = decay_of(z[0] + p.z_bias[hd * d + c], p.rule, p.inv_tau);
+      qs[c] = bf16_to_float(p.q[(size_t)s * p.q_stride + hd * d + c]) * p.q_scale;
+      ks[c] = bf16_to_float(p.k[(size_t)s * p.k_stride + hd * d + c]);
+      us[c] = BEFORE ? p.bonus[hd * d + c] : 0.f;
+    }
+  }
+  for (int x = tid; x < dv; x += nt) vs[x] = bf16_to_float(p.v[(size_t)s * p.v_stride + hd * dv + x]);
+  __syncthreads();
+  float acc[RV];
+  const float *q8 = qs + cg * REC_R, *k8 = ks + cg * REC_R, *d8 = ds + cg * REC_R, *u8 = us + cg * REC_R;
+#pragma unroll
+  for (int r = 0; r < RV; ++r) {
+    const float vv = col + r < dv ? vs[col + r] : 0.f;
+    float a = 0.f;
+#pragma unroll
+    for (int j = 0; j < REC_R; ++j) {
+      const float kv = k8[j] * vv;
+      if (BEFORE) {
+        a = fmaf(q8[j], fmaf(u8[j], kv, S[r][j]), a);
+        S[r][j] = fmaf(d8[j], S[r][j], kv);
+      } else {
+        S[r][j] = fmaf(d8[j], S[r][j], kv);
+        a = fmaf(q8[j], S[r][j], a);
+      }
+    }
+    acc[r] = a;
+  }
+#pragma unroll
+  for (int r = 0; r < RV; ++r)
+    if (col + r < dv) {
+      *(float4*)(st + (size_t)r * d) = float4{S[r][0], S[r][1], S[r][2], S[r][3]};
+      *(float4*)(st + (size_t)r * d + 4) = float4{S[r][4], S[r][5], S[r][6], S[r][7]};
+    }
+  lanes_sum_up(acc, CS);
+  if (cg == 0)
+#pragma unroll
+    for (int r = 0; r < RV; ++r)
+      if (col + r < dv) os[col + r] = acc[r];
+  __syncthreads();
+  float ss = 0.f;
+  for (int x = tid; x < dv; x += nt) ss = fmaf(os[x], os[x], ss);
+  ss = block_sum(ss, red);
+  const float inv = 1.0f / sqrtf(ss / (float)dv + p.eps);
+  const bf16_t* gr = p.gate + (size_t)s * p.gate_stride + (size_t)hd * dv;
+  bf16_t* row = p.out + (size_t)s * p.out_stride + (size_t)hd * dv;
+  const float* gn = p.gain == nullptr ? nullptr : p.gain + (p.gain_per_head ? hd * dv : 0);
+  for (int x = tid; x < dv; x += nt) {
+    const float gv = bf16_to_float(gr[x]), sig = 1.0f / (1.0f + expf(-gv));
+    row[x] = float_to_bf16(os[x] * inv * (gn != nullptr ? gn[x] : 1.0f) * (p.gate_kind == 0 ? gv * sig : sig));
+  }
+}
+
+// Columns a thread: as few as 1024 threads take; none: the head is too large.
+static int decay_step_columns(int d, int dv) {
+  for (int rv = 1; rv <= 4; rv *= 2)
+    if ((long long)((dv + rv - 1) / rv) * (d / REC_R) <= (rv < 4 ? 512 : 1024)) return rv;
+  return 0;
+}
+static bool decay_step_covers(int d, int dv, int rank) {
+  auto power = [](int n) { return n > 0 && (n & (n - 1)) == 0; };
+  return d > 0 && dv > 0 && d % 8 == 0 && power(d / 8) && d / 8 <= 32 && rank % 8 == 0 && power(rank / 8) &&
+         rank / 8 <= 64 && decay_step_columns(d, dv) > 0;
+}
+
+// q, k, v, low, gate and out: bfloat16 rows [n_seqs, ..] at their strides; low rows and up [H * d, rank] 16-byte
+// aligned (strides too); the state's slots as decay_recurrence keeps them, 16-byte aligned.
+extern "C" int zf_decay_step(const void* q, long long q_stride, const void* k, long long k_stride, const void* v,
+                             long long v_stride, const void* low, long long low_stride, const void* up, int rank,
+                             const float* z_bias, const float* bonus, float* state, long long slot_stride,
+                             const int* state_slots, const float* gain, int gain_per_head, const void* gate,
+                             long long gate_stride, int gate_kind, void* out, long long out_stride, int n_seqs,
+                             int H, int d, int dv, int rule, float inv_tau, float q_scale, float eps,
+                             hipStream_t stream) {
+  if (n_seqs <= 0) return 0;
+  if (H <= 0 || !decay_step_covers(d, dv, rank) || low_stride % 8 != 0 || slot_stride % 4 != 0 ||
+      ((uintptr_t)low | (uintptr_t)up | (uintptr_t)state) % 16 != 0 || rule < 0 || rule > 1)
+    return -2;
+  const DecayStep p{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)low, (const bf16_t*)up,
+                    (const bf16_t*)gate, q_stride, k_stride, v_stride, low_stride, gate_stride, out_stride,
+                    slot_stride, z_bias, bonus, gain, state, state_slots, (bf16_t*)out, H, d, dv, d / REC_R,
+                    rank / 8, rule, gain_per_head, gate_kind, inv_tau, q_scale, eps};
+  const int rv = decay_step_columns(d, dv);
+  const int threads = ((dv + rv - 1) / rv * (d / REC_R) + ZF_WAVE - 1) / ZF_WAVE * ZF_WAVE;
+  const size_t smem = (size_t)(4 * d + (dv + 3) / 4 * 4 + dv) * sizeof(float);
+#define ZF_DECAY_STEP(B, RV)                                                                     \
+  hipLaunchKernelGGL((decay_step_kernel<B, RV>), dim3(n_seqs, H), dim3(threads), smem, stream, p)
+  if (bonus != nullptr) {
+    if (rv == 1) ZF_DECAY_STEP(true, 1);
+    else if (rv == 2) ZF_DECAY_STEP(true, 2);
+    else ZF_DECAY_STEP(true, 4);
+  } else {
+    if (rv == 1) ZF_DECAY_STEP(false, 1);
+    else if (rv == 2) ZF_DECAY_STEP(false, 2);
+    else ZF_DECAY_STEP(false, 4);
+  }
+#undef ZF_DECAY_STEP
+  ZF_CHECK_LAUNCH();
+}
+
 // ---------------------------------------------------------------- gate, then a norm over equal parts
 // u = o * gate(g); out[t, p, :] = u / sqrt(mean(u^2) + eps) * gain over the P parts of dv columns a
 // row has; gain [P dv].  Otherwise as above: a wave a (token, part), or (WIDE) a workgroup of four

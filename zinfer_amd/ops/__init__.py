@@ -3202,6 +3202,58 @@ def decay_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch
 GATE_KINDS = {"silu": 0, "sigmoid": 1}
 
 
+def decay_step_sizes(key_dim: int, value_dim: int, rank: int) -> bool:
+    """The sizes of heads and of the middle that ``zf_decay_step`` takes."""
+    lanes, parts = key_dim // 8, rank // 8
+    power = lambda n: n > 0 and n & (n - 1) == 0
+    return key_dim % 8 == 0 and rank % 8 == 0 and power(lanes) and power(parts) and lanes <= 32 \
+        and parts <= 64 and 0 < (value_dim + 3) // 4 * lanes <= 1024
+
+
+def decay_step_covers(key_dim: int, value_dim: int, state: torch.Tensor, low: torch.Tensor,
+                      up: torch.Tensor) -> bool:
+    """Whether ``decay_step`` takes a step of single tokens of such heads: bfloat16, key sizes and middles of
+    eight times a power of two."""
+    return low.is_cuda and low.dtype == up.dtype == torch.bfloat16 and up.is_contiguous() \
+        and low.stride(1) == 1 and low.stride(0) % 8 == 0 and state.stride(0) % 4 == 0 \
+        and all(t.data_ptr() % 16 == 0 for t in (low, up, state)) \
+        and decay_step_sizes(int(key_dim), int(value_dim), up.shape[1])
+
+
+@_launches("attention")
+def decay_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, low: torch.Tensor, up: torch.Tensor,
+               z_bias: torch.Tensor, bonus: Optional[torch.Tensor], state: torch.Tensor,
+               state_slots: torch.Tensor, gain: Optional[torch.Tensor], gate: torch.Tensor,
+               out: torch.Tensor, n_heads: int, key_dim: int, value_dim: int, rule: str,
+               tau: float, q_scale: float, eps: float, gate_kind: str = "silu") -> None:
+    """A step of one token a sequence (row s is sequence s's) in one kernel: z = low up^T as ``gemm`` stores it in
+    32-bit (``low`` [T, rank], ``up`` [H * d, rank] in rows), ``decay_recurrence`` of q, k, v and z, then
+    ``head_norm_gate`` into ``out``.  bfloat16 rows; sizes of ``decay_step_covers``."""
+    _need_gpu(z_bias, bonus, state, state_slots, up)
+    _i32(state_slots, "state_slots")
+    T, H, d, dv = q.shape[0], int(n_heads), int(key_dim), int(value_dim)
+    rows = ((q, H * d), (k, H * d), (v, H * dv), (gate, H * dv), (out, H * dv), (low, up.shape[1]))
+    if rule not in ("sigmoid_root", "double_exp") or gate_kind not in GATE_KINDS or not tau > 0.0 \
+            or any(t.shape != (T, w) or t.dtype != torch.bfloat16 or not t.is_cuda for t, w in rows) \
+            or up.shape[0] != H * d or z_bias.shape != (H * d,) or z_bias.dtype != torch.float32 \
+            or (bonus is not None and (bonus.shape != (H * d,) or bonus.dtype != torch.float32)) \
+            or (gain is not None and (gain.dtype != torch.float32 or gain.shape not in ((dv,), (H * dv,)))) \
+            or state_slots.shape[0] != T or state.dtype != torch.float32 or state.dim() != 2 \
+            or state.shape[1] < recurrence_state_size(H, d, dv) \
+            or not decay_step_covers(d, dv, state, low, up):
+        raise KernelUnavailable(f"decay_step: q {tuple(q.shape)}, v {tuple(v.shape)} {q.dtype}, low "
+                                f"{tuple(low.shape)}, up {tuple(up.shape)}, state {tuple(state.shape)} for {H} "
+                                f"heads of {d} x {dv}, rule {rule!r}")
+    at = lambda t: ctypes.c_longlong(_columns(t, "decay_step"))
+    lib = build.load("recurrent")
+    _check(lib.zf_decay_step(
+        _ptr(q), at(q), _ptr(k), at(k), _ptr(v), at(v), _ptr(low), at(low), _ptr(up), up.shape[1],
+        _ptr(z_bias), _ptr(bonus), _ptr(state), ctypes.c_longlong(state.stride(0)), _ptr(state_slots),
+        _ptr(gain), 1 if gain is not None and gain.shape == (H * dv,) and H > 1 else 0, _ptr(gate),
+        at(gate), GATE_KINDS[gate_kind], _ptr(out), at(out), T, H, d, dv, DECAY_RULES[rule],
+        ctypes.c_float(1.0 / tau), ctypes.c_float(q_scale), ctypes.c_float(eps), _stream()), "decay_step")
+
+
 @_launches("norm_rope_write")
 def head_norm_gate(o: torch.Tensor, gain: Optional[torch.Tensor], gate: torch.Tensor,
                    out: torch.Tensor, n_heads: int, eps: float, gate_kind: str = "silu") -> None:

@@ -13,7 +13,7 @@ from . import (gated_act, moe_grouped, norm_add_norm, tied_attention_mfma)
 from . import delta_recurrence, short_conv, streams_step
 from . import add_row, bias_act_rows, fixed_decay, rotation_table
 from . import embed_norm, gate_norm, gated_rows, gemm_geglu, state_space
-from . import (concat_rows, decay_recurrence, embed_sinusoid, head_norm_gate, token_shift_mix)
+from . import (concat_rows, decay_recurrence, decay_step, embed_sinusoid, head_norm_gate, token_shift_mix)
 from . import gemm_many
 from . import (activation, head_products, masked_attention, masked_attention_mfma,
                norm_add_store, project_rows)
@@ -117,6 +117,8 @@ KERNELS: Dict[str, KernelEntry] = {
                                    "row before it, the last row kept as state"),
     "decay_recurrence": KernelEntry(decay_recurrence, "recurrent", "own: a matrix a head, decayed "
                                     "a key channel and grown by k v^T, token by token"),
+    "decay_step": KernelEntry(decay_step, "recurrent", "own: that of single tokens from the decays' narrow "
+                              "middle to the normed, gated output"),
     "head_norm_gate": KernelEntry(head_norm_gate, "recurrent", "own: RMS norm a head, gain and "
                                   "silu gate"),
     "streams_step": KernelEntry(streams_step, "norms", "own: a residual stream in several "

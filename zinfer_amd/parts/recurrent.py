@@ -29,6 +29,12 @@ def _middle(tensors, down_name: str, up_name: str, rank) -> int:
     return have
 
 
+def _single_tokens(step, T: int, cache) -> bool:
+    """A step of one token a sequence on the GPU, whose recurrence may run in one kernel (``decay_step``, of
+    bfloat16 builds)."""
+    return step.max_q_len == 1 and T == step.state_slots.shape[0] and cache.state.is_cuda
+
+
 class GatedLinearAttention(Mixer):
     """The mixer of ``GatedLinearAttentionSpec``: q, k, v and the output gate come from one
     product over the stacked matrices (each output keeps its own dot product); the decay's
@@ -71,7 +77,8 @@ class GatedLinearAttention(Mixer):
         self.o = Linear(place_matrix(tensors[p + s.o_name], self.ctx))
         self.rank = _middle(tensors, p + s.decay_down_name, p + s.decay_up_name, s.decay_rank)
         self.decay_down = Linear(place_matrix(tensors[p + s.decay_down_name], self.ctx))
-        self.decay_up = Linear(place_matrix(tensors[p + s.decay_up_name], self.ctx))
+        self.decay_rows = place_matrix(tensors[p + s.decay_up_name], self.ctx)
+        self.decay_up = Linear(self.decay_rows)
         self.decay_bias = place_gain(tensors[p + s.decay_bias_name], self.ctx)
         self.gain = place_gain(tensors[p + s.norm_name], self.ctx)
 
@@ -88,6 +95,15 @@ class GatedLinearAttention(Mixer):
         proj = step.scratch("rec_proj", (T, self.proj.out_features), act)
         low = step.scratch("rec_decay_low", (T, self.rank), act)
         products([(h, self.proj, proj, None), (h, self.decay_down, low, None)])
+        mixed = step.scratch("rec_mixed", (T, V), act)
+        if _single_tokens(step, T, cache) and \
+                ops.decay_step_covers(s.head_dim, s.value_dim, cache.state, low, self.decay_rows):
+            ops.decay_step(proj[:, :QK], proj[:, QK:2 * QK], proj[:, 2 * QK:2 * QK + V], low, self.decay_rows,
+                           self.decay_bias, None, cache.state, step.state_slots, self.gain,
+                           proj[:, 2 * QK + V:], mixed, s.n_heads, s.head_dim, s.value_dim,
+                           "sigmoid_root", float(s.tau), self.q_scale, float(s.norm_eps))
+            self.o.forward(mixed, residual, accumulate=True, step=step)
+            return
         z = step.scratch("rec_decay_z", (T, QK), torch.float32)
         self.decay_up.forward(low, z)
         o = step.scratch("rec_out", (T, V), torch.float32)
@@ -95,7 +111,6 @@ class GatedLinearAttention(Mixer):
                              self.decay_bias, None, cache.state, step.state_slots, step.q_start,
                              o, s.n_heads, s.head_dim, s.value_dim, "sigmoid_root",
                              tau=float(s.tau), q_scale=self.q_scale, max_q_len=step.max_q_len)
-        mixed = step.scratch("rec_mixed", (T, V), act)
         ops.head_norm_gate(o, self.gain, proj[:, 2 * QK + V:], mixed, s.n_heads,
                            float(s.norm_eps))
         self.o.forward(mixed, residual, accumulate=True, step=step)
@@ -141,7 +156,8 @@ class TokenShiftRecurrence(Mixer):
                          for n in (s.r_name, s.k_name, s.v_name, s.gate_name)]
         self.rank = _middle(tensors, p + s.decay_down_name, p + s.decay_up_name, s.decay_rank)
         self.decay_down = Linear(place_matrix(tensors[p + s.decay_down_name], self.ctx))
-        self.decay_up = Linear(place_matrix(tensors[p + s.decay_up_name], self.ctx))
+        self.decay_rows = place_matrix(tensors[p + s.decay_up_name], self.ctx)
+        self.decay_up = Linear(self.decay_rows)
         self.decay_bias = place_gain(tensors[p + s.decay_bias_name], self.ctx)
         self.bonus = place_gain(tensors[p + s.bonus_name].reshape(-1), self.ctx)
         self.gain = place_gain(tensors[p + s.norm_name], self.ctx)
@@ -164,13 +180,20 @@ class TokenShiftRecurrence(Mixer):
         low = step.scratch("rec_decay_low", (T, self.rank), act)
         products([(mixes[i], product, rkvg[i], None) for i, product in enumerate(self.products)]
                  + [(mixes[4], self.decay_down, low, "tanh")])
+        mixed = step.scratch("rec_mixed", (T, self.width), act)
+        if _single_tokens(step, T, cache) and \
+                ops.decay_step_covers(s.head_dim, s.head_dim, cache.state, low, self.decay_rows):
+            ops.decay_step(rkvg[0], rkvg[1], rkvg[2], low, self.decay_rows, self.decay_bias, self.bonus,
+                           cache.state, step.state_slots, self.gain, rkvg[3], mixed, s.n_heads,
+                           s.head_dim, s.head_dim, "double_exp", 1.0, 1.0, float(s.norm_eps))
+            self.o.forward(mixed, residual, accumulate=True, step=step)
+            return
         z = step.scratch("rec_decay_z", (T, self.width), torch.float32)
         self.decay_up.forward(low, z)
         o = step.scratch("rec_out", (T, self.width), torch.float32)
         ops.decay_recurrence(rkvg[0], rkvg[1], rkvg[2], z, self.decay_bias, self.bonus,
                              cache.state, step.state_slots, step.q_start, o, s.n_heads,
                              s.head_dim, s.head_dim, "double_exp", max_q_len=step.max_q_len)
-        mixed = step.scratch("rec_mixed", (T, self.width), act)
         ops.head_norm_gate(o, self.gain, rkvg[3], mixed, s.n_heads, float(s.norm_eps))
         self.o.forward(mixed, residual, accumulate=True, step=step)
 
