@@ -167,6 +167,7 @@ TESTED_AGAINST = {
     "decay_step": "plain_nupovik.py:decayed_outer_recurrence",
     "head_norm_gate": "test_nupovik_kernels_gpu.py:test_head_norm_gate",
     "streams_step": "plain_kugisun.py:stream_step",
+    "delta_step": "plain_kugisun.py:short_convolution",
     "short_conv": "plain_kugisun.py:short_convolution",
     "delta_recurrence": "plain_kugisun.py:delta_rule",
     "rotation_table": "plain_fumanex.py:rotate", "fixed_decay": "plain_fumanex.py:decayed_sums",

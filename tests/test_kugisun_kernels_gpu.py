@@ -450,6 +450,50 @@ def test_delta_rule_in_chunks_keeps_what_is_not_finite_from_the_tokens_before(wh
     assert torch.equal(got[0][before], clean[0][before]) and before[:token].all()
 
 
+@pytest.mark.parametrize("n,H,KH,d,dv,taps", [(1, 1, 1, 8, 1, 1), (8, 16, 8, 128, 128, 4), (5, 6, 2, 64, 50, 3),
+                                              (3, 4, 1, 128, 128, 2), (2, 3, 3, 16, 33, 8), (17, 32, 16, 32, 64, 4)])
+def test_a_decode_step_in_one_kernel(n, H, KH, d, dv, taps):
+    """Three single tokens behind each other against the convolutions, the delta rule and the norm one after the
+    other: 32-bit sums in another order (1e-5 of the largest state), outputs rounded to bfloat16 last.  Slots nobody
+    named stay."""
+    dt = torch.bfloat16
+    C, need = 2 * KH * d + H * dv, ops.delta_state_size(H, d, dv)
+    conv_at = (need + 3) // 4 * 4
+    width = (conv_at + (taps - 1) * C + 3) // 4 * 4
+    assert ops.delta_step_sizes(H, KH, d, dv)
+    w = _rand((C, taps), 1, 0.5).to(DEV)
+    a_log, dt_bias = _rand((H,), 2, 0.5).to(DEV), _rand((H,), 3, 0.5).to(DEV)
+    gain = (_rand((dv,), 4, 0.1) + 1.0).to(DEV)
+    state = _rand((n + 2, width), 5, 0.3).to(DEV)
+    slots, starts = _i32([(i + 1) % (n + 2) for i in range(n)]), _i32(list(range(n + 1)))
+    seq = _i32(list(range(n)))
+    states = [state.clone(), state.clone()]
+    for token in range(3):
+        proj = _rand((n, C + H * dv), 10 + token, 1.0, dt).to(DEV)
+        ab = _rand((n, 2 * H), 20 + token).to(DEV)
+        want, got = (torch.full((n, H * dv), float("nan"), dtype=dt, device=DEV) for _ in range(2))
+        qkv, o = torch.empty((n, C), device=DEV), torch.empty((n, H * dv), device=DEV)
+        ops.short_conv(proj, w, states[0], conv_at, slots, seq, starts, qkv, unit_heads=2 * KH, head_dim=d,
+                       scaled_heads=KH, scale=0.125, unit_eps=1e-6, single_tokens=True)
+        ops.delta_recurrence(qkv, 0, KH * d, 2 * KH * d, ab, a_log, dt_bias, states[0], slots, starts, o, H,
+                             KH, d, dv)
+        ops.head_norm_gate(o, gain, proj[:, C:], want, H, 1e-6)
+        ops.delta_step(proj, w, ab, a_log, dt_bias, states[1], conv_at, slots, gain, proj[:, C:], got, H, KH,
+                       d, dv, 0.125, 1e-6, 1e-6)
+        assert rel_err(states[1], states[0]) <= 1e-5
+        assert rel_err(got, want) <= tol(dt)
+        assert float((got != want).float().mean()) <= 0.02
+    assert torch.equal(states[1][:, conv_at:], states[0][:, conv_at:])
+    named = set(slots.tolist())
+    for row in set(range(n + 2)) - named:
+        assert torch.equal(states[1][row], state[row])
+
+
+def test_delta_step_refuses_what_it_does_not_take():
+    for H, KH, d, dv in ((3, 2, 64, 64), (4, 2, 24, 64), (4, 2, 256, 64), (16, 1, 128, 128), (8, 1, 64, 255)):
+        assert not ops.delta_step_sizes(H, KH, d, dv)
+
+
 def test_a_token_far_back_is_kept_without_decay_and_lost_with_it():
     """Two heads, 600 tokens.  Token 3 alone writes the key e_0 with a value that stands out;
     the last token asks for e_0.  The head whose decay is 1 to rounding (a rate of exp(-30))

@@ -28,6 +28,7 @@ template <typename TO> __device__ __forceinline__ float dl_silu_to(float z) {
     return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
   return dl_silu(z);
 }
+#define DL_STEP_TAPS 8          // most taps of a decode step in one kernel
 __device__ __forceinline__ float dl_softplus(float z) {
   return z > 20.f ? z : log1pf(expf(z));
 }
@@ -642,6 +643,176 @@ extern "C" int zf_delta_recurrence(const float* qkv, int C, int q_off, int k_off
   DL_REC_LAUNCH(8, 4) DL_REC_LAUNCH(12, 4) DL_REC_LAUNCH(8, 8) DL_REC_LAUNCH(12, 8)
   DL_REC_LAUNCH(8, 16) DL_REC_LAUNCH(12, 16) DL_REC_LAUNCH(16, 16)
   if (!launched) return -2;
+  ZF_CHECK_LAUNCH();
+}
+
+// ------------------------------------------------------------------ a decode step, whole
+// One token a sequence (bfloat16 rows): a workgroup a (q/k head, sequence) runs the convolutions of its channels
+// and moves their kept rows on, makes q and k unit vectors, walks the token for the value heads that share them,
+// norms each of these and applies gain and gate.  As three kernels a layer of 8 tokens took 4.7 + 9.8 + 4.6 us for
+// 16 heads of 128 x 128 on 8, each waiting for its first loads; here the matrices are asked for ahead of all else:
+// 10.7 us; 1 to 64 sequences gain 1 to 7 % of a pass of four layers.  Thread (vl, cg) = (tid / CG, tid % CG) holds the channels 8 cg .. + 8 of RV neighbouring
+// columns of the heads side by side; CG = d / 8.
+struct DeltaStep {
+  const bf16_t *src, *gate;
+  const float *taps, *ab, *a_log, *dt_bias, *gain;
+  float* state;
+  const int* state_slots;
+  bf16_t* out;
+  long long src_stride, gate_stride, out_stride, state_stride, conv_at;
+  int n_taps, H, KH, d, dv, CG;
+  float scale, unit_eps, norm_eps;
+};
+template <int RV>
+__global__ __launch_bounds__(1024) void delta_step_kernel(DeltaStep p) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  __shared__ float s_unit[3];               // 1 / |q| times the scale, 1 / |k|, q . k of the unit vectors
+  const int d = p.d, dv = p.dv, HG = p.H / p.KH, N = HG * dv, C = 2 * p.KH * d + p.H * dv, CG = p.CG;
+  float* qs = lds;                          // [d]
+  float* ks = qs + d;
+  float* vs = ks + d;                       // [N]
+  float* os = vs + N;                       // [N]
+  float* gs = os + N;                       // [HG] decay
+  float* bs = gs + HG;                      // [HG] step size
+  const int kh = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, nt = blockDim.x;
+  const int wave = tid / ZF_WAVE, lane = tid % ZF_WAVE, waves = nt / ZF_WAVE;
+  float* slot = p.state + (size_t)p.state_slots[s] * p.state_stride;
+  const int cg = tid % CG, col = tid / CG * RV;
+  const bool live = col < N;                // (dv is a multiple of RV: a thread's columns are one head's)
+  float* S_mem = slot + ((size_t)kh * N + (live ? col : 0)) * d + cg * 8;
+  float S[RV][8];
+#pragma unroll
+  for (int r = 0; r < RV; ++r) {
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+    if (live) {
+      a = *(const float4*)(S_mem + (size_t)r * d);
+      b = *(const float4*)(S_mem + (size_t)r * d + 4);
+    }
+    S[r][0] = a.x; S[r][1] = a.y; S[r][2] = a.z; S[r][3] = a.w;
+    S[r][4] = b.x; S[r][5] = b.y; S[r][6] = b.z; S[r][7] = b.w;
+  }
+  const int hist = p.n_taps - 1;
+  for (int i = tid; i < 2 * d + N; i += nt) {
+    const int c = i < d ? kh * d + i : i < 2 * d ? p.KH * d + kh * d + i - d : 2 * p.KH * d + kh * N + i - 2 * d;
+    const float x = bf16_to_float(p.src[(size_t)s * p.src_stride + c]);
+    float* kept = slot + p.conv_at + c;
+    float w[DL_STEP_TAPS - 1];
+#pragma unroll
+    for (int k = 0; k < DL_STEP_TAPS - 1; ++k) w[k] = k < hist ? kept[(size_t)k * C] : 0.f;
+    float acc = 0.f;
+#pragma unroll
+    for (int k = 0; k < DL_STEP_TAPS - 1; ++k)
+      if (k < hist) {
+        acc += p.taps[(size_t)c * p.n_taps + k] * w[k];
+        kept[(size_t)k * C] = k + 1 < hist ? w[k + 1 < DL_STEP_TAPS - 1 ? k + 1 : k] : x;
+      }
+    acc += p.taps[(size_t)c * p.n_taps + hist] * x;
+    lds[i] = dl_silu_to<float>(acc);        // q, k and v side by side
+  }
+  for (int j = tid; j < HG; j += nt) {
+    const int h = kh * HG + j;
+    const float* z = p.ab + (size_t)s * 2 * p.H;
+    gs[j] = expf(-(expf(p.a_log[h]) * dl_softplus(z[h] + p.dt_bias[h])));
+    bs[j] = 1.0f / (1.0f + expf(-z[p.H + h]));
+  }
+  __syncthreads();
+  if (wave == 0) {
+    float qq = 0.f, kk = 0.f, qk = 0.f;
+    for (int c = lane; c < d; c += ZF_WAVE) {
+      qq = fmaf(qs[c], qs[c], qq);
+      kk = fmaf(ks[c], ks[c], kk);
+      qk = fmaf(qs[c], ks[c], qk);
+    }
+    qq = wave_sum(qq);
+    kk = wave_sum(kk);
+    qk = wave_sum(qk);
+    if (lane == 0) {
+      const float iq = 1.0f / sqrtf(qq + p.unit_eps) * p.scale, ik = 1.0f / sqrtf(kk + p.unit_eps);
+      s_unit[0] = iq;
+      s_unit[1] = ik;
+      s_unit[2] = qk * iq * ik;
+    }
+  }
+  __syncthreads();
+  if (live) {
+    const float iq = s_unit[0], ik = s_unit[1], qk = s_unit[2];
+    const int j = col / dv;
+    const float g = gs[j], b = bs[j];
+    float k8[8], rs[RV], ps[RV];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) k8[e] = ks[cg * 8 + e] * ik;
+#pragma unroll
+    for (int r = 0; r < RV; ++r) {
+      float r0 = 0.f, r1 = 0.f, p0 = 0.f, p1 = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        r0 = fmaf(k8[e], S[r][e], r0);
+        r1 = fmaf(k8[e + 1], S[r][e + 1], r1);
+        p0 = fmaf(qs[cg * 8 + e], S[r][e], p0);
+        p1 = fmaf(qs[cg * 8 + e + 1], S[r][e + 1], p1);
+      }
+      rs[r] = r0 + r1;
+      ps[r] = p0 + p1;
+    }
+    lanes_sum_up(rs, CG);
+    lanes_sum_up(ps, CG);
+#pragma unroll
+    for (int r = 0; r < RV; ++r) {
+      const float w = b * (vs[col + r] - g * rs[r]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) S[r][e] = g * S[r][e] + k8[e] * w;
+      if (cg == 0) os[col + r] = g * (ps[r] * iq) + qk * w;
+      *(float4*)(S_mem + (size_t)r * d) = make_float4(S[r][0], S[r][1], S[r][2], S[r][3]);
+      *(float4*)(S_mem + (size_t)r * d + 4) = make_float4(S[r][4], S[r][5], S[r][6], S[r][7]);
+    }
+  }
+  __syncthreads();
+  for (int j = wave; j < HG; j += waves) {
+    float ss = 0.f;
+    for (int x = lane; x < dv; x += ZF_WAVE) ss = fmaf(os[j * dv + x], os[j * dv + x], ss);
+    const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)dv + p.norm_eps);
+    const size_t at = (size_t)(kh * HG + j) * dv;
+    for (int x = lane; x < dv; x += ZF_WAVE) {
+      const float gv = bf16_to_float(p.gate[(size_t)s * p.gate_stride + at + x]);
+      p.out[(size_t)s * p.out_stride + at + x] =
+          float_to_bf16(os[j * dv + x] * inv * p.gain[x] * (gv * (1.0f / (1.0f + expf(-gv)))));
+    }
+  }
+}
+
+// Columns a thread, 0: not these sizes.
+static int delta_step_columns(int H, int KH, int d, int dv) {
+  const int CG = d / 8;
+  if (H < 1 || KH < 1 || H % KH != 0 || d % 8 != 0 || CG < 1 || CG > 16 || (CG & (CG - 1)) != 0 || dv < 1)
+    return 0;
+  for (int rv = 1; rv <= 8; rv *= 2)
+    if (dv % rv == 0 && (long long)(H / KH) * dv / rv * CG <= 1024) return rv;
+  return 0;
+}
+
+// A step of one token a sequence: src bfloat16 rows [n_seqs, >= C], taps [C][n_taps]; the convolutions' kept rows
+// at conv_at of a slot, behind the matrices; slots 16-byte aligned.  gain [dv], gate and out rows [H dv].
+extern "C" int zf_delta_step(const void* src, long long src_stride, const float* taps, int n_taps,
+                             const float* ab, const float* a_log, const float* dt_bias, float* state,
+                             long long state_stride, long long conv_at, const int* state_slots,
+                             const float* gain, const void* gate, long long gate_stride, void* out,
+                             long long out_stride, int n_seqs, int H, int KH, int d, int dv, float scale,
+                             float unit_eps, float norm_eps, hipStream_t stream) {
+  if (n_seqs <= 0) return 0;
+  const int rv = delta_step_columns(H, KH, d, dv);
+  if (rv == 0 || n_taps < 1 || n_taps > DL_STEP_TAPS || state_stride % 4 != 0 || (uintptr_t)state % 16 != 0)
+    return -2;
+  const int HG = H / KH, N = HG * dv;
+  const DeltaStep p{(const bf16_t*)src, (const bf16_t*)gate, taps, ab, a_log, dt_bias, gain, state, state_slots,
+                    (bf16_t*)out, src_stride, gate_stride, out_stride, state_stride, conv_at, n_taps, H, KH, d, dv,
+                    d / 8, scale, unit_eps, norm_eps};
+  const int threads = (N / rv * (d / 8) + ZF_WAVE - 1) / ZF_WAVE * ZF_WAVE;
+  const size_t smem = (size_t)(2 * d + 2 * N + 2 * HG) * sizeof(float);
+  const dim3 grid(KH, n_seqs);
+  if (rv == 1) hipLaunchKernelGGL(delta_step_kernel<1>, grid, dim3(threads), smem, stream, p);
+  else if (rv == 2) hipLaunchKernelGGL(delta_step_kernel<2>, grid, dim3(threads), smem, stream, p);
+  else if (rv == 4) hipLaunchKernelGGL(delta_step_kernel<4>, grid, dim3(threads), smem, stream, p);
+  else hipLaunchKernelGGL(delta_step_kernel<8>, grid, dim3(threads), smem, stream, p);
   ZF_CHECK_LAUNCH();
 }
 

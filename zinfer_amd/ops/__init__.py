@@ -3533,6 +3533,58 @@ def delta_state_matrix(state: torch.Tensor, n_heads: int, key_dim: int,
     return m[..., :key_dim].transpose(2, 3).contiguous()
 
 
+DELTA_STEP_THREADS = 1024
+
+
+def delta_step_sizes(n_heads: int, n_kv_heads: int, key_dim: int, value_dim: int) -> bool:
+    """The heads that ``delta_step`` takes: key sizes of 8 to 128, a power of two, and value heads of a q/k
+    head whose columns a workgroup holds."""
+    lanes = key_dim // 8
+    return n_kv_heads > 0 and n_heads % n_kv_heads == 0 and key_dim % 8 == 0 and 0 < lanes <= 16 \
+        and lanes & (lanes - 1) == 0 and any(
+            value_dim % rv == 0 and n_heads // n_kv_heads * value_dim // rv * lanes <= DELTA_STEP_THREADS
+            for rv in (1, 2, 4, 8))
+
+
+def delta_step_covers(n_heads: int, n_kv_heads: int, key_dim: int, value_dim: int,
+                      src: torch.Tensor, state: torch.Tensor) -> bool:
+    """Whether ``delta_step`` takes a step of single tokens of such heads."""
+    return src.is_cuda and src.dtype == torch.bfloat16 and state.stride(0) % 4 == 0 \
+        and state.data_ptr() % 16 == 0 and delta_step_sizes(n_heads, n_kv_heads, key_dim, value_dim)
+
+
+@_launches("attention")
+def delta_step(src: torch.Tensor, taps: torch.Tensor, ab: torch.Tensor, a_log: torch.Tensor,
+               dt_bias: torch.Tensor, state: torch.Tensor, conv_offset: int,
+               state_slots: torch.Tensor, gain: torch.Tensor, gate: torch.Tensor, out: torch.Tensor,
+               n_heads: int, n_kv_heads: int, key_dim: int, value_dim: int, scale: float,
+               unit_eps: float, norm_eps: float) -> None:
+    """A step of one token a sequence (row s is sequence s's) in one kernel: ``short_conv`` of the leading columns
+    of ``src`` [T, >= C] bfloat16 (q and k heads as unit vectors, q times ``scale``), ``delta_recurrence`` and
+    ``head_norm_gate`` (silu) into ``out``; the convolutions' kept rows lie at ``conv_offset`` of a slot."""
+    _need_gpu(taps, ab, a_log, dt_bias, state, state_slots, gain)
+    _i32(state_slots, "state_slots")
+    T, H, KH, d, dv = src.shape[0], int(n_heads), int(n_kv_heads), int(key_dim), int(value_dim)
+    C = 2 * KH * d + H * dv
+    if not delta_step_covers(H, KH, d, dv, src, state) or src.shape[1] < C or taps.dim() != 2 \
+            or taps.shape[0] != C or not 1 <= taps.shape[1] <= SHORT_CONV_MAX_TAPS \
+            or ab.shape != (T, 2 * H) or a_log.shape != (H,) or dt_bias.shape != (H,) or gain.shape != (dv,) \
+            or any(t.dtype != torch.float32 or not t.is_contiguous() for t in (taps, ab, a_log, dt_bias, gain)) \
+            or any(t.shape != (T, H * dv) or t.dtype != torch.bfloat16 or not t.is_cuda for t in (gate, out)) \
+            or state.dtype != torch.float32 or state.dim() != 2 or state_slots.shape[0] != T \
+            or conv_offset < delta_state_size(H, d, dv) \
+            or state.shape[1] < conv_offset + (taps.shape[1] - 1) * C:
+        raise KernelUnavailable(f"delta_step: src {tuple(src.shape)} {src.dtype}, taps {tuple(taps.shape)}, "
+                                f"state {tuple(state.shape)} for {H} heads of {d} x {dv} on {KH}")
+    at = lambda t: ctypes.c_longlong(_columns(t, "delta_step"))
+    lib = build.load("delta")
+    _check(lib.zf_delta_step(
+        _ptr(src), at(src), _ptr(taps), taps.shape[1], _ptr(ab), _ptr(a_log), _ptr(dt_bias), _ptr(state),
+        ctypes.c_longlong(state.stride(0)), ctypes.c_longlong(conv_offset), _ptr(state_slots), _ptr(gain),
+        _ptr(gate), at(gate), _ptr(out), at(out), T, H, KH, d, dv, ctypes.c_float(scale),
+        ctypes.c_float(unit_eps), ctypes.c_float(norm_eps), _stream()), "delta_step")
+
+
 @_launches("norm_rope_write")
 def short_conv(src: torch.Tensor, taps: torch.Tensor, state: torch.Tensor, state_offset: int,
                state_slots: torch.Tensor, seq_index: torch.Tensor, q_start: torch.Tensor,

@@ -10,7 +10,7 @@ from dataclasses import dataclass
 from typing import Callable, Dict
 
 from . import (gated_act, moe_grouped, norm_add_norm, tied_attention_mfma)
-from . import delta_recurrence, short_conv, streams_step
+from . import delta_recurrence, delta_step, short_conv, streams_step
 from . import add_row, bias_act_rows, fixed_decay, rotation_table
 from . import embed_norm, gate_norm, gated_rows, gemm_geglu, state_space
 from . import (concat_rows, decay_recurrence, decay_step, embed_sinusoid, head_norm_gate, token_shift_mix)
@@ -126,6 +126,8 @@ KERNELS: Dict[str, KernelEntry] = {
                                 "is read from them and normed"),
     "short_conv": KernelEntry(short_conv, "delta", "own: causal convolutions over time a channel "
                               "with silu and unit heads, the last rows kept as state"),
+    "delta_step": KernelEntry(delta_step, "delta", "own: a decode step's convolutions, delta rule, norm and "
+                              "gate"),
     "delta_recurrence": KernelEntry(delta_recurrence, "delta", "own: a matrix a head, decayed "
                                     "and corrected towards every token's value"),
     "rotation_table": KernelEntry(rotation_table, "fixed_decay", "own: cosines and sines a token"),

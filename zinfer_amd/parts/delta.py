@@ -17,7 +17,8 @@ class GatedDeltaRule(Mixer):
     its accumulators as 32-bit numbers.  One kernel runs the short convolutions with their silu
     from the product's rows and the request's last rows, makes q and k unit vectors and scales
     q, all in 32-bit; the recurrence kernel forms decay and step size a head and token and walks
-    the step's tokens; one more kernel norms each head and applies gain and gate.  A request's
+    the step's tokens; one more kernel norms each head and applies gain and gate.  (Single tokens under
+    bfloat16: all of it in one kernel.)  A request's
     state slot holds the matrices and, behind them, the convolutions' last rows (32-bit)."""
     graph_safe = True
     stores_output = True
@@ -105,6 +106,14 @@ class GatedDeltaRule(Mixer):
         proj, ab = rows
         T = proj.shape[0]
         QK, V = self.qk_width, self.v_width
+        mixed = step.scratch("delta_mixed", (T, V), self.ctx.act_dtype)
+        if proj.is_cuda and step.max_q_len == 1 and T == step.state_slots.shape[0] and ops.delta_step_covers(
+                s.n_heads, s.n_kv_heads, s.head_dim, s.value_dim, proj, cache.state):
+            ops.delta_step(proj, self.taps, ab, self.decay_log, self.decay_bias, cache.state, self.matrix_size,
+                           step.state_slots, self.gain, proj[:, 2 * QK + V:], mixed, s.n_heads,
+                           s.n_kv_heads, s.head_dim, s.value_dim, self.q_scale, float(s.unit_eps),
+                           float(s.norm_eps))
+            return mixed
         qkv = step.scratch("delta_qkv", (T, self.conv_width), torch.float32)
         ops.short_conv(proj, self.taps, cache.state, self.matrix_size, step.state_slots,
                        step.seq_index, step.q_start, qkv, unit_heads=2 * s.n_kv_heads,
@@ -115,7 +124,6 @@ class GatedDeltaRule(Mixer):
                              step.state_slots, step.q_start, o, s.n_heads, s.n_kv_heads,
                              s.head_dim, s.value_dim,
                              q_lens=self._portions(step))
-        mixed = step.scratch("delta_mixed", (T, V), self.ctx.act_dtype)
         ops.head_norm_gate(o, self.gain, proj[:, 2 * QK + V:], mixed, s.n_heads,
                            float(s.norm_eps))
         return mixed

@@ -41,7 +41,8 @@ class GatedLinearAttention(Mixer):
     numbers z = W_a2 (W_a1 h) leave their product as 32-bit numbers, and the recurrence kernel
     turns them into decays, walks the step's tokens (long portions in spans side by side) and
     keeps every request's matrices in its state slot (32-bit); one more kernel norms each head,
-    applies the gain and the gate."""
+    applies the gain and the gate.  (Single tokens under bfloat16: from the decay's narrow middle on in one
+    kernel.)"""
     graph_safe = True
     kernel_modules = ("gemm", "recurrent")
 
