@@ -85,6 +85,25 @@ def test_embed_position(dt):
     assert rel_err(out, ref) < 1e-6
 
 
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("H,off", [(2048, 0), (8, 0), (50, 0), (2056, 1), (4104, 0)])
+def test_embed_position_in_wide_loads_and_in_copies(H, off, dt):
+    """Rows whose width or place keeps 8 columns a thread out, and every copy of a stream kept several times:
+    the same bits everywhere."""
+    E, Pt = _rand((9, H), 6, dtype=dt), _rand((7, H), 7, dtype=dt)
+    ids, pos = torch.tensor([8, 0, 3], dtype=torch.int32), torch.tensor([6, 0, 5], dtype=torch.int32)
+    flat = torch.empty((9 * H + off,), dtype=dt, device=DEV)
+    table = flat[off:].view(9, H)
+    table.copy_(E)
+    out = torch.full((4, 3, H), float("nan"), device=DEV)
+    ops.embed_position(table, ids.to(DEV), Pt.to(DEV), pos.to(DEV), out, 1.5)
+    one = torch.full((3, H), float("nan"), device=DEV)
+    ops.embed_position(table, ids.to(DEV), Pt.to(DEV), pos.to(DEV), one, 1.5)
+    ref = E.double()[ids.long()] * 1.5 + Pt.double()[pos.long()]
+    assert rel_err(one, ref) < 1e-6
+    assert all(torch.equal(out[c], one) for c in range(4))
+
+
 # ------------------------------------------------------------------------------ experts
 @pytest.mark.parametrize("T, W, E, top", [(7, 48, 6, 2), (3, 50, 1, 1), (5, 72, 9, 9),
                                            (4, 64, 130, 70), (2, 384, 12, 5)])

@@ -97,7 +97,9 @@ extern "C" int zf_embed(const void* table, int table_dtype, const int* ids, floa
 
 // ---------------------------------------------------------------- embedding plus a computed position vector
 // x[t, 2i] = E[id[t], 2i] + sin(p f_i), x[t, 2i + 1] = E[id[t], 2i + 1] + cos(p f_i) with
-// p = positions[t] and the angle p * f_i formed in 32-bit; freq [ceil(H / 2)] float32
+// p = positions[t] and the angle p * f_i formed in 32-bit; freq [ceil(H / 2)] float32.  A pair of columns a
+// thread: a decode step's few rows wait for one sine, not for four behind each other (16 rows of 2048
+// columns 6.4 -> 3.1 us).
 template <typename TW>
 __global__ void embed_sinusoid_kernel(const TW* __restrict__ table, const int* __restrict__ ids,
                                       const int* __restrict__ positions,
@@ -107,23 +109,24 @@ __global__ void embed_sinusoid_kernel(const TW* __restrict__ table, const int* _
   const TW* row = table + (size_t)ids[t] * H;
   float* o = out + (size_t)t * H;
   const float p = (float)positions[t];
-  for (int i = threadIdx.x; i < (H + 1) / 2; i += blockDim.x) {
-    float sn, cs;
-    sincosf(p * freq[i], &sn, &cs);
-    o[2 * i] = load_as_float<TW>(row + 2 * i) * scale + sn;
-    if (2 * i + 1 < H) o[2 * i + 1] = load_as_float<TW>(row + 2 * i + 1) * scale + cs;
-  }
+  const int i = blockIdx.y * blockDim.x + threadIdx.x;
+  if (i >= (H + 1) / 2) return;
+  float sn, cs;
+  sincosf(p * freq[i], &sn, &cs);
+  o[2 * i] = load_as_float<TW>(row + 2 * i) * scale + sn;
+  if (2 * i + 1 < H) o[2 * i + 1] = load_as_float<TW>(row + 2 * i + 1) * scale + cs;
 }
 
 extern "C" int zf_embed_sinusoid(const void* table, int table_dtype, const int* ids,
                                  const int* positions, const float* freq, float* out, int T,
                                  int H, float scale, hipStream_t stream) {
   if (T <= 0) return 0;
+  const dim3 grid(T, ((H + 1) / 2 + 255) / 256);
   if (table_dtype == ZF_F32)
-    hipLaunchKernelGGL(embed_sinusoid_kernel<float>, dim3(T), dim3(256), 0, stream,
+    hipLaunchKernelGGL(embed_sinusoid_kernel<float>, grid, dim3(256), 0, stream,
                        (const float*)table, ids, positions, freq, out, H, scale);
   else
-    hipLaunchKernelGGL(embed_sinusoid_kernel<bf16_t>, dim3(T), dim3(256), 0, stream,
+    hipLaunchKernelGGL(embed_sinusoid_kernel<bf16_t>, grid, dim3(256), 0, stream,
                        (const bf16_t*)table, ids, positions, freq, out, H, scale);
   ZF_CHECK_LAUNCH();
 }

@@ -183,8 +183,9 @@ class DecoderModel:
                                                      float(s.embedding_multiplier), x, first, out):
                 step.norm_ready = NormedRows(first, x, out)
         elif self.position_table is not None:
-            ops.embed_position(self.embedding, step.token_ids, self.position_table,
-                               step.positions, x, float(s.embedding_multiplier))
+            # (into every copy of the stream)
+            ops.embed_position(self.embedding, step.token_ids, self.position_table, step.positions,
+                               x if copies is None else copies, float(s.embedding_multiplier))
         elif self.position_freq is not None:
             ops.embed_sinusoid(self.embedding, step.token_ids, step.positions,
                                self.position_freq, x, float(s.embedding_multiplier))
@@ -201,8 +202,9 @@ class DecoderModel:
             x0 = step.scratch("embedding_out", (T, s.hidden_size), torch.float32)
             x0.copy_(x)
         if copies is not None:
-            for c in range(1, s.streams):
-                copies[c].copy_(x)
+            if self.position_table is None or self.embedding_norm is not None:
+                for c in range(1, s.streams):
+                    copies[c].copy_(x)
             x = copies
         in_one = self.one_launch is not None and self.one_launch.takes(self, step, caches, step.norm_ready)
         if in_one:

@@ -1868,20 +1868,23 @@ def embed_norm(table: torch.Tensor, ids: torch.Tensor, gain: torch.Tensor, eps: 
 @_launches("other")
 def embed_position(table: torch.Tensor, ids: torch.Tensor, pos_table: torch.Tensor,
                    positions: torch.Tensor, out: torch.Tensor, scale: float = 1.0) -> None:
-    """out[t, :] = table[ids[t], :] * scale + pos_table[positions[t], :], in float32."""
+    """out[t, :] = table[ids[t], :] * scale + pos_table[positions[t], :], in float32; ``out`` [S, T, H]: in
+    every one of its S copies."""
     _need_gpu(table, ids, pos_table, positions, out)
     _i32(ids, "ids")
     _i32(positions, "positions")
-    T, H = out.shape
+    copies = out.shape[0] if out.dim() == 3 else 1
+    T, H = out.shape[-2:]
     if table.shape[1] != H or pos_table.shape[1] != H or table.dtype != pos_table.dtype \
-            or ids.shape[0] != T or positions.shape[0] != T or out.dtype != torch.float32:
+            or ids.shape[0] != T or positions.shape[0] != T or out.dtype != torch.float32 \
+            or (copies > 1 and not out.is_contiguous()):
         raise KernelUnavailable(f"embed_position: table {tuple(table.shape)} {table.dtype}, "
                                 f"positions' table {tuple(pos_table.shape)} {pos_table.dtype}, "
                                 f"out {tuple(out.shape)} {out.dtype}")
     lib = build.load("norms")
     _check(lib.zf_embed_position(_ptr(table), _ptr(pos_table), _dt(table), _ptr(ids),
-                                 _ptr(positions), _ptr(out), T, H, ctypes.c_float(scale),
-                                 _stream()), "embed_position")
+                                 _ptr(positions), _ptr(out), T, H, ctypes.c_float(scale), copies,
+                                 ctypes.c_longlong(T * H), _stream()), "embed_position")
 
 
 # ------------------------------------------------------------------------- attention whose values are its keys
