@@ -450,6 +450,24 @@ def test_delta_rule_in_chunks_keeps_what_is_not_finite_from_the_tokens_before(wh
     assert torch.equal(got[0][before], clean[0][before]) and before[:token].all()
 
 
+@pytest.mark.parametrize("S,T,W", [(2, 8, 2048), (4, 1, 4096), (4, 3, 50), (8, 5, 68)])
+def test_the_final_norm_of_a_streams_last_step(S, T, W):
+    """The kernel that lets the last sublayer join the copies norms their sum as the sum's own kernel and the norm
+    behind it do: the squares' sum in another order, then one rounding to bfloat16."""
+    x = [(t := _rand((S, T, W), 1).to(DEV)), t.clone()]
+    y, gain = _rand((T, W), 2).to(DEV), (_rand((W,), 3, 0.1) + 1.0).to(DEV)
+    mix, out_coef = _rand((S, S), 4, 0.5).to(DEV), _rand((S,), 5).to(DEV)
+    want, got = (torch.empty((T, W), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    total = torch.empty((T, W), device=DEV)
+    ops.streams_step(x[0], [(y, 1.5)], mix, out_coef)
+    ops.streams_step(x[0], read=True, out=total)
+    ops.norm_rows(total, gain, None, 1e-6, want, False)
+    ops.streams_step(x[1], [(y, 1.5)], mix, out_coef, read=True, gain=gain, eps=1e-6, out=got)
+    assert torch.equal(x[0], x[1])
+    assert rel_err(got, want) <= tol(torch.bfloat16)
+    assert float((got != want).float().mean()) <= 0.01
+
+
 @pytest.mark.parametrize("n,H,KH,d,dv,taps", [(1, 1, 1, 8, 1, 1), (8, 16, 8, 128, 128, 4), (5, 6, 2, 64, 50, 3),
                                               (3, 4, 1, 128, 128, 2), (2, 3, 3, 16, 33, 8), (17, 32, 16, 32, 64, 4)])
 def test_a_decode_step_in_one_kernel(n, H, KH, d, dv, taps):

@@ -229,7 +229,8 @@ class DecoderModel:
             if self.layer_probe is not None:
                 self.layer_probe(pos, x if copies is None else self._sum(copies, step))
         left, step.norm_ready, step.norm_after_block = step.norm_ready, None, None
-        if copies is not None:
+        if copies is not None and not (isinstance(left, NormedRows) and step.wants_all_rows
+                                       and left.fits(self.final_norm, copies)):
             x, left = self._sum(copies, step), None
         n_rows = step.n_want
         logits = step.scratch("logits", (n_rows, s.vocab_size), torch.float32)

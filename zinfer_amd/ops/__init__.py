@@ -110,8 +110,8 @@ class kernel_class:
 
 
 def measures_classes() -> bool:
-    """Whether a per-class measurement is running (``only_classes``)."""
-    return _class_filter is not None
+    """Whether kernels of some classes are left out (``only_classes``)."""
+    return _class_filter is not None and _class_filter != frozenset(KERNEL_CLASSES)
 
 
 def _left_out(cls: str) -> bool:

@@ -552,12 +552,16 @@ class StreamBlock(Block):
                 reader = self.read_args(c + 1)
             else:
                 reader = after.read_args(0) if isinstance(after, StreamBlock) else None
+                if type(after) is LayerNorm and after.plain and act == torch.bfloat16 and x.dim() == 3:
+                    # (the final norm, of rows that all go to the head: the copies' sum is its alone)
+                    reader = dict(in_coef=None, gain=after.gain, eps=float(after.spec.eps))
             if reader is not None:
                 # (the sublayer is done with the buffer its input lay in)
                 h = step.scratch("normed_ff" if c % 2 == 0 else "normed", (T, W), act)
                 ops.streams_step(xs, branches, mix, out_coef, read=True, out=h, **reader)
                 if c + 1 == len(sublayers):
-                    handed = StreamRead(after, x, h)
+                    handed = StreamRead(after, x, h) if isinstance(after, StreamBlock) \
+                        else NormedRows(after, x, h)
             else:
                 ops.streams_step(xs, branches, mix, out_coef)
         step.norm_after = None
