@@ -1,10 +1,10 @@
 // All layers of a decoder in one launch, for a decode step of very few tokens (pre-norm layers:
 // RMSNorm, grouped-query attention with normed and rotated heads, RMSNorm, SwiGLU; bfloat16).
 //
-// In launches of their own a layer's ten kernels each ramp up and drain while memory idles (28 us a layer
-// of the 0.6B shape, whose 31 MB of weights take 4.5 at 7 TB/s; 90 of 55 at the 8B shape).  Here a layer
-// takes 14 us and 75: the weights, and where these are few the five times that rows travel between all
-// workgroups (2.4 us each).  Decode steps of one token of Qwen3 shapes behind 120 tokens, four layers and
+// In launches of their own a layer's six kernels each ramp up and drain while memory idles (26 us a layer
+// of the 0.6B shape, whose 31 MB of weights take 4.5 at 7 TB/s; 81 of 55 at the 8B shape).  Here a layer
+// takes 15 us and 69: the weights, and where these are few the five times that rows travel between all
+// workgroups (1.9 us each, the words' way alone).  Decode steps of one token of Qwen3 shapes behind 120 tokens, four layers and
 // the head, before and after: 0.6B 197 -> 164 us, 1.7B 285 -> 244, 4B 372 -> 350, 8B 560 -> 527; from
 // 14B on the launches' ends are small beside the weights (800 -> 795).  Two tokens 0.6B 196 -> 168, 8B 542 ->
 // 521; three 200 -> 179, 547 -> 535; four tokens of the 0.6B and 1.7B shapes 202 -> 187 and 291 -> 273: what the
@@ -376,8 +376,8 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
     look();
     const uint32_t lane_at = lane * 16;
     constexpr int NT = 2;           // read once
-    // two batches of pairs of tiles (three pairs a batch: 12 KB a wave under way; four and six were slower
-    // by 1 and 3 % on the narrow shapes, whose phases end within a batch)
+    // two batches of pairs of tiles (three pairs a batch, 24 KB a wave under way: one user of the 0.6B and
+    // 8B shapes 17.3 and 138.0 ms; two pairs 17.8 and 138.3, four 17.7 and 139.0)
     u32x4_t w0[2][BATCH][2], w1[2][BATCH][2];
     auto ask = [&](int b) __attribute__((always_inline)) {
       if (left <= 0) next_run();
