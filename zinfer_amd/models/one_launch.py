@@ -99,8 +99,7 @@ class OneLaunchLayers:
         M = x.shape[0]
         words = step.made(f"decode_words.{M}", lambda device: kernel.words(
             M, self.hidden, self.ff, self.heads, self.kv_heads, device))
-        status = step.made(STATUS, lambda device: torch.zeros((1,), dtype=torch.int32,
-                                                                      pin_memory=True))
+        status = step.made(STATUS, lambda device: torch.zeros((1,), dtype=torch.int32, pin_memory=True))
         kernel.decode_layers(
             self._table(model, step, caches), len(caches), x, given.xg, given.sq, self.ff, self.heads,
             self.kv_heads, cache.page_size, float(b.mixer_norm.spec.eps), float(b.ff_norm.spec.eps),

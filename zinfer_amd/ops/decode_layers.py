@@ -89,7 +89,11 @@ def decode_layers(table: torch.Tensor, n_layers: int, x: torch.Tensor, xg: torch
             or sq.dtype != torch.float32 or sq.shape != (H // 16, 16) or ctx_len.shape[0] != M \
             or block_table.shape[0] != M or positions.shape[0] != M or slot_mapping.shape[0] != M \
             or table.numel() != n_layers * ctypes.sizeof(Layer) \
-            or block_table.shape[1] * page_size > MAX_CONTEXT or (cos is None) != (sin is None):
+            or block_table.shape[1] * page_size > MAX_CONTEXT or (cos is None) != (sin is None) \
+            or any(t is not None and (t.dtype != torch.float32 or t.shape != cos.shape
+                                      or t.shape[1] != HEAD_DIM // 2 or not t.is_contiguous())
+                   for t in (cos, sin)) \
+            or not all(t.is_contiguous() for t in (x, xg, sq, block_table)):
         raise KernelUnavailable(f"decode_layers: x {tuple(x.shape)}, ff {ff}, {n_heads} heads on "
                                 f"{n_kv_heads}, tables {tuple(block_table.shape)} of {page_size} rows")
     for t, name in ((positions, "positions"), (slot_mapping, "slot_mapping"),
