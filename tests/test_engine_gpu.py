@@ -701,3 +701,40 @@ def test_debug_tables_finds_a_page_that_is_not_the_pools(tmp_path_factory):
     eng.cache.set_table_entry(0, "x", 1, eng.cache.groups[0].pages.num_pages + 7)
     with pytest.raises(StepError, match=r"BlockTableOutOfBounds: group 0, sequence 1, page index 1"):
         eng.step([StepEntry("y", [5], [0]), StepEntry("x", [6], [0])])
+
+
+def test_no_garbage_is_collected_while_a_graph_is_recorded(tmp_path_factory, monkeypatch):
+    """An engine in a reference cycle holds graphs when another engine records its own, and a collection is
+    due with every allocation."""
+    import gc
+    import weakref
+    from zinfer_amd.engine import StepEntry
+    from zinfer_amd.engine.replay import make_engine
+    path, _, requests, _ = _setup("D", "bfloat16", tmp_path_factory)
+    toks = requests["r1"]
+    first, second = (make_engine(path, "bfloat16", 64, DEV) for _ in range(2))
+    for eng in (first, second):
+        eng.step([StepEntry("r", toks[:3], [2])])
+    want = first.step([StepEntry("r", toks[3:4], [0])]).cpu()
+    assert first.graph_replays + len(first._graphs) > 0
+    first.cycle, gone, thresholds, recorded = first, weakref.ref(first), gc.get_threshold(), []
+    forward = second.model.forward
+
+    def under_pressure(ctx, views):
+        if torch.cuda.is_current_stream_capturing():
+            recorded.append(gone() is not None)
+            gc.set_threshold(1, 1, 1)
+            kept = [[i] for i in range(100)]
+            recorded.append(gone() is not None and len(kept) == 100)
+        return forward(ctx, views)
+
+    monkeypatch.setattr(second.model, "forward", under_pressure)
+    gc.set_threshold(1 << 30)
+    try:
+        del eng, first
+        got = second.step([StepEntry("r", toks[3:4], [0])]).cpu()
+    finally:
+        gc.set_threshold(*thresholds)
+    assert recorded == [True, True] and torch.equal(got, want) and gc.isenabled()
+    gc.collect()
+    assert gone() is None

@@ -8,6 +8,9 @@ are kept as errors raised before anything is launched: a token id beyond the voc
 """
 from __future__ import annotations
 
+import contextlib
+import gc
+import threading
 from typing import Dict, List, Optional, Sequence
 
 import numpy as np
@@ -24,6 +27,29 @@ from .batch import KVStepTables, Scratch, StepContext, StepEntry
 
 def _pad4(n: int) -> int:
     return (n + 3) // 4 * 4
+
+
+_recordings = [0, False]        # under way; whether garbage was collected before the first of them
+_recordings_lock = threading.Lock()
+
+
+@contextlib.contextmanager
+def recording(graph):
+    """``torch.cuda.graph`` with no garbage collected meanwhile: of an engine in a reference cycle it would
+    end the graphs, which waits for the device, and that aborts the process while a graph is recorded."""
+    with _recordings_lock:
+        if _recordings[0] == 0:
+            _recordings[1] = gc.isenabled()
+            gc.disable()
+        _recordings[0] += 1
+    try:
+        with torch.cuda.graph(graph):
+            yield
+    finally:
+        with _recordings_lock:
+            _recordings[0] -= 1
+            if _recordings[0] == 0 and _recordings[1]:
+                gc.enable()
 
 
 class Engine:
@@ -340,7 +366,7 @@ class Engine:
                     graph = torch.cuda.CUDAGraph()
                     capturing[0] = True
                     try:
-                        with torch.cuda.graph(graph):
+                        with recording(graph):
                             run_steps()
                     finally:
                         capturing[0] = False
@@ -397,7 +423,7 @@ class Engine:
                 stream.synchronize()
                 graph = torch.cuda.CUDAGraph()
                 with ops.only_classes(only):
-                    with torch.cuda.graph(graph):
+                    with recording(graph):
                         self.model.forward(ctx, self.views)
                 graph.replay()
                 before = torch.cuda.Event(enable_timing=True)
@@ -463,7 +489,7 @@ class Engine:
             self._graphs.pop(next(iter(self._graphs)))
         torch.cuda.current_stream(self.device).synchronize()
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
+        with recording(graph):
             logits = self.model.forward(ctx, self.views)
         self._graphs[key] = (graph, logits, self._generations())
         graph.replay()
