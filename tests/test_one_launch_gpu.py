@@ -213,3 +213,107 @@ def test_a_failed_wait_is_an_error_of_the_next_step():
     with pytest.raises(StepError, match="hear"):
         eng.step([StepEntry("r", [5], [0])])
     assert eng.length("r") == 4
+
+
+def _flag(eng):
+    eng._scratch.kept(one_launch.STATUS)[0] = 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("reader", ["argmax", "to_host", "sample"])
+def test_a_step_that_failed_is_taken_back_where_the_host_waits_for_it(reader):
+    """(the flag set by the host, between the launch and the wait)  The step's request holds what it held
+    before, and the same step then gives the same bits."""
+    from zinfer_amd import ops
+    from zinfer_amd.engine import StepEntry
+    from zinfer_amd.errors import StepError
+    cfg = _qwen3(512, 4, 2, 512)
+    eng = _engine(cfg, _weights(cfg, 7), tokens=128)
+    eng.argmax(eng.step([StepEntry("r", [1, 2, 3], [2])]))
+    want = eng.to_host(eng.step([StepEntry("r", [4], [0])])).clone()
+    logits = eng.step([StepEntry("r", [5], [0]), StepEntry("new", [9], [0])])
+    records = np.zeros((2,), dtype=ops.SAMPLE_ROW_DTYPE)
+    records[:] = (1.0, 1.0, 0.0, 1, 0.0)
+    _flag(eng)
+    with pytest.raises(StepError, match="hear"):
+        eng.sample(logits, records) if reader == "sample" else getattr(eng, reader)(logits)
+    assert eng.length("r") == 4 and not eng.has_request("new")
+    eng.release("r")
+    eng.argmax(eng.step([StepEntry("r", [1, 2, 3], [2])]))
+    assert torch.equal(eng.to_host(eng.step([StepEntry("r", [4], [0])])), want)
+
+
+@pytest.mark.gpu
+def test_runs_of_steps_that_failed_return_no_tokens(monkeypatch):
+    """The flag set while the steps run: as one graph and one by one."""
+    from zinfer_amd import ops
+    from zinfer_amd.engine import StepEntry
+    from zinfer_amd.errors import StepError
+    cfg = _qwen3(512, 4, 2, 512)
+    eng = _engine(cfg, _weights(cfg, 7), tokens=128)
+    eng.argmax(eng.step([StepEntry("r", [1, 2, 3], [2])]))
+    pages = eng.cache.num_free_pages()
+    go = lambda: eng.decode_steps([StepEntry("r", [4], [0])], 8)
+    want = go()
+    eng.release("r")
+    for run in range(4):
+        eng.argmax(eng.step([StepEntry("r", [1, 2, 3], [2])]))
+        with monkeypatch.context() as m:
+            upload = eng._upload
+            m.setattr(eng, "_upload", lambda host: (upload(host), _flag(eng))[0])
+            with pytest.raises(StepError, match="hear"):
+                go()
+        assert eng.length("r") == 3 and eng.cache.num_free_pages() == pages
+        assert go() == want
+        eng.release("r")
+    assert eng.graph_replays > 8
+
+
+@pytest.mark.gpu
+def test_requests_of_a_failed_step_that_nobody_waited_for_can_only_be_released():
+    from zinfer_amd.engine import StepEntry
+    from zinfer_amd.errors import StepError
+    cfg = _qwen3(512, 4, 2, 512)
+    eng = _engine(cfg, _weights(cfg, 7), tokens=128)
+    for r in ("r", "s"):
+        eng.argmax(eng.step([StepEntry(r, [1, 2, 3], [2])]))
+    eng.step([StepEntry("r", [4], [0])])
+    torch.cuda.synchronize()
+    _flag(eng)
+    with pytest.raises(StepError, match="hear"):
+        eng.step([StepEntry("s", [5], [0])])
+    with pytest.raises(StepError, match="released"):
+        eng.step([StepEntry("r", [5], [0])])
+    assert np.isfinite(eng.to_host(eng.step([StepEntry("s", [5], [0])])).numpy()).all()
+    eng.release("r")
+    assert len(eng.argmax(eng.step([StepEntry("r", [5], [0])]))) == 1
+
+
+@pytest.mark.gpu
+def test_the_scheduler_accepts_no_token_of_a_failed_step(monkeypatch):
+    from zinfer_amd.engine.scheduler import Scheduler
+    from zinfer_amd.errors import StepError
+    from zinfer_amd.sampling import SamplingParams
+    cfg = _qwen3(512, 4, 2, 512)
+    eng = _engine(cfg, _weights(cfg, 7), tokens=128)
+    answers = []
+    for spoiled in (False, True):
+        for multi, top_k in ((1, 1), (4, 1), (1, 5000)):
+            sched = Scheduler(eng, multi_step=multi)
+            sched.add_request([1, 2, 3], SamplingParams(
+                temperature=0.0 if top_k == 1 else 0.7, top_k=top_k, seed=3, max_new_tokens=9, ignore_eos=True))
+            req = sched.waiting[-1]
+            sched.step()
+            if spoiled:
+                sched.step()
+                had = list(req.generated)
+                upload = eng._upload
+                monkeypatch.setattr(eng, "_upload", lambda host: (upload(host), _flag(eng))[0])
+                with pytest.raises(StepError, match="hear"):
+                    sched.step()
+                monkeypatch.setattr(eng, "_upload", upload)
+                assert list(req.generated) == had
+            while not req.finished:
+                sched.step()
+            answers.append(list(req.generated))
+    assert answers[:3] == answers[3:]

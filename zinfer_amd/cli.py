@@ -432,7 +432,7 @@ def cmd_probe_model(args: List[str]) -> int:
     from .engine import StepEntry
     model_dir, _, (token, top_k), opt = _probe_args(args, 2, (0, 8))
     llm = _llm(model_dir, opt, max_tokens=64)
-    logits = llm.engine.step([StepEntry("probe", [token], [0])], end=["probe"])[0]
+    logits = llm.engine.to_host(llm.engine.step([StepEntry("probe", [token], [0])], end=["probe"]))[0]
     top = logits.topk(min(top_k, logits.numel()))
     print("Zinfer model probe")
     print(f"token_id: {token}")

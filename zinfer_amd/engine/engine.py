@@ -85,6 +85,10 @@ class Engine:
         # pool before its kernels run (one small kernel and a wait for its report a step)
         self.debug_tables = debug_tables and self.device.type == "cuda"
         self._scratch = Scratch(self.device)
+        # by the cache's number of a request: what it held before the steps whose waits between
+        # workgroups (one_launch) nobody has looked behind yet; and requests that such a step spoiled
+        self._unheard: Dict[int, int] = {}
+        self._lost: set = set()
         self._meta_host = None          # two pinned buffers that take turns
         self._meta_dev: Optional[torch.Tensor] = None
         self._meta_generation = 0
@@ -122,8 +126,11 @@ class Engine:
         [number of wanted places, vocab] in the order of the entries and of their ``want``.
         Requests in ``end`` give back what they hold after the step.  On an error the cache
         is as before: what can be refused is refused before anything runs, and a failure
-        inside the run gives back what the step had reserved."""
-        self._check_waits()
+        inside the run gives back what the step had reserved.  (A decode step whose workgroups did
+        not hear from each other leaves rows of NaN.  ``argmax``, ``sample`` and ``to_host`` raise then,
+        and its requests hold what they held before it; whoever reads the rows in another way hears of
+        it with the next step, and its requests can only be released.)"""
+        self._check_waits(waited=False)
         seen, wanted_len = self._check_entries(entries)
         for rid in end:
             if rid not in seen and not self.cache.has_request(rid):
@@ -156,6 +163,13 @@ class Engine:
             except BaseException:
                 self._roll_back(wanted_len, added)
                 raise
+            if self.model.one_launch is not None and ctx.max_q_len == 1 \
+                    and ctx.n_seqs <= one_launch.kernel.MAX_TOKENS:
+                live = self.cache.requests
+                if len(self._unheard) > 2 * len(live) + 64:       # (most of them released)
+                    self._unheard = {n: self._unheard[n] for n in live.values() if n in self._unheard}
+                for rid, new_len in wanted_len:
+                    self._unheard.setdefault(live[rid], new_len - 1)
             for rid, new_len in wanted_len:
                 self.cache.commit(rid, new_len)
             self.steps_run += 1
@@ -275,6 +289,9 @@ class Engine:
                 if not (0 <= int(w) < n):
                     raise StepError(f"request {e.request_id!r}: want {w} outside its {n} tokens")
             start = self.cache.length(e.request_id) if self.cache.has_request(e.request_id) else 0
+            if self._lost and self.cache.requests.get(e.request_id) in self._lost:
+                raise StepError(f"request {e.request_id!r} was in a decode step that failed: it can only "
+                                "be released")
             if start + n + extra > spec.max_positions:
                 raise PositionOutOfBounds(
                     f"PositionOutOfBounds: request {e.request_id!r} would reach position "
@@ -300,7 +317,7 @@ class Engine:
             raise StepError("decode_steps: every entry brings one token and wants its logits")
         if records is not None and records.shape != (n_steps, n):
             raise StepError(f"decode_steps: records must be [{n_steps}, {n}]")
-        self._check_waits()
+        self._check_waits(waited=False)
         extra = n_steps - 1
         _, wanted_len = self._check_entries(entries, extra)
         if not self.cache.can_reserve(wanted_len):
@@ -380,6 +397,7 @@ class Engine:
                 self._trace((n * n_steps, n, t1 - t0, time.perf_counter() - t1, before, after,
                              False))
             tokens = out.tolist()
+            self._check_waits(waited=True)
         except BaseException:
             self._roll_back(wanted_len, added)
             raise
@@ -452,11 +470,34 @@ class Engine:
         for pool, index, rows in saved:
             pool.index_copy_(0, index, rows)
 
-    def _check_waits(self) -> None:
-        """Raises once a kernel whose workgroups wait for each other has given up (its rows are NaN)."""
+    def _check_waits(self, waited: bool) -> None:
+        """Raises if a kernel whose workgroups wait for each other has given up (its rows are NaN).
+        ``waited``: the host has just waited for every step; a step that failed is then taken back."""
         status = self._scratch.kept(one_launch.STATUS)
-        if status is not None and int(status[0]) != 0:
+        if status is None:
+            return
+        if int(status[0]) == 0:
+            if waited:
+                self._unheard.clear()
+            return
+        torch.cuda.current_stream(self.device).synchronize()
+        status[0] = 0
+        spoiled, self._unheard = self._unheard, {}
+        if not waited:
+            self._lost = {n for n in self._lost | set(spoiled) if n in self.cache.requests.values()}
             raise StepError("the workgroups of an earlier decode step did not hear from each other")
+        live = {number: rid for rid, number in self.cache.requests.items()}
+        for number, length in spoiled.items():
+            rid = live.get(number)
+            if rid is None:
+                continue
+            if length == 0:
+                self.cache.release(rid)
+            else:
+                self.cache.commit(rid, length)
+                self.cache.trim(rid)
+        raise StepError("the workgroups of a decode step did not hear from each other; its requests hold "
+                        "what they held before it")
 
     def _generations(self) -> tuple:
         from .. import ops
@@ -503,7 +544,15 @@ class Engine:
             return []
         out = self._scratch.get("argmax", (n,), torch.int32)
         ops.argmax(logits, out)
-        return out.tolist()
+        tokens = out.tolist()
+        self._check_waits(waited=True)
+        return tokens
+
+    def to_host(self, logits: torch.Tensor) -> torch.Tensor:
+        """``logits`` in 32-bit on the host."""
+        rows = logits.detach().to("cpu", torch.float32)
+        self._check_waits(waited=True)
+        return rows
 
     def sample(self, logits: torch.Tensor, records, penalties=None) -> List[int]:
         """Draws one token per row on the device.  ``records`` is a numpy array of
@@ -522,7 +571,9 @@ class Engine:
         rec = torch.from_numpy(records.view(np.uint8).reshape(-1).copy()).to(dev)
         out = self._scratch.get("sampled", (n,), torch.int32)
         ops.sample_topk(logits, rec, out)
-        return out.tolist()
+        tokens = out.tolist()
+        self._check_waits(waited=True)
+        return tokens
 
     # ------------------------------------------------------------------ metadata
     def _build_context(self, entries: Sequence[StepEntry], bucket_pages: bool = False,

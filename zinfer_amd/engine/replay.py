@@ -88,7 +88,7 @@ def run_trace(engine: Engine, lines, out_dir: str, report=None) -> int:
                                      [int(w) for w in e.get("want", [])]))
         logits = engine.step(entries, end=obj.get("end", []))
         if logits.shape[0] > 0:
-            arr = logits.detach().to("cpu", torch.float32).numpy().astype("<f4", copy=False)
+            arr = engine.to_host(logits).numpy().astype("<f4", copy=False)
             arr.tofile(os.path.join(out_dir, f"{step}.f32"))
         n += 1
         if report is not None:

@@ -364,7 +364,8 @@ class Scheduler:
         if hasattr(self.engine, "sample") and all(
                 sp.greedy or 1 <= sp.top_k <= 1024 for sp in params):
             return self._sample_on_device(logits, sampling)
-        rows = logits.detach().to("cpu", torch.float32).numpy()
+        to_host = getattr(self.engine, "to_host", lambda t: t.detach().to("cpu", torch.float32))
+        rows = to_host(logits).numpy()
         out = []
         for i, p in enumerate(sampling):
             req = p.request
