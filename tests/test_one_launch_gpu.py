@@ -317,3 +317,77 @@ def test_the_scheduler_accepts_no_token_of_a_failed_step(monkeypatch):
                 sched.step()
             answers.append(list(req.generated))
     assert answers[:3] == answers[3:]
+
+
+# (width, heads, kv heads, feed-forward, page), prompts' lengths, numbers of workgroups: one alone; a few; one less
+# than hold a phase's sums, by its products or (the first) by its splits of contexts
+FEW = [((512, 4, 4, 512, 16), (1500, 1410, 40, 1300), (1, 3, 31)), ((576, 15, 1, 1088, 48), (140, 33, 12), (2, 27)),
+       ((832, 4, 4, 832, 16), (262, 40), (1, 11)), ((1024, 16, 8, 3072, 16), (133,), (1, 15)),
+       ((4096, 32, 8, 12288, 16), (530,), (5, 23))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,lengths,numbers", FEW, ids=str)
+def test_fewer_workgroups_than_hold_a_phase_give_the_same_bits(shape, lengths, numbers, monkeypatch):
+    """Workgroups that are too few for a phase's sums take it a piece at a time."""
+    hidden, heads, kv, ff, page = shape
+    cfg = _qwen3(hidden, heads, kv, ff)
+    w = _weights(cfg, hidden + heads)
+    requests = {f"r{i}": tiny.random_tokens(n, cfg["vocab_size"], n) for i, n in enumerate(lengths)}
+    want = _together(_engine(cfg, w, page, tokens=8192), requests, 5)
+    monkeypatch.setattr(kernel, "sizes_covered", lambda *sizes: True)
+    for n in numbers:
+        monkeypatch.setattr(kernel, "workgroups", lambda index: n)
+        monkeypatch.setattr(one_launch.OneLaunchLayers, "forward", _counted(calls := []))
+        got = _together(_engine(cfg, w, page, tokens=8192), requests, 5)
+        assert len(calls) >= 2
+        for r in requests:
+            assert np.array_equal(got[r], want[r]), (n, r)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lengths", [(70,), (133, 10, 300, 31)], ids=str)
+def test_workgroups_that_do_not_wait_for_the_others_give_the_same_bits(lengths, monkeypatch):
+    """The meeting closes as soon as one has come: as many do the step as came by then."""
+    cfg = _qwen3(1024, 16, 8, 3072)
+    w = _weights(cfg, 3)
+    requests = {f"r{i}": tiny.random_tokens(n, cfg["vocab_size"], n) for i, n in enumerate(lengths)}
+    want = _together(_engine(cfg, w), requests, 6)
+    monkeypatch.setattr(kernel, "MEET_TICKS", 0)
+    monkeypatch.setattr(kernel, "MEET_MOST", 0)
+    eng = _engine(cfg, w)
+    for _ in range(4):
+        got = _together(eng, requests, 6)
+        assert all(np.array_equal(got[r], want[r]) for r in requests)
+
+
+@pytest.mark.gpu
+def test_three_engines_that_need_more_than_a_third_of_the_workgroups_each():
+    """None of three launches that meet waits for what another holds: the same bits as alone."""
+    from zinfer_amd.engine import StepEntry
+    cfg = _qwen3(1024, 32, 8, 3072, layers=6)
+    w = _weights(cfg, 5)
+    requests = {f"r{i}": tiny.random_tokens(n, cfg["vocab_size"], n) for i, n in enumerate((40, 25, 61, 90))}
+    engines = [_engine(cfg, w, tokens=512) for _ in range(3)]
+    assert 3 * 96 > engines[0].model.one_launch.wgs >= 2 * 96       # (48 x 8 row groups of q, k and v, 4 a workgroup)
+    want = [_together(e, requests, 20) for e in engines][0]
+    for e in engines:
+        for r, t in requests.items():
+            e.step([StepEntry(r, t[:-20], [])])
+    torch.cuda.synchronize()
+    got = [{r: [] for r in requests} for _ in engines]
+
+    def go(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for k in range(20, 0, -1):
+                logits = engines[i].step([StepEntry(r, [t[-k]], [0]) for r, t in requests.items()])
+                rows = engines[i].to_host(logits).numpy()
+                for j, r in enumerate(requests):
+                    got[i][r].append(rows[j].copy())
+    threads = [threading.Thread(target=go, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for rows in got:
+        assert all(np.array_equal(np.stack(rows[r]), want[r]) for r in requests)

@@ -17,16 +17,21 @@
 // its sums, run norms, residual, activation and attention, and hand the result on.
 //
 // Rows travel between workgroups as words of 8 bytes, 4 of data and 4 that say of which layer they
-// are (`epoch`), written and read with relaxed 64-bit atomics at agent scope: a word that carries
-// the epoch carries its data, so a reader waits for the words themselves and nothing else orders the
-// workgroups.  A phase's words are overwritten a layer later at the earliest, and whoever is about
+// are (`epoch`): a word that carries the epoch carries its data, so a reader waits for the words
+// themselves and nothing else orders the workgroups.  They are written and read by buffer accesses of 8
+// or 16 bytes past the XCDs' own caches (sc1).  What this rests on: an aligned 8-byte half of such an
+// access arrives whole, and a reader's loads are issued anew at every look (an asm statement that may
+// change memory stands ahead of them, so that the compiler neither joins nor hoists them).  A phase's words are overwritten a layer later at the earliest, and whoever is about
 // to write them has read, directly or through others, what every workgroup made from the last
 // ones; two sets of words in turn leave another layer between.
 // Workgroups that are resident at once do the step: they arrive one after the other, and what there is
 // to do is dealt among those that have come when all have or, where another stream or process holds
-// CUs, DL_MEET later; whoever comes then leaves again.  So no workgroup waits for one that has no CU,
+// CUs, `meet_ticks` later; whoever comes then leaves again.  So no workgroup waits for one that has no CU,
 // whatever runs beside (a cooperative launch promises the same from a queue of its own: 15 us a step to
 // go there and back, and half a microsecond more for every later kernel of the process).
+// However few have come `meet_most` later, one included, do it: a launch that held CUs until it had more could
+// wait for another that does the same.  Fewer than `need`, whose shares would not fit a phase's sums, take
+// theirs a piece at a time (FEW, below), in the same order of sums.
 // Every wait ends: a reader that has looked DL_SPINS times gives up for its workgroup, which leaves
 // without handing on what it owes, so that the others leave in turn; the rows that go to the head are
 // then NaN and `status` is 1.
@@ -45,8 +50,6 @@
 #define DL_SPLIT 128             // keys a workgroup takes
 #define DL_PART (DL_HD + 2)      // words of a split's partial result: O, max, sum
 #define DL_SPINS (1 << 21)
-#define DL_MEET 5000             // ticks of 10 ns that the workgroups which have come wait for the others
-#define DL_MEET_MOST 1000000000  // and until a step that too few came to fails
 #define DL_CLOSED (1u << 31)
 #define DL_UNITS 16              // most units of 16 outputs a workgroup has in a phase, times tokens
 #define DL_FF_UNITS 32           // and at gate/up, where a unit is two row groups
@@ -95,7 +98,9 @@ struct DecodeLayers {
   float* sq;                     // [hidden / 16][16] the sums of x^2 over 16 columns, in place
   dl_word* words;                // zero at first
   DecodeMeet* meet;
-  int need;                      // workgroups that the sizes take at least
+  int need;                      // workgroups whose shares of a phase fit its sums
+  int meet_ticks;                // of 10 ns that the workgroups which have come wait for the others
+  int meet_most;                 // and while they are fewer than `need`
   int* status;
 };
 
@@ -204,20 +209,12 @@ __device__ __forceinline__ void dl_meet(const DecodeLayers& p, int& wg, int& wgs
     }
     __builtin_amdgcn_s_sleep(1);
     const long long waited = wall_clock64() - first;
-    if (waited < DL_MEET) continue;
+    if (waited < p.meet_ticks) continue;
     const unsigned come = dl_get(&meet->arrived);
-    if ((come & DL_CLOSED) || (come < (unsigned)p.need && waited < DL_MEET_MOST)) continue;
+    if ((come & DL_CLOSED) || (come < (unsigned)p.need && waited < p.meet_most)) continue;
     const unsigned n = __hip_atomic_fetch_or(&meet->arrived, DL_CLOSED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if ((n & DL_CLOSED) || n == all) continue;       // (another says, or the last to come does)
-    if (n < (unsigned)p.need) {
-      const int M = p.tokens;
-      for (int i = 0; i < M * p.hidden; ++i) {
-        p.x[i] = __uint_as_float(0x7fc00000u);
-        p.xg[i] = 0x7fc0;
-      }
-      __hip_atomic_store(p.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    dl_put(&meet->go, tag | (n < (unsigned)p.need ? 0u : n));
+    dl_put(&meet->go, tag | n);
   }
 }
 
@@ -252,33 +249,38 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
   auto count = [&](int first, int units) { return first < units ? (units - first + wgs - 1) / wgs : 0; };
   const int n_qkv = count(qkv_first, qkv_units), n_sum = count(wg, sum_units), n_ff = count(ff_first, ff_units);
 
-  if (tid < 64) {                 // the splits of contexts that are this workgroup's
-    int n = 0;
-    for (int item = wg; item < p.max_splits * M * p.nKV; item += wgs) {
-      const int kvh = item % p.nKV, s = (item / p.nKV) % M, sp = item / (p.nKV * M), ps = p.page_size;
-      const int ctx = p.ctx_len[s];
-      if (sp * DL_SPLIT >= ctx) continue;
-      if (tid < 8) {
-        const int kb = sp * DL_SPLIT + (tid / 2) * DL_WAVE_KEYS, end = min(ctx, kb + DL_WAVE_KEYS);
-        // (a group without a key may have no page: it reads the group of one that exists and is masked)
-        const int key = kb + 16 * (tid % 2) < end ? kb + 16 * (tid % 2) : kb;
-        sh.blk[n][tid / 2][tid % 2] = kb >= end ? 0
-            : (((size_t)p.block_table[(size_t)s * p.max_pages + key / ps] * p.nKV + kvh) * ps + key % ps) *
-                  DL_HD;
-      }
-      if (tid == 0) {
-        const int slot = p.slot_mapping[s], own = (ctx - 1) / DL_SPLIT == sp;
-        sh.item[n] = kvh | sp << 8 | s << 16 | own << 24;
-        // the row within the sixteen in the low bits
-        sh.put[n] = ((((size_t)(slot / ps) * p.nKV + kvh) * ps + (slot % ps) / 16 * 16) * DL_HD) |
-                    (size_t)(slot % 16);
-      }
-      ++n;
+  // split `item` of a context as entry n, by threads t = 0 .. 7; false: the context does not reach it
+  auto put_split = [&](int item, int n, int t) __attribute__((always_inline)) {
+    const int kvh = item % p.nKV, s = (item / p.nKV) % M, sp = item / (p.nKV * M), ps = p.page_size;
+    const int ctx = p.ctx_len[s];
+    if (sp * DL_SPLIT >= ctx) return false;
+    if (t < 8) {
+      const int kb = sp * DL_SPLIT + (t / 2) * DL_WAVE_KEYS, end = min(ctx, kb + DL_WAVE_KEYS);
+      // (a group without a key may have no page: it reads the group of one that exists and is masked)
+      const int key = kb + 16 * (t % 2) < end ? kb + 16 * (t % 2) : kb;
+      sh.blk[n][t / 2][t % 2] = kb >= end ? 0
+          : (((size_t)p.block_table[(size_t)s * p.max_pages + key / ps] * p.nKV + kvh) * ps + key % ps) *
+                DL_HD;
     }
+    if (t == 0) {
+      const int slot = p.slot_mapping[s], own = (ctx - 1) / DL_SPLIT == sp;
+      sh.item[n] = kvh | sp << 8 | s << 16 | own << 24;
+      // the row within the sixteen in the low bits
+      sh.put[n] = ((((size_t)(slot / ps) * p.nKV + kvh) * ps + (slot % ps) / 16 * 16) * DL_HD) |
+                  (size_t)(slot % 16);
+    }
+    return true;
+  };
+  const int n_splits = p.max_splits * M * p.nKV;
+  const bool few = wgs < p.need;
+  if (!few && tid < 64) {         // the splits of contexts that are this workgroup's
+    int n = 0;
+    for (int item = wg; item < n_splits; item += wgs)
+      if (put_split(item, n, tid)) ++n;
     if (tid == 0) sh.n_att = n;
   }
-  if (tid == 64) {
-    sh.dead = 0;
+  if (tid == 64) sh.dead = 0;
+  if (!few && tid == 64) {
     // in the order of the layer; `late` is the first run behind the attention (-1: there is none)
     int n = 0, late = -1;
     for (int m = 0; m < 4; ++m) {
@@ -304,10 +306,11 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
           (d < DL_HD / 2 ? p.cos_t : p.sin_t)[(size_t)row * (DL_HD / 2) + d % (DL_HD / 2)];
     }
   dl_barrier();
-  const int n_att = dl_uniform(sh.n_att);
+  const int n_att = few ? 0 : dl_uniform(sh.n_att);
   volatile __attribute__((address_space(3))) int* dead =
       (volatile __attribute__((address_space(3))) int*)&sh.dead;
 
+  if (few && wave < DL_CW) return;
   if (wave < DL_CW) {
     // ------------------------------------------------------------ streaming and multiplying
     const int lane = tid % 64, g = lane / 16, j = min(lane % 16, M - 1);
@@ -619,383 +622,457 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
   };
   // the stream's element it keeps
   auto column = [&](const Place& e) __attribute__((always_inline)) { return (wg + e.unit * wgs) * 16 + e.r; };
-  const bool keeps = place().unit < (uint32_t)n_sum;
-  float res = 0.f;
-  if (keeps) {
-    const Place e = place();
-    res = p.x[(size_t)e.tok * p.hidden + column(e)];
-    if constexpr (M > 1) sh.res[thread()] = res;
-  }
-  // The sum joins the stream's element, and what the next norm needs of the result goes to the words
-  // at `to` and `to_sq`, or (last) back to memory.
-  auto residual = [&](float gain, uint32_t to, uint32_t to_sq, unsigned epoch, bool last) __attribute__((always_inline)) {
-    if (!keeps) return;
-    const Place e = place();
-    const uint32_t e_r = e.r, e_tok = e.tok, keeps_at = column(e);
-    float now = M > 1 ? sh.res[thread()] : res;
-    now += sum_waves(e.pair, e_r);
-    if constexpr (M > 1) sh.res[thread()] = now;
-    else res = now;
-    const float sq = lanes_sum<16>(now * now);
-    uint32_t d0, d1;
-    quad_words(now * gain, e_r, d0, d1);
-    const uint32_t c = e_r % DL_COPIES;
-    const uint32_t row = (c * M + e_tok) * p.hidden + (keeps_at & ~3u);       // numbers, 4 a pair of words
-    if (!last) {
-      store2(row * 4, to * 16, d0, d1, epoch);
-      if (e_r < DL_COPIES)
-        __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{__float_as_uint(sq), epoch}, words,
-                                              ((e_r * M + e_tok) * groups + keeps_at / 16) * 8, to_sq * 16, SC1);
-      return;
-    }
-    const DecodeArgs pp = args();
-    const size_t n = (size_t)e_tok * p.hidden + keeps_at;
-    pp->x[n] = now;
-    if (c == 0) *(u32x2_t*)(pp->xg + n) = u32x2_t{d0, d1};
-    if (e_r == 0) pp->sq[(size_t)(keeps_at / 16) * 16 + e_tok] = sq;
-  };
-
-  bool split = false;             // a context of more than one split: the partials are merged
-  for (int s = 0; s < M; ++s) split = split || dl_const(p.ctx_len)[s] > DL_SPLIT;
-
-  // A split's part of the norm's gains and of the keys and values that the cache holds: asked for while
-  // the other waves run the down product of the layer before, behind whose loads they may wait.
-  f32x4_t g0 = f32x4_t{1.f, 1.f, 1.f, 1.f}, g1 = g0;
-  u32x4_t kf[2][DL_HD / 32];
-  u32x2_t vf[2][DL_HD / 16];
-  auto ask_keys = [&](int layer, int att) __attribute__((always_inline)) {
-    if (att >= n_att || layer >= n_layers) return;
-    DL_CONST DecodeLayer& L = dl_const(args()->layers)[layer];
-    const uint32_t t = thread(), lane = t % 64, l16 = t % 16;
-    const int item = dl_uniform(sh.item[att]);
-    const int kb = (item >> 8 & 255) * DL_SPLIT + cwave * DL_WAVE_KEYS;
-    if (L.q_gain != nullptr) {
-      const float* gain = (int)t / 16 < G ? L.q_gain : L.k_gain;
-      g0 = dl_global<f32x4_t>(gain + 4 * l16);
-      g1 = dl_global<f32x4_t>(gain + DL_HD / 2 + 4 * l16);
-    }
-    if (kb >= dl_const(p.ctx_len)[item >> 16 & 255]) return;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const u32x2_t b = *(const u32x2_t*)&sh.blk[att][cwave][h];
-      const size_t blk = ((size_t)(uint32_t)dl_uniform(b[0]) | (size_t)(uint32_t)dl_uniform(b[1]) << 32) * 2;
-#pragma unroll
-      for (int stp = 0; stp < DL_HD / 32; ++stp)
-        kf[h][stp] = dl_stream<u32x4_t>(L.k_pool, blk + stp * 1024, lane * 16);
-#pragma unroll
-      for (int dt = 0; dt < DL_HD / 16; ++dt)
-        vf[h][dt] = dl_stream<u32x2_t>(L.v_pool, blk + dt * 512, lane * 8);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  ask_keys(0, 0);
-
-  for (int layer = 0; layer < n_layers; ++layer) {
-    DL_CONST DecodeLayer& L = dl_const(args()->layers)[layer];
-    const unsigned epoch = base + layer + 1;
-    const uint32_t set = (epoch & 1) * at.all;
-    float ff_gain = 0.f, next_gain = 0.f;
-    if (keeps) {
-      const uint32_t at = column(place());
-      ff_gain = dl_global<float>(L.ff_gain + at);
-      next_gain = dl_global<float>(L.next_gain + at);
-    }
-    // ---- q, k and v
-    if (n_qkv > 0) {
-      const uint32_t t = thread();
-      if (layer == 0) {
-        const DecodeArgs pp = args();
-        const uint32_t per = p.hidden / 8;
-        for (uint32_t i = t; i < M * per; i += 256)
-          *(u32x4_t*)(s_rows + (size_t)(i / per) * row_bytes + (i % per) * 16) = *((const u32x4_t*)pp->xg + i);
-        for (uint32_t i = t; i < M * (uint32_t)groups; i += 256)
-          s_sq[i] = pp->sq[(size_t)(i % groups) * 16 + i / groups];
-      } else {
-        // (the rows the layer before left, under its own epoch)
-        const uint32_t before = ((epoch - 1) & 1) * at.all;
-        gather_normed(before + at.next, before + at.next_sq, epoch - 1);
-      }
-      dl_barrier();
-      float inv[M];
-      inv_rms(p.eps_in, inv);
-      const bool leave = dl_uniform(*dead) != 0;
-      dl_barrier();
-      if (leave) { dl_barrier(); break; }
+  // FEW: the workgroups are fewer than `need`.  These four waves do the products too, so many units of a
+  // phase at a time, and find their splits of contexts as they go; the other eight have left.
+  auto all_layers = [&](auto few_) __attribute__((always_inline)) {
+    constexpr bool FEW = decltype(few_)::value;
+    constexpr int PIECE = DL_UNITS / M, FF_PIECE = DL_FF_UNITS / M;
+    const bool keeps = place().unit < (uint32_t)n_sum;
+    float res = 0.f;
+    if (!FEW && keeps) {
       const Place e = place();
-      if (e.unit < (uint32_t)n_qkv) {
-        float f = inv[0];
-#pragma unroll
-        for (int tok = 1; tok < M; ++tok) f = e.tok == tok ? inv[tok] : f;
-        uint32_t d0, d1;
-        quad_words(sum_waves(e.pair, e.r) * f, e.r, d0, d1);
-        if (e.r % 4 == 0)
-          store2((e.tok * qkv_units + qkv_first + e.unit * wgs) * 64 + e.r * 4, (set + at.qkv) * 16, d0, d1,
-                 epoch);
-      }
-      dl_barrier();
+      res = p.x[(size_t)e.tok * p.hidden + column(e)];
+      if constexpr (M > 1) sh.res[thread()] = res;
     }
-    // ---- attention, a split of a context at a time
-    for (int att = 0; att < n_att; ++att) {
-      const uint32_t t = thread();
+    // The sum joins the stream's element, and what the next norm needs of the result goes to the words
+    // at `to` and `to_sq`, or (last) back to memory.  Of a piece the units from k0 on, whose elements lie
+    // in memory and whose gains are read here.
+    auto residual = [&](float gain, const float* gains, int k0, uint32_t to, uint32_t to_sq, unsigned epoch, bool last) __attribute__((always_inline)) {
+      Place e = place();
+      if (FEW ? e.unit >= (uint32_t)min(PIECE, n_sum - k0) : !keeps) return;
+      if constexpr (FEW) e.unit += k0;
+      const uint32_t e_r = e.r, e_tok = e.tok, keeps_at = column(e);
+      float* mine = FEW ? args()->x + (size_t)e_tok * args()->hidden + keeps_at : nullptr;
+      if constexpr (FEW) gain = dl_global<float>(gains + keeps_at);
+      float now = FEW ? *mine : M > 1 ? sh.res[thread()] : res;
+      now += sum_waves(e.pair, e_r);
+      if constexpr (FEW) *mine = now;
+      else if constexpr (M > 1) sh.res[thread()] = now;
+      else res = now;
+      const float sq = lanes_sum<16>(now * now);
+      uint32_t d0, d1;
+      quad_words(now * gain, e_r, d0, d1);
+      const uint32_t c = e_r % DL_COPIES;
+      const uint32_t row = (c * M + e_tok) * p.hidden + (keeps_at & ~3u);       // numbers, 4 a pair of words
+      if (!last) {
+        store2(row * 4, to * 16, d0, d1, epoch);
+        if (e_r < DL_COPIES)
+          __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{__float_as_uint(sq), epoch}, words,
+                                                ((e_r * M + e_tok) * groups + keeps_at / 16) * 8, to_sq * 16, SC1);
+        return;
+      }
       const DecodeArgs pp = args();
+      const size_t n = (size_t)e_tok * p.hidden + keeps_at;
+      pp->x[n] = now;
+      if (c == 0) *(u32x2_t*)(pp->xg + n) = u32x2_t{d0, d1};
+      if (e_r == 0) pp->sq[(size_t)(keeps_at / 16) * 16 + e_tok] = sq;
+    };
+
+    bool split = false;             // a context of more than one split: the partials are merged
+    for (int s = 0; s < M; ++s) split = split || dl_const(p.ctx_len)[s] > DL_SPLIT;
+
+    // A split's part of the norm's gains and of the keys and values that the cache holds: asked for while
+    // the other waves run the down product of the layer before, behind whose loads they may wait.
+    f32x4_t g0 = f32x4_t{1.f, 1.f, 1.f, 1.f}, g1 = g0;
+    u32x4_t kf[2][DL_HD / 32];
+    u32x2_t vf[2][DL_HD / 16];
+    auto ask_keys = [&](int layer, int att) __attribute__((always_inline)) {
+      if ((!FEW && att >= n_att) || layer >= n_layers) return;
+      DL_CONST DecodeLayer& L = dl_const(args()->layers)[layer];
+      const uint32_t t = thread(), lane = t % 64, l16 = t % 16;
       const int item = dl_uniform(sh.item[att]);
-      const int kvh = item & 255, sp = item >> 8 & 255, s = item >> 16 & 255;
-      const bool own = item >> 24;
-      const int ctx = dl_const(pp->ctx_len)[s], pos = ctx - 1;
-      const int lane = t % 64, j = lane % 16, qd = lane / 16;
-      const int kb = sp * DL_SPLIT + cwave * DL_WAVE_KEYS, k_end = min(ctx, kb + DL_WAVE_KEYS);
-      const bool has_keys = kb < k_end;
-      const int hi = t / 16, l16 = t % 16, n_items = own ? G + 1 : G;
-      // the head's words: elements 4 l16 .. + 3 and 64 further on; the new value: 8 elements a thread
-      const uint32_t row = (set + at.qkv + s * (qkv_units * 4)) * 16;
-      const uint32_t head_at = (hi < G ? kvh * G + hi : nH + kvh) * (DL_HD / 4 * 16) + l16 * 16;
-      u32x4_t r0, r1, v0, v1;
-      wait_for([&]() __attribute__((always_inline)) {
-        r0 = load2(head_at, row);
-        r1 = load2(head_at, row + DL_HD / 8 * 16);
-        const uint32_t bad = (r0[1] ^ epoch) | (r0[3] ^ epoch) | (r1[1] ^ epoch) | (r1[3] ^ epoch);
-        return hi < n_items && bad != 0;
-      });
-      if (own && cwave == 0) {
-        const uint32_t value_at = row + (nH + p.nKV + kvh) * (DL_HD / 4 * 16);
-        wait_for([&]() __attribute__((always_inline)) {
-          v0 = load2(l16 * 32, value_at);
-          v1 = load2(l16 * 32, value_at + 16);
-          return ((v0[1] ^ epoch) | (v0[3] ^ epoch) | (v1[1] ^ epoch) | (v1[3] ^ epoch)) != 0;
-        });
+      const int kb = (item >> 8 & 255) * DL_SPLIT + cwave * DL_WAVE_KEYS;
+      if (L.q_gain != nullptr) {
+        const float* gain = (int)t / 16 < G ? L.q_gain : L.k_gain;
+        g0 = dl_global<f32x4_t>(gain + 4 * l16);
+        g1 = dl_global<f32x4_t>(gain + DL_HD / 2 + 4 * l16);
       }
-      const size_t put = sh.put[att];
-      const int r = put % 16;
-      {
-        float x0[4], x1[4];
+      if (kb >= dl_const(p.ctx_len)[item >> 16 & 255]) return;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          x0[e] = bf16_to_float((bf16_t)(r0[2 * (e / 2)] >> (16 * (e % 2))));
-          x1[e] = bf16_to_float((bf16_t)(r1[2 * (e / 2)] >> (16 * (e % 2))));
-        }
-        HeadCoef cf;
-        cf.has_gain = L.q_gain != nullptr;
-        cf.has_rotation = p.cos_t != nullptr;
-        const f32x4_t c = *(const f32x4_t*)&sh.turn[s][0][4 * l16], sn = *(const f32x4_t*)&sh.turn[s][1][4 * l16];
+      for (int h = 0; h < 2; ++h) {
+        const u32x2_t b = *(const u32x2_t*)&sh.blk[att][cwave][h];
+        const size_t blk = ((size_t)(uint32_t)dl_uniform(b[0]) | (size_t)(uint32_t)dl_uniform(b[1]) << 32) * 2;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          cf.g0[e] = g0[e];
-          cf.g1[e] = g1[e];
-          cf.c[e] = c[e];
-          cf.sn[e] = sn[e];
-        }
-        head_norm_rotate<16>(x0, x1, DL_HD, true, pp->eps_head, cf);
-        if (hi < n_items) {
-          const u32x2_t y0 = u32x2_t{pack_bf16x2(x0[0], x0[1]), pack_bf16x2(x0[2], x0[3])};
-          const u32x2_t y1 = u32x2_t{pack_bf16x2(x1[0], x1[1]), pack_bf16x2(x1[2], x1[3])};
-          bf16_t* dst = sh.q[hi < G ? hi : 16];
-          *(u32x2_t*)(dst + 4 * l16) = y0;
-          *(u32x2_t*)(dst + DL_HD / 2 + 4 * l16) = y1;
-          if (hi == G) {          // element d of row r at [d / 32][16 ((d % 32) / 8) + r][d % 8]
-            auto* grp = (DL_GLOBAL bf16_t*)(uintptr_t)L.k_pool + (put & ~(size_t)15);
-            const int d0 = 4 * l16, at0 = (d0 / 32) * 512 + (((d0 % 32) / 8) * 16 + r) * 8 + d0 % 8;
-            *(DL_GLOBAL u32x2_t*)(grp + at0) = y0;
-            *(DL_GLOBAL u32x2_t*)(grp + at0 + (DL_HD / 64) * 512) = y1;
-          }
-        }
-        if (own && t < DL_HD / 8) {           // [d / 16][16 (r / 4) + d % 16][r % 4]
-          *(u32x4_t*)(sh.q[17] + 8 * l16) = u32x4_t{v0[0], v0[2], v1[0], v1[2]};
-          auto* grp = (DL_GLOBAL bf16_t*)(uintptr_t)L.v_pool + (put & ~(size_t)15) + (r / 4) * 64 + r % 4;
+        for (int stp = 0; stp < DL_HD / 32; ++stp)
+          kf[h][stp] = dl_stream<u32x4_t>(L.k_pool, blk + stp * 1024, lane * 16);
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const int d = 8 * l16 + i;
-            grp[(d / 16) * 256 + (d % 16) * 4] =
-                (bf16_t)((i < 4 ? v0 : v1)[(i / 2) % 2 * 2] >> (16 * (i % 2)));
-          }
-        }
+        for (int dt = 0; dt < DL_HD / 16; ++dt)
+          vf[h][dt] = dl_stream<u32x2_t>(L.v_pool, blk + dt * 512, lane * 8);
       }
-      dl_barrier();
-      float m = -INFINITY, l = 0.f;
-      f32x4_t o[DL_HD / 16];
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (!FEW) ask_keys(0, 0);
+    // The units [k0, k0 + n) of product m, which begin at `first`, into the sums: what the other eight waves do,
+    // two of them a wave.
+    auto multiply = [&](int layer, int m, int first, int k0, int n) __attribute__((always_inline)) {
+      const DecodeArgs pp = args();
+      DL_CONST DecodeLayer& L = dl_const(pp->layers)[layer];
+      const int lane = thread() % 64, per = (m == 1 ? nH * DL_HD : m == 3 ? pp->ff : pp->hidden) / 64;
+      for (int i = 0; i < (m == 2 ? 2 * n : n); ++i) {
+        const size_t rg = m == 2 ? 2 * (first + (k0 + i / 2) * wgs) + i % 2 : first + (k0 + i) * wgs;
+        for (int w = cwave; w < DL_CW; w += 4) {
+          const int tiles = (per - w + DL_CW - 1) / DL_CW;
+          const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(
+              (void*)((const char*)L.w[m] + (rg * per + w) * 2048), 0, max(per - w, 0) * 2048, 0x00020000);
+          const char* a = s_rows + (size_t)min(lane % 16, M - 1) * row_bytes + (lane / 16) * 32 + w * 128;
+          f32x4_t acc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+          constexpr int AHEAD = 8;
+          for (int t = 0; t < tiles; t += AHEAD) {
+            u32x4_t w0[AHEAD], w1[AHEAD];
 #pragma unroll
-      for (int dt = 0; dt < DL_HD / 16; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      if (has_keys) {
-        bf16x8_t qf[DL_HD / 32];
-#pragma unroll
-        for (int st = 0; st < DL_HD / 32; ++st) {
-          u32x4_t v = *(const u32x4_t*)(sh.q[min(j, G - 1)] + st * 32 + 8 * qd);
-          qf[st] = *(bf16x8_t*)&v;
-        }
-        // the token's own key and value, which the cache did not hold when it was read, where its lanes
-        // hold a key's elements 32 stp + 8 qd .. + 7 (lane j: key j of the group) and four keys' values
-        // (lane j: element 16 dt + j of keys 4 qd .. + 3)
-        if (pos >= kb && pos < kb + DL_WAVE_KEYS) {
-          const int jn = (pos - kb) % 16;
-          auto patch = [&](u32x4_t (&k)[DL_HD / 32], u32x2_t (&v)[DL_HD / 16]) __attribute__((always_inline)) {
-#pragma unroll
-            for (int stp = 0; stp < DL_HD / 32; ++stp) {
-              const u32x4_t kx = *(const u32x4_t*)(sh.q[16] + stp * 32 + 8 * qd);
-              if (j == jn) k[stp] = kx;
+            for (int b = 0; b < AHEAD; ++b) {
+              w0[b] = __builtin_amdgcn_raw_buffer_load_b128(from, lane * 16, (t + b) * DL_CW * 2048, 2);
+              w1[b] = __builtin_amdgcn_raw_buffer_load_b128(from, lane * 16 + 1024, (t + b) * DL_CW * 2048, 2);
             }
-            const uint32_t keep = jn % 2 ? 0x0000ffffu : 0xffff0000u;
 #pragma unroll
-            for (int dt = 0; dt < DL_HD / 16; ++dt) {
-              const uint32_t vn = (uint32_t)sh.q[17][16 * dt + j] << (16 * (jn % 2));
-              if (qd == jn / 4) {
-                if ((jn % 4) / 2 == 0) v[dt][0] = (v[dt][0] & keep) | vn;
-                else v[dt][1] = (v[dt][1] & keep) | vn;
+            for (int b = 0; b < AHEAD; ++b)
+              if (t + b < tiles) {
+                const u32x4_t a0 = *(const u32x4_t*)(a + (t + b) * DL_CW * 128);
+                const u32x4_t a1 = *(const u32x4_t*)(a + (t + b) * DL_CW * 128 + 16);
+                acc[b % 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&w0[b], *(const bf16x8_t*)&a0,
+                                                                     acc[b % 2], 0, 0, 0);
+                acc[b % 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&w1[b], *(const bf16x8_t*)&a1,
+                                                                     acc[b % 2], 0, 0, 0);
               }
-            }
-          };
-          if (pos - kb < 16) patch(kf[0], vf[0]);
-          else patch(kf[1], vf[1]);
+          }
+          if (lane % 16 < M) *(f32x4_t*)&sh.part[i * M + lane % 16][w][4 * (lane / 16)] = acc[0] + acc[1];
         }
-        float sc[8];
-        decode_scores<DL_HD, false, 2>(kf, qf, kb, kb, k_end, qd, p.scale_log2e, m, l, sc, -1, nullptr);
-        decode_values<DL_HD, false, 2>(vf, sc, kb, kb, k_end, qd, o, -1, nullptr);
       }
-      if (j < G) {
-#pragma unroll
-        for (int dt = 0; dt < DL_HD / 16; ++dt) *(f32x4_t*)&sh.o[cwave][j][dt * 16 + 4 * qd] = o[dt];
+    };
+
+    // false: given up
+    auto run_layer = [&](int layer) __attribute__((always_inline)) {
+      DL_CONST DecodeLayer& L = dl_const(args()->layers)[layer];
+      const unsigned epoch = base + layer + 1;
+      const uint32_t set = (epoch & 1) * at.all;
+      float ff_gain = 0.f, next_gain = 0.f;
+      if (!FEW && keeps) {
+        const uint32_t at = column(place());
+        ff_gain = dl_global<float>(L.ff_gain + at);
+        next_gain = dl_global<float>(L.next_gain + at);
       }
-      if (qd == 0) {
-        sh.m[cwave][j] = m;
-        sh.l[cwave][j] = l;
-      }
-      dl_barrier();
-      // a head a wave, two elements a lane
-      for (int col = cwave; col < G; col += 4) {
-        float pm[4], mx = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) pm[w] = sh.m[w][col];
-#pragma unroll
-        for (int w = 0; w < 4; ++w) mx = fmaxf(mx, pm[w]);
-        float a0 = 0.f, a1 = 0.f, den = 0.f;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {         // (a wave without keys has max -inf: weight 0)
-          const float f = exp2_raw(pm[w] - mx);
-          const float2 ov = *(const float2*)&sh.o[w][col][2 * lane];
-          a0 = fmaf(f, ov.x, a0);
-          a1 = fmaf(f, ov.y, a1);
-          den = fmaf(f, sh.l[w][col], den);
-        }
-        const int head = s * nH + kvh * G + col;
-        if (ctx <= DL_SPLIT) {
-          const uint32_t mine = pack_bf16x2(a0 / den, a1 / den);
-          const uint32_t other = __float_as_uint(lane_xor<1>(__uint_as_float(mine)));
-          const uint32_t d0 = lane % 2 ? other : mine, d1 = lane % 2 ? mine : other;
-          // copies lane % 2 and lane % 2 + 2
-          const uint32_t to = ((lane % 2) * M * nH * (DL_HD / 4) + head * (DL_HD / 4) + lane / 2) * 16;
-          store2(to, (set + at.attn) * 16, d0, d1, epoch);
-          store2(to, (set + at.attn + 2 * M * nH * (DL_HD / 4)) * 16, d0, d1, epoch);
+      // ---- q, k and v
+      if (n_qkv > 0) {
+        const uint32_t t = thread();
+        if (layer == 0) {
+          const DecodeArgs pp = args();
+          const uint32_t per = p.hidden / 8;
+          for (uint32_t i = t; i < M * per; i += 256)
+            *(u32x4_t*)(s_rows + (size_t)(i / per) * row_bytes + (i % per) * 16) = *((const u32x4_t*)pp->xg + i);
+          for (uint32_t i = t; i < M * (uint32_t)groups; i += 256)
+            s_sq[i] = pp->sq[(size_t)(i % groups) * 16 + i / groups];
         } else {
-          const uint32_t to = (set + at.part + (head * p.max_splits + sp) * (DL_PART / 2)) * 16;
-          store2(lane * 16, to, __float_as_uint(a0), __float_as_uint(a1), epoch);
-          if (lane == 0) store2(DL_HD / 2 * 16, to, __float_as_uint(mx), __float_as_uint(den), epoch);
+          // (the rows the layer before left, under its own epoch)
+          const uint32_t before = ((epoch - 1) & 1) * at.all;
+          gather_normed(before + at.next, before + at.next_sq, epoch - 1);
         }
-      }
-      ask_keys(layer, att + 1);
-      dl_barrier();               // (the next split's partial outputs go where these are)
-    }
-    // ---- contexts of several splits: eight elements of a head a wave, eight splits side by side
-    if (split) {
-      const int lane = thread() % 64, d8 = lane % 8, slot = lane / 8;
-      constexpr int pieces = DL_HD / 8;
-      for (int item = cwave * wgs + wg; item < M * nH * pieces; item += 4 * wgs) {
-        const int piece = item % pieces, head = item / pieces, s = M == 1 ? 0 : head / nH;
-        const int last = (dl_const(args()->ctx_len)[s] - 1) / DL_SPLIT;
-        if (last == 0) continue;
-        const uint32_t from = (set + at.part + head * p.max_splits * (DL_PART / 2)) * 16;
-        float mx = -INFINITY, acc = 0.f, den = 0.f;
-        for (int sp0 = 0; sp0 <= last; sp0 += 8) {
-          const uint32_t mine = min(sp0 + slot, last) * (DL_PART * 8);
-          u32x4_t ml;
-          u32x2_t v;
-          wait_for([&]() __attribute__((always_inline)) {
-            v = __builtin_amdgcn_raw_buffer_load_b64(words, mine + (piece * 8 + d8) * 8, from, SC1);
-            ml = load2(mine + DL_HD * 8, from);
-            return ((v[1] ^ epoch) | (ml[1] ^ epoch) | (ml[3] ^ epoch)) != 0;
-          });
-          const float pm = sp0 + slot <= last ? __uint_as_float(ml[0]) : -INFINITY;
-          const float most = fmaxf(mx, pm);
-          const float f0 = most == mx ? 1.f : exp2_raw(mx - most), f1 = most == pm ? 1.f : exp2_raw(pm - most);
-          const float w = sp0 + slot <= last ? f1 : 0.f;
-          acc = fmaf(w, __uint_as_float(v[0]), acc * f0);
-          den = fmaf(w, __uint_as_float(ml[2]), den * f0);
-          mx = most;
-        }
-        float top = fmaxf(mx, lane_xor<8>(mx));
-        top = apart_max<16>(top);
-        top = apart_max<32>(top);
-        const float f = exp2_raw(mx - top);
-        acc *= f;
-        den *= f;
-        acc += lane_xor<8>(acc);
-        den += lane_xor<8>(den);
-        acc = apart_sum<16>(acc);
-        den = apart_sum<16>(den);
-        acc = apart_sum<32>(acc);
-        den = apart_sum<32>(den);
-        uint32_t d0, d1;
-        quad_words(acc / den, d8, d0, d1);
-        if (slot == 0)
-          store2((((d8 % 4) * M * nH + head) * (DL_HD / 4) + piece * 2 + d8 / 4) * 16, (set + at.attn) * 16, d0,
-                 d1, epoch);
-      }
-    }
-    // ---- the attention's output into the stream
-    if (n_sum > 0) {
-      gather_rows(set + at.attn + copy * (M * nH * (DL_HD / 4)), nH * DL_HD, epoch);
-      dl_barrier();
-      const bool leave = dl_uniform(*dead) != 0;
-      dl_barrier();
-      if (leave) { dl_barrier(); break; }
-      residual(ff_gain, set + at.mid, set + at.mid_sq, epoch, false);
-      dl_barrier();
-    }
-    // ---- gate and up
-    if (n_ff > 0) {
-      gather_normed(set + at.mid, set + at.mid_sq, epoch);
-      dl_barrier();
-      float inv[M];
-      inv_rms(p.eps_ff, inv);
-      const bool leave = dl_uniform(*dead) != 0;
-      dl_barrier();
-      if (leave) { dl_barrier(); break; }
-      const uint32_t e_r = place().r;
-      for (uint32_t e = place().pair; e < (uint32_t)n_ff * M; e += 16) {
-        const uint32_t tok = e % M, unit = e / M;
-        float f = inv[0];
+        dl_barrier();
+        float inv[M];
+        inv_rms(p.eps_in, inv);
+        const bool leave = dl_uniform(*dead) != 0;
+        for (int k0 = 0; k0 == 0 || (FEW && k0 < n_qkv); k0 += PIECE) {
+          const int n = FEW ? min(PIECE, n_qkv - k0) : n_qkv;
+          if (FEW && !leave) multiply(layer, 0, qkv_first, k0, n);
+          dl_barrier();
+          if (leave) { dl_barrier(); return false; }
+          const Place e = place();
+          if (e.unit < (uint32_t)n) {
+            float f = inv[0];
 #pragma unroll
-        for (int k = 1; k < M; ++k) f = tok == k ? inv[k] : f;
-        const float gv = sum_waves(2 * M * unit + tok, e_r) * f, uv = sum_waves((2 * unit + 1) * M + tok, e_r) * f;
-        uint32_t d0, d1;
-        quad_words(gv / (1.0f + expf(-gv)) * uv, e_r, d0, d1);
-        const uint32_t row = (e_r % DL_COPIES) * M + tok;
-        store2((row * (p.ff / 4) + (ff_first + unit * wgs) * 4 + e_r / 4) * 16, (set + at.act) * 16, d0, d1,
-               epoch);
+            for (int tok = 1; tok < M; ++tok) f = e.tok == tok ? inv[tok] : f;
+            uint32_t d0, d1;
+            quad_words(sum_waves(e.pair, e.r) * f, e.r, d0, d1);
+            if (e.r % 4 == 0)
+              store2((e.tok * qkv_units + qkv_first + (k0 + e.unit) * wgs) * 64 + e.r * 4, (set + at.qkv) * 16, d0,
+                     d1, epoch);
+          }
+          dl_barrier();
+        }
       }
-      dl_barrier();
+      // ---- attention, a split of a context at a time
+      for (int turn = 0, split_at = wg; FEW ? split_at < n_splits : turn < n_att; ++turn, split_at += wgs) {
+        const uint32_t t = thread();
+        const int att = FEW ? 0 : turn;
+        if constexpr (FEW) {
+          if (!put_split(split_at, 0, t)) continue;
+          dl_barrier();
+          ask_keys(layer, 0);
+        }
+        const DecodeArgs pp = args();
+        const int item = dl_uniform(sh.item[att]);
+        const int kvh = item & 255, sp = item >> 8 & 255, s = item >> 16 & 255;
+        const bool own = item >> 24;
+        const int ctx = dl_const(pp->ctx_len)[s], pos = ctx - 1;
+        const int lane = t % 64, j = lane % 16, qd = lane / 16;
+        const int kb = sp * DL_SPLIT + cwave * DL_WAVE_KEYS, k_end = min(ctx, kb + DL_WAVE_KEYS);
+        const bool has_keys = kb < k_end;
+        const int hi = t / 16, l16 = t % 16, n_items = own ? G + 1 : G;
+        // the head's words: elements 4 l16 .. + 3 and 64 further on; the new value: 8 elements a thread
+        const uint32_t row = (set + at.qkv + s * (qkv_units * 4)) * 16;
+        const uint32_t head_at = (hi < G ? kvh * G + hi : nH + kvh) * (DL_HD / 4 * 16) + l16 * 16;
+        u32x4_t r0, r1, v0, v1;
+        wait_for([&]() __attribute__((always_inline)) {
+          r0 = load2(head_at, row);
+          r1 = load2(head_at, row + DL_HD / 8 * 16);
+          const uint32_t bad = (r0[1] ^ epoch) | (r0[3] ^ epoch) | (r1[1] ^ epoch) | (r1[3] ^ epoch);
+          return hi < n_items && bad != 0;
+        });
+        if (own && cwave == 0) {
+          const uint32_t value_at = row + (nH + p.nKV + kvh) * (DL_HD / 4 * 16);
+          wait_for([&]() __attribute__((always_inline)) {
+            v0 = load2(l16 * 32, value_at);
+            v1 = load2(l16 * 32, value_at + 16);
+            return ((v0[1] ^ epoch) | (v0[3] ^ epoch) | (v1[1] ^ epoch) | (v1[3] ^ epoch)) != 0;
+          });
+        }
+        const size_t put = sh.put[att];
+        const int r = put % 16;
+        {
+          float x0[4], x1[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            x0[e] = bf16_to_float((bf16_t)(r0[2 * (e / 2)] >> (16 * (e % 2))));
+            x1[e] = bf16_to_float((bf16_t)(r1[2 * (e / 2)] >> (16 * (e % 2))));
+          }
+          HeadCoef cf;
+          cf.has_gain = L.q_gain != nullptr;
+          cf.has_rotation = p.cos_t != nullptr;
+          const f32x4_t c = *(const f32x4_t*)&sh.turn[s][0][4 * l16], sn = *(const f32x4_t*)&sh.turn[s][1][4 * l16];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            cf.g0[e] = g0[e];
+            cf.g1[e] = g1[e];
+            cf.c[e] = c[e];
+            cf.sn[e] = sn[e];
+          }
+          head_norm_rotate<16>(x0, x1, DL_HD, true, pp->eps_head, cf);
+          if (hi < n_items) {
+            const u32x2_t y0 = u32x2_t{pack_bf16x2(x0[0], x0[1]), pack_bf16x2(x0[2], x0[3])};
+            const u32x2_t y1 = u32x2_t{pack_bf16x2(x1[0], x1[1]), pack_bf16x2(x1[2], x1[3])};
+            bf16_t* dst = sh.q[hi < G ? hi : 16];
+            *(u32x2_t*)(dst + 4 * l16) = y0;
+            *(u32x2_t*)(dst + DL_HD / 2 + 4 * l16) = y1;
+            if (hi == G) {          // element d of row r at [d / 32][16 ((d % 32) / 8) + r][d % 8]
+              auto* grp = (DL_GLOBAL bf16_t*)(uintptr_t)L.k_pool + (put & ~(size_t)15);
+              const int d0 = 4 * l16, at0 = (d0 / 32) * 512 + (((d0 % 32) / 8) * 16 + r) * 8 + d0 % 8;
+              *(DL_GLOBAL u32x2_t*)(grp + at0) = y0;
+              *(DL_GLOBAL u32x2_t*)(grp + at0 + (DL_HD / 64) * 512) = y1;
+            }
+          }
+          if (own && t < DL_HD / 8) {           // [d / 16][16 (r / 4) + d % 16][r % 4]
+            *(u32x4_t*)(sh.q[17] + 8 * l16) = u32x4_t{v0[0], v0[2], v1[0], v1[2]};
+            auto* grp = (DL_GLOBAL bf16_t*)(uintptr_t)L.v_pool + (put & ~(size_t)15) + (r / 4) * 64 + r % 4;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              const int d = 8 * l16 + i;
+              grp[(d / 16) * 256 + (d % 16) * 4] =
+                  (bf16_t)((i < 4 ? v0 : v1)[(i / 2) % 2 * 2] >> (16 * (i % 2)));
+            }
+          }
+        }
+        dl_barrier();
+        float m = -INFINITY, l = 0.f;
+        f32x4_t o[DL_HD / 16];
+#pragma unroll
+        for (int dt = 0; dt < DL_HD / 16; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (has_keys) {
+          bf16x8_t qf[DL_HD / 32];
+#pragma unroll
+          for (int st = 0; st < DL_HD / 32; ++st) {
+            u32x4_t v = *(const u32x4_t*)(sh.q[min(j, G - 1)] + st * 32 + 8 * qd);
+            qf[st] = *(bf16x8_t*)&v;
+          }
+          // the token's own key and value, which the cache did not hold when it was read, where its lanes
+          // hold a key's elements 32 stp + 8 qd .. + 7 (lane j: key j of the group) and four keys' values
+          // (lane j: element 16 dt + j of keys 4 qd .. + 3)
+          if (pos >= kb && pos < kb + DL_WAVE_KEYS) {
+            const int jn = (pos - kb) % 16;
+            auto patch = [&](u32x4_t (&k)[DL_HD / 32], u32x2_t (&v)[DL_HD / 16]) __attribute__((always_inline)) {
+#pragma unroll
+              for (int stp = 0; stp < DL_HD / 32; ++stp) {
+                const u32x4_t kx = *(const u32x4_t*)(sh.q[16] + stp * 32 + 8 * qd);
+                if (j == jn) k[stp] = kx;
+              }
+              const uint32_t keep = jn % 2 ? 0x0000ffffu : 0xffff0000u;
+#pragma unroll
+              for (int dt = 0; dt < DL_HD / 16; ++dt) {
+                const uint32_t vn = (uint32_t)sh.q[17][16 * dt + j] << (16 * (jn % 2));
+                if (qd == jn / 4) {
+                  if ((jn % 4) / 2 == 0) v[dt][0] = (v[dt][0] & keep) | vn;
+                  else v[dt][1] = (v[dt][1] & keep) | vn;
+                }
+              }
+            };
+            if (pos - kb < 16) patch(kf[0], vf[0]);
+            else patch(kf[1], vf[1]);
+          }
+          float sc[8];
+          decode_scores<DL_HD, false, 2>(kf, qf, kb, kb, k_end, qd, p.scale_log2e, m, l, sc, -1, nullptr);
+          decode_values<DL_HD, false, 2>(vf, sc, kb, kb, k_end, qd, o, -1, nullptr);
+        }
+        if (j < G) {
+#pragma unroll
+          for (int dt = 0; dt < DL_HD / 16; ++dt) *(f32x4_t*)&sh.o[cwave][j][dt * 16 + 4 * qd] = o[dt];
+        }
+        if (qd == 0) {
+          sh.m[cwave][j] = m;
+          sh.l[cwave][j] = l;
+        }
+        dl_barrier();
+        // a head a wave, two elements a lane
+        for (int col = cwave; col < G; col += 4) {
+          float pm[4], mx = -INFINITY;
+#pragma unroll
+          for (int w = 0; w < 4; ++w) pm[w] = sh.m[w][col];
+#pragma unroll
+          for (int w = 0; w < 4; ++w) mx = fmaxf(mx, pm[w]);
+          float a0 = 0.f, a1 = 0.f, den = 0.f;
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {         // (a wave without keys has max -inf: weight 0)
+            const float f = exp2_raw(pm[w] - mx);
+            const float2 ov = *(const float2*)&sh.o[w][col][2 * lane];
+            a0 = fmaf(f, ov.x, a0);
+            a1 = fmaf(f, ov.y, a1);
+            den = fmaf(f, sh.l[w][col], den);
+          }
+          const int head = s * nH + kvh * G + col;
+          if (ctx <= DL_SPLIT) {
+            const uint32_t mine = pack_bf16x2(a0 / den, a1 / den);
+            const uint32_t other = __float_as_uint(lane_xor<1>(__uint_as_float(mine)));
+            const uint32_t d0 = lane % 2 ? other : mine, d1 = lane % 2 ? mine : other;
+            // copies lane % 2 and lane % 2 + 2
+            const uint32_t to = ((lane % 2) * M * nH * (DL_HD / 4) + head * (DL_HD / 4) + lane / 2) * 16;
+            store2(to, (set + at.attn) * 16, d0, d1, epoch);
+            store2(to, (set + at.attn + 2 * M * nH * (DL_HD / 4)) * 16, d0, d1, epoch);
+          } else {
+            const uint32_t to = (set + at.part + (head * p.max_splits + sp) * (DL_PART / 2)) * 16;
+            store2(lane * 16, to, __float_as_uint(a0), __float_as_uint(a1), epoch);
+            if (lane == 0) store2(DL_HD / 2 * 16, to, __float_as_uint(mx), __float_as_uint(den), epoch);
+          }
+        }
+        if constexpr (!FEW) ask_keys(layer, att + 1);
+        dl_barrier();               // (the next split's partial outputs go where these are)
+      }
+      // ---- contexts of several splits: eight elements of a head a wave, eight splits side by side
+      if (split) {
+        const int lane = thread() % 64, d8 = lane % 8, slot = lane / 8;
+        constexpr int pieces = DL_HD / 8;
+        for (int item = cwave * wgs + wg; item < M * nH * pieces; item += 4 * wgs) {
+          const int piece = item % pieces, head = item / pieces, s = M == 1 ? 0 : head / nH;
+          const int last = (dl_const(args()->ctx_len)[s] - 1) / DL_SPLIT;
+          if (last == 0) continue;
+          const uint32_t from = (set + at.part + head * p.max_splits * (DL_PART / 2)) * 16;
+          float mx = -INFINITY, acc = 0.f, den = 0.f;
+          for (int sp0 = 0; sp0 <= last; sp0 += 8) {
+            const uint32_t mine = min(sp0 + slot, last) * (DL_PART * 8);
+            u32x4_t ml;
+            u32x2_t v;
+            wait_for([&]() __attribute__((always_inline)) {
+              v = __builtin_amdgcn_raw_buffer_load_b64(words, mine + (piece * 8 + d8) * 8, from, SC1);
+              ml = load2(mine + DL_HD * 8, from);
+              return ((v[1] ^ epoch) | (ml[1] ^ epoch) | (ml[3] ^ epoch)) != 0;
+            });
+            const float pm = sp0 + slot <= last ? __uint_as_float(ml[0]) : -INFINITY;
+            const float most = fmaxf(mx, pm);
+            const float f0 = most == mx ? 1.f : exp2_raw(mx - most), f1 = most == pm ? 1.f : exp2_raw(pm - most);
+            const float w = sp0 + slot <= last ? f1 : 0.f;
+            acc = fmaf(w, __uint_as_float(v[0]), acc * f0);
+            den = fmaf(w, __uint_as_float(ml[2]), den * f0);
+            mx = most;
+          }
+          float top = fmaxf(mx, lane_xor<8>(mx));
+          top = apart_max<16>(top);
+          top = apart_max<32>(top);
+          const float f = exp2_raw(mx - top);
+          acc *= f;
+          den *= f;
+          acc += lane_xor<8>(acc);
+          den += lane_xor<8>(den);
+          acc = apart_sum<16>(acc);
+          den = apart_sum<16>(den);
+          acc = apart_sum<32>(acc);
+          den = apart_sum<32>(den);
+          uint32_t d0, d1;
+          quad_words(acc / den, d8, d0, d1);
+          if (slot == 0)
+            store2((((d8 % 4) * M * nH + head) * (DL_HD / 4) + piece * 2 + d8 / 4) * 16, (set + at.attn) * 16, d0,
+                   d1, epoch);
+        }
+      }
+      // ---- the attention's output into the stream
+      if (n_sum > 0) {
+        gather_rows(set + at.attn + copy * (M * nH * (DL_HD / 4)), nH * DL_HD, epoch);
+        dl_barrier();
+        const bool leave = dl_uniform(*dead) != 0;
+        for (int k0 = 0; k0 == 0 || (FEW && k0 < n_sum); k0 += PIECE) {
+          if (FEW && !leave) multiply(layer, 1, wg, k0, min(PIECE, n_sum - k0));
+          dl_barrier();
+          if (leave) { dl_barrier(); return false; }
+          residual(ff_gain, L.ff_gain, k0, set + at.mid, set + at.mid_sq, epoch, false);
+          dl_barrier();
+        }
+      }
+      // ---- gate and up
+      if (n_ff > 0) {
+        gather_normed(set + at.mid, set + at.mid_sq, epoch);
+        dl_barrier();
+        float inv[M];
+        inv_rms(p.eps_ff, inv);
+        const bool leave = dl_uniform(*dead) != 0;
+        for (int k0 = 0; k0 == 0 || (FEW && k0 < n_ff); k0 += FF_PIECE) {
+          const int n = FEW ? min(FF_PIECE, n_ff - k0) : n_ff;
+          if (FEW && !leave) multiply(layer, 2, ff_first, k0, n);
+          dl_barrier();
+          if (leave) { dl_barrier(); return false; }
+          const uint32_t e_r = place().r;
+          for (uint32_t e = place().pair; e < (uint32_t)n * M; e += 16) {
+            const uint32_t tok = e % M, unit = e / M;
+            float f = inv[0];
+#pragma unroll
+            for (int k = 1; k < M; ++k) f = tok == k ? inv[k] : f;
+            const float gv = sum_waves(2 * M * unit + tok, e_r) * f, uv = sum_waves((2 * unit + 1) * M + tok, e_r) * f;
+            uint32_t d0, d1;
+            quad_words(gv / (1.0f + expf(-gv)) * uv, e_r, d0, d1);
+            const uint32_t row = (e_r % DL_COPIES) * M + tok;
+            store2((row * (p.ff / 4) + (ff_first + (k0 + unit) * wgs) * 4 + e_r / 4) * 16, (set + at.act) * 16, d0,
+                   d1, epoch);
+          }
+          dl_barrier();
+        }
+      }
+      // ---- down into the stream
+      if (n_sum > 0) {
+        gather_rows(set + at.act + copy * (M * p.ff / 4), p.ff, epoch);
+        dl_barrier();
+        if constexpr (!FEW) ask_keys(layer + 1, 0);
+        const bool leave = dl_uniform(*dead) != 0;
+        for (int k0 = 0; k0 == 0 || (FEW && k0 < n_sum); k0 += PIECE) {
+          if (FEW && !leave) multiply(layer, 3, wg, k0, min(PIECE, n_sum - k0));
+          dl_barrier();
+          if (leave) { dl_barrier(); return false; }
+          residual(next_gain, L.next_gain, k0, set + at.next, set + at.next_sq, epoch, layer + 1 == n_layers);
+          dl_barrier();
+        }
+        return true;
+      }
+      if constexpr (!FEW) ask_keys(layer + 1, 0);
+      return true;
+    };
+    for (int layer = 0; layer < n_layers; ++layer)
+      if (!run_layer(layer)) break;
+    const DecodeArgs pp = args();
+    if (dl_uniform(*dead) != 0) {
+      Place e = place();
+      for (; e.unit < (uint32_t)n_sum; e.unit += PIECE) {
+        const size_t n = (size_t)e.tok * p.hidden + column(e);
+        pp->x[n] = __uint_as_float(0x7fc00000u);
+        pp->xg[n] = 0x7fc0;
+      }
+      if (cwave == 0) __hip_atomic_store(pp->status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
-    // ---- down into the stream
-    if (n_sum > 0) {
-      gather_rows(set + at.act + copy * (M * p.ff / 4), p.ff, epoch);
-      dl_barrier();
-      ask_keys(layer + 1, 0);
-      const bool leave = dl_uniform(*dead) != 0;
-      dl_barrier();
-      if (leave) { dl_barrier(); break; }
-      residual(next_gain, set + at.next, set + at.next_sq, epoch, layer + 1 == n_layers);
-      dl_barrier();
-    } else {
-      ask_keys(layer + 1, 0);
-    }
-  }
-  const DecodeArgs pp = args();
-  if (dl_uniform(*dead) != 0) {
-    if (keeps) {
-      const Place e = place();
-      const size_t n = (size_t)e.tok * p.hidden + column(e);
-      pp->x[n] = __uint_as_float(0x7fc00000u);
-      pp->xg[n] = 0x7fc0;
-    }
-    if (cwave == 0) __hip_atomic_store(pp->status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
+  };
+  if (few) all_layers(std::true_type{});
+  else all_layers(std::false_type{});
 }
 
 template <int M>
@@ -1022,13 +1099,13 @@ extern "C" int zf_decode_layers(const DecodeLayers* args, int workgroups, hipStr
       p.nH % p.nKV != 0 || p.nH / p.nKV > 15 || p.nH * DL_HD < 512 || p.page_size % 16 != 0 ||
       p.max_splits < 1 || p.max_splits > 255)
     return -3;
-  int units = (p.nH + 2 * p.nKV) * (DL_HD / 16);
+  int units = (p.nH + 2 * p.nKV) * (DL_HD / 16), table = (p.max_pages * p.page_size + DL_SPLIT - 1) / DL_SPLIT;
   if (p.hidden / 16 > units) units = p.hidden / 16;
-  const int per = DL_UNITS / M, ff_per = DL_FF_UNITS / M, splits = M * p.nKV * p.max_splits;
+  if (table > p.max_splits) return -3;
+  const int per = DL_UNITS / M, ff_per = DL_FF_UNITS / M, splits = M * p.nKV * table;
   p.need = (units + per - 1) / per;
   if ((p.ff / 16 + ff_per - 1) / ff_per > p.need) p.need = (p.ff / 16 + ff_per - 1) / ff_per;
   if ((splits + DL_ATT - 1) / DL_ATT > p.need) p.need = (splits + DL_ATT - 1) / DL_ATT;
-  if (2 * p.need > workgroups) return -3;        // (of two launches that meet at once one goes on)
   if ((p.cos_t == nullptr) != (p.sin_t == nullptr) || (p.cos_t != nullptr && p.table_rows < 1)) return -3;
   const size_t lds = M == 1 ? dl_lds<1>(p) : M == 2 ? dl_lds<2>(p) : M == 3 ? dl_lds<3>(p) : dl_lds<4>(p);
   if (lds > 160 * 1024) return -3;

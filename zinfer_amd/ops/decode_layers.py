@@ -19,6 +19,10 @@ MAX_FF_UNITS = 32            # DL_FF_UNITS
 MAX_ATTENTION = 8            # DL_ATT
 MAX_TOKENS = 4               # DL_TOKENS
 MEETING = 512                # bytes of DecodeMeet
+# Of 10 ns: how long the workgroups that have come wait for the others, and while they are fewer than hold a
+# phase's sums (longer than most kernels keep a CU; the 0.6B shape on 16 workgroups, which do, 1.3 ms a step, on
+# 15 4.9, on all 256 0.47; eight layers of the 8B shape on 24 2.4, on 16 6.0, on all 0.60)
+MEET_TICKS, MEET_MOST = 5000, 100000
 
 _vp, _i, _f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
 
@@ -37,7 +41,8 @@ class _Layers(ctypes.Structure):
         + [(n, _f) for n in ("eps_in", "eps_ff", "eps_head", "scale_log2e")] \
         + [("cos", _vp), ("sin", _vp), ("table_rows", _i), ("positions", _vp), ("slot_mapping", _vp),
            ("block_table", _vp), ("ctx_len", _vp), ("x", _vp), ("xg", _vp), ("sq", _vp),
-           ("words", _vp), ("meet", _vp), ("need", _i), ("status", _vp)]
+           ("words", _vp), ("meet", _vp)] \
+        + [(n, _i) for n in ("need", "meet_ticks", "meet_most")] + [("status", _vp)]
 
 
 @functools.lru_cache(maxsize=None)
@@ -56,7 +61,7 @@ def sizes_covered(tokens: int, hidden: int, ff: int, n_heads: int, n_kv_heads: i
         return False
     units = (hidden // 16, (n_heads + 2 * n_kv_heads) * head_dim // 16)
     row = 2 * max(hidden, ff, n_heads * head_dim) + 16
-    most = wgs // 2                # (decode_layers.hip: of two launches that meet one goes on)
+    most = wgs // 2                # (the half of a launch that meets another one runs as it is meant to)
     return max(units) <= MAX_UNITS // tokens * most and ff // 16 <= MAX_FF_UNITS // tokens * most \
         and tokens * n_kv_heads * MAX_SPLITS <= MAX_ATTENTION * most \
         and 80 * 1024 + tokens * (row + hidden // 4 + 512) <= 160 * 1024
@@ -104,6 +109,6 @@ def decode_layers(table: torch.Tensor, n_layers: int, x: torch.Tensor, xg: torch
                 MAX_SPLITS, eps_in, eps_ff, eps_head, scale * 1.4426950408889634, ptr(cos), ptr(sin),
                 0 if cos is None else cos.shape[0], ptr(positions), ptr(slot_mapping),
                 ptr(block_table), ptr(ctx_len), ptr(x), ptr(xg), ptr(sq), ptr(word_buffer),
-                word_buffer.data_ptr() + word_buffer.numel() - MEETING, 0, ptr(status))
+                word_buffer.data_ptr() + word_buffer.numel() - MEETING, 0, MEET_TICKS, MEET_MOST, ptr(status))
     lib = build.load("decode_layers")
     _check(lib.zf_decode_layers(ctypes.byref(p), wgs, _stream()), "decode_layers")
