@@ -391,3 +391,51 @@ def test_three_engines_that_need_more_than_a_third_of_the_workgroups_each():
         t.join()
     for rows in got:
         assert all(np.array_equal(np.stack(rows[r]), want[r]) for r in requests)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,lengths,workgroups", [
+    ((512, 4, 4, 512, 16), (1500, 1410, 40, 1300), None), ((1024, 16, 8, 3072, 16), (133,), None),
+    ((576, 15, 1, 1088, 48), (140, 33, 12), 7)], ids=str)
+def test_waits_that_give_up_hand_on_nothing_that_did_not_come(shape, lengths, workgroups, monkeypatch):
+    """Every wait gives up at the first look that misses a word, in workgroups of every kind (some of the first
+    shape's have attention alone) and in too few of them: rows of NaN, an error where the host waits, nothing in
+    the pools that the whole step does not write, and the next step as if there had been none."""
+    from zinfer_amd.engine import StepEntry
+    from zinfer_amd.errors import StepError
+    hidden, heads, kv, ff, page = shape
+    cfg = _qwen3(hidden, heads, kv, ff)
+    requests = {f"r{i}": tiny.random_tokens(n, cfg["vocab_size"], n) for i, n in enumerate(lengths)}
+    if workgroups is not None:
+        monkeypatch.setattr(kernel, "sizes_covered", lambda *sizes: True)
+        monkeypatch.setattr(kernel, "workgroups", lambda index: workgroups)
+    eng = _engine(cfg, _weights(cfg, hidden + heads), page, tokens=8192, graphs=False)
+    for r, t in requests.items():
+        eng.step([StepEntry(r, t[:-1], [])])
+    pools = [p for view in eng.views for p in (view.k_pool, view.v_pool)]
+    before = [p.clone() for p in pools]
+
+    def step():
+        return eng.step([StepEntry(r, t[-1:], [0]) for r, t in requests.items()])
+
+    def back():
+        for r, n in zip(requests, lengths):
+            eng.cache.commit(r, n - 1)
+            eng.cache.trim(r)
+        for p, b in zip(pools, before):
+            p.copy_(b)
+    want = eng.to_host(step()).clone()
+    written = [p.clone() for p in pools]
+    for _ in range(3):
+        back()
+        with monkeypatch.context() as m:
+            m.setattr(kernel, "SPIN_FROM", (1 << 21) | 15)
+            rows = step()
+        assert torch.isnan(rows).all().item()
+        with pytest.raises(StepError, match="hear"):
+            eng.to_host(rows)
+        assert [eng.length(r) for r in requests] == [n - 1 for n in lengths]
+        for p, b, w in zip(pools, before, written):
+            assert ((p == b) | (p == w)).all().item()
+        back()
+        assert torch.equal(eng.to_host(step()), want)

@@ -33,8 +33,9 @@
 // wait for another that does the same.  Fewer than `need`, whose shares would not fit a phase's sums, take
 // theirs a piece at a time (FEW, below), in the same order of sums.
 // Every wait ends: a reader that has looked DL_SPINS times gives up for its workgroup, which leaves
-// without handing on what it owes, so that the others leave in turn; the rows that go to the head are
-// then NaN and `status` is 1.
+// without handing on what it owes, so that the others leave in turn: what follows from words that did
+// not come is neither handed on nor written to the pools.  The rows that go to the head are then NaN and
+// `status` is 1.
 //
 // A product's sums run in the order of the kernel that has a launch of its own for it (gemm.hip's
 // weight-streaming product, K dealt to eight waves in blocks of 64), whoever takes them.
@@ -101,6 +102,7 @@ struct DecodeLayers {
   int need;                      // workgroups whose shares of a phase fit its sums
   int meet_ticks;                // of 10 ns that the workgroups which have come wait for the others
   int meet_most;                 // and while they are fewer than `need`
+  int spin_from;                 // looks of a wait that count as taken (0)
   int* status;
 };
 
@@ -531,14 +533,16 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
   auto store2 = [&](uint32_t lane_bytes, uint32_t to, uint32_t d0, uint32_t d1, unsigned epoch) __attribute__((always_inline)) {
     __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{d0, epoch, d1, epoch}, words, lane_bytes, to, SC1);
   };
-  // look() loads and says (a lane) whether words are missing; until none of the wave's are
+  // look() loads and says (a lane) whether words are missing; until none of the wave's are (true), or the
+  // workgroup has given up
+  const int spin_from = p.spin_from;
   auto wait_for = [&](auto look) __attribute__((always_inline)) {
-    for (int spin = 0;; ++spin) {
+    for (int spin = spin_from;; ++spin) {
       asm volatile("" ::: "memory");
       const bool missing = look();
-      if (__builtin_amdgcn_ballot_w64(missing) == 0) return;
+      if (__builtin_amdgcn_ballot_w64(missing) == 0) return true;
       if (spin >= DL_SPINS) *dead = 1;
-      if ((spin & 15) == 15 && dl_uniform(*dead) != 0) return;
+      if ((spin & 15) == 15 && dl_uniform(*dead) != 0) return false;
     }
   };
   // `n` pairs of words behind one another from pair `from`, a pair a thread, N at a time; to(number, data)
@@ -811,7 +815,7 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
         const uint32_t row = (set + at.qkv + s * (qkv_units * 4)) * 16;
         const uint32_t head_at = (hi < G ? kvh * G + hi : nH + kvh) * (DL_HD / 4 * 16) + l16 * 16;
         u32x4_t r0, r1, v0, v1;
-        wait_for([&]() __attribute__((always_inline)) {
+        bool came = wait_for([&]() __attribute__((always_inline)) {
           r0 = load2(head_at, row);
           r1 = load2(head_at, row + DL_HD / 8 * 16);
           const uint32_t bad = (r0[1] ^ epoch) | (r0[3] ^ epoch) | (r1[1] ^ epoch) | (r1[3] ^ epoch);
@@ -819,7 +823,7 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
         });
         if (own && cwave == 0) {
           const uint32_t value_at = row + (nH + p.nKV + kvh) * (DL_HD / 4 * 16);
-          wait_for([&]() __attribute__((always_inline)) {
+          came &= wait_for([&]() __attribute__((always_inline)) {
             v0 = load2(l16 * 32, value_at);
             v1 = load2(l16 * 32, value_at + 16);
             return ((v0[1] ^ epoch) | (v0[3] ^ epoch) | (v1[1] ^ epoch) | (v1[3] ^ epoch)) != 0;
@@ -852,14 +856,14 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
             bf16_t* dst = sh.q[hi < G ? hi : 16];
             *(u32x2_t*)(dst + 4 * l16) = y0;
             *(u32x2_t*)(dst + DL_HD / 2 + 4 * l16) = y1;
-            if (hi == G) {          // element d of row r at [d / 32][16 ((d % 32) / 8) + r][d % 8]
+            if (hi == G && came) {  // element d of row r at [d / 32][16 ((d % 32) / 8) + r][d % 8]
               auto* grp = (DL_GLOBAL bf16_t*)(uintptr_t)L.k_pool + (put & ~(size_t)15);
               const int d0 = 4 * l16, at0 = (d0 / 32) * 512 + (((d0 % 32) / 8) * 16 + r) * 8 + d0 % 8;
               *(DL_GLOBAL u32x2_t*)(grp + at0) = y0;
               *(DL_GLOBAL u32x2_t*)(grp + at0 + (DL_HD / 64) * 512) = y1;
             }
           }
-          if (own && t < DL_HD / 8) {           // [d / 16][16 (r / 4) + d % 16][r % 4]
+          if (own && came && t < DL_HD / 8) {   // [d / 16][16 (r / 4) + d % 16][r % 4]
             *(u32x4_t*)(sh.q[17] + 8 * l16) = u32x4_t{v0[0], v0[2], v1[0], v1[2]};
             auto* grp = (DL_GLOBAL bf16_t*)(uintptr_t)L.v_pool + (put & ~(size_t)15) + (r / 4) * 64 + r % 4;
 #pragma unroll
@@ -871,6 +875,7 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
           }
         }
         dl_barrier();
+        const bool lost = dl_uniform(*dead) != 0;       // (nothing of this split is handed on)
         float m = -INFINITY, l = 0.f;
         f32x4_t o[DL_HD / 16];
 #pragma unroll
@@ -936,6 +941,7 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
             den = fmaf(f, sh.l[w][col], den);
           }
           const int head = s * nH + kvh * G + col;
+          if (lost) continue;
           if (ctx <= DL_SPLIT) {
             const uint32_t mine = pack_bf16x2(a0 / den, a1 / den);
             const uint32_t other = __float_as_uint(lane_xor<1>(__uint_as_float(mine)));
@@ -963,11 +969,12 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
           if (last == 0) continue;
           const uint32_t from = (set + at.part + head * p.max_splits * (DL_PART / 2)) * 16;
           float mx = -INFINITY, acc = 0.f, den = 0.f;
+          bool came = true;
           for (int sp0 = 0; sp0 <= last; sp0 += 8) {
             const uint32_t mine = min(sp0 + slot, last) * (DL_PART * 8);
             u32x4_t ml;
             u32x2_t v;
-            wait_for([&]() __attribute__((always_inline)) {
+            came &= wait_for([&]() __attribute__((always_inline)) {
               v = __builtin_amdgcn_raw_buffer_load_b64(words, mine + (piece * 8 + d8) * 8, from, SC1);
               ml = load2(mine + DL_HD * 8, from);
               return ((v[1] ^ epoch) | (ml[1] ^ epoch) | (ml[3] ^ epoch)) != 0;
@@ -994,7 +1001,7 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
           den = apart_sum<32>(den);
           uint32_t d0, d1;
           quad_words(acc / den, d8, d0, d1);
-          if (slot == 0)
+          if (came && slot == 0)
             store2((((d8 % 4) * M * nH + head) * (DL_HD / 4) + piece * 2 + d8 / 4) * 16, (set + at.attn) * 16, d0,
                    d1, epoch);
         }
@@ -1056,7 +1063,7 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
         return true;
       }
       if constexpr (!FEW) ask_keys(layer + 1, 0);
-      return true;
+      return dl_uniform(*dead) == 0;
     };
     for (int layer = 0; layer < n_layers; ++layer)
       if (!run_layer(layer)) break;
@@ -1068,7 +1075,7 @@ __global__ __launch_bounds__(DL_THREADS) void decode_layers_kernel(DecodeLayers 
         pp->x[n] = __uint_as_float(0x7fc00000u);
         pp->xg[n] = 0x7fc0;
       }
-      if (cwave == 0) __hip_atomic_store(pp->status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(pp->status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
   };
   if (few) all_layers(std::true_type{});

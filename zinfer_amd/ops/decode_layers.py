@@ -23,6 +23,7 @@ MEETING = 512                # bytes of DecodeMeet
 # phase's sums (longer than most kernels keep a CU; the 0.6B shape on 16 workgroups, which do, 1.3 ms a step, on
 # 15 4.9, on all 256 0.47; eight layers of the 8B shape on 24 2.4, on 16 6.0, on all 0.60)
 MEET_TICKS, MEET_MOST = 5000, 100000
+SPIN_FROM = 0                # looks that a wait between workgroups begins with (of DL_SPINS)
 
 _vp, _i, _f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
 
@@ -42,7 +43,7 @@ class _Layers(ctypes.Structure):
         + [("cos", _vp), ("sin", _vp), ("table_rows", _i), ("positions", _vp), ("slot_mapping", _vp),
            ("block_table", _vp), ("ctx_len", _vp), ("x", _vp), ("xg", _vp), ("sq", _vp),
            ("words", _vp), ("meet", _vp)] \
-        + [(n, _i) for n in ("need", "meet_ticks", "meet_most")] + [("status", _vp)]
+        + [(n, _i) for n in ("need", "meet_ticks", "meet_most", "spin_from")] + [("status", _vp)]
 
 
 @functools.lru_cache(maxsize=None)
@@ -109,6 +110,7 @@ def decode_layers(table: torch.Tensor, n_layers: int, x: torch.Tensor, xg: torch
                 MAX_SPLITS, eps_in, eps_ff, eps_head, scale * 1.4426950408889634, ptr(cos), ptr(sin),
                 0 if cos is None else cos.shape[0], ptr(positions), ptr(slot_mapping),
                 ptr(block_table), ptr(ctx_len), ptr(x), ptr(xg), ptr(sq), ptr(word_buffer),
-                word_buffer.data_ptr() + word_buffer.numel() - MEETING, 0, MEET_TICKS, MEET_MOST, ptr(status))
+                word_buffer.data_ptr() + word_buffer.numel() - MEETING, 0, MEET_TICKS, MEET_MOST, SPIN_FROM,
+                ptr(status))
     lib = build.load("decode_layers")
     _check(lib.zf_decode_layers(ctypes.byref(p), wgs, _stream()), "decode_layers")
