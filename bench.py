@@ -212,7 +212,8 @@ def step_classes(eng, sched, trace, steps: int, seconds: float) -> dict:
     the layers' matrix products with what is fused into them (norms, SwiGLU, residual sums),
     attention = attention over the cache, in steps of up to 32 sequences with the per-head
     norm, rotation and cache write; norm_rope_write = those as kernels of their own;
-    head_sampling = final norm, head, arg-max)."""
+    head_sampling = final norm, head, arg-max).  At one to four sequences of a Qwen3 shape the timed
+    steps run all layers in one launch; the classes and ``graph_step_ms`` are of a launch a product."""
     from zinfer_amd.engine import StepEntry
     host = sum(r[2] + r[3] for r in trace) / steps
     device = sum(r[4].elapsed_time(r[5]) for r in trace) / 1e3 / steps

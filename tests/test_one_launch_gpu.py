@@ -439,3 +439,26 @@ def test_waits_that_give_up_hand_on_nothing_that_did_not_come(shape, lengths, wo
             assert ((p == b) | (p == w)).all().item()
         back()
         assert torch.equal(eng.to_host(step()), want)
+
+
+@pytest.mark.gpu
+def test_the_classes_and_the_step_they_add_up_to_are_of_one_program(monkeypatch):
+    """A step measured by class, and all classes together, has a launch a product; the step itself has not."""
+    from zinfer_amd import ops
+    from zinfer_amd.engine import StepEntry
+    cfg = _qwen3(512, 4, 2, 512)
+    eng = _engine(cfg, _weights(cfg, 7), tokens=128)
+    eng.step([StepEntry("r", [1, 2, 3], [2])])
+    want = eng.to_host(eng.step([StepEntry("r", [4], [0])])).clone()
+    measured, forward = [], one_launch.OneLaunchLayers.forward
+
+    def counted(self, *args):
+        measured.append(ops._class_filter is not None)
+        return forward(self, *args)
+    monkeypatch.setattr(one_launch.OneLaunchLayers, "forward", counted)
+    times = eng.class_times([StepEntry("r", [5], [0])], repeats=5)
+    assert set(times) == set(ops.KERNEL_CLASSES) | {"step"} and not any(measured)
+    assert times["products"] > 0 and times["attention"] > 0 and times["step"] > 0
+    eng.release("r")
+    eng.step([StepEntry("r", [1, 2, 3], [2])])
+    assert torch.equal(eng.to_host(eng.step([StepEntry("r", [4], [0])])), want)

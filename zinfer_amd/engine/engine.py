@@ -412,7 +412,9 @@ class Engine:
         graph of the step with only that class's kernels launched is captured and replayed
         ``repeats`` times between two events.  What the runs compute means nothing (the kernels
         of the other classes did not run) and nothing of it is kept: the requests hold what
-        they held before.  The reference's per-op timing harness is
+        they held before.  (A step that runs all layers in one launch is measured as the step with
+        a launch a product, "step" included, so that the classes add up to it.)  The reference's
+        per-op timing harness is
         `src/app/cli/tools/bench/ops.zig:516-543`."""
         from .. import ops
         if not self.use_graphs:

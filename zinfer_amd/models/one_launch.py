@@ -60,7 +60,8 @@ class OneLaunchLayers:
 
     def takes(self, model, step, caches, given) -> bool:
         """Whether this step runs here: a token a sequence, with what the first norm needs of the
-        stream's rows already made (``given``)."""
+        stream's rows already made (``given``).  Not where classes of kernels are measured, each alone or
+        all together: the layers' one launch is of no class."""
         if step.max_q_len != 1 or model.layer_probe is not None or ops.measures_classes() \
                 or not isinstance(given, GivenRmsNorm):
             return False

@@ -110,8 +110,8 @@ class kernel_class:
 
 
 def measures_classes() -> bool:
-    """Whether kernels of some classes are left out (``only_classes``)."""
-    return _class_filter is not None and _class_filter != frozenset(KERNEL_CLASSES)
+    """Whether launches are counted by class (``only_classes``, of all classes too)."""
+    return _class_filter is not None
 
 
 def _left_out(cls: str) -> bool:
