@@ -88,7 +88,7 @@ class OneLaunchLayers:
                 at(t) for t in (m.q_gain, m.k_gain, b.ff_norm.gain, after.gain))
             r.k_pool, r.v_pool = at(c.k_pool), at(c.v_pool)
         raw = bytes(records)
-        return step.made(f"decode_layers.{hash(raw)}", lambda device: torch.frombuffer(
+        return step.made("decode_layers." + raw.hex(), lambda device: torch.frombuffer(
             bytearray(raw), dtype=torch.uint8).to(device))
 
     def forward(self, model, step, caches, x, given):
