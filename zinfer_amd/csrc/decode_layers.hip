@@ -6,7 +6,7 @@
 // takes 15 us and 69: the weights, and where these are few the five times that rows travel between all
 // workgroups (1.9 us each, the words' way alone).  Decode steps of one token of Qwen3 shapes behind 120 tokens, four layers and
 // the head, before and after: 0.6B 197 -> 164 us, 1.7B 285 -> 244, 4B 372 -> 350, 8B 560 -> 527; from
-// 14B on the launches' ends are small beside the weights (800 -> 795).  Two tokens 0.6B 196 -> 168, 8B 542 ->
+// 14B on the launches' ends are small beside the weights (800 -> 795).  Two tokens 0.6B 196 -> 168, 8B 544 ->
 // 521; three 200 -> 179, 547 -> 535; four tokens of the 0.6B and 1.7B shapes 202 -> 187 and 291 -> 273: what the
 // workgroups hand each other grows with the tokens.
 //
@@ -21,14 +21,21 @@
 // themselves and nothing else orders the workgroups.  They are written and read by buffer accesses of 8
 // or 16 bytes past the XCDs' own caches (sc1).  What this rests on: an aligned 8-byte half of such an
 // access arrives whole, and a reader's loads are issued anew at every look (an asm statement that may
-// change memory stands ahead of them, so that the compiler neither joins nor hoists them).  A phase's words are overwritten a layer later at the earliest, and whoever is about
-// to write them has read, directly or through others, what every workgroup made from the last
-// ones; two sets of words in turn leave another layer between.
+// change memory stands ahead of them, so that the compiler neither joins nor hoists them).  A phase's
+// words are overwritten a layer later at the earliest, and whoever is about to write them has read,
+// directly or through others, what every workgroup made from the last ones; two sets of words in turn
+// leave another layer between.
+//
 // Workgroups that are resident at once do the step: they arrive one after the other, and what there is
 // to do is dealt among those that have come when all have or, where another stream or process holds
 // CUs, `meet_ticks` later; whoever comes then leaves again.  So no workgroup waits for one that has no CU,
 // whatever runs beside (a cooperative launch promises the same from a queue of its own: 15 us a step to
 // go there and back, and half a microsecond more for every later kernel of the process).
+// Launches side by side: a step holds every CU it got until its end, so two engines that decode at once run
+// their steps one behind the other, where launches a product fill each other's gaps (us a step, two engines of one
+// user each, drawing included: 0.6B 952 and 969, eight layers of the 8B shape 1165 and 1047; of three users 1302
+// and 1064, 1304 and 1105), and beside another's whole prompts a step waits for CUs once and not at every product (0.6B
+// 682 and 5019 us a step, while a prompt of 2048 tokens through four layers of the 8B shape takes 8.2 ms and 3.4).
 // However few have come `meet_most` later, one included, do it: a launch that held CUs until it had more could
 // wait for another that does the same.  Fewer than `need`, whose shares would not fit a phase's sums, take
 // theirs a piece at a time (FEW, below), in the same order of sums.
