@@ -42,6 +42,19 @@ def test_the_sizes_python_accepts_are_accepted_by_the_entry():
     assert accepted > 200
 
 
+@pytest.mark.parametrize("shape,most_keys", [       # (per number of tokens)
+    ((1024, 16, 8, 3072), (4096, 4096, 4096, 3072)), ((2048, 32, 8, 8192), (4096, 4096, 3072, 1024)),
+    ((2560, 24, 8, 6912), (4096, 4096, 3072, 1024)), ((4096, 32, 8, 12288), (4096, 4096, 3072, 1024)),
+    ((5120, 32, 8, 13824), (4096, 0, 0, 0)), ((4608, 36, 4, 14336), (0, 0, 0, 0)), ((5120, 40, 8, 17408), (0, 0, 0, 0)),
+    ((5120, 64, 8, 25600), (0, 0, 0, 0))], ids=str)
+def test_where_one_launch_pays(shape, most_keys):
+    """As measured on 256 CUs: to which tables, if at all, a step of one to four tokens is the faster one so."""
+    hidden, heads, kv, ff = shape
+    for tokens, most in enumerate(most_keys, 1):
+        for keys in (16, 256, 1024, 1040, 3072, 3088, 4096):
+            assert kernel.pays(tokens, hidden, ff, heads, kv, keys, 256) == (keys <= most), (tokens, keys)
+
+
 def _qwen3(hidden, heads, kv, ff, layers=2, vocab=1030):
     return dict(architectures=["Qwen3ForCausalLM"], model_type="qwen3", num_hidden_layers=layers,
                 hidden_size=hidden, num_attention_heads=heads, num_key_value_heads=kv, head_dim=128,
@@ -462,3 +475,17 @@ def test_the_classes_and_the_step_they_add_up_to_are_of_one_program(monkeypatch)
     eng.release("r")
     eng.step([StepEntry("r", [1, 2, 3], [2])])
     assert torch.equal(eng.to_host(eng.step([StepEntry("r", [4], [0])])), want)
+
+
+@pytest.mark.gpu
+def test_steps_where_it_does_not_pay_have_a_launch_a_product(monkeypatch):
+    cfg = _qwen3(512, 4, 2, 512)
+    w, toks = _weights(cfg, 7), tiny.random_tokens(40, cfg["vocab_size"], 2)
+    apart = _engine(cfg, w)
+    apart.model.one_launch = None
+    monkeypatch.setattr(one_launch.OneLaunchLayers, "forward", _counted(calls := []))
+    asked = []
+    monkeypatch.setattr(kernel, "pays", lambda *sizes: asked.append(sizes))
+    got = _answer(_engine(cfg, w), toks, 4)
+    assert asked[0] == (1, 512, 512, 4, 2, 256, kernel.compute_units(0)) and not calls
+    assert np.array_equal(got, _answer(apart, toks, 4))

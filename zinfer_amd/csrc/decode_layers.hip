@@ -5,8 +5,9 @@
 // of the 0.6B shape, whose 31 MB of weights take 4.5 at 7 TB/s; 81 of 55 at the 8B shape).  Here a layer
 // takes 15 us and 69: the weights, and where these are few the five times that rows travel between all
 // workgroups (1.9 us each, the words' way alone).  Decode steps of one token of Qwen3 shapes behind 120 tokens, four layers and
-// the head, before and after: 0.6B 197 -> 164 us, 1.7B 285 -> 244, 4B 372 -> 350, 8B 560 -> 527; from
-// 14B on the launches' ends are small beside the weights (800 -> 795).  Two tokens 0.6B 196 -> 168, 8B 544 ->
+// the head, before and after: 0.6B 197 -> 164 us, 1.7B 285 -> 244, 4B 372 -> 350, 8B 560 -> 527; where
+// row groups deal out unevenly, as at 14B, the phases' ends cost what the launches' did, and such steps keep a launch a
+// product (ops/decode_layers.py, `pays`, has the lines and both sides' figures).  Two tokens 0.6B 196 -> 168, 8B 544 ->
 // 521; three 200 -> 179, 547 -> 535; four tokens of the 0.6B and 1.7B shapes 202 -> 187 and 291 -> 273: what the
 // workgroups hand each other grows with the tokens.
 //

@@ -25,7 +25,8 @@ class OneLaunchLayers:
         self.hidden = model.spec.hidden_size
         self.heads, self.kv_heads = a.n_heads, a.n_kv_heads
         self.tables = model.blocks[0].mixer.position.rotation_tables()
-        self.wgs = kernel.workgroups(torch.device(model.ctx.device).index or 0)
+        index = torch.device(model.ctx.device).index or 0
+        self.wgs, self.cus = kernel.workgroups(index), kernel.compute_units(index)
 
     @staticmethod
     def of(model):
@@ -66,7 +67,9 @@ class OneLaunchLayers:
                 or not isinstance(given, GivenRmsNorm):
             return False
         cache = caches[0]
-        if step.kv_tables(cache.group).max_pages * cache.page_size > kernel.MAX_CONTEXT:
+        keys = step.kv_tables(cache.group).max_pages * cache.page_size
+        if keys > kernel.MAX_CONTEXT or not kernel.pays(step.n_tokens, self.hidden, self.ff, self.heads,
+                                                        self.kv_heads, keys, self.cus):
             return False
         if not kernel.sizes_covered(step.n_tokens, self.hidden, self.ff, self.heads, self.kv_heads,
                                     model.blocks[0].mixer.spec.head_dim, cache.page_size, self.wgs):

@@ -47,9 +47,13 @@ class _Layers(ctypes.Structure):
 
 
 @functools.lru_cache(maxsize=None)
+def compute_units(device_index: int) -> int:
+    return torch.cuda.get_device_properties(device_index).multi_processor_count
+
+
 def workgroups(device_index: int) -> int:
     """A workgroup a CU."""
-    return torch.cuda.get_device_properties(device_index).multi_processor_count
+    return compute_units(device_index)
 
 
 def sizes_covered(tokens: int, hidden: int, ff: int, n_heads: int, n_kv_heads: int, head_dim: int,
@@ -66,6 +70,32 @@ def sizes_covered(tokens: int, hidden: int, ff: int, n_heads: int, n_kv_heads: i
     return max(units) <= MAX_UNITS // tokens * most and ff // 16 <= MAX_FF_UNITS // tokens * most \
         and tokens * n_kv_heads * MAX_SPLITS <= MAX_ATTENTION * most \
         and 80 * 1024 + tokens * (row + hidden // 4 + 512) <= 160 * 1024
+
+
+def uneven_bytes(hidden: int, ff: int, n_heads: int, n_kv_heads: int, cus: int) -> int:
+    """What all workgroups would read of a layer's weights if each read as much as the busiest one of
+    each phase, beyond what there is."""
+    q = n_heads * HEAD_DIM
+    phases = (((q + 2 * n_kv_heads * HEAD_DIM) // 16, 32 * hidden), (hidden // 16, 32 * (q + ff)),
+              (ff // 16, 64 * hidden))
+    return sum((-(-units // cus) * cus - units) * unit for units, unit in phases)
+
+
+def pays(tokens: int, hidden: int, ff: int, n_heads: int, n_kv_heads: int, keys: int, cus: int) -> bool:
+    """Whether a step of so many tokens under tables of ``keys`` keys is faster in one launch than with a
+    launch a product.  Measured in us a layer gained, head and draw in both.  A phase ends with its busiest
+    workgroup: by ``uneven_bytes``, one token behind 100 to 3900 keys 17 MB (8B shape) +8.6 to 10.1, 79
+    (4B) +5.4 to 7.3, 183 (5120 wide, 32 heads, 13824) +1.2 to 3.9, 197 (4608, 36, 14336) -1.8 to +0.8,
+    211 (14B) -1.9 to +1.2, 291 (32B) -4.9 to -2.0; two tokens 71 (3584, 28, 18944) -0.1 to +2.6, 183 -2.8 to
+    +1.2, 211 -8.4 to -0.7.  The rows that splits of contexts hand on grow with tokens, heads and keys: behind 2400 and
+    3900 keys three tokens of 32 heads gain +4.0 and -0.4 (2048 wide), +1.0 and -3.0 (4B), of 24 +2.2 and
+    -1.8, of 16 (1.7B) +2.4 at 3900; four tokens of 16 heads +1.0 and -1.3, of 24 (2560 wide) behind 700, 1400 and
+    2400 +3.3, -0.8 and -2.2."""
+    narrow = n_heads <= 16
+    most_keys = MAX_CONTEXT if tokens <= 2 else \
+        (4096 if narrow else 3072) if tokens == 3 else (3072 if narrow else 1024)
+    return keys <= most_keys and \
+        uneven_bytes(hidden, ff, n_heads, n_kv_heads, cus) <= (185e6 if tokens == 1 else 130e6)
 
 
 def words(tokens: int, hidden: int, ff: int, n_heads: int, n_kv_heads: int, device) -> torch.Tensor:
