@@ -361,6 +361,23 @@ def test_shared_arrays_accessed_in_16_byte_pieces_say_that_they_are_aligned():
     assert not found
 
 
+def test_rows_that_change_lanes_in_a_waves_slab_do_so_across_fences():
+    """`store_blocks_bf16` has lanes read what other lanes of their wave wrote, without a barrier: a fence behind
+    the writes and one behind the reads, before the slab is written again, or nothing holds the
+    compiler to that order."""
+    import os
+    import re
+    from zinfer_amd.ops import build
+    with open(os.path.join(build.CSRC, "gemm.hip")) as f:
+        body = re.search(r"void store_blocks_bf16\(.*?\n}\n", f.read(), re.S).group(0)
+    places = [m.start() for m in re.finditer(r"wave_fence\(\);", body)]
+    writes = [m.start() for m in re.finditer(r"\brow\[[^\]]*\] =", body)]
+    reads = [m.start() for m in re.finditer(r"= slab\[", body)]
+    assert len(writes) == 2 and len(reads) == 1 and len(places) == 2
+    assert max(writes) < places[0] < reads[0] < places[1]
+    assert body.count("for (int i = 0; i < FM; i += 2)") == 1 and body[places[1]:].rstrip().endswith("}\n}")
+
+
 @pytest.mark.parametrize("rows,width,outputs,pays", [
     (1, 1024, 151936, False), (10, 1024, 16448, False), (16, 512, 32768, False), (8, 1280, 65536, False),
     (11, 1024, 151936, True), (1, 1024, 16384, True), (1, 1536, 151936, True), (16, 768, 32768, True),

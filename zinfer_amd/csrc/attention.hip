@@ -155,14 +155,6 @@ __global__ __launch_bounds__(ZF_WAVE) void paged_attention_wave_kernel(
 // faster at 512 behind 1536.
 #define SPLIT_WAVES 4
 
-// a wave's own LDS accesses run in order; this keeps the compiler from moving them
-__device__ __forceinline__ void wave_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-//
 // FUSED, a decode step (sequence s's one token; the grid's x counts sequences): q, k and v come as the row of
 // the q/k/v product.  The first wave norms and rotates the head's q and its kv head's k as
 // zf_qk_norm_rope_kv_write does, a part of the wave each, and the first head of a group stores the

@@ -1537,6 +1537,7 @@ __device__ __forceinline__ void store_blocks_bf16(const f32x4_t (&acc)[FM][FN], 
         }
       }
     }
+    wave_fence();               // the slab is written
     const int n_out = EPI_GLU(EPI) ? N / 2 : N, nw_out = EPI_GLU(EPI) ? nw / 2 : nw;
 #pragma unroll
     for (int it = 0; it < (32 * LPR + 63) / 64; ++it) {
@@ -1546,6 +1547,7 @@ __device__ __forceinline__ void store_blocks_bf16(const f32x4_t (&acc)[FM][FN], 
         if (m < M && n < n_out) *(u32x4_t*)((bf16_t*)Cv + (size_t)m * n_out + n) = v;
       }
     }
+    wave_fence();               // and read, before it is written again
   }
 }
 

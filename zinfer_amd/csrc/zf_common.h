@@ -39,6 +39,14 @@ template <> __device__ __forceinline__ void store_from_float<bf16_t>(bf16_t* p, 
   *p = float_to_bf16(v);
 }
 
+// Between what a wave's lanes lay down in LDS and what its other lanes read there (or the other way round): a
+// wave's LDS accesses run in order, this keeps the compiler from moving them.  No instruction.
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The value of lane l xor OFF, OFF 1, 2, 4 or 8: register moves within a row of 16 lanes instead of a
 // shuffle's way through LDS (about 60 cycles a step).  OFF 4 takes the quads of four lanes with
 // an even number from the quad behind and those with an odd one from the quad before.
