@@ -338,6 +338,19 @@ def test_residual_sums_of_several_hundred_tokens_over_a_long_k_take_wide_tiles_s
         assert ops._wide_ksplit(M, N, K) is None, (M, N, K)
 
 
+def test_residual_sums_that_were_split_keep_their_norm():
+    """What `_tile_ksplit` would split along K `gemm_sum_norm` takes, whichever tiles come first by the
+    rules; and a plan of the whole K is the ring's alone."""
+    from types import SimpleNamespace
+    for M in (129, 200, 256, 333, 400, 512, 640, 777, 1000, 1280, 2048):
+        for N in (192, 256, 1024, 2048, 2560, 4096, 4160, 5120, 8192):
+            for K in (1024, 2048, 2112, 3072, 4096, 5120, 9728, 12288, 17408):
+                w = SimpleNamespace(dtype=torch.bfloat16, is_cuda=True, shape=(N, K))
+                plan = ops.sum_norm_plan(M, N, K, w, True)
+                assert plan is not None or ops._tile_ksplit(M, N, K) < 2, (M, N, K)
+                assert plan is None or plan[-1] >= 2 or plan[0] == "ring", (M, N, K, plan)
+
+
 def test_shared_arrays_accessed_in_16_byte_pieces_say_that_they_are_aligned():
     """A kernel's LDS arrays of smaller elements that it reads or writes as vectors carry the
     alignment: their type alone promises two or four bytes."""

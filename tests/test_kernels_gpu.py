@@ -2161,11 +2161,11 @@ def test_gemm_tiles_through_a_ring_of_stages(shape, M, N, K):
             assert bool(((normed.double() - norm).abs() <= (2.0 ** -8 + (N + 8) * 2.0 ** -24) * norm.abs()).all())
 
 
-@pytest.mark.parametrize("M,N,K,plan", [(256, 1024, 2048, ("ring", 32, 3)), (512, 2048, 1024, None),
-                                        (384, 4096, 2048, None), (400, 4096, 12288, ("ring", 33, 4))])
+@pytest.mark.parametrize("M,N,K,plan", [(256, 1024, 2048, ("ring", 32, 3)), (512, 2048, 1024, ("ring", 32, 1)),
+                                        (384, 4096, 2048, ("ring", 31, 1)), (400, 4096, 12288, ("ring", 33, 4))])
 def test_gemm_takes_the_ring_where_the_rule_says(M, N, K, plan):
     """The products that the rules send there have the bits of the kernel called by itself, and a residual sum
-    the same ones with and without the norm behind it."""
+    the same ones with and without the norm behind it; behind a sum of the whole K that norm is its kernel's."""
     ops = _ops()
     a = _rand((M, K), torch.bfloat16, 116).to(DEV)
     wt = ops.pretile_weight(_rand((N, K), torch.bfloat16, 117, 0.05).to(DEV))
@@ -2173,13 +2173,16 @@ def test_gemm_takes_the_ring_where_the_rule_says(M, N, K, plan):
     one = _rand((M, N), torch.float32, 118).to(DEV)
     two, normed = one.clone(), torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
     ops.gemm(a, wt, one, True, w_tiled=True)
-    if plan is not None:
-        ops.gemm_sum_norm(a, wt, two, torch.ones(N, device=DEV), 1e-6, normed)
-    else:
-        shape, parts = ops._ring_sum(M, N, K)
-        assert parts == 1
-        ops.gemm(a, wt, two, True, w_tiled=True, tile_variant=shape)
+    gain = (1 + 0.1 * _rand((N,), torch.float32, 119)).to(DEV)
+    base = two.clone()
+    ops.gemm_sum_norm(a, wt, two, gain, 1e-6, normed)
     assert torch.equal(one, two)
+    if plan[-1] == 1:
+        ops.gemm(a, wt, base, True, w_tiled=True, tile_variant=plan[1])
+        assert torch.equal(base, two)
+        alone = torch.empty_like(normed)
+        ops.rmsnorm(two, gain, 1e-6, alone)
+        assert torch.equal(alone, normed)
     for call, width in ((ops.gemm, N), (ops.gemm_swiglu, N // 2)):
         shape = ops._ring_choice(M, N, K, width != N)
         if shape is not None:

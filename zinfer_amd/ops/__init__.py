@@ -1433,8 +1433,9 @@ def sum_norm_plan(M: int, N: int, K: int, w: torch.Tensor, w_tiled: bool):
     """The plan if ``gemm_sum_norm`` covers residual += a w^T: a product that is split along K
     anyway (by measurement at 1 to 64 tokens, by rule at 17 to 128, or a few hundred tokens on
     a narrow output, or up to 2048 on a long K), whose partials one kernel can add, sum into the
-    residual and norm; else None.  ('mid' | 'tile' | 'wide' | 'tile256' | 'skinny' | 'ring', [row groups per workgroup
-    or the tile,] workgroups along K)."""
+    residual and norm, or one through the ring's tiles with its K whole, behind which the norm's own
+    kernel runs; else None.  ('mid' | 'tile' | 'wide' | 'tile256' | 'skinny' | 'ring', [row groups
+    per workgroup or the tile,] workgroups along K)."""
     if not (w_tiled and w.dtype == torch.bfloat16 and w.is_cuda and N % 16 == 0 and N <= 8192):
         return None
     if M <= NORM_FOLD_MAX_M:
@@ -1450,7 +1451,7 @@ def sum_norm_plan(M: int, N: int, K: int, w: torch.Tensor, w_tiled: bool):
         return ("wide", wide)
     ring = _ring_sum(M, N, K)
     if ring is not None:
-        return ("ring",) + ring if ring[1] > 1 else None
+        return ("ring",) + ring
     ks = _tile_ksplit(M, N, K)
     return ("tile", ks) if ks >= 2 else None
 
@@ -1509,7 +1510,8 @@ def _wide_ksplit(M: int, N: int, K: int):
 def gemm_sum_norm(a: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, gain: torch.Tensor,
                   eps: float, normed: torch.Tensor) -> None:
     """residual += a w^T in 32-bit (``w`` pre-tiled) and normed = bfloat16(rmsnorm(residual,
-    gain, eps)), the norm from the kernel that adds the product's partials.  float32 operands
+    gain, eps)), the norm from the kernel that adds the product's partials (behind a product that
+    is not split, from its own).  float32 operands
     (``f32_sum_norm_covers``): ``w`` in rows, ``normed`` float32."""
     _need_gpu(a, w, residual, gain, normed)
     M, K = a.shape
@@ -1536,9 +1538,15 @@ def gemm_sum_norm(a: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, gain
         raise KernelUnavailable(f"gemm_sum_norm: a {tuple(a.shape)} {a.dtype}, w "
                                 f"{tuple(w.shape)}, residual {tuple(residual.shape)} "
                                 f"{residual.dtype}")
-    ks = plan[-1]
-    ws = _workspace("gemm_splitk", ks * M * N, torch.float32, a.device)
     lib = build.load("gemm")
+    ks = plan[-1]
+    if plan[0] == "ring" and ks == 1:
+        _check(lib.zf_gemm_bf16_tile(_ptr(a), _ptr(w), _ptr(residual), M, N, K, _EPI_ACC_F32, plan[1], 1,
+                                     _stream()), "gemm_sum_norm (tiles through a ring of stages)")
+        _check(build.load("elementwise").zf_rmsnorm(_ptr(residual), _ptr(gain), _ptr(normed), _dt(normed), M, N,
+                                                    ctypes.c_float(eps), _stream()), "gemm_sum_norm (norm)")
+        return
+    ws = _workspace("gemm_splitk", ks * M * N, torch.float32, a.device)
     if plan[0] == "tile256":
         _check(lib.zf_gemm_bf16_tile256_splitk(_ptr(a), _ptr(w), _ptr(residual), _ptr(ws), M, N, K, ks,
                                                _ptr(gain), ctypes.c_float(eps), _ptr(normed),
