@@ -391,6 +391,29 @@ def test_rows_that_change_lanes_in_a_waves_slab_do_so_across_fences():
     assert body.count("for (int i = 0; i < FM; i += 2)") == 1 and body[places[1]:].rstrip().endswith("}\n}")
 
 
+def test_tiles_of_products_keep_their_sums_in_registers(tmp_path):
+    """No product's kernel in the built library has scratch memory: up to 256 accumulators and what the loop
+    and either epilogue need fit a lane's 512 registers."""
+    import os
+    import re
+    import shutil
+    import subprocess
+    from zinfer_amd.ops import build
+    tools = "/opt/rocm/llvm/bin/"
+    if not os.path.exists(tools + "llvm-readelf"):
+        pytest.skip("no tools that list a library's kernels")
+    shutil.copy(build.load("gemm")._name, tmp_path / "gemm.so")
+    subprocess.run([tools + "llvm-objdump", "--offloading", "gemm.so"], cwd=tmp_path, check=True,
+                   capture_output=True)
+    code, = tmp_path.glob("*gfx950")
+    notes = subprocess.run([tools + "llvm-readelf", "--notes", str(code)], check=True, capture_output=True,
+                           text=True).stdout
+    scratch = dict(zip(re.findall(r"\.symbol: +'?(\w+)\.kd", notes),
+                       map(int, re.findall(r"\.private_segment_fixed_size: (\d+)", notes))))
+    assert sum("gemm_bf16_tile256_kernel" in name for name in scratch) >= 21
+    assert not {name: size for name, size in scratch.items() if size}
+
+
 @pytest.mark.parametrize("rows,width,outputs,pays", [
     (1, 1024, 151936, False), (10, 1024, 16448, False), (16, 512, 32768, False), (8, 1280, 65536, False),
     (11, 1024, 151936, True), (1, 1024, 16384, True), (1, 1536, 151936, True), (16, 768, 32768, True),

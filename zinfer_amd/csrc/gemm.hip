@@ -1475,6 +1475,17 @@ constexpr int reads_before(int m, int nr) { return (m + 1) / 2 < nr ? (m + 1) / 
 // What the kernels leave whose waves hold FM x FN blocks of 16 tokens x 16 outputs with W's rows as the
 // first operand: lane 16 g + c has outputs 4 g .. 4 g + 3 of token c of a block; the wave's first
 // token and output are mw and nw.  Two blocks of tokens at a time.
+// (256 accumulators stay where the MFMAs left them until their block is stored: the compiler would take
+// all of them into the other half of the registers ahead of the first branch, and where two epilogues
+// follow spill 15 to 60.  Measured, us, without -> with: 4096 tokens into 5120 over 25600 added, its last round split,
+// 769 -> 734, SwiGLU pairs of 2048 tokens into 24576 over 4096 291 -> 284, 8192 added into 4096 over 12288
+// 575 -> 558, GEGLU pairs of 8192 into 51200 over 5120 2894 -> 2911.)
+template <int FM, int FN>
+__device__ __forceinline__ f32x4_t block_of(const f32x4_t& sums) {
+  f32x4_t v = sums;
+  if constexpr (FM * FN >= 64) asm volatile("" : "+a"(v));
+  return v;
+}
 // float32: 16 bytes a lane as they are, 64 bytes of a row in a run.
 template <int FM, int FN, bool ADD>
 __device__ __forceinline__ void store_blocks_f32(const f32x4_t (&acc)[FM][FN], float* to, int mw, int nw, int M,
@@ -1496,8 +1507,10 @@ __device__ __forceinline__ void store_blocks_f32(const f32x4_t (&acc)[FM][FN], f
       const int m = mw + 16 * (i + ii) + tok;
 #pragma unroll
       for (int j = 0; j < FN; ++j)
-        if (m < M && nw + 16 * j < N)
-          *(f32x4_t*)(to + (size_t)m * N + nw + 16 * j + n4) = ADD ? old[ii][j] + acc[i + ii][j] : acc[i + ii][j];
+        if (m < M && nw + 16 * j < N) {
+          const f32x4_t v = block_of<FM, FN>(acc[i + ii][j]);
+          *(f32x4_t*)(to + (size_t)m * N + nw + 16 * j + n4) = ADD ? old[ii][j] + v : v;
+        }
     }
   }
 }
@@ -1520,7 +1533,7 @@ __device__ __forceinline__ void store_blocks_bf16(const f32x4_t (&acc)[FM][FN], 
       if constexpr (EPI_GLU(EPI)) {       // gate columns, then the up columns that belong to them
 #pragma unroll
         for (int j = 0; j < FN; j += 2) {
-          f32x4_t g = acc[i + ii][j], u = acc[i + ii][j + 1];
+          f32x4_t g = block_of<FM, FN>(acc[i + ii][j]), u = block_of<FM, FN>(acc[i + ii][j + 1]);
           if constexpr (EPI == EPI_GEGLU)
             if (glu_bias != nullptr && nw + 16 * j < N) {
               g += *(const f32x4_t*)(glu_bias + nw + 16 * j + n4);
@@ -1532,7 +1545,7 @@ __device__ __forceinline__ void store_blocks_bf16(const f32x4_t (&acc)[FM][FN], 
       } else {
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-          const f32x4_t v = acc[i + ii][j];
+          const f32x4_t v = block_of<FM, FN>(acc[i + ii][j]);
           row[4 * j] = u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
         }
       }
