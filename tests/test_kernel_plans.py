@@ -391,9 +391,8 @@ def test_rows_that_change_lanes_in_a_waves_slab_do_so_across_fences():
     assert body.count("for (int i = 0; i < FM; i += 2)") == 1 and body[places[1]:].rstrip().endswith("}\n}")
 
 
-def test_tiles_of_products_keep_their_sums_in_registers(tmp_path):
-    """No product's kernel in the built library has scratch memory: up to 256 accumulators and what the loop
-    and either epilogue need fit a lane's 512 registers."""
+def _built_kernels(module, folder):
+    """Scratch bytes and vector registers of the kernels in the built library, by name."""
     import os
     import re
     import shutil
@@ -402,16 +401,33 @@ def test_tiles_of_products_keep_their_sums_in_registers(tmp_path):
     tools = "/opt/rocm/llvm/bin/"
     if not os.path.exists(tools + "llvm-readelf"):
         pytest.skip("no tools that list a library's kernels")
-    shutil.copy(build.load("gemm")._name, tmp_path / "gemm.so")
-    subprocess.run([tools + "llvm-objdump", "--offloading", "gemm.so"], cwd=tmp_path, check=True,
-                   capture_output=True)
-    code, = tmp_path.glob("*gfx950")
+    shutil.copy(build.load(module)._name, folder / "built.so")
+    subprocess.run([tools + "llvm-objdump", "--offloading", "built.so"], cwd=folder, check=True, capture_output=True)
+    code, = folder.glob("*gfx950")
     notes = subprocess.run([tools + "llvm-readelf", "--notes", str(code)], check=True, capture_output=True,
                            text=True).stdout
-    scratch = dict(zip(re.findall(r"\.symbol: +'?(\w+)\.kd", notes),
-                       map(int, re.findall(r"\.private_segment_fixed_size: (\d+)", notes))))
-    assert sum("gemm_bf16_tile256_kernel" in name for name in scratch) >= 21
-    assert not {name: size for name, size in scratch.items() if size}
+    # (a kernel's fields come in alphabetical order)
+    return {name: (int(scratch), int(registers)) for scratch, name, registers in re.findall(
+        r"\.private_segment_fixed_size: (\d+).*?\.symbol: +'?(\w+)\.kd.*?\.vgpr_count: +(\d+)", notes, re.S)}
+
+
+def test_tiles_of_products_keep_their_sums_in_registers(tmp_path):
+    """No product's kernel in the built library has scratch memory: up to 256 accumulators and what the loop
+    and either epilogue need fit a lane's 512 registers."""
+    kernels = _built_kernels("gemm", tmp_path)
+    assert sum("gemm_bf16_tile256_kernel" in name for name in kernels) >= 21
+    assert not {name: scratch for name, (scratch, _) in kernels.items() if scratch}
+
+
+def test_attention_in_32_bit_leaves_a_simd_its_waves(tmp_path):
+    """The 32-bit attention of many waves that only reads the pools: five waves a SIMD with heads of 64 (512
+    registers among them), two with heads of 128; the decode step's too without scratch memory."""
+    kernels = {name: k for name, k in _built_kernels("attention", tmp_path).items()
+               if "paged_attention_split_kernel" in name}
+    assert len(kernels) == 12 and not any(scratch for scratch, _ in kernels.values())
+    for name, (_, registers) in kernels.items():
+        reads_only_64 = "kernelILi4E" in name and "ELb0E" in name
+        assert registers <= (512 // 5 if reads_only_64 else 256), (name, registers)
 
 
 @pytest.mark.parametrize("rows,width,outputs,pays", [

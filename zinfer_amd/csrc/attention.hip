@@ -171,9 +171,16 @@ struct FusedRows {
   int table_rows;
 };
 
+// The pools as the kernel reads them.  Not FUSED it writes nothing that they could hold, and the compiler is told:
+// it else keeps loads apart from the stores ahead of the loop at the price of 26 to 38 registers, which is
+// waves of other workgroups (heads of 64: 135 for 100, three waves a SIMD for five; 64 sequences of 2360 tokens
+// in portions, 16 heads over 2, 155 us for 120; heads of 128, 1354 tokens behind up to 1000, 598 for 518).
+template <bool FUSED> struct ReadPool { typedef const float* __restrict__ type; };
+template <> struct ReadPool<true> { typedef const float* type; };
+
 template <int NV, int NW, bool FUSED>
 __global__ __launch_bounds__(NW * ZF_WAVE, 2) void paged_attention_split_kernel(
-    const float* __restrict__ q, const float* k_pool, const float* v_pool,
+    const float* __restrict__ q, typename ReadPool<FUSED>::type k_pool, typename ReadPool<FUSED>::type v_pool,
     const int* __restrict__ block_table, const int* __restrict__ q_start,
     const int* __restrict__ ctx_len, const int* __restrict__ seq_index, float* __restrict__ out,
     float scale, int window, int nH, int nKV, int page_size, int max_pages, FusedRows rows) {
