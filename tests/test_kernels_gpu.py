@@ -2116,6 +2116,17 @@ def test_gemm_float32_tiles_keep_the_order_of_few_rows(M, N, K, accumulate):
     assert bool(((got.double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(70, 2052, 64), (65, 100, 736), (80, 100, 768), (170, 4096, 992), (170, 4096, 1024),
+                                   (171, 4100, 96), (520, 58260, 64), (2050, 1000, 32), (1000, 8, 32),
+                                   (20, 24580, 288), (20, 24572, 288), (32, 260, 352), (5, 65540, 320), (9, 65532, 320),
+                                   (16, 12, 256), (16, 12, 260), (8, 4112, 384),
+                                   (9, 4112, 384), (3, 4100, 1285), (3, 4096, 1285)])
+def test_gemm_float32_on_either_side_of_its_rules(M, N, K):
+    """Tiles of 32 with one and two groups of waves, 32 x 64 and 64 x 64, one step of K; one and two steps in
+    flight, of spans of one, two and three steps, narrow and wide: every choice keeps the order."""
+    test_gemm_float32_tiles_keep_the_order_of_few_rows(M, N, K, False)
+
+
 # k-tiles of 64: fewer than the ring's stages, and every end of its turn (3, 4 or 5 of them)
 @pytest.mark.parametrize("M,N,K", [(129, 80, 64), (200, 64, 128), (191, 336, 192), (65, 144, 320), (321, 176, 384),
                                    (128, 128, 448), (300, 400, 512), (450, 272, 576), (257, 656, 1088)])

@@ -161,7 +161,7 @@ __device__ __forceinline__ void tile_of_workgroup(int b, int tiles_m, int tiles_
 //   * up to 64 rows, bound by reading W (one user of the 0.6B shape's float32 weights: 1.9 GB a
 //     token): a workgroup of eight waves, one span each, takes 16 rows of W (32 with a wide
 //     output) for all tokens; a wave's loads of a step are 16 whole lines of 128 bytes, straight
-//     into the operands, two steps in flight; the eight partials meet in LDS.  For narrow outputs
+//     into the operands, up to two steps in flight; the eight partials meet in LDS.  For narrow outputs
 //     every span is a workgroup, and a second kernel adds the spans (gemm_f32_spans_kernel).
 //   * above, bound by the MFMAs: tiles through a ring of LDS stages (gemm_f32_ring_kernel); of other
 //     sizes, alignments and outputs tiles of 128 x 128, 64 x 64 or 32 x 32 through LDS (rows of 36
@@ -209,7 +209,7 @@ __device__ __forceinline__ void f32_store4(TO* __restrict__ C, int m, int n, int
 // row groups are the same rows of both, and silu(gate) * up of the 32-bit sums is stored: the bits of
 // the product and zf_swiglu behind it, without the launch and the way through memory (4 tokens,
 // 6144 rows of 1024: 8.1 + 4.7 -> 9.1 us in the trace).
-template <typename TO, bool ACC, int RG, int MT, bool VEC, bool GLU = false>
+template <typename TO, bool ACC, int RG, int MT, bool VEC, int SETS, bool GLU = false>
 __global__ __launch_bounds__(F32_SPANS * 64) void gemm_f32_stream_kernel(
     const float* __restrict__ A, const float* __restrict__ W, TO* __restrict__ C, int M, int N,
     int K, int span, bool vec_out) {
@@ -230,11 +230,8 @@ __global__ __launch_bounds__(F32_SPANS * 64) void gemm_f32_stream_kernel(
   for (int i = 0; i < RG; ++i)
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  // Two steps in flight: the next but one is asked for behind the products that free its registers (as
-  // a loop that asked for two or four steps and then multiplied them, 4 tokens: 4096 rows of 1024 6.7 ->
-  // 5.9 us, of 4096 24.4 -> 16.2, SwiGLU of 3072 pairs of 1024 9.4 -> 8.7).  With four groups of tokens one
-  // step at a time: the registers of two leave a CU fewer waves (64 tokens into 6144 over 1024 22.9 -> 23.6).
-  constexpr int SETS = RG * MT >= 4 ? 1 : 2;
+  // SETS 2, two steps in flight: the next but one is asked for behind the products that free its registers.
+  // SETS 1, a loop that asks for a few steps and then multiplies them: fewer registers and so more waves.
   const int k_first = wave * span, k_end = min(K, k_first + span);
   f32x4_t wf[SETS][RG][2], af[SETS][MT][2];
   auto load = [&](int b, int k0) __attribute__((always_inline)) {      // (steps beyond the span: zeros)
@@ -259,7 +256,7 @@ __global__ __launch_bounds__(F32_SPANS * 64) void gemm_f32_stream_kernel(
                                                            acc[i][j], 0, 0, 0);
   };
   if constexpr (SETS == 1) {
-#pragma unroll 1
+#pragma unroll (RG * MT >= 4 ? 1 : RG * MT == 2 ? 2 : 4)
     for (int k0 = k_first; k0 < k_end; k0 += 32) {
       load(0, k0);
       multiply(0);
@@ -272,6 +269,7 @@ __global__ __launch_bounds__(F32_SPANS * 64) void gemm_f32_stream_kernel(
     for (int k0 = k_first; k0 < k_end; k0 += 64) {
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
+        if (b == 1 && k0 + 32 >= k_end) break;
         multiply(b);
         __builtin_amdgcn_sched_barrier(0);
         if (k0 + 64 < k_end) {
@@ -549,7 +547,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_f32_ring_kernel(
   for (int c = 0; c < WC; ++c) wsrc[c] = source(tid + 256 * c, N - n0);
   // this group's steps: from `first` on; steps behind the last are the last again, and not added
   const int steps = K / 32, per = span / 32, last = steps - 1, first = kg * (F32_SPANS / 2) * per;
-  const int stages = KG > 1 ? F32_SPANS / 2 * per : steps;
+  const int stages = KG > 1 ? min(F32_SPANS / 2 * per, steps) : steps;
   auto copies = [&](int stage, u32x4_t* to) __attribute__((always_inline)) {
     const uint32_t at = (uint32_t)min(first + stage, last) * 128;
 #pragma unroll
@@ -635,11 +633,20 @@ __global__ __launch_bounds__(256 * KG) void gemm_f32_ring_kernel(
       ++span_at;
     }
   };
-  for (int t = 0; t < stages; t += NS) {
+  int t = 0;
+  for (; t + NS <= stages; t += NS) {
     step(t, I0{});
     step(t + 1, I1{});
     step(t + 2, I2{});
     if constexpr (NS > 3) step(t + 3, I3{});
+  }
+  if (t < stages) {
+    step(t, I0{});
+    if (t + 1 < stages) {
+      step(t + 1, I1{});
+      if constexpr (NS > 3)
+        if (t + 2 < stages) step(t + 2, I2{});
+    }
   }
   // nothing may still be on its way into LDS when the workgroup ends
   __builtin_amdgcn_s_waitcnt(0x0f70);       // vmcnt(0)
@@ -663,12 +670,25 @@ __global__ __launch_bounds__(256 * KG) void gemm_f32_ring_kernel(
 #endif
 }
 
+// Whether the streaming kernel keeps two steps in flight: not in spans of one step, not where the outputs are so
+// many that more waves a CU do as well, and of few rows not where they are one and a half workgroups of 16 a CU or
+// two.  Measured, us, one step / two: 1 row into 1024 over 1024 6.1 / 5.2, over 4096 17.7 / 12.0, into 16384 over 4096
+// 53.8 / 51.0, into 65536 over 256 13.6 / 15.4, over 1024 49.7 / 49.7; 17 into 6144 over 4096 43.9 / 40.8, into
+// 16384 over 320 9.0 / 9.2, into 32768 over 256 12.8 / 14.4, over 320 16.0 / 17.1, over 1024 44.8 / 44.7; 1 into 6144
+// over 768 6.7 / 7.2, over 2048 15.8 / 15.3, 16 over 768 8.5 / 8.4.  Of rows that are not aligned, number by number,
+// only into few outputs over a long K: 4 into 4096 over 541 6.9 / 7.6, over 1743 20.5 / 18.6.
+static bool f32_two_sets(int M, int N, int K, bool vec) {
+  if (K <= 256 || N >= (M <= 16 ? 65536 : 24576)) return false;
+  if (!vec) return N <= 4096 && K > 1280;
+  return M > 8 || N <= 4096 || N > 8192 || K >= 2048;
+}
+
 template <typename TO, bool ACC, bool VEC>
 static void launch_f32(const float* A, const float* W, TO* C, int M, int N, int K, bool vec_out,
                        hipStream_t stream) {
   const int span = f32_span(K);
-#define F32_STREAM(RG, MT)                                                                       \
-  hipLaunchKernelGGL((gemm_f32_stream_kernel<TO, ACC, RG, MT, VEC>),                             \
+#define F32_STREAM(RG, MT, SETS)                                                                 \
+  hipLaunchKernelGGL((gemm_f32_stream_kernel<TO, ACC, RG, MT, VEC, SETS>),                       \
                      dim3((N + 16 * RG - 1) / (16 * RG), (M + 16 * MT - 1) / (16 * MT)),         \
                      dim3(F32_SPANS * 64), 0, stream, A, W, C, M, N, K, span, vec_out)
 #define F32_TILE(B, ST)                                                                          \
@@ -676,19 +696,32 @@ static void launch_f32(const float* A, const float* W, TO* C, int M, int N, int 
                      (M + B - 1) / B), dim3(256), 0, stream, A, W, C, M, N, K, span, vec_out)
   const auto tiles = [&](int b) { return (long long)((M + b - 1) / b) * ((N + b - 1) / b); };
   if (M <= 16) {
-    if (N >= 16384) F32_STREAM(2, 1); else F32_STREAM(1, 1);
+    const bool two = f32_two_sets(M, N, K, VEC);
+    if (N >= 16384) {
+      if (two) F32_STREAM(2, 1, 2); else F32_STREAM(2, 1, 1);
+    } else {
+      if (two) F32_STREAM(1, 1, 2); else F32_STREAM(1, 1, 1);
+    }
   } else if (M <= 32) {
-    F32_STREAM(1, 2);
+    if (f32_two_sets(M, N, K, VEC)) F32_STREAM(1, 2, 2); else F32_STREAM(1, 2, 1);
   } else if (M <= 64) {
-    F32_STREAM(1, 4);
-  } else if (VEC && std::is_same<TO, float>::value && vec_out && K > 0 && K % 32 == 0) {
-    // Two groups of waves on tiles of 32 x 32 while there are up to three of those a CU (131 rows into 4096
-    // over 1024, 640 tiles, 17.1 us, 32 x 64 20.6; 256 rows, 1024 tiles, 21.9 and 21.0); 64 x 64 where those
-    // are many and K long (1024 rows into 7168 over 2048 237 us, 32 x 64 245; 2048 into 6144 over 1024 209
-    // and 203)
-#define F32_RING(BM, BN, KG)                                                                       hipLaunchKernelGGL((gemm_f32_ring_kernel<BM, BN, KG, ACC>),                                                         dim3(((N + BN - 1) / BN) * ((M + BM - 1) / BM)), dim3(256 * KG), 0, stream, A, W,                      (float*)C, M, N, K, span, (M + BM - 1) / BM, (N + BN - 1) / BN)
-    if (tiles(32) <= 768) F32_RING(32, 32, 2);
-    else if (K >= 2048 && tiles(64) >= 1024) F32_RING(64, 64, 1);
+    F32_STREAM(1, 4, 1);
+  } else if (VEC && std::is_same<TO, float>::value && vec_out && K > 0 && K % 32 == 0 &&
+             (K > 32 || tiles(32) <= 768)) {
+    // Up to three tiles of 32 x 32 a CU those, from K = 768 on (1024 where they are more than two) with two
+    // groups of waves (us, one group / two: 65 rows into 2048 over 256 4.5 / 5.3, over 512 6.4 / 6.4, over 1024
+    // 9.7 / 8.7; 152 into 4096 over 512 11.2 / 12.7, over 1024 19.0 / 19.1; 131 over 1024, 640 tiles, so 17.1,
+    // 32 x 64 20.6); behind that 32 x 64 (256 rows, 1024 tiles, 21.9 and 21.0), and 64 x 64 where those are many
+    // and K long (1024 rows into 7168 over 2048 237 us, 32 x 64 245; 2048 into 6144 over 1024 209 and 203) or
+    // they are very many (2000 into 32768 over 64 124, 32 x 64 141).  One step of 32 over more tiles leaves a
+    // ring nothing to run ahead of: the tiles below (2000 into 32768 91 us, 32 x 64 here 114).
+#define F32_RING(BM, BN, KG)                                                                   \
+  hipLaunchKernelGGL((gemm_f32_ring_kernel<BM, BN, KG, ACC>),                                  \
+                     dim3(((N + BN - 1) / BN) * ((M + BM - 1) / BM)), dim3(256 * KG), 0, stream, A, W, \
+                     (float*)C, M, N, K, span, (M + BM - 1) / BM, (N + BN - 1) / BN)
+    if (tiles(32) <= 768 && K >= (tiles(32) <= 512 ? 768 : 1024)) F32_RING(32, 32, 2);
+    else if (tiles(32) <= 768) F32_RING(32, 32, 1);
+    else if (tiles(64) >= (K >= 2048 ? 1024 : 8192)) F32_RING(64, 64, 1);
     else F32_RING(32, 64, 1);
 #undef F32_RING
   } else if (tiles(128) >= 256) {
@@ -737,12 +770,16 @@ extern "C" int zf_gemm_f32_swiglu(const float* A, const float* W, float* C, int 
   const bool vec = K % 4 == 0 && ((uintptr_t)A | (uintptr_t)W) % 16 == 0;
   const bool vec_out = I % 4 == 0 && (uintptr_t)C % 16 == 0;
   const dim3 grid((I + 15) / 16);
-  if (vec)
-    hipLaunchKernelGGL((gemm_f32_stream_kernel<float, false, 2, 1, true, true>), grid,
-                       dim3(F32_SPANS * 64), 0, stream, A, W, C, M, I, K, f32_span(K), vec_out);
-  else
-    hipLaunchKernelGGL((gemm_f32_stream_kernel<float, false, 2, 1, false, true>), grid,
-                       dim3(F32_SPANS * 64), 0, stream, A, W, C, M, I, K, f32_span(K), vec_out);
+#define F32_GLU(VEC, SETS)                                                                             \
+  hipLaunchKernelGGL((gemm_f32_stream_kernel<float, false, 2, 1, VEC, SETS, true>), grid,              \
+                     dim3(F32_SPANS * 64), 0, stream, A, W, C, M, I, K, f32_span(K), vec_out)
+  const bool two = K > 256;       // (1 row, 3072 pairs over 1024 10.4 us, so 9.2; 24576 over 256 11.9, 14.8)
+  if (vec) {
+    if (two) F32_GLU(true, 2); else F32_GLU(true, 1);
+  } else {
+    if (two) F32_GLU(false, 2); else F32_GLU(false, 1);
+  }
+#undef F32_GLU
   ZF_CHECK_LAUNCH();
 }
 
