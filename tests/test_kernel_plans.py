@@ -474,6 +474,20 @@ def test_256_token_tiles_are_chosen_where_they_are_the_faster_per_flop():
         assert ops._tile256_ksplit(M, N, K) != 2, (M, N, K)
 
 
+def test_256_token_tiles_leave_what_they_slow_down():
+    """On both sides of the lines that `_tile256_choice` and `_tile256_tail_split` draw by measurement: tiles of
+    192 outputs against a split last round and of one round, residual sums into few outputs, short K."""
+    for M, N, K, acc in ((698, 24576, 4096, False), (3648, 5120, 5120, True), (1920, 10240, 5120, False),
+                         (2688, 7168, 5120, False), (2816, 6144, 2560, False)):
+        assert ops._tile_tail_split(M, N, K) is not None and ops._tile256_choice(M, N, K, acc) != 21, (M, N, K)
+    assert ops._tile_tail_split(1024, 34816, 5120) is not None and ops._tile256_choice(1024, 34816, 5120) == 21
+    for M, N, K in ((1184, 4096, 4096), (3200, 2048, 6144), (2432, 2560, 4096)):
+        assert ops._tile256_choice(M, N, K, True) is None, (M, N, K)
+    assert ops._tile256_choice(1408, 5120, 5120, True) == 22
+    assert ops._tile256_tail_split(698, 24576, 4096) is not None
+    assert ops._tile256_tail_split(3381, 5120, 2048) is None and ops._tile256_tail_split(2816, 6144, 2560) is None
+
+
 def test_256_token_tiles_split_their_last_round_where_it_is_short():
     """`_tile256_tail_split`: whole rounds of 256 tiles and up to 128 behind them, in two to eight parts of
     at least 512 that fit the chip; not where a tile width fills it without."""

@@ -1075,19 +1075,26 @@ def _tile256_choice(M: int, N: int, K: int, accumulate: bool = False):
     the norm behind: 4096 into 4096 over 12288 359 -> 310, 8192 713 -> 622, over 4096 291 -> 265.
     Not where they are the slower ones: K under 2048 (what a tile costs besides; 4096 tokens into 6144
     over 1024 51 -> 52), tiles of 192 outputs over a K of 8192 and more (4096 tokens into 5120 over
-    17408 637 -> 668), residual sums whose last round is short (8192 tokens into 5120 over 8192
+    17408 637 -> 668), or of a round or less, and up to a round and three quarters where the 128 x 256 tiles split
+    a short last round (698 tokens into 24576 over 4096 140 -> 150, 3648 into 5120 over 5120 198 -> 215); residual
+    sums into few outputs through tiles of 128 (1184 tokens into 4096 over 4096 61 -> 67, 3200 into 2048 over
+    6144 89 -> 99; into 5120 over 5120 87 -> 84) or whose last round is short (8192 tokens into 5120 over 8192
     602 -> 616), and a last round that the 128 x 256 tiles split along K unless a tenth is gained
-    (512 tokens into 34816 over 5120 165 -> 172).  Of 131 products of six shapes, 256 to 8192 tokens,
-    one is 1 % slower so and none more."""
+    (512 tokens into 34816 over 5120 165 -> 172).  Of 1062 drawn products that this rule could move, timed in
+    changing order, it gains 7 % in the mean and makes 33 slower by more than 3 %, the worst by 8."""
     even = _tile256_variant(M, N, K, accumulate)
     if even is not None:
         return even
     now = _tile_variant(M, N, True, accumulate, K)
     if now not in (10, 12) or not _tile256_covers(M, N, K, accumulate):
         return None
-    best = min((20, 21, 22) if K < 8192 else (20, 22),
+    tail = now == 10 and _tile_tail_split(M, N, K) is not None
+    tiles = ((M + 255) // 256) * ((N + 191) // 192)
+    best = min((20, 22) if K >= 8192 or tiles <= (448 if tail else 256) else (20, 21, 22),
                key=lambda v: _tile256_estimate(v, M, N, K, accumulate))
-    gain = 0.9 if now == 10 and _tile_tail_split(M, N, K) is not None else 0.95
+    if accumulate and best == 22 and now == 12 and N <= 4096 and K <= 6144:
+        return None
+    gain = 0.9 if tail else 0.95
     return best if _tile256_estimate(best, M, N, K, accumulate) < gain * _tile128_estimate(M, N, K, now) \
         else None
 
@@ -1105,7 +1112,8 @@ def _tile256_tail_split(M: int, N: int, K: int, accumulate: bool = False):
     """(whole, split) if a product should run through the 256 x 256 tiles with the last, short round
     of them split along K, else None: ``whole`` tiles fill whole rounds of the chip's 256 CUs, each of
     the others goes to ``split`` workgroups.  Where the estimates see a gain of 3 % over what runs
-    otherwise.  Measured on MI355X, us: 4096 tokens into 5120 over 25600 (320 tiles, the last 64 in four
+    otherwise, and not over a K under 3072 in the place of 128 x 256 tiles that split theirs (3381 tokens into
+    5120 over 2048, SwiGLU, 9 % slower).  Measured on MI355X, us: 4096 tokens into 5120 over 25600 (320 tiles, the last 64 in four
     parts) 920 -> 782, over 17408 626 -> 553, 8192 over 25600 1661 -> 1540; 512 tokens into 34816 over 5120
     (the last 16 of 272 in eight) 165 -> 156, 1024 into 51200 446 -> 404, 768 342 -> 321."""
     if not _tile256_covers(M, N, K, accumulate):
@@ -1124,6 +1132,8 @@ def _tile256_tail_split(M: int, N: int, K: int, accumulate: bool = False):
     else:
         now = _tile_variant(M, N, True, accumulate, K)
         if now not in (10, 12):
+            return None
+        if K < 3072 and now == 10 and _tile_tail_split(M, N, K) is not None:
             return None
         other = _tile128_estimate(M, N, K, now)
     return (tiles - rest, split) if _tile256_estimate(20, M, N, K, accumulate, split) < 0.97 * other else None
