@@ -521,6 +521,16 @@ def test_decode_attention_takes_partials_in_one_round_of_the_chip():
         assert not takes(*args), args
 
 
+def test_decode_attention_in_32_bit_where_it_pays():
+    """`decode_attention_float32_pays`: not with four heads and more to a kv head, 2048 workgroups and more, and
+    contexts between two chunks of keys and 1024."""
+    pays = ops.decode_attention_float32_pays
+    for args in ((64, 32, 4, 200), (64, 32, 8, 129), (128, 16, 1, 1024), (32, 64, 8, 600)):
+        assert not pays(*args), args
+    for args in ((63, 32, 8, 200), (64, 32, 4, 128), (64, 32, 4, 1025), (200, 16, 8, 200), (4, 16, 8, 4000)):
+        assert pays(*args), args
+
+
 def test_tiles_through_a_ring_are_chosen_where_one_round_holds_the_product():
     """`_ring_choice` takes the smallest tile of which 256 hold the product, `_ring_sum` one round of tiles in up
     to six parts of K behind the splits of larger tiles; neither where the kernels do not cover the sizes."""

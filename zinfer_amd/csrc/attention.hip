@@ -162,7 +162,7 @@ __global__ __launch_bounds__(ZF_WAVE) void paged_attention_wave_kernel(
 // on its way there or anything else and is not used.  The same bits as the two kernels, in one launch
 // less.  Measured (16 heads of 128 over 8, us, the two kernels / this one): one sequence of 32 keys 6.5 / 4.8, 4 of
 // 200 10.1 / 8.3, 16 of 1000 31.8 / 29.8, 200 of 200 90 / 87; heads of 64 16 of 200 8.8 / 7.1; 32 heads over 4, 64
-// of 200 35.8 / 36.2, of 40 11.8 / 10.0.
+// of 200 35.8 / 36.2 (such steps keep the two kernels), of 40 11.8 / 10.0.
 struct FusedRows {
   const float *qkv, *q_gain, *k_gain, *cos_t, *sin_t;
   const int *positions, *slot_mapping;

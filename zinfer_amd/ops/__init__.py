@@ -1932,6 +1932,18 @@ def decode_attention_float32_covers(qkv, q_gain, k_gain, cos, sin, k_pool, v_poo
                 for t in given)
 
 
+def decode_attention_float32_pays(n_seqs: int, n_heads: int, n_kv_heads: int, max_ctx_len: int) -> bool:
+    """Whether a step should take ``decode_attention_float32`` where it covers the sizes.  Every head of a group
+    norms and rotates its kv head's key again, and of many workgroups of four waves (contexts of more than two
+    chunks of keys) the longer start costs what the launch saved, until the keys themselves take over.  Measured on
+    MI355X, us, two kernels -> this one, heads of 128: 64 sequences of 200 keys, 32 heads over 4, 35.8 -> 36.2, over
+    8 42.0 -> 42.1, 64 over 8 64.2 -> 67.0, 128 of 200 118.2 -> 127.0, 64 of 600 141.0 -> 143.3;
+    but of 60 22.2 -> 19.5, 32 over 4 of 2000 229.7 -> 227.0, 32 sequences of 200 18.3 -> 17.5, and 128 with 16 over
+    8 56.8 -> 54.6."""
+    return n_heads < 4 * n_kv_heads or n_seqs * n_heads < 2048 \
+        or not 2 * ATTENTION_CHUNK_KEYS < max_ctx_len <= 1024
+
+
 @_launches("attention")
 def decode_attention_float32(qkv, q_gain, k_gain, eps, cos, sin, positions, slot_mapping, k_pool, v_pool,
                              block_table, q_start, ctx_len, out, scale, window, n_heads, n_kv_heads,

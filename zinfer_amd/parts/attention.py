@@ -149,10 +149,11 @@ class GqaAttention(Mixer):
             self.o.forward(attn, residual, accumulate=True, step=step)
             return
         if plain_position and step.max_q_len == 1 and T == step.n_seqs and cache.writes:
-            # and in 32-bit, where the step's sizes are that kernel's
+            # and in 32-bit, where the step's sizes are that kernel's and few enough
             cos, sin = tables if tables is not None else (None, None)
-            if ops.decode_attention_float32_covers(qkv, self.q_gain, self.k_gain, cos, sin, cache.k_pool,
-                                                   cache.v_pool, s.head_dim, cache.page_size, window):
+            if ops.decode_attention_float32_pays(step.n_seqs, s.n_heads, s.n_kv_heads, step.max_ctx_len) \
+                    and ops.decode_attention_float32_covers(qkv, self.q_gain, self.k_gain, cos, sin, cache.k_pool,
+                                                            cache.v_pool, s.head_dim, cache.page_size, window):
                 ops.decode_attention_float32(
                     qkv, self.q_gain, self.k_gain, eps, cos, sin, step.positions, kv.slot_mapping,
                     cache.k_pool, cache.v_pool, kv.block_table, step.q_start, step.ctx_len, attn,
