@@ -521,6 +521,16 @@ def test_decode_attention_takes_partials_in_one_round_of_the_chip():
         assert not takes(*args), args
 
 
+def test_decode_attention_counts_the_waves_that_it_launches():
+    """`decode_attention_waves`: four a split of 256 keys; eight a whole context of two to four splits from 192
+    pairs of sequence and kv head on, with four heads and more to a kv head of 128."""
+    waves = ops.decode_attention_waves
+    assert waves(24, 32, 8, 128, 2) == 8 * 192 and waves(64, 64, 8, 128, 4) == 8 * 512
+    for n, nH, nKV, hd, splits in ((24, 32, 8, 128, 1), (24, 32, 8, 128, 5), (23, 32, 8, 128, 2), (24, 24, 8, 128, 2),
+                                   (24, 32, 8, 64, 2), (1, 1, 1, 256, 7), (2000, 32, 8, 128, 40)):
+        assert waves(n, nH, nKV, hd, splits) == 4 * n * nKV * splits, (n, nH, nKV, hd, splits)
+
+
 def test_decode_attention_in_32_bit_where_it_pays():
     """`decode_attention_float32_pays`: not with four heads and more to a kv head, 2048 workgroups and more, and
     contexts between two chunks of keys and 1024."""

@@ -1130,6 +1130,14 @@ static bool decode_takes_whole(int n_seqs, int nH, int nKV, int hd, int max_spli
          nH / nKV >= 4;
 }
 
+// Waves that a decode step's attention is launched with (host rules count them)
+extern "C" long long zf_attn_decode_waves(int n_seqs, int nH, int nKV, int hd, int max_splits) {
+  const long long pairs = (long long)n_seqs * nKV;
+  return decode_takes_whole(n_seqs, nH, nKV, hd, max_splits)
+      ? pairs * WHOLE_WAVES
+      : pairs * max_splits * (DEC_SPLIT / DEC_WAVE_KEYS);
+}
+
 extern "C" int zf_attn_decode_bf16(const void* q, const void* k_pool, const void* v_pool,
                                    const int* block_table, const int* q_start,
                                    const int* ctx_len, void* out, float* ws_o, float* ws_ml,

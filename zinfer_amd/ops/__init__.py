@@ -1840,6 +1840,14 @@ FUSED_DECODE_MAX_SEQS = 32
 FUSED_DECODE_MAX_PARTS = 8
 
 
+@functools.lru_cache(maxsize=4096)
+def decode_attention_waves(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, splits: int) -> int:
+    """Waves of the bfloat16 decode attention's launch, as the launcher itself counts them."""
+    waves = build.load("attention").zf_attn_decode_waves
+    waves.restype = ctypes.c_longlong
+    return waves(n_seqs, n_heads, n_kv_heads, head_dim, splits)
+
+
 def fused_decode_takes_parts(n_seqs: int, ksplit: int, n_heads: int, n_kv_heads: int, head_dim: int,
                              max_ctx_len: int) -> bool:
     """Whether ``decode_attention_fused`` should take a split product's partials: where its workgroups
@@ -1850,10 +1858,8 @@ def fused_decode_takes_parts(n_seqs: int, ksplit: int, n_heads: int, n_kv_heads:
     22.8 -> 20.5 (whole contexts), 64 of 600 31.2 -> 32.7; 20 of 500 (two splits) 16.3 -> 15.2; 32 of 2000
     43.7 -> 46.0."""
     splits = max(1, (max_ctx_len + DECODE_SPLIT_KEYS - 1) // DECODE_SPLIT_KEYS)
-    pairs = n_seqs * n_kv_heads
-    whole = head_dim == 128 and 1 < splits <= 4 and pairs >= 192 and n_heads // n_kv_heads >= 4
-    waves = 8 * pairs if whole else 4 * pairs * splits
-    return head_dim == 128 and ksplit <= FUSED_DECODE_MAX_PARTS and waves <= 2048
+    return head_dim == 128 and ksplit <= FUSED_DECODE_MAX_PARTS \
+        and decode_attention_waves(n_seqs, n_heads, n_kv_heads, head_dim, splits) <= 2048
 
 
 @_launches("attention")
