@@ -2034,12 +2034,17 @@ def test_gemm_256_token_tiles_last_round_split_is_chosen():
         call(a, wt, whole, w_tiled=True, tile_variant=20)
         assert torch.equal(chosen, forced)
         assert rel_err(chosen, whole) <= tol(torch.bfloat16) and (chosen == whole).float().mean().item() > 0.9
-    chosen, forced = (torch.empty((M, N // 2), dtype=torch.bfloat16, device=DEV) for _ in range(2))
-    bias = _rand((N,), torch.float32, 106).to(DEV)
-    ops.gemm_geglu(a, wt, bias, chosen)
-    assert lib.zf_gemm_geglu(ops._ptr(a), ops._ptr(wt), ops._ptr(bias), ops._ptr(forced), ops._ptr(None), M, N, K,
-                             0, 20, 1, ops._stream()) == 0
-    assert rel_err(chosen, forced) <= tol(torch.bfloat16)
+    ws = torch.empty((260 - tail[0]) * tail[1] * 256 * 256, device=DEV)
+    for bias in (_rand((N,), torch.float32, 106).to(DEV), None):
+        chosen, forced, whole = (torch.empty((M, N // 2), dtype=torch.bfloat16, device=DEV) for _ in range(3))
+        ops.gemm_geglu(a, wt, bias, chosen)
+        for out, way, number, split in ((forced, 4) + tail, (whole, 0, 20, 1)):
+            assert lib.zf_gemm_geglu(ops._ptr(a), ops._ptr(wt), ops._ptr(bias), ops._ptr(out), ops._ptr(ws), M, N, K,
+                                     way, number, split, ops._stream()) == 0
+        assert torch.equal(chosen, forced)
+        assert rel_err(chosen, whole) <= tol(torch.bfloat16) and (chosen == whole).float().mean().item() > 0.9
+        # (that another path has other bits is what tells the two apart: a few of the split tiles' sums round apart)
+        assert not torch.equal(chosen, whole)
 
 
 @pytest.mark.parametrize("nH,nKV,page_size,window,n,longest,parts", [
