@@ -436,11 +436,25 @@ def test_gemm_256_token_tiles_are_chosen_and_agree():
         assert torch.equal(chosen, forced) and torch.equal(chosen, small)
 
 
+@pytest.mark.parametrize("M,N,K", [(512, 1024, 512), (300, 320, 192), (2049, 4096, 128)])
+def test_gemm_tiles_by_their_other_numbers(M, N, K):
+    """7 and 11 name tiles too: the bits of 6 and 10, for K's with and without an even number of k-tiles
+    and for more and fewer than the 384 tiles from which 6 copies the tokens straight into LDS."""
+    ops = _ops()
+    a = _rand((M, K), torch.bfloat16, 108).to(DEV)
+    wt = ops.pretile_weight(_rand((N, K), torch.bfloat16, 109, 0.05).to(DEV))
+    for other, variant in ((7, 6), (11, 10)):
+        got, want = (torch.full((M, N), float("nan"), dtype=torch.float32, device=DEV) for _ in range(2))
+        ops.gemm(a, wt, got, w_tiled=True, tile_variant=other)
+        ops.gemm(a, wt, want, w_tiled=True, tile_variant=variant)
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("variant", [20, 21, 22, 10, 16])
 @pytest.mark.parametrize("K", [4096, 12288])
 def test_gemm_tiled_kernels_at_a_served_k(variant, K):
-    """The tiled kernels at the K the engine runs them with (4096: 128 trips round the
-    256-token tiles' ring of four k-tiles of 32; 12288: the down product's), where the offsets
+    """The tiled kernels at the K the engine runs them with (4096: 64 k-tiles of 64 through
+    the 256-token tiles' stages; 12288: the down product's), where the offsets
     into both operands are largest: against the plain product and, bit for bit, the 128 x 128
     tiles; 64-token tiles of 128 outputs likewise."""
     ops = _ops()

@@ -2219,6 +2219,8 @@ static int launch_tile(const void* A, const void* W, void* C, int M, int N, int 
 //          each over half of K (K % 256 == 0): for 256 tiles or fewer, where a CU has one
 //          workgroup either way.  20, 21 and 22 = 256 tokens x 256, 192 and 128 (K % 128 == 0).
 //          30, 31 and 32 = 128x128, 128x64 and 64x64 with both operands in a ring of LDS stages.
+//          7 = 6 with the tokens through registers at any size, 11 = 10 by another number: no rule
+//          asks for them, callers that name a kernel may.
 extern "C" int zf_gemm_bf16_tile(const void* A, const void* W, void* C, int M, int N, int K,
                                  int epi, int variant, int w_tiled, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
@@ -2227,10 +2229,11 @@ extern "C" int zf_gemm_bf16_tile(const void* A, const void* W, void* C, int M, i
     if (N % 16 != 0 || K % 64 != 0) return -3;
     if (variant == 6 && (long long)((M + 127) / 128) * ((N + 127) / 128) >= 384)
       return launch_tile_wdirect<128, 128, 64, 64, TK, false, true>(A, W, C, M, N, K, epi, stream);
-    if (variant == 6) return launch_tile_wdirect<128, 128, 64, 64>(A, W, C, M, N, K, epi, stream);
+    if (variant == 6 || variant == 7)
+      return launch_tile_wdirect<128, 128, 64, 64>(A, W, C, M, N, K, epi, stream);
     if (variant == 16)
       return launch_tile_wdirect<128, 128, 128, 32, 128>(A, W, C, M, N, K, epi, stream);
-    if (variant == 10) {
+    if (variant == 10 || variant == 11) {
       if (K % (2 * TK) == 0)     // W two k-tiles ahead: an even number of k-tiles
         return launch_tile_wdirect<128, 256, 128, 64, TK, true, true>(A, W, C, M, N, K, epi,
                                                                       stream);
