@@ -31,10 +31,12 @@ HOST_MODULES = ("cache_core",)
 HEADERS = ("zf_common.h", "zf_no_alloc.h", "zf_chunks.h", "zf_decode.h")
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-Wall"]
 # -packed-fp32-ops off: hipcc must not form packed 32-bit float instructions by itself
-# kernarg preload: a wave starts with the first 16 words of its arguments in scalar registers instead of asking
-# memory for them, which every load of a short kernel waits for.  Measured on MI355X, ms without -> with: a 0.6B
-# decoder in 32-bit, 23.7 -> 22.8; 64 users of an 8B one 283 -> 280,
-# a 14B one's mixed steps 205 -> 201; nothing was slower.
+# kernarg preload: a wave starts with the first words of its arguments in scalar registers instead of asking
+# memory for them, which every load of a short kernel waits for.  16 is what is asked for; a kernel gets the
+# words for which it has user registers left, 14 at most (16 registers less the arguments' address), 9 to 13
+# where it takes other inputs or an 8-byte argument would be cut in two.  Measured on MI355X, ms without ->
+# with: a 0.6B decoder in 32-bit, 23.7 -> 22.8; 64 users of an 8B one 283 -> 280, a 14B one's mixed steps
+# 205 -> 201; nothing was slower.
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-mllvm", "-amdgpu-kernarg-preload-count=16",
