@@ -486,6 +486,12 @@ def test_256_token_tiles_leave_what_they_slow_down():
     assert ops._tile256_choice(1408, 5120, 5120, True) == 22
     assert ops._tile256_tail_split(698, 24576, 4096) is not None
     assert ops._tile256_tail_split(3381, 5120, 2048) is None and ops._tile256_tail_split(2816, 6144, 2560) is None
+    # many tokens of few outputs, and more than four rounds of 192 outputs over a short K
+    for M, N, K in ((3091, 1728, 4992), (5358, 896, 11520), (4820, 1280, 14464), (7144, 704, 11136)):
+        assert ops._tile256_choice(M, N, K) is None, (M, N, K)
+    assert ops._tile256_choice(4501, 1152, 7168, True) is None and ops._tile256_choice(4978, 1152, 4736, True) == 22
+    assert ops._tile256_choice(4036, 1152, 17536) == 22 and ops._tile256_choice(2597, 1728, 4992) == 22
+    assert ops._tile256_choice(3919, 13760, 3840) != 21 and ops._tile256_choice(4503, 15232, 4096) == 21
 
 
 def test_256_token_tiles_split_their_last_round_where_it_is_short():
@@ -539,6 +545,20 @@ def test_decode_attention_in_32_bit_where_it_pays():
         assert not pays(*args), args
     for args in ((63, 32, 8, 200), (64, 32, 4, 128), (64, 32, 4, 1025), (200, 16, 8, 200), (4, 16, 8, 4000)):
         assert pays(*args), args
+
+
+def test_tiles_through_a_ring_leave_splits_that_are_faster():
+    """Both sides of the lines towards products split along K: stored ones of three parts and more over a K from
+    6000 on, sums of more than 1024 tokens by the estimates, 64 x 64 tiles of many tokens over long parts."""
+    for M, N, K in ((768, 896, 7424), (887, 1344, 6400), (356, 1920, 6976), (646, 384, 7616)):
+        assert ops._tile_ksplit(M, N, K, False) >= 3 and ops._ring_choice(M, N, K) is None, (M, N, K)
+        assert ops._ring_choice(M, N, K, True) is not None
+    assert ops._ring_choice(2525, 768, 7424) == 31 and ops._ring_choice(1181, 448, 4864) == 32
+    assert ops._ring_choice(388, 896, 6528) == 32          # (in the place of tiles of 64 tokens, unsplit)
+    for M, N, K in ((2505, 896, 3008), (1383, 1088, 18432), (7700, 384, 17728), (5849, 320, 4992)):
+        assert ops._tile_ksplit(M, N, K) > 1 and ops._ring_sum(M, N, K) is None, (M, N, K)
+    assert ops._ring_sum(903, 3136, 18368) == (33, 2) and ops._ring_sum(4610, 448, 4224) == (33, 3)
+    assert ops._ring_sum(1905, 256, 6464)[0] != 32 and ops._ring_sum(470, 384, 19840) == (32, 5)
 
 
 def test_tiles_through_a_ring_are_chosen_where_one_round_holds_the_product():

@@ -954,12 +954,17 @@ def _ring_choice(M: int, N: int, K: int, gated: bool = False):
     -> 38.2), and over a long K 128 x 128 tiles that leave a third of the chip idle or have weights too
     many to wait for (384 tokens into 6144 over 4096, 144 tiles, 33.3 -> 34.6; 512 into 7168 over 5120 47.3 ->
     47.5); nor in the place of one round of 64 x 128 tiles (521 tokens into 3584 over 1024 8.7 -> 10.3).
-    Under 64 tiles of 64 x 64 the split along K stays, and over a K beyond 8192 for a stored product (871
-    tokens into 1280 over 14336 52.7 -> 75.8; a gated one has none: 692 into 2048 over 12288 99 -> 57).  Of 210
-    drawn products two lose, 3 % each; stored ones gain a quarter in the mean, gated ones four fifths."""
+    Under 64 tiles of 64 x 64 the split along K stays, over a K beyond 8192 for a stored product (871
+    tokens into 1280 over 14336 52.7 -> 75.8; a gated one has none: 692 into 2048 over 12288 99 -> 57), and
+    from 6000 on for one that would be split in three or more (768 into 896 over 7424 25.7 -> 32.9, 887 into 1344
+    over 6400 31.2 -> 39.7; eight over 5300 to 5900 gain 5 % in the mean, 0.93 to 1.23; in two 2525 into 768 over
+    7424 44.8 -> 35.9).  Of 181
+    drawn products none loses more than 2 %; they gain three fifths in the mean."""
     if M <= 128 or K % 64 != 0 or N % 16 != 0:
         return None
     if K > 8192 and not gated:
+        return None
+    if K >= 6000 and not gated and not _tile64_covers(M, N, K, False) and _tile_ksplit(M, N, K, False) >= 3:
         return None
     shape = next((s for s in (32, 31, 30) if _ring_tiles(s, M, N) <= 256), None)
     if shape is None or _ring_tiles(shape, M, N) < 64:
@@ -979,17 +984,21 @@ _RING_STEP = {32: (0.086, 0.073), 31: (0.142, 0.158), 30: (0.295, 0.258), 33: (0
 def _ring_sum(M: int, N: int, K: int):
     """(shape, parts of K) if a residual sum with the norm behind it should run through the ring kernels: the
     tile and split that fill five eighths of one round of the chip or more (half of it whole over a K of up to
-    2048) and that the estimate likes best, which is 6 % off in the mean over 700 measured ones.  Measured on MI355X, us, the norm's kernel included, what
-    ran before -> these: 64 x 64 tiles 256 tokens into 2048 over 2048 in two parts 16.4 -> 11.9, 512 into
+    2048) and that the estimate likes best, which is 6 % off in the mean over 700 measured ones.  Measured on
+    MI355X, us, the norm's kernel included, what ran before -> these: 64 x 64 tiles 256 tokens into 2048 over 2048 in two parts 16.4 -> 11.9, 512 into
     1024 over 3072 16.8 -> 13.7, 1024 whole 22.0 -> 17.2; 128 x 64 256 into 2560 over 4096 in three 20.4
     -> 16.8, into 4096 over 4096 in two 24.1 -> 21.7; 128 x 128 1024 into 4096 over 4096 55.2 -> 47.5, 1536 into
     2048 over 6144 68.4 -> 53.3; 128 x 256 384 into 4096 over 12288 in five 60.7 -> 54.7, into 5120 over 17408
     in four 93.9 -> 81.6.  The small tiles read W and the tokens more often, which the estimate misses where
     the weights are many or a part is long, so each has its bounds (128 x 64 whole 509 tokens into 3584 over 5120
     34.5 -> 37.4, in two parts 384 into 2560 over 9728 36.8 -> 38.2; 64 x 64 whole 160 into 3584 over 6144 25.2
-    -> 27.5; 128 x 128 in two 374 into 4608 over 9216 53 -> 55, in four 245 into 4096 over 14336 45.8 -> 47.0;
-    and of short parts the larger ones' partials cost more, 399 into 4608 over 896 21.0 -> 23.8).
-    The splits of larger tiles stay where they are chosen (768 into 4096 over 12288 88.5 -> 102)."""
+    -> 27.5, in two 1905 into 256 over 6464 21.3 -> 23.0; 128 x 128 in two 374 into 4608 over 9216 53 -> 55, in
+    four 245 into 4096 over 14336 45.8 -> 47.0; and of short parts the larger ones' partials cost more, 399 into
+    4608 over 896 21.0 -> 23.8).  More than 1024 tokens that would be split anyway stay so unless the
+    estimates are 15 % apart (2505 into 896 over 3008 32.2 -> 36.7, 1383 into 1088 over 18432 79.0 -> 86.9; fewer
+    gain, 903 into 3136 over 18368 156 -> 139).  Of 187 drawn sums two lose more than 3 %, the worst 12, and they
+    gain a quarter in the mean.  The splits of larger tiles stay where they are chosen (768 into
+    4096 over 12288 88.5 -> 102)."""
     if M <= 128 or K % 64 != 0 or N % 16 != 0 or N > 8192 \
             or _tile256_ksplit(M, N, K) is not None or _wide_ksplit(M, N, K) is not None:
         return None
@@ -997,8 +1006,10 @@ def _ring_sum(M: int, N: int, K: int):
     for shape, (alone, full) in _RING_STEP.items():
         for parts in range(2 if shape == 33 else 1, 7):
             places, k = _ring_tiles(shape, M, N) * parts, K // parts
-            if not (128 if parts == 1 and K <= 2048 else 160) <= places <= 256 or (parts > 1 and k < (1024 if shape == 33 else 512 if shape == 30 else 256)) \
-                    or (shape in (31, 32) and weights > (15 if parts == 1 else 25)) or (shape == 32 and k > 5000) \
+            if not (128 if parts == 1 and K <= 2048 else 160) <= places <= 256 \
+                    or (parts > 1 and k < (1024 if shape == 33 else 512 if shape == 30 else 256)) \
+                    or (shape in (31, 32) and weights > (15 if parts == 1 else 25)) \
+                    or (shape == 32 and k > (3200 if parts > 1 and M > 900 else 5000)) \
                     or (shape == 31 and k > 4200) or (shape == 30 and weights > (40 if parts < 3 else 55)):
                 continue
             # the product, and its partials written and added or the sum read again by the norm
@@ -1006,6 +1017,10 @@ def _ring_sum(M: int, N: int, K: int):
                 + (1.2 + 1.34e-6 * M * N * parts if parts > 1 else 1.3 + 1.0e-6 * M * N)
             if best_t is None or t < best_t:
                 best, best_t = (shape, parts), t
+    split = _tile_ksplit(M, N, K)
+    if best is not None and M > 1024 and split > 1:
+        other = _tile128_time(M, N, K, _tile_variant(M, N, True, True, K), split)
+        return best if best_t * 1e-6 < 0.845 * other else None
     return best
 
 
@@ -1075,13 +1090,16 @@ def _tile256_choice(M: int, N: int, K: int, accumulate: bool = False):
     the norm behind: 4096 into 4096 over 12288 359 -> 310, 8192 713 -> 622, over 4096 291 -> 265.
     Not where they are the slower ones: K under 2048 (what a tile costs besides; 4096 tokens into 6144
     over 1024 51 -> 52), tiles of 192 outputs over a K of 8192 and more (4096 tokens into 5120 over
-    17408 637 -> 668), or of a round or less, and up to a round and three quarters where the 128 x 256 tiles split
+    17408 637 -> 668), in more than four rounds over one under 4096 (GEGLU, 3919 tokens into 13760 over 3840 355 ->
+    380), or of a round or less, and up to a round and three quarters where the 128 x 256 tiles split
     a short last round (698 tokens into 24576 over 4096 140 -> 150, 3648 into 5120 over 5120 198 -> 215); residual
     sums into few outputs through tiles of 128 (1184 tokens into 4096 over 4096 61 -> 67, 3200 into 2048 over
-    6144 89 -> 99; into 5120 over 5120 87 -> 84) or whose last round is short (8192 tokens into 5120 over 8192
+    6144 89 -> 99; into 5120 over 5120 87 -> 84) or, over a K under 16000, any other product of more than 1.6
+    times as many tokens (3091 into 1728 over 4992 61 -> 68, 5358 into 896 over 11520 121 -> 131: two thirds of 36
+    drawn ones slower, 2 % in the mean), sums whose last round is short (8192 tokens into 5120 over 8192
     602 -> 616), and a last round that the 128 x 256 tiles split along K unless a tenth is gained
-    (512 tokens into 34816 over 5120 165 -> 172).  Of 1062 drawn products that this rule could move, timed in
-    changing order, it gains 7 % in the mean and makes 33 slower by more than 3 %, the worst by 8."""
+    (512 tokens into 34816 over 5120 165 -> 172).  Of 287 drawn products that this rule moves, timed in
+    changing order, it gains 7 % in the mean and makes nine slower by more than 3 %, the worst by 9."""
     even = _tile256_variant(M, N, K, accumulate)
     if even is not None:
         return even
@@ -1090,9 +1108,12 @@ def _tile256_choice(M: int, N: int, K: int, accumulate: bool = False):
         return None
     tail = now == 10 and _tile_tail_split(M, N, K) is not None
     tiles = ((M + 255) // 256) * ((N + 191) // 192)
-    best = min((20, 22) if K >= 8192 or tiles <= (448 if tail else 256) else (20, 21, 22),
+    no_192 = K >= 8192 or tiles <= (448 if tail else 256) or K < 4096 and tiles > 4 * 256
+    best = min((20, 22) if no_192 else (20, 21, 22),
                key=lambda v: _tile256_estimate(v, M, N, K, accumulate))
-    if accumulate and best == 22 and now == 12 and N <= 4096 and K <= 6144:
+    tall = M > 1.6 * N
+    if best == 22 and (accumulate and now == 12 and N <= 4096 and K <= (8192 if tall else 6144)
+                       or not accumulate and tall and K < 16000):
         return None
     gain = 0.9 if tail else 0.95
     return best if _tile256_estimate(best, M, N, K, accumulate) < gain * _tile128_estimate(M, N, K, now) \
